@@ -153,6 +153,23 @@ def load():
     return lib
 
 
+_host = None
+
+
+def host():
+    """The native host path (csrc/host.cpp) with the library's entry points bound to it. Raises like :func:`load`."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as ex:
+            raise ImportError(f"{_HERE}/_host.so: {ex}; build it with `python -m keys_values_amd.build`") from ex
+        module.bind(LIB_PATH, KvxError, torch.OutOfMemoryError)
+        _host = module
+    return _host
+
+
 def load_error():
     return _load_error
 

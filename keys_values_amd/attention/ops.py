@@ -64,14 +64,7 @@ def get_device_info(device_id: int = 0) -> str:
     return buf.value.decode()
 
 
-# ---- argument plumbing ----------------------------------------------------------------------------
-
-
-def _check_bhtd(name: str, t: torch.Tensor):
-    if t.ndim != 4:
-        raise ValueError(f"{name} must be a 4D tensor, got shape {tuple(t.shape)}")
-    if t.stride(-1) != 1:
-        raise ValueError(f"{name}: the head dimension must be contiguous (stride {t.stride(-1)})")
+# ---- argument blocks for callers that launch through the C ABI themselves ------------------------------
 
 
 def _fill_common(a: _lib.SdpaArgs, query, key, value, scale, input_pos, token_positions, quant, num_splits):
@@ -106,32 +99,6 @@ def _fill_common(a: _lib.SdpaArgs, query, key, value, scale, input_pos, token_po
         a.tp_stride_b, a.tp_stride_h = token_positions.stride(0), token_positions.stride(1)
 
 
-def _row_len(D: int, key: torch.Tensor, quant) -> int:
-    """Last-axis length a cache row must have: D, or D/2 bytes for the 4-bit store."""
-    return D // 2 if (quant is not None and key.shape[3] * 2 == D) else D
-
-
-def _check_dtypes(query, key, value, quant):
-    if query.dtype not in ALLOWED_DTYPES:
-        raise NotImplementedError(f"query.dtype must be torch.bfloat16 or torch.float16, got {query.dtype}")
-    want = torch.uint8 if quant is not None else query.dtype
-    for name, t in (("key", key), ("value", value)):
-        if t is not None and t.dtype != want:
-            raise NotImplementedError(f"{name}.dtype must be {want}, got {t.dtype}")
-
-
-def _token_positions_i32(token_positions, B, Hkv, T):
-    if token_positions is None:
-        return None
-    if token_positions.shape != (B, Hkv, T):
-        raise ValueError(f"token_positions.shape = {tuple(token_positions.shape)}, must be {(B, Hkv, T)}")
-    if token_positions.dtype != torch.int32:
-        token_positions = token_positions.to(torch.int32)
-    if token_positions.stride(-1) != 1:
-        token_positions = token_positions.contiguous()
-    return token_positions
-
-
 def prefill_core(
     query: torch.Tensor,
     key: torch.Tensor,
@@ -150,78 +117,13 @@ def prefill_core(
     Returns ``(out, weights, lse)``: ``out`` is (B, q, Hq, D) if ``output_transposed`` (the layout
     of the reference extension) else (B, Hq, q, D); ``weights`` fp32 (B, Hkv, T) summed over queries
     and averaged over the group; ``lse`` fp32 (B, q, Hq) in base 2."""
-    _lib.require_gpu(query, key, value)
-    for n, t in (("query", query), ("key", key), ("value", value)):
-        _check_bhtd(n, t)
-    _check_dtypes(query, key, value, quant)
-    B, Hq, q_len, D = query.shape
-    Hkv, T = key.shape[1], key.shape[2]
-    if key.shape != value.shape or key.shape[0] != B or key.shape[3] != _row_len(D, key, quant):
-        raise ValueError(f"key.shape = {tuple(key.shape)}, value.shape = {tuple(value.shape)} do not fit query {tuple(query.shape)}")
-    if not (0 < q_len <= T):
-        raise ValueError(f"Must have 0 < q_len = {q_len} <= kv_len = {T}")
-    if Hkv <= 0 or Hq % Hkv != 0:
-        raise ValueError(f"n_head = {Hq} must be a positive multiple of n_query_groups = {Hkv}")
-    if D not in (ALLOWED_HEAD_SIZES if quant is None else QUANTIZED_HEAD_SIZES):
-        raise NotImplementedError(f"head size {D} not in {ALLOWED_HEAD_SIZES if quant is None else QUANTIZED_HEAD_SIZES}")
-    token_positions = _token_positions_i32(token_positions, B, Hkv, T)
-    dev = query.device
-    lib = _lib.load()
-    with torch.cuda.device(dev):
-        if output_transposed:
-            out = torch.empty((B, q_len, Hq, D), dtype=query.dtype, device=dev)
-            o_view = out.permute(0, 2, 1, 3)
-        else:
-            out = torch.empty((B, Hq, q_len, D), dtype=query.dtype, device=dev)
-            o_view = out
-        need_lse = return_lse or return_weights
-        lse = torch.empty((B, q_len, Hq), dtype=torch.float32, device=dev) if need_lse else None
-        w = torch.empty((B, Hkv, T), dtype=torch.float32, device=dev) if return_weights else None
-        a = _lib.SdpaArgs()
-        _fill_common(a, query, key, value, scale, input_pos, token_positions, quant, num_splits)
-        a.o = o_view.data_ptr()
-        a.o_stride_b, a.o_stride_h, a.o_stride_t = o_view.stride(0), o_view.stride(1), o_view.stride(2)
-        a.lse = _lib.ptr(lse)
-        a.w = _lib.ptr(w)
-        nbytes = lib.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a))
-        ws = _lib.workspace(dev, nbytes)
-        a.workspace = _lib.ptr(ws)
-        a.workspace_bytes = 0 if ws is None else ws.numel()
-        fn = lib.kvx_sdpa_prefill_weights if return_weights else lib.kvx_sdpa_prefill
-        _lib.check(fn(ctypes.byref(a), _lib.stream_ptr(dev)))
-    return out, w, (lse if return_lse else None)
+    return _lib.host().prefill(query, key, value, scale, input_pos, token_positions, return_weights, return_lse, output_transposed, quant, num_splits)
 
 
 def score_sum_core(query, key, lse, scale, input_pos, token_positions=None, quant: Optional[QuantState] = None):
     """Score-sums from Q, K and a base-2 LSE (B, q, Hq): the stand-in for ``triton_score_sum``
     (keys_values/attention/flashinfer_wrapper.py:156-273) on strided (B, H, len, D) views."""
-    _lib.require_gpu(query, key, lse)
-    _check_bhtd("query", query)
-    _check_bhtd("key", key)
-    _check_dtypes(query, key, None, quant)
-    B, Hq, q_len, D = query.shape
-    Hkv, T = key.shape[1], key.shape[2]
-    if lse.shape != (B, q_len, Hq) or lse.dtype != torch.float32 or not lse.is_contiguous():
-        raise ValueError(f"lse must be contiguous float32 {(B, q_len, Hq)}, got {tuple(lse.shape)} {lse.dtype}")
-    if D not in (ALLOWED_HEAD_SIZES if quant is None else QUANTIZED_HEAD_SIZES):
-        raise NotImplementedError(f"head size {D} not in {ALLOWED_HEAD_SIZES if quant is None else QUANTIZED_HEAD_SIZES}")
-    token_positions = _token_positions_i32(token_positions, B, Hkv, T)
-    dev = query.device
-    with torch.cuda.device(dev):
-        w = torch.empty((B, Hkv, T), dtype=torch.float32, device=dev)
-        a = _lib.SdpaArgs()
-        if quant is not None:
-            quant = QuantState(quant.k_scale, quant.k_zp, quant.k_scale, quant.k_zp)
-        _fill_common(a, query, key, None, scale, input_pos, token_positions, quant, 0)
-        a.lse = lse.data_ptr()
-        a.w = w.data_ptr()
-        lib = _lib.load()
-        # short caches split the query rows over more workgroups; the partial sums need a workspace
-        ws = _lib.workspace(dev, lib.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a)))
-        a.workspace = _lib.ptr(ws)
-        a.workspace_bytes = 0 if ws is None else ws.numel()
-        _lib.check(lib.kvx_score_sum(ctypes.byref(a), _lib.stream_ptr(dev)))
-    return w
+    return _lib.host().score_sum(query, key, lse, scale, input_pos, token_positions, quant)
 
 
 def decode_core(
@@ -239,43 +141,7 @@ def decode_core(
     Returns ``(out (B, Hq, D), weights (B, Hkv, T) or None, lse (B, 1, Hq) or None)``.
     ``scratch_splits``: optional one-element int32 device tensor that receives the number of KV splits whose logits
     went through the HBM scratch instead of staying on the chip (0 in the normal case)."""
-    _lib.require_gpu(query, key, value)
-    for n, t in (("query", query), ("key", key), ("value", value)):
-        _check_bhtd(n, t)
-    _check_dtypes(query, key, value, quant)
-    B, Hq, q_len, D = query.shape
-    Hkv, T = key.shape[1], key.shape[2]
-    if q_len != 1:
-        raise ValueError(f"decode needs q_len == 1, got {q_len}")
-    if key.shape != value.shape or key.shape[0] != B or key.shape[3] != _row_len(D, key, quant):
-        raise ValueError(f"key.shape = {tuple(key.shape)}, value.shape = {tuple(value.shape)} do not fit query {tuple(query.shape)}")
-    if Hkv <= 0 or Hq % Hkv != 0:
-        raise ValueError(f"n_head = {Hq} must be a positive multiple of n_query_groups = {Hkv}")
-    if D not in (ALLOWED_HEAD_SIZES if quant is None else QUANTIZED_HEAD_SIZES):
-        raise NotImplementedError(f"head size {D} not in {ALLOWED_HEAD_SIZES if quant is None else QUANTIZED_HEAD_SIZES}")
-    dev = query.device
-    lib = _lib.load()
-    with torch.cuda.device(dev):
-        out = torch.empty((B, Hq, D), dtype=query.dtype, device=dev)
-        o_view = out.unsqueeze(2)
-        w = torch.empty((B, Hkv, T), dtype=torch.float32, device=dev) if return_weights else None
-        lse = torch.empty((B, 1, Hq), dtype=torch.float32, device=dev) if return_lse else None
-        a = _lib.SdpaArgs()
-        _fill_common(a, query, key, value, scale, max(T - 1, 0), None, quant, num_splits)
-        a.o = o_view.data_ptr()
-        a.o_stride_b, a.o_stride_h, a.o_stride_t = o_view.stride(0), o_view.stride(1), o_view.stride(2)
-        a.w = _lib.ptr(w)
-        a.lse = _lib.ptr(lse)
-        if scratch_splits is not None:
-            if scratch_splits.dtype != torch.int32 or scratch_splits.numel() != 1 or scratch_splits.device != dev:
-                raise ValueError("scratch_splits must be a one-element int32 tensor on the query's device")
-            a.decode_scratch_splits = scratch_splits.data_ptr()
-        nbytes = lib.kvx_sdpa_decode_workspace_bytes(ctypes.byref(a))
-        ws = _lib.workspace(dev, nbytes)
-        a.workspace = _lib.ptr(ws)
-        a.workspace_bytes = 0 if ws is None else ws.numel()
-        _lib.check(lib.kvx_sdpa_decode(ctypes.byref(a), _lib.stream_ptr(dev)))
-    return out, w, lse
+    return _lib.host().decode(query, key, value, scale, return_weights, return_lse, quant, num_splits, scratch_splits)
 
 
 # ---- the reference's entry points (keys_values/attention/flashinfer_ops.py:193-440) --------------

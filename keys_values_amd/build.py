@@ -1,16 +1,20 @@
 """
-Build recipe of libkvx.so: hipcc for gfx950 on the HIP sources under csrc/, linked into one shared
-library next to this file. Cross-compiles without a GPU. Run as `python -m keys_values_amd.build`.
+Build recipe of libkvx.so (hipcc for gfx950 on the HIP sources under csrc/, linked into one shared library next to this
+file) and of _host.so (the extension module of csrc/host.cpp, host code only, against the installed PyTorch).
+Cross-compiles without a GPU. Run as `python -m keys_values_amd.build`.
 """
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
+from importlib.util import find_spec
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libkvx.so")
+HOST = os.path.join(HERE, "_host.so")
 SOURCES = ["kvx_api.hip", "sdpa_prefill.hip", "score_sum.hip", "sdpa_decode.hip", "quantize.hip", "h2o.hip", "norm_rope.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -41,9 +45,23 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _build_host():
+    torch_dir = os.path.dirname(find_spec("torch").origin)
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           "-I" + sysconfig.get_paths()["include"], "-isystem", os.path.join(rocm, "include"), "-isystem", os.path.join(torch_dir, "include"),
+           "-isystem", os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"), os.path.join(CSRC, "host.cpp"), "-o", HOST,
+           "-L" + os.path.join(torch_dir, "lib"), "-ltorch_python", "-ltorch_cpu", "-ltorch_hip", "-lc10_hip", "-lc10", "-ldl"]
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on host.cpp:\n{res.stdout}")
+
+
 def build(verbose: bool = True) -> str:
-    with ThreadPoolExecutor(max_workers=min(7, os.cpu_count() or 1)) as ex:
+    with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as ex:
+        host = ex.submit(_build_host)
         objs = list(ex.map(_compile, SOURCES))
+        host.result()
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs
     res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if res.returncode != 0:

@@ -206,6 +206,11 @@ class H2OKVCache:
             self._kv_zp = torch.zeros((2, b, h, length), dtype=torch.int32, device=self.device)
             self.k_scale, self.v_scale = self._kv_scale[0], self._kv_scale[1]
             self.k_zp, self.v_zp = self._kv_zp[0], self._kv_zp[1]
+        # what the slot write and the attention kernels see: the codes, or (plain stores, blocks over the heads) 16-bit rows
+        self._store_quantized = quantized and not self.blocks_over_heads
+        self._store_dtype = _lib.quant_kv_dtype(num_bits, self.dtype) if self._store_quantized else _lib.elem_kv_dtype(self.dtype)
+        # any run of slots that all heads share (the prefill, free slots, the initial rule) is a view of this
+        self._all_slots = torch.arange(length, dtype=torch.int32, device=self.device)
         self.token_pos = torch.zeros((b, h, length), dtype=torch.int32, device=self.device)  # attn_weights.py:466-470
         self.scores = torch.zeros((b, h, length), dtype=torch.float32, device=self.device)  # h2o.py:85-91
         # further score buffers, moved and initialised with the slots (h2o.py:405-413, qh2o.py:107-113)
@@ -411,19 +416,24 @@ class H2OKVCache:
             raise ValueError(f"token_idx must be given with shape {(self.batch_size, num)} while the replay log is on")
         self._log_chunks.append(token_idx.detach().clone())  # keys_values/kvcache/base.py:844-855
 
+    def _run_of_slots(self, start: int, num: int) -> torch.Tensor:
+        """Slots ``start .. start + num - 1`` for every (batch, head): a view with strides 0."""
+        return self._all_slots[start : start + num].expand(self.batch_size, self.n_query_groups, num)
+
+    def _in_use(self, t: torch.Tensor, T: int) -> torch.Tensor:
+        """The part of a (max_batch, n_query_groups, cache_length, ...) buffer that the current sequences use."""
+        return t if self.batch_size == self.max_batch_size and T == self.cache_length else t[: self.batch_size, :, :T]
+
     def _quant_state(self, T: int) -> Optional[ops.QuantState]:
-        if not self.quantized or self.blocks_over_heads:  # blocks over heads: the kernels read the working buffer
+        if not self._store_quantized:  # blocks over heads: the kernels read the working buffer
             return None
-        b = self.batch_size
-        return ops.QuantState(self.k_scale[:b, :, :T], self.k_zp[:b, :, :T], self.v_scale[:b, :, :T], self.v_zp[:b, :, :T])
+        return ops.QuantState(self._in_use(self.k_scale, T), self._in_use(self.k_zp, T), self._in_use(self.v_scale, T), self._in_use(self.v_zp, T))
 
     def _next_index_for(self, num: int, peek: bool = False) -> Optional[torch.Tensor]:
-        b, h = self.batch_size, self.n_query_groups
         if self.current_length is None:
             return None
         if self.current_length < self.cache_length:  # free slots, attn_weights.py:1001-1016
-            start = self.current_length
-            return torch.arange(start, start + num, dtype=torch.int32, device=self.device).view(1, 1, -1).expand(b, h, -1).contiguous()
+            return self._run_of_slots(self.current_length, num)
         if self._use_initial_rule:  # attn_weights.py:536-550
             n0 = min(int(self._keep_initial_fraction * self.cache_length), self.cache_length - num)
             # with a grace period the evicted slots must stay below the ring (the reference's formula
@@ -431,27 +441,19 @@ class H2OKVCache:
             n0 = min(n0, self.cache_length - self.grace_period - num)
             if not peek:
                 self._use_initial_rule = False
-            return torch.arange(n0, n0 + num, dtype=torch.int32, device=self.device).view(1, 1, -1).expand(b, h, -1).contiguous()
+            return self._run_of_slots(n0, num)
         if not self._have_next:
             return None
         if num > self._next_count:
             self._select_more(num)
-        return self._next_index[:b, :, :num]
+        return self._next_index[: self.batch_size, :, :num]
 
     def _select_more(self, num: int):
         """The step before chose fewer slots than are asked for now (it could not know): choose ``num`` from
         the same scores. Nothing is added to them (no weights), so the first entries come out as before."""
         if num > self._select_k:
             raise ValueError(f"num = {num} exceeds what a full cache hands out ({self._select_k})")
-        a = self._h2o_args(True, num)
-        a.next_index = self._next_flat.data_ptr()
-        lib = _lib.load()
-        with torch.cuda.device(self.device):
-            nbytes = lib.kvx_h2o_workspace_bytes(ctypes.byref(a))
-            ws = _lib.workspace(self.device, nbytes)
-            a.workspace = _lib.ptr(ws)
-            a.workspace_bytes = 0 if ws is None else ws.numel()
-            _lib.check(lib.kvx_h2o_update_select(ctypes.byref(a), _lib.stream_ptr(self.device)))
+        _lib.host().cache_update(self, None, 1, num, True)
         self._next_count = num
 
     # -- the step (keys_values/kvcache/base.py:554-595) -----------------------------------------
@@ -459,12 +461,8 @@ class H2OKVCache:
     def forward(self, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, token_idx: Optional[torch.Tensor] = None) -> torch.Tensor:
         """query (B, n_head, num, hs); key/value (B, n_query_groups, num, hs). Returns the attention
         output (B, num, n_head * hs) (keys_values/attention/base.py:378-380)."""
-        _lib.require_gpu(query, key, value)
-        if query.ndim != 4 or key.ndim != 4 or key.shape != value.shape:
-            raise ValueError("query, key, value must be 4D and key.shape == value.shape")
-        b, hq, num, d = query.shape
-        if key.shape != (b, self.n_query_groups, num, d) or hq != self.n_head or d != self.head_size:
-            raise ValueError(f"shapes {tuple(query.shape)}, {tuple(key.shape)} do not fit the cache")
+        host = _lib.host()
+        b, num = host.check_qkv(query, key, value, self.n_head, self.n_query_groups, self.head_size)
         input_pos = self._input_pos
         self.wait_for_selection()
         if self.blocks_over_heads:
@@ -482,6 +480,21 @@ class H2OKVCache:
             if 0 < diff < num:
                 raise ValueError(f"key.shape[2] = {num}, must be <= {diff} as long as the cache is not full")
             raise ValueError(f"key.shape[2] = {num}, must be in [1, {self.max_forward_length()}]")
+        if num == 1 and diff == 0 and not self.blocks_over_heads:
+            # one token into a full cache: slot write, attention, score update and eviction choice in one call
+            index = None  # the slots chosen by the step before
+            if self._use_initial_rule or not self._have_next:
+                index = self._next_index_for(num)
+                if index is None:
+                    raise IndexError("Cache needs to be initialized with 'prefill' before being used")
+            self._log_token_chunk(token_idx, num, prefill=False)
+            ring, log = self._ring_and_log(num, input_pos)
+            out = host.cache_decode_step(self, query, key, value, index, input_pos, ring, log)
+            self._input_pos = input_pos + 1
+            # the lowest-score slot only: a following single-token step needs no more, anything longer selects again
+            self._have_next = True
+            self._next_count = 1
+            return out
         index = self._next_index_for(num)
         if index is None:
             raise IndexError("Cache needs to be initialized with 'prefill' before being used")
@@ -494,24 +507,22 @@ class H2OKVCache:
             self.current_length += num
         self._have_next = False
         self._input_pos += num
-        T = self.current_length
-        kc, vc = self.k[:b, :, :T], self.v[:b, :, :T]
-        tp = self.token_pos[:b, :, :T]
+        T, hq, d = self.current_length, self.n_head, self.head_size
+        kc, vc = self._in_use(self.k, T), self._in_use(self.v, T)
         quant = self._quant_state(T)
         if num == 1 and T == self.cache_length:
-            # one token into a full cache: attention, score update and eviction choice in one call
-            out = self._decode_h2o_step(query, kc, vc, quant).unsqueeze(1)
-            return out.reshape(b, num, hq * d)
+            # blocks over the heads: what is left after the write-back, in one call
+            return self._decode_h2o_step(query, kc, vc, quant).view(b, num, hq * d)
         if num == 1:
-            out, w, _ = ops.decode_core(query, kc, vc, self.scale_factor, return_weights=True, quant=quant)
-            out = out.unsqueeze(1)
+            out, w, _ = host.decode(query, kc, vc, self.scale_factor, True, False, quant, 0, None)
         else:
+            tp = self._in_use(self.token_pos, T)
             rows = num * (hq // self.n_query_groups)
             if quant is not None and self.dequantize_chunk_rows is not None and rows >= self.dequantize_chunk_rows:
                 # attention over the bf16 copy; the score-sum pass keeps the codes (it dequantises each key
                 # once per wavefront whatever the chunk length, and reads half the bytes)
                 kd, vd = self._dequantized(b, T)
-                out, _, lse = ops.prefill_core(query, kd, vd, self.scale_factor, input_pos, tp, return_lse=True, output_transposed=True)
+                out, _, lse = host.prefill(query, kd, vd, self.scale_factor, input_pos, tp, False, True, True, None, 0)
                 if self._overlap:
                     # the score-sum pass too runs beside the caller's next launches: nothing needs the score-sums
                     # before the next chunk's eviction choice
@@ -521,17 +532,16 @@ class H2OKVCache:
                     ready.record(main)
                     with torch.cuda.stream(side):
                         side.wait_event(ready)
-                        w = ops.score_sum_core(query, kc, lse, self.scale_factor, input_pos, tp, quant=quant)
+                        w = host.score_sum(query, kc, lse, self.scale_factor, input_pos, tp, quant)
                         self._update(w, num)
                     query.record_stream(side)
                     lse.record_stream(side)
-                    return out.reshape(b, num, hq * d)
-                w = ops.score_sum_core(query, kc, lse, self.scale_factor, input_pos, tp, quant=quant)
+                    return out.view(b, num, hq * d)
+                w = host.score_sum(query, kc, lse, self.scale_factor, input_pos, tp, quant)
             else:
-                out, w, _ = ops.prefill_core(query, kc, vc, self.scale_factor, input_pos, tp, return_weights=True,
-                                             output_transposed=True, quant=quant)
+                out, w, _ = host.prefill(query, kc, vc, self.scale_factor, input_pos, tp, True, False, True, quant, 0)
         self._update(w, num)
-        return out.reshape(b, num, hq * d)
+        return out.view(b, num, hq * d)
 
     __call__ = forward
 
@@ -604,19 +614,13 @@ class H2OKVCache:
         h, length, d = self.n_query_groups, self.cache_length, self.head_size
         rows = b * h * length
         kd, vd, _ = _dequant_scratch(self.device, rows * d, self.dtype)
-        lib = _lib.load()
-        bits, elem = self.num_bits, _lib.elem_kv_dtype(self.dtype)
-
-        def fn(c, s, z, n, dd, o, stride, stream):
-            return lib.kvx_dequantize_rows_typed(c, s, z, n, dd, bits, elem, o, stride, stream)
-
-        with torch.cuda.device(self.device):
-            stream = _lib.stream_ptr(self.device)
-            if b == self.max_batch_size:  # K and V are adjacent in the store and in the scratch: one launch
-                _lib.check(fn(self._kv.data_ptr(), self._kv_scale.data_ptr(), self._kv_zp.data_ptr(), 2 * rows, d, kd.data_ptr(), d, stream))
-            else:
-                _lib.check(fn(self.k.data_ptr(), self.k_scale.data_ptr(), self.k_zp.data_ptr(), rows, d, kd.data_ptr(), d, stream))
-                _lib.check(fn(self.v.data_ptr(), self.v_scale.data_ptr(), self.v_zp.data_ptr(), rows, d, vd.data_ptr(), d, stream))
+        host = _lib.host()
+        if b == self.max_batch_size:  # K and V are adjacent in the store and in the scratch: one launch
+            both = kd.as_strided((2 * rows, d), (d, 1))
+            host.dequantize_rows(self._kv, self._kv_scale, self._kv_zp, self.num_bits, both)
+        else:
+            host.dequantize_rows(self.k, self.k_scale, self.k_zp, self.num_bits, kd.view(rows, d))
+            host.dequantize_rows(self.v, self.v_scale, self.v_zp, self.num_bits, vd.view(rows, d))
         return kd.view(b, h, length, d)[:, :, :T], vd.view(b, h, length, d)[:, :, :T]
 
     def _prefill_step(self, query, key, value):
@@ -628,7 +632,7 @@ class H2OKVCache:
         if num > self.max_prefill_length:
             raise ValueError(f"prefill length {num} exceeds cache_length {self.cache_length}")
         self.batch_size = b
-        index = torch.arange(num, dtype=torch.int32, device=self.device).view(1, 1, -1).expand(b, self.n_query_groups, -1).contiguous()
+        index = self._run_of_slots(0, num)
         self.scores.zero_()
         for extra in (self.v_norm, self.q_errors):
             if extra is not None:
@@ -646,62 +650,33 @@ class H2OKVCache:
         self._input_pos = num
         out, _, _ = ops.prefill_core(query, key.to(self.dtype), value.to(self.dtype), self.scale_factor, 0, None,
                                      return_weights=False, output_transposed=True)
-        return out.reshape(b, num, hq * d)
+        return out.view(b, num, hq * d)
 
-    def _write(self, index: torch.Tensor, key: torch.Tensor, value: torch.Tensor, input_pos: int):
-        b, h, num = index.shape
-        key = key.to(self.dtype)
-        value = value.to(self.dtype)
-        if key.stride(-1) != 1:
-            key = key.contiguous()
-        if value.stride(-1) != 1:
-            value = value.contiguous()
-        a = _lib.CacheWriteArgs()
-        a.B, a.Hkv, a.num, a.D, a.cache_len = b, h, num, self.head_size, self.cache_length
-        a.input_pos = input_pos
-        codes = self.quantized and not self.blocks_over_heads
-        a.kv_dtype = _lib.quant_kv_dtype(self.num_bits, self.dtype) if codes else _lib.elem_kv_dtype(self.dtype)
-        a.index = index.data_ptr()
-        a.index_stride_b, a.index_stride_h = index.stride(0), index.stride(1)
-        a.key = key.data_ptr()
-        a.key_stride_b, a.key_stride_h, a.key_stride_t = key.stride(0), key.stride(1), key.stride(2)
-        a.value = value.data_ptr()
-        a.value_stride_b, a.value_stride_h, a.value_stride_t = value.stride(0), value.stride(1), value.stride(2)
-        a.k_cache = self.k.data_ptr()
-        a.kc_stride_b, a.kc_stride_h, a.kc_stride_t = self.k.stride(0), self.k.stride(1), self.k.stride(2)
-        a.v_cache = self.v.data_ptr()
-        a.vc_stride_b, a.vc_stride_h, a.vc_stride_t = self.v.stride(0), self.v.stride(1), self.v.stride(2)
-        if codes:
-            a.k_scale, a.k_zp = self.k_scale.data_ptr(), self.k_zp.data_ptr()
-            a.v_scale, a.v_zp = self.v_scale.data_ptr(), self.v_zp.data_ptr()
-            a.qs_stride_b, a.qs_stride_h = self.k_scale.stride(0), self.k_scale.stride(1)
-        a.token_pos = self.token_pos.data_ptr()
-        a.tp_stride_b, a.tp_stride_h = self.token_pos.stride(0), self.token_pos.stride(1)
-        a.scores = self.scores.data_ptr()
-        a.sc_stride_b, a.sc_stride_h = self.scores.stride(0), self.scores.stride(1)
-        # blocks over the heads: the row-quantising write cannot give the blocks' errors (_block_errors does)
-        a.v_norm, a.q_errors = _lib.ptr(self.v_norm), (None if self.blocks_over_heads else _lib.ptr(self.q_errors))
-        if self._log_on and self._log_arena is not None and input_pos >= self.cache_length:
+    def _ring_and_log(self, num: int, input_pos: int):
+        """What a slot write of ``num`` tokens at ``input_pos`` moves and records besides: the ring slots that make
+        room (None without a grace period) and the replay log's ``(arena, blocksize, position)`` (None when off)."""
+        log = ring = None
+        if input_pos < self.cache_length:
+            return ring, log
+        if self._log_on and self._log_arena is not None:
             # keys_values/kvcache/attn_weights.py:629-633: the slots are recorded by the kernel that consumes them
             log_pos = input_pos - self.cache_length
             self._log_arena.reserve(log_pos + num)
-            arena = self._log_arena.data
-            a.replay_log, a.log_blocksize, a.log_pos = arena.data_ptr(), self.replay_log_blocksize, log_pos
-            a.log_stride_block, a.log_stride_b, a.log_stride_h = arena.stride(0), arena.stride(1), arena.stride(2)
-        ring = None
-        if self.grace_period > 0 and input_pos >= self.cache_length:
+            log = (self._log_arena.data, self.replay_log_blocksize, log_pos)
+        if self.grace_period > 0:
             # keys_values/kvcache/attn_weights.py:267-303: the num2 oldest ring slots move out to
             # `index` and take the last num2 new tokens; wrap-around run starting at next_grace_pos
             gp = self.grace_period
             prefix = self.cache_length - gp
-            num2 = min(num, gp)
             start = self.next_grace_pos - prefix
-            ring = self._ring_twice[start : start + num2]
-            a.grace_num, a.grace_period, a.grace_slots = num2, gp, ring.data_ptr()
+            ring = self._ring_twice[start : start + min(num, gp)]
             if num <= gp:  # attn_weights.py:601-606
-                self.next_grace_pos = (self.next_grace_pos - prefix + num) % gp + prefix
-        with torch.cuda.device(self.device):
-            _lib.check(_lib.load().kvx_cache_write(ctypes.byref(a), _lib.stream_ptr(self.device)))
+                self.next_grace_pos = (start + num) % gp + prefix
+        return ring, log
+
+    def _write(self, index: torch.Tensor, key: torch.Tensor, value: torch.Tensor, input_pos: int):
+        ring, log = self._ring_and_log(index.shape[2], input_pos)
+        _lib.host().cache_write(self, index, key, value, input_pos, ring, log)
         return ring
 
     def _h2o_args(self, full: bool, k: int = 1) -> _lib.H2OArgs:
@@ -777,43 +752,26 @@ class H2OKVCache:
         if attn_weights.dtype != torch.float32:
             raise ValueError(f"attn_weights.dtype={attn_weights.dtype}, must be {torch.float32}")
         _lib.require_gpu(attn_weights)
-        attn_weights = attn_weights.contiguous()
         full = self.current_length == self.cache_length
         k_now = min(self._select_k, EAGER_SELECT) if select is None else min(select, self._select_k)
-        a = self._h2o_args(full, k_now)
-        a.w = attn_weights.data_ptr()
-        a.q_len = query_length
-        lib = _lib.load()
-        with torch.cuda.device(self.device):
-            if full:
-                nxt = self._next_flat
-            else:  # only the accumulation matters while slots are free; the choice is discarded
-                nxt = torch.empty((self.batch_size, self.n_query_groups, 1), dtype=torch.int32, device=self.device)
-            a.next_index = nxt.data_ptr()
-            nbytes = lib.kvx_h2o_workspace_bytes(ctypes.byref(a))
-            if not self._overlap:
-                ws = _lib.workspace(self.device, nbytes)
-                a.workspace = _lib.ptr(ws)
-                a.workspace_bytes = 0 if ws is None else ws.numel()
-                _lib.check(lib.kvx_h2o_update_select(ctypes.byref(a), _lib.stream_ptr(self.device)))
-            else:
-                main = torch.cuda.current_stream(self.device)
-                self._second_stream()
-                ready = torch.cuda.Event()
-                ready.record(main)
-                with torch.cuda.stream(self._side_stream):
-                    self._side_stream.wait_event(ready)
-                    ws = _lib.workspace(self.device, nbytes)  # one buffer per stream
-                    a.workspace = _lib.ptr(ws)
-                    a.workspace_bytes = 0 if ws is None else ws.numel()
-                    _lib.check(lib.kvx_h2o_update_select(ctypes.byref(a), self._side_stream.cuda_stream))
-                    done = torch.cuda.Event()
-                    done.record(self._side_stream)
-                self._select_done = done
-                # the second stream reads these: tell the allocator, and keep them until the wait
-                attn_weights.record_stream(self._side_stream)
-                nxt.record_stream(self._side_stream)
-                self._select_keep = (attn_weights, nxt)
+        if not self._overlap:
+            _lib.host().cache_update(self, attn_weights, query_length, k_now, full)
+        else:
+            attn_weights = attn_weights.contiguous()
+            main = torch.cuda.current_stream(self.device)
+            self._second_stream()
+            ready = torch.cuda.Event()
+            ready.record(main)
+            with torch.cuda.stream(self._side_stream):
+                self._side_stream.wait_event(ready)
+                _lib.host().cache_update(self, attn_weights, query_length, k_now, full)
+                done = torch.cuda.Event()
+                done.record(self._side_stream)
+            self._select_done = done
+            # the second stream uses these: tell the allocator, and keep the weights until the wait
+            attn_weights.record_stream(self._side_stream)
+            self._next_flat.record_stream(self._side_stream)
+            self._select_keep = attn_weights
         self._have_next = full
         self._next_count = k_now if full else 0
 

@@ -12,7 +12,6 @@ two codes per byte, the first half of the block in the high nibbles (:384-393,45
 
 ``RowQuantizer8`` is the 8-bit, one-block-per-row case under its earlier name.
 """
-import ctypes
 from typing import Optional, Tuple
 
 import torch
@@ -96,24 +95,6 @@ class RowQuantizer:
 
     # -- quantise / dequantise -----------------------------------------------------------------------
 
-    def _block_args(self, x: torch.Tensor, start: int, buffer, scales, zps) -> _lib.BlockQuantArgs:
-        """x (B, Hkv, num, D) bf16 with D contiguous; blocks land in slots start.. of the buffers."""
-        b, hkv, num, d = x.shape
-        a = _lib.BlockQuantArgs()
-        a.x = x.data_ptr()
-        if self.blocks_over_heads:  # block (b, t): all heads of a token
-            a.n_outer, a.n_inner, a.nseg = b, num, hkv
-            a.x_stride_outer, a.x_stride_inner, a.x_stride_seg = x.stride(0), x.stride(2), x.stride(1)
-        else:  # block (b * Hkv + h, t)
-            a.n_outer, a.n_inner, a.nseg = b * hkv, num, 1
-            a.x_stride_outer, a.x_stride_inner, a.x_stride_seg = x.stride(1), x.stride(2), 0
-        a.D, a.bits, a.elem_dtype = d, self.num_bits, _lib.elem_kv_dtype(self.source_dtype)
-        a.codes = buffer[0, start].data_ptr()
-        a.codes_stride_outer = buffer.stride(0)
-        a.scale, a.zp = scales[0, start:].data_ptr(), zps[0, start:].data_ptr()
-        a.state_stride_outer = scales.stride(0)
-        return a
-
     def _kernel_view(self, x: torch.Tensor) -> torch.Tensor:
         """A view (or copy) of x the block kernels can address: rows 16-byte aligned, strides multiples
         of 8 and, for one block per row, the (batch, head) axes collapsible into one."""
@@ -137,19 +118,12 @@ class RowQuantizer:
             return
         _lib.require_gpu(values)
         values = values.to(self.source_dtype)
-        lib = _lib.load()
-        dev = self.device
-        with torch.cuda.device(dev):
-            st = _lib.stream_ptr(dev)
-            if not self.blocks_over_heads and d in (64, 128, 256) and start == 0 and end == length and values.is_contiguous():
-                # the whole store in one pass of the row kernels (16 or 8 lanes per row)
-                _lib.check(lib.kvx_quantize_rows_typed(values.data_ptr(), d, b * hkv * length, d, self.num_bits,
-                                                       _lib.elem_kv_dtype(self.source_dtype), self.quant_buffer.data_ptr(),
-                                                       self.quant_scales.data_ptr(), self.quant_zero_points.data_ptr(), st))
-                return
-            x = self._kernel_view(values)
-            a = self._block_args(x, start, self.quant_buffer, self.quant_scales, self.quant_zero_points)
-            _lib.check(lib.kvx_quantize_blocks(ctypes.byref(a), st))
+        if not self.blocks_over_heads and d in (64, 128, 256) and num == length and values.is_contiguous():
+            # the whole store in one pass of the row kernels (16 or 8 lanes per row)
+            _lib.host().quantize_rows(values, self.quant_buffer, self.quant_scales, self.quant_zero_points, self.num_bits)
+            return
+        _lib.host().quantize_blocks(self._kernel_view(values), start, self.quant_buffer, self.quant_scales, self.quant_zero_points,
+                                    self.blocks_over_heads, self.num_bits)
 
     def dequantize(self, start: int, end: int, out: Optional[torch.Tensor] = None, block_idx: Optional[int] = None):
         """Dequantise slots ``range(start, end)`` to (B, Hkv, end - start, D) in the source dtype
@@ -167,10 +141,7 @@ class RowQuantizer:
             raise ValueError(f"out must be contiguous {self.source_dtype} of shape {(b, hkv, num, d)}")
         if num == 0:
             return out
-        lib = _lib.load()
-        with torch.cuda.device(dev):
-            a = self._block_args(out, start, self.quant_buffer, self.quant_scales, self.quant_zero_points)
-            _lib.check(lib.kvx_dequantize_blocks(ctypes.byref(a), _lib.stream_ptr(dev)))
+        _lib.host().dequantize_blocks(out, start, self.quant_buffer, self.quant_scales, self.quant_zero_points, self.blocks_over_heads, self.num_bits)
         return out
 
     def quantization_error(self, x: torch.Tensor) -> torch.Tensor:
@@ -183,16 +154,14 @@ class RowQuantizer:
         xs = self._kernel_view(x.to(self.source_dtype))
         b, hkv, n, d = xs.shape
         dev = xs.device
-        lib = _lib.load()
+        host = _lib.host()
         first = b if self.blocks_over_heads else b * hkv
-        with torch.cuda.device(dev):
-            st = _lib.stream_ptr(dev)
-            codes = torch.empty((first, n, self.blocksize * self.num_bits // 8), dtype=torch.uint8, device=dev)
-            sc = torch.empty((first, n), dtype=torch.float32, device=dev)
-            zp = torch.empty((first, n), dtype=torch.int32, device=dev)
-            back = torch.empty((b, hkv, n, d), dtype=self.source_dtype, device=dev)
-            _lib.check(lib.kvx_quantize_blocks(ctypes.byref(self._block_args(xs, 0, codes, sc, zp)), st))
-            _lib.check(lib.kvx_dequantize_blocks(ctypes.byref(self._block_args(back, 0, codes, sc, zp)), st))
+        codes = torch.empty((first, n, self.blocksize * self.num_bits // 8), dtype=torch.uint8, device=dev)
+        sc = torch.empty((first, n), dtype=torch.float32, device=dev)
+        zp = torch.empty((first, n), dtype=torch.int32, device=dev)
+        back = torch.empty((b, hkv, n, d), dtype=self.source_dtype, device=dev)
+        host.quantize_blocks(xs, 0, codes, sc, zp, self.blocks_over_heads, self.num_bits)
+        host.dequantize_blocks(back, 0, codes, sc, zp, self.blocks_over_heads, self.num_bits)
         return torch.linalg.vector_norm(xs - back, dim=-1, dtype=torch.float32)  # difference in the source dtype, as the reference
 
 
