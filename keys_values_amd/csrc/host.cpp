@@ -31,7 +31,7 @@ namespace {
 #define KVX_HOST_SYMBOLS(X)                                                                                                 \
   X(kvx_last_error) X(kvx_sdpa_prefill) X(kvx_sdpa_prefill_workspace_bytes) X(kvx_score_sum) X(kvx_sdpa_prefill_weights)     \
   X(kvx_sdpa_decode) X(kvx_sdpa_decode_workspace_bytes) X(kvx_sdpa_decode_h2o) X(kvx_sdpa_decode_h2o_workspace_bytes)        \
-  X(kvx_quantize_blocks) X(kvx_dequantize_blocks) X(kvx_quantize_rows_typed) X(kvx_dequantize_rows_typed) X(kvx_cache_write) \
+  X(kvx_quantize_blocks) X(kvx_dequantize_blocks) X(kvx_dequantize_rows_typed) X(kvx_cache_write) \
   X(kvx_h2o_update_select) X(kvx_h2o_workspace_bytes) X(kvx_rmsnorm_rows) X(kvx_add_rmsnorm_rows) X(kvx_swiglu_rows)         \
   X(kvx_qk_norm_rope)
 
@@ -644,19 +644,30 @@ PyObject* cache_decode_step(PyObject* const* args, Py_ssize_t n) {
 
 // ---- quantiser --------------------------------------------------------------------------------------------------------------
 
+// x, or a copy of it that the block kernels can address: rows 16-byte aligned, strides multiples of 8 and, for one block
+// per row, the (batch, head) axes collapsible into one
+at::Tensor block_view(const at::Tensor& x, bool over_heads) {
+  bool ok = x.stride(3) == 1 && (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0;
+  for (int i = 0; i < 3; ++i) ok = ok && x.stride(i) % 8 == 0;
+  if (!over_heads && x.size(0) > 1) ok = ok && x.stride(0) == x.size(1) * x.stride(1);
+  return ok ? x : x.contiguous();
+}
+
 // quantize_blocks(x, start, codes, scales, zero_points, over_heads, bits) and dequantize_blocks: x (B, Hkv, num, D) of
 // the source type, a block per row or, over_heads, per token over all heads; slots start .. of the buffers (first, L,
 // final), (first, L), (first, L)
 PyObject* blocks_call(PyObject* const* args, Py_ssize_t n, bool quantize) {
   require_args(n, 7, "quantize_blocks");
-  const at::Tensor &x = tensor(args[0], "x"), &codes = tensor(args[2], "codes"), &scale = tensor(args[3], "scales"), &zp = tensor(args[4], "zero_points");
+  const at::Tensor &given = tensor(args[0], "x"), &codes = tensor(args[2], "codes"), &scale = tensor(args[3], "scales"), &zp = tensor(args[4], "zero_points");
   const int64_t start = integer(args[1]);
-  require_gpu(x);
+  const bool over_heads = truth(args[5]);
+  require_gpu(given);
   const Launch L(codes);
+  const at::Tensor x = quantize ? block_view(given, over_heads) : given;  // dequantised rows: always contiguous
   kvx_block_quant_args a{};
   const int64_t b = x.size(0), hkv = x.size(1), num = x.size(2), d = x.size(3);
   a.x = x.data_ptr();
-  if (truth(args[5])) {
+  if (over_heads) {
     a.n_outer = (int32_t)b;
     a.n_inner = (int32_t)num;
     a.nseg = (int32_t)hkv;
@@ -684,17 +695,7 @@ PyObject* blocks_call(PyObject* const* args, Py_ssize_t n, bool quantize) {
 PyObject* quantize_blocks(PyObject* const* args, Py_ssize_t n) { return blocks_call(args, n, true); }
 PyObject* dequantize_blocks(PyObject* const* args, Py_ssize_t n) { return blocks_call(args, n, false); }
 
-// quantize_rows(rows, codes, scales, zero_points, bits), dequantize_rows(codes, scales, zero_points, bits, out): everything
-// contiguous, rows of D = out's / rows' last axis
-PyObject* quantize_rows(PyObject* const* args, Py_ssize_t n) {
-  require_args(n, 5, "quantize_rows");
-  const at::Tensor &x = tensor(args[0], "rows"), &codes = tensor(args[1], "codes"), &scale = tensor(args[2], "scales"), &zp = tensor(args[3], "zero_points");
-  const Launch L(codes);
-  const int64_t d = x.size(-1);
-  check(lib.kvx_quantize_rows_typed(x.data_ptr(), d, x.numel() / d, (int32_t)d, (int32_t)integer(args[4]), elem_dtype(x.scalar_type()),
-                                    (uint8_t*)codes.data_ptr(), (float*)scale.data_ptr(), (int32_t*)zp.data_ptr(), L.stream));
-  Py_RETURN_NONE;
-}
+// dequantize_rows(codes, scales, zero_points, bits, out): everything contiguous, rows of out's last axis
 PyObject* dequantize_rows(PyObject* const* args, Py_ssize_t n) {
   require_args(n, 5, "dequantize_rows");
   const at::Tensor &codes = tensor(args[0], "codes"), &scale = tensor(args[1], "scales"), &zp = tensor(args[2], "zero_points"), &out = tensor(args[4], "out");
@@ -828,7 +829,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyMethodDef methods[] = {
     {"bind", (PyCFunction)(void (*)(void))entry<bind, false>, METH_FASTCALL, nullptr},
     METHOD(prefill), METHOD(score_sum), METHOD(decode), METHOD(check_qkv), METHOD(cache_write), METHOD(cache_update), METHOD(cache_decode_step),
-    METHOD(quantize_blocks), METHOD(dequantize_blocks), METHOD(quantize_rows), METHOD(dequantize_rows), METHOD(rmsnorm), METHOD(add_rmsnorm),
+    METHOD(quantize_blocks), METHOD(dequantize_blocks), METHOD(dequantize_rows), METHOD(rmsnorm), METHOD(add_rmsnorm),
     METHOD(swiglu), METHOD(qk_norm_rope), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", "Native host path of the kernels (see csrc/host.cpp).", -1, methods};
 

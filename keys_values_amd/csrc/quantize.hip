@@ -1,4 +1,4 @@
-// Affine 8-bit row quantiser / dequantiser and the cache-slot write for gfx950 (HBM-bound byte work).
+// Affine 8-bit and 4-bit quantiser / dequantiser and the cache-slot write for gfx950 (HBM-bound byte work).
 //
 // Reference behaviour: keys_values/kvcache/quantize/pytorch.py:100-139,312-355 (quantise),
 // :143-154,411-478 (dequantise); keys_values/kvcache/attn_weights.py:305-316,679-681 and
@@ -51,8 +51,9 @@ template <int LPR>
 __device__ __forceinline__ bool row_any(bool bad) {
   const unsigned long long m = __ballot(bad);
   if (m == 0) return false;
+  if constexpr (LPR == 64) return true;
   const int first = (int)(__lane_id() & ~(unsigned)(LPR - 1));
-  return ((m >> first) & ((1ull << LPR) - 1ull)) != 0;
+  return ((m >> first) & (~0ull >> (64 - LPR))) != 0;
 }
 
 // Codes of 4 values packed into a dword, byte e = clamp(rint(x[e] * inv) + zf, 0, 255). The sum is an
@@ -159,10 +160,27 @@ __device__ __forceinline__ u32x2_t quantize8(u32x4_t raw, float& scale, int32_t&
   return out;
 }
 
+// Where the rows of a call lie: `n_outer` runs of `rows` rows each. A contiguous store is one run; a range of slots of a
+// store is one run per (batch, head). A launch takes the runs along blockIdx.y.
+struct RowRuns {
+  uint16_t* x;
+  int64_t x_row_stride, x_run_stride;  // elements
+  uint8_t* codes;
+  int64_t codes_run_stride;            // bytes; the rows of a run are adjacent
+  float* scale;
+  int32_t* zp;
+  int64_t state_run_stride;            // elements
+  int64_t rows;
+  int n_outer;
+};
+
 template <int D, bool F16>
-__global__ __launch_bounds__(NTHREADS) void quantize_rows_kernel(const uint16_t* __restrict__ x, int64_t x_row_stride,
-                                                                 int64_t rows, uint8_t* __restrict__ codes,
-                                                                 float* __restrict__ scale, int32_t* __restrict__ zp) {
+__global__ __launch_bounds__(NTHREADS) void quantize_rows_kernel(const RowRuns a) {
+  const int64_t rows = a.rows, x_row_stride = a.x_row_stride;
+  const uint16_t* __restrict__ x = a.x + blockIdx.y * a.x_run_stride;
+  uint8_t* __restrict__ codes = a.codes + blockIdx.y * a.codes_run_stride;
+  float* __restrict__ scale = a.scale + blockIdx.y * a.state_run_stride;
+  int32_t* __restrict__ zp = a.zp + blockIdx.y * a.state_run_stride;
   constexpr int LPR = D / 8;
   constexpr int RPB = NTHREADS / LPR;  // rows per block per step
   const int col = threadIdx.x % LPR;
@@ -191,10 +209,12 @@ __global__ __launch_bounds__(NTHREADS) void quantize_rows_kernel(const uint16_t*
 }
 
 template <int D, bool F16>
-__global__ __launch_bounds__(NTHREADS) void dequantize_rows_kernel(const uint8_t* __restrict__ codes,
-                                                                   const float* __restrict__ scale,
-                                                                   const int32_t* __restrict__ zp, int64_t rows,
-                                                                   uint16_t* __restrict__ out, int64_t out_row_stride) {
+__global__ __launch_bounds__(NTHREADS) void dequantize_rows_kernel(const RowRuns a) {
+  const int64_t rows = a.rows, out_row_stride = a.x_row_stride;
+  const uint8_t* __restrict__ codes = a.codes + blockIdx.y * a.codes_run_stride;
+  const float* __restrict__ scale = a.scale + blockIdx.y * a.state_run_stride;
+  const int32_t* __restrict__ zp = a.zp + blockIdx.y * a.state_run_stride;
+  uint16_t* __restrict__ out = a.x + blockIdx.y * a.x_run_stride;
   constexpr int LPR = D / 8;
   constexpr int RPB = NTHREADS / LPR;
   const int col = threadIdx.x % LPR;
@@ -252,9 +272,12 @@ __device__ __forceinline__ u32x2_t quantize4(u32x4_t raw, float& scale, int32_t&
 // Element d shares its byte with element d + D/2 (high nibble = first half of the row): the lanes of
 // the first half fetch their partner's codes from the lane LPR/2 away and store 8 packed bytes.
 template <int D, bool F16>
-__global__ __launch_bounds__(NTHREADS) void quantize_rows4_kernel(const uint16_t* __restrict__ x, int64_t x_row_stride, int64_t rows,
-                                                                  uint8_t* __restrict__ codes, float* __restrict__ scale,
-                                                                  int32_t* __restrict__ zp) {
+__global__ __launch_bounds__(NTHREADS) void quantize_rows4_kernel(const RowRuns a) {
+  const int64_t rows = a.rows, x_row_stride = a.x_row_stride;
+  const uint16_t* __restrict__ x = a.x + blockIdx.y * a.x_run_stride;
+  uint8_t* __restrict__ codes = a.codes + blockIdx.y * a.codes_run_stride;
+  float* __restrict__ scale = a.scale + blockIdx.y * a.state_run_stride;
+  int32_t* __restrict__ zp = a.zp + blockIdx.y * a.state_run_stride;
   constexpr int LPR = D / 8;
   constexpr int RPB = NTHREADS / LPR;
   const int col = threadIdx.x % LPR;
@@ -282,42 +305,52 @@ __global__ __launch_bounds__(NTHREADS) void quantize_rows4_kernel(const uint16_t
   }
 }
 
-// One lane per 8 packed bytes: the high nibbles are elements col*8.., the low nibbles D/2 + col*8...
+// One lane per 8 packed bytes of ROWS_PER_THREAD rows: the high nibbles are elements col*8.., the low nibbles D/2 + col*8...
 template <int D, bool F16>
-__global__ __launch_bounds__(NTHREADS) void dequantize_rows4_kernel(const uint8_t* __restrict__ codes, const float* __restrict__ scale,
-                                                                    const int32_t* __restrict__ zp, int64_t rows,
-                                                                    uint16_t* __restrict__ out, int64_t out_row_stride) {
+__global__ __launch_bounds__(NTHREADS) void dequantize_rows4_kernel(const RowRuns a) {
+  const int64_t rows = a.rows, out_row_stride = a.x_row_stride;
+  const uint8_t* __restrict__ codes = a.codes + blockIdx.y * a.codes_run_stride;
+  const float* __restrict__ scale = a.scale + blockIdx.y * a.state_run_stride;
+  const int32_t* __restrict__ zp = a.zp + blockIdx.y * a.state_run_stride;
+  uint16_t* __restrict__ out = a.x + blockIdx.y * a.x_run_stride;
   constexpr int LPR = D / 16;
-  const int64_t gid = (int64_t)blockIdx.x * NTHREADS + threadIdx.x;
-  const int col = (int)(gid % LPR);
-  const int64_t r = gid / LPR;
-  if (r >= rows) return;
-  const u32x2_t c = *(const u32x2_t*)(codes + r * (D / 2) + col * 8);
-  const float s = scale[r];
-  const int32_t z = zp[r];
-  u32x4_t hi, lo;
+  constexpr int RPB = NTHREADS / LPR;
+  const int col = threadIdx.x % LPR;
+  const int64_t row0 = (int64_t)blockIdx.x * (RPB * ROWS_PER_THREAD) + threadIdx.x / LPR;
+  u32x2_t c[ROWS_PER_THREAD];
+  float s[ROWS_PER_THREAD];
+  int32_t z[ROWS_PER_THREAD];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const uint32_t w = c[e >> 1] >> ((e & 1) * 16);
-    hi[e] = dequant_pair<F16>((w >> 4) & 0xf, (w >> 12) & 0xf, z, s);
-    lo[e] = dequant_pair<F16>(w & 0xf, (w >> 8) & 0xf, z, s);
+  for (int i = 0; i < ROWS_PER_THREAD; ++i) {
+    const int64_t r = row0 + (int64_t)i * RPB;
+    const bool ok = r < rows;
+    c[i] = ok ? *(const u32x2_t*)(codes + r * (D / 2) + col * 8) : u32x2_t{0, 0};
+    s[i] = ok ? scale[r] : 0.0f;
+    z[i] = ok ? zp[r] : 0;
   }
-  *(u32x4_t*)(out + r * out_row_stride + col * 8) = hi;
-  *(u32x4_t*)(out + r * out_row_stride + D / 2 + col * 8) = lo;
+#pragma unroll
+  for (int i = 0; i < ROWS_PER_THREAD; ++i) {
+    const int64_t r = row0 + (int64_t)i * RPB;
+    if (r >= rows) continue;
+    u32x4_t hi, lo;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t w = c[i][e >> 1] >> ((e & 1) * 16);
+      hi[e] = dequant_pair<F16>((w >> 4) & 0xf, (w >> 12) & 0xf, z[i], s[i]);
+      lo[e] = dequant_pair<F16>(w & 0xf, (w >> 8) & 0xf, z[i], s[i]);
+    }
+    *(u32x4_t*)(out + r * out_row_stride + col * 8) = hi;
+    *(u32x4_t*)(out + r * out_row_stride + D / 2 + col * 8) = lo;
+  }
 }
 
-// ---- general blocks (several segments per block, 8 or 4 bits): one wavefront per block ------------
-
-__device__ __forceinline__ float wave_min(float v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = fminf(v, __shfl_xor(v, off, 64));
-  return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
-}
+// ---- general blocks (several segments per block, 8 or 4 bits) -------------------------------------------------------
+//
+// A block of n chunks of 8 values (n is even: D is a multiple of 16) is held by LPB lanes, lane l taking the chunk pairs
+// (l + LPB i, l + LPB i + n / 2), i < NP: the two halves of the block are what shares the bytes of the 4-bit store, and
+// two 16-byte loads a pair keep enough bytes in flight. LPB is the power of two from 8 to 64 that n / 2 needs, so short
+// blocks share a wavefront; longer ones take up to NP = 8 pairs a lane. The values stay in registers between the
+// extremes and the codes: HBM sees every byte once.
 
 template <bool F16>
 __device__ __forceinline__ u32x2_t codes_of_chunk(u32x4_t raw, float inv, float zf, float qmax) {
@@ -329,88 +362,113 @@ __device__ __forceinline__ u32x2_t codes_of_chunk(u32x4_t raw, float inv, float 
   return out;
 }
 
-template <int BITS, bool F16>
-__global__ __launch_bounds__(NTHREADS) void quantize_blocks_kernel(const kvx_block_quant_args a) {
-  const int lane = threadIdx.x & 63;
-  const int64_t blk = (int64_t)blockIdx.x * (NTHREADS / 64) + (threadIdx.x >> 6);
-  if (blk >= (int64_t)a.n_outer * a.n_inner) return;  // a whole wavefront at a time
-  const int64_t outer = blk / a.n_inner, inner = blk % a.n_inner;
-  const uint16_t* base = (const uint16_t*)a.x + outer * a.x_stride_outer + inner * a.x_stride_inner;
-  const int cps = a.D / 8;  // chunks of 8 values per segment
-  const int nchunks = a.nseg * cps;
-  auto chunk = [&](int c) { return *(const u32x4_t*)(base + (int64_t)(c / cps) * a.x_stride_seg + (c % cps) * 8); };
-  float mn = INFINITY, mx = -INFINITY, bad = 0.0f;
-  for (int c = lane; c < nchunks; c += 64) {
-    const u32x4_t raw = chunk(c);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      mn = fminf(mn, fminf(elem_lo<F16>(raw[e]), elem_hi<F16>(raw[e])));
-      mx = fmaxf(mx, fmaxf(elem_lo<F16>(raw[e]), elem_hi<F16>(raw[e])));
-      bad = __builtin_isunordered(elem_lo<F16>(raw[e]), elem_hi<F16>(raw[e])) ? 1.0f : bad;
-    }
+// Addresses of this lane's chunks; cps = chunks per segment, magic = ceil(2^21 / cps): c / cps == c magic >> 21 for c < 1024.
+template <int LPB, int NP>
+struct BlockLane {
+  bool live;
+  int64_t outer, inner;
+  uint16_t* base;
+  int half, cps, sub;
+  uint32_t magic;
+  int64_t seg;
+  __device__ __forceinline__ BlockLane(const kvx_block_quant_args& a, uint32_t magic_) : magic(magic_) {
+    const int64_t blk = ((int64_t)blockIdx.x * NTHREADS + threadIdx.x) / LPB;
+    live = blk < (int64_t)a.n_outer * a.n_inner;
+    const int64_t b = live ? blk : 0;
+    outer = b / a.n_inner;
+    inner = b % a.n_inner;
+    base = (uint16_t*)a.x + outer * a.x_stride_outer + inner * a.x_stride_inner;
+    cps = a.D / 8;
+    half = a.nseg * cps / 2;
+    sub = threadIdx.x % LPB;
+    seg = a.x_stride_seg;
   }
-  mn = wave_min(mn);
-  mx = wave_max(mx);
-  if (wave_max(bad) != 0.0f) mn = mx = __builtin_nanf("");  // as torch.aminmax: a NaN in the block is the block's extreme
+  __device__ __forceinline__ int pair(int i) const { return sub + LPB * i; }
+  __device__ __forceinline__ u32x4_t* chunk(int c) const {
+    const int s = (int)(((uint32_t)c * magic) >> 21);
+    return (u32x4_t*)(base + s * seg + (c - s * cps) * 8);
+  }
+};
+
+template <int BITS, bool F16, int LPB, int NP>
+__global__ __launch_bounds__(NTHREADS) void quantize_blocks_kernel(const kvx_block_quant_args a, const uint32_t magic) {
+  const BlockLane<LPB, NP> bl(a, magic);
+  u32x4_t raw[NP][2];
+  float mn = INFINITY, mx = -INFINITY;
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      raw[i][h] = bl.live && bl.pair(i) < bl.half ? __builtin_nontemporal_load(bl.chunk(bl.pair(i) + h * bl.half)) : u32x4_t{0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    if (bl.pair(i) < bl.half) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lo = elem_lo<F16>(raw[i][h][e]), hi = elem_hi<F16>(raw[i][h][e]);
+          mn = fminf(mn, fminf(lo, hi));
+          mx = fmaxf(mx, fmaxf(lo, hi));
+          bad |= __builtin_isunordered(lo, hi);
+        }
+    }
+#pragma unroll
+  for (int off = LPB / 2; off >= 1; off >>= 1) {
+    mn = fminf(mn, __shfl_xor(mn, off, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+  }
+  if (row_any<LPB>(bad)) mn = mx = __builtin_nanf("");  // as torch.aminmax: a NaN in the block is the block's extreme
+  if (!bl.live) return;
   constexpr float qmax = BITS == 8 ? 255.0f : 15.0f;
   float s;
   int32_t z;
   quant_params(mn, mx, s, z, qmax);
   const float inv = 1.0f / s, zf = (float)z;
-  uint8_t* out = a.codes + outer * a.codes_stride_outer + inner * ((int64_t)nchunks * BITS);  // nchunks * 8 values * BITS / 8 bytes
-  if constexpr (BITS == 8) {
-    for (int c = lane; c < nchunks; c += 64) *(u32x2_t*)(out + c * 8) = codes_of_chunk<F16>(chunk(c), inv, zf, qmax);
-  } else {
-    const int half = nchunks / 2;
-    for (int c = lane; c < half; c += 64) {
-      const u32x2_t hi = codes_of_chunk<F16>(chunk(c), inv, zf, qmax), lo = codes_of_chunk<F16>(chunk(c + half), inv, zf, qmax);
-      *(u32x2_t*)(out + c * 8) = u32x2_t{(hi[0] << 4) | lo[0], (hi[1] << 4) | lo[1]};
+  uint8_t* out = a.codes + bl.outer * a.codes_stride_outer + bl.inner * ((int64_t)bl.half * 2 * BITS);  // 8 values a chunk, BITS / 8 bytes each
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    if (bl.pair(i) < bl.half) {
+      const u32x2_t c0 = codes_of_chunk<F16>(raw[i][0], inv, zf, qmax), c1 = codes_of_chunk<F16>(raw[i][1], inv, zf, qmax);
+      if constexpr (BITS == 8) {
+        *(u32x2_t*)(out + bl.pair(i) * 8) = c0;
+        *(u32x2_t*)(out + (bl.pair(i) + bl.half) * 8) = c1;
+      } else {
+        *(u32x2_t*)(out + bl.pair(i) * 8) = u32x2_t{(c0[0] << 4) | c1[0], (c0[1] << 4) | c1[1]};
+      }
     }
-  }
-  if (lane == 0) {
-    a.scale[outer * a.state_stride_outer + inner] = s;
-    a.zp[outer * a.state_stride_outer + inner] = z;
+  if (bl.sub == 0) {
+    a.scale[bl.outer * a.state_stride_outer + bl.inner] = s;
+    a.zp[bl.outer * a.state_stride_outer + bl.inner] = z;
   }
 }
 
-template <int BITS, bool F16>
-__global__ __launch_bounds__(NTHREADS) void dequantize_blocks_kernel(const kvx_block_quant_args a) {
-  const int lane = threadIdx.x & 63;
-  const int64_t blk = (int64_t)blockIdx.x * (NTHREADS / 64) + (threadIdx.x >> 6);
-  if (blk >= (int64_t)a.n_outer * a.n_inner) return;
-  const int64_t outer = blk / a.n_inner, inner = blk % a.n_inner;
-  uint16_t* base = (uint16_t*)a.x + outer * a.x_stride_outer + inner * a.x_stride_inner;
-  const int cps = a.D / 8;
-  const int nchunks = a.nseg * cps;
-  auto chunk_ptr = [&](int c) { return (u32x4_t*)(base + (int64_t)(c / cps) * a.x_stride_seg + (c % cps) * 8); };
-  const float s = a.scale[outer * a.state_stride_outer + inner];
-  const int32_t z = a.zp[outer * a.state_stride_outer + inner];
-  const uint8_t* in = a.codes + outer * a.codes_stride_outer + inner * ((int64_t)nchunks * BITS);
-  if constexpr (BITS == 8) {
-    for (int c = lane; c < nchunks; c += 64) {
-      const u32x2_t cc = *(const u32x2_t*)(in + c * 8);
-      u32x4_t o;
-      o[0] = dequant_pair<F16>(cc[0] & 0xff, (cc[0] >> 8) & 0xff, z, s);
-      o[1] = dequant_pair<F16>((cc[0] >> 16) & 0xff, cc[0] >> 24, z, s);
-      o[2] = dequant_pair<F16>(cc[1] & 0xff, (cc[1] >> 8) & 0xff, z, s);
-      o[3] = dequant_pair<F16>((cc[1] >> 16) & 0xff, cc[1] >> 24, z, s);
-      *chunk_ptr(c) = o;
-    }
-  } else {
-    const int half = nchunks / 2;
-    for (int c = lane; c < half; c += 64) {
-      const u32x2_t cc = *(const u32x2_t*)(in + c * 8);
-      u32x4_t hi, lo;
+template <int BITS, bool F16, int LPB, int NP>
+__global__ __launch_bounds__(NTHREADS) void dequantize_blocks_kernel(const kvx_block_quant_args a, const uint32_t magic) {
+  const BlockLane<LPB, NP> bl(a, magic);
+  if (!bl.live) return;
+  const float s = a.scale[bl.outer * a.state_stride_outer + bl.inner];
+  const int32_t z = a.zp[bl.outer * a.state_stride_outer + bl.inner];
+  const uint8_t* in = a.codes + bl.outer * a.codes_stride_outer + bl.inner * ((int64_t)bl.half * 2 * BITS);
+  u32x2_t c[NP][2];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t w = cc[e >> 1] >> ((e & 1) * 16);
-        hi[e] = dequant_pair<F16>((w >> 4) & 0xf, (w >> 12) & 0xf, z, s);
-        lo[e] = dequant_pair<F16>(w & 0xf, (w >> 8) & 0xf, z, s);
-      }
-      *chunk_ptr(c) = hi;
-      *chunk_ptr(c + half) = lo;
-    }
+  for (int i = 0; i < NP; ++i) {
+    const bool ok = bl.pair(i) < bl.half;
+    c[i][0] = ok ? *(const u32x2_t*)(in + bl.pair(i) * 8) : u32x2_t{0, 0};
+    if constexpr (BITS == 8) c[i][1] = ok ? *(const u32x2_t*)(in + (bl.pair(i) + bl.half) * 8) : u32x2_t{0, 0};
   }
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+    if (bl.pair(i) < bl.half) {
+      u32x2_t c0 = c[i][0], c1 = c[i][1];
+      if constexpr (BITS == 4) {
+        c1 = u4_codes(c0, 0);
+        c0 = u4_codes(c0, 4);
+      }
+      *bl.chunk(bl.pair(i)) = dequant_words<F16>(c0[0], c0[1], z, s);
+      *bl.chunk(bl.pair(i) + bl.half) = dequant_words<F16>(c1[0], c1[1], z, s);
+    }
 }
 
 // Sum over the LPR adjacent lanes holding one row; every lane gets the result.
@@ -583,78 +641,86 @@ __global__ __launch_bounds__(NTHREADS) void cache_write_kernel(const kvx_cache_w
 
 // D in {64, 128, 256}, bits in {8, 4}, f16: the rows are float16 (else bfloat16)
 template <int D, bool F16>
-int launch_quantize_rows_t(const void* x, int64_t x_row_stride, int64_t rows, int bits, uint8_t* codes, float* scale, int32_t* zp, hipStream_t st) {
-  const int rpb = (NTHREADS / (D / 8)) * ROWS_PER_THREAD;
-  const unsigned grid = (unsigned)((rows + rpb - 1) / rpb);
-  if (bits == 8) hipLaunchKernelGGL((quantize_rows_kernel<D, F16>), dim3(grid), dim3(NTHREADS), 0, st, (const uint16_t*)x, x_row_stride, rows, codes, scale, zp);
-  else hipLaunchKernelGGL((quantize_rows4_kernel<D, F16>), dim3(grid), dim3(NTHREADS), 0, st, (const uint16_t*)x, x_row_stride, rows, codes, scale, zp);
-  KVX_HIP(hipGetLastError());
+int launch_rows_t(const RowRuns& a, int bits, bool quantize, hipStream_t st) {
+  const int lpr = bits == 4 && !quantize ? D / 16 : D / 8;
+  const int rpb = (NTHREADS / lpr) * ROWS_PER_THREAD;
+  RowRuns r = a;
+  for (int done = 0; done < a.n_outer; done += 65535) {  // runs along a grid dimension of 16 bits
+    const dim3 grid((unsigned)((a.rows + rpb - 1) / rpb), (unsigned)min(a.n_outer - done, 65535));
+    if (quantize && bits == 8) hipLaunchKernelGGL((quantize_rows_kernel<D, F16>), grid, dim3(NTHREADS), 0, st, r);
+    else if (quantize) hipLaunchKernelGGL((quantize_rows4_kernel<D, F16>), grid, dim3(NTHREADS), 0, st, r);
+    else if (bits == 8) hipLaunchKernelGGL((dequantize_rows_kernel<D, F16>), grid, dim3(NTHREADS), 0, st, r);
+    else hipLaunchKernelGGL((dequantize_rows4_kernel<D, F16>), grid, dim3(NTHREADS), 0, st, r);
+    KVX_HIP(hipGetLastError());
+    r.x += 65535 * a.x_run_stride;
+    r.codes += 65535 * a.codes_run_stride;
+    r.scale += 65535 * a.state_run_stride;
+    r.zp += 65535 * a.state_run_stride;
+  }
   return KVX_OK;
+}
+
+static int launch_rows(const RowRuns& a, int D, int bits, bool f16, bool quantize, hipStream_t st) {
+  if (a.rows == 0 || a.n_outer == 0) return KVX_OK;
+  if (D == 256) return f16 ? launch_rows_t<256, true>(a, bits, quantize, st) : launch_rows_t<256, false>(a, bits, quantize, st);
+  if (D == 128) return f16 ? launch_rows_t<128, true>(a, bits, quantize, st) : launch_rows_t<128, false>(a, bits, quantize, st);
+  return f16 ? launch_rows_t<64, true>(a, bits, quantize, st) : launch_rows_t<64, false>(a, bits, quantize, st);
 }
 
 int launch_quantize_rows(const void* x, int64_t x_row_stride, int64_t rows, int D, int bits, bool f16, uint8_t* codes, float* scale,
                          int32_t* zp, hipStream_t st) {
-  if (rows == 0) return KVX_OK;
-  if (D == 256) return f16 ? launch_quantize_rows_t<256, true>(x, x_row_stride, rows, bits, codes, scale, zp, st)
-                           : launch_quantize_rows_t<256, false>(x, x_row_stride, rows, bits, codes, scale, zp, st);
-  if (D == 128) return f16 ? launch_quantize_rows_t<128, true>(x, x_row_stride, rows, bits, codes, scale, zp, st)
-                           : launch_quantize_rows_t<128, false>(x, x_row_stride, rows, bits, codes, scale, zp, st);
-  return f16 ? launch_quantize_rows_t<64, true>(x, x_row_stride, rows, bits, codes, scale, zp, st)
-             : launch_quantize_rows_t<64, false>(x, x_row_stride, rows, bits, codes, scale, zp, st);
-}
-
-template <int D, bool F16>
-int launch_dequantize_rows_t(const uint8_t* codes, const float* scale, const int32_t* zp, int64_t rows, int bits, void* out,
-                             int64_t out_row_stride, hipStream_t st) {
-  if (bits == 8) {
-    const int rpb = (NTHREADS / (D / 8)) * ROWS_PER_THREAD;
-    const unsigned grid = (unsigned)((rows + rpb - 1) / rpb);
-    hipLaunchKernelGGL((dequantize_rows_kernel<D, F16>), dim3(grid), dim3(NTHREADS), 0, st, codes, scale, zp, rows, (uint16_t*)out, out_row_stride);
-  } else {
-    const int64_t lanes = rows * (D / 16);
-    const unsigned grid = (unsigned)((lanes + NTHREADS - 1) / NTHREADS);
-    hipLaunchKernelGGL((dequantize_rows4_kernel<D, F16>), dim3(grid), dim3(NTHREADS), 0, st, codes, scale, zp, rows, (uint16_t*)out, out_row_stride);
-  }
-  KVX_HIP(hipGetLastError());
-  return KVX_OK;
+  return launch_rows(RowRuns{(uint16_t*)x, x_row_stride, 0, codes, 0, scale, zp, 0, rows, 1}, D, bits, f16, true, st);
 }
 
 int launch_dequantize_rows(const uint8_t* codes, const float* scale, const int32_t* zp, int64_t rows, int D, int bits, bool f16,
                            void* out, int64_t out_row_stride, hipStream_t st) {
-  if (rows == 0) return KVX_OK;
-  if (D == 256) return f16 ? launch_dequantize_rows_t<256, true>(codes, scale, zp, rows, bits, out, out_row_stride, st)
-                           : launch_dequantize_rows_t<256, false>(codes, scale, zp, rows, bits, out, out_row_stride, st);
-  if (D == 128) return f16 ? launch_dequantize_rows_t<128, true>(codes, scale, zp, rows, bits, out, out_row_stride, st)
-                           : launch_dequantize_rows_t<128, false>(codes, scale, zp, rows, bits, out, out_row_stride, st);
-  return f16 ? launch_dequantize_rows_t<64, true>(codes, scale, zp, rows, bits, out, out_row_stride, st)
-             : launch_dequantize_rows_t<64, false>(codes, scale, zp, rows, bits, out, out_row_stride, st);
+  return launch_rows(RowRuns{(uint16_t*)out, out_row_stride, 0, (uint8_t*)codes, 0, (float*)scale, (int32_t*)zp, 0, rows, 1}, D, bits, f16, false, st);
 }
 
-int launch_quantize_blocks(const kvx_block_quant_args& a, hipStream_t st) {
-  const int64_t blocks = (int64_t)a.n_outer * a.n_inner;
-  if (blocks == 0) return KVX_OK;
-  const unsigned grid = (unsigned)((blocks + NTHREADS / 64 - 1) / (NTHREADS / 64));
-  const bool f16 = a.elem_dtype == KVX_KV_F16;
-  if (a.bits == 8 && f16) hipLaunchKernelGGL((quantize_blocks_kernel<8, true>), dim3(grid), dim3(NTHREADS), 0, st, a);
-  else if (a.bits == 8) hipLaunchKernelGGL((quantize_blocks_kernel<8, false>), dim3(grid), dim3(NTHREADS), 0, st, a);
-  else if (f16) hipLaunchKernelGGL((quantize_blocks_kernel<4, true>), dim3(grid), dim3(NTHREADS), 0, st, a);
-  else hipLaunchKernelGGL((quantize_blocks_kernel<4, false>), dim3(grid), dim3(NTHREADS), 0, st, a);
+template <int BITS, bool F16, int LPB, int NP>
+int launch_blocks_t(const kvx_block_quant_args& a, bool quantize, hipStream_t st) {
+  const int64_t lanes = (int64_t)a.n_outer * a.n_inner * LPB;
+  const unsigned grid = (unsigned)((lanes + NTHREADS - 1) / NTHREADS);
+  const uint32_t cps = (uint32_t)a.D / 8, magic = ((1u << 21) + cps - 1) / cps;
+  if (quantize) hipLaunchKernelGGL((quantize_blocks_kernel<BITS, F16, LPB, NP>), dim3(grid), dim3(NTHREADS), 0, st, a, magic);
+  else hipLaunchKernelGGL((dequantize_blocks_kernel<BITS, F16, LPB, NP>), dim3(grid), dim3(NTHREADS), 0, st, a, magic);
   KVX_HIP(hipGetLastError());
   return KVX_OK;
 }
 
-int launch_dequantize_blocks(const kvx_block_quant_args& a, hipStream_t st) {
-  const int64_t blocks = (int64_t)a.n_outer * a.n_inner;
-  if (blocks == 0) return KVX_OK;
-  const unsigned grid = (unsigned)((blocks + NTHREADS / 64 - 1) / (NTHREADS / 64));
-  const bool f16 = a.elem_dtype == KVX_KV_F16;
-  if (a.bits == 8 && f16) hipLaunchKernelGGL((dequantize_blocks_kernel<8, true>), dim3(grid), dim3(NTHREADS), 0, st, a);
-  else if (a.bits == 8) hipLaunchKernelGGL((dequantize_blocks_kernel<8, false>), dim3(grid), dim3(NTHREADS), 0, st, a);
-  else if (f16) hipLaunchKernelGGL((dequantize_blocks_kernel<4, true>), dim3(grid), dim3(NTHREADS), 0, st, a);
-  else hipLaunchKernelGGL((dequantize_blocks_kernel<4, false>), dim3(grid), dim3(NTHREADS), 0, st, a);
-  KVX_HIP(hipGetLastError());
-  return KVX_OK;
+template <int BITS, bool F16>
+int launch_blocks_bits(const kvx_block_quant_args& a, bool quantize, hipStream_t st) {
+  const int half = a.nseg * a.D / 16;  // chunk pairs of a block, 1 .. 512
+  if (half <= 8) return launch_blocks_t<BITS, F16, 8, 1>(a, quantize, st);
+  if (half <= 16) return launch_blocks_t<BITS, F16, 16, 1>(a, quantize, st);
+  if (half <= 32) return launch_blocks_t<BITS, F16, 32, 1>(a, quantize, st);
+  if (half <= 64) return launch_blocks_t<BITS, F16, 64, 1>(a, quantize, st);
+  if (half <= 128) return launch_blocks_t<BITS, F16, 64, 2>(a, quantize, st);
+  if (half <= 256) return launch_blocks_t<BITS, F16, 64, 4>(a, quantize, st);
+  return launch_blocks_t<BITS, F16, 64, 8>(a, quantize, st);
 }
+
+// One segment of 64, 128 or 256 values is a row: the row kernels (four rows in flight a lane, the state's arithmetic
+// shared between them) serve a range of slots as one run per (batch, head), or as a single run where the runs are adjacent.
+// Measured, one (1, 8, 65536, 128) tensor of 8-bit codes to rows: 99 us with a wavefront per row, 33 us this way.
+static int launch_blocks(const kvx_block_quant_args& a, bool quantize, hipStream_t st) {
+  if (a.n_outer == 0 || a.n_inner == 0) return KVX_OK;
+  const bool f16 = a.elem_dtype == KVX_KV_F16;
+  const int64_t code_bytes = (int64_t)a.D * a.bits / 8;
+  if (a.nseg == 1 && (a.D == 64 || a.D == 128 || a.D == 256)) {
+    RowRuns r{(uint16_t*)a.x, a.x_stride_inner, a.x_stride_outer, a.codes, a.codes_stride_outer, a.scale, a.zp, a.state_stride_outer, a.n_inner, a.n_outer};
+    if (r.x_run_stride == r.rows * r.x_row_stride && r.codes_run_stride == r.rows * code_bytes && r.state_run_stride == r.rows) {
+      r.rows *= r.n_outer;
+      r.n_outer = 1;
+    }
+    return launch_rows(r, a.D, a.bits, f16, quantize, st);
+  }
+  if (a.bits == 8) return f16 ? launch_blocks_bits<8, true>(a, quantize, st) : launch_blocks_bits<8, false>(a, quantize, st);
+  return f16 ? launch_blocks_bits<4, true>(a, quantize, st) : launch_blocks_bits<4, false>(a, quantize, st);
+}
+
+int launch_quantize_blocks(const kvx_block_quant_args& a, hipStream_t st) { return launch_blocks(a, true, st); }
+int launch_dequantize_blocks(const kvx_block_quant_args& a, hipStream_t st) { return launch_blocks(a, false, st); }
 
 template <int D>
 int launch_cache_write_d(const kvx_cache_write_args& a, unsigned grid, hipStream_t st) {

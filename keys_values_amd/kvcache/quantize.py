@@ -95,14 +95,6 @@ class RowQuantizer:
 
     # -- quantise / dequantise -----------------------------------------------------------------------
 
-    def _kernel_view(self, x: torch.Tensor) -> torch.Tensor:
-        """A view (or copy) of x the block kernels can address: rows 16-byte aligned, strides multiples
-        of 8 and, for one block per row, the (batch, head) axes collapsible into one."""
-        ok = x.stride(-1) == 1 and x.data_ptr() % 16 == 0 and all(s % 8 == 0 for s in x.stride()[:3])
-        if ok and not self.blocks_over_heads and x.shape[0] > 1:
-            ok = x.stride(0) == x.shape[1] * x.stride(1)
-        return x if ok else x.contiguous()
-
     def quantize(self, start: int, end: int, values: torch.Tensor, block_idx: Optional[int] = None):
         """Quantise slots ``range(start, end)`` from ``values`` (B, Hkv, end - start, D)
         (keys_values/kvcache/quantize/pytorch.py:312-355)."""
@@ -118,12 +110,7 @@ class RowQuantizer:
             return
         _lib.require_gpu(values)
         values = values.to(self.source_dtype)
-        if not self.blocks_over_heads and d in (64, 128, 256) and num == length and values.is_contiguous():
-            # the whole store in one pass of the row kernels (16 or 8 lanes per row)
-            _lib.host().quantize_rows(values, self.quant_buffer, self.quant_scales, self.quant_zero_points, self.num_bits)
-            return
-        _lib.host().quantize_blocks(self._kernel_view(values), start, self.quant_buffer, self.quant_scales, self.quant_zero_points,
-                                    self.blocks_over_heads, self.num_bits)
+        _lib.host().quantize_blocks(values, start, self.quant_buffer, self.quant_scales, self.quant_zero_points, self.blocks_over_heads, self.num_bits)
 
     def dequantize(self, start: int, end: int, out: Optional[torch.Tensor] = None, block_idx: Optional[int] = None):
         """Dequantise slots ``range(start, end)`` to (B, Hkv, end - start, D) in the source dtype
@@ -151,7 +138,7 @@ class RowQuantizer:
         _lib.require_gpu(x)
         if x.ndim != 4 or x.shape[1] != self.shape[1] or x.shape[3] != self.shape[3]:
             raise ValueError(f"x.shape = {tuple(x.shape)}, must be (batch, {self.shape[1]}, n, {self.shape[3]})")
-        xs = self._kernel_view(x.to(self.source_dtype))
+        xs = x.to(self.source_dtype)
         b, hkv, n, d = xs.shape
         dev = xs.device
         host = _lib.host()

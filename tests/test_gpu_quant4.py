@@ -187,3 +187,38 @@ def test_attention_over_4bit_cache(kvx, gpu, B, Hq, Hkv, q_len, T, D):
     torch.cuda.synchronize()
     assert rel_err(out1.float().cpu().unsqueeze(2), o1_ref.float()) < 2e-2
     torch.testing.assert_close(w1.cpu(), w1_ref, rtol=1e-3, atol=1e-6)
+
+
+@pytest.mark.parametrize("num_bits", [8, 4])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape,blocks_over_heads,span", [
+    ((1, 1, 3, 16), False, (0, 3)),      # one pair of chunks a block
+    ((2, 3, 5, 80), True, (1, 5)),       # 15 pairs, segments of 10 chunks
+    ((1, 2, 7, 128), True, (0, 7)),      # 16 pairs: the last size of 16 lanes
+    ((1, 5, 9, 112), True, (2, 8)),      # 35 pairs on 64 lanes
+    ((1, 8, 3, 128), True, (0, 3)),      # 64 pairs: the last size of one pair a lane
+    ((2, 9, 3, 128), True, (0, 2)),      # 72 pairs: two a lane
+    ((1, 20, 3, 128), True, (0, 3)),     # 160 pairs: four a lane
+    ((1, 32, 2, 256), True, (0, 2)),     # 512 pairs: the longest block
+    ((2, 3, 37, 64), False, (5, 20)),    # rows of a range of slots: one run per (batch, head)
+    ((2, 3, 70, 128), False, (0, 69)),
+    ((1, 2, 33, 256), False, (1, 33)),
+])
+def test_block_sizes_and_slot_ranges_bit_exact(gpu, shape, blocks_over_heads, span, dtype, num_bits):
+    """Every split of a block over lanes, and ranges of slots of a row store, from a strided input, against the oracle:
+    codes, scales, zero points and dequantised values are defined to the bit. Slots outside the range stay as they are."""
+    B, Hkv, L, D = shape
+    lo, hi = span
+    gen = torch.Generator().manual_seed(D + L)
+    wide = (torch.randn(B, Hkv, L, 2 * D, generator=gen) * 3).to(dtype)  # the input is the first half of every row
+    x = wide[..., :D]
+    qz = RowQuantizer(shape, dtype, num_bits, blocks_over_heads, allocate_buffers=True, device=gpu)
+    qz.quant_buffer.fill_(9)
+    want = qz.quant_buffer.cpu()
+    qz.quantize(lo, hi, wide.to(gpu)[:, :, lo:hi, :D])
+    buf, s, z = O.quantize_store(x[:, :, lo:hi].contiguous(), num_bits, blocks_over_heads)
+    want[:, lo:hi] = buf
+    assert torch.equal(qz.quant_buffer.cpu(), want)
+    assert torch.equal(qz.quant_scales[:, lo:hi].cpu(), s) and torch.equal(qz.quant_zero_points[:, lo:hi].cpu(), z)
+    back = O.dequantize_store(buf, s, z, (B, Hkv, hi - lo, D), num_bits, blocks_over_heads, dtype)
+    assert torch.equal(qz.dequantize(lo, hi).cpu(), back)
