@@ -359,6 +359,15 @@ typedef struct kvx_h2o_args {
 int kvx_h2o_update_select(const kvx_h2o_args* args, void* stream);
 size_t kvx_h2o_workspace_bytes(const kvx_h2o_args* args);
 
+/* One new token into a full cache, the whole step (DefaultKVCache.forward, keys_values/kvcache/base.py:554-595):
+ * kvx_cache_write of `w` (w->num == 1), attention of the token over all slots, then the score update and the choice of one
+ * slot of `h` (h->k == 1; h->w and h->workspace are ignored), every policy variant included. Same results as the separate
+ * calls; two launches, three with q_errors: the slot write also clears the counters by which the splits of the attention
+ * kernel find out who is last, and the score-sums never leave the chip. args->workspace from
+ * kvx_h2o_decode_step_workspace_bytes; args->w (the score-sums) and args->lse optional. */
+int kvx_h2o_decode_step(const kvx_cache_write_args* w, const kvx_sdpa_args* args, const kvx_h2o_args* h, void* stream);
+size_t kvx_h2o_decode_step_workspace_bytes(const kvx_sdpa_args* args, const kvx_h2o_args* h);
+
 /* kvx_h2o_update_select for callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc). It has no counterpart in the reference. Same
  * arguments, same kernels, same results; args->workspace and args->workspace_bytes are ignored: the

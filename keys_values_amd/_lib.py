@@ -117,6 +117,8 @@ SYMBOLS = {
     "kvx_dequantize_blocks": (ctypes.c_int, [POINTER(BlockQuantArgs), c_void_p]),
     "kvx_cache_write": (ctypes.c_int, [POINTER(CacheWriteArgs), c_void_p]),
     "kvx_h2o_update_select": (ctypes.c_int, [POINTER(H2OArgs), c_void_p]),
+    "kvx_h2o_decode_step": (ctypes.c_int, [POINTER(CacheWriteArgs), POINTER(SdpaArgs), POINTER(H2OArgs), c_void_p]),
+    "kvx_h2o_decode_step_workspace_bytes": (c_size_t, [POINTER(SdpaArgs), POINTER(H2OArgs)]),
     "kvx_h2o_workspace_bytes": (c_size_t, [POINTER(H2OArgs)]),
     "kvx_h2o_update_select_static": (ctypes.c_int, [POINTER(H2OArgs), c_void_p]),
     "kvx_rmsnorm_rows": (ctypes.c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64, c_int32, ctypes.c_float, c_void_p]),

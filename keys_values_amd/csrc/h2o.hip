@@ -70,14 +70,15 @@ __device__ __forceinline__ Modify load_modify(const kvx_h2o_args& a, const float
   return m;
 }
 
+__device__ __forceinline__ float combined_value(float v, float qerr, const Modify& m) {
+  const float s = (v - m.smin) / m.sden;
+  const float q = (qerr - m.qmin) / m.qden;
+  return __fadd_rn(__fadd_rn(__fmul_rn(m.c, s), __fmul_rn(m.c2, q)), m.c3);
+}
+
 __device__ __forceinline__ float select_value(float score, const kvx_h2o_args& a, const int32_t* tp_row, int idx, const Modify& m) {
-  float v = residency_value(score, a, tp_row, idx);
-  if (m.qe) {
-    const float s = (v - m.smin) / m.sden;
-    const float q = (m.qe[idx] - m.qmin) / m.qden;
-    v = __fadd_rn(__fadd_rn(__fmul_rn(m.c, s), __fmul_rn(m.c2, q)), m.c3);
-  }
-  return v;
+  const float v = residency_value(score, a, tp_row, idx);
+  return m.qe ? combined_value(v, m.qe[idx], m) : v;
 }
 
 // ---- policy variants: the accumulation pass ---------------------------------------------------
@@ -230,6 +231,81 @@ __global__ __launch_bounds__(256) void update_argmin_kernel(const kvx_h2o_args a
 __global__ void argmin_finish_kernel(const unsigned long long* best, int32_t* next_index, int rows) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < rows) next_index[i] = (int32_t)(best[i] & 0xffffffffull);
+}
+
+// ---- k == 1 of a single-token step with the Q-Hitter combination ------------------------------
+//
+// The scores are up to date and their extremes (and those of the errors) lie in `per_row` records a row; what is left is
+// one pass over scores and errors. Workgroups of SEL_ONE slots; the last one of a row (counted in a word the caller zeroed)
+// publishes the row's slot. One launch instead of four (statistics, reset, minimum, publication).
+constexpr int SEL_ONE = 8 * SEL_THREADS;
+
+__global__ __launch_bounds__(SEL_THREADS) void select_one_kernel(const kvx_h2o_args a, const float* stats, int per_row, uint32_t* counters,
+                                                                 unsigned long long* part) {
+  __shared__ float red[SEL_THREADS / 64];
+  __shared__ unsigned long long wbest[SEL_THREADS / 64];
+  __shared__ uint32_t last;
+  const int tid = threadIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
+  float v4[4] = {INFINITY, -INFINITY, INFINITY, -INFINITY};
+  const float* st = stats + (int64_t)b * a.Hkv * per_row * 4;
+  for (int i = tid; i < a.Hkv * per_row; i += SEL_THREADS) {
+    const f32x4_t s = *(const f32x4_t*)(st + i * 4);
+    v4[0] = fminf(v4[0], s[0]);
+    v4[1] = fmaxf(v4[1], s[1]);
+    v4[2] = fminf(v4[2], s[2]);
+    v4[3] = fmaxf(v4[3], s[3]);
+  }
+  const int64_t off = b * a.sc_stride_b + hh * a.sc_stride_h;
+  const float *sc = a.scores + off, *qe = a.q_errors + off;
+  const int32_t* tpr = a.token_pos ? a.token_pos + b * a.tp_stride_b + hh * a.tp_stride_h : nullptr;
+  const int base = blockIdx.x * SEL_ONE + tid;
+  float s8[8], q8[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int k = min(base + i * SEL_THREADS, a.limit - 1);
+    s8[i] = sc[k];
+    q8[i] = qe[k];
+  }
+  auto mn = [](float x, float y) { return fminf(x, y); };
+  auto mx = [](float x, float y) { return fmaxf(x, y); };
+  Modify m;
+  m.qe = qe;
+  m.smin = block_reduce(v4[0], red, mn);
+  m.sden = block_reduce(v4[1], red, mx) - m.smin;
+  m.qmin = block_reduce(v4[2], red, mn);
+  m.qden = block_reduce(v4[3], red, mx) - m.qmin;
+  m.c = (float)a.combination;
+  m.c2 = (float)((a.combination - 1.0) / 2.0);
+  m.c3 = (float)(1.0 - a.combination);
+  unsigned long long mine = ~0ull;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int k = base + i * SEL_THREADS;
+    if (k >= a.limit) break;
+    const unsigned long long key = ((unsigned long long)ordered_bits(combined_value(residency_value(s8[i], a, tpr, k), q8[i], m)) << 32) | (unsigned)k;
+    mine = key < mine ? key : mine;
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    const unsigned long long x = __shfl_xor(mine, o, 64);
+    mine = x < mine ? x : mine;
+  }
+  if ((tid & 63) == 0) wbest[tid >> 6] = mine;
+  __syncthreads();
+  if (tid != 0) return;
+  for (int i = 1; i < SEL_THREADS / 64; ++i) mine = wbest[i] < mine ? wbest[i] : mine;
+  if (gridDim.x > 1) {
+    // device-coherent hand-over to the row's last workgroup
+    __hip_atomic_store(part + (int64_t)row * gridDim.x + blockIdx.x, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(counters + row * kDecodeCounterStride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    if (!last) return;
+    for (unsigned i = 0; i < gridDim.x; ++i) {
+      const unsigned long long x = __hip_atomic_load(part + (int64_t)row * gridDim.x + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      mine = x < mine ? x : mine;
+    }
+  }
+  a.next_index[row] = (int32_t)(mine & 0xffffffffull);
 }
 
 // ---- k > 1 ----------------------------------------------------------------------------------
@@ -527,6 +603,14 @@ int launch_h2o_update_select(const kvx_h2o_args& a_in, hipStream_t st) {
   }
   return KVX_OK;
 }
+
+int launch_select_one(const kvx_h2o_args& a, const float* stats, int per_row, uint32_t* counters, unsigned long long* part, hipStream_t st) {
+  const int wgs = (a.limit + SEL_ONE - 1) / SEL_ONE;
+  hipLaunchKernelGGL(select_one_kernel, dim3(wgs, a.B * a.Hkv), dim3(SEL_THREADS), 0, st, a, stats, per_row, counters, part);
+  KVX_HIP(hipGetLastError());
+  return KVX_OK;
+}
+int select_one_parts(int limit) { return (limit + SEL_ONE - 1) / SEL_ONE; }
 
 // ---- the same call for callers that cannot allocate -------------------------------------------
 //

@@ -30,7 +30,7 @@ namespace {
 
 #define KVX_HOST_SYMBOLS(X)                                                                                                 \
   X(kvx_last_error) X(kvx_sdpa_prefill) X(kvx_sdpa_prefill_workspace_bytes) X(kvx_score_sum) X(kvx_sdpa_prefill_weights)     \
-  X(kvx_sdpa_decode) X(kvx_sdpa_decode_workspace_bytes) X(kvx_sdpa_decode_h2o) X(kvx_sdpa_decode_h2o_workspace_bytes)        \
+  X(kvx_sdpa_decode) X(kvx_sdpa_decode_workspace_bytes) X(kvx_h2o_decode_step) X(kvx_h2o_decode_step_workspace_bytes)        \
   X(kvx_quantize_blocks) X(kvx_dequantize_blocks) X(kvx_dequantize_rows_typed) X(kvx_cache_write) \
   X(kvx_h2o_update_select) X(kvx_h2o_workspace_bytes) X(kvx_rmsnorm_rows) X(kvx_add_rmsnorm_rows) X(kvx_swiglu_rows)         \
   X(kvx_qk_norm_rope)
@@ -622,23 +622,12 @@ PyObject* cache_decode_step(PyObject* const* args, Py_ssize_t n) {
   h.q_len = 1;
   const at::Tensor out = L.empty({a.B, 1, (int64_t)a.Hq * a.D}, q.scalar_type());
   const at::Tensor next = attr_tensor(cache, names._next_flat);
-  check(lib.kvx_cache_write(&c, L.stream));
-  if (h.v_norm || h.q_errors) {
-    const at::Tensor wt = L.empty({a.B, a.Hkv, a.kv_len}, at::kFloat);
-    run_decode(a, L, out, wt, at::Tensor());
-    h.w = (const float*)wt.data_ptr();
-    run_update(h, L, next);
-    return wrap(out);
-  }
   set_o(a, out, (int64_t)a.Hq * a.D, a.D, a.D);
   h.next_index = (int32_t*)next.data_ptr();
-  const size_t nb_h = (lib.kvx_h2o_workspace_bytes(&h) + 255) / 256 * 256, nb_a = lib.kvx_sdpa_decode_h2o_workspace_bytes(&a);
-  const at::Tensor ws = L.scratch(nb_h + nb_a);
-  h.workspace = data(ws);
-  h.workspace_bytes = nb_h;
-  a.workspace = (char*)data(ws) + nb_h;
-  a.workspace_bytes = nb_a;
-  check(lib.kvx_sdpa_decode_h2o(&a, &h, L.stream));
+  const at::Tensor ws = L.scratch(lib.kvx_h2o_decode_step_workspace_bytes(&a, &h));
+  a.workspace = data(ws);
+  a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
+  check(lib.kvx_h2o_decode_step(&c, &a, &h, L.stream));
   return wrap(out);
 }
 

@@ -253,7 +253,7 @@ int kvx_dequantize_blocks(const kvx_block_quant_args* a, void* stream) {
   return launch_dequantize_blocks(*a, (hipStream_t)stream);
 }
 
-int kvx_cache_write(const kvx_cache_write_args* a, void* stream) {
+static int check_cache_write(const kvx_cache_write_args* a) {
   KVX_REQUIRE(a != nullptr, KVX_ERR_INVALID, "kvx_cache_write: args is NULL");
   KVX_REQUIRE(a->B > 0 && a->Hkv > 0 && a->num > 0 && a->cache_len > 0, KVX_ERR_INVALID, "kvx_cache_write: sizes must be positive");
   KVX_REQUIRE(kv_valid(a->kv_dtype), KVX_ERR_UNSUPPORTED, "kvx_cache_write: unknown kv_dtype %d", a->kv_dtype);
@@ -280,7 +280,12 @@ int kvx_cache_write(const kvx_cache_write_args* a, void* stream) {
   KVX_REQUIRE(!a->replay_log || (a->log_blocksize > 0 && a->log_pos >= 0), KVX_ERR_INVALID,
               "kvx_cache_write: replay log needs log_blocksize > 0 and log_pos >= 0");
   KVX_REQUIRE(!a->q_errors || !kv_is_plain(a->kv_dtype), KVX_ERR_INVALID, "kvx_cache_write: q_errors needs a quantised cache");
-  return launch_cache_write(*a, (hipStream_t)stream);
+  return KVX_OK;
+}
+
+int kvx_cache_write(const kvx_cache_write_args* a, void* stream) {
+  const int rc = check_cache_write(a);
+  return rc != KVX_OK ? rc : launch_cache_write(*a, nullptr, (hipStream_t)stream);
 }
 
 size_t kvx_h2o_workspace_bytes(const kvx_h2o_args* a) { return a ? h2o_workspace(*a) : 0; }
@@ -325,6 +330,36 @@ int kvx_sdpa_decode_h2o(const kvx_sdpa_args* a, const kvx_h2o_args* h, void* str
   KVX_REQUIRE(aligned16(a->workspace), KVX_ERR_WORKSPACE, "kvx_sdpa_decode_h2o: workspace must be 16-byte aligned");
   KVX_REQUIRE(h->workspace && h->workspace_bytes >= h2o_workspace(*h), KVX_ERR_WORKSPACE, "kvx_sdpa_decode_h2o: h2o workspace of %zu bytes needed", h2o_workspace(*h));
   return launch_sdpa_decode(*a, h, (hipStream_t)stream);
+}
+
+static int check_decode_step(const kvx_sdpa_args* a, const kvx_h2o_args* h, const char* who) {
+  int rc = check_sdpa_common(a, who, true);
+  if (rc != KVX_OK) return rc;
+  rc = check_h2o(h, who);
+  if (rc != KVX_OK) return rc;
+  KVX_REQUIRE(a->q_len == 1, KVX_ERR_INVALID, "%s: q_len must be 1, got %d", who, a->q_len);
+  const int G = a->Hq / a->Hkv;
+  KVX_REQUIRE(G >= 1 && G <= 16 && (G <= 8 || a->D <= 128), KVX_ERR_UNSUPPORTED, "%s: group size %d not in 1 .. 16 (1 .. 8 with head size 256)", who, G);
+  KVX_REQUIRE(h->k == 1 && h->kv_len == a->kv_len && h->B == a->B && h->Hkv == a->Hkv, KVX_ERR_INVALID,
+              "%s: needs k == 1 and the cache shape of the attention call", who);
+  KVX_REQUIRE(!h->v_norm || h->q_len > 0, KVX_ERR_INVALID, "%s: v_norm needs q_len > 0", who);
+  return KVX_OK;
+}
+
+size_t kvx_h2o_decode_step_workspace_bytes(const kvx_sdpa_args* a, const kvx_h2o_args* h) {
+  if (check_decode_step(a, h, "kvx_h2o_decode_step_workspace_bytes") != KVX_OK) return 0;
+  return decode_step_workspace(*a, *h);
+}
+
+int kvx_h2o_decode_step(const kvx_cache_write_args* w, const kvx_sdpa_args* a, const kvx_h2o_args* h, void* stream) {
+  int rc = check_cache_write(w);
+  if (rc != KVX_OK) return rc;
+  rc = check_decode_step(a, h, "kvx_h2o_decode_step");
+  if (rc != KVX_OK) return rc;
+  KVX_REQUIRE(w->num == 1 && w->B == a->B && w->Hkv == a->Hkv && w->D == a->D && w->kv_dtype == a->kv_dtype && w->cache_len == a->kv_len, KVX_ERR_INVALID,
+              "kvx_h2o_decode_step: the slot write must be one token into the cache the attention call reads");
+  KVX_REQUIRE(aligned16(a->workspace), KVX_ERR_WORKSPACE, "kvx_h2o_decode_step: workspace must be 16-byte aligned");
+  return launch_decode_step(*w, *a, *h, (hipStream_t)stream);
 }
 
 int kvx_rmsnorm_rows(const void* x, int64_t x_row_stride, void* out, int64_t out_row_stride, const float* weight, int64_t rows,

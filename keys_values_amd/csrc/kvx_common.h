@@ -58,7 +58,22 @@ int launch_dequantize_rows(const uint8_t* codes, const float* scale, const int32
                            int64_t out_row_stride, hipStream_t st);
 int launch_quantize_blocks(const kvx_block_quant_args& a, hipStream_t st);
 int launch_dequantize_blocks(const kvx_block_quant_args& a, hipStream_t st);
-int launch_cache_write(const kvx_cache_write_args& a, hipStream_t st);
+// Counters that a single-token step needs at zero when its split kernel starts: kDecodeCounters 32-bit words at the head
+// of a line of kDecodeCounterStride words per (batch, KV head) row, and the caller's count of scratch splits (or NULL).
+constexpr int kDecodeCounterStride = 64, kDecodeCounters = 3;
+struct DecodeCounters {
+  uint32_t* rows;
+  uint32_t* scratch_splits;
+};
+// `clear`: counters the launch also sets to zero (a step of its own would cost as much as the write), or NULL
+int launch_cache_write(const kvx_cache_write_args& a, const DecodeCounters* clear, hipStream_t st);
+int launch_decode_step(const kvx_cache_write_args& w, const kvx_sdpa_args& a, const kvx_h2o_args& h, hipStream_t st);
+size_t decode_step_workspace(const kvx_sdpa_args& a, const kvx_h2o_args& h);
+// the k == 1 choice of the Q-Hitter combination from `per_row` statistics records a row (4 floats each: extremes of the
+// compared value and of the errors); counters: one zeroed word per row, kDecodeCounterStride words apart
+// part: select_one_parts(a.limit) keys a row
+int launch_select_one(const kvx_h2o_args& a, const float* stats, int per_row, uint32_t* counters, unsigned long long* part, hipStream_t st);
+int select_one_parts(int limit);
 int launch_h2o_update_select(const kvx_h2o_args& a, hipStream_t st);
 size_t h2o_workspace(const kvx_h2o_args& a);
 int launch_h2o_update_select_static(const kvx_h2o_args& a, hipStream_t st);

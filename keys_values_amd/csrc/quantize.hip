@@ -520,12 +520,17 @@ __device__ __forceinline__ float row_quant_error(u32x4_t raw, u32x2_t codes, flo
 // the read and the write of that slot are issued by the same wavefront, in this order, and the
 // read's data is consumed before the write is issued.
 template <int D, int KV>
-__global__ __launch_bounds__(NTHREADS) void cache_write_kernel(const kvx_cache_write_args a) {
+__global__ __launch_bounds__(NTHREADS) void cache_write_kernel(const kvx_cache_write_args a, const DecodeCounters clear) {
   constexpr bool U8 = !kv_is_plain(KV);  // a quantised store: codes + row state
   constexpr bool U4 = kv_is_u4(KV);       // two codes per byte: only the lanes of the first half of a row store
   constexpr bool F16 = kv_elem_f16(KV);   // the rows are float16
   constexpr int LPR = D / 8;
   const int64_t gid = (int64_t)blockIdx.x * NTHREADS + threadIdx.x;
+  if (clear.rows) {  // one line per (batch, KV head) row: there are at least as many lanes (LPR of them a job)
+    if (gid < (int64_t)a.B * a.Hkv)
+      for (int c = 0; c < kDecodeCounters; ++c) clear.rows[gid * kDecodeCounterStride + c] = 0u;
+    if (gid == 0 && clear.scratch_splits) *clear.scratch_splits = 0u;
+  }
   const int col = (int)(gid % LPR);
   const int64_t rid = gid / LPR;
   const int64_t total = (int64_t)a.B * a.Hkv * a.num;
@@ -723,26 +728,27 @@ int launch_quantize_blocks(const kvx_block_quant_args& a, hipStream_t st) { retu
 int launch_dequantize_blocks(const kvx_block_quant_args& a, hipStream_t st) { return launch_blocks(a, false, st); }
 
 template <int D>
-int launch_cache_write_d(const kvx_cache_write_args& a, unsigned grid, hipStream_t st) {
+int launch_cache_write_d(const kvx_cache_write_args& a, const DecodeCounters& clear, unsigned grid, hipStream_t st) {
   switch (a.kv_dtype) {
-    case KVX_KV_F16: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_F16>), dim3(grid), dim3(NTHREADS), 0, st, a); break;
-    case KVX_KV_BF16: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_BF16>), dim3(grid), dim3(NTHREADS), 0, st, a); break;
-    case KVX_KV_U4: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U4>), dim3(grid), dim3(NTHREADS), 0, st, a); break;
-    case KVX_KV_U8: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U8>), dim3(grid), dim3(NTHREADS), 0, st, a); break;
-    case KVX_KV_U4_F16: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U4_F16>), dim3(grid), dim3(NTHREADS), 0, st, a); break;
-    default: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U8_F16>), dim3(grid), dim3(NTHREADS), 0, st, a); break;
+    case KVX_KV_F16: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_F16>), dim3(grid), dim3(NTHREADS), 0, st, a, clear); break;
+    case KVX_KV_BF16: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_BF16>), dim3(grid), dim3(NTHREADS), 0, st, a, clear); break;
+    case KVX_KV_U4: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U4>), dim3(grid), dim3(NTHREADS), 0, st, a, clear); break;
+    case KVX_KV_U8: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U8>), dim3(grid), dim3(NTHREADS), 0, st, a, clear); break;
+    case KVX_KV_U4_F16: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U4_F16>), dim3(grid), dim3(NTHREADS), 0, st, a, clear); break;
+    default: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U8_F16>), dim3(grid), dim3(NTHREADS), 0, st, a, clear); break;
   }
   KVX_HIP(hipGetLastError());
   return KVX_OK;
 }
 
-int launch_cache_write(const kvx_cache_write_args& a, hipStream_t st) {
+int launch_cache_write(const kvx_cache_write_args& a, const DecodeCounters* clear, hipStream_t st) {
+  const DecodeCounters none{nullptr, nullptr}, &c = clear ? *clear : none;
   const int64_t total = (int64_t)a.B * a.Hkv * a.num * (a.D / 8);
   if (total == 0) return KVX_OK;
   const unsigned grid = (unsigned)((total + NTHREADS - 1) / NTHREADS);
-  if (a.D == 256) return launch_cache_write_d<256>(a, grid, st);
-  if (a.D == 128) return launch_cache_write_d<128>(a, grid, st);
-  return launch_cache_write_d<64>(a, grid, st);
+  if (a.D == 256) return launch_cache_write_d<256>(a, c, grid, st);
+  if (a.D == 128) return launch_cache_write_d<128>(a, c, grid, st);
+  return launch_cache_write_d<64>(a, c, grid, st);
 }
 
 }  // namespace kvx

@@ -53,14 +53,20 @@ struct DecodeParams {
   float* logits;   // (B, Hkv, Tpad, G), G the padded group size
   float* part_o;   // (B, Hq, S, D)
   float* part_ml;  // (B, Hq, S, 2)
+  // one-launch form (everything but logits that go through the scratch by plan):
+  uint32_t* row_count;            // a line per (b, kvh) row: [kArrived] splits that have published their partial,
+                                  // [kFinished] splits that have done their share of the row's output and weights
+  unsigned long long* part_best;  // (B, Hkv, S): (value, slot) minimum of the split's keys (fused H2O form)
+  float* part_vn;                 // (B, Hq, S): sum of |V row| 2^(logit - maximum) (scores weighted by the V norms)
+  float* part_stats;              // (B, Hkv, S, 4): extremes of the compared value and of the quantisation errors
+  uint32_t* split_pending;        // (B, Hkv, S): 1 where the wait ran out and the logits are in the scratch
+  // logits through the scratch by plan, two launches:
   unsigned long long* best;  // fused H2O form: (value, slot) minimum per (b, kvh) row, else NULL
-  uint32_t* row_count;       // splits of a (b, kvh) row that have published their partial (resident form), then, in
-                             // the fused H2O form, the row's workgroups of the tail kernel that have finished
-  uint32_t* split_done;      // (B, Hkv, S): 1 where the split kernel itself turned its logits into weights
   uint32_t* tail_count;      // fused H2O form: workgroups of the tail kernel's second kind that have finished
   uint32_t* scratch_splits;  // caller's counter of the splits whose logits went through the scratch, or NULL
   int32_t qs_vec;            // quantiser state arrays are 16-byte aligned with strides that keep them so (vector loads of 4 keys)
   int32_t resident;          // the logits of a split stay in LDS
+  int32_t one_launch;        // the splits themselves combine their outputs (always, but for logits through the scratch by plan)
   int32_t spin_limit;        // polls of row_count before a workgroup gives up and sends its logits out
   int32_t poll_sleep;        // pause between two polls, in units of 512 cycles
   int32_t B, Hq, Hkv, kv_len, Tpad, num_splits, keys_per_split;
@@ -97,7 +103,10 @@ __device__ __forceinline__ float row_group_sum(float x) {
 // Two workgroups per compute unit share 160 KB of LDS: the logits take what the merge buffer (4 G D floats) leaves of
 // 80 KB, in whole pairs of steps of the widest kernel (256 keys).
 constexpr int logit_floats(int G, int D) { return G * D <= 512 ? 16384 : (G * D <= 1024 ? (G == 16 ? 12288 : 14336) : 8192); }
-constexpr int kCountStride = 64;  // a row's arrival counter has 256 bytes to itself: the polls of different rows go to different channels
+constexpr int kCountStride = 64;  // a row's counters have 256 bytes to themselves: the polls of different rows go to different channels
+constexpr int kArrived = 0, kFinished = 1, kSelected = 2;
+static_assert(kCountStride == kDecodeCounterStride, "the slot write clears these counters");
+constexpr uint32_t kPending = 1u << 16;  // added to kFinished by a split that leaves its weights to the row's last one
 constexpr float kNegBig = -1.0e30f;  // running maximum before the first key (finite: no inf - inf)
 constexpr float kRescaleSlack = 8.0f;  // the running maximum moves only when a logit exceeds it by this
 
@@ -141,114 +150,336 @@ __device__ __forceinline__ void flush_logits(const float* lgbuf, float* lgrow, i
   for (int j = tid; j < nkeys * G / 4; j += NTHREADS) dst[j] = ((const f32x4_t*)lgbuf)[j];
 }
 
-// What a split does once its wavefronts have left their partial results in LDS (red: unnormalised outputs, rml:
-// maximum and sum, per wavefront and head): combine them into the split's partial, and, in the resident form, wait
-// for the row's other splits and turn this split's logits (lgbuf, [key][head]) into weights.
-template <int D, int G, int LGK, int CHUNK>
-__device__ __forceinline__ void finish_split(const DecodeParams& p, const kvx_h2o_args& hh, const int h2o, const float* lgbuf,
-                                             const float (&red)[WAVES][G][D], const float (&rml)[WAVES][G][2], float* lgrow,
-                                             const int lg_base, const int k_begin, const int k_end) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
-  __syncthreads();
-  for (int i = tid; i < G * D; i += NTHREADS) {
-    const int g = i / D, d = i % D;
-    if (g >= p.Gr) continue;
-    float M = rml[0][g][0];
-#pragma unroll
-    for (int w = 1; w < WAVES; ++w) M = fmaxf(M, rml[w][g][0]);
-    float x = 0.0f, l = 0.0f;
-#pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      const float sc = fast_exp2(rml[w][g][0] - M);
-      x += red[w][g][d] * sc;
-      l += rml[w][g][1] * sc;
-    }
-    const int64_t o = ((int64_t)b * p.Hq + kvh * p.Gr + g) * p.num_splits + split;
-    p.part_o[o * D + d] = x;
-    if (d == 0) {
-      // read by the row's other workgroups while this kernel runs: a device-coherent store
-      const unsigned long long mlbits = ((unsigned long long)__float_as_uint(l) << 32) | __float_as_uint(M);
-      __hip_atomic_store((unsigned long long*)(p.part_ml + o * 2), mlbits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-  if (!lgrow || !p.resident) return;
+// Values that cross workgroups inside one launch: device-coherent (they bypass the caches that the dies do not share).
+template <typename T>
+__device__ __forceinline__ T coherent_load(const T* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+template <typename T>
+__device__ __forceinline__ void coherent_store(T* p, T v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ unsigned long long pair_bits(float lo, float hi) {
+  return ((unsigned long long)__float_as_uint(hi) << 32) | __float_as_uint(lo);
+}
 
-  // ---- the row's log-sum-exp, and this split's logits into weights, without leaving the chip --------
-  __shared__ float lse_sh[G];
-  __shared__ int row_ready;
-  __shared__ unsigned long long wbest[WAVES];
-  const int row = b * p.Hkv + kvh;
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partial above has reached device-coherent memory
-  __syncthreads();
-  if (tid == 0) {
-    uint32_t* cnt = p.row_count + row * kCountStride;
-    __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    int ok = 0;
-    for (int spin = 0; spin < p.spin_limit; ++spin) {  // bounded: a workgroup that gives up takes the scratch route
-      if (__hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= (uint32_t)p.num_splits) {
-        ok = 1;
-        break;
+// The row's outputs for the value pairs [e0, e1) of its Gr * D / 2: O = sum over the splits of part_o 2^(m - lse).
+// 16 threads share a pair, thread class j taking splits j, j + 16, ...; their sums are added in that order, so the
+// result does not depend on which workgroup takes which pairs. `buf`: 256 pairs of floats of LDS.
+template <int D, bool F16>
+__device__ __forceinline__ void merge_pairs(const DecodeParams& p, const int b, const int kvh, const float* lse_sh, const int e0, const int e1, f32x2_t* buf) {
+  const int tid = threadIdx.x, j = tid >> 4, c = tid & 15;
+  const int S = p.num_splits;
+  for (int base = e0; base < e1; base += 16) {
+    const int e = base + c;
+    f32x2_t acc = {0.0f, 0.0f};
+    if (e < e1) {
+      const int g = e / (D / 2);
+      const int64_t hd = (int64_t)b * p.Hq + kvh * p.Gr + g;
+      const unsigned long long* po = (const unsigned long long*)(p.part_o + hd * S * D) + e % (D / 2);
+      const float* ml = p.part_ml + hd * S * 2;
+      const float lse = lse_sh[g];
+      for (int s0 = j; s0 < S; s0 += 64) {  // four loads in flight
+        unsigned long long x[4];
+        float m[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int sp = min(s0 + 16 * u, S - 1);
+          x[u] = coherent_load(po + (int64_t)sp * (D / 2));
+          m[u] = coherent_load(ml + 2 * sp);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const float w = s0 + 16 * u < S ? fast_exp2(m[u] - lse) : 0.0f;
+          acc[0] += __uint_as_float((uint32_t)x[u]) * w;
+          acc[1] += __uint_as_float((uint32_t)(x[u] >> 32)) * w;
+        }
       }
-      for (int z = 0; z < p.poll_sleep; ++z) __builtin_amdgcn_s_sleep(8);
     }
-    row_ready = ok;
-  }
-  __syncthreads();
-  if (!row_ready) {
-    flush_logits<G, LGK, CHUNK>(lgbuf, lgrow, lg_base, k_end, tid);
-    if (tid == 0) {
-      p.split_done[(int64_t)row * p.num_splits + split] = 0u;
-      if (p.scratch_splits) atomicAdd(p.scratch_splits, 1u);
+    __syncthreads();
+    buf[j * 16 + c] = acc;
+    __syncthreads();
+    if (j == 0 && e < e1) {
+      f32x2_t t = buf[c];
+#pragma unroll
+      for (int i = 1; i < 16; ++i) t += buf[i * 16 + c];
+      const int g = e / (D / 2);
+      *(uint32_t*)(p.o + b * p.o_sb + (int64_t)(kvh * p.Gr + g) * p.o_sh + 2 * (e % (D / 2))) = pack_pair<F16>(t[0], t[1]);
     }
-    return;
   }
+}
+
+// LDS of the part of a workgroup's life after its key loop.
+template <int G>
+struct FinishShared {
+  float lse[G];
+  float z;  // scores weighted by the V norms: the row's sum of |V row| W
+  float vn[G];
+  float red[WAVES][4];
+  unsigned long long best[WAVES];
+  uint32_t ready, last, finished;
+};
+
+// The row's log-sum-exps (and z) from its splits' partials, in LDS for the whole workgroup. All splits have published.
+template <int G>
+__device__ __forceinline__ void row_state(const DecodeParams& p, const bool vnorm, const int b, const int kvh, FinishShared<G>& sh) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int g = wave; g < G; g += WAVES) {  // a wavefront per head: lane s takes splits s, s + 64, ...
-    float lse = INFINITY;  // dummy heads: exp2(x - inf) = 0
-    if (g < p.Gr) lse = row_lse<true>(p.part_ml + ((int64_t)b * p.Hq + kvh * p.Gr + g) * p.num_splits * 2, p.num_splits, lane);
-    if (lane == 0) lse_sh[g] = lse;
+    float lse = INFINITY, z = 0.0f;        // dummy heads: exp2(x - inf) = 0
+    if (g < p.Gr) {
+      const int64_t hd = (int64_t)b * p.Hq + kvh * p.Gr + g;
+      lse = row_lse<true>(p.part_ml + hd * p.num_splits * 2, p.num_splits, lane);
+      if (vnorm) {
+        for (int sp = lane; sp < p.num_splits; sp += 64)
+          z += coherent_load(p.part_vn + hd * p.num_splits + sp) * fast_exp2(coherent_load(p.part_ml + (hd * p.num_splits + sp) * 2) - lse);
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) z += __shfl_xor(z, off, 64);
+      }
+    }
+    if (lane == 0) {
+      sh.lse[g] = lse;
+      sh.vn[g] = z;
+    }
   }
   __syncthreads();
+  if (vnorm && threadIdx.x == 0) {
+    float z = 0.0f;
+    for (int g = 0; g < p.Gr; ++g) z += sh.vn[g];
+    sh.z = z / (float)p.Gr;
+  }
+  if (vnorm) __syncthreads();
+}
+
+// Weights of the keys [k0, k1) of split `split`, logits(k, x) giving the logits of key k: W, and in the fused H2O form
+// scores += W (or the V-norm weighted increment) and what the eviction choice needs of these keys -- their
+// (value, slot) minimum, or, where the compared value is normalised over the batch element first, its extremes.
+template <int G, typename F>
+__device__ __forceinline__ void weigh_split(const DecodeParams& p, const kvx_h2o_args& hh, const int h2o, const int b, const int kvh, FinishShared<G>& sh,
+                                            const int split, const int k0, const int k1, F logits) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int row = b * p.Hkv + kvh;
   float lse[G];
 #pragma unroll
-  for (int g = 0; g < G; ++g) lse[g] = lse_sh[g];
+  for (int g = 0; g < G; ++g) lse[g] = sh.lse[g];
   float* wr = p.w ? p.w + (int64_t)row * p.kv_len : nullptr;
-  float* sc = h2o ? hh.scores + b * hh.sc_stride_b + kvh * hh.sc_stride_h : nullptr;
+  const int64_t so = h2o ? b * hh.sc_stride_b + kvh * hh.sc_stride_h : 0;
+  float* sc = h2o ? hh.scores + so : nullptr;
+  const float* vn = h2o && hh.v_norm ? hh.v_norm + so : nullptr;
+  const float* qe = h2o && hh.q_errors ? hh.q_errors + so : nullptr;
   const int32_t* tpr = (h2o && hh.token_pos) ? hh.token_pos + b * hh.tp_stride_b + kvh * hh.tp_stride_h : nullptr;
-  const float inv_g = 1.0f / (float)p.Gr;
+  const float inv_g = 1.0f / (float)p.Gr, z = sh.z, ql = (float)hh.q_len;
   unsigned long long mine = ~0ull;
-  for (int k = k_begin + tid; k < k_end; k += NTHREADS) {
-    const float* lg = lgbuf + (k - k_begin) * G;
+  float smin = INFINITY, smax = -INFINITY, qmin = INFINITY, qmax = -INFINITY;
+  for (int k = k0 + tid; k < k1; k += NTHREADS) {
+    float x[G];
+    logits(k, x);
     float acc = 0.0f;
 #pragma unroll
-    for (int g = 0; g < G; ++g) acc += fast_exp2(lg[g] - lse[g]);
+    for (int g = 0; g < G; ++g) acc += fast_exp2(x[g] - lse[g]);
     acc *= inv_g;
     if (wr) wr[k] = acc;
-    if (h2o) {
-      float val = sc[k] + acc;
-      sc[k] = val;
-      if (k < hh.limit) {
-        if (hh.normalize) val = val / (float)(hh.input_pos - max(tpr[k], hh.prefill_len - 1));
+    if (!h2o) continue;
+    // every product and sum rounded on its own, as the reference's tensor expressions are
+    const float inst = vn ? __fmul_rn(__fmul_rn(vn[k], acc) / z, ql) : acc;
+    float val = __fadd_rn(sc[k], inst);
+    sc[k] = val;
+    if (k < hh.limit) {
+      if (hh.normalize) val = val / (float)(hh.input_pos - max(tpr[k], hh.prefill_len - 1));
+      if (qe) {
+        smin = fminf(smin, val);
+        smax = fmaxf(smax, val);
+        qmin = fminf(qmin, qe[k]);
+        qmax = fmaxf(qmax, qe[k]);
+      } else {
         const unsigned long long key = ((unsigned long long)ordered_bits(val) << 32) | (unsigned)k;
         mine = key < mine ? key : mine;
       }
     }
   }
-  if (h2o) {
+  if (!h2o) return;
+  if (qe) {
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+      smin = fminf(smin, __shfl_xor(smin, off, 64));
+      smax = fmaxf(smax, __shfl_xor(smax, off, 64));
+      qmin = fminf(qmin, __shfl_xor(qmin, off, 64));
+      qmax = fmaxf(qmax, __shfl_xor(qmax, off, 64));
+    }
+    if (lane == 0) {
+      sh.red[wave][0] = smin;
+      sh.red[wave][1] = smax;
+      sh.red[wave][2] = qmin;
+      sh.red[wave][3] = qmax;
+    }
+    __syncthreads();
+    if (tid < 4) {
+      float r = sh.red[0][tid];
+      for (int i = 1; i < WAVES; ++i) r = (tid & 1) ? fmaxf(r, sh.red[i][tid]) : fminf(r, sh.red[i][tid]);
+      p.part_stats[((int64_t)row * p.num_splits + split) * 4 + tid] = r;  // read by the next launch
+    }
+    __syncthreads();
+    return;
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    const unsigned long long o = __shfl_xor(mine, off, 64);
+    mine = o < mine ? o : mine;
+  }
+  if (lane == 0) sh.best[wave] = mine;
+  __syncthreads();
+  if (tid == 0) {
+    unsigned long long mn = sh.best[0];
+    for (int i = 1; i < WAVES; ++i) mn = sh.best[i] < mn ? sh.best[i] : mn;
+    coherent_store(p.part_best + (int64_t)row * p.num_splits + split, mn);
+  }
+  __syncthreads();
+}
+
+// What a split does once its wavefronts have left their partial results in LDS (red: unnormalised outputs, rml:
+// maximum and sum, per wavefront and head).
+//
+// One launch does the whole step. The split publishes its partial and counts itself in. Without weights the split
+// that arrives last combines the row's outputs. With weights every split waits (boundedly) for the row's others, then
+// takes an equal share of the row's outputs and turns its own logits (lgbuf, [key][head]) into weights; a split whose
+// wait ran out puts its logits into the scratch instead. The split that finishes last makes up what such splits left
+// undone and publishes the row's slot. A second launch for the outputs and a third to reset the counters cost 4 to 8 us
+// of every step, a third of a step over 4096 slots.
+template <int D, int G, int LGK, int CHUNK, bool F16>
+__device__ __forceinline__ void finish_split(const DecodeParams& p, const kvx_h2o_args& hh, const int h2o, const float* lgbuf,
+                                             float (&red)[WAVES][G][D], const float (&rml)[WAVES][G][2], float* lgrow,
+                                             const int lg_base, const int k_begin, const int k_end) {
+  __shared__ FinishShared<G> sh;
+  __shared__ f32x2_t buf[256];
+  const int tid = threadIdx.x;
+  const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
+  const int row = b * p.Hkv + kvh, S = p.num_splits, E = p.Gr * (D / 2);
+  __syncthreads();
+  for (int i = tid; i < E; i += NTHREADS) {
+    const int g = i / (D / 2), d = 2 * (i % (D / 2));
+    float M = rml[0][g][0];
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) M = fmaxf(M, rml[w][g][0]);
+    float x0 = 0.0f, x1 = 0.0f, l = 0.0f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float sc = fast_exp2(rml[w][g][0] - M);
+      x0 += red[w][g][d] * sc;
+      x1 += red[w][g][d + 1] * sc;
+      l += rml[w][g][1] * sc;
+    }
+    const int64_t o = ((int64_t)b * p.Hq + kvh * p.Gr + g) * S + split;
+    // read by other workgroups while this kernel runs
+    coherent_store((unsigned long long*)(p.part_o + o * D + d), pair_bits(x0, x1));
+    if (d == 0) coherent_store((unsigned long long*)(p.part_ml + o * 2), pair_bits(M, l));
+  }
+  if (!p.one_launch) return;
+  const bool vnorm = h2o && hh.v_norm;
+  if (vnorm) {  // this split's part of z: sum over its keys of |V row| 2^(logit - maximum), per head
+    const float* vn = hh.v_norm + b * hh.sc_stride_b + kvh * hh.sc_stride_h;
+    float M[G], a[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      M[g] = rml[0][g][0];
+#pragma unroll
+      for (int w = 1; w < WAVES; ++w) M[g] = fmaxf(M[g], rml[w][g][0]);
+      a[g] = 0.0f;
+    }
+    for (int k = k_begin + tid; k < k_end; k += NTHREADS) {
+      const float v = vn[k];
+#pragma unroll
+      for (int g = 0; g < G; ++g) a[g] += v * fast_exp2(lgbuf[(k - k_begin) * G + g] - M[g]);
+    }
+    __syncthreads();  // red has been read
+    float* part = &red[0][0][0];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+#pragma unroll
+      for (int off = 32; off >= 1; off >>= 1) a[g] += __shfl_xor(a[g], off, 64);
+      if ((tid & 63) == 0) part[(tid >> 6) * G + g] = a[g];
+    }
+    __syncthreads();
+    if (tid < p.Gr) {
+      float t = part[tid];
+      for (int w = 1; w < WAVES; ++w) t += part[w * G + tid];
+      coherent_store(p.part_vn + ((int64_t)b * p.Hq + kvh * p.Gr + tid) * S + split, t);
+    }
+  }
+  uint32_t* cnt = p.row_count + row * kCountStride;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partial above has reached device-coherent memory
+  __syncthreads();
+  if (tid == 0) {
+    const bool last = S == 1 || __hip_atomic_fetch_add(cnt + kArrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)S - 1u;
+    uint32_t ok = 0;
+    if (lgrow) {
+      for (int spin = 0; spin < p.spin_limit; ++spin) {  // bounded: a workgroup that gives up takes the scratch route
+        if (S == 1 || coherent_load(cnt + kArrived) >= (uint32_t)S) {
+          ok = 1;
+          break;
+        }
+        // short pauses first: splits of a row that run side by side arrive within a microsecond of each other
+        const int pause = min(p.poll_sleep, 1 + (spin >> 2));
+        for (int z = 0; z < pause; ++z) __builtin_amdgcn_s_sleep(8);
+      }
+    }
+    sh.last = last;
+    sh.ready = ok;
+  }
+  __syncthreads();
+  if (!lgrow) {
+    if (!sh.last) return;
+    row_state<G>(p, false, b, kvh, sh);
+    merge_pairs<D, F16>(p, b, kvh, sh.lse, 0, E, buf);
+    if (p.lse_out && tid < p.Gr) p.lse_out[(int64_t)b * p.Hq + kvh * p.Gr + tid] = sh.lse[tid];
+    return;
+  }
+  const bool ready = sh.ready;
+  if (ready) {
+    row_state<G>(p, vnorm, b, kvh, sh);
+    merge_pairs<D, F16>(p, b, kvh, sh.lse, (int)((int64_t)E * split / S), (int)((int64_t)E * (split + 1) / S), buf);
+    weigh_split<G>(p, hh, h2o, b, kvh, sh, split, k_begin, k_end, [&](int k, float (&x)[G]) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) x[g] = lgbuf[(k - k_begin) * G + g];
+    });
+  } else {
+    const int n = (k_end - k_begin) * G;
+    float* dst = lgrow + (int64_t)k_begin * G;
+    for (int i = tid; i < n; i += NTHREADS) coherent_store(dst + i, lgbuf[i]);
+    if (tid == 0 && p.scratch_splits) atomicAdd(p.scratch_splits, 1u);
+  }
+  if (tid == 0) coherent_store(p.split_pending + (int64_t)row * S + split, ready ? 0u : 1u);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    const uint32_t mine = ready ? 1u : 1u + kPending;
+    sh.finished = S == 1 ? mine : mine + __hip_atomic_fetch_add(cnt + kFinished, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  const uint32_t finished = sh.finished;
+  if ((finished & (kPending - 1u)) != (uint32_t)S) return;
+
+  // ---- the row's last split: the shares of the splits that gave up, the log-sum-exps, the chosen slot ---------------
+  if (!ready && (finished >= kPending || p.lse_out)) row_state<G>(p, vnorm, b, kvh, sh);
+  if (finished >= kPending)
+    for (int sp = 0; sp < S; ++sp) {
+      if (!coherent_load(p.split_pending + (int64_t)row * S + sp)) continue;  // the same for every thread
+      merge_pairs<D, F16>(p, b, kvh, sh.lse, (int)((int64_t)E * sp / S), (int)((int64_t)E * (sp + 1) / S), buf);
+      const int k0 = sp * p.keys_per_split, k1 = min(k0 + p.keys_per_split, p.kv_len);
+      weigh_split<G>(p, hh, h2o, b, kvh, sh, sp, k0, k1, [&](int k, float (&x)[G]) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) x[g] = coherent_load(lgrow + (int64_t)k * G + g);
+      });
+    }
+  if (p.lse_out && tid < p.Gr) p.lse_out[(int64_t)b * p.Hq + kvh * p.Gr + tid] = sh.lse[tid];
+  if (h2o && !hh.q_errors && tid < 64) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    unsigned long long mine = ~0ull;
+    for (int sp = tid; sp < S; sp += 64) {
+      const unsigned long long o = coherent_load(p.part_best + (int64_t)row * S + sp);
+      mine = o < mine ? o : mine;
+    }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
       const unsigned long long o = __shfl_xor(mine, off, 64);
       mine = o < mine ? o : mine;
     }
-    if (lane == 0) wbest[wave] = mine;
-    __syncthreads();
-    if (tid == 0) {
-      unsigned long long mn = wbest[0];
-      for (int i = 1; i < WAVES; ++i) mn = wbest[i] < mn ? wbest[i] : mn;
-      if (mn != ~0ull) atomicMin(p.best + row, mn);
-    }
+    if (tid == 0) hh.next_index[row] = (int32_t)(mine & 0xffffffffull);
   }
-  if (tid == 0) p.split_done[(int64_t)row * p.num_splits + split] = 1u;
 }
 
 template <int D, int G, int KV>
@@ -260,7 +491,7 @@ __global__ __launch_bounds__(NTHREADS) void decode_split_kernel(const DecodePara
   constexpr int CH = U * RPI;    // keys per wavefront and step, contiguous
   constexpr int LGK = logit_floats(G, D) / G;  // keys whose logits are gathered in LDS before they go out in one burst
   __shared__ __align__(16) float lgbuf[LGK * G];  // [key][head]
-  __shared__ float red[WAVES][G][D];
+  __shared__ __align__(16) float red[WAVES][G][D];
   __shared__ float rml[WAVES][G][2];
 
   const int tid = threadIdx.x;
@@ -446,7 +677,7 @@ __global__ __launch_bounds__(NTHREADS) void decode_split_kernel(const DecodePara
       rml[wave][g][1] = l;
     }
   }
-  finish_split<D, G, LGK, CH>(p, hh, h2o, lgbuf, red, rml, lgrow, lg_base, k_begin, k_end);
+  finish_split<D, G, LGK, CH, F16>(p, hh, h2o, lgbuf, red, rml, lgrow, lg_base, k_begin, k_end);
 }
 
 // ---- the same split with both products on the matrix cores --------------------------------------------------------
@@ -488,7 +719,7 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
   constexpr int VW = U4 ? (DPL + 7) / 8 : (U8 ? (DPL + 3) / 4 : DPL / 2);  // dwords per key of V
   constexpr int LGK = logit_floats(G, D) / G;
   __shared__ __align__(16) float lgbuf[LGK * G];  // [key][head]
-  __shared__ float red[WAVES][G][D];
+  __shared__ __align__(16) float red[WAVES][G][D];
   __shared__ float rml[WAVES][G][2];
   static_assert(D == 64 || D == 128 || (D == 256 && U8), "plain rows of 256 values take the vector-ALU kernel");
 
@@ -764,15 +995,17 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
       rml[wave][m][1] = l;
     }
   }
-  finish_split<D, G, LGK, CH>(p, hh, h2o, lgbuf, red, rml, lgrow, lg_base, k_begin, k_end);
+  finish_split<D, G, LGK, CH, F16>(p, hh, h2o, lgbuf, red, rml, lgrow, lg_base, k_begin, k_end);
 }
 
-// Before the split kernel: no split of a row has arrived, no row has a lowest-score slot yet.
+// Before the split kernel, where the slot write does not do it: no split of a row has arrived, no row has a
+// lowest-score slot yet.
 __global__ void decode_init_kernel(uint32_t* row_count, unsigned long long* best, uint32_t* tail_count, int rows,
                                    uint32_t* scratch_splits, uint32_t scratch_splits_init) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < rows) {
-    if (row_count) row_count[i * kCountStride] = 0u;
+    if (row_count)
+      for (int c = 0; c < kDecodeCounters; ++c) row_count[i * kCountStride + c] = 0u;
     if (best) best[i] = ~0ull;
   }
   if (i == 0 && tail_count) *tail_count = 0u;
@@ -819,8 +1052,7 @@ __device__ __forceinline__ void merge_job(const DecodeParams& p, const int bh) {
 }
 
 // W[b, kvh, k] = (1/G) sum_g exp2(logit[b, kvh, k, g] - lse[b, kvh*G+g]); one key per lane and pass,
-// 4096 keys per workgroup of NT threads, for the splits whose logits went to the scratch (in the resident form:
-// those whose wait ran out, normally none). With H2O set it also does the cache's score update and eviction choice
+// 4096 keys per workgroup of NT threads, where the logits went to the scratch. With H2O set it also does the cache's score update and eviction choice
 // in the same pass (keys_values/kvcache/h2o.py:175-196, keys_values/kvcache/attn_weights.py:773-774
 // for one slot): scores += W, then the (value, slot) minimum of the row through an integer atomicMin; the workgroup
 // that finishes last publishes the slot of every row's minimum. (That needs no fence: the minima and the count of
@@ -835,16 +1067,8 @@ __device__ __forceinline__ void weights_job(const DecodeParams& p, const kvx_h2o
   __shared__ float lse_sh[G];
   __shared__ unsigned long long wbest[NT / 64];
   __shared__ int last_job;
-  const uint32_t* done = p.resident ? p.split_done + ((int64_t)b * p.Hkv + kvh) * p.num_splits : nullptr;
-  int pending = 1;
-  if (done) {
-    const int s0 = bx * 4096 / p.keys_per_split, s1 = min((bx * 4096 + 4095) / p.keys_per_split, p.num_splits - 1);
-    pending = 0;
-    for (int sp = s0 + tid; sp <= s1; sp += NT) pending |= done[sp] == 0u;
-    pending = __syncthreads_or(pending);
-  }
   unsigned long long mine = ~0ull;
-  if (pending) {
+  {
     // the row's log-sum-exps from the splits' partials, by the routine the split kernel and the merge use
     for (int g = wave; g < G; g += NT / 64) {
       float l = INFINITY;  // dummy heads: exp2(x - inf) = 0
@@ -870,7 +1094,6 @@ __device__ __forceinline__ void weights_job(const DecodeParams& p, const kvx_h2o
     for (int it = 0; it < PASSES; ++it) {
       const int k = bx * 4096 + it * NT + tid;
       if (k >= p.kv_len) break;
-      if (done && done[k / p.keys_per_split]) continue;
       float acc = 0.0f;
 #pragma unroll
       for (int g = 0; g < G; ++g) {
@@ -894,28 +1117,23 @@ __device__ __forceinline__ void weights_job(const DecodeParams& p, const kvx_h2o
     }
   }
   if constexpr (H2O) {
-    if (pending) {
 #pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) {
-        const unsigned long long o = __shfl_xor(mine, off, 64);
-        mine = o < mine ? o : mine;
-      }
-      if (lane == 0) wbest[wave] = mine;
-      __syncthreads();
+    for (int off = 32; off >= 1; off >>= 1) {
+      const unsigned long long o = __shfl_xor(mine, off, 64);
+      mine = o < mine ? o : mine;
     }
+    if (lane == 0) wbest[wave] = mine;
+    __syncthreads();
     if (tid == 0) {
-      if (pending) {
-        unsigned long long mn = wbest[0];
-        for (int i = 1; i < NT / 64; ++i) mn = wbest[i] < mn ? wbest[i] : mn;
-        if (mn != ~0ull) {
-          const unsigned long long old = __hip_atomic_fetch_min(p.best + b * p.Hkv + kvh, mn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          asm volatile("s_waitcnt vmcnt(0)" : : "v"(old) : "memory");  // performed before this workgroup counts itself
-        }
+      unsigned long long mn = wbest[0];
+      for (int i = 1; i < NT / 64; ++i) mn = wbest[i] < mn ? wbest[i] : mn;
+      if (mn != ~0ull) {
+        const unsigned long long old = __hip_atomic_fetch_min(p.best + b * p.Hkv + kvh, mn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" : : "v"(old) : "memory");  // performed before this workgroup counts itself
       }
-      // counted per row first (the row's counter goes on from where the split kernel's arrivals left it), rows second:
-      // no counter sees more than a few dozen increments
+      // counted per row first, rows second: no counter sees more than a few dozen increments
       const int wx = jobs / (p.B * p.Hkv);
-      const uint32_t row_full = (p.resident ? (uint32_t)p.num_splits : 0u) + (uint32_t)wx - 1u;
+      const uint32_t row_full = (uint32_t)wx - 1u;
       const bool row_last = __hip_atomic_fetch_add(p.row_count + (b * p.Hkv + kvh) * kCountStride, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == row_full;
       last_job = row_last && __hip_atomic_fetch_add(p.tail_count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(p.B * p.Hkv - 1);
     }
@@ -927,7 +1145,7 @@ __device__ __forceinline__ void weights_job(const DecodeParams& p, const kvx_h2o
   }
 }
 
-// What follows the split kernel, in one launch: the first merge_jobs workgroups combine the splits of one (batch,
+// What follows the split kernel where the logits go through the scratch by plan, in one launch: the first merge_jobs workgroups combine the splits of one (batch,
 // query head) each; the others (MODE 1: weights wanted, MODE 2: fused H2O step) take 4096 keys of a (batch, KV head)
 // row each. The two kinds do not depend on each other: both read what the split kernel left.
 template <int D, bool F16, int G, int MODE>
@@ -936,15 +1154,13 @@ __global__ __launch_bounds__(4 * D) void decode_tail_kernel(const DecodeParams p
     merge_job<D, F16>(p, blockIdx.x);
     return;
   }
-  if constexpr (MODE > 0) {
-    const int j = blockIdx.x - merge_jobs;
-    weights_job<G, MODE == 2, 4 * D>(p, hh, j % wx, (j / wx) % p.Hkv, j / (wx * p.Hkv), (int)gridDim.x - merge_jobs);
-  }
+  const int j = blockIdx.x - merge_jobs;
+  weights_job<G, MODE == 2, 4 * D>(p, hh, j % wx, (j / wx) % p.Hkv, j / (wx * p.Hkv), (int)gridDim.x - merge_jobs);
 }
 
 struct Plan {
-  int G, num_splits, keys_per_split, Tpad, resident;
-  size_t off_logits, off_part_o, off_part_ml, off_best, off_tail, off_count, off_done, total;
+  int G, num_splits, keys_per_split, Tpad, resident, one_launch;
+  size_t off_logits, off_part_o, off_part_ml, off_part_best, off_part_vn, off_part_stats, off_pending, off_best, off_tail, off_count, total;
 };
 
 // Switches of the route the logits take, process-wide. Defaults come from the environment, read ONCE (first use):
@@ -1010,24 +1226,28 @@ Plan make_plan(const kvx_sdpa_args& a, bool fused_h2o) {
   pl.keys_per_split = kps;
   pl.num_splits = (a.kv_len + kps - 1) / kps;
   pl.Tpad = ((a.kv_len + 63) / 64) * 64;
-  size_t off = 0;
-  pl.off_logits = off;
-  off += weights ? (size_t)a.B * a.Hkv * pl.G * pl.Tpad * 4 : 0;
-  pl.off_part_o = off;
-  off += (size_t)a.B * a.Hq * pl.num_splits * a.D * 4;
-  pl.off_part_ml = off;
-  off += (size_t)a.B * a.Hq * pl.num_splits * 2 * 4;
-  off = (off + 7) & ~(size_t)7;
-  pl.off_best = off;
-  off += fused_h2o ? (size_t)a.B * a.Hkv * 8 : 0;
-  pl.off_tail = off;
-  off += fused_h2o ? 8 : 0;
   pl.resident = allow_resident && kps <= lgk;
+  pl.one_launch = pl.resident || !weights;
+  size_t off = 0;
+  auto take = [&off](size_t bytes) {  // 16-byte aligned pieces
+    const size_t at = off;
+    off += (bytes + 15) & ~(size_t)15;
+    return at;
+  };
+  const size_t rows = (size_t)a.B * a.Hkv, row_splits = rows * pl.num_splits, head_splits = (size_t)a.B * a.Hq * pl.num_splits;
+  const bool fused_one = fused_h2o && pl.one_launch, fused_two = fused_h2o && !pl.one_launch;
+  pl.off_logits = take(weights ? rows * pl.G * pl.Tpad * 4 : 0);
+  pl.off_part_o = take(head_splits * a.D * 4);
+  pl.off_part_ml = take(head_splits * 2 * 4);
+  // the choice after the combination with the errors hands its minima over in the same place
+  pl.off_part_best = take(fused_one ? rows * max(pl.num_splits, select_one_parts(a.kv_len)) * 8 : 0);
+  pl.off_part_vn = take(fused_one ? head_splits * 4 : 0);
+  pl.off_part_stats = take(fused_one ? row_splits * 16 : 0);
+  pl.off_pending = take(pl.resident ? row_splits * 4 : 0);
+  pl.off_best = take(fused_two ? rows * 8 : 0);
+  pl.off_tail = take(fused_two ? 8 : 0);
   off = (off + 255) & ~(size_t)255;
-  pl.off_count = off;
-  off += (pl.resident || fused_h2o) ? (size_t)a.B * a.Hkv * kCountStride * 4 : 0;
-  pl.off_done = off;
-  off += pl.resident ? (size_t)a.B * a.Hkv * pl.num_splits * 4 : 0;
+  pl.off_count = take(pl.one_launch || fused_h2o ? rows * kCountStride * 4 : 0);
   pl.total = (off + 255) & ~(size_t)255;
   return pl;
 }
@@ -1035,26 +1255,27 @@ Plan make_plan(const kvx_sdpa_args& a, bool fused_h2o) {
 template <int D, bool F16, int G>
 int launch_tail(const DecodeParams& p, const kvx_h2o_args* hh, hipStream_t st) {
   const int merge_jobs = p.B * p.Hq, wx = (p.kv_len + 4095) / 4096;
-  const int weight_jobs = (hh || p.w) ? wx * p.Hkv * p.B : 0;
+  const int weight_jobs = wx * p.Hkv * p.B;
   const dim3 grid(merge_jobs + weight_jobs), block(4 * D);
   const kvx_h2o_args h2 = hh ? *hh : kvx_h2o_args{};
   if (hh) hipLaunchKernelGGL((decode_tail_kernel<D, F16, G, 2>), grid, block, 0, st, p, h2, merge_jobs, wx);
-  else if (p.w) hipLaunchKernelGGL((decode_tail_kernel<D, F16, G, 1>), grid, block, 0, st, p, h2, merge_jobs, wx);
-  else hipLaunchKernelGGL((decode_tail_kernel<D, F16, 1, 0>), grid, block, 0, st, p, h2, merge_jobs, wx);
+  else hipLaunchKernelGGL((decode_tail_kernel<D, F16, G, 1>), grid, block, 0, st, p, h2, merge_jobs, wx);
   KVX_HIP(hipGetLastError());
   return KVX_OK;
 }
 
-// Three launches: the counters' reset (only when something counts), the split kernel, the tail.
+// The counters' reset (unless `counters_clear`: the slot write before did it, or there is a single split), the split
+// kernel and, where the logits go through the scratch by plan, the tail.
 template <int D, int G>
-int launch_dg(const DecodeParams& p, int kv, const kvx_h2o_args* hh, hipStream_t st) {
+int launch_dg(const DecodeParams& p, int kv, const kvx_h2o_args* hh, bool counters_clear, hipStream_t st) {
   dim3 grid(p.num_splits, p.Hkv, p.B);
   const int rows = p.B * p.Hkv;
-  if (p.resident || hh || p.scratch_splits) {
+  const bool counts = p.one_launch ? p.num_splits > 1 && !counters_clear : hh != nullptr;
+  if (counts || (p.scratch_splits && !counters_clear)) {
     // splits that take the scratch route by plan (the resident form switched off or too long for the LDS) count from the start
     const uint32_t by_plan = (p.logits && !p.resident) ? (uint32_t)(rows * p.num_splits) : 0u;
-    hipLaunchKernelGGL(decode_init_kernel, dim3((rows + 255) / 256), dim3(256), 0, st, (p.resident || hh) ? p.row_count : nullptr,
-                       hh ? p.best : nullptr, hh ? p.tail_count : nullptr, rows, p.scratch_splits, by_plan);
+    hipLaunchKernelGGL(decode_init_kernel, dim3((rows + 255) / 256), dim3(256), 0, st, counts ? p.row_count : nullptr, p.best, p.tail_count, rows,
+                       p.scratch_splits, by_plan);
     KVX_HIP(hipGetLastError());
   }
   const kvx_h2o_args h2 = hh ? *hh : kvx_h2o_args{};
@@ -1077,18 +1298,19 @@ int launch_dg(const DecodeParams& p, int kv, const kvx_h2o_args* hh, hipStream_t
     }
   }
   KVX_HIP(hipGetLastError());
+  if (p.one_launch) return KVX_OK;
   return kv_elem_f16(kv) ? launch_tail<D, true, G>(p, hh, st) : launch_tail<D, false, G>(p, hh, st);
 }
 
 template <int D>
-int launch_d(const DecodeParams& p, int G, int kv, const kvx_h2o_args* hh, hipStream_t st) {
+int launch_d(const DecodeParams& p, int G, int kv, const kvx_h2o_args* hh, bool counters_clear, hipStream_t st) {
   switch (G) {
-    case 1: return launch_dg<D, 1>(p, kv, hh, st);
-    case 2: return launch_dg<D, 2>(p, kv, hh, st);
-    case 4: return launch_dg<D, 4>(p, kv, hh, st);
-    case 8: return launch_dg<D, 8>(p, kv, hh, st);
+    case 1: return launch_dg<D, 1>(p, kv, hh, counters_clear, st);
+    case 2: return launch_dg<D, 2>(p, kv, hh, counters_clear, st);
+    case 4: return launch_dg<D, 4>(p, kv, hh, counters_clear, st);
+    case 8: return launch_dg<D, 8>(p, kv, hh, counters_clear, st);
     case 16:
-      if constexpr (D <= 128) return launch_dg<D, 16>(p, kv, hh, st);
+      if constexpr (D <= 128) return launch_dg<D, 16>(p, kv, hh, counters_clear, st);
       break;
   }
   return set_error(KVX_ERR_UNSUPPORTED, "kvx_sdpa_decode: %d query heads per KV head (at most 16; at most 8 with head size 256)", p.Gr);
@@ -1105,15 +1327,14 @@ void set_decode_tuning(int resident, int spin_limit, int poll_sleep) {
   t.poll_sleep = poll_sleep < 0 ? t.env_sleep : clampi(poll_sleep, 0, kSleepMax);
 }
 
-int launch_sdpa_decode(const kvx_sdpa_args& a, const kvx_h2o_args* hh, hipStream_t st) {
-  const Plan pl = make_plan(a, hh != nullptr);
+namespace {
+int decode_params(DecodeParams& p, const kvx_sdpa_args& a, const kvx_h2o_args* hh, const Plan& pl) {
   KVX_REQUIRE(a.workspace && a.workspace_bytes >= pl.total, KVX_ERR_WORKSPACE,
               "kvx_sdpa_decode: workspace of %zu bytes needed, %zu given", pl.total, a.workspace_bytes);
   const int64_t es = kv_is_plain(a.kv_dtype) ? 2 : 1;
   KVX_REQUIRE((int64_t)a.kv_len * a.k_stride_t * es < (1ll << 32) && (int64_t)a.kv_len * a.v_stride_t * es < (1ll << 32), KVX_ERR_UNSUPPORTED,
               "kvx_sdpa_decode: one (batch, head) row set of K or V must span less than 4 GiB (kv_len %d, slot strides %lld / %lld)",
               a.kv_len, (long long)a.k_stride_t, (long long)a.v_stride_t);
-  DecodeParams p;
   char* ws = (char*)a.workspace;
   p.q = (const uint16_t*)a.q;
   p.k = a.k;
@@ -1125,12 +1346,17 @@ int launch_sdpa_decode(const kvx_sdpa_args& a, const kvx_h2o_args* hh, hipStream
   p.logits = (a.w || hh) ? (float*)(ws + pl.off_logits) : nullptr;
   p.part_o = (float*)(ws + pl.off_part_o);
   p.part_ml = (float*)(ws + pl.off_part_ml);
-  p.best = hh ? (unsigned long long*)(ws + pl.off_best) : nullptr;
-  p.tail_count = hh ? (uint32_t*)(ws + pl.off_tail) : nullptr;
+  const bool two = hh && !pl.one_launch;
+  p.best = two ? (unsigned long long*)(ws + pl.off_best) : nullptr;
+  p.tail_count = two ? (uint32_t*)(ws + pl.off_tail) : nullptr;
   p.row_count = (uint32_t*)(ws + pl.off_count);
-  p.split_done = (uint32_t*)(ws + pl.off_done);
+  p.part_best = (unsigned long long*)(ws + pl.off_part_best);
+  p.part_vn = (float*)(ws + pl.off_part_vn);
+  p.part_stats = (float*)(ws + pl.off_part_stats);
+  p.split_pending = (uint32_t*)(ws + pl.off_pending);
   p.scratch_splits = a.decode_scratch_splits;
   p.resident = pl.resident;
+  p.one_launch = pl.one_launch;
   p.spin_limit = tuning().spin_limit.load();
   p.poll_sleep = tuning().poll_sleep.load();
   p.B = a.B; p.Hq = a.Hq; p.Hkv = a.Hkv; p.kv_len = a.kv_len; p.Tpad = pl.Tpad;
@@ -1144,10 +1370,71 @@ int launch_sdpa_decode(const kvx_sdpa_args& a, const kvx_h2o_args* hh, hipStream
   p.v_sb = a.v_stride_b; p.v_sh = a.v_stride_h; p.v_st = a.v_stride_t;
   p.o_sb = a.o_stride_b; p.o_sh = a.o_stride_h;
   p.qs_sb = a.qs_stride_b; p.qs_sh = a.qs_stride_h;
-  if (a.D == 128) return launch_d<128>(p, pl.G, a.kv_dtype, hh, st);
-  if (a.D == 64) return launch_d<64>(p, pl.G, a.kv_dtype, hh, st);
-  if (a.D == 256) return launch_d<256>(p, pl.G, a.kv_dtype, hh, st);
-  return set_error(KVX_ERR_UNSUPPORTED, "kvx_sdpa_decode: head size %d not in {64, 128, 256}", a.D);
+  return KVX_OK;
+}
+
+int launch_split(const DecodeParams& p, int D, int G, int kv, const kvx_h2o_args* hh, bool counters_clear, hipStream_t st) {
+  if (D == 128) return launch_d<128>(p, G, kv, hh, counters_clear, st);
+  if (D == 64) return launch_d<64>(p, G, kv, hh, counters_clear, st);
+  if (D == 256) return launch_d<256>(p, G, kv, hh, counters_clear, st);
+  return set_error(KVX_ERR_UNSUPPORTED, "kvx_sdpa_decode: head size %d not in {64, 128, 256}", D);
+}
+}  // namespace
+
+int launch_sdpa_decode(const kvx_sdpa_args& a, const kvx_h2o_args* hh, hipStream_t st) {
+  const Plan pl = make_plan(a, hh != nullptr);
+  DecodeParams p;
+  const int rc = decode_params(p, a, hh, pl);
+  return rc != KVX_OK ? rc : launch_split(p, a.D, pl.G, a.kv_dtype, hh, false, st);
+}
+
+// ---- a whole cache step of one token: the slot write clears the counters, the split kernel does the rest -----------
+
+static bool step_is_variant(const kvx_h2o_args& h) { return h.v_norm || h.q_errors; }
+static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
+
+size_t decode_step_workspace(const kvx_sdpa_args& a, const kvx_h2o_args& h) {
+  const Plan pl = make_plan(a, true);
+  if (pl.one_launch) return pl.total;
+  // logits through the scratch by plan: the calls this one stands for, one after the other
+  if (!step_is_variant(h)) return align256(h2o_workspace(h)) + pl.total;
+  kvx_sdpa_args aw = a;
+  aw.w = (float*)a.k;  // any pointer: score-sums are wanted
+  return align256(h2o_workspace(h)) + align256((size_t)a.B * a.Hkv * a.kv_len * 4) + make_plan(aw, false).total;
+}
+
+int launch_decode_step(const kvx_cache_write_args& w, const kvx_sdpa_args& a, const kvx_h2o_args& h, hipStream_t st) {
+  const Plan pl = make_plan(a, true);
+  KVX_REQUIRE(a.workspace && a.workspace_bytes >= decode_step_workspace(a, h), KVX_ERR_WORKSPACE,
+              "kvx_h2o_decode_step: workspace of %zu bytes needed, %zu given", decode_step_workspace(a, h), a.workspace_bytes);
+  if (!pl.one_launch) {
+    int rc = launch_cache_write(w, nullptr, st);
+    if (rc != KVX_OK) return rc;
+    kvx_sdpa_args a2 = a;
+    kvx_h2o_args h2 = h;
+    char* ws = (char*)a.workspace;
+    h2.workspace = ws;
+    h2.workspace_bytes = align256(h2o_workspace(h));
+    ws += h2.workspace_bytes;
+    if (step_is_variant(h)) {
+      a2.w = (float*)ws;
+      h2.w = a2.w;
+      ws += align256((size_t)a.B * a.Hkv * a.kv_len * 4);
+    }
+    a2.workspace = ws;
+    a2.workspace_bytes = (size_t)((char*)a.workspace + a.workspace_bytes - ws);
+    rc = launch_sdpa_decode(a2, step_is_variant(h) ? nullptr : &h2, st);
+    return rc != KVX_OK || !step_is_variant(h) ? rc : launch_h2o_update_select(h2, st);
+  }
+  DecodeParams p;
+  int rc = decode_params(p, a, &h, pl);
+  if (rc != KVX_OK) return rc;
+  const DecodeCounters counters{p.row_count, p.scratch_splits};
+  rc = launch_cache_write(w, &counters, st);
+  if (rc != KVX_OK) return rc;
+  rc = launch_split(p, a.D, pl.G, a.kv_dtype, &h, true, st);
+  if (rc != KVX_OK || !h.q_errors) return rc;
+  return launch_select_one(h, p.part_stats, p.num_splits, p.row_count + kSelected, p.part_best, st);
 }
 
 }  // namespace kvx

@@ -7,6 +7,7 @@ import torch
 
 from helpers import rel_err
 from keys_values_amd import _lib
+from keys_values_amd.attention import ops
 from keys_values_amd.kvcache.h2o import (H2OKVCache, KVCacheParams, QuantizedH2OKVCache, QuantizedVLengthH2OKVCache,
                                           VLengthH2OKVCache, create_kv_cache)
 from oracle import kvx_oracle as O
@@ -347,3 +348,38 @@ def test_replay_log(gpu, kwargs):
         cache.forward(q[:, :, :1].to(gpu), k[:, :, :1].to(gpu), v[:, :, :1].to(gpu), tokens[:, :1].to(gpu))
     with pytest.raises(ValueError):
         H2OKVCache(KVCacheParams(B, Hkv, L, D, Hq), replay_log_blocksize=0, device=gpu)
+
+
+@pytest.mark.parametrize("name,L,gp,normalize", [
+    ("h2o-default", 200, 0, False),                     # one split: no hand-over between workgroups
+    ("h2o-vlen-default", 777, 5, True),                 # several splits, the last one ragged
+    ("h2o-vlen-torch-quantized8", 4097, 0, False),
+    ("qh2o-torch-quantized8", 777, 7, False),
+    ("qh2o-vlen-torch-quantized4", 9001, 64, True),     # the choice spread over two workgroups a row
+])
+def test_fused_single_token_step_matches_the_separate_calls(gpu, decode_route, name, L, gp, normalize):
+    """A single-token step into a full cache is one call (slot write, attention, weighted score update, eviction choice),
+    whatever route the logits take. Against the same step as separate calls on a second cache in the same state. The
+    two add the score increments in different orders and form the normaliser of the V-norm weighting from differently
+    ordered fp32 sums over L terms: relative differences of a few 2^-24 sqrt(L)."""
+    B, Hq, Hkv, D, chunk = 2, 6, 2, 64, 32
+    q, k, v = _inputs(L, B, Hq, Hkv, L + chunk + 4, D, spread=True)
+    q, k, v = q.to(gpu), k.to(gpu), v.to(gpu)
+    fused, apart = (create_kv_cache(name, KVCacheParams(B, Hkv, L, D, Hq), max_chunk_size=chunk, grace_period=gp, normalize_scores=normalize, device=gpu)
+                    for _ in range(2))
+    for c in (fused, apart):
+        c.forward(q[:, :, :L], k[:, :, :L], v[:, :, :L])
+        c.forward(q[:, :, L : L + chunk], k[:, :, L : L + chunk], v[:, :, L : L + chunk])
+    for i in range(L + chunk, L + chunk + 4):
+        new = tuple(t[:, :, i : i + 1] for t in (q, k, v))
+        apart.set_next_positions(fused._next_index[:, :, :1])  # keep the two in step where scores tie in the last bits
+        out = fused.forward(*new)
+        apart._write(apart._next_index_for(1), new[1], new[2], apart.input_pos)
+        apart._input_pos += 1
+        o_ref, w, _ = ops.decode_core(new[0], apart.k, apart.v, apart.scale_factor, return_weights=True, quant=apart._quant_state(L))
+        apart._update(w, 1, select=1)
+        for x, y in ((fused.k, apart.k), (fused.v, apart.v), (fused.token_pos, apart.token_pos)):
+            assert torch.equal(x, y)
+        torch.testing.assert_close(out.view(B, Hq, D).float(), o_ref.float(), rtol=2e-2, atol=1e-3)
+        torch.testing.assert_close(fused.scores, apart.scores, rtol=1e-5, atol=1e-9)
+        assert torch.equal(fused._next_index, apart._next_index), f"step {i}"
