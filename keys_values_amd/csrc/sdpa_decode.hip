@@ -98,6 +98,28 @@ __device__ __forceinline__ float row_group_sum(float x) {
   return x;
 }
 
+// Exchanges between the 16-lane rows and the halves of a wavefront on the vector ALU (v_permlane16_swap,
+// v_permlane32_swap: the odd rows (the upper half) of the first operand change places with the even rows (the lower
+// half) of the second).
+__device__ __forceinline__ float dpp_ror8(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128, 0xf, 0xf, false));
+}
+// even rows: sum of a over the row pair, odd rows: sum of b over it
+__device__ __forceinline__ float swap_rows_add(float a, float b) {
+  const u32pair_t r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float sum_row_pairs(float v) { return swap_rows_add(v, v); }
+__device__ __forceinline__ float max_row_pairs(float v) {
+  const u32pair_t r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// lower half: sum of a over the two halves, upper half: sum of b
+__device__ __forceinline__ float swap_halves_add(float a, float b) {
+  const u32pair_t r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // Logits a workgroup holds in LDS: 64 KB where the merge buffer beside them is small enough for two workgroups
 // per compute unit (what the registers allow), else 32 KB.
 // Two workgroups per compute unit share 160 KB of LDS: the logits take what the merge buffer (4 G D floats) leaves of
@@ -159,52 +181,6 @@ __device__ __forceinline__ unsigned long long pair_bits(float lo, float hi) {
   return ((unsigned long long)__float_as_uint(hi) << 32) | __float_as_uint(lo);
 }
 
-// The row's outputs for the value pairs [e0, e1) of its Gr * D / 2: O = sum over the splits of part_o 2^(m - lse).
-// 16 threads share a pair, thread class j taking splits j, j + 16, ...; their sums are added in that order, so the
-// result does not depend on which workgroup takes which pairs. `buf`: 256 pairs of floats of LDS.
-template <int D, bool F16>
-__device__ __forceinline__ void merge_pairs(const DecodeParams& p, const int b, const int kvh, const float* lse_sh, const int e0, const int e1, f32x2_t* buf) {
-  const int tid = threadIdx.x, j = tid >> 4, c = tid & 15;
-  const int S = p.num_splits;
-  for (int base = e0; base < e1; base += 16) {
-    const int e = base + c;
-    f32x2_t acc = {0.0f, 0.0f};
-    if (e < e1) {
-      const int g = e / (D / 2);
-      const int64_t hd = (int64_t)b * p.Hq + kvh * p.Gr + g;
-      const unsigned long long* po = (const unsigned long long*)(p.part_o + hd * S * D) + e % (D / 2);
-      const float* ml = p.part_ml + hd * S * 2;
-      const float lse = lse_sh[g];
-      for (int s0 = j; s0 < S; s0 += 64) {  // four loads in flight
-        unsigned long long x[4];
-        float m[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int sp = min(s0 + 16 * u, S - 1);
-          x[u] = coherent_load(po + (int64_t)sp * (D / 2));
-          m[u] = coherent_load(ml + 2 * sp);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const float w = s0 + 16 * u < S ? fast_exp2(m[u] - lse) : 0.0f;
-          acc[0] += __uint_as_float((uint32_t)x[u]) * w;
-          acc[1] += __uint_as_float((uint32_t)(x[u] >> 32)) * w;
-        }
-      }
-    }
-    __syncthreads();
-    buf[j * 16 + c] = acc;
-    __syncthreads();
-    if (j == 0 && e < e1) {
-      f32x2_t t = buf[c];
-#pragma unroll
-      for (int i = 1; i < 16; ++i) t += buf[i * 16 + c];
-      const int g = e / (D / 2);
-      *(uint32_t*)(p.o + b * p.o_sb + (int64_t)(kvh * p.Gr + g) * p.o_sh + 2 * (e % (D / 2))) = pack_pair<F16>(t[0], t[1]);
-    }
-  }
-}
-
 // LDS of the part of a workgroup's life after its key loop.
 template <int G>
 struct FinishShared {
@@ -213,7 +189,7 @@ struct FinishShared {
   float vn[G];
   float red[WAVES][4];
   unsigned long long best[WAVES];
-  uint32_t ready, last, finished;
+  uint32_t ready, finished;
 };
 
 // The row's log-sum-exps (and z) from its splits' partials, in LDS for the whole workgroup. All splits have published.
@@ -244,6 +220,63 @@ __device__ __forceinline__ void row_state(const DecodeParams& p, const bool vnor
     sh.z = z / (float)p.Gr;
   }
   if (vnorm) __syncthreads();
+}
+
+// The row's outputs for the value pairs [e0, e1) of its Gr * D / 2: O = sum over the splits of part_o 2^(m - lse).
+// J threads share a pair, thread class j taking splits j, j + J, ...; their sums are added in that order, so the
+// result does not depend on which workgroup takes which pairs. J grows with the number of splits (a thread then has at
+// most four loads to make up to 64 splits: one memory latency a pass of 256 / J pairs). The loads of the first pass go out
+// before the row's log-sum-exps are worked out (STATE), which wait for memory themselves. `buf`: 256 pairs of floats of LDS.
+template <int D, bool F16, int G, bool STATE>
+__device__ __forceinline__ void merge_pairs(const DecodeParams& p, const bool vnorm, const int b, const int kvh, FinishShared<G>& sh, const int e0, const int e1,
+                                            f32x2_t* buf) {
+  const int tid = threadIdx.x, S = p.num_splits;
+  const int lj = S <= 4 ? 0 : S <= 8 ? 1 : S <= 16 ? 2 : S <= 32 ? 3 : 4, J = 1 << lj;
+  const int P = NTHREADS >> lj, j = tid >> (8 - lj), c = tid & (P - 1);
+  static_assert(NTHREADS == 256, "thread classes");
+  bool first = STATE;
+  for (int base = e0; base < e1 || first; base += P) {
+    const int e = base + c;
+    const bool live = e < e1;
+    const int ec = live ? e : 0, g = ec / (D / 2);
+    const int64_t hd = (int64_t)b * p.Hq + kvh * p.Gr + g;
+    const unsigned long long* po = (const unsigned long long*)(p.part_o + hd * S * D) + ec % (D / 2);
+    const float* ml = p.part_ml + hd * S * 2;
+    unsigned long long x[4];
+    float m[4];
+    auto load = [&](int s0) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int sp = min(s0 + J * u, S - 1);
+        x[u] = coherent_load(po + (int64_t)sp * (D / 2));
+        m[u] = coherent_load(ml + 2 * sp);
+      }
+    };
+    if (live) load(j);
+    if (first) row_state<G>(p, vnorm, b, kvh, sh);
+    first = false;
+    f32x2_t acc = {0.0f, 0.0f};
+    if (live) {
+      const float lse = sh.lse[g];
+      for (int s0 = j; s0 < S; s0 += 4 * J) {
+        if (s0 != j) load(s0);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const float w = s0 + J * u < S ? fast_exp2(m[u] - lse) : 0.0f;
+          acc[0] += __uint_as_float((uint32_t)x[u]) * w;
+          acc[1] += __uint_as_float((uint32_t)(x[u] >> 32)) * w;
+        }
+      }
+    }
+    if (J > 1) {  // the same for every thread
+      __syncthreads();
+      buf[tid] = acc;
+      __syncthreads();
+      for (int i = 1; i < J; ++i) acc += buf[i * P + c];  // meaningful in class 0
+    }
+    if (j == 0 && live)
+      *(uint32_t*)(p.o + b * p.o_sb + (int64_t)(kvh * p.Gr + g) * p.o_sh + 2 * (e % (D / 2))) = pack_pair<F16>(acc[0], acc[1]);
+  }
 }
 
 // Weights of the keys [k0, k1) of split `split`, logits(k, x) giving the logits of key k: W, and in the fused H2O form
@@ -334,11 +367,10 @@ __device__ __forceinline__ void weigh_split(const DecodeParams& p, const kvx_h2o
 // What a split does once its wavefronts have left their partial results in LDS (red: unnormalised outputs, rml:
 // maximum and sum, per wavefront and head).
 //
-// One launch does the whole step. The split publishes its partial and counts itself in. Without weights the split
-// that arrives last combines the row's outputs. With weights every split waits (boundedly) for the row's others, then
-// takes an equal share of the row's outputs and turns its own logits (lgbuf, [key][head]) into weights; a split whose
-// wait ran out puts its logits into the scratch instead. The split that finishes last makes up what such splits left
-// undone and publishes the row's slot. A second launch for the outputs and a third to reset the counters cost 4 to 8 us
+// One launch does the whole step. The split publishes its partial, counts itself in and waits (boundedly) for the row's
+// others; then it takes an equal share of the row's outputs and, with weights wanted, turns its own logits (lgbuf,
+// [key][head]) into weights. A split whose wait ran out puts its logits into the scratch instead. The split that finishes
+// last makes up what such splits left undone and publishes the row's slot. A second launch for the outputs and a third to reset the counters cost 4 to 8 us
 // of every step, a third of a step over 4096 slots.
 template <int D, int G, int LGK, int CHUNK, bool F16>
 __device__ __forceinline__ void finish_split(const DecodeParams& p, const kvx_h2o_args& hh, const int h2o, const float* lgbuf,
@@ -405,10 +437,10 @@ __device__ __forceinline__ void finish_split(const DecodeParams& p, const kvx_h2
   __syncthreads();
   if (tid == 0) {
     const bool last = S == 1 || __hip_atomic_fetch_add(cnt + kArrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)S - 1u;
-    uint32_t ok = 0;
-    if (lgrow) {
+    uint32_t ok = last && p.spin_limit > 0;
+    if (!ok) {
       for (int spin = 0; spin < p.spin_limit; ++spin) {  // bounded: a workgroup that gives up takes the scratch route
-        if (S == 1 || coherent_load(cnt + kArrived) >= (uint32_t)S) {
+        if (coherent_load(cnt + kArrived) >= (uint32_t)S) {
           ok = 1;
           break;
         }
@@ -417,26 +449,18 @@ __device__ __forceinline__ void finish_split(const DecodeParams& p, const kvx_h2
         for (int z = 0; z < pause; ++z) __builtin_amdgcn_s_sleep(8);
       }
     }
-    sh.last = last;
     sh.ready = ok;
   }
   __syncthreads();
-  if (!lgrow) {
-    if (!sh.last) return;
-    row_state<G>(p, false, b, kvh, sh);
-    merge_pairs<D, F16>(p, b, kvh, sh.lse, 0, E, buf);
-    if (p.lse_out && tid < p.Gr) p.lse_out[(int64_t)b * p.Hq + kvh * p.Gr + tid] = sh.lse[tid];
-    return;
-  }
   const bool ready = sh.ready;
   if (ready) {
-    row_state<G>(p, vnorm, b, kvh, sh);
-    merge_pairs<D, F16>(p, b, kvh, sh.lse, (int)((int64_t)E * split / S), (int)((int64_t)E * (split + 1) / S), buf);
-    weigh_split<G>(p, hh, h2o, b, kvh, sh, split, k_begin, k_end, [&](int k, float (&x)[G]) {
+    merge_pairs<D, F16, G, true>(p, vnorm, b, kvh, sh, E * split / S, E * (split + 1) / S, buf);
+    if (lgrow)
+      weigh_split<G>(p, hh, h2o, b, kvh, sh, split, k_begin, k_end, [&](int k, float (&x)[G]) {
 #pragma unroll
-      for (int g = 0; g < G; ++g) x[g] = lgbuf[(k - k_begin) * G + g];
-    });
-  } else {
+        for (int g = 0; g < G; ++g) x[g] = lgbuf[(k - k_begin) * G + g];
+      });
+  } else if (lgrow) {
     const int n = (k_end - k_begin) * G;
     float* dst = lgrow + (int64_t)k_begin * G;
     for (int i = tid; i < n; i += NTHREADS) coherent_store(dst + i, lgbuf[i]);
@@ -458,7 +482,8 @@ __device__ __forceinline__ void finish_split(const DecodeParams& p, const kvx_h2
   if (finished >= kPending)
     for (int sp = 0; sp < S; ++sp) {
       if (!coherent_load(p.split_pending + (int64_t)row * S + sp)) continue;  // the same for every thread
-      merge_pairs<D, F16>(p, b, kvh, sh.lse, (int)((int64_t)E * sp / S), (int)((int64_t)E * (sp + 1) / S), buf);
+      merge_pairs<D, F16, G, false>(p, vnorm, b, kvh, sh, E * sp / S, E * (sp + 1) / S, buf);
+      if (!lgrow) continue;
       const int k0 = sp * p.keys_per_split, k1 = min(k0 + p.keys_per_split, p.kv_len);
       weigh_split<G>(p, hh, h2o, b, kvh, sh, sp, k0, k1, [&](int k, float (&x)[G]) {
 #pragma unroll
@@ -656,21 +681,34 @@ __global__ __launch_bounds__(NTHREADS) void decode_split_kernel(const DecodePara
   }
 
   // ---- merge the RPI row groups of the wavefront, then the wavefronts, into one partial -----------
+  // Sums over the groups by swapping register halves between lanes (reduce-scatter): at each level a lane keeps half of
+  // its values, so 8 values take 8 swaps and adds instead of 16 shuffles and adds. (This code runs once per split,
+  // from a cold instruction cache; with shuffles it took 3.2 us of a 15 us split of 256 keys.)
 #pragma unroll
   for (int g = 0; g < G; ++g) {
     float M = m_run[g];
-#pragma unroll
-    for (int off = LPR; off < 64; off <<= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+    if constexpr (LPR == 8) M = fmaxf(M, dpp_ror8(M));
+    if constexpr (LPR <= 16) M = max_row_pairs(M);
+    M = max_halves(M);
     const float sc = fast_exp2(m_run[g] - M);
     float l = l_run[g] * sc;
-#pragma unroll
-    for (int off = LPR; off < 64; off <<= 1) l += __shfl_xor(l, off, 64);
+    if constexpr (LPR == 8) l += dpp_ror8(l);
+    if constexpr (LPR <= 16) l = sum_row_pairs(l);
+    l = sum_halves(l);
+    float x[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      float x = acc[g][e] * sc;
+      x[e] = acc[g][e] * sc;
+      if constexpr (LPR == 8) x[e] += dpp_ror8(x[e]);  // the two groups of a 16-lane row
+    }
+    float y[4];  // lanes 0-31: values 0 .. 3, lanes 32-63: values 4 .. 7
 #pragma unroll
-      for (int off = LPR; off < 64; off <<= 1) x += __shfl_xor(x, off, 64);
-      if (lane < LPR) red[wave][g][lane * 8 + e] = x;
+    for (int e = 0; e < 4; ++e) y[e] = swap_halves_add(x[e], x[e + 4]);
+    if constexpr (LPR <= 16) {  // even 16-lane rows: the first two of these, odd rows: the last two
+      const f32x2_t z = {swap_rows_add(y[0], y[2]), swap_rows_add(y[1], y[3])};
+      if (LPR == 16 || (lane & 8) == 0) *(f32x2_t*)&red[wave][g][8 * dc + 4 * (lane >> 5) + 2 * ((lane >> 4) & 1)] = z;
+    } else {
+      *(f32x4_t*)&red[wave][g][8 * dc + 4 * (lane >> 5)] = f32x4_t{y[0], y[1], y[2], y[3]};
     }
     if (lane == 0) {
       rml[wave][g][0] = M;
@@ -1200,24 +1238,25 @@ Plan make_plan(const kvx_sdpa_args& a, bool fused_h2o) {
   Plan pl;
   const int gr = a.Hq / a.Hkv;
   pl.G = gr <= 1 ? 1 : (gr <= 2 ? 2 : (gr <= 4 ? 4 : (gr <= 8 ? 8 : 16)));
-  // One full round of workgroups (two per compute unit, what the registers allow) over the whole grid:
-  // rows * kv_len / (2 CUs) keys per split, at least 256; with weights at most what the LDS holds of a split's
-  // logits (a split that waits for its row holds its place, so the device then runs several rounds) and, LDS
-  // permitting, at least kv_len / 128 (2 rows of 65536 keys: 45 us with 128 splits waiting for each other, 56 with 256).
-  // Measured, with weights: 8 x 8 rows of 131072 keys, 4 rounds of 4096 keys beat 8 rounds of 2048 by 2 %; 8 rows of
-  // 262144 keys take 182 us in one round of 4096 keys and 265 in four of 1024. Without weights: 32 rows of 262144
-  // keys 631 us in 16 splits, 658 in 128; 8 rows of 16384 keys 22 us in 32 splits, 26 in 16 of 1024.
+  // Keys per split: one workgroup per compute unit over the whole grid, at least 128 keys (a wavefront's steps take
+  // about 1 us each; shorter splits only add partials to combine), at least what keeps a row to 128 splits (to 64 below
+  // 16384 keys: the splits of a row wait for each other), and with weights at most what the LDS holds of a split's logits
+  // (longer rows of many heads then run several rounds). Two workgroups per compute unit, as many as fit, were worse
+  // wherever one round covers the call. Measured, us, two -> one per compute unit: 8 rows of 16384 keys 25.0 -> 21.4, of
+  // 65536 keys 55 -> 50, 32 rows of 16384 keys 52.6 -> 49.8; 8-bit codes 8 rows of 32768 keys 29 -> 25, 32 rows of
+  // 16384 keys 39 -> 37; head size 256, 8-bit codes, 32 rows of 8192 keys 49 -> 40; 8 rows of 1024 keys, 256 -> 128 keys
+  // a split 13.1 -> 11.8. 64 rows of 32768 keys take 170 in two rounds of 4096 keys, 183 in splits of 1024.
   const bool weights = a.w || fused_h2o;
   const int allow_resident = weights ? tuning().resident.load() : 0;
   const int lgk = logit_floats(pl.G, a.D) / pl.G;
   int splits = a.num_splits;
   if (splits <= 0) {
-    int64_t keys = (int64_t)a.B * a.Hkv * a.kv_len / (2 * num_cus());
-    if (keys < 256) keys = 256;
-    if (allow_resident) {  // at most 128 splits wait for each other, unless the LDS limit asks for more
-      if (keys < (a.kv_len + 127) / 128) keys = (a.kv_len + 127) / 128;
-      if (keys > lgk) keys = lgk;
-    }
+    int64_t keys = (int64_t)a.B * a.Hkv * a.kv_len / num_cus();
+    keys = max(keys, (int64_t)max(max(128, min(256, a.kv_len / 64)), (a.kv_len + 127) / 128));
+    // codes are bound by the vector arithmetic of their dequantisation: long splits gain from a second workgroup a unit
+    // (32 rows of 16384 keys, 4 bits: 33 us against 36)
+    if (!kv_is_plain(a.kv_dtype) && a.D <= 128 && keys > 1024) keys = max((int64_t)1024, keys / 2);
+    if (allow_resident && keys > lgk) keys = lgk;
     splits = (int)((a.kv_len + keys - 1) / keys);
   }
   splits = max(1, min(splits, 512));
@@ -1226,8 +1265,11 @@ Plan make_plan(const kvx_sdpa_args& a, bool fused_h2o) {
   pl.keys_per_split = kps;
   pl.num_splits = (a.kv_len + kps - 1) / kps;
   pl.Tpad = ((a.kv_len + 63) / 64) * 64;
-  pl.resident = allow_resident && kps <= lgk;
-  pl.one_launch = pl.resident || !weights;
+  // The splits of a row wait for each other: they have to fit the device side by side (workgroups are dispatched in index
+  // order, a row's splits are neighbours). At head size 256 a compute unit holds one workgroup, else two.
+  const bool side_by_side = pl.num_splits <= (a.D > 128 ? 1 : 2) * num_cus();
+  pl.resident = allow_resident && kps <= lgk && side_by_side;
+  pl.one_launch = side_by_side && (pl.resident || !weights);
   size_t off = 0;
   auto take = [&off](size_t bytes) {  // 16-byte aligned pieces
     const size_t at = off;
@@ -1243,7 +1285,7 @@ Plan make_plan(const kvx_sdpa_args& a, bool fused_h2o) {
   pl.off_part_best = take(fused_one ? rows * max(pl.num_splits, select_one_parts(a.kv_len)) * 8 : 0);
   pl.off_part_vn = take(fused_one ? head_splits * 4 : 0);
   pl.off_part_stats = take(fused_one ? row_splits * 16 : 0);
-  pl.off_pending = take(pl.resident ? row_splits * 4 : 0);
+  pl.off_pending = take(pl.one_launch ? row_splits * 4 : 0);
   pl.off_best = take(fused_two ? rows * 8 : 0);
   pl.off_tail = take(fused_two ? 8 : 0);
   off = (off + 255) & ~(size_t)255;
@@ -1255,7 +1297,7 @@ Plan make_plan(const kvx_sdpa_args& a, bool fused_h2o) {
 template <int D, bool F16, int G>
 int launch_tail(const DecodeParams& p, const kvx_h2o_args* hh, hipStream_t st) {
   const int merge_jobs = p.B * p.Hq, wx = (p.kv_len + 4095) / 4096;
-  const int weight_jobs = wx * p.Hkv * p.B;
+  const int weight_jobs = hh || p.w ? wx * p.Hkv * p.B : 0;
   const dim3 grid(merge_jobs + weight_jobs), block(4 * D);
   const kvx_h2o_args h2 = hh ? *hh : kvx_h2o_args{};
   if (hh) hipLaunchKernelGGL((decode_tail_kernel<D, F16, G, 2>), grid, block, 0, st, p, h2, merge_jobs, wx);
