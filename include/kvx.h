@@ -101,6 +101,12 @@ typedef struct kvx_sdpa_args {
    * instead of staying on the chip -- all of them when the splits are too long for the LDS or that form is switched
    * off, else those whose bounded wait for their row ran out (normally 0; such a call is about 15 % slower). */
   uint32_t* decode_scratch_splits;
+
+  /* kvx_sdpa_prefill* over a quantised store: 1 = dequantise inside the attention kernel whatever the size of the chunk;
+   * 0 = where it is faster, dequantise the store once into the workspace (kvx_sdpa_prefill_workspace_bytes then counts
+   * 2 * B * Hkv * kv_len * D 16-bit values) and attend over the copy. Same results. A workspace too small for the copy
+   * but not for the rest means the same as 1. */
+  int32_t fused_dequant;
 } kvx_sdpa_args;
 
 /* ---- library ------------------------------------------------------------------------------- */

@@ -40,6 +40,7 @@ class SdpaArgs(ctypes.Structure):
         ("lse", c_void_p), ("w", c_void_p),
         ("workspace", c_void_p), ("workspace_bytes", c_size_t),
         ("decode_scratch_splits", c_void_p),
+        ("fused_dequant", c_int32),
     ]
 
 

@@ -117,7 +117,7 @@ def prefill_core(
     Returns ``(out, weights, lse)``: ``out`` is (B, q, Hq, D) if ``output_transposed`` (the layout
     of the reference extension) else (B, Hq, q, D); ``weights`` fp32 (B, Hkv, T) summed over queries
     and averaged over the group; ``lse`` fp32 (B, q, Hq) in base 2."""
-    return _lib.host().prefill(query, key, value, scale, input_pos, token_positions, return_weights, return_lse, output_transposed, quant, num_splits)
+    return _lib.host().prefill(query, key, value, scale, input_pos, token_positions, return_weights, return_lse, output_transposed, quant, num_splits, False)
 
 
 def score_sum_core(query, key, lse, scale, input_pos, token_positions=None, quant: Optional[QuantState] = None):

@@ -309,9 +309,9 @@ AttnOut run_prefill(kvx_sdpa_args& a, const Launch& L, at::ScalarType type, bool
 }
 
 // prefill(query, key, value, scale, input_pos, token_positions, return_weights, return_lse, output_transposed, quant,
-// num_splits) -> (out, weights or None, lse or None)
+// num_splits, fused_dequant) -> (out, weights or None, lse or None)
 PyObject* prefill(PyObject* const* args, Py_ssize_t n) {
-  require_args(n, 11, "prefill");
+  require_args(n, 12, "prefill");
   const at::Tensor &q = tensor(args[0], "query"), &k = tensor(args[1], "key"), &v = tensor(args[2], "value");
   for (const at::Tensor* t : {&q, &k, &v}) require_gpu(*t);
   check_bhtd("query", q);
@@ -329,6 +329,7 @@ PyObject* prefill(PyObject* const* args, Py_ssize_t n) {
   kvx_sdpa_args a = sdpa_args(q, k, &v, real(args[3]), integer(args[4]), qs ? &*qs : nullptr, integer(args[10]));
   at::Tensor keep;
   set_positions(a, opt_tensor(args[5], "token_positions"), keep);
+  a.fused_dequant = truth(args[11]);
   const bool want_lse = truth(args[7]);
   AttnOut r = run_prefill(a, L, q.scalar_type(), truth(args[6]), want_lse, truth(args[8]));
   return three(r.out, r.w, want_lse ? r.lse : at::Tensor());

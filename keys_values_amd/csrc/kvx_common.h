@@ -56,6 +56,8 @@ int launch_quantize_rows(const void* x, int64_t x_row_stride, int64_t rows, int 
                          int32_t* zp, hipStream_t st);
 int launch_dequantize_rows(const uint8_t* codes, const float* scale, const int32_t* zp, int64_t rows, int D, int bits, bool f16, void* out,
                            int64_t out_row_stride, hipStream_t st);
+// K and V of a quantised store (8 or 4 bits, any strides) to dense rows: (B, Hkv, kv_len, D) of K at out, V behind it
+int launch_dequantize_kv(const kvx_sdpa_args& a, void* out, hipStream_t st);
 int launch_quantize_blocks(const kvx_block_quant_args& a, hipStream_t st);
 int launch_dequantize_blocks(const kvx_block_quant_args& a, hipStream_t st);
 // Counters that a single-token step needs at zero when its split kernel starts: kDecodeCounters 32-bit words at the head

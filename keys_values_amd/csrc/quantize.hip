@@ -344,6 +344,48 @@ __global__ __launch_bounds__(NTHREADS) void dequantize_rows4_kernel(const RowRun
   }
 }
 
+// K (blockIdx.z = 0) and V (1) of an attention call's quantised store, one (batch, KV head) pair per blockIdx.y, to dense
+// rows. A lane owns 8 values of ROWS_PER_THREAD rows, as above; the codes' rows lie wherever the strides say.
+template <int D, int KV>
+__global__ __launch_bounds__(NTHREADS) void dequantize_kv_kernel(const kvx_sdpa_args a, uint16_t* __restrict__ out) {
+  constexpr bool U4 = kv_is_u4(KV), F16 = kv_elem_f16(KV);
+  constexpr int LPR = U4 ? D / 16 : D / 8;  // lanes per row: 8 bytes of codes each
+  constexpr int RPB = NTHREADS / LPR;
+  const bool is_v = blockIdx.z != 0;
+  const int b = blockIdx.y / a.Hkv, h = blockIdx.y % a.Hkv;
+  const int64_t sb = is_v ? a.v_stride_b : a.k_stride_b, sh = is_v ? a.v_stride_h : a.k_stride_h, stt = is_v ? a.v_stride_t : a.k_stride_t;
+  const uint8_t* __restrict__ codes = (const uint8_t*)(is_v ? a.v : a.k) + b * sb + h * sh;
+  const int64_t so = b * a.qs_stride_b + h * a.qs_stride_h;
+  const float* __restrict__ scale = (is_v ? a.v_scale : a.k_scale) + so;
+  const int32_t* __restrict__ zp = (is_v ? a.v_zp : a.k_zp) + so;
+  uint16_t* __restrict__ o = out + ((int64_t)blockIdx.z * a.B * a.Hkv + blockIdx.y) * a.kv_len * D;
+  const int col = threadIdx.x % LPR;
+  const int row0 = blockIdx.x * (RPB * ROWS_PER_THREAD) + threadIdx.x / LPR;
+  u32x2_t c[ROWS_PER_THREAD];
+  float s[ROWS_PER_THREAD];
+  int32_t z[ROWS_PER_THREAD];
+#pragma unroll
+  for (int i = 0; i < ROWS_PER_THREAD; ++i) {
+    const int r = min(row0 + i * RPB, a.kv_len - 1);
+    c[i] = *(const u32x2_t*)(codes + r * stt + col * 8);
+    s[i] = scale[r];
+    z[i] = zp[r];
+  }
+#pragma unroll
+  for (int i = 0; i < ROWS_PER_THREAD; ++i) {
+    const int r = row0 + i * RPB;
+    if (r >= a.kv_len) continue;
+    uint16_t* w = o + (int64_t)r * D + col * 8;
+    if constexpr (U4) {
+      const u32x2_t hi = u4_codes(c[i], 4), lo = u4_codes(c[i], 0);
+      *(u32x4_t*)w = dequant_words<F16>(hi[0], hi[1], z[i], s[i]);
+      *(u32x4_t*)(w + D / 2) = dequant_words<F16>(lo[0], lo[1], z[i], s[i]);
+    } else {
+      *(u32x4_t*)w = dequant_words<F16>(c[i][0], c[i][1], z[i], s[i]);
+    }
+  }
+}
+
 // ---- general blocks (several segments per block, 8 or 4 bits) -------------------------------------------------------
 //
 // A block of n chunks of 8 values (n is even: D is a multiple of 16) is held by LPB lanes, lane l taking the chunk pairs
@@ -680,6 +722,24 @@ int launch_quantize_rows(const void* x, int64_t x_row_stride, int64_t rows, int 
 int launch_dequantize_rows(const uint8_t* codes, const float* scale, const int32_t* zp, int64_t rows, int D, int bits, bool f16,
                            void* out, int64_t out_row_stride, hipStream_t st) {
   return launch_rows(RowRuns{(uint16_t*)out, out_row_stride, 0, (uint8_t*)codes, 0, (float*)scale, (int32_t*)zp, 0, rows, 1}, D, bits, f16, false, st);
+}
+
+template <int D>
+int launch_dequantize_kv_d(const kvx_sdpa_args& a, void* out, hipStream_t st) {
+  const int lpr = kv_is_u4(a.kv_dtype) ? D / 16 : D / 8, rpb = NTHREADS / lpr * ROWS_PER_THREAD;
+  const dim3 grid((a.kv_len + rpb - 1) / rpb, a.B * a.Hkv, 2);
+  switch (a.kv_dtype) {
+    case KVX_KV_U8: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U8>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out); break;
+    case KVX_KV_U4: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U4>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out); break;
+    case KVX_KV_U8_F16: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U8_F16>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out); break;
+    default: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U4_F16>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out); break;
+  }
+  KVX_HIP(hipGetLastError());
+  return KVX_OK;
+}
+
+int launch_dequantize_kv(const kvx_sdpa_args& a, void* out, hipStream_t st) {
+  return a.D == 256 ? launch_dequantize_kv_d<256>(a, out, st) : a.D == 128 ? launch_dequantize_kv_d<128>(a, out, st) : launch_dequantize_kv_d<64>(a, out, st);
 }
 
 template <int BITS, bool F16, int LPB, int NP>

@@ -287,7 +287,9 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
   const int h = lane >> 5;  // which half of each 8-wide k group / which 4-row group of the MFMA output
 
   const int group = blockIdx.x;  // b * Hkv + kvh: fastest-varying so that a KV head stays on one XCD
-  const int mblk = blockIdx.y;
+  // slots in position order (a causal first chunk): the later rows see more tiles; they start first, so that the short
+  // ones fill up the end (a first chunk of 8192 tokens, 32 heads of 128: 597 -> 543 us)
+  const int mblk = p.tp ? blockIdx.y : gridDim.y - 1 - blockIdx.y;
   const int split = blockIdx.z;
   const int b = group / p.Hkv;
   const int kvh = group % p.Hkv;
@@ -603,31 +605,66 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
   }
 }
 
-// Combine the per-split partials of a row: one workgroup of D/4 threads... one thread per 4 d.
-template <int D, bool F16>
+// Combine the per-split partials of a row: D / 4 threads a row, each four values, times SC split classes that take
+// splits j, j + SC, ... and are added through LDS. Bound by HBM (every partial is read once) where there are many rows;
+// with few rows (32 queries over 32768 keys: 1024 rows of 32 splits) a thread's walk over the splits was the time, a memory
+// latency per split and 15 us of a 46 us call: four loads in flight and SC classes make it about two latencies.
+template <int D, bool F16, int SC>
 __global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(const PrefillParams p) {
-  constexpr int TPR = D / 4;              // threads per row
-  constexpr int ROWS = 256 / TPR;         // rows per workgroup
+  constexpr int TPR = D / 4;                // threads per row and split class
+  constexpr int ROWS = 256 / (TPR * SC);    // rows per workgroup
+  static_assert(ROWS >= 1, "a row's threads fit a workgroup");
+  __shared__ f32x4_t red_o[SC > 1 ? 256 : 1];
+  __shared__ float red_l[SC > 1 ? 256 : 1];
+  const int S = p.num_splits;
   const int64_t total_rows = (int64_t)p.B * p.Hkv * p.R;
-  const int64_t grow = (int64_t)blockIdx.x * ROWS + threadIdx.x / TPR;
-  if (grow >= total_rows) return;
-  const int dq = threadIdx.x % TPR;
+  const int64_t grow = (int64_t)blockIdx.x * ROWS + threadIdx.x / (TPR * SC);
+  const bool live = grow < total_rows;
+  const int64_t growc = live ? grow : total_rows - 1;
+  const int dq = threadIdx.x % TPR, j = (threadIdx.x / TPR) % SC;
+  const f32x2_t* ml = (const f32x2_t*)p.part_ml + growc;  // (maximum, sum) of split s at s * total_rows
+  const float* po = p.part_o + growc * D + dq * 4;
+  float M = -INFINITY;
+  for (int s0 = 0; s0 < S; s0 += 4) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) M = fmaxf(M, ml[(int64_t)min(s0 + u, S - 1) * total_rows][0]);
+  }
+  const float Mu = (M == -INFINITY) ? 0.0f : M;
+  float L = 0.0f;
+  f32x4_t acc = {0, 0, 0, 0};
+  for (int s0 = j; s0 < S; s0 += 4 * SC) {
+    f32x2_t m[4];
+    f32x4_t x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t at = (int64_t)min(s0 + u * SC, S - 1) * total_rows;
+      m[u] = ml[at];
+      x[u] = *(const f32x4_t*)(po + at * D);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (s0 + u * SC < S) {
+        const float w = fast_exp2(m[u][0] - Mu);
+        L += m[u][1] * w;
+        acc += x[u] * w;
+      }
+  }
+  if constexpr (SC > 1) {
+    red_o[threadIdx.x] = acc;
+    red_l[threadIdx.x] = L;
+    __syncthreads();
+    if (j != 0) return;
+#pragma unroll
+    for (int i = 1; i < SC; ++i) {
+      acc += red_o[threadIdx.x + i * TPR];
+      L += red_l[threadIdx.x + i * TPR];
+    }
+  }
+  if (!live) return;
   const int group = (int)(grow / p.R);
   const int row = (int)(grow % p.R);
   const int b = group / p.Hkv, kvh = group % p.Hkv;
   const int qi = row / p.G, g = row % p.G;
-  float M = -INFINITY;
-  for (int s = 0; s < p.num_splits; ++s) M = fmaxf(M, p.part_ml[((int64_t)s * total_rows + grow) * 2]);
-  const float Mu = (M == -INFINITY) ? 0.0f : M;
-  float L = 0.0f;
-  f32x4_t acc = {0, 0, 0, 0};
-  for (int s = 0; s < p.num_splits; ++s) {
-    const int64_t pr = (int64_t)s * total_rows + grow;
-    const float w = fast_exp2(p.part_ml[pr * 2] - Mu);
-    L += p.part_ml[pr * 2 + 1] * w;
-    const f32x4_t x = *(const f32x4_t*)(p.part_o + pr * D + dq * 4);
-    acc += x * w;
-  }
   const float inv = L > 0.0f ? 1.0f / L : 0.0f;
   uint16_t* op = p.o + b * p.o_sb + (int64_t)(kvh * p.G + g) * p.o_sh + (int64_t)qi * p.o_st + dq * 4;
   u32x2_t w2;
@@ -637,15 +674,35 @@ __global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(const PrefillPa
   if (p.lse && dq == 0) p.lse[((int64_t)b * p.q_len + qi) * p.Hq + kvh * p.G + g] = Mu + fast_log2(L);
 }
 
+// The number of KV splits with the least estimated time: c workgroups share a compute unit, one after the other or side by
+// side, and each walks its split's tiles; more splits balance the device better and shorten the walk, but every partial
+// is written, read again and combined by one more launch. The constants are measured (ns): a tile of 64 keys for a workgroup
+// that has its compute unit to itself is 700 / 1130 / 2050 at head size 64 / 128 / 256, two side by side gain 20 %; the
+// combining launch takes 2 us and reads its partials at 4 TB/s. A full count of rounds with a nearly empty last one is what
+// the rule avoids: 2 x 4 heads, 333 queries x 7, 5001 keys: 4 splits (608 workgroups, three to a unit) 83 us, 3 splits
+// (456, two) 63 us; 4 x 4 heads, 541 x 7 over 5238: 2 splits 177, none 152.
 int pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
   if (a.num_splits > 0) return min(a.num_splits, num_tiles);
-  // Aim for one resident round of workgroups (2 per compute unit, 1 with the uint8 cache): more
-  // splits only add partials to write, merge and re-read. At least 8 key tiles per split.
-  const int64_t base = (int64_t)a.B * a.Hkv * m_blocks;
-  const int target = ((kv_is_plain(a.kv_dtype) && a.D <= 128) ? 2 : 1) * num_cus();
-  int s = (int)((target + base - 1) / base);
-  s = max(1, min(s, num_tiles / 8));
-  return max(1, min(s, 64));
+  const int64_t base = (int64_t)a.B * a.Hkv * m_blocks, cus = num_cus();
+  const bool plain = kv_is_plain(a.kv_dtype);
+  int64_t tile_ns = a.D == 64 ? 700 : a.D == 128 ? 1130 : 2050;
+  if (!plain) tile_ns = a.D == 256 ? 5500 : 2 * tile_ns + 300;  // 256 rows a workgroup, codes to dequantise (at 256: 128 rows)
+  const bool pairs = plain && a.D <= 128;
+  const int64_t rows = (int64_t)a.B * a.Hq * a.q_len;
+  int best = 1;
+  int64_t best_ns = INT64_MAX;
+  for (int s = 1; s <= min(64, num_tiles); ++s) {
+    const int tps = (num_tiles + s - 1) / s;
+    if ((num_tiles + tps - 1) / tps != s) continue;
+    const int64_t c = (base * s + cus - 1) / cus;
+    const int64_t walk = c * tps * (pairs && c > 1 ? tile_ns * 4 / 5 : tile_ns);
+    const int64_t merge = s == 1 ? 0 : 2000 + s * rows * (a.D * 4 + 8) / 4000;
+    if (walk + merge < best_ns) {
+      best_ns = walk + merge;
+      best = s;
+    }
+  }
+  return best;
 }
 
 void fill_params(PrefillParams& p, const kvx_sdpa_args& a) {
@@ -696,9 +753,15 @@ int launch_t(PrefillParams& p, hipStream_t st) {
   hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
   KVX_HIP(hipGetLastError());
   if (p.num_splits > 1) {
-    constexpr int ROWS = 256 / (D / 4);
     const int64_t total_rows = (int64_t)p.B * p.Hkv * p.R;
-    hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kv_elem_f16(KV)>), dim3((unsigned)((total_rows + ROWS - 1) / ROWS)), dim3(256), 0, st, p);
+    auto merge = [&](auto sc_tag) {
+      constexpr int SC = decltype(sc_tag)::value, ROWS = 256 / (D / 4 * SC);
+      hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kv_elem_f16(KV), SC>), dim3((unsigned)((total_rows + ROWS - 1) / ROWS)), dim3(256), 0, st, p);
+    };
+    // split classes while a walk is longer than four splits and the rows alone leave the device short of threads
+    constexpr int MAX_SC = 256 / (D / 4) < 8 ? 256 / (D / 4) : 8;
+    if (p.num_splits <= 4 || total_rows * (D / 4) >= (int64_t)num_cus() * 256) merge(std::integral_constant<int, 1>{});
+    else merge(std::integral_constant<int, MAX_SC>{});
     KVX_HIP(hipGetLastError());
   }
   return KVX_OK;
@@ -706,16 +769,55 @@ int launch_t(PrefillParams& p, hipStream_t st) {
 
 }  // namespace
 
+// Whether a call over a quantised store first dequantises the store into the workspace and then attends over plain rows.
+// Every workgroup of the attention kernel walks the whole store (of its split) and the dequantising one pays its vector work
+// each time, once per 256 rows; the copy pays it once, for one write and one more read of the 16-bit rows. Measured on
+// 65536 x 8 rows of 128, 1024 x 4 queries: 1298 us against 75 + 1048; the lines meet near 2048 rows. At head size 256 the
+// dequantising kernel runs 128 rows a workgroup out of its registers (4 x 4 heads, 541 x 7 queries over 5238: 890 us against
+// 26 + 340), and the copy pays from the second workgroup on.
+static bool wants_copy(const kvx_sdpa_args& a) {
+  if (kv_is_plain(a.kv_dtype) || a.fused_dequant || (int64_t)a.B * a.Hkv > 65535) return false;  // pairs are a grid dimension of 16 bits
+  const int64_t rows = (int64_t)a.q_len * (a.Hq / a.Hkv);
+  return a.D == 256 ? rows > 128 : rows >= 2048;
+}
+static size_t copy_bytes(const kvx_sdpa_args& a) { return ((size_t)2 * a.B * a.Hkv * a.kv_len * a.D * 2 + 255) / 256 * 256; }
+// the call on the dequantised rows at `rows` (K, then V, each (B, Hkv, kv_len, D))
+static kvx_sdpa_args on_copy(const kvx_sdpa_args& a, void* rows) {
+  kvx_sdpa_args c = a;
+  c.kv_dtype = kv_elem_f16(a.kv_dtype) ? KVX_KV_F16 : KVX_KV_BF16;
+  c.k = rows;
+  c.v = (char*)rows + (size_t)a.B * a.Hkv * a.kv_len * a.D * 2;
+  c.k_stride_t = c.v_stride_t = a.D;
+  c.k_stride_h = c.v_stride_h = (int64_t)a.kv_len * a.D;
+  c.k_stride_b = c.v_stride_b = (int64_t)a.Hkv * a.kv_len * a.D;
+  return c;
+}
+
 size_t sdpa_prefill_workspace(const kvx_sdpa_args& a) {
   PrefillParams p;
-  fill_params(p, a);
+  const bool copy = wants_copy(a);
+  const kvx_sdpa_args c = copy ? on_copy(a, nullptr) : a;
+  fill_params(p, c);
   // the score-sum pass that may follow on the same stream reuses the workspace for its partial sums
-  const size_t own = partial_bytes(p, a.D), after = score_sum_workspace(a);
+  const size_t own = partial_bytes(p, a.D) + (copy ? copy_bytes(a) : 0), after = score_sum_workspace(a);
   return own > after ? own : after;
 }
 
-int launch_sdpa_prefill(const kvx_sdpa_args& a, hipStream_t st) {
+int launch_sdpa_prefill(const kvx_sdpa_args& a_in, hipStream_t st) {
   PrefillParams p;
+  kvx_sdpa_args a = a_in;
+  if (wants_copy(a)) {
+    // a workspace too small for the copy (sized for another call, or by a caller that has no room): the fused form
+    const kvx_sdpa_args c = on_copy(a, a.workspace);
+    fill_params(p, c);
+    if (a.workspace && a.workspace_bytes >= copy_bytes(a) + partial_bytes(p, a.D)) {
+      const int rc = launch_dequantize_kv(a, a.workspace, st);
+      if (rc != KVX_OK) return rc;
+      a = c;
+      a.workspace = (char*)a_in.workspace + copy_bytes(a_in);
+      a.workspace_bytes = a_in.workspace_bytes - copy_bytes(a_in);
+    }
+  }
   fill_params(p, a);
   const size_t need = partial_bytes(p, a.D);
   if (need) {

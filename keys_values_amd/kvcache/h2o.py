@@ -61,6 +61,7 @@ EAGER_SELECT = 4096
 # is faster than dequantising it inside the attention kernels (every 256 rows walk the whole store):
 # the copy costs two passes over the store, the kernels gain in proportion to the rows.
 DEFAULT_DEQUANTIZE_CHUNK_ROWS = 2048
+DEFAULT_DEQUANTIZE_CHUNK_ROWS_256 = 129  # head size 256
 
 _dequant_buffers = {}
 _dequant_owner = {}  # per buffer: the cache whose rows it holds as that cache's working buffer (blocks over heads), else None
@@ -126,7 +127,10 @@ class H2OKVCache:
         # blocks_over_heads (quantised stores only): one quantisation block per slot over all heads; see the module text
         self.blocks_over_heads = bool(blocks_over_heads) and quantized
         # dequantize_chunk_rows: a chunk with at least this many query rows (tokens x heads per KV head) is
-        # attended to over a bf16 copy of the quantised store made once for the chunk; None = never.
+        # attended to over a bf16 copy of the quantised store made once for the chunk; None = never. Left at its default it
+        # is lower at head size 256, where the dequantising kernel has no registers to spare.
+        if dequantize_chunk_rows == DEFAULT_DEQUANTIZE_CHUNK_ROWS and params.head_size == 256:
+            dequantize_chunk_rows = DEFAULT_DEQUANTIZE_CHUNK_ROWS_256
         self.dequantize_chunk_rows = dequantize_chunk_rows
         # overlap_select: launch the score update + eviction choice of a chunk step (and, for a long chunk over
         # a quantised store, the score-sum pass before them) on a second stream, so
@@ -522,7 +526,7 @@ class H2OKVCache:
                 # attention over the bf16 copy; the score-sum pass keeps the codes (it dequantises each key
                 # once per wavefront whatever the chunk length, and reads half the bytes)
                 kd, vd = self._dequantized(b, T)
-                out, _, lse = host.prefill(query, kd, vd, self.scale_factor, input_pos, tp, False, True, True, None, 0)
+                out, _, lse = host.prefill(query, kd, vd, self.scale_factor, input_pos, tp, False, True, True, None, 0, False)
                 if self._overlap:
                     # the score-sum pass too runs beside the caller's next launches: nothing needs the score-sums
                     # before the next chunk's eviction choice
@@ -539,7 +543,7 @@ class H2OKVCache:
                     return out.view(b, num, hq * d)
                 w = host.score_sum(query, kc, lse, self.scale_factor, input_pos, tp, quant)
             else:
-                out, w, _ = host.prefill(query, kc, vc, self.scale_factor, input_pos, tp, True, False, True, quant, 0)
+                out, w, _ = host.prefill(query, kc, vc, self.scale_factor, input_pos, tp, True, False, True, quant, 0, True)
         self._update(w, num)
         return out.view(b, num, hq * d)
 

@@ -5,7 +5,9 @@ import ctypes
 import pytest
 import torch
 
+from helpers import rel_err
 from keys_values_amd import _lib
+from keys_values_amd.attention import ops
 from keys_values_amd.kvcache.quantize import RowQuantizer
 from oracle import kvx_oracle as O
 
@@ -222,3 +224,32 @@ def test_block_sizes_and_slot_ranges_bit_exact(gpu, shape, blocks_over_heads, sp
     assert torch.equal(qz.quant_scales[:, lo:hi].cpu(), s) and torch.equal(qz.quant_zero_points[:, lo:hi].cpu(), z)
     back = O.dequantize_store(buf, s, z, (B, Hkv, hi - lo, D), num_bits, blocks_over_heads, dtype)
     assert torch.equal(qz.dequantize(lo, hi).cpu(), back)
+
+
+@pytest.mark.parametrize("num_bits,dtype,D,q_len,T,token_major", [
+    (8, torch.bfloat16, 64, 512, 777, False), (4, torch.float16, 128, 513, 1025, True), (4, torch.bfloat16, 64, 600, 640, True),
+    (8, torch.float16, 256, 40, 333, False), (4, torch.bfloat16, 256, 33, 130, True),
+])
+def test_prefill_over_a_copy_of_the_store(gpu, num_bits, dtype, D, q_len, T, token_major):
+    """A long chunk over a quantised store attends over rows dequantised once into the workspace: the same bits as the
+    plain kernels give on the dequantised rows, for any strides of the codes; and what the dequantising kernel gives up
+    to the order of its sums (other tiles per workgroup; outputs are rounded to 16 bits)."""
+    B, Hq, Hkv = 2, 8, 2
+    gen = torch.Generator().manual_seed(T)
+    q = torch.randn(B, Hq, q_len, D, generator=gen).to(dtype).to(gpu)
+    codes, state, rows = [], [], []
+    for _ in range(2):
+        qz = RowQuantizer((B, Hkv, T, D), dtype, num_bits, allocate_buffers=True, device=gpu)
+        qz.quantize(0, T, torch.randn(B, Hkv, T, D, generator=gen).to(dtype).to(gpu))
+        c = qz.quant_buffer.view(B, Hkv, T, -1)
+        codes.append(c.transpose(1, 2).contiguous().transpose(1, 2) if token_major else c)
+        state += [qz.quant_scales.view(B, Hkv, T), qz.quant_zero_points.view(B, Hkv, T)]
+        rows.append(qz.dequantize(0, T))
+    quant = ops.QuantState(*state)
+    args = (D ** -0.5, T - q_len, None)
+    out, w, lse = ops.prefill_core(q, *codes, *args, return_weights=True, return_lse=True, quant=quant)
+    out_p, _, lse_p = ops.prefill_core(q, *rows, *args, return_lse=True)
+    assert torch.equal(out, out_p) and torch.equal(lse, lse_p)
+    out_f, w_f, _ = _lib.host().prefill(q, *codes, *args, True, False, True, quant, 0, True)
+    assert rel_err(out.float(), out_f.float()) < 1e-2
+    torch.testing.assert_close(w, w_f, rtol=1e-4, atol=1e-7)
