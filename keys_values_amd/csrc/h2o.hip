@@ -8,12 +8,16 @@
 //   k == 1 (single-token decode): a streaming pass over all rows with many workgroups; each folds
 //          its slice into one 64-bit key (ordered value bits << 32 | slot) and publishes it with
 //          an integer atomicMin, which is order independent and therefore deterministic.
-//   k  > 1 (chunked prefill): one workgroup per (batch, head) row. The first pass adds the weights and
+//   k  > 1 (chunked prefill): a row is spread over workgroups of 1024 slots. The first launch adds the weights
+//          and sorts every workgroup's 64-bit (value, slot) keys; the second gives every key that can be among
+//          the first k its rank in the row by binary searches in the other lists and writes it there.
+//          Without the workspace for the lists (one workgroup per row): the first pass adds the weights and
 //          leaves the row's ordered value bits in LDS (rows of up to ~36K slots; longer rows are
 //          re-read from global memory). A 4-pass 8-bit radix select finds the k-th smallest value;
 //          elements below it, plus the lowest-slot elements equal to it, are gathered and
 //          bitonic-sorted as 64-bit (value, slot) keys.
 #include <mutex>
+#include <type_traits>
 
 #include "kvx_common.h"
 
@@ -308,7 +312,223 @@ __global__ __launch_bounds__(SEL_THREADS) void select_one_kernel(const kvx_h2o_a
   a.next_index[row] = (int32_t)(mine & 0xffffffffull);
 }
 
-// ---- k > 1 ----------------------------------------------------------------------------------
+// ---- k > 1, a row over several workgroups -----------------------------------------------------
+//
+// A row has few keys for a device (8 rows of 16384 slots) and many for one workgroup: with one workgroup per row the
+// choice of 1024 slots took 40 us, bound by one compute unit's LDS and instruction issue. Lists of 1024 keys are sorted
+// side by side instead, and ranks need no hand-over between workgroups but the launch boundary.
+// List c of a row takes the 64-slot blocks c, c + C, c + 2C, ... (C lists): old and new tokens lie in runs of slots, and
+// this way every list is a sample of the whole row, so that the bound below is tight whatever the order of the slots.
+
+constexpr int LIST = 1024;  // keys per list, one per thread of the sorting workgroup
+constexpr int RANK_THREADS = 512;
+constexpr int RANK_STAGED = 6144;  // keys of the lists' heads that the ranking workgroup holds in LDS
+
+// What the launches hand on, per (row, list).
+struct SelectLists {
+  unsigned long long* keys;  // LIST sorted keys
+  float* part_z;             // v_norm: sum of v_norm * w
+  float* stats;              // q_errors: extremes of the compared value and of the errors (4 floats)
+  int C;
+};
+__device__ __forceinline__ int list_slot(int c, int C, int t) { return ((t >> 6) * C + c) * 64 + (t & 63); }
+
+__global__ __launch_bounds__(LIST) void list_norm_kernel(const kvx_h2o_args a, const SelectLists sl) {
+  __shared__ float red[LIST / 64];
+  const int c = blockIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
+  const int slot = list_slot(c, sl.C, threadIdx.x);
+  float x = 0.0f;
+  if (slot < a.kv_len) x = a.v_norm[b * a.sc_stride_b + hh * a.sc_stride_h + slot] * a.w[(int64_t)row * a.kv_len + slot];
+  x = block_reduce(x, red, [](float u, float v) { return u + v; });
+  if (threadIdx.x == 0) sl.part_z[row * sl.C + c] = x;
+}
+
+// The score of this thread's slot after the update (stored), and the slot. Every product and sum rounded on its own.
+__device__ __forceinline__ float updated_score(const kvx_h2o_args& a, const SelectLists& sl, float* red, int row, int b, int hh, int slot) {
+  const int64_t off = b * a.sc_stride_b + hh * a.sc_stride_h;
+  float z = 1.0f;
+  const bool in = slot < a.kv_len;
+  const float s = in ? a.scores[off + slot] : 0.0f;
+  if (!a.w) return s;
+  const float w = in ? a.w[(int64_t)row * a.kv_len + slot] : 0.0f;
+  float inst = w;
+  if (a.v_norm) {
+    const float vn = in ? a.v_norm[off + slot] : 0.0f;
+    z = 0.0f;
+    for (int i = threadIdx.x; i < sl.C; i += LIST) z += sl.part_z[row * sl.C + i];
+    z = block_reduce(z, red, [](float u, float v) { return u + v; });
+    inst = __fmul_rn(__fmul_rn(vn, w) / z, (float)a.q_len);
+  }
+  const float v = __fadd_rn(s, inst);
+  if (in) a.scores[off + slot] = v;
+  return v;
+}
+
+// q_errors: the update and the lists' extremes, before anything can be compared
+__global__ __launch_bounds__(LIST) void list_stats_kernel(const kvx_h2o_args a, const SelectLists sl) {
+  __shared__ float red[LIST / 64];
+  const int c = blockIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
+  const int slot = list_slot(c, sl.C, threadIdx.x);
+  const bool in = slot < a.limit;
+  const float qe = in ? a.q_errors[b * a.sc_stride_b + hh * a.sc_stride_h + slot] : 0.0f;
+  const float v = updated_score(a, sl, red, row, b, hh, slot);
+  const int32_t* tpr = a.token_pos ? a.token_pos + b * a.tp_stride_b + hh * a.tp_stride_h : nullptr;
+  const float cv = in ? residency_value(v, a, tpr, slot) : 0.0f;
+  auto mn = [](float x, float y) { return fminf(x, y); };
+  auto mx = [](float x, float y) { return fmaxf(x, y); };
+  const float smin = block_reduce(in ? cv : INFINITY, red, mn), smax = block_reduce(in ? cv : -INFINITY, red, mx);
+  const float qmin = block_reduce(in ? qe : INFINITY, red, mn), qmax = block_reduce(in ? qe : -INFINITY, red, mx);
+  if (threadIdx.x == 0) *(f32x4_t*)(sl.stats + ((int64_t)row * sl.C + c) * 4) = f32x4_t{smin, smax, qmin, qmax};
+}
+
+// The value of the lane whose index differs in bit log2(S), on the vector ALU.
+template <int S>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+  auto dpp = [](uint32_t x, auto ctrl) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, decltype(ctrl)::value, 0xf, 0xf, true); };
+  if constexpr (S == 1) return dpp(v, std::integral_constant<int, 0xB1>{});        // quad_perm [1,0,3,2]
+  else if constexpr (S == 2) return dpp(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+  else if constexpr (S == 4) return dpp(dpp(v, std::integral_constant<int, 0x141>{}), std::integral_constant<int, 0x1B>{});  // half mirror, quad mirror
+  else if constexpr (S == 8) return dpp(v, std::integral_constant<int, 0x128>{});  // row_ror:8
+  else if constexpr (S == 16) {
+    const u32pair_t r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return (threadIdx.x & 16) ? r[0] : r[1];
+  } else {
+    const u32pair_t r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return (threadIdx.x & 32) ? r[0] : r[1];
+  }
+}
+
+template <int S>
+__device__ __forceinline__ unsigned long long sort_step(unsigned long long x, int size) {
+  const unsigned long long y = ((unsigned long long)lane_xor<S>((uint32_t)(x >> 32)) << 32) | lane_xor<S>((uint32_t)x);
+  const bool keep_min = ((threadIdx.x & S) == 0) == ((threadIdx.x & size) == 0);
+  return (y < x) == keep_min ? y : x;
+}
+
+// Bitonic sort of LIST keys, one a thread: steps between lanes of a wavefront on the vector ALU, the ten others through
+// LDS (two buffers in turn: one barrier each).
+__device__ __forceinline__ unsigned long long sort_list(unsigned long long x, unsigned long long (&buf)[2][LIST]) {
+  const int t = threadIdx.x;
+  int which = 0;
+#pragma unroll 1
+  for (int size = 2; size <= LIST; size <<= 1) {
+#pragma unroll 1
+    for (int stride = size >> 1; stride >= 64; stride >>= 1) {
+      buf[which][t] = x;
+      __syncthreads();
+      const unsigned long long y = buf[which][t ^ stride];
+      const bool keep_min = ((t & stride) == 0) == ((t & size) == 0);
+      x = (y < x) == keep_min ? y : x;
+      which ^= 1;
+    }
+    if (size >= 64) x = sort_step<32>(x, size);
+    if (size >= 32) x = sort_step<16>(x, size);
+    if (size >= 16) x = sort_step<8>(x, size);
+    if (size >= 8) x = sort_step<4>(x, size);
+    if (size >= 4) x = sort_step<2>(x, size);
+    x = sort_step<1>(x, size);
+  }
+  return x;
+}
+
+__global__ __launch_bounds__(LIST) void list_sort_kernel(const kvx_h2o_args a, const SelectLists sl) {
+  __shared__ float red[LIST / 64];
+  __shared__ unsigned long long buf[2][LIST];
+  const int tid = threadIdx.x, c = blockIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
+  const int slot = list_slot(c, sl.C, tid);
+  const bool in = slot < a.limit;
+  const int32_t* tpr = a.token_pos ? a.token_pos + b * a.tp_stride_b + hh * a.tp_stride_h : nullptr;
+  unsigned long long x = ~0ull;
+  if (a.q_errors) {
+    const int64_t off = b * a.sc_stride_b + hh * a.sc_stride_h;
+    const float v = in ? a.scores[off + slot] : 0.0f, qe = in ? a.q_errors[off + slot] : 0.0f;
+    float v4[4] = {INFINITY, -INFINITY, INFINITY, -INFINITY};
+    const float* st = sl.stats + (int64_t)b * a.Hkv * sl.C * 4;
+    for (int i = tid; i < a.Hkv * sl.C; i += LIST) {
+      const f32x4_t s4 = *(const f32x4_t*)(st + i * 4);
+      v4[0] = fminf(v4[0], s4[0]);
+      v4[1] = fmaxf(v4[1], s4[1]);
+      v4[2] = fminf(v4[2], s4[2]);
+      v4[3] = fmaxf(v4[3], s4[3]);
+    }
+    auto mn = [](float u, float w) { return fminf(u, w); };
+    auto mx = [](float u, float w) { return fmaxf(u, w); };
+    Modify m;
+    m.smin = block_reduce(v4[0], red, mn);
+    m.sden = block_reduce(v4[1], red, mx) - m.smin;
+    m.qmin = block_reduce(v4[2], red, mn);
+    m.qden = block_reduce(v4[3], red, mx) - m.qmin;
+    m.c = (float)a.combination;
+    m.c2 = (float)((a.combination - 1.0) / 2.0);
+    m.c3 = (float)(1.0 - a.combination);
+    if (in) x = ((unsigned long long)ordered_bits(combined_value(residency_value(v, a, tpr, slot), qe, m)) << 32) | (unsigned)slot;
+  } else {
+    const float v = updated_score(a, sl, red, row, b, hh, slot);
+    if (in) x = ((unsigned long long)ordered_bits(residency_value(v, a, tpr, slot)) << 32) | (unsigned)slot;
+  }
+  x = sort_list(x, buf);
+  if (sl.C == 1) {  // the row is one list
+    if (tid < a.k) a.next_index[(int64_t)row * a.k + tid] = (int32_t)(x & 0xffffffffull);
+  } else {
+    sl.keys[((int64_t)row * sl.C + c) * LIST + tid] = x;
+  }
+}
+
+// Ranks of the keys of list c. `per` = ceil(k / C) keys of every list are at or below U, the largest of the lists'
+// per-th keys, so the first k keys of the row are all at or below U: about per of each list when the lists are alike.
+// Only those are ranked: a key's rank is its place in its list plus its places in the others, found by binary search in
+// the lists' heads (`staged` keys each, in LDS; in memory beyond them).
+__global__ __launch_bounds__(RANK_THREADS) void list_rank_kernel(const unsigned long long* __restrict__ lists, int C, int k, int per, int staged, int32_t* __restrict__ next) {
+  __shared__ unsigned long long head[RANK_STAGED];
+  __shared__ uint32_t rank[LIST];
+  __shared__ unsigned long long wmax[RANK_THREADS / 64];
+  const int tid = threadIdx.x, c = blockIdx.x, row = blockIdx.y;
+  const unsigned long long* base = lists + (int64_t)row * C * LIST;
+  for (int i = tid; i < C * staged; i += RANK_THREADS) head[i] = base[(i / staged) * LIST + i % staged];
+  unsigned long long u = 0ull;
+  for (int i = tid; i < C; i += RANK_THREADS) {
+    const unsigned long long x = base[i * LIST + per - 1];
+    u = x > u ? x : u;
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    const unsigned long long o = __shfl_xor(u, off, 64);
+    u = o > u ? o : u;
+  }
+  if ((tid & 63) == 0) wmax[tid >> 6] = u;
+  for (int i = tid; i < LIST; i += RANK_THREADS) rank[i] = 0u;
+  __syncthreads();
+  for (int i = 0; i < RANK_THREADS / 64; ++i) u = wmax[i] > u ? wmax[i] : u;
+  u = u == ~0ull ? u - 1 : u;  // places without a slot are never ranked
+  auto at = [&](int list, int i) { return i < staged ? head[list * staged + i] : base[list * LIST + i]; };
+  // keys of `list` below x (or up to and including it)
+  auto below = [&](int list, unsigned long long x, bool inclusive) {
+    int lo = 0, n = LIST;
+    if (staged < LIST && (inclusive ? head[list * staged + staged - 1] > x : head[list * staged + staged - 1] >= x)) n = staged;
+    while (n > 0) {
+      const int half = n >> 1;
+      const unsigned long long y = at(list, lo + half);
+      if (inclusive ? y <= x : y < x) {
+        lo += half + 1;
+        n -= half + 1;
+      } else {
+        n = half;
+      }
+    }
+    return lo;
+  };
+  const int n = below(c, u, true);
+  for (int i = tid; i < n * C; i += RANK_THREADS) {
+    const int list = i / n, e = i - list * n;
+    const int r = list == c ? e : below(list, at(c, e), false);
+    if (r) atomicAdd(&rank[e], (uint32_t)r);
+  }
+  __syncthreads();
+  for (int e = tid; e < n; e += RANK_THREADS)
+    if (rank[e] < (uint32_t)k) next[(int64_t)row * k + rank[e]] = (int32_t)(at(c, e) & 0xffffffffull);
+}
+
+// ---- k > 1, one workgroup per row --------------------------------------------------------------
 
 // CACHED: the row's ordered keys live in LDS after the first pass (rows of up to ~36K slots), so the
 // radix passes and the gather never go back to global memory.
@@ -548,14 +768,63 @@ static size_t best_bytes(const kvx_h2o_args& a) {
   return (a.k == 1 || a.k > MAX_PASS_K) ? ((size_t)a.B * a.Hkv * sizeof(unsigned long long) + 15) / 16 * 16 : 0;
 }
 
-size_t h2o_workspace(const kvx_h2o_args& a) { return best_bytes(a) + (a.q_errors ? (size_t)a.B * a.Hkv * 4 * sizeof(float) : 0); }
+// what the one-workgroup-per-row form cannot do without
+static size_t min_workspace(const kvx_h2o_args& a) { return best_bytes(a) + (a.q_errors ? (size_t)a.B * a.Hkv * 4 * sizeof(float) : 0); }
+
+// Sorted lists of 1024 keys for k > 1: taken while their number and size stay reasonable (256 lists a row, 1 GiB), else
+// (and where the caller's workspace does not hold them) one workgroup per row.
+struct ListPlan {
+  int C;  // lists per row, 0: not this way
+  size_t off_z, off_stats, total;
+};
+static ListPlan list_plan(const kvx_h2o_args& a) {
+  ListPlan p{};
+  if (a.k <= 1 || a.B <= 0 || a.Hkv <= 0 || a.kv_len <= 0 || (int64_t)a.B * a.Hkv > 65535) return p;
+  const int64_t C = ((int64_t)a.kv_len + LIST - 1) / LIST, rows = (int64_t)a.B * a.Hkv;
+  if (C > 256 || rows * C * LIST * 8 > (1ll << 30)) return p;
+  p.C = (int)C;
+  const size_t n = (size_t)(rows * C);
+  p.off_z = C > 1 ? n * LIST * 8 : 0;
+  p.off_stats = p.off_z + (n * 4 + 15) / 16 * 16;
+  p.total = p.off_stats + n * 16;
+  return p;
+}
+
+size_t h2o_workspace(const kvx_h2o_args& a) {
+  const size_t least = min_workspace(a), lists = list_plan(a).total;
+  return least > lists ? least : lists;
+}
+
+static int launch_lists(const kvx_h2o_args& a, const ListPlan& p, hipStream_t st) {
+  SelectLists sl;
+  char* ws = (char*)a.workspace;
+  sl.keys = (unsigned long long*)ws;
+  sl.part_z = (float*)(ws + p.off_z);
+  sl.stats = (float*)(ws + p.off_stats);
+  sl.C = p.C;
+  const dim3 grid(p.C, a.B * a.Hkv);
+  if (a.w && a.v_norm) hipLaunchKernelGGL(list_norm_kernel, grid, dim3(LIST), 0, st, a, sl);
+  if (a.q_errors) hipLaunchKernelGGL(list_stats_kernel, grid, dim3(LIST), 0, st, a, sl);
+  hipLaunchKernelGGL(list_sort_kernel, grid, dim3(LIST), 0, st, a, sl);
+  if (p.C > 1) {
+    const int per = (a.k + p.C - 1) / p.C;
+    int staged = 16;
+    while (staged < 2 * per && staged < LIST) staged <<= 1;
+    while (staged * p.C > RANK_STAGED) staged >>= 1;
+    hipLaunchKernelGGL(list_rank_kernel, grid, dim3(RANK_THREADS), 0, st, (const unsigned long long*)sl.keys, p.C, a.k, per, staged, a.next_index);
+  }
+  KVX_HIP(hipGetLastError());
+  return KVX_OK;
+}
 
 int launch_h2o_update_select(const kvx_h2o_args& a_in, hipStream_t st) {
   kvx_h2o_args a = a_in;
   const int rows = a.B * a.Hkv;
   if (rows == 0) return KVX_OK;
-  KVX_REQUIRE(h2o_workspace(a) == 0 || (a.workspace && a.workspace_bytes >= h2o_workspace(a)), KVX_ERR_WORKSPACE,
-              "kvx_h2o_update_select: workspace of %zu bytes needed", h2o_workspace(a));
+  KVX_REQUIRE(min_workspace(a) == 0 || (a.workspace && a.workspace_bytes >= min_workspace(a)), KVX_ERR_WORKSPACE,
+              "kvx_h2o_update_select: workspace of %zu bytes needed", min_workspace(a));
+  const ListPlan lists = list_plan(a);
+  if (lists.C && a.workspace && a.workspace_bytes >= lists.total && ((uintptr_t)a.workspace & 15) == 0) return launch_lists(a, lists, st);
   float* stats = nullptr;
   if (is_variant(a)) {
     // the accumulation (and the batch statistics of the combination) first; what follows only selects
@@ -644,7 +913,7 @@ static int static_scratch_ptr(void** out) {
 
 int launch_h2o_update_select_static(const kvx_h2o_args& a_in, hipStream_t st) {
   kvx_h2o_args a = a_in;
-  const size_t need = h2o_workspace(a);
+  const size_t need = min_workspace(a);
   KVX_REQUIRE(need <= kStaticScratchBytes, KVX_ERR_WORKSPACE,
               "kvx_h2o_update_select_static: B * Hkv = %d rows need %zu bytes of scratch, the static array holds %zu", a.B * a.Hkv, need,
               kStaticScratchBytes);

@@ -457,7 +457,7 @@ class H2OKVCache:
         the same scores. Nothing is added to them (no weights), so the first entries come out as before."""
         if num > self._select_k:
             raise ValueError(f"num = {num} exceeds what a full cache hands out ({self._select_k})")
-        _lib.host().cache_update(self, None, 1, num, True)
+        _lib.host().cache_update(self, None, 1, num, True, False)
         self._next_count = num
 
     # -- the step (keys_values/kvcache/base.py:554-595) -----------------------------------------
@@ -759,7 +759,7 @@ class H2OKVCache:
         full = self.current_length == self.cache_length
         k_now = min(self._select_k, EAGER_SELECT) if select is None else min(select, self._select_k)
         if not self._overlap:
-            _lib.host().cache_update(self, attn_weights, query_length, k_now, full)
+            _lib.host().cache_update(self, attn_weights, query_length, k_now, full, False)
         else:
             attn_weights = attn_weights.contiguous()
             main = torch.cuda.current_stream(self.device)
@@ -768,7 +768,7 @@ class H2OKVCache:
             ready.record(main)
             with torch.cuda.stream(self._side_stream):
                 self._side_stream.wait_event(ready)
-                _lib.host().cache_update(self, attn_weights, query_length, k_now, full)
+                _lib.host().cache_update(self, attn_weights, query_length, k_now, full, True)
                 done = torch.cuda.Event()
                 done.record(self._side_stream)
             self._select_done = done

@@ -383,3 +383,52 @@ def test_fused_single_token_step_matches_the_separate_calls(gpu, decode_route, n
         torch.testing.assert_close(out.view(B, Hq, D).float(), o_ref.float(), rtol=2e-2, atol=1e-3)
         torch.testing.assert_close(fused.scores, apart.scores, rtol=1e-5, atol=1e-9)
         assert torch.equal(fused._next_index, apart._next_index), f"step {i}"
+
+
+@pytest.mark.parametrize("policy", ["h2o", "normalize", "vlen", "q_errors"])
+@pytest.mark.parametrize("B,Hkv,L,gp,k", [
+    (1, 2, 100, 0, 7),         # one list, partly filled
+    (2, 1, 1024, 24, 1000),    # one full list, all of it chosen
+    (1, 2, 1025, 0, 2),        # a second list of one slot
+    (2, 2, 6000, 128, 200),    # the lists' last blocks ragged, a ring behind the limit
+    (1, 1, 9000, 1, 8999),     # the whole row sorted, beyond what one launch of the other form sorts
+    (1, 2, 70000, 0, 1024),    # more lists than their heads fit the staging at full length
+])
+def test_selection_over_lists_matches_one_workgroup_per_row(kvx, gpu, B, Hkv, L, gp, k, policy):
+    """The choice of k slots with a row spread over sorted lists, against the one-workgroup-per-row form that runs when the
+    workspace holds no lists: the same keys, so the same slots in the same order, exact ties included (scores on a coarse
+    grid). The V-norm normaliser is a sum over the row in another order: scores to a few 2^-24 sqrt(L), slots where the
+    update leaves no near-ties to decide."""
+    gen = torch.Generator().manual_seed(L + k)
+    limit = L - gp
+    scores = (torch.randint(0, 50, (B, Hkv, L), generator=gen) / 8.0).to(gpu)
+    scores[..., : L // 3] += 20.0  # old tokens in a run of slots, with much larger scores
+    w = (torch.randint(0, 9, (B, Hkv, L), generator=gen) / 16.0).to(gpu)
+    tp = torch.randint(0, 2 * L, (B, Hkv, L), generator=gen).to(torch.int32).to(gpu)
+    vn = (0.5 + torch.rand(B, Hkv, L, generator=gen)).to(gpu) if policy == "vlen" else None
+    qe = torch.rand(B, Hkv, L, generator=gen).to(gpu) if policy == "q_errors" else None
+    got = []
+    for lists in (True, False):
+        sc, nxt = scores.clone(), torch.full((B, Hkv, k), -1, dtype=torch.int32, device=gpu)
+        a = _lib.H2OArgs()
+        a.B, a.Hkv, a.kv_len, a.limit, a.k, a.q_len = B, Hkv, L, limit, k, 5
+        a.scores, a.sc_stride_b, a.sc_stride_h, a.w = sc.data_ptr(), sc.stride(0), sc.stride(1), w.data_ptr()
+        a.token_pos, a.tp_stride_b, a.tp_stride_h = tp.data_ptr(), tp.stride(0), tp.stride(1)
+        a.normalize, a.input_pos, a.prefill_len = int(policy in ("normalize", "q_errors")), 2 * L + 1, L // 2
+        a.v_norm, a.q_errors, a.combination = _lib.ptr(vn), _lib.ptr(qe), 0.6
+        a.next_index = nxt.data_ptr()
+        rows = B * Hkv  # the other form's scratch: a bound per row beyond 4096 slots a launch, four statistics with the errors
+        full, least = kvx.kvx_h2o_workspace_bytes(ctypes.byref(a)), ((8 * rows + 15) // 16 * 16 if k > 4096 else 0) + (16 * rows if qe is not None else 0)
+        assert full > least
+        ws = torch.empty(full, dtype=torch.uint8, device=gpu)
+        a.workspace, a.workspace_bytes = ws.data_ptr(), full if lists else least
+        print(f"select lists={lists} L={L} k={k} {policy}", flush=True)
+        _lib.check(kvx.kvx_h2o_update_select(ctypes.byref(a), _lib.stream_ptr(gpu)))
+        got.append((sc.cpu(), nxt.cpu().long()))
+    (s0, n0), (s1, n1) = got
+    assert (n0 >= 0).all() and (n0 < limit).all() and all(len(set(r.tolist())) == k for r in n0.view(-1, k))
+    if policy != "vlen":
+        assert torch.equal(s0, s1) and torch.equal(n0, n1)
+    else:
+        torch.testing.assert_close(s0, s1, rtol=1e-5, atol=0)
+        _sets_equal_away_from_ties(n0, n1, s1[..., :limit], k)
