@@ -1238,26 +1238,32 @@ Plan make_plan(const kvx_sdpa_args& a, bool fused_h2o) {
   Plan pl;
   const int gr = a.Hq / a.Hkv;
   pl.G = gr <= 1 ? 1 : (gr <= 2 ? 2 : (gr <= 4 ? 4 : (gr <= 8 ? 8 : 16)));
-  // Keys per split: one workgroup per compute unit over the whole grid, at least 128 keys (a wavefront's steps take
-  // about 1 us each; shorter splits only add partials to combine), at least what keeps a row to 128 splits (to 64 below
-  // 16384 keys: the splits of a row wait for each other), and with weights at most what the LDS holds of a split's logits
-  // (longer rows of many heads then run several rounds). Two workgroups per compute unit, as many as fit, were worse
-  // wherever one round covers the call. Measured, us, two -> one per compute unit: 8 rows of 16384 keys 25.0 -> 21.4, of
-  // 65536 keys 55 -> 50, 32 rows of 16384 keys 52.6 -> 49.8; 8-bit codes 8 rows of 32768 keys 29 -> 25, 32 rows of
-  // 16384 keys 39 -> 37; head size 256, 8-bit codes, 32 rows of 8192 keys 49 -> 40; 8 rows of 1024 keys, 256 -> 128 keys
-  // a split 13.1 -> 11.8. 64 rows of 32768 keys take 170 in two rounds of 4096 keys, 183 in splits of 1024.
+  // Splits: as many as give every compute unit one workgroup and not one more (a few workgroups too many are a second
+  // round for everybody: 16 rows of 35407 8-bit keys at head size 256 in 17 splits took 137 us, in 16 they take 80), of at
+  // least 128 keys (a wavefront's steps take about 1 us each; shorter splits only add partials to combine), at most 128
+  // a row (64 below 16384 keys: the splits of a row wait for each other), and with weights no longer than what the LDS
+  // holds of a split's logits (long rows of many heads then run several full rounds). Two workgroups per compute unit, as
+  // many as fit, were worse wherever one round covers the call. Measured, us, two -> one per compute unit: 8 rows of
+  // 16384 keys 25.0 -> 21.4, of 65536 keys 55 -> 50, 32 rows of 16384 keys 52.6 -> 49.8; 8-bit codes 8 rows of 32768 keys
+  // 29 -> 25; head size 256, 8-bit codes, 32 rows of 8192 keys 49 -> 40; 8 rows of 1024 keys, 256 -> 128 keys a split
+  // 13.1 -> 11.8. 64 rows of 32768 keys take 170 in two rounds of 4096 keys, 183 in splits of 1024.
   const bool weights = a.w || fused_h2o;
   const int allow_resident = weights ? tuning().resident.load() : 0;
   const int lgk = logit_floats(pl.G, a.D) / pl.G;
   int splits = a.num_splits;
   if (splits <= 0) {
-    int64_t keys = (int64_t)a.B * a.Hkv * a.kv_len / num_cus();
-    keys = max(keys, (int64_t)max(max(128, min(256, a.kv_len / 64)), (a.kv_len + 127) / 128));
+    const int64_t rows = (int64_t)a.B * a.Hkv, cus = num_cus();
+    auto in_rounds = [&](int64_t r) { return max((int64_t)1, r * cus / rows); };  // splits of r rounds of one workgroup per compute unit
+    int64_t n = in_rounds(1);
     // codes are bound by the vector arithmetic of their dequantisation: long splits gain from a second workgroup a unit
     // (32 rows of 16384 keys, 4 bits: 33 us against 36)
-    if (!kv_is_plain(a.kv_dtype) && a.D <= 128 && keys > 1024) keys = max((int64_t)1024, keys / 2);
-    if (allow_resident && keys > lgk) keys = lgk;
-    splits = (int)((a.kv_len + keys - 1) / keys);
+    if (!kv_is_plain(a.kv_dtype) && a.D <= 128 && a.kv_len / n > 1024) n = min(in_rounds(2), max(n, (int64_t)a.kv_len / 1024));
+    n = min(n, min((int64_t)(a.kv_len + 127) / 128, (int64_t)(a.kv_len < 16384 ? 64 : 128)));
+    if (allow_resident && a.kv_len > n * lgk) {
+      const int64_t least = (a.kv_len + lgk - 1) / lgk;
+      n = max(least, in_rounds((least * rows + cus - 1) / cus));
+    }
+    splits = (int)min(n, (int64_t)512);
   }
   splits = max(1, min(splits, 512));
   int kps = (a.kv_len + splits - 1) / splits;
