@@ -680,7 +680,7 @@ __global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(const PrefillPa
 // that has its compute unit to itself is 700 / 1130 / 2050 at head size 64 / 128 / 256, two side by side gain 20 %; the
 // combining launch takes 2 us and reads its partials at 4 TB/s. A full count of rounds with a nearly empty last one is what
 // the rule avoids: 2 x 4 heads, 333 queries x 7, 5001 keys: 4 splits (608 workgroups, three to a unit) 83 us, 3 splits
-// (456, two) 63 us; 4 x 4 heads, 541 x 7 over 5238: 2 splits 177, none 152.
+// (456, two) 63 us, 5 splits (760, three) 73 us; 4 x 4 heads, 541 x 7 over 5238: 2 splits 177, none 152.
 int pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
   if (a.num_splits > 0) return min(a.num_splits, num_tiles);
   const int64_t base = (int64_t)a.B * a.Hkv * m_blocks, cus = num_cus();
@@ -695,7 +695,8 @@ int pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
     const int tps = (num_tiles + s - 1) / s;
     if ((num_tiles + tps - 1) / tps != s) continue;
     const int64_t c = (base * s + cus - 1) / cus;
-    const int64_t walk = c * tps * (pairs && c > 1 ? tile_ns * 4 / 5 : tile_ns);
+    // an odd workgroup after the pairs gains nothing and waits for one of them to end
+    const int64_t walk = tps * tile_ns * (!pairs || c == 1 ? 100 * c : 160 * (c / 2) + 135 * (c % 2)) / 100;
     const int64_t merge = s == 1 ? 0 : 2000 + s * rows * (a.D * 4 + 8) / 4000;
     if (walk + merge < best_ns) {
       best_ns = walk + merge;
