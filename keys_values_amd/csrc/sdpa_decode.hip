@@ -727,28 +727,22 @@ __global__ __launch_bounds__(NTHREADS) void decode_split_kernel(const DecodePara
 // O^T += V^T P^T per 32 keys. The accumulator layout of S^T (lane = (head, keys 4 kg .. 4 kg + 3)) becomes the B
 // operand of the second product without any exchange once the 32 keys of a block are taken in the order (tile 0:
 // 4 kg .. 4 kg + 3, tile 1: 4 kg .. 4 kg + 3) per lane group kg; V^T is gathered to match: a lane loads, from each of
-// its 8 keys, the D / 16 values of its d rows and regroups them, one byte permute per pair of values.
-// The running maximum is one per head (the four lane groups of a head column agree on it), it moves lazily as above.
-// Everything after the key loop is shared with the kernel above.
-//
-// Codes: the vector ALU's work per element is what bounds the kernel (3.5 instructions to dequantise one: 4 x 8 rows of
-// 16384 8-bit keys of 128 took 38 us, 3.7 TB/s). Keys are dequantised and rounded, the score-sums are defined on the
-// rounded rows (forming them as fma(code, scale, -zp scale), one instruction less, moves a few 4-bit rows' score-sums by
-// half a percent). V needs no dequantisation: with p'_k = p_k scale_k, sum_k p_k scale_k (code_k - zp_k) =
-// sum_k p'_k code_k - sum_k p'_k zp_k, and a code is a bf16 number as it stands: the bits 0x00cc are cc 2^-133 (below
-// 128 a subnormal, above it the first binade, at the same spacing), which the matrix cores take as is.
-// So the permute that regroups the bytes is all, 0.5 instructions an element (0.75 for 4-bit codes, whose upper half
-// stays where it is and counts 16 fold). Both sums use the same rounded p', so that its rounding error meets
-// code - zp, as it met the dequantised value before. p' carries 2^48 to keep the products inside fp32: V rows from
-// 1e-20 to 1e20 are served. float16 rows, whose p had 11 bits, take p' in two bf16 terms (16 bits).
+// its 8 keys, the D / 16 values of its d rows and regroups them (one byte permute per pair of bf16 values; for codes
+// the regrouping is part of the dequantisation). What is left for the vector ALU is the dequantisation (3.5
+// instructions per element, as the reference rounds) or half an instruction per V element, and the softmax of 16
+// head columns per key. The running maximum is one per head (the four lane groups of a head column agree on it), it
+// moves lazily as above. Everything after the key loop is shared with the kernel above.
 template <bool F16>
 __device__ __forceinline__ f32x4_t mfma_16x16x32(u32x4_t a, u32x4_t b, f32x4_t c) {
   if constexpr (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
   else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
-constexpr float kCodeLift = 48.0f;     // log2 of what p' carries
-constexpr float kCodeScale = 0x1p85f;  // 2^(133 - 48): what the sum of p' times a code's bits has to be multiplied by
+// elem( (float)((int)code - zp) * scale ) for two codes with their own row state (two keys)
+template <bool F16>
+__device__ __forceinline__ uint32_t dequant_pair2(uint32_t c0, int32_t zp0, float sc0, uint32_t c1, int32_t zp1, float sc1) {
+  return pack_pair<F16>((float)((int32_t)c0 - zp0) * sc0, (float)((int32_t)c1 - zp1) * sc1);
+}
 
 template <int D, int G, int KV>
 __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel(const DecodeParams p, const kvx_h2o_args hh, const int h2o) {
@@ -812,7 +806,6 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
 #pragma unroll
   for (int t = 0; t < DPL; ++t) acc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   float m_run = kNegBig, l_run = 0.0f;
-  float z_run = 0.0f;  // codes: sum of p' zp (l_run and z_run carry the 2^48 of p' too)
 
   struct Rows {
     u32x4_t k[2][KR];
@@ -924,8 +917,7 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
       return dequant_words<F16>(c[0], c[1], r.kz[gi], r.ks[gi]);
     }
   };
-  // A operand t of the second product: value (or code, as the bits of a bf16) t of each of this lane's 8 keys, in key
-  // order. 4-bit rows: byte tb of this lane's share, the first half of the row its high nibbles (16 code).
+  // A operand t of the second product: value t of each of this lane's 8 keys, in key order
   auto v_operand = [&](const Rows& r, int t) -> u32x4_t {
     u32x4_t a;
 #pragma unroll
@@ -934,10 +926,17 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
       if constexpr (!U8) {
         a[jj] = __builtin_amdgcn_perm(r.v[j1][t >> 1], r.v[j0][t >> 1], (t & 1) ? 0x07060302u : 0x05040100u);
       } else {
-        const int tb = U4 && t >= DPL / 2 ? t - DPL / 2 : t;
-        const uint32_t mask = !U4 ? 0xffffffffu : t < DPL / 2 ? 0xf0f0f0f0u : 0x0f0f0f0fu;
-        const uint32_t sel = 0x0c040c00u + 0x00010001u * (uint32_t)(tb & 3);  // byte of j0, 0, byte of j1, 0
-        a[jj] = __builtin_amdgcn_perm(r.v[j1][tb >> 2] & mask, r.v[j0][tb >> 2] & mask, sel);
+        uint32_t c0, c1;
+        if constexpr (!U4) {
+          c0 = (r.v[j0][t >> 2] >> (8 * (t & 3))) & 0xffu;
+          c1 = (r.v[j1][t >> 2] >> (8 * (t & 3))) & 0xffu;
+        } else {
+          const int tb = t < DPL / 2 ? t : t - DPL / 2;  // byte of this lane's share; first half of the row: high nibble
+          const int sh = 8 * (tb & 3) + (t < DPL / 2 ? 4 : 0);
+          c0 = (r.v[j0][tb >> 2] >> sh) & 0xfu;
+          c1 = (r.v[j1][tb >> 2] >> sh) & 0xfu;
+        }
+        a[jj] = dequant_pair2<F16>(c0, r.vz[j0], r.vs[j0], c1, r.vz[j1], r.vs[j1]);
       }
     }
     return a;
@@ -980,39 +979,18 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
       const float al = fast_exp2(m_run - mn);
       m_run = mn;
       l_run *= al;
-      z_run *= al;
 #pragma unroll
       for (int t = 0; t < DPL; ++t) acc[t] *= al;
     }
-    const float lift = U8 ? m_run - kCodeLift : m_run;
     float pv[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      pv[i] = fast_exp2(sv[i] - lift);
+      pv[i] = fast_exp2(sv[i] - m_run);
       l_run += pv[i];
-      if constexpr (U8) pv[i] *= r.vs[i];
     }
-    if constexpr (!U8) {
-      const u32x4_t pb = {pack_pair<F16>(pv[0], pv[1]), pack_pair<F16>(pv[2], pv[3]), pack_pair<F16>(pv[4], pv[5]), pack_pair<F16>(pv[6], pv[7])};
+    const u32x4_t pb = {pack_pair<F16>(pv[0], pv[1]), pack_pair<F16>(pv[2], pv[3]), pack_pair<F16>(pv[4], pv[5]), pack_pair<F16>(pv[6], pv[7])};
 #pragma unroll
-      for (int t = 0; t < DPL; ++t) acc[t] = mfma_16x16x32<F16>(v_operand(r, t), pb, acc[t]);
-    } else {
-      u32x4_t pb, pl;  // p' and, for float16 rows, what its rounding left
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        pb[i] = pack_pair<false>(pv[2 * i], pv[2 * i + 1]);
-        const float h0 = __uint_as_float(pb[i] << 16), h1 = __uint_as_float(pb[i] & 0xffff0000u);
-        if constexpr (F16) pl[i] = pack_pair<false>(pv[2 * i] - h0, pv[2 * i + 1] - h1);
-        z_run = fmaf(F16 ? pv[2 * i] : h0, (float)r.vz[2 * i], z_run);
-        z_run = fmaf(F16 ? pv[2 * i + 1] : h1, (float)r.vz[2 * i + 1], z_run);
-      }
-#pragma unroll
-      for (int t = 0; t < DPL; ++t) {
-        const u32x4_t codes = v_operand(r, t);
-        acc[t] = mfma_16x16x32<false>(codes, pb, acc[t]);
-        if constexpr (F16) acc[t] = mfma_16x16x32<false>(codes, pl, acc[t]);
-      }
-    }
+    for (int t = 0; t < DPL; ++t) acc[t] = mfma_16x16x32<F16>(v_operand(r, t), pb, acc[t]);
   };
 
   // Two steps in flight per wavefront: the loads of step i + 1 are issued before step i is consumed.
@@ -1045,17 +1023,6 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
   float l = l_run;
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
-  if constexpr (U8) {
-    float z = z_run;
-    z += __shfl_xor(z, 16, 64);
-    z += __shfl_xor(z, 32, 64);
-    z *= 0x1p-48f;
-    l *= 0x1p-48f;
-#pragma unroll
-    for (int t = 0; t < DPL; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[t][i] = acc[t][i] * (U4 && t < DPL / 2 ? kCodeScale / 16.0f : kCodeScale) - z;
-  }
   if (m < G) {
 #pragma unroll
     for (int t = 0; t < DPL; ++t)

@@ -253,27 +253,3 @@ def test_prefill_over_a_copy_of_the_store(gpu, num_bits, dtype, D, q_len, T, tok
     out_f, w_f, _ = _lib.host().prefill(q, *codes, *args, True, False, True, quant, 0, True)
     assert rel_err(out.float(), out_f.float()) < 1e-2
     torch.testing.assert_close(w, w_f, rtol=1e-4, atol=1e-7)
-
-
-@pytest.mark.parametrize("num_bits", [8, 4])
-@pytest.mark.parametrize("dtype,size", [(torch.bfloat16, 1e18), (torch.bfloat16, 1.0), (torch.bfloat16, 1e-4), (torch.float16, 1e4), (torch.float16, 1e-4)])
-@pytest.mark.parametrize("D,Hq,T", [(64, 3, 33), (128, 16, 257), (256, 8, 500)])
-def test_single_token_sums_codes_of_values(gpu, num_bits, dtype, size, D, Hq, T):
-    """The single-token kernel sums V's codes and zero points, not dequantised values: V rows at both ends of what it
-    serves, some far from zero (zero points in the thousands), one constant, at every head size. Bound: the output's
-    rounding and p's (bf16: 2^-9 each, float16: the output's 2^-12) and the dequantised rows' of the oracle (2^-9, 2^-12)."""
-    gen = torch.Generator().manual_seed(D)
-    q, k, v = (torch.randn(1, h, n, D, generator=gen) for h, n in ((Hq, 1), (1, T), (1, T)))
-    v[:, :, ::5] += 300.0
-    v[:, :, 7] = -2.0
-    if dtype == torch.float16 and size > 1:
-        v = v / 100.0
-    q, k, v = q.to(dtype), k.to(dtype), (v * size).to(dtype)
-    (kc, ks, kz), (vc, vs, vz) = O.quantize_rows(k, num_bits), O.quantize_rows(v, num_bits)
-    want, w_ref = O.sdpa_in_blocks(q, O.dequantize_rows(kc, ks, kz, dtype), O.dequantize_rows(vc, vs, vz, dtype), D ** -0.5, 10 * T, None)
-    if num_bits == 4:
-        kc, vc = O.compress4(kc), O.compress4(vc)
-    quant = ops.QuantState(*(t.to(gpu) for t in (ks, kz, vs, vz)))
-    out, w, _ = ops.decode_core(q.to(gpu), kc.to(gpu), vc.to(gpu), D ** -0.5, return_weights=True, quant=quant)
-    assert rel_err(out.double().cpu().unsqueeze(2), want.double()) < 3 * (2 ** -9 if dtype == torch.bfloat16 else 2 ** -12)
-    torch.testing.assert_close(w.cpu(), w_ref, rtol=1e-3, atol=1e-6)
