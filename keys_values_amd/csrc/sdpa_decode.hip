@@ -120,11 +120,15 @@ __device__ __forceinline__ float swap_halves_add(float a, float b) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Logits a workgroup holds in LDS: 64 KB where the merge buffer beside them is small enough for two workgroups
-// per compute unit (what the registers allow), else 32 KB.
-// Two workgroups per compute unit share 160 KB of LDS: the logits take what the merge buffer (4 G D floats) leaves of
-// 80 KB, in whole pairs of steps of the widest kernel (256 keys).
-constexpr int logit_floats(int G, int D) { return G * D <= 512 ? 16384 : (G * D <= 1024 ? (G == 16 ? 12288 : 14336) : 8192); }
+// Logits a workgroup holds in LDS, in whole pairs of steps of the widest kernel (256 keys). Two workgroups per compute
+// unit share 160 KB of LDS: the logits take what the merge buffer (4 G D floats) leaves of 80 KB. At head size 256 the
+// kernel over codes takes 320 to 370 registers and has its compute unit to itself: the logits take what is left of the
+// whole 160 KB, so that rows of many heads run in one round of splits instead of three (16 rows of 35407 8-bit keys, 7 heads
+// each, with weights: 133 -> 73 us).
+constexpr int logit_floats(int G, int D, bool codes) {
+  if (D == 256 && codes) return G == 8 ? 30720 : 32768;
+  return G * D <= 512 ? 16384 : (G * D <= 1024 ? (G == 16 ? 12288 : 14336) : 8192);
+}
 constexpr int kCountStride = 64;  // a row's counters have 256 bytes to themselves: the polls of different rows go to different channels
 constexpr int kArrived = 0, kFinished = 1, kSelected = 2;
 static_assert(kCountStride == kDecodeCounterStride, "the slot write clears these counters");
@@ -514,7 +518,7 @@ __global__ __launch_bounds__(NTHREADS) void decode_split_kernel(const DecodePara
   constexpr int RPI = 64 / LPR;  // rows per load instruction of a wavefront
   constexpr int U = 4;           // load instructions per step and tensor (even: rows pair up for dot2)
   constexpr int CH = U * RPI;    // keys per wavefront and step, contiguous
-  constexpr int LGK = logit_floats(G, D) / G;  // keys whose logits are gathered in LDS before they go out in one burst
+  constexpr int LGK = logit_floats(G, D, false) / G;  // keys whose logits are gathered in LDS before they go out in one burst
   __shared__ __align__(16) float lgbuf[LGK * G];  // [key][head]
   __shared__ __align__(16) float red[WAVES][G][D];
   __shared__ float rml[WAVES][G][2];
@@ -755,7 +759,7 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
   constexpr int NL4 = D >= 128 ? D / 128 : 1;                              // 4-bit rows: 16-byte loads per key of K
   constexpr int KR = U4 ? NL4 : (U8 ? D / 64 : KJ);                        // 16-byte loads per key of K
   constexpr int VW = U4 ? (DPL + 7) / 8 : (U8 ? (DPL + 3) / 4 : DPL / 2);  // dwords per key of V
-  constexpr int LGK = logit_floats(G, D) / G;
+  constexpr int LGK = logit_floats(G, D, U8) / G;
   __shared__ __align__(16) float lgbuf[LGK * G];  // [key][head]
   __shared__ __align__(16) float red[WAVES][G][D];
   __shared__ float rml[WAVES][G][2];
@@ -1249,7 +1253,7 @@ Plan make_plan(const kvx_sdpa_args& a, bool fused_h2o) {
   // 13.1 -> 11.8. 64 rows of 32768 keys take 170 in two rounds of 4096 keys, 183 in splits of 1024.
   const bool weights = a.w || fused_h2o;
   const int allow_resident = weights ? tuning().resident.load() : 0;
-  const int lgk = logit_floats(pl.G, a.D) / pl.G;
+  const int lgk = logit_floats(pl.G, a.D, !kv_is_plain(a.kv_dtype)) / pl.G;
   int splits = a.num_splits;
   if (splits <= 0) {
     const int64_t rows = (int64_t)a.B * a.Hkv, cus = num_cus();

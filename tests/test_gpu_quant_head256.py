@@ -97,3 +97,21 @@ def test_attention_over_quantised_cache_256(kvx, gpu, bits, dtype, B, Hq, Hkv, q
     torch.cuda.synchronize()
     assert rel_err(out1.float().cpu().unsqueeze(2), o1_ref.float()) < 2e-2
     torch.testing.assert_close(w1.cpu(), w1_ref, rtol=1e-3, atol=1e-6)
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("Hq,T", [(8, 3840), (8, 3841), (4, 8192), (3, 8256), (1, 4000)])
+def test_single_token_logits_at_the_room_a_split_has(gpu, bits, Hq, T):
+    """One split, its logits just inside and just beyond what a workgroup holds (3840 keys of 8 heads, 8192 of 4): on the
+    chip or through the scratch, same results."""
+    gen = torch.Generator().manual_seed(T)
+    q, k, v = (torch.randn(1, h, n, D, generator=gen).to(torch.bfloat16) for h, n in ((Hq, 1), (1, T), (1, T)))
+    (kc, ks, kz), (vc, vs, vz) = O.quantize_rows(k, bits), O.quantize_rows(v, bits)
+    want, w_ref = O.sdpa_in_blocks(q, O.dequantize_rows(kc, ks, kz, torch.bfloat16), O.dequantize_rows(vc, vs, vz, torch.bfloat16), D ** -0.5, 10 * T, None)
+    if bits == 4:
+        kc, vc = O.compress4(kc), O.compress4(vc)
+    quant = ops.QuantState(*(t.to(gpu) for t in (ks, kz, vs, vz)))
+    for splits in (1, 0):
+        out, w, _ = ops.decode_core(q.to(gpu), kc.to(gpu), vc.to(gpu), D ** -0.5, return_weights=True, quant=quant, num_splits=splits)
+        assert rel_err(out.float().cpu().unsqueeze(2), want.float()) < 2e-2
+        torch.testing.assert_close(w.cpu(), w_ref, rtol=1e-3, atol=1e-6)
