@@ -7,7 +7,7 @@
 #include <stdio.h>
 #include <string.h>
 
-#include "kvx_common.h"
+#include "prefill_merge.h"
 
 namespace kvx {
 
@@ -145,9 +145,11 @@ int kvx_sdpa_prefill_weights(const kvx_sdpa_args* a, void* stream) {
               a->kv_len);
   KVX_REQUIRE(a->lse && a->w, KVX_ERR_INVALID, "kvx_sdpa_prefill_weights: lse and w must be given");
   KVX_REQUIRE(aligned16(a->workspace), KVX_ERR_WORKSPACE, "kvx_sdpa_prefill_weights: workspace must be 16-byte aligned");
-  rc = launch_sdpa_prefill(*a, (hipStream_t)stream);
+  MergeParams rest{};
+  const bool combines = score_sum_combines(*a);
+  rc = launch_sdpa_prefill(*a, (hipStream_t)stream, combines ? &rest : nullptr);
   if (rc != KVX_OK) return rc;
-  return launch_score_sum(*a, (hipStream_t)stream);
+  return launch_score_sum(*a, (hipStream_t)stream, combines ? &rest : nullptr);
 }
 
 size_t kvx_sdpa_decode_workspace_bytes(const kvx_sdpa_args* a) {

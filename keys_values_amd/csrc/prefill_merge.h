@@ -1,0 +1,93 @@
+// The combination of the attention kernel's per-split partials, as a job of one workgroup: the combining kernel
+// (sdpa_prefill.hip) runs it alone, the score-sum kernel of short chunks (score_sum.hip) beside its own work.
+#pragma once
+#include "kvx_common.h"
+
+namespace kvx {
+
+struct MergeParams {
+  const float* part_o;   // [split][group][R][D] fp32, unnormalised
+  const float* part_ml;  // [split][group][R][2]  (max in log2 units, sum)
+  uint16_t* o;
+  float* lse;  // (B, q_len, Hq) or NULL
+  int32_t B, Hq, Hkv, G, q_len, R, num_splits;
+  int64_t o_sb, o_sh, o_st;
+};
+
+// Combine the per-split partials of a row: D / 4 threads a row, each four values, times SC split classes that take
+// splits j, j + SC, ... and are added through LDS. Bound by HBM (every partial is read once) where there are many rows;
+// with few rows (32 queries over 32768 keys: 1024 rows of 32 splits) a thread's walk over the splits was the time, a memory
+// latency per split and 15 us of a 46 us call: four loads in flight and SC classes make it about two latencies.
+// ROWS: rows of one workgroup of 256 threads.
+constexpr int merge_rows(int D, int SC) { return 256 / (D / 4 * SC); }
+// split classes while a walk is longer than four splits and the rows alone leave the device short of threads
+constexpr int merge_classes(int D) { return 256 / (D / 4) < 8 ? 256 / (D / 4) : 8; }
+inline bool merge_wants_classes(const MergeParams& p, int D) {
+  return p.num_splits > 4 && (int64_t)p.B * p.Hkv * p.R * (D / 4) < (int64_t)num_cus() * 256;
+}
+template <int D, bool F16, int SC>
+__device__ __forceinline__ void merge_job(const MergeParams& p, const int64_t block) {
+  constexpr int TPR = D / 4;                // threads per row and split class
+  constexpr int ROWS = merge_rows(D, SC);    // rows per workgroup
+  static_assert(ROWS >= 1, "a row's threads fit a workgroup");
+  __shared__ f32x4_t red_o[SC > 1 ? 256 : 1];
+  __shared__ float red_l[SC > 1 ? 256 : 1];
+  const int S = p.num_splits;
+  const int64_t total_rows = (int64_t)p.B * p.Hkv * p.R;
+  const int64_t grow = block * ROWS + threadIdx.x / (TPR * SC);
+  const bool live = grow < total_rows;
+  const int64_t growc = live ? grow : total_rows - 1;
+  const int dq = threadIdx.x % TPR, j = (threadIdx.x / TPR) % SC;
+  const f32x2_t* ml = (const f32x2_t*)p.part_ml + growc;  // (maximum, sum) of split s at s * total_rows
+  const float* po = p.part_o + growc * D + dq * 4;
+  float M = -INFINITY;
+  for (int s0 = 0; s0 < S; s0 += 4) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) M = fmaxf(M, ml[(int64_t)min(s0 + u, S - 1) * total_rows][0]);
+  }
+  const float Mu = (M == -INFINITY) ? 0.0f : M;
+  float L = 0.0f;
+  f32x4_t acc = {0, 0, 0, 0};
+  for (int s0 = j; s0 < S; s0 += 4 * SC) {
+    f32x2_t m[4];
+    f32x4_t x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t at = (int64_t)min(s0 + u * SC, S - 1) * total_rows;
+      m[u] = ml[at];
+      x[u] = *(const f32x4_t*)(po + at * D);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (s0 + u * SC < S) {
+        const float w = fast_exp2(m[u][0] - Mu);
+        L += m[u][1] * w;
+        acc += x[u] * w;
+      }
+  }
+  if constexpr (SC > 1) {
+    red_o[threadIdx.x] = acc;
+    red_l[threadIdx.x] = L;
+    __syncthreads();
+    if (j != 0) return;
+#pragma unroll
+    for (int i = 1; i < SC; ++i) {
+      acc += red_o[threadIdx.x + i * TPR];
+      L += red_l[threadIdx.x + i * TPR];
+    }
+  }
+  if (!live) return;
+  const int group = (int)(grow / p.R);
+  const int row = (int)(grow % p.R);
+  const int b = group / p.Hkv, kvh = group % p.Hkv;
+  const int qi = row / p.G, g = row % p.G;
+  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+  uint16_t* op = p.o + b * p.o_sb + (int64_t)(kvh * p.G + g) * p.o_sh + (int64_t)qi * p.o_st + dq * 4;
+  u32x2_t w2;
+  w2[0] = pack_pair<F16>(acc[0] * inv, acc[1] * inv);
+  w2[1] = pack_pair<F16>(acc[2] * inv, acc[3] * inv);
+  *(u32x2_t*)op = w2;
+  if (p.lse && dq == 0) p.lse[((int64_t)b * p.q_len + qi) * p.Hq + kvh * p.G + g] = Mu + fast_log2(L);
+}
+
+}  // namespace kvx

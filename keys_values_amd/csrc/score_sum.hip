@@ -13,7 +13,7 @@
 // per-lane running sum and the two halves of the wavefront are added once at the end.
 #include <type_traits>
 
-#include "kvx_common.h"
+#include "prefill_merge.h"
 
 namespace kvx {
 namespace {
@@ -410,6 +410,165 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
   }
 }
 
+// Short chunks: the same sums with the query rows split over the four wavefronts of a workgroup instead of streamed past
+// each of them. A workgroup owns 64 keys, held by every wavefront as B operands; wavefront w takes the 32-row blocks w,
+// w + 4, ... straight from memory (the next block's rows are fetched while one is worked on, no LDS, no barriers in the
+// loop), and the four sums are added in order at the end. What bounds the kernel above on few rows is its serial walk: a
+// wavefront meets every tile of 64 rows, about 1 us each, whatever the number of keys, with a barrier a tile; here the walk is a
+// quarter as long and a workgroup four (eight) times as small, and the partials of the attention kernel's KV splits are
+// combined in the same launch: the first workgroups take 64 keys each and work out the rows' log-sum-exps from the splits'
+// (maximum, sum) pairs for themselves, the others write the outputs. Rows are read from the L2 once per 64 keys instead of
+// once per 256 or 512, which is why many rows keep the kernel above.
+constexpr int SHORT_ROWS = 1024;  // rows whose log-sum-exps and positions the workgroup keeps in LDS
+
+template <int D, int KV, int SC>
+__global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void score_sum_short_kernel(const ScoreParams p, const MergeParams m, const int score_jobs) {
+  constexpr bool F16 = kv_elem_f16(KV);
+  constexpr int KS = D / 16;
+  if ((int)blockIdx.x >= score_jobs) {
+    merge_job<D, F16, SC>(m, (int)blockIdx.x - score_jobs);
+    return;
+  }
+  __shared__ __align__(16) float lse_sh[SHORT_ROWS];
+  __shared__ __align__(16) int32_t qpos_sh[SHORT_ROWS];
+  __shared__ float red[4][NW];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31;
+  const int h = lane >> 5;
+  const int groups = p.B * p.Hkv;
+  const int group = blockIdx.x % groups;  // fastest: a KV head's query rows stay on one XCD
+  const int b = group / p.Hkv, kvh = group % p.Hkv;
+  const int key0 = (int)blockIdx.x / groups * NW;
+  const float inv_G = 1.0f / (float)p.G;  // (int)((r + 0.5f) * inv_G) == r / G for the r < 1024 of a chunk
+  auto query_of = [&](int r) { return (int)(((float)r + 0.5f) * inv_G); };
+  const uint16_t* qbase = p.q + b * p.q_sb + (int64_t)(kvh * p.G) * p.q_sh;
+
+  // Q fragments (A operand) of a block of 32 rows: lane holds row n, d = 16 j + 8 h .. +8; rows past the end re-read the last one
+  auto load_q = [&](u32x4_t (&qq)[KS], int blk) {
+    const int r = min(blk * 32 + n, p.R - 1);
+    const int qi = query_of(r);
+    const uint16_t* qp = qbase + (int64_t)(r - qi * p.G) * p.q_sh + (int64_t)qi * p.q_st + 8 * h;
+#pragma unroll
+    for (int j = 0; j < KS; ++j) qq[j] = *(const u32x4_t*)(qp + 16 * j);
+  };
+  const int nblk = (p.R + 31) / 32;
+  u32x4_t qa[KS], qb[KS];
+  load_q(qa, min(wave, nblk - 1));
+
+  // K fragments (B operand): lane holds key column n of tile nt, d = 16 j + 8 h .. +8; keys past the end re-read the last
+  // one (nothing of theirs is stored)
+  u32x4_t kf[2][KS];
+  int32_t tpk[2];
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt) {
+    const int key = min(key0 + nt * 32 + n, p.kv_len - 1);
+    tpk[nt] = p.tp ? p.tp[b * p.tp_sb + kvh * p.tp_sh + key] : key;
+    if constexpr (kv_is_plain(KV)) {
+      const uint16_t* kp = (const uint16_t*)p.k + b * p.k_sb + kvh * p.k_sh + (int64_t)key * p.k_st + 8 * h;
+#pragma unroll
+      for (int j = 0; j < KS; ++j) kf[nt][j] = *(const u32x4_t*)(kp + 16 * j);
+    } else {
+      const uint8_t* kp = (const uint8_t*)p.k + b * p.k_sb + kvh * p.k_sh + (int64_t)key * p.k_st;
+      const int64_t so = b * p.qs_sb + kvh * p.qs_sh + key;
+      const float sc = p.k_scale[so];
+      const int32_t zp = p.k_zp[so];
+#pragma unroll
+      for (int j = 0; j < KS; ++j) {
+        u32x2_t cc;
+        if constexpr (kv_is_u4(KV)) cc = u4_codes(*(const u32x2_t*)(kp + u4_byte_off<D>(2 * j + h)), u4_shift<D>(2 * j + h));
+        else cc = *(const u32x2_t*)(kp + 16 * j + 8 * h);
+        kf[nt][j] = dequant_words<F16>(cc[0], cc[1], zp, sc);
+      }
+    }
+  }
+
+  // the rows' base-2 log-sum-exps and positions; rows up to the end of the last block weigh nothing
+  const int S = m.num_splits;
+  const int64_t total_rows = (int64_t)groups * p.R;
+  for (int r = tid; r < nblk * 32; r += 256) {
+    const bool ok = r < p.R;
+    const int rc = min(r, p.R - 1), qi = query_of(rc);
+    float lse;
+    if (S <= 1) {
+      lse = p.lse[((int64_t)b * p.q_len + qi) * p.Hq + kvh * p.G + (rc - qi * p.G)];
+    } else {
+      const f32x2_t* ml = (const f32x2_t*)m.part_ml + (int64_t)group * p.R + rc;
+      float M = -INFINITY, L = 0.0f;
+      for (int s0 = 0; s0 < S; s0 += 16) {  // 16 splits a memory latency
+        f32x2_t x[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) x[u] = ml[(int64_t)min(s0 + u, S - 1) * total_rows];
+        float Mn = M;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) Mn = fmaxf(Mn, x[u][0]);
+        const float Mu = Mn == -INFINITY ? 0.0f : Mn;
+        L *= fast_exp2(M - Mu);
+        M = Mn;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) L += s0 + u < S ? x[u][1] * fast_exp2(x[u][0] - Mu) : 0.0f;
+      }
+      lse = (M == -INFINITY ? 0.0f : M) + fast_log2(L);
+    }
+    lse_sh[r] = ok ? lse : INFINITY;
+    qpos_sh[r] = p.input_pos + qi;
+  }
+  int tpmax = max(tpk[0], tpk[1]);
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) tpmax = max(tpmax, __shfl_xor(tpmax, off, 64));
+  tpmax = __builtin_amdgcn_readfirstlane(tpmax);
+  __syncthreads();
+
+  float wacc[2] = {0.0f, 0.0f};
+  auto block = [&](const u32x4_t (&qq)[KS], int blk) {
+    f32x16_t s[2];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[nt][i] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < KS; ++j)
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) s[nt] = mfma_32x32x16<F16>(qq[j], kf[nt][j], s[nt]);
+    const bool masked = tpmax > p.input_pos + query_of(blk * 32);
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const f32x4_t ls = *(const f32x4_t*)&lse_sh[blk * 32 + 8 * a + 4 * h];
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        float e[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) e[i] = fast_exp2(fmaf(s[nt][4 * a + i], p.c, -ls[i]));
+        if (masked) {
+          const int4 qp = *(const int4*)&qpos_sh[blk * 32 + 8 * a + 4 * h];
+          e[0] = tpk[nt] > qp.x ? 0.0f : e[0];
+          e[1] = tpk[nt] > qp.y ? 0.0f : e[1];
+          e[2] = tpk[nt] > qp.z ? 0.0f : e[2];
+          e[3] = tpk[nt] > qp.w ? 0.0f : e[3];
+        }
+        wacc[nt] += (e[0] + e[1]) + (e[2] + e[3]);
+      }
+    }
+  };
+  for (int blk = wave; blk < nblk; blk += 8) {
+    if (blk + 4 < nblk) load_q(qb, blk + 4);
+    block(qa, blk);
+    if (blk + 4 < nblk) {
+      if (blk + 8 < nblk) load_q(qa, blk + 8);
+      block(qb, blk + 4);
+    }
+  }
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt) {
+    const float t = sum_halves(wacc[nt]);
+    if (h == 0) red[wave][nt * 32 + n] = t;
+  }
+  __syncthreads();
+  if (tid < NW && key0 + tid < p.kv_len)
+    p.w[(int64_t)group * p.kv_len + key0 + tid] = (((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid]) * p.inv_g;
+}
+
 // W = (1/G) * (part[0] + part[1] + ...), in that order.
 __global__ void score_sum_reduce_kernel(const float* part, float* w, int64_t n, int splits, float inv_g) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -439,9 +598,31 @@ ScorePlan score_plan(const kvx_sdpa_args& a) {
   return pl;
 }
 
+// Few rows over few keys take the short kernel: 64 keys a workgroup then still leave one compute unit a workgroup, and the
+// wavefronts that walk the query rows side by side would idle otherwise. Attention with weights, us, long -> short kernel:
+// 2 KV heads x 1024 keys of 64, 128 / 512 / 1024 / 2000 rows 16.0 -> 12.3, 23.7 -> 17.3, 26.5 -> 24.2, 30.9 -> 37.9; 8 x 1024 of 128,
+// the same rows 23.4 -> 21.2, 34.9 -> 27.7, 39.9 -> 36.4, 46.2 -> 53.8. With more keys every wavefront of the long kernel
+// has work of its own and reads a quarter of the query rows: 8 x 4096 of 128, 512 rows 38.1 -> 42.5.
+bool is_short(const kvx_sdpa_args& a) {
+  return (int64_t)a.q_len * (a.Hq / a.Hkv) <= SHORT_ROWS && (int64_t)a.B * a.Hkv * ((a.kv_len + NW - 1) / NW) <= num_cus();
+}
+
 template <int D, int KV>
-int launch_t(const ScoreParams& p, int splits, hipStream_t st) {
+int launch_t(const ScoreParams& p, int splits, const MergeParams* rest, bool brief, hipStream_t st) {
   const int groups = p.B * p.Hkv;
+  if (brief) {
+    const int64_t score_jobs = (int64_t)groups * ((p.kv_len + NW - 1) / NW);
+    const MergeParams m = rest ? *rest : MergeParams{};
+    auto launch = [&](auto sc_tag) {
+      constexpr int SC = decltype(sc_tag)::value, ROWS = merge_rows(D, SC);
+      const int64_t merge_jobs = m.num_splits > 1 ? ((int64_t)groups * p.R + ROWS - 1) / ROWS : 0;
+      hipLaunchKernelGGL((score_sum_short_kernel<D, KV, SC>), dim3((unsigned)(score_jobs + merge_jobs)), dim3(256), 0, st, p, m, (int)score_jobs);
+    };
+    if (merge_wants_classes(m, D)) launch(std::integral_constant<int, merge_classes(D)>{});
+    else launch(std::integral_constant<int, 1>{});
+    KVX_HIP(hipGetLastError());
+    return KVX_OK;
+  }
   if (splits > 1) {
     hipLaunchKernelGGL((score_sum_kernel<D, KV, 4, true>), dim3(groups, (p.kv_len + 4 * NW - 1) / (4 * NW), splits), dim3(256), 0, st, p);
     KVX_HIP(hipGetLastError());
@@ -466,11 +647,14 @@ int launch_t(const ScoreParams& p, int splits, hipStream_t st) {
 }  // namespace
 
 size_t score_sum_workspace(const kvx_sdpa_args& a) {
+  if (is_short(a)) return 0;
   const ScorePlan pl = score_plan(a);
   return pl.splits > 1 ? (size_t)pl.splits * a.B * a.Hkv * a.kv_len * sizeof(float) : 0;
 }
 
-int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st) {
+bool score_sum_combines(const kvx_sdpa_args& a) { return is_short(a); }
+
+int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* rest) {
   // the query rows are split only if the caller's workspace holds the partial sums
   ScorePlan pl = score_plan(a);
   if (pl.splits > 1 && !(a.workspace && a.workspace_bytes >= score_sum_workspace(a) && ((uintptr_t)a.workspace & 15) == 0)) pl.splits = 1;
@@ -501,7 +685,8 @@ int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st) {
   p.tp_sb = a.tp_stride_b; p.tp_sh = a.tp_stride_h;
 #define KVX_SCORE_SUM_CASE(KV) \
   case KV: \
-    return a.D == 256 ? launch_t<256, KV>(p, pl.splits, st) : a.D == 128 ? launch_t<128, KV>(p, pl.splits, st) : launch_t<64, KV>(p, pl.splits, st);
+    return a.D == 256 ? launch_t<256, KV>(p, pl.splits, rest, is_short(a), st) : a.D == 128 ? launch_t<128, KV>(p, pl.splits, rest, is_short(a), st) \
+                                                                      : launch_t<64, KV>(p, pl.splits, rest, is_short(a), st);
   if (a.D == 256 || a.D == 128 || a.D == 64) {
     switch (a.kv_dtype) {
       KVX_SCORE_SUM_CASE(KVX_KV_BF16)

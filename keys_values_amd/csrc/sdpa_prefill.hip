@@ -22,7 +22,7 @@
 #include <type_traits>
 #include <utility>
 
-#include "kvx_common.h"
+#include "prefill_merge.h"
 
 namespace kvx {
 namespace {
@@ -605,74 +605,8 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
   }
 }
 
-// Combine the per-split partials of a row: D / 4 threads a row, each four values, times SC split classes that take
-// splits j, j + SC, ... and are added through LDS. Bound by HBM (every partial is read once) where there are many rows;
-// with few rows (32 queries over 32768 keys: 1024 rows of 32 splits) a thread's walk over the splits was the time, a memory
-// latency per split and 15 us of a 46 us call: four loads in flight and SC classes make it about two latencies.
 template <int D, bool F16, int SC>
-__global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(const PrefillParams p) {
-  constexpr int TPR = D / 4;                // threads per row and split class
-  constexpr int ROWS = 256 / (TPR * SC);    // rows per workgroup
-  static_assert(ROWS >= 1, "a row's threads fit a workgroup");
-  __shared__ f32x4_t red_o[SC > 1 ? 256 : 1];
-  __shared__ float red_l[SC > 1 ? 256 : 1];
-  const int S = p.num_splits;
-  const int64_t total_rows = (int64_t)p.B * p.Hkv * p.R;
-  const int64_t grow = (int64_t)blockIdx.x * ROWS + threadIdx.x / (TPR * SC);
-  const bool live = grow < total_rows;
-  const int64_t growc = live ? grow : total_rows - 1;
-  const int dq = threadIdx.x % TPR, j = (threadIdx.x / TPR) % SC;
-  const f32x2_t* ml = (const f32x2_t*)p.part_ml + growc;  // (maximum, sum) of split s at s * total_rows
-  const float* po = p.part_o + growc * D + dq * 4;
-  float M = -INFINITY;
-  for (int s0 = 0; s0 < S; s0 += 4) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) M = fmaxf(M, ml[(int64_t)min(s0 + u, S - 1) * total_rows][0]);
-  }
-  const float Mu = (M == -INFINITY) ? 0.0f : M;
-  float L = 0.0f;
-  f32x4_t acc = {0, 0, 0, 0};
-  for (int s0 = j; s0 < S; s0 += 4 * SC) {
-    f32x2_t m[4];
-    f32x4_t x[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int64_t at = (int64_t)min(s0 + u * SC, S - 1) * total_rows;
-      m[u] = ml[at];
-      x[u] = *(const f32x4_t*)(po + at * D);
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (s0 + u * SC < S) {
-        const float w = fast_exp2(m[u][0] - Mu);
-        L += m[u][1] * w;
-        acc += x[u] * w;
-      }
-  }
-  if constexpr (SC > 1) {
-    red_o[threadIdx.x] = acc;
-    red_l[threadIdx.x] = L;
-    __syncthreads();
-    if (j != 0) return;
-#pragma unroll
-    for (int i = 1; i < SC; ++i) {
-      acc += red_o[threadIdx.x + i * TPR];
-      L += red_l[threadIdx.x + i * TPR];
-    }
-  }
-  if (!live) return;
-  const int group = (int)(grow / p.R);
-  const int row = (int)(grow % p.R);
-  const int b = group / p.Hkv, kvh = group % p.Hkv;
-  const int qi = row / p.G, g = row % p.G;
-  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-  uint16_t* op = p.o + b * p.o_sb + (int64_t)(kvh * p.G + g) * p.o_sh + (int64_t)qi * p.o_st + dq * 4;
-  u32x2_t w2;
-  w2[0] = pack_pair<F16>(acc[0] * inv, acc[1] * inv);
-  w2[1] = pack_pair<F16>(acc[2] * inv, acc[3] * inv);
-  *(u32x2_t*)op = w2;
-  if (p.lse && dq == 0) p.lse[((int64_t)b * p.q_len + qi) * p.Hq + kvh * p.G + g] = Mu + fast_log2(L);
-}
+__global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(const MergeParams p) { merge_job<D, F16, SC>(p, blockIdx.x); }
 
 // The number of KV splits with the least estimated time: c workgroups share a compute unit, one after the other or side by
 // side, and each walks its split's tiles; more splits balance the device better and shorten the walk, but every partial
@@ -748,21 +682,25 @@ size_t partial_bytes(const PrefillParams& p, int D) {
   return rows * (size_t)D * 4 + rows * 2 * 4;
 }
 
+// `rest`: where the partials are left for another launch to combine, their description (num_splits 1: nothing to combine)
 template <int D, int KV>
-int launch_t(PrefillParams& p, hipStream_t st) {
+int launch_t(PrefillParams& p, hipStream_t st, MergeParams* rest) {
   dim3 grid(p.B * p.Hkv, p.m_blocks, p.num_splits);
   hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
   KVX_HIP(hipGetLastError());
+  const MergeParams m = {p.part_o, p.part_ml, p.o, p.lse, p.B, p.Hq, p.Hkv, p.G, p.q_len, p.R, p.num_splits, p.o_sb, p.o_sh, p.o_st};
+  if (rest) {
+    *rest = m;
+    return KVX_OK;
+  }
   if (p.num_splits > 1) {
     const int64_t total_rows = (int64_t)p.B * p.Hkv * p.R;
     auto merge = [&](auto sc_tag) {
-      constexpr int SC = decltype(sc_tag)::value, ROWS = 256 / (D / 4 * SC);
-      hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kv_elem_f16(KV), SC>), dim3((unsigned)((total_rows + ROWS - 1) / ROWS)), dim3(256), 0, st, p);
+      constexpr int SC = decltype(sc_tag)::value, ROWS = merge_rows(D, SC);
+      hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kv_elem_f16(KV), SC>), dim3((unsigned)((total_rows + ROWS - 1) / ROWS)), dim3(256), 0, st, m);
     };
-    // split classes while a walk is longer than four splits and the rows alone leave the device short of threads
-    constexpr int MAX_SC = 256 / (D / 4) < 8 ? 256 / (D / 4) : 8;
-    if (p.num_splits <= 4 || total_rows * (D / 4) >= (int64_t)num_cus() * 256) merge(std::integral_constant<int, 1>{});
-    else merge(std::integral_constant<int, MAX_SC>{});
+    if (merge_wants_classes(m, D)) merge(std::integral_constant<int, merge_classes(D)>{});
+    else merge(std::integral_constant<int, 1>{});
     KVX_HIP(hipGetLastError());
   }
   return KVX_OK;
@@ -804,7 +742,7 @@ size_t sdpa_prefill_workspace(const kvx_sdpa_args& a) {
   return own > after ? own : after;
 }
 
-int launch_sdpa_prefill(const kvx_sdpa_args& a_in, hipStream_t st) {
+int launch_sdpa_prefill(const kvx_sdpa_args& a_in, hipStream_t st, MergeParams* rest) {
   PrefillParams p;
   kvx_sdpa_args a = a_in;
   if (wants_copy(a)) {
@@ -829,7 +767,7 @@ int launch_sdpa_prefill(const kvx_sdpa_args& a_in, hipStream_t st) {
     p.part_ml = p.part_o + rows * (size_t)a.D;
   }
 #define KVX_PREFILL_CASE(KV) \
-  case KV: return a.D == 256 ? launch_t<256, KV>(p, st) : a.D == 128 ? launch_t<128, KV>(p, st) : launch_t<64, KV>(p, st);
+  case KV: return a.D == 256 ? launch_t<256, KV>(p, st, rest) : a.D == 128 ? launch_t<128, KV>(p, st, rest) : launch_t<64, KV>(p, st, rest);
   if (a.D == 256 || a.D == 128 || a.D == 64) {
     switch (a.kv_dtype) {
       KVX_PREFILL_CASE(KVX_KV_BF16)

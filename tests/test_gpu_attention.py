@@ -129,6 +129,40 @@ def test_score_sum_with_eight_wavefront_workgroups(gpu, store):
     torch.testing.assert_close(w.sum(-1).cpu(), torch.full((B, Hkv), float(q_len)), rtol=1e-4, atol=1e-3)
 
 
+@pytest.mark.parametrize("store", ["bf16", "u8", "u4"])
+@pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D,splits", [
+    (1, 1, 1, 2, 2, 64, 0),          # less than a block of rows, a handful of keys
+    (1, 7, 1, 9, 65, 128, 0),        # 63 rows, one key beyond a workgroup's 64
+    (2, 6, 2, 43, 190, 128, 3),      # 129 rows of 3 heads
+    (1, 8, 2, 256, 1087, 64, 17),    # 1024 rows, the most; one split more than a pass over the partials takes
+    (1, 2, 1, 16, 2200, 64, 33),     # the partials in three passes
+    (1, 12, 1, 85, 700, 256, 2),     # 1020 rows of 12 heads
+    (1, 5, 1, 205, 640, 128, 2),     # 1025 rows: the long kernel
+])
+def test_score_sums_of_few_rows_over_few_keys(gpu, store, B, Hq, Hkv, q_len, T, D, splits):
+    # score-sums and the combination of the KV splits in one launch; tolerances of the path
+    q, k, v, gen = make_qkv(310 + T, B, Hq, Hkv, q_len, T, D)
+    quant = None
+    kd, vd = k.to(gpu), v.to(gpu)
+    if store != "bf16":
+        bits = 8 if store == "u8" else 4
+        (kc, ks, kz), (vc, vs, vz) = ([t.view(B, Hkv, T, -1) if t.dim() > 1 else t.view(B, Hkv, T) for t in O.quantize_rows(x.reshape(-1, D), bits)] for x in (k, v))
+        k, v = ((O.dequantize_rows(c.reshape(-1, D), s.reshape(-1), z.reshape(-1), torch.bfloat16)).view(B, Hkv, T, D) for c, s, z in ((kc, ks, kz), (vc, vs, vz)))
+        if bits == 4:
+            kc, vc = (O.compress4(c.reshape(-1, D)).view(B, Hkv, T, D // 2) for c in (kc, vc))
+        kd, vd = kc.to(gpu), vc.to(gpu)
+        quant = ops.QuantState(*(t.to(gpu) for t in (ks, kz, vs, vz)))
+    tp = scattered_positions(gen, B, Hkv, T, 2 * T, q_len)
+    scale = 1.0 / math.sqrt(D)
+    for pos, tpos in ((2 * T, tp), (T - q_len, None)):
+        o_ref, w_ref = O.sdpa_in_blocks(q, k, v, scale, pos, None if tpos is None else tpos.to(torch.int64))
+        out, w, lse = ops.prefill_core(q.to(gpu), kd, vd, scale, pos, None if tpos is None else tpos.to(gpu), return_weights=True, return_lse=True,
+                                       output_transposed=False, quant=quant, num_splits=splits)
+        check_o(out, o_ref)
+        check_w(w, w_ref, q_len)
+        torch.testing.assert_close(lse.cpu(), O.lse2(q, k, scale, pos, tpos), rtol=1e-4, atol=1e-3)
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D", [(1, 8, 2, 700, 900, 128), (2, 4, 1, 1100, 1100, 64), (1, 16, 2, 300, 2048, 128)])
 def test_score_sum_over_split_query_rows(kvx, gpu, B, Hq, Hkv, q_len, T, D):
     # a short cache: with a workspace the query rows are split over several workgroups and the partial sums
