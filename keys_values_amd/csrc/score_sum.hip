@@ -21,8 +21,8 @@ namespace {
 constexpr int BQ = 64;    // query rows per LDS tile
 constexpr int NW = 64;    // keys per wavefront
 // Wavefronts per workgroup, a template argument W: 8 (512 keys per workgroup, one workgroup per compute unit: the
-// Q tile staged into LDS serves twice the keys, 4 % on the kernel) when that still gives every compute unit a
-// workgroup, else 4 (256 keys, two workgroups per compute unit).
+// Q tile staged into LDS serves twice the keys, 4 % on the kernel) or 4 (256 keys, two workgroups per compute unit); see
+// score_plan.
 
 struct ScoreParams {
   const uint16_t* q;
@@ -34,6 +34,7 @@ struct ScoreParams {
   float* w;
   float* part;           // query rows split over several workgroups: (splits, B, Hkv, kv_len) partial sums, else NULL
   int32_t tiles_per_z;   // query tiles per split
+  int32_t rows_per_tile; // see tile_rows
   int32_t B, Hq, Hkv, G, q_len, kv_len, R, input_pos;
   float c, inv_g;
   int64_t q_sb, q_sh, q_st, k_sb, k_sh, k_st, qs_sb, qs_sh, tp_sb, tp_sh;
@@ -53,16 +54,25 @@ struct alignas(16) Smem {
   int32_t qpos[4][BQ];  // read through the whole step (only by tiles that need the mask): a ring of four
 };
 
+// Rows of a tile: as many whole queries as its BQ rows hold (G = 7: 63, G = 12: 60), the rest of the tile stays empty. Every
+// row then keeps its head from tile to tile and the steady steps serve any group size; with full tiles a group that does not
+// divide 64 went through the general step, bounds checks and mask on every tile (attention with weights, 2 x 4 KV heads, 4096 rows
+// of 7 heads over 5001 keys 168 -> 157 us; 2 x 8, 4096 rows of 3 heads over 6000 333 -> 322). Where that would leave
+// more than an eighth of the tile empty (G = 24), and beyond 64 heads, tiles are full and the general step does it.
+constexpr int tile_rows(int G) { return G <= BQ && BQ / G * G >= BQ - BQ / 8 ? BQ / G * G : BQ; }
+
 // Streams the packed query rows (row r = query r / G, head r % G) of one (batch, KV head) pair into LDS, tile by
 // tile, with global -> LDS transfers: no registers hold the rows on their way. Wavefront w issues instructions
 // w, w + W, ... of the CPR that make a tile (RPW = 64 / CPR rows each); lane l of instruction i fills LDS position
 // l % CPR of row i RPW + l / CPR, so it fetches the chunk that belongs there under the swizzle. Addresses are a
 // uniform base plus a 32-bit byte offset per lane (the host checks the range). Wavefront 0 also fetches the rows'
 // log-sum-exps (4 bytes per lane) and writes their positions.
-//   issue_steady: G divides the tile height and the tile is full. Every row keeps its head and moves by BQ / G
+//   issue_steady: the tile is one of whole queries and full. Every row keeps its head and moves by BQ / G
 //     queries from tile to tile: the base advances by scalar adds and the lane offsets stay.
 //   issue: any tile. The offsets are formed per lane from the row's (query, head); rows past the end re-read the
-//     last valid row, and land() overwrites their log-sum-exp with +inf, so their weight is exactly zero.
+//     last valid row.
+//   land() overwrites the log-sum-exps of the rows a tile leaves empty and of those past the end with +inf: their weight
+//     is exactly zero.
 template <int D, int W>
 struct QLoader {
   static constexpr int CPR = D / 8;
@@ -80,7 +90,7 @@ struct QLoader {
   int rin[NI];         // row inside the tile
   uint32_t q_shb, q_stb, qstep, lstep;
   float inv_g;         // 1 / G: (int)((r + 0.5f) * inv_g) == r / G for the small r of a tile
-  int G, R, Hq, input_pos, dq, dg, wave, lane;
+  int G, R, RT, Hq, input_pos, dq, dg, wave, lane;
   int q0, g0;          // (query, head) of the first row of the next tile to fetch
   uint32_t lds_qw, lds_lse, lds_qpos;
   int next_row0;       // first row of the next tile to fetch
@@ -89,17 +99,17 @@ struct QLoader {
   __device__ __forceinline__ void init(const ScoreParams& p, Smem<D>& sm, int b, int kvh, int tid, int row_start, int steady_first) {
     wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     lane = tid & 63;
-    G = p.G; R = p.R; Hq = p.Hq; input_pos = p.input_pos;
+    G = p.G; R = p.R; RT = p.rows_per_tile; Hq = p.Hq; input_pos = p.input_pos;
     q_shb = (uint32_t)p.q_sh * 2u; q_stb = (uint32_t)p.q_st * 2u;
     qbase = (const char*)(p.q + b * p.q_sb + (int64_t)(kvh * p.G) * p.q_sh);
     lbase = (const char*)(p.lse + (int64_t)b * p.q_len * p.Hq + kvh * p.G);
-    dq = BQ / G; dg = BQ % G;
+    dq = RT / G; dg = RT % G;
     inv_g = 1.0f / (float)G;
     qstep = (uint32_t)dq * q_stb;
     lstep = (uint32_t)(dq * Hq) * 4u;
     q0 = row_start / G;
     g0 = row_start % G;
-    const int qs = q0 + steady_first * dq;        // dg == 0: row_start is a multiple of BQ, hence of G
+    const int qs = q0 + steady_first * dq;        // dg == 0: row_start is a multiple of RT, hence of G
     qtile = qbase + (uint64_t)qs * q_stb;
     ltile = lbase + (uint64_t)(qs * Hq) * 4u;
     qpv = input_pos + qs + lane / G;
@@ -110,9 +120,11 @@ struct QLoader {
     for (int i = 0; i < NI; ++i) {
       rin[i] = (wave + W * i) * RPW + lane / CPR;
       cb[i] = (uint32_t)(((lane % CPR) ^ swz<CPR>(rin[i])) * 16);
-      voff0[i] = (uint32_t)(rin[i] % G) * q_shb + (uint32_t)(rin[i] / G) * q_stb + cb[i];
+      const int rt = min(rin[i], RT - 1);  // the rows a tile leaves empty re-read its last one
+      voff0[i] = (uint32_t)(rt % G) * q_shb + (uint32_t)(rt / G) * q_stb + cb[i];
     }
-    loff0 = (uint32_t)((lane / G) * Hq + lane % G) * 4u;
+    const int lt = min(lane, RT - 1);
+    loff0 = (uint32_t)((lt / G) * Hq + lt % G) * 4u;
     next_row0 = row_start;
   }
 
@@ -132,7 +144,7 @@ struct QLoader {
     qtile += qstep;
     ltile += lstep;
     q0 += dq;
-    next_row0 += BQ;
+    next_row0 += RT;
   }
 
   // start the transfers of the next tile into Q / lse buffer `buf` and position buffer `ring`
@@ -158,12 +170,12 @@ struct QLoader {
       g0 -= G;
       q0 += 1;
     }
-    next_row0 = row0 + BQ;
+    next_row0 = row0 + RT;
   }
 
   // after s_waitcnt vmcnt(0), before the barrier that publishes the tile whose first row is row0
   __device__ __forceinline__ void land(Smem<D>& sm, int row0, int buf) const {
-    if (row0 + BQ > R && wave == 0 && row0 + lane >= R) sm.lse[buf][lane] = INFINITY;  // exp2(... - inf) = 0
+    if (wave == 0 && (lane >= RT || row0 + lane >= R)) sm.lse[buf][lane] = INFINITY;  // exp2(... - inf) = 0
   }
 };
 
@@ -230,21 +242,22 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
 
   float wacc[2] = {0.0f, 0.0f};
   const int tbase = QSPLIT ? (int)blockIdx.z * p.tiles_per_z : 0;  // first query tile of this workgroup
-  const int num_qt = QSPLIT ? min(p.tiles_per_z, (p.R + BQ - 1) / BQ - tbase) : (p.R + BQ - 1) / BQ;
-  // Steps [0, t_steady) are steady: G divides the tile height and tiles t + 1 and t + 2 exist and are full.
-  // Steps [0, t_masked) need the mask: the first query position of tile t, input_pos + (tbase + t) BQ / G, is below
+  const int RT = p.rows_per_tile;
+  const int num_qt = QSPLIT ? min(p.tiles_per_z, (p.R + RT - 1) / RT - tbase) : (p.R + RT - 1) / RT;
+  // Steps [0, t_steady) are steady: tiles are of whole queries and tiles t + 1 and t + 2 exist and are full.
+  // Steps [0, t_masked) need the mask: the first query position of tile t, input_pos + (tbase + t) RT / G, is below
   // the largest key position of this wavefront. Both are even, so the buffer index stays a compile-time constant.
-  const int nfull = min(num_qt, p.R / BQ - tbase);
-  const int t_steady = (BQ % p.G == 0) ? (max(nfull - 2, 0) & ~1) : 0;
+  const int nfull = min(num_qt, p.R / RT - tbase);
+  const int t_steady = (RT % p.G == 0) ? (max(nfull - 2, 0) & ~1) : 0;
   int t_masked;
   {
     const int64_t need = (int64_t)max(min(tpmax, p.input_pos + p.q_len) - p.input_pos, 0) * p.G;  // rows whose position is below tpmax
-    const int64_t tiles = (need + BQ - 1) / BQ - tbase;
+    const int64_t tiles = (need + RT - 1) / RT - tbase;
     t_masked = (int)max((int64_t)0, min(tiles, (int64_t)num_qt));
     t_masked = min((t_masked + 1) & ~1, t_steady);
   }
   QLoader<D, W> ld;
-  ld.init(p, sm, b, kvh, tid, tbase * BQ, 2);
+  ld.init(p, sm, b, kvh, tid, tbase * RT, 2);
   // LDS byte offsets of this lane's Q fragments (A operand): row mt 32 + n, chunk 2 j + h at position chunk ^ swz(row)
   constexpr int CPR = D / 8;
   uint32_t qa[D / 16];
@@ -331,8 +344,8 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
   ld.issue(sm, 0, 0);
   if (num_qt > 1) ld.issue(sm, 1, 1);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the K fragments and the first tiles have arrived
-  ld.land(sm, tbase * BQ, 0);
-  if (num_qt > 1) ld.land(sm, (tbase + 1) * BQ, 1);
+  ld.land(sm, tbase * RT, 0);
+  if (num_qt > 1) ld.land(sm, (tbase + 1) * RT, 1);
   __syncthreads();
   f32x16_t sa[2], sb[2];  // blocks 0 and 1 of the current tile
   u32x4_t qq[D / 16];
@@ -360,8 +373,8 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
     __builtin_amdgcn_sched_barrier(0);
     load_lse(ls, buf_tag, I1);  // into registers before the barrier that hands the buffer to tile t + 2
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's part of tile t + 1 has landed
-    if constexpr (!STEADY) {
-      if (more) ld.land(sm, (tbase + t + 1) * BQ, BUF ^ 1);
+    if (!STEADY || RT < BQ) {
+      if (more) ld.land(sm, (tbase + t + 1) * RT, BUF ^ 1);
     }
     __syncthreads();
     if constexpr (STEADY) {
@@ -578,24 +591,38 @@ __global__ void score_sum_reduce_kernel(const float* part, float* w, int64_t n, 
   w[i] = acc * inv_g;
 }
 
-// Splits of the query rows: none when the keys alone give every compute unit two workgroups of 256 keys; else as
-// many as that takes, each at least 8 tiles of 64 rows (the second launch costs a short chunk more than it
-// gains), at most 16.
+// Wavefronts per workgroup and splits of the query rows with the least estimated time. c workgroups share a compute unit: of
+// four wavefronts two run side by side, of eight (and at head size 256 of four) one; a full count with a nearly empty last round
+// is what the estimate avoids. Measured constants (ns, head size 128): a tile of 64 rows takes a pair of workgroups 2600, one alone
+// 1500, a workgroup of eight wavefronts 2500; its keys cost a workgroup 3000 before the first tile; the launch that adds
+// the splits' sums 4000 and its reads at 4 TB/s. Against splits to two workgroups a unit, each of 8 tiles or more (attention with
+// weights, us): 8 KV heads x 4096 keys, 600 rows 44.3 -> 40.8, x 10000 keys, 4096 rows 261 -> 255; 4 x 6000 keys of 256, 600 / 1500
+// rows 73 -> 62, 123 -> 108.
 struct ScorePlan {
-  int splits, tiles_per_z;
+  int splits, tiles_per_z, waves;
 };
 ScorePlan score_plan(const kvx_sdpa_args& a) {
-  const int G = a.Hq / a.Hkv;
-  const int num_qt = (int)(((int64_t)a.q_len * G + BQ - 1) / BQ);
-  const int64_t wgs = (int64_t)a.B * a.Hkv * ((a.kv_len + 4 * NW - 1) / (4 * NW));
-  int64_t splits = (2 * num_cus() + wgs - 1) / wgs;
-  if (splits > num_qt / 8) splits = num_qt / 8;
-  if (splits > 16) splits = 16;
-  if (splits < 1) splits = 1;
-  ScorePlan pl;
-  pl.tiles_per_z = (num_qt + (int)splits - 1) / (int)splits;
-  pl.splits = (num_qt + pl.tiles_per_z - 1) / pl.tiles_per_z;
-  return pl;
+  const int G = a.Hq / a.Hkv, RT = tile_rows(G);
+  const int num_qt = (int)(((int64_t)a.q_len * G + RT - 1) / RT);
+  const int64_t groups = (int64_t)a.B * a.Hkv, cus = num_cus(), scale = a.D;  // of the tiles' and keys' times: D / 128
+  const int64_t wgs = groups * ((a.kv_len + 4 * NW - 1) / (4 * NW)), wide = groups * ((a.kv_len + 8 * NW - 1) / (8 * NW));
+  ScorePlan best = {1, num_qt, 4};
+  int64_t best_ns = INT64_MAX;
+  auto consider = [&](int splits, int waves) {
+    const int64_t tiles = (num_qt + splits - 1) / splits;
+    splits = (int)((num_qt + tiles - 1) / tiles);
+    const bool pairs = waves == 4 && a.D <= 128;
+    const int64_t c = ((waves == 8 ? wide : wgs * splits) + cus - 1) / cus;
+    const int64_t walk = pairs ? tiles * (2600 * (c / 2) + 1500 * (c % 2)) + 3000 * ((c + 1) / 2) : c * (tiles * (waves == 8 ? 2500 : 1500) + 3000);
+    const int64_t ns = walk * scale / 128 + (splits > 1 ? 4000 + splits * groups * a.kv_len / 1000 : 0);
+    if (ns < best_ns) {
+      best_ns = ns;
+      best = {splits, (int)tiles, waves};
+    }
+  };
+  if (a.D <= 128) consider(1, 8);
+  for (int s = 1; s <= min(16, (num_qt + 1) / 2); ++s) consider(s, 4);
+  return best;
 }
 
 // Few rows over few keys take the short kernel: 64 keys a workgroup then still leave one compute unit a workgroup, and the
@@ -608,7 +635,7 @@ bool is_short(const kvx_sdpa_args& a) {
 }
 
 template <int D, int KV>
-int launch_t(const ScoreParams& p, int splits, const MergeParams* rest, bool brief, hipStream_t st) {
+int launch_t(const ScoreParams& p, int splits, int waves, const MergeParams* rest, bool brief, hipStream_t st) {
   const int groups = p.B * p.Hkv;
   if (brief) {
     const int64_t score_jobs = (int64_t)groups * ((p.kv_len + NW - 1) / NW);
@@ -632,9 +659,8 @@ int launch_t(const ScoreParams& p, int splits, const MergeParams* rest, bool bri
     return KVX_OK;
   }
   if constexpr (D <= 128) {
-    const int wide = (p.kv_len + 8 * NW - 1) / (8 * NW);
-    if ((int64_t)groups * wide >= num_cus()) {
-      hipLaunchKernelGGL((score_sum_kernel<D, KV, 8, false>), dim3(groups, wide), dim3(512), 0, st, p);
+    if (waves == 8) {
+      hipLaunchKernelGGL((score_sum_kernel<D, KV, 8, false>), dim3(groups, (p.kv_len + 8 * NW - 1) / (8 * NW)), dim3(512), 0, st, p);
       KVX_HIP(hipGetLastError());
       return KVX_OK;
     }
@@ -657,7 +683,7 @@ bool score_sum_combines(const kvx_sdpa_args& a) { return is_short(a); }
 int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* rest) {
   // the query rows are split only if the caller's workspace holds the partial sums
   ScorePlan pl = score_plan(a);
-  if (pl.splits > 1 && !(a.workspace && a.workspace_bytes >= score_sum_workspace(a) && ((uintptr_t)a.workspace & 15) == 0)) pl.splits = 1;
+  if (pl.splits > 1 && !(a.workspace && a.workspace_bytes >= score_sum_workspace(a) && ((uintptr_t)a.workspace & 15) == 0)) pl = {1, 0, pl.waves};
   // the query rows are fetched at a uniform base plus a 32-bit byte offset per lane
   {
     const int64_t G = a.Hq / a.Hkv;
@@ -668,6 +694,7 @@ int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* 
   ScoreParams p;
   p.part = pl.splits > 1 ? (float*)a.workspace : nullptr;
   p.tiles_per_z = pl.tiles_per_z;
+  p.rows_per_tile = tile_rows(a.Hq / a.Hkv);
   p.q = (const uint16_t*)a.q;
   p.k = a.k;
   p.k_scale = a.k_scale;
@@ -685,8 +712,8 @@ int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* 
   p.tp_sb = a.tp_stride_b; p.tp_sh = a.tp_stride_h;
 #define KVX_SCORE_SUM_CASE(KV) \
   case KV: \
-    return a.D == 256 ? launch_t<256, KV>(p, pl.splits, rest, is_short(a), st) : a.D == 128 ? launch_t<128, KV>(p, pl.splits, rest, is_short(a), st) \
-                                                                      : launch_t<64, KV>(p, pl.splits, rest, is_short(a), st);
+    return a.D == 256 ? launch_t<256, KV>(p, pl.splits, pl.waves, rest, is_short(a), st) : a.D == 128 ? launch_t<128, KV>(p, pl.splits, pl.waves, rest, is_short(a), st) \
+                                                                      : launch_t<64, KV>(p, pl.splits, pl.waves, rest, is_short(a), st);
   if (a.D == 256 || a.D == 128 || a.D == 64) {
     switch (a.kv_dtype) {
       KVX_SCORE_SUM_CASE(KVX_KV_BF16)

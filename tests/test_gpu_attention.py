@@ -163,6 +163,27 @@ def test_score_sums_of_few_rows_over_few_keys(gpu, store, B, Hq, Hkv, q_len, T, 
         torch.testing.assert_close(lse.cpu(), O.lse2(q, k, scale, pos, tpos), rtol=1e-4, atol=1e-3)
 
 
+@pytest.mark.parametrize("scattered", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D", [
+    (1, 7, 1, 297, 600, 128),    # 2079 rows: 33 tiles of 63, all full
+    (1, 7, 1, 298, 4500, 64),    # one query more
+    (2, 6, 2, 460, 900, 128),    # 21 queries of 3 heads a tile
+    (1, 12, 1, 171, 400, 128),   # tiles of 60 rows
+    (1, 9, 1, 190, 700, 64),     # 63 rows of 9 heads
+    (1, 24, 1, 90, 300, 128),    # 48 of 64 rows would be used: full tiles, the general step
+    (1, 5, 1, 420, 1200, 256),
+])
+def test_score_sums_of_tiles_of_whole_queries(gpu, B, Hq, Hkv, q_len, T, D, scattered):
+    # group sizes that do not divide the 64 rows of a query tile, more than the 1024 rows the short kernel takes
+    q, k, v, gen = make_qkv(610 + T, B, Hq, Hkv, q_len, T, D)
+    pos = 2 * T if scattered else T - q_len
+    tp = scattered_positions(gen, B, Hkv, T, pos, q_len) if scattered else None
+    scale = 1.0 / math.sqrt(D)
+    _, w_ref = O.sdpa_in_blocks(q, k, v, scale, pos, None if tp is None else tp.to(torch.int64))
+    _, w, _ = ops.prefill_core(q.to(gpu), k.to(gpu), v.to(gpu), scale, pos, None if tp is None else tp.to(gpu), return_weights=True)
+    check_w(w, w_ref, q_len)
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D", [(1, 8, 2, 700, 900, 128), (2, 4, 1, 1100, 1100, 64), (1, 16, 2, 300, 2048, 128)])
 def test_score_sum_over_split_query_rows(kvx, gpu, B, Hq, Hkv, q_len, T, D):
     # a short cache: with a workspace the query rows are split over several workgroups and the partial sums
