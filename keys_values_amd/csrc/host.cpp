@@ -302,7 +302,14 @@ AttnOut run_prefill(kvx_sdpa_args& a, const Launch& L, at::ScalarType type, bool
   if (weights) r.w = L.empty({a.B, a.Hkv, a.kv_len}, at::kFloat);
   a.lse = (float*)data(r.lse);
   a.w = (float*)data(r.w);
-  const at::Tensor ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
+  at::Tensor ws;
+  try {
+    ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
+  } catch (const c10::OutOfMemoryError&) {
+    if (a.fused_dequant) throw;
+    a.fused_dequant = 1;  // no room for a copy of a quantised store: the form that needs none
+    ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
+  }
   a.workspace = data(ws);
   a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
   check((weights ? lib.kvx_sdpa_prefill_weights : lib.kvx_sdpa_prefill)(&a, L.stream));
@@ -362,6 +369,7 @@ PyObject* score_sum(PyObject* const* args, Py_ssize_t n) {
   const at::Tensor w = L.empty({a.B, a.Hkv, a.kv_len}, at::kFloat);
   a.lse = (float*)lse.data_ptr();
   a.w = (float*)w.data_ptr();
+  a.fused_dequant = 1;  // the workspace is for partial sums only
   const at::Tensor ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
   a.workspace = data(ws);
   a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;

@@ -711,13 +711,19 @@ int launch_t(PrefillParams& p, hipStream_t st, MergeParams* rest) {
 // Whether a call over a quantised store first dequantises the store into the workspace and then attends over plain rows.
 // Every workgroup of the attention kernel walks the whole store (of its split) and the dequantising one pays its vector work
 // each time, once per 256 rows; the copy pays it once, for one write and one more read of the 16-bit rows. Measured on
-// 65536 x 8 rows of 128, 1024 x 4 queries: 1298 us against 75 + 1048; the lines meet near 2048 rows. At head size 256 the
+// 65536 x 8 rows of 128, 1024 x 4 queries: 1298 us against 75 + 1048. In units of 5 us there (8 x 32768 rows), a block of 256
+// rows of the dequantising kernel takes 8, one of 128 of the plain kernel 3 and the copy 7: it pays from 1025 rows on, and
+// below where 256-row blocks would be half empty. us, codes -> copy: 8 x 32768 8-bit rows of 128, 600 / 1024 / 1400 queries
+// 133 -> 121, 168 -> 165, 261 -> 222; 16 x 6000 of 64, 1400 74 -> 66; 768 queries over the first 136 -> 137: not taken. Below 3 M
+// values the copy's launch is what counts (8 x 1500 of 128, 600 queries 28.2 -> 28.9). At head size 256 the
 // dequantising kernel runs 128 rows a workgroup out of its registers (4 x 4 heads, 541 x 7 queries over 5238: 890 us against
 // 26 + 340), and the copy pays from the second workgroup on.
 static bool wants_copy(const kvx_sdpa_args& a) {
   if (kv_is_plain(a.kv_dtype) || a.fused_dequant || (int64_t)a.B * a.Hkv > 65535) return false;  // pairs are a grid dimension of 16 bits
   const int64_t rows = (int64_t)a.q_len * (a.Hq / a.Hkv);
-  return a.D == 256 ? rows > 128 : rows >= 2048;
+  if (a.D == 256) return rows > 128;
+  if (rows >= 2048) return true;
+  return (int64_t)a.B * a.Hkv * a.kv_len * a.D >= 3000000 && 8 * ((rows + 255) / 256) > 3 * ((rows + 127) / 128) + 7;
 }
 static size_t copy_bytes(const kvx_sdpa_args& a) { return ((size_t)2 * a.B * a.Hkv * a.kv_len * a.D * 2 + 255) / 256 * 256; }
 // the call on the dequantised rows at `rows` (K, then V, each (B, Hkv, kv_len, D))

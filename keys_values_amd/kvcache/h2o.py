@@ -129,6 +129,7 @@ class H2OKVCache:
         # dequantize_chunk_rows: a chunk with at least this many query rows (tokens x heads per KV head) is
         # attended to over a bf16 copy of the quantised store made once for the chunk; None = never. Left at its default it
         # is lower at head size 256, where the dequantising kernel has no registers to spare.
+        self._default_chunk_rows = dequantize_chunk_rows == DEFAULT_DEQUANTIZE_CHUNK_ROWS
         if dequantize_chunk_rows == DEFAULT_DEQUANTIZE_CHUNK_ROWS and params.head_size == 256:
             dequantize_chunk_rows = DEFAULT_DEQUANTIZE_CHUNK_ROWS_256
         self.dequantize_chunk_rows = dequantize_chunk_rows
@@ -543,7 +544,9 @@ class H2OKVCache:
                     return out.view(b, num, hq * d)
                 w = host.score_sum(query, kc, lse, self.scale_factor, input_pos, tp, quant)
             else:
-                out, w, _ = host.prefill(query, kc, vc, self.scale_factor, input_pos, tp, True, False, True, quant, 0, True)
+                # at the default threshold the call itself decides whether a copy pays below it; a threshold (or None) that
+                # the caller chose is kept to
+                out, w, _ = host.prefill(query, kc, vc, self.scale_factor, input_pos, tp, True, False, True, quant, 0, not self._default_chunk_rows)
         self._update(w, num)
         return out.view(b, num, hq * d)
 

@@ -229,6 +229,7 @@ def test_block_sizes_and_slot_ranges_bit_exact(gpu, shape, blocks_over_heads, sp
 @pytest.mark.parametrize("num_bits,dtype,D,q_len,T,token_major", [
     (8, torch.bfloat16, 64, 512, 777, False), (4, torch.float16, 128, 513, 1025, True), (4, torch.bfloat16, 64, 600, 640, True),
     (8, torch.float16, 256, 40, 333, False), (4, torch.bfloat16, 256, 33, 130, True),
+    (8, torch.bfloat16, 128, 257, 5900, True), (4, torch.float16, 64, 130, 11800, False),  # below 2048 rows: 1028 and 520
 ])
 def test_prefill_over_a_copy_of_the_store(gpu, num_bits, dtype, D, q_len, T, token_major):
     """A long chunk over a quantised store attends over rows dequantised once into the workspace: the same bits as the
