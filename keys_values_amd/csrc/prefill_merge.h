@@ -19,7 +19,7 @@ struct MergeParams {
 // with few rows (32 queries over 32768 keys: 1024 rows of 32 splits) a thread's walk over the splits was the time, a memory
 // latency per split and 15 us of a 46 us call: four loads in flight and SC classes make it about two latencies.
 // ROWS: rows of one workgroup of 256 threads.
-constexpr int merge_rows(int D, int SC) { return 256 / (D / 4 * SC); }
+constexpr int merge_rows(int D, int SC) { return 256 / (D / 4 * SC); }  // D: 64, 128 or 256
 // split classes while a walk is longer than four splits and the rows alone leave the device short of threads
 constexpr int merge_classes(int D) { return 256 / (D / 4) < 8 ? 256 / (D / 4) : 8; }
 inline bool merge_wants_classes(const MergeParams& p, int D) {

@@ -423,6 +423,49 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
   }
 }
 
+// The base-2 log-sum-exps and positions of the rows of nblk blocks of 32, in LDS, by a workgroup of 256; rows past the end
+// weigh nothing. With KV splits (m.num_splits) from their (maximum, sum) pairs, else from p.lse. A pass over 16 splits is a memory
+// latency of 1 to 2 us; few rows share a row's splits out over up to eight neighbouring lanes.
+__device__ __forceinline__ void row_weights(const ScoreParams& p, const MergeParams& m, int b, int kvh, int nblk, float* lse_sh, int32_t* qpos_sh) {
+  const float inv_G = 1.0f / (float)p.G;
+  const int S = m.num_splits, group = b * p.Hkv + kvh;
+  const int64_t total_rows = (int64_t)p.B * p.Hkv * p.R;
+  const int lt = nblk <= 1 ? 3 : nblk <= 2 ? 2 : nblk <= 4 ? 1 : 0, T = 1 << lt, part = threadIdx.x & (T - 1);
+  for (int r = threadIdx.x >> lt; r < nblk * 32; r += 256 >> lt) {  // the lanes of a row leave the loop together
+    const int rc = min(r, p.R - 1), qi = (int)(((float)rc + 0.5f) * inv_G);
+    float lse;
+    if (S <= 1) {
+      lse = p.lse[((int64_t)b * p.q_len + qi) * p.Hq + kvh * p.G + (rc - qi * p.G)];
+    } else {
+      const f32x2_t* ml = (const f32x2_t*)m.part_ml + (int64_t)group * p.R + rc;
+      float M = -INFINITY, L = 0.0f;
+      for (int s0 = part; s0 < S; s0 += 16 * T) {
+        f32x2_t x[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) x[u] = ml[(int64_t)min(s0 + u * T, S - 1) * total_rows];
+        float Mn = M;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) Mn = fmaxf(Mn, x[u][0]);
+        const float Mu = Mn == -INFINITY ? 0.0f : Mn;
+        L *= fast_exp2(M - Mu);
+        M = Mn;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) L += s0 + u * T < S ? x[u][1] * fast_exp2(x[u][0] - Mu) : 0.0f;
+      }
+      float Mr = M;
+      for (int off = 1; off < T; off <<= 1) Mr = fmaxf(Mr, __shfl_xor(Mr, off, 64));
+      const float Mu = Mr == -INFINITY ? 0.0f : Mr;
+      L *= fast_exp2(M - Mu);
+      for (int off = 1; off < T; off <<= 1) L += __shfl_xor(L, off, 64);
+      lse = Mu + fast_log2(L);
+    }
+    if (part == 0) {
+      lse_sh[r] = r < p.R ? lse : INFINITY;
+      qpos_sh[r] = p.input_pos + qi;
+    }
+  }
+}
+
 // Short chunks: the same sums with the query rows split over the four wavefronts of a workgroup instead of streamed past
 // each of them. A workgroup owns 64 keys, held by every wavefront as B operands; wavefront w takes the 32-row blocks w,
 // w + 4, ... straight from memory (the next block's rows are fetched while one is worked on, no LDS, no barriers in the
@@ -497,36 +540,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void score_sum_short_kernel(
     }
   }
 
-  // the rows' base-2 log-sum-exps and positions; rows up to the end of the last block weigh nothing
-  const int S = m.num_splits;
-  const int64_t total_rows = (int64_t)groups * p.R;
-  for (int r = tid; r < nblk * 32; r += 256) {
-    const bool ok = r < p.R;
-    const int rc = min(r, p.R - 1), qi = query_of(rc);
-    float lse;
-    if (S <= 1) {
-      lse = p.lse[((int64_t)b * p.q_len + qi) * p.Hq + kvh * p.G + (rc - qi * p.G)];
-    } else {
-      const f32x2_t* ml = (const f32x2_t*)m.part_ml + (int64_t)group * p.R + rc;
-      float M = -INFINITY, L = 0.0f;
-      for (int s0 = 0; s0 < S; s0 += 16) {  // 16 splits a memory latency
-        f32x2_t x[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) x[u] = ml[(int64_t)min(s0 + u, S - 1) * total_rows];
-        float Mn = M;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) Mn = fmaxf(Mn, x[u][0]);
-        const float Mu = Mn == -INFINITY ? 0.0f : Mn;
-        L *= fast_exp2(M - Mu);
-        M = Mn;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) L += s0 + u < S ? x[u][1] * fast_exp2(x[u][0] - Mu) : 0.0f;
-      }
-      lse = (M == -INFINITY ? 0.0f : M) + fast_log2(L);
-    }
-    lse_sh[r] = ok ? lse : INFINITY;
-    qpos_sh[r] = p.input_pos + qi;
-  }
+  row_weights(p, m, b, kvh, nblk, lse_sh, qpos_sh);
   int tpmax = max(tpk[0], tpk[1]);
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) tpmax = max(tpmax, __shfl_xor(tpmax, off, 64));
@@ -582,6 +596,145 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void score_sum_short_kernel(
     p.w[(int64_t)group * p.kv_len + key0 + tid] = (((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid]) * p.inv_g;
 }
 
+// Few rows over many keys: the rows stay in LDS and the keys stream past. The tiled kernel meets a new
+// workgroup of keys with a memory latency for its keys, another for its first tile and two barriers a tile, for two tiles of
+// work (8 x 65536 keys of 128, 32 to 128 rows: 54 us, 2.5 TB/s). Here a wavefront walks blocks of 64 keys, the next block's
+// rows in flight to registers while one is multiplied by all query rows, without barriers; as in the short kernel the partials
+// of the attention's KV splits are combined by the first workgroups of the same launch. Bound by the read of K.
+constexpr int stream_rows(int D) { return D <= 128 ? 256 : 128; }
+
+template <int D, int KV, int SC>
+__global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void score_sum_stream_kernel(const ScoreParams p, const MergeParams m, const int merge_jobs, const int wgs_per_group) {
+  constexpr bool F16 = kv_elem_f16(KV), PLAIN = kv_is_plain(KV), U4 = kv_is_u4(KV);
+  constexpr int KS = D / 16, CPR = D / 8, ROWS = stream_rows(D);
+  if ((int)blockIdx.x < merge_jobs) {
+    merge_job<D, F16, SC>(m, (int)blockIdx.x);
+    return;
+  }
+  __shared__ u32x4_t q_sh[ROWS][CPR];  // chunk c of row r at c ^ swz(r)
+  __shared__ __align__(16) float lse_sh[ROWS];
+  __shared__ __align__(16) int32_t qpos_sh[ROWS];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31;
+  const int h = lane >> 5;
+  const int job = (int)blockIdx.x - merge_jobs, groups = p.B * p.Hkv;
+  const int group = job % groups;  // fastest: a KV head's query rows stay on one XCD
+  const int b = group / p.Hkv, kvh = group % p.Hkv;
+  const float inv_G = 1.0f / (float)p.G;
+  const int nblk = (p.R + 31) / 32, nkb = (p.kv_len + NW - 1) / NW;
+
+  // a block of 64 keys (B operand): lane holds key column n of tile nt, d = 16 j + 8 h .. +8; keys past the end re-read
+  // the last one (nothing of theirs is stored)
+  struct Keys {
+    u32x4_t k[PLAIN ? 2 : 1][PLAIN ? KS : 1];
+    u32x2_t c[PLAIN ? 1 : 2][PLAIN ? 1 : (U4 ? KS / 2 : KS)];
+    int32_t tp[2], zp[2];
+    float sc[2];
+  };
+  const char* kbase = (const char*)p.k + (b * p.k_sb + kvh * p.k_sh) * (PLAIN ? 2 : 1);
+  const int64_t so = b * p.qs_sb + kvh * p.qs_sh;
+  const int32_t* tpb = p.tp ? p.tp + b * p.tp_sb + kvh * p.tp_sh : nullptr;
+  auto load_k = [&](Keys& x, int kb) {
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      const int key = min(kb * NW + nt * 32 + n, p.kv_len - 1);
+      const char* kp = kbase + (int64_t)key * p.k_st * (PLAIN ? 2 : 1);
+      x.tp[nt] = tpb ? tpb[key] : key;
+      if constexpr (PLAIN) {
+#pragma unroll
+        for (int j = 0; j < KS; ++j) x.k[nt][j] = *(const u32x4_t*)(kp + 32 * j + 16 * h);
+      } else {
+        x.sc[nt] = p.k_scale[so + key];
+        x.zp[nt] = p.k_zp[so + key];
+#pragma unroll
+        for (int j = 0; j < (U4 ? KS / 2 : KS); ++j) x.c[nt][j] = *(const u32x2_t*)(kp + (U4 ? u4_byte_off<D>(2 * j + h) : (uint32_t)(16 * j + 8 * h)));
+      }
+    }
+  };
+  const int stride = 4 * wgs_per_group;
+  int kb = job / groups * 4 + wave;
+  Keys ka, kc;
+  if (kb < nkb) load_k(ka, kb);
+
+  for (int i = tid; i < nblk * 32 * CPR; i += 256) {
+    const int r = i / CPR, c = i % CPR, rc = min(r, p.R - 1), qi = (int)(((float)rc + 0.5f) * inv_G);
+    q_sh[r][c ^ swz<CPR>(r)] = *(const u32x4_t*)(p.q + b * p.q_sb + (int64_t)(kvh * p.G + rc - qi * p.G) * p.q_sh + (int64_t)qi * p.q_st + 8 * c);
+  }
+  row_weights(p, m, b, kvh, nblk, lse_sh, qpos_sh);
+  __syncthreads();
+
+  auto weigh = [&](const u32x4_t (&kf)[2][KS], const int32_t (&tpk)[2], int kb) {
+    float wacc[2] = {0.0f, 0.0f};
+    const int tpm = max(tpk[0], tpk[1]);
+    for (int blk = 0; blk < nblk; ++blk) {
+      f32x16_t s[2];
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[nt][i] = 0.0f;
+#pragma unroll
+      for (int j = 0; j < KS; ++j) {
+        const u32x4_t qq = q_sh[blk * 32 + n][(2 * j + h) ^ swz<CPR>(n)];
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) s[nt] = mfma_32x32x16<F16>(qq, kf[nt][j], s[nt]);
+      }
+      const bool masked = __any(tpm > p.input_pos + (int)(((float)(blk * 32) + 0.5f) * inv_G));
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const f32x4_t ls = *(const f32x4_t*)&lse_sh[blk * 32 + 8 * a + 4 * h];
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) {
+          float e[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) e[i] = fast_exp2(fmaf(s[nt][4 * a + i], p.c, -ls[i]));
+          if (masked) {
+            const int4 qp = *(const int4*)&qpos_sh[blk * 32 + 8 * a + 4 * h];
+            e[0] = tpk[nt] > qp.x ? 0.0f : e[0];
+            e[1] = tpk[nt] > qp.y ? 0.0f : e[1];
+            e[2] = tpk[nt] > qp.z ? 0.0f : e[2];
+            e[3] = tpk[nt] > qp.w ? 0.0f : e[3];
+          }
+          wacc[nt] += (e[0] + e[1]) + (e[2] + e[3]);
+        }
+      }
+    }
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      const float t = sum_halves(wacc[nt]);
+      const int key = kb * NW + nt * 32 + n;
+      if (h == 0 && key < p.kv_len) p.w[(int64_t)group * p.kv_len + key] = t * p.inv_g;
+    }
+  };
+  if constexpr (PLAIN) {
+    for (; kb < nkb; kb += 2 * stride) {
+      const bool more = kb + stride < nkb;
+      if (more) load_k(kc, kb + stride);
+      weigh(ka.k, ka.tp, kb);
+      if (more) {
+        if (kb + 2 * stride < nkb) load_k(ka, kb + 2 * stride);
+        weigh(kc.k, kc.tp, kb + stride);
+      }
+    }
+  } else {
+    for (; kb < nkb; kb += stride) {
+      u32x4_t kf[2][KS];
+      const int32_t tpk[2] = {ka.tp[0], ka.tp[1]};
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+        for (int j = 0; j < KS; ++j) {
+          u32x2_t cc = ka.c[nt][U4 ? j % (KS / 2) : j];
+          if constexpr (U4) cc = u4_codes(cc, u4_shift<D>(2 * j + h));
+          kf[nt][j] = dequant_words<F16>(cc[0], cc[1], ka.zp[nt], ka.sc[nt]);
+        }
+      if (kb + stride < nkb) load_k(ka, kb + stride);
+      weigh(kf, tpk, kb);
+    }
+  }
+}
+
 // W = (1/G) * (part[0] + part[1] + ...), in that order.
 __global__ void score_sum_reduce_kernel(const float* part, float* w, int64_t n, int splits, float inv_g) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -625,6 +778,8 @@ ScorePlan score_plan(const kvx_sdpa_args& a) {
   return best;
 }
 
+enum { TILED, SHORT, STREAMED };
+
 // Few rows over few keys take the short kernel: 64 keys a workgroup then still leave one compute unit a workgroup, and the
 // wavefronts that walk the query rows side by side would idle otherwise. Attention with weights, us, long -> short kernel:
 // 2 KV heads x 1024 keys of 64, 128 / 512 / 1024 / 2000 rows 16.0 -> 12.3, 23.7 -> 17.3, 26.5 -> 24.2, 30.9 -> 37.9; 8 x 1024 of 128,
@@ -634,16 +789,48 @@ bool is_short(const kvx_sdpa_args& a) {
   return (int64_t)a.q_len * (a.Hq / a.Hkv) <= SHORT_ROWS && (int64_t)a.B * a.Hkv * ((a.kv_len + NW - 1) / NW) <= num_cus();
 }
 
+// The combination runs at the score jobs' occupancy, two workgroups a compute unit in the streaming kernel: more jobs than
+// compute units are quicker in a launch of their own (8 x 4096 keys of 128, 32 / 128 rows: 20.6 -> 16.3 and 27 -> 34 us combined).
+bool merge_fits(const kvx_sdpa_args& a) {
+  const int per_job = merge_rows(a.D, merge_classes(a.D));
+  return ((int64_t)a.B * a.Hq * a.q_len + per_job - 1) / per_job <= num_cus();
+}
+// Where the streaming kernel is the faster one: one block of rows, up to four of rows of 64 values whose splits it can combine,
+// and any number it holds over 256 K keys or more; over fewer a wavefront has no second block of keys to fetch ahead.
+// Attention with weights, us, tiled -> streamed: 8 x 4096 keys of 128, 32 / 64 / 128 rows 20.6 -> 16.3, 23.2 -> 24.2, 27 -> 30;
+// 8 x 65536, 32 / 128 / 256 rows 99 -> 87, 126 -> 112, 150 -> 143; of 64, 4 x 9001, 128 rows 27 -> 22, 8 x 16384, 64 / 128 rows
+// 27 -> 24, 28 -> 29; 16 x 20000 of 256, 32 / 128 rows 190 -> 163, 216 -> 196.
+bool is_streamed(const kvx_sdpa_args& a) {
+  const int64_t rows = (int64_t)a.q_len * (a.Hq / a.Hkv);
+  if (is_short(a) || rows > stream_rows(a.D)) return false;
+  return rows <= 32 || (a.D == 64 && rows <= 128 && merge_fits(a)) || (int64_t)a.B * a.Hkv * a.kv_len >= 256 * 1024;
+}
+
 template <int D, int KV>
-int launch_t(const ScoreParams& p, int splits, int waves, const MergeParams* rest, bool brief, hipStream_t st) {
+int launch_t(const ScoreParams& p, int splits, int waves, const MergeParams* rest, int kind, hipStream_t st) {
   const int groups = p.B * p.Hkv;
-  if (brief) {
+  if (kind == SHORT) {
     const int64_t score_jobs = (int64_t)groups * ((p.kv_len + NW - 1) / NW);
     const MergeParams m = rest ? *rest : MergeParams{};
     auto launch = [&](auto sc_tag) {
       constexpr int SC = decltype(sc_tag)::value, ROWS = merge_rows(D, SC);
       const int64_t merge_jobs = m.num_splits > 1 ? ((int64_t)groups * p.R + ROWS - 1) / ROWS : 0;
       hipLaunchKernelGGL((score_sum_short_kernel<D, KV, SC>), dim3((unsigned)(score_jobs + merge_jobs)), dim3(256), 0, st, p, m, (int)score_jobs);
+    };
+    if (merge_wants_classes(m, D)) launch(std::integral_constant<int, merge_classes(D)>{});
+    else launch(std::integral_constant<int, 1>{});
+    KVX_HIP(hipGetLastError());
+    return KVX_OK;
+  }
+  if (kind == STREAMED) {
+    const MergeParams m = rest ? *rest : MergeParams{};
+    const int nkb = (p.kv_len + NW - 1) / NW, most = (nkb + 3) / 4;
+    const int per_group = max(1, min(most, (D <= 128 ? 2 : 1) * num_cus() / groups));
+    auto launch = [&](auto sc_tag) {
+      constexpr int SC = decltype(sc_tag)::value, ROWS = merge_rows(D, SC);
+      const int64_t merge_jobs = m.num_splits > 1 ? ((int64_t)groups * p.R + ROWS - 1) / ROWS : 0;
+      hipLaunchKernelGGL((score_sum_stream_kernel<D, KV, SC>), dim3((unsigned)(merge_jobs + (int64_t)groups * per_group)), dim3(256), 0, st, p, m, (int)merge_jobs,
+                         per_group);
     };
     if (merge_wants_classes(m, D)) launch(std::integral_constant<int, merge_classes(D)>{});
     else launch(std::integral_constant<int, 1>{});
@@ -672,13 +859,13 @@ int launch_t(const ScoreParams& p, int splits, int waves, const MergeParams* res
 
 }  // namespace
 
+bool score_sum_combines(const kvx_sdpa_args& a) { return is_short(a) || (is_streamed(a) && merge_fits(a)); }
+
 size_t score_sum_workspace(const kvx_sdpa_args& a) {
-  if (is_short(a)) return 0;
+  if (is_short(a) || is_streamed(a)) return 0;
   const ScorePlan pl = score_plan(a);
   return pl.splits > 1 ? (size_t)pl.splits * a.B * a.Hkv * a.kv_len * sizeof(float) : 0;
 }
-
-bool score_sum_combines(const kvx_sdpa_args& a) { return is_short(a); }
 
 int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* rest) {
   // the query rows are split only if the caller's workspace holds the partial sums
@@ -710,10 +897,11 @@ int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* 
   p.k_sb = a.k_stride_b; p.k_sh = a.k_stride_h; p.k_st = a.k_stride_t;
   p.qs_sb = a.qs_stride_b; p.qs_sh = a.qs_stride_h;
   p.tp_sb = a.tp_stride_b; p.tp_sh = a.tp_stride_h;
+  const int kind = is_short(a) ? SHORT : is_streamed(a) ? STREAMED : TILED;
 #define KVX_SCORE_SUM_CASE(KV) \
   case KV: \
-    return a.D == 256 ? launch_t<256, KV>(p, pl.splits, pl.waves, rest, is_short(a), st) : a.D == 128 ? launch_t<128, KV>(p, pl.splits, pl.waves, rest, is_short(a), st) \
-                                                                      : launch_t<64, KV>(p, pl.splits, pl.waves, rest, is_short(a), st);
+    return a.D == 256 ? launch_t<256, KV>(p, pl.splits, pl.waves, rest, kind, st) : a.D == 128 ? launch_t<128, KV>(p, pl.splits, pl.waves, rest, kind, st) \
+                                                                      : launch_t<64, KV>(p, pl.splits, pl.waves, rest, kind, st);
   if (a.D == 256 || a.D == 128 || a.D == 64) {
     switch (a.kv_dtype) {
       KVX_SCORE_SUM_CASE(KVX_KV_BF16)

@@ -163,6 +163,19 @@ def test_score_sums_of_few_rows_over_few_keys(gpu, store, B, Hq, Hkv, q_len, T, 
         torch.testing.assert_close(lse.cpu(), O.lse2(q, k, scale, pos, tpos), rtol=1e-4, atol=1e-3)
 
 
+@pytest.mark.parametrize("store", ["bf16", "u8", "u4"])
+@pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D,splits", [
+    (2, 8, 8, 2, 1100, 128, 2),       # 2 rows, 17.2 blocks of keys
+    (2, 24, 8, 10, 1090, 256, 5),     # 30 rows of 3 heads
+    (1, 32, 8, 8, 2112, 128, 17),     # a full block of rows; the partials in two passes
+    (5, 4, 4, 32, 5000, 64, 0),       # several blocks of keys a wavefront
+    (4, 28, 4, 18, 1030, 64, 3),      # 126 rows
+])
+def test_score_sums_with_streamed_keys(gpu, store, B, Hq, Hkv, q_len, T, D, splits):
+    # few rows over more keys than the short kernel takes, alone and with the combination of the KV splits
+    test_score_sums_of_few_rows_over_few_keys(gpu, store, B, Hq, Hkv, q_len, T, D, splits)
+
+
 @pytest.mark.parametrize("scattered", [False, True])
 @pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D", [
     (1, 7, 1, 297, 600, 128),    # 2079 rows: 33 tiles of 63, all full
