@@ -11,6 +11,8 @@
 // double-buffered, shared by the four or eight wavefronts of the workgroup (256 or 512 keys per workgroup).
 // S = Q K^T is computed with rows along M, so a lane owns one key column: the sum over queries is a
 // per-lane running sum and the two halves of the wavefront are added once at the end.
+// Two further kernels take short chunks: score_sum_short_kernel (few rows, few keys) and score_sum_stream_kernel (few
+// rows, many keys); both can also combine the partial outputs that the attention kernel's KV splits left.
 #include <type_traits>
 
 #include "prefill_merge.h"

@@ -20,10 +20,11 @@
 // W = (1/G) sum_g exp2(logit_g - lse_g) on the spot; in the fused H2O form it also adds W to the cumulative
 // scores and feeds the row's lowest-score slot. Longer splits, and a workgroup whose wait ran out, send the
 // logits to an fp32 scratch in bursts of 32 KB (a write stream mixed into the reads costs HBM far more than
-// its share of the bytes). One more launch follows the split kernel: some of its workgroups combine the splits'
-// outputs, the others do the weights work of the splits that took the scratch route, and the one that finishes
-// last publishes the chosen slots. K and V are touched once: they are loaded non-temporally. No float atomics
-// anywhere.
+// its share of the bytes). The splits of a row also combine its outputs, each an equal share, and the one that
+// finishes last publishes the chosen slot (finish_split). Only where the logits go through the scratch by plan one more
+// launch follows: some of its workgroups combine the splits' outputs, the others do the weights work, and the one that
+// finishes last publishes the chosen slots. K and V are touched once: they are loaded non-temporally. No float
+// atomics anywhere.
 // Quantised stores, and plain rows with 8 to 16 query heads per KV head, take a second form of the split kernel
 // (decode_mfma_kernel, below) that does both products on the matrix cores: with codes to dequantise, or with that
 // many dot products per loaded value, the form above is bound by its vector arithmetic, not by HBM.
