@@ -144,11 +144,16 @@ __device__ __forceinline__ uint32_t ordered_bits(float x) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-// Base-2 log-sum-exp of a query head from its splits' (maximum, sum) pairs, by one wavefront: lane s takes
+// Maximum and sum (relative to it) of a query head from its splits' (maximum, sum) pairs, by one wavefront: lane s takes
 // splits s, s + 64, ..., then butterflies; every lane returns the same bits. COHERENT: the pairs were
-// written by other workgroups of the running kernel (device-coherent loads).
+// written by other workgroups of the running kernel (device-coherent loads). The outputs are scaled by these two:
+// the log-sum-exp, one number, is rounded at the size of the logits (at 10^6 by 2^-5, 2 % of a weight).
+struct RowSum {
+  float top, sum;
+  __device__ __forceinline__ float lse() const { return top + fast_log2(sum); }  // base 2
+};
 template <bool COHERENT>
-__device__ __forceinline__ float row_lse(const float* part_ml, int num_splits, int lane) {
+__device__ __forceinline__ RowSum row_sum(const float* part_ml, int num_splits, int lane) {
   const unsigned long long* ml = (const unsigned long long*)part_ml;
   float M = -INFINITY, L = 0.0f;
   for (int base = 0; base < num_splits; base += 64) {
@@ -166,7 +171,7 @@ __device__ __forceinline__ float row_lse(const float* part_ml, int num_splits, i
   L = M > -INFINITY ? L * fast_exp2(M - Mw) : 0.0f;
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) L += __shfl_xor(L, off, 64);
-  return Mw + fast_log2(L);
+  return {Mw, L};
 }
 
 // The logits gathered in LDS leave as one contiguous burst (keys past the end of a chunk of CHUNK keys are -inf).
@@ -190,6 +195,7 @@ __device__ __forceinline__ unsigned long long pair_bits(float lo, float hi) {
 template <int G>
 struct FinishShared {
   float lse[G];
+  float top[G], inv[G];  // maximum of the head's logits, 1 / sum relative to it
   float z;  // scores weighted by the V norms: the row's sum of |V row| W
   float vn[G];
   float red[WAVES][4];
@@ -197,15 +203,18 @@ struct FinishShared {
   uint32_t ready, finished;
 };
 
-// The row's log-sum-exps (and z) from its splits' partials, in LDS for the whole workgroup. All splits have published.
+// The row's maxima, sums and log-sum-exps (and z) from its splits' partials, in LDS for the whole workgroup. All splits have
+// published.
 template <int G>
 __device__ __forceinline__ void row_state(const DecodeParams& p, const bool vnorm, const int b, const int kvh, FinishShared<G>& sh) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int g = wave; g < G; g += WAVES) {  // a wavefront per head: lane s takes splits s, s + 64, ...
     float lse = INFINITY, z = 0.0f;        // dummy heads: exp2(x - inf) = 0
+    RowSum rs = {0.0f, 1.0f};
     if (g < p.Gr) {
       const int64_t hd = (int64_t)b * p.Hq + kvh * p.Gr + g;
-      lse = row_lse<true>(p.part_ml + hd * p.num_splits * 2, p.num_splits, lane);
+      rs = row_sum<true>(p.part_ml + hd * p.num_splits * 2, p.num_splits, lane);
+      lse = rs.lse();
       if (vnorm) {
         for (int sp = lane; sp < p.num_splits; sp += 64)
           z += coherent_load(p.part_vn + hd * p.num_splits + sp) * fast_exp2(coherent_load(p.part_ml + (hd * p.num_splits + sp) * 2) - lse);
@@ -215,6 +224,8 @@ __device__ __forceinline__ void row_state(const DecodeParams& p, const bool vnor
     }
     if (lane == 0) {
       sh.lse[g] = lse;
+      sh.top[g] = rs.top;
+      sh.inv[g] = 1.0f / rs.sum;
       sh.vn[g] = z;
     }
   }
@@ -227,11 +238,11 @@ __device__ __forceinline__ void row_state(const DecodeParams& p, const bool vnor
   if (vnorm) __syncthreads();
 }
 
-// The row's outputs for the value pairs [e0, e1) of its Gr * D / 2: O = sum over the splits of part_o 2^(m - lse).
+// The row's outputs for the value pairs [e0, e1) of its Gr * D / 2: O = (sum over the splits of part_o 2^(m - top)) / sum.
 // J threads share a pair, thread class j taking splits j, j + J, ...; their sums are added in that order, so the
 // result does not depend on which workgroup takes which pairs. J grows with the number of splits (a thread then has at
 // most four loads to make up to 64 splits: one memory latency a pass of 256 / J pairs). The loads of the first pass go out
-// before the row's log-sum-exps are worked out (STATE), which wait for memory themselves. `buf`: 256 pairs of floats of LDS.
+// before the row's maxima and sums are worked out (STATE), which wait for memory themselves. `buf`: 256 pairs of floats of LDS.
 template <int D, bool F16, int G, bool STATE>
 __device__ __forceinline__ void merge_pairs(const DecodeParams& p, const bool vnorm, const int b, const int kvh, FinishShared<G>& sh, const int e0, const int e1,
                                             f32x2_t* buf) {
@@ -262,12 +273,12 @@ __device__ __forceinline__ void merge_pairs(const DecodeParams& p, const bool vn
     first = false;
     f32x2_t acc = {0.0f, 0.0f};
     if (live) {
-      const float lse = sh.lse[g];
+      const float top = sh.top[g];
       for (int s0 = j; s0 < S; s0 += 4 * J) {
         if (s0 != j) load(s0);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const float w = s0 + J * u < S ? fast_exp2(m[u] - lse) : 0.0f;
+          const float w = s0 + J * u < S ? fast_exp2(m[u] - top) : 0.0f;
           acc[0] += __uint_as_float((uint32_t)x[u]) * w;
           acc[1] += __uint_as_float((uint32_t)(x[u] >> 32)) * w;
         }
@@ -279,8 +290,10 @@ __device__ __forceinline__ void merge_pairs(const DecodeParams& p, const bool vn
       __syncthreads();
       for (int i = 1; i < J; ++i) acc += buf[i * P + c];  // meaningful in class 0
     }
-    if (j == 0 && live)
-      *(uint32_t*)(p.o + b * p.o_sb + (int64_t)(kvh * p.Gr + g) * p.o_sh + 2 * (e % (D / 2))) = pack_pair<F16>(acc[0], acc[1]);
+    if (j == 0 && live) {
+      const float inv = sh.inv[g];
+      *(uint32_t*)(p.o + b * p.o_sb + (int64_t)(kvh * p.Gr + g) * p.o_sh + 2 * (e % (D / 2))) = pack_pair<F16>(acc[0] * inv, acc[1] * inv);
+    }
   }
 }
 
@@ -1071,7 +1084,7 @@ __device__ __forceinline__ void merge_job(const DecodeParams& p, const int bh) {
     for (int off = 32; off >= 1; off >>= 1) mloc = fmaxf(mloc, __shfl_xor(mloc, off, 64));
     if (threadIdx.x == 0) sM = mloc;
     // the log-sum-exp by the routine the split kernel uses for its own weights: the same bits on either route
-    const float lse = row_lse<false>(ml, p.num_splits, threadIdx.x);
+    const float lse = row_sum<false>(ml, p.num_splits, threadIdx.x).lse();
     if (threadIdx.x == 0 && p.lse_out) p.lse_out[bh] = lse;
   }
   __syncthreads();
@@ -1115,7 +1128,7 @@ __device__ __forceinline__ void weights_job(const DecodeParams& p, const kvx_h2o
     // the row's log-sum-exps from the splits' partials, by the routine the split kernel and the merge use
     for (int g = wave; g < G; g += NT / 64) {
       float l = INFINITY;  // dummy heads: exp2(x - inf) = 0
-      if (g < p.Gr) l = row_lse<false>(p.part_ml + ((int64_t)b * p.Hq + kvh * p.Gr + g) * p.num_splits * 2, p.num_splits, lane);
+      if (g < p.Gr) l = row_sum<false>(p.part_ml + ((int64_t)b * p.Hq + kvh * p.Gr + g) * p.num_splits * 2, p.num_splits, lane).lse();
       if (lane == 0) lse_sh[g] = l;
     }
     __syncthreads();

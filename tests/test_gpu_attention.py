@@ -9,6 +9,7 @@ from helpers import make_qkv, rel_err, scattered_positions
 from keys_values_amd import _lib
 from keys_values_amd.attention import ops
 from keys_values_amd.attention.sdpa import HipSDPA
+from keys_values_amd.kvcache.quantize import RowQuantizer
 from oracle import kvx_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -575,3 +576,35 @@ def test_decode_with_weights_beside_other_work(gpu):
     o_ref, w_ref = O.sdpa_in_blocks(q, k, v, scale, T - 1, None)
     check_o(out0.unsqueeze(2), o_ref)
     check_w(w0, w_ref, 1)
+
+
+@pytest.mark.parametrize("T", [777, 5000, 9001])
+@pytest.mark.parametrize("D,G,store", [(128, 4, "plain"), (64, 1, "plain"), (128, 8, "plain"), (128, 4, "u8"), (256, 2, "u4")])
+def test_decode_output_at_large_logits(gpu, decode_route, D, G, store, T):
+    """Every key the same row, the logits around 10^6: all weights are equal and the output is the mean of the V rows,
+    whatever the logits round to. Outputs are float16 (each within 2^-11 of its value) and sums run in float32, so 1e-3
+    covers both; a normaliser taken from a log-sum-exp in float32 is off by up to 2^-5 here."""
+    Hkv = 2
+    gen = torch.Generator(device=gpu).manual_seed(T + D + G)
+
+    def uniform(*shape):
+        return (200 + 100 * torch.rand(*shape, generator=gen, device=gpu)).to(torch.float16)
+
+    q = uniform(1, Hkv * G, 1, D)
+    k = uniform(1, Hkv, 1, D).expand(1, Hkv, T, D).contiguous()
+    v = (torch.randn(1, Hkv, T, D, generator=gen, device=gpu) + 1).to(torch.float16)
+    quant, kd, vd = None, k, v
+    if store != "plain":
+        codes, state, rows = [], [], []
+        for x in (k, v):
+            qz = RowQuantizer((1, Hkv, T, D), torch.float16, 8 if store == "u8" else 4, allocate_buffers=True, device=gpu)
+            qz.quantize(0, T, x)
+            codes.append(qz.quant_buffer.view(1, Hkv, T, -1))
+            state += [qz.quant_scales.view(1, Hkv, T), qz.quant_zero_points.view(1, Hkv, T)]
+            rows.append(qz.dequantize(0, T))
+        (kd, vd), (k, v), quant = codes, rows, ops.QuantState(*state)
+    want = v.double().mean(2).repeat_interleave(G, 1)
+    for weights in (True, False):
+        out, _, lse = ops.decode_core(q, kd, vd, D ** -0.5, return_weights=weights, return_lse=True, quant=quant)
+        assert lse.min() > 2.0 ** 17
+        assert rel_err(out, want) < 1e-3, (weights, rel_err(out, want))
