@@ -35,7 +35,8 @@
 extern "C" {
 #endif
 
-#define KVX_VERSION 103 /* major*10000 + minor*100 + patch */
+#define KVX_VERSION 104 /* major*10000 + minor*100 + patch */
+/* 104: kvx_sdpa_prefill_copying, kvx_h2o_decode_step. The argument blocks are those of 103. */
 
 enum kvx_status {
   KVX_OK = 0,
@@ -64,7 +65,8 @@ enum kvx_kv_dtype {
                         keys_values/kvcache/quantize/pytorch.py:333,478), and q and o are float16 */
 };
 
-/* One attention call. Unused pointers are NULL. All strides in elements. */
+/* One attention call. Unused pointers are NULL. All strides in elements. The prefill and score-sum calls read nothing
+ * behind workspace_bytes. */
 typedef struct kvx_sdpa_args {
   int32_t B, Hq, Hkv, q_len, kv_len, D;
   int32_t input_pos;   /* position of the first query; >= 0 */
@@ -101,12 +103,6 @@ typedef struct kvx_sdpa_args {
    * instead of staying on the chip -- all of them when the splits are too long for the LDS or that form is switched
    * off, else those whose bounded wait for their row ran out (normally 0; such a call is about 15 % slower). */
   uint32_t* decode_scratch_splits;
-
-  /* kvx_sdpa_prefill* over a quantised store: 1 = dequantise inside the attention kernel whatever the size of the chunk;
-   * 0 = where it is faster, dequantise the store once into the workspace (kvx_sdpa_prefill_workspace_bytes then counts
-   * 2 * B * Hkv * kv_len * D 16-bit values) and attend over the copy. Same results. A workspace too small for the copy
-   * but not for the rest means the same as 1. */
-  int32_t fused_dequant;
 } kvx_sdpa_args;
 
 /* ---- library ------------------------------------------------------------------------------- */
@@ -153,6 +149,15 @@ int kvx_score_sum(const kvx_sdpa_args* args, void* stream);
  * (keys_values/attention/flashinfer_wrapper.py:476-494). args->lse must be given (it carries the
  * log-sum-exp between the two kernels); workspace as for kvx_sdpa_prefill. */
 int kvx_sdpa_prefill_weights(const kvx_sdpa_args* args, void* stream);
+
+/* kvx_sdpa_prefill (args->w NULL) or kvx_sdpa_prefill_weights, for callers with memory to spare. Every workgroup of the
+ * attention kernel dequantises the whole of a quantised store (or of its split) for itself; here the store is
+ * dequantised once into the workspace instead, and attention reads the copy, wherever that is faster (long chunks). The
+ * results agree to the order of sums. kvx_sdpa_prefill_copying_workspace_bytes then counts
+ * 2 * B * Hkv * kv_len * D 16-bit values for the copy. With a workspace too small for the copy but not for the other call,
+ * over a plain store and where no copy pays, this is the other call. */
+int kvx_sdpa_prefill_copying(const kvx_sdpa_args* args, void* stream);
+size_t kvx_sdpa_prefill_copying_workspace_bytes(const kvx_sdpa_args* args);
 
 /* Single-token decode (q_len == 1): O over the whole cache and, if args->w is set, the score-sums
  * W = (1/G) sum_g softmax_g. No mask: the new token is the newest

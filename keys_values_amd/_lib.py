@@ -40,7 +40,6 @@ class SdpaArgs(ctypes.Structure):
         ("lse", c_void_p), ("w", c_void_p),
         ("workspace", c_void_p), ("workspace_bytes", c_size_t),
         ("decode_scratch_splits", c_void_p),
-        ("fused_dequant", c_int32),
     ]
 
 
@@ -101,6 +100,8 @@ SYMBOLS = {
     "kvx_device_info": (ctypes.c_int, [ctypes.c_int, ctypes.c_char_p, c_size_t]),
     "kvx_sdpa_prefill": (ctypes.c_int, [POINTER(SdpaArgs), c_void_p]),
     "kvx_sdpa_prefill_workspace_bytes": (c_size_t, [POINTER(SdpaArgs)]),
+    "kvx_sdpa_prefill_copying": (ctypes.c_int, [POINTER(SdpaArgs), c_void_p]),
+    "kvx_sdpa_prefill_copying_workspace_bytes": (c_size_t, [POINTER(SdpaArgs)]),
     "kvx_score_sum": (ctypes.c_int, [POINTER(SdpaArgs), c_void_p]),
     "kvx_sdpa_prefill_weights": (ctypes.c_int, [POINTER(SdpaArgs), c_void_p]),
     "kvx_sdpa_decode": (ctypes.c_int, [POINTER(SdpaArgs), c_void_p]),

@@ -31,6 +31,7 @@ namespace {
 
 #define KVX_HOST_SYMBOLS(X)                                                                                                 \
   X(kvx_last_error) X(kvx_sdpa_prefill) X(kvx_sdpa_prefill_workspace_bytes) X(kvx_score_sum) X(kvx_sdpa_prefill_weights)     \
+  X(kvx_sdpa_prefill_copying) X(kvx_sdpa_prefill_copying_workspace_bytes)                                                    \
   X(kvx_sdpa_decode) X(kvx_sdpa_decode_workspace_bytes) X(kvx_h2o_decode_step) X(kvx_h2o_decode_step_workspace_bytes)        \
   X(kvx_quantize_blocks) X(kvx_dequantize_blocks) X(kvx_dequantize_rows_typed) X(kvx_cache_write) \
   X(kvx_h2o_update_select) X(kvx_h2o_workspace_bytes) X(kvx_rmsnorm_rows) X(kvx_add_rmsnorm_rows) X(kvx_swiglu_rows)         \
@@ -288,8 +289,8 @@ struct AttnOut {
   at::Tensor out, w, lse;
 };
 
-// prefill attention on checked operands
-AttnOut run_prefill(kvx_sdpa_args& a, const Launch& L, at::ScalarType type, bool weights, bool want_lse, bool transposed) {
+// prefill attention on checked operands; `copy`: a quantised store may be dequantised into the scratch where that is faster
+AttnOut run_prefill(kvx_sdpa_args& a, const Launch& L, at::ScalarType type, bool weights, bool want_lse, bool transposed, bool copy) {
   AttnOut r;
   if (transposed) {
     r.out = L.empty({a.B, a.q_len, a.Hq, a.D}, type);
@@ -304,15 +305,15 @@ AttnOut run_prefill(kvx_sdpa_args& a, const Launch& L, at::ScalarType type, bool
   a.w = (float*)data(r.w);
   at::Tensor ws;
   try {
-    ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
+    ws = L.scratch((copy ? lib.kvx_sdpa_prefill_copying_workspace_bytes : lib.kvx_sdpa_prefill_workspace_bytes)(&a));
   } catch (const c10::OutOfMemoryError&) {
-    if (a.fused_dequant) throw;
-    a.fused_dequant = 1;  // no room for a copy of a quantised store: the form that needs none
+    if (!copy) throw;
+    copy = false;  // no room for a copy of a quantised store: the form that needs none
     ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
   }
   a.workspace = data(ws);
   a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
-  check((weights ? lib.kvx_sdpa_prefill_weights : lib.kvx_sdpa_prefill)(&a, L.stream));
+  check((copy ? lib.kvx_sdpa_prefill_copying : weights ? lib.kvx_sdpa_prefill_weights : lib.kvx_sdpa_prefill)(&a, L.stream));
   return r;
 }
 
@@ -337,9 +338,8 @@ PyObject* prefill(PyObject* const* args, Py_ssize_t n) {
   kvx_sdpa_args a = sdpa_args(q, k, &v, real(args[3]), integer(args[4]), qs ? &*qs : nullptr, integer(args[10]));
   at::Tensor keep;
   set_positions(a, opt_tensor(args[5], "token_positions"), keep);
-  a.fused_dequant = truth(args[11]);
   const bool want_lse = truth(args[7]);
-  AttnOut r = run_prefill(a, L, q.scalar_type(), truth(args[6]), want_lse, truth(args[8]));
+  AttnOut r = run_prefill(a, L, q.scalar_type(), truth(args[6]), want_lse, truth(args[8]), qs && !truth(args[11]));
   return three(r.out, r.w, want_lse ? r.lse : at::Tensor());
 }
 
@@ -369,7 +369,6 @@ PyObject* score_sum(PyObject* const* args, Py_ssize_t n) {
   const at::Tensor w = L.empty({a.B, a.Hkv, a.kv_len}, at::kFloat);
   a.lse = (float*)lse.data_ptr();
   a.w = (float*)w.data_ptr();
-  a.fused_dequant = 1;  // the workspace is for partial sums only
   const at::Tensor ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
   a.workspace = data(ws);
   a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;

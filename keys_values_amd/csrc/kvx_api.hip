@@ -120,16 +120,28 @@ int kvx_device_info(int device, char* buf, size_t buf_len) {
 
 size_t kvx_sdpa_prefill_workspace_bytes(const kvx_sdpa_args* a) {
   if (check_sdpa_common(a, "kvx_sdpa_prefill_workspace_bytes", false) != KVX_OK) return 0;
-  return sdpa_prefill_workspace(*a);
+  return sdpa_prefill_workspace(*a, false);
 }
 
-int kvx_sdpa_prefill(const kvx_sdpa_args* a, void* stream) {
-  int rc = check_sdpa_common(a, "kvx_sdpa_prefill", true);
-  if (rc != KVX_OK) return rc;
-  KVX_REQUIRE(a->q_len <= a->kv_len, KVX_ERR_INVALID, "kvx_sdpa_prefill: q_len=%d exceeds kv_len=%d", a->q_len, a->kv_len);
-  KVX_REQUIRE(aligned16(a->workspace), KVX_ERR_WORKSPACE, "kvx_sdpa_prefill: workspace must be 16-byte aligned");
-  return launch_sdpa_prefill(*a, (hipStream_t)stream);
+size_t kvx_sdpa_prefill_copying_workspace_bytes(const kvx_sdpa_args* a) {
+  if (check_sdpa_common(a, "kvx_sdpa_prefill_copying_workspace_bytes", false) != KVX_OK) return 0;
+  return sdpa_prefill_workspace(*a, true);
 }
+
+static int prefill_checked(const kvx_sdpa_args* a, const char* who, bool weights, bool may_copy, hipStream_t st) {
+  int rc = check_sdpa_common(a, who, true);
+  if (rc != KVX_OK) return rc;
+  KVX_REQUIRE(a->q_len <= a->kv_len, KVX_ERR_INVALID, "%s: q_len=%d exceeds kv_len=%d", who, a->q_len, a->kv_len);
+  KVX_REQUIRE(!weights || (a->lse && a->w), KVX_ERR_INVALID, "%s: lse and w must be given", who);
+  KVX_REQUIRE(aligned16(a->workspace), KVX_ERR_WORKSPACE, "%s: workspace must be 16-byte aligned", who);
+  MergeParams rest{};
+  const bool combines = weights && score_sum_combines(*a);
+  rc = launch_sdpa_prefill(*a, may_copy, st, combines ? &rest : nullptr);
+  if (rc != KVX_OK || !weights) return rc;
+  return launch_score_sum(*a, st, combines ? &rest : nullptr);
+}
+
+int kvx_sdpa_prefill(const kvx_sdpa_args* a, void* stream) { return prefill_checked(a, "kvx_sdpa_prefill", false, false, (hipStream_t)stream); }
 
 int kvx_score_sum(const kvx_sdpa_args* a, void* stream) {
   int rc = check_sdpa_common(a, "kvx_score_sum", false);
@@ -139,17 +151,11 @@ int kvx_score_sum(const kvx_sdpa_args* a, void* stream) {
 }
 
 int kvx_sdpa_prefill_weights(const kvx_sdpa_args* a, void* stream) {
-  int rc = check_sdpa_common(a, "kvx_sdpa_prefill_weights", true);
-  if (rc != KVX_OK) return rc;
-  KVX_REQUIRE(a->q_len <= a->kv_len, KVX_ERR_INVALID, "kvx_sdpa_prefill_weights: q_len=%d exceeds kv_len=%d", a->q_len,
-              a->kv_len);
-  KVX_REQUIRE(a->lse && a->w, KVX_ERR_INVALID, "kvx_sdpa_prefill_weights: lse and w must be given");
-  KVX_REQUIRE(aligned16(a->workspace), KVX_ERR_WORKSPACE, "kvx_sdpa_prefill_weights: workspace must be 16-byte aligned");
-  MergeParams rest{};
-  const bool combines = score_sum_combines(*a);
-  rc = launch_sdpa_prefill(*a, (hipStream_t)stream, combines ? &rest : nullptr);
-  if (rc != KVX_OK) return rc;
-  return launch_score_sum(*a, (hipStream_t)stream, combines ? &rest : nullptr);
+  return prefill_checked(a, "kvx_sdpa_prefill_weights", true, false, (hipStream_t)stream);
+}
+
+int kvx_sdpa_prefill_copying(const kvx_sdpa_args* a, void* stream) {
+  return prefill_checked(a, "kvx_sdpa_prefill_copying", a && a->w, true, (hipStream_t)stream);
 }
 
 size_t kvx_sdpa_decode_workspace_bytes(const kvx_sdpa_args* a) {

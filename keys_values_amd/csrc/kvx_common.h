@@ -46,11 +46,12 @@ int hip_error(hipError_t e, const char* what);
 
 // ---- launchers implemented one per translation unit ---------------------------------------
 struct MergeParams;  // prefill_merge.h
+// may_copy: a quantised store may be dequantised into the workspace first; no field behind workspace_bytes is read.
 // `rest` not NULL: the KV splits' partials are left in the workspace, described in *rest, for launch_score_sum to combine
-int launch_sdpa_prefill(const kvx_sdpa_args& a, hipStream_t st, MergeParams* rest = nullptr);
+int launch_sdpa_prefill(const kvx_sdpa_args& a, bool may_copy, hipStream_t st, MergeParams* rest = nullptr);
 // whether launch_score_sum takes the kernel that can combine the attention's partials in the same launch
 bool score_sum_combines(const kvx_sdpa_args& a);
-size_t sdpa_prefill_workspace(const kvx_sdpa_args& a);
+size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy);
 int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* rest = nullptr);
 size_t score_sum_workspace(const kvx_sdpa_args& a);
 int launch_sdpa_decode(const kvx_sdpa_args& a, const kvx_h2o_args* fused_h2o, hipStream_t st);

@@ -19,6 +19,9 @@
 //   K/V tiles travel global -> LDS by DMA (global_load_lds_dwordx4, no registers), double-buffered,
 //   rows unpadded and XOR-swizzled against bank conflicts. The loop is software-pipelined: the
 //   matrix cores add V(t-1) P(t-1) to O while the vector ALU turns S(t) into P(t).
+#include <stddef.h>
+#include <string.h>
+
 #include <type_traits>
 #include <utility>
 
@@ -719,16 +722,22 @@ int launch_t(PrefillParams& p, hipStream_t st, MergeParams* rest) {
 // dequantising kernel runs 128 rows a workgroup out of its registers (4 x 4 heads, 541 x 7 queries over 5238: 890 us against
 // 26 + 340), and the copy pays from the second workgroup on.
 static bool wants_copy(const kvx_sdpa_args& a) {
-  if (kv_is_plain(a.kv_dtype) || a.fused_dequant || (int64_t)a.B * a.Hkv > 65535) return false;  // pairs are a grid dimension of 16 bits
+  if (kv_is_plain(a.kv_dtype) || (int64_t)a.B * a.Hkv > 65535) return false;  // pairs are a grid dimension of 16 bits
   const int64_t rows = (int64_t)a.q_len * (a.Hq / a.Hkv);
   if (a.D == 256) return rows > 128;
   if (rows >= 2048) return true;
   return (int64_t)a.B * a.Hkv * a.kv_len * a.D >= 3000000 && 8 * ((rows + 255) / 256) > 3 * ((rows + 127) / 128) + 7;
 }
 static size_t copy_bytes(const kvx_sdpa_args& a) { return ((size_t)2 * a.B * a.Hkv * a.kv_len * a.D * 2 + 255) / 256 * 256; }
+// the block up to workspace_bytes: callers of the prefill calls may not have the rest
+static kvx_sdpa_args prefill_block(const kvx_sdpa_args& a) {
+  kvx_sdpa_args c{};
+  memcpy(&c, &a, offsetof(kvx_sdpa_args, workspace_bytes) + sizeof(a.workspace_bytes));
+  return c;
+}
 // the call on the dequantised rows at `rows` (K, then V, each (B, Hkv, kv_len, D))
 static kvx_sdpa_args on_copy(const kvx_sdpa_args& a, void* rows) {
-  kvx_sdpa_args c = a;
+  kvx_sdpa_args c = prefill_block(a);
   c.kv_dtype = kv_elem_f16(a.kv_dtype) ? KVX_KV_F16 : KVX_KV_BF16;
   c.k = rows;
   c.v = (char*)rows + (size_t)a.B * a.Hkv * a.kv_len * a.D * 2;
@@ -738,20 +747,19 @@ static kvx_sdpa_args on_copy(const kvx_sdpa_args& a, void* rows) {
   return c;
 }
 
-size_t sdpa_prefill_workspace(const kvx_sdpa_args& a) {
+size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy) {
   PrefillParams p;
-  const bool copy = wants_copy(a);
-  const kvx_sdpa_args c = copy ? on_copy(a, nullptr) : a;
-  fill_params(p, c);
+  const bool copy = may_copy && wants_copy(a);
+  fill_params(p, copy ? on_copy(a, nullptr) : prefill_block(a));
   // the score-sum pass that may follow on the same stream reuses the workspace for its partial sums
   const size_t own = partial_bytes(p, a.D) + (copy ? copy_bytes(a) : 0), after = score_sum_workspace(a);
   return own > after ? own : after;
 }
 
-int launch_sdpa_prefill(const kvx_sdpa_args& a_in, hipStream_t st, MergeParams* rest) {
+int launch_sdpa_prefill(const kvx_sdpa_args& a_in, bool may_copy, hipStream_t st, MergeParams* rest) {
   PrefillParams p;
-  kvx_sdpa_args a = a_in;
-  if (wants_copy(a)) {
+  kvx_sdpa_args a = prefill_block(a_in);
+  if (may_copy && wants_copy(a)) {
     // a workspace too small for the copy (sized for another call, or by a caller that has no room): the fused form
     const kvx_sdpa_args c = on_copy(a, a.workspace);
     fill_params(p, c);

@@ -30,7 +30,7 @@ def test_library_exports_every_declared_symbol(kvx):
     assert sorted(_lib.SYMBOLS) == names, "ctypes table and header disagree"
     for n in names:
         assert hasattr(kvx, n), f"libkvx.so does not export {n}"
-    assert kvx.kvx_version() == 103
+    assert kvx.kvx_version() == 104
 
 
 def test_struct_layouts_match_c(tmp_path):
@@ -50,6 +50,49 @@ def test_struct_layouts_match_c(tmp_path):
         assert int(got[cname]) == ctypes.sizeof(cls)
         for fname, _ in cls._fields_:
             assert int(got[f"{cname}.{fname}"]) == getattr(cls, fname).offset, f"{cname}.{fname}"
+
+
+_OLD_CALLER = r"""
+import ctypes, mmap, sys
+from keys_values_amd import _lib
+kvx = _lib.load()
+libc = ctypes.CDLL(None, use_errno=True)
+libc.mmap.restype, libc.mmap.argtypes = ctypes.c_void_p, [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long]
+libc.mprotect.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+page = mmap.PAGESIZE
+base = libc.mmap(None, 2 * page, mmap.PROT_READ | mmap.PROT_WRITE, mmap.MAP_PRIVATE | mmap.MAP_ANONYMOUS, -1, 0)
+assert libc.mprotect(base + page, page, 0) == 0
+size = _lib.SdpaArgs.workspace_bytes.offset + 8  # the block as callers of the attention calls have written it from the start
+a = ctypes.cast(base + page - size, ctypes.POINTER(_lib.SdpaArgs))
+calls = (kvx.kvx_sdpa_prefill, kvx.kvx_sdpa_prefill_weights)
+for kv_dtype in (0, 1, 2, 3, 4, 5):
+    for D in (64, 128, 256):
+        b = _lib.SdpaArgs()
+        b.B, b.Hq, b.Hkv, b.q_len, b.kv_len, b.D, b.input_pos, b.kv_dtype, b.sm_scale, b.num_splits = 1, 32, 8, 1024, 65536, D, 64512, kv_dtype, 0.1, 4
+        for name, ctype in b._fields_:
+            if ctype is ctypes.c_void_p and name != "workspace":
+                setattr(b, name, 0x10000)
+        b.q_stride_t = b.k_stride_t = b.v_stride_t = b.o_stride_t = D
+        ctypes.memmove(a, ctypes.byref(b), size)
+        partials = 4 * 32 * 1024 * (D + 2) * 4  # of the four splits
+        assert kvx.kvx_sdpa_prefill_workspace_bytes(a) == partials, (kv_dtype, D)
+        for call in calls:  # no workspace: refused before anything is launched
+            assert call(a, None) == _lib.KVX_ERR_WORKSPACE, kvx.kvx_last_error()
+        b.lse = None
+        ctypes.memmove(a, ctypes.byref(b), size)
+        assert kvx.kvx_score_sum(a, None) == _lib.KVX_ERR_INVALID
+print("read nothing behind the block")
+"""
+
+
+def test_prefill_reads_no_further_than_the_block_of_its_first_callers(kvx):
+    """kvx_sdpa_args has grown behind workspace_bytes. The prefill and score-sum calls read nothing there, and ask for no
+    more workspace than their partial results need: callers that end the block at workspace_bytes (here: at the end of
+    their memory) get what they always got."""
+    import sys
+
+    r = subprocess.run([sys.executable, "-c", _OLD_CALLER], cwd=ROOT, capture_output=True, text=True)
+    assert r.returncode == 0 and "read nothing" in r.stdout, (r.returncode, r.stderr[-2000:])
 
 
 def test_validation_answers_without_a_gpu(kvx):
@@ -144,10 +187,10 @@ def test_random_arguments_are_answered_not_trusted(kvx):
         # half of the blocks are random throughout, half are valid ones with up to two fields replaced
         a = fill(_lib.SdpaArgs()) if it % 2 else mutate(valid_sdpa(), rnd.choice([0, 1, 1, 2]))
         h = fill(_lib.H2OArgs())
-        for fn in (kvx.kvx_sdpa_prefill, kvx.kvx_score_sum, kvx.kvx_sdpa_decode):
+        for fn in (kvx.kvx_sdpa_prefill, kvx.kvx_sdpa_prefill_copying, kvx.kvx_score_sum, kvx.kvx_sdpa_decode):
             assert fn(ctypes.byref(a), None) in codes
         assert kvx.kvx_sdpa_decode_h2o(ctypes.byref(a), ctypes.byref(h), None) in codes
-        for fn in (kvx.kvx_sdpa_prefill_workspace_bytes, kvx.kvx_sdpa_decode_workspace_bytes, kvx.kvx_sdpa_decode_h2o_workspace_bytes):
+        for fn in (kvx.kvx_sdpa_prefill_workspace_bytes, kvx.kvx_sdpa_prefill_copying_workspace_bytes, kvx.kvx_sdpa_decode_workspace_bytes, kvx.kvx_sdpa_decode_h2o_workspace_bytes):
             assert fn(ctypes.byref(a)) >= 0
         assert kvx.kvx_h2o_update_select(ctypes.byref(h), None) in codes
         assert kvx.kvx_h2o_workspace_bytes(ctypes.byref(h)) >= 0
