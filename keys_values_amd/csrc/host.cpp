@@ -10,7 +10,8 @@
 // Error behaviour is that of the Python functions this serves: ValueError for shapes, NotImplementedError for
 // unsupported sizes and types, RuntimeError for tensors that are not on the device. Scratch comes from PyTorch's caching
 // allocator per call, on the caller's stream, and goes back to it when the call returns: nothing outlives a call, and
-// calls from several threads or streams share nothing.
+// calls from several threads or streams share nothing. Python objects are read with the interpreter lock held; allocation
+// and launch run without it (`unlocked`).
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -20,6 +21,7 @@
 #include <dlfcn.h>
 
 #include <algorithm>
+#include <array>
 #include <optional>
 #include <string>
 
@@ -60,6 +62,19 @@ void check(int rc) {
   if (rc == KVX_ERR_INVALID) raise(PyExc_ValueError, "%s", lib.kvx_last_error());
   if (rc == KVX_ERR_UNSUPPORTED) raise(PyExc_NotImplementedError, "%s", lib.kvx_last_error());
   raise(kvx_error, "kvx status %d: %s", rc, lib.kvx_last_error());
+}
+
+// f() without the interpreter lock: the allocator may have to free blocks and wait for the device, a launch for room in a
+// hardware queue, and what they wait for may need Python (a host function in a stream). f touches no Python object and raises
+// no Python error (its status goes to check() afterwards; C++ exceptions pass); tensors it uses are arguments of the call,
+// which the caller holds, or held by the call itself.
+template <typename F>
+auto unlocked(F&& f) {
+  struct Release {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Release() { PyEval_RestoreThread(state); }
+  } release;
+  return f();
 }
 
 std::string shape_str(const at::Tensor& t) {
@@ -120,13 +135,19 @@ struct Ref {  // an owned reference
 };
 Ref attr(PyObject* o, PyObject* name) { return Ref(PyObject_GetAttr(o, name)); }
 int64_t attr_int(PyObject* o, PyObject* name) { return integer(attr(o, name).p); }
-// the object keeps the tensor alive for the call (the GIL is held throughout)
 at::Tensor attr_tensor(PyObject* o, PyObject* name) { return tensor(attr(o, name).p, PyUnicode_AsUTF8(name)); }
 std::optional<at::Tensor> attr_opt_tensor(PyObject* o, PyObject* name) {
   Ref r = attr(o, name);
   if (r.p == Py_None) return std::nullopt;
   return tensor(r.p, PyUnicode_AsUTF8(name));
 }
+
+// The cache's tensors that a call's argument block points into: another thread may give the object new ones meanwhile.
+struct Held {
+  std::array<at::Tensor, 16> tensors;  // eleven at most
+  size_t n = 0;
+  const at::Tensor& operator()(at::Tensor t) { return tensors.at(n++) = std::move(t); }
+};
 
 // Device and stream of a call: the tensors' device is made current if it is not.
 struct Launch {
@@ -242,8 +263,11 @@ void set_positions(kvx_sdpa_args& a, const at::Tensor* tp, at::Tensor& keep) {
   if (!tp) return;
   if (tp->dim() != 3 || tp->size(0) != a.B || tp->size(1) != a.Hkv || tp->size(2) != a.kv_len)
     raise(PyExc_ValueError, "token_positions.shape = %s, must be (%d, %d, %d)", shape_str(*tp).c_str(), a.B, a.Hkv, a.kv_len);
-  keep = tp->scalar_type() == at::kInt ? *tp : tp->to(at::kInt);
-  if (keep.stride(2) != 1) keep = keep.contiguous();
+  if (tp->scalar_type() == at::kInt && tp->stride(2) == 1) keep = *tp;
+  else keep = unlocked([&] {
+    at::Tensor t = tp->to(at::kInt);
+    return t.stride(2) == 1 ? t : t.contiguous();
+  });
   a.token_positions = (const int32_t*)keep.data_ptr();
   a.tp_stride_b = keep.stride(0);
   a.tp_stride_h = keep.stride(1);
@@ -292,28 +316,30 @@ struct AttnOut {
 // prefill attention on checked operands; `copy`: a quantised store may be dequantised into the scratch where that is faster
 AttnOut run_prefill(kvx_sdpa_args& a, const Launch& L, at::ScalarType type, bool weights, bool want_lse, bool transposed, bool copy) {
   AttnOut r;
-  if (transposed) {
-    r.out = L.empty({a.B, a.q_len, a.Hq, a.D}, type);
-    set_o(a, r.out, r.out.stride(0), r.out.stride(2), r.out.stride(1));
-  } else {
-    r.out = L.empty({a.B, a.Hq, a.q_len, a.D}, type);
-    set_o(a, r.out, r.out.stride(0), r.out.stride(1), r.out.stride(2));
-  }
-  if (weights || want_lse) r.lse = L.empty({a.B, a.q_len, a.Hq}, at::kFloat);
-  if (weights) r.w = L.empty({a.B, a.Hkv, a.kv_len}, at::kFloat);
-  a.lse = (float*)data(r.lse);
-  a.w = (float*)data(r.w);
-  at::Tensor ws;
-  try {
-    ws = L.scratch((copy ? lib.kvx_sdpa_prefill_copying_workspace_bytes : lib.kvx_sdpa_prefill_workspace_bytes)(&a));
-  } catch (const c10::OutOfMemoryError&) {
-    if (!copy) throw;
-    copy = false;  // no room for a copy of a quantised store: the form that needs none
-    ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
-  }
-  a.workspace = data(ws);
-  a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
-  check((copy ? lib.kvx_sdpa_prefill_copying : weights ? lib.kvx_sdpa_prefill_weights : lib.kvx_sdpa_prefill)(&a, L.stream));
+  check(unlocked([&] {
+    if (transposed) {
+      r.out = L.empty({a.B, a.q_len, a.Hq, a.D}, type);
+      set_o(a, r.out, r.out.stride(0), r.out.stride(2), r.out.stride(1));
+    } else {
+      r.out = L.empty({a.B, a.Hq, a.q_len, a.D}, type);
+      set_o(a, r.out, r.out.stride(0), r.out.stride(1), r.out.stride(2));
+    }
+    if (weights || want_lse) r.lse = L.empty({a.B, a.q_len, a.Hq}, at::kFloat);
+    if (weights) r.w = L.empty({a.B, a.Hkv, a.kv_len}, at::kFloat);
+    a.lse = (float*)data(r.lse);
+    a.w = (float*)data(r.w);
+    at::Tensor ws;
+    try {
+      ws = L.scratch((copy ? lib.kvx_sdpa_prefill_copying_workspace_bytes : lib.kvx_sdpa_prefill_workspace_bytes)(&a));
+    } catch (const c10::OutOfMemoryError&) {
+      if (!copy) throw;
+      copy = false;  // no room for a copy of a quantised store: the form that needs none
+      ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
+    }
+    a.workspace = data(ws);
+    a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
+    return (copy ? lib.kvx_sdpa_prefill_copying : weights ? lib.kvx_sdpa_prefill_weights : lib.kvx_sdpa_prefill)(&a, L.stream);
+  }));
   return r;
 }
 
@@ -366,25 +392,17 @@ PyObject* score_sum(PyObject* const* args, Py_ssize_t n) {
   kvx_sdpa_args a = sdpa_args(q, k, nullptr, real(args[3]), integer(args[4]), qs ? &*qs : nullptr, 0);
   at::Tensor keep;
   set_positions(a, opt_tensor(args[5], "token_positions"), keep);
-  const at::Tensor w = L.empty({a.B, a.Hkv, a.kv_len}, at::kFloat);
   a.lse = (float*)lse.data_ptr();
-  a.w = (float*)w.data_ptr();
-  const at::Tensor ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
-  a.workspace = data(ws);
-  a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
-  check(lib.kvx_score_sum(&a, L.stream));
+  at::Tensor w;
+  check(unlocked([&] {
+    w = L.empty({a.B, a.Hkv, a.kv_len}, at::kFloat);
+    a.w = (float*)w.data_ptr();
+    const at::Tensor ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
+    a.workspace = data(ws);
+    a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
+    return lib.kvx_score_sum(&a, L.stream);
+  }));
   return wrap(w);
-}
-
-// single-token attention on checked operands; out (B, Hq, D), or (B, 1, Hq * D) for the cache
-void run_decode(kvx_sdpa_args& a, const Launch& L, const at::Tensor& out, const at::Tensor& w, const at::Tensor& lse) {
-  set_o(a, out, (int64_t)a.Hq * a.D, a.D, a.D);
-  a.w = (float*)data(w);
-  a.lse = (float*)data(lse);
-  const at::Tensor ws = L.scratch(lib.kvx_sdpa_decode_workspace_bytes(&a));
-  a.workspace = data(ws);
-  a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
-  check(lib.kvx_sdpa_decode(&a, L.stream));
 }
 
 // decode(query, key, value, scale, return_weights, return_lse, quant, num_splits, scratch_splits) -> (out, weights, lse)
@@ -410,11 +428,21 @@ PyObject* decode(PyObject* const* args, Py_ssize_t n) {
       raise(PyExc_ValueError, "scratch_splits must be a one-element int32 tensor on the query's device");
     a.decode_scratch_splits = (uint32_t*)s->data_ptr();
   }
-  const at::Tensor out = L.empty({a.B, a.Hq, a.D}, q.scalar_type());
-  const at::Tensor w = truth(args[4]) ? L.empty({a.B, a.Hkv, a.kv_len}, at::kFloat) : at::Tensor();
-  const at::Tensor lse = truth(args[5]) ? L.empty({a.B, 1, a.Hq}, at::kFloat) : at::Tensor();
-  run_decode(a, L, out, w, lse);
-  return three(out, w, lse);
+  const bool want_w = truth(args[4]), want_lse = truth(args[5]);
+  AttnOut r;
+  check(unlocked([&] {
+    r.out = L.empty({a.B, a.Hq, a.D}, q.scalar_type());
+    if (want_w) r.w = L.empty({a.B, a.Hkv, a.kv_len}, at::kFloat);
+    if (want_lse) r.lse = L.empty({a.B, 1, a.Hq}, at::kFloat);
+    set_o(a, r.out, (int64_t)a.Hq * a.D, a.D, a.D);
+    a.w = (float*)data(r.w);
+    a.lse = (float*)data(r.lse);
+    const at::Tensor ws = L.scratch(lib.kvx_sdpa_decode_workspace_bytes(&a));
+    a.workspace = data(ws);
+    a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
+    return lib.kvx_sdpa_decode(&a, L.stream);
+  }));
+  return three(r.out, r.w, r.lse);
 }
 
 // ---- the cache object --------------------------------------------------------------------------------------------------
@@ -431,8 +459,8 @@ PyObject* check_qkv(PyObject* const* args, Py_ssize_t n) {
   return Py_BuildValue("LL", (long long)b, (long long)num);
 }
 
-void set_cache_tensors(kvx_cache_write_args& a, PyObject* cache) {
-  const at::Tensor k = attr_tensor(cache, names.k), v = attr_tensor(cache, names.v);
+void set_cache_tensors(kvx_cache_write_args& a, PyObject* cache, Held& held) {
+  const at::Tensor &k = held(attr_tensor(cache, names.k)), &v = held(attr_tensor(cache, names.v));
   a.k_cache = k.data_ptr();
   a.kc_stride_b = k.stride(0);
   a.kc_stride_h = k.stride(1);
@@ -444,41 +472,45 @@ void set_cache_tensors(kvx_cache_write_args& a, PyObject* cache) {
   a.kv_dtype = (int32_t)attr_int(cache, names._store_dtype);
   const bool codes = truth(attr(cache, names._store_quantized).p);
   if (codes) {
-    const at::Tensor ks = attr_tensor(cache, names.k_scale), kz = attr_tensor(cache, names.k_zp);
+    const at::Tensor& ks = held(attr_tensor(cache, names.k_scale));
     a.k_scale = (float*)ks.data_ptr();
-    a.k_zp = (int32_t*)kz.data_ptr();
-    a.v_scale = (float*)attr_tensor(cache, names.v_scale).data_ptr();
-    a.v_zp = (int32_t*)attr_tensor(cache, names.v_zp).data_ptr();
+    a.k_zp = (int32_t*)held(attr_tensor(cache, names.k_zp)).data_ptr();
+    a.v_scale = (float*)held(attr_tensor(cache, names.v_scale)).data_ptr();
+    a.v_zp = (int32_t*)held(attr_tensor(cache, names.v_zp)).data_ptr();
     a.qs_stride_b = ks.stride(0);
     a.qs_stride_h = ks.stride(1);
   }
-  const at::Tensor tp = attr_tensor(cache, names.token_pos), sc = attr_tensor(cache, names.scores);
+  const at::Tensor &tp = held(attr_tensor(cache, names.token_pos)), &sc = held(attr_tensor(cache, names.scores));
   a.token_pos = (int32_t*)tp.data_ptr();
   a.tp_stride_b = tp.stride(0);
   a.tp_stride_h = tp.stride(1);
   a.scores = (float*)sc.data_ptr();
   a.sc_stride_b = sc.stride(0);
   a.sc_stride_h = sc.stride(1);
-  if (auto t = attr_opt_tensor(cache, names.v_norm)) a.v_norm = (float*)t->data_ptr();
+  if (auto t = attr_opt_tensor(cache, names.v_norm)) a.v_norm = (float*)held(*t).data_ptr();
   // a working buffer whose codes live elsewhere (blocks over the heads): the row-quantising write has no errors to give
   if (codes)
-    if (auto t = attr_opt_tensor(cache, names.q_errors)) a.q_errors = (float*)t->data_ptr();
+    if (auto t = attr_opt_tensor(cache, names.q_errors)) a.q_errors = (float*)held(*t).data_ptr();
 }
 
 at::Tensor rows_of(const at::Tensor& t, at::ScalarType type) {
-  at::Tensor r = t.scalar_type() == type ? t : t.to(type);
-  return r.stride(3) == 1 ? r : r.contiguous();
+  if (t.scalar_type() == type && t.stride(3) == 1) return t;
+  return unlocked([&] {
+    at::Tensor r = t.to(type);
+    return r.stride(3) == 1 ? r : r.contiguous();
+  });
 }
 
 struct WriteCall {
   kvx_cache_write_args a{};
   at::Tensor key, value;  // as handed to the kernel
+  Held held;
 };
 // key / value (B, Hkv, num, D) into the slots `index` (int32, strides for batch and head; NULL: the slots chosen last)
 WriteCall write_args(PyObject* cache, const at::Tensor* index, const at::Tensor& key, const at::Tensor& value, int64_t input_pos, PyObject* ring, PyObject* log) {
   WriteCall w;
   kvx_cache_write_args& a = w.a;
-  set_cache_tensors(a, cache);
+  set_cache_tensors(a, cache, w.held);
   const at::ScalarType type =
       (a.kv_dtype == KVX_KV_F16 || a.kv_dtype == KVX_KV_U8_F16 || a.kv_dtype == KVX_KV_U4_F16) ? at::kHalf : at::kBFloat16;
   w.key = rows_of(key, type);
@@ -495,7 +527,7 @@ WriteCall write_args(PyObject* cache, const at::Tensor* index, const at::Tensor&
     a.index_stride_h = index->stride(1);
   } else {
     const int64_t c = attr_int(cache, names._next_count);
-    a.index = (const int32_t*)attr_tensor(cache, names._next_flat).data_ptr();
+    a.index = (const int32_t*)w.held(attr_tensor(cache, names._next_flat)).data_ptr();
     a.index_stride_b = a.Hkv * c;
     a.index_stride_h = c;
   }
@@ -532,13 +564,13 @@ PyObject* cache_write(PyObject* const* args, Py_ssize_t n) {
   const at::Tensor &key = tensor(args[2], "key"), &value = tensor(args[3], "value");
   const Launch L(key);
   const WriteCall w = write_args(args[0], opt_tensor(args[1], "index"), key, value, integer(args[4]), args[5], args[6]);
-  check(lib.kvx_cache_write(&w.a, L.stream));
+  check(unlocked([&] { return lib.kvx_cache_write(&w.a, L.stream); }));
   Py_RETURN_NONE;
 }
 
 // Arguments of the score update and the choice of k slots; `full`: the cache has no free slot (else nothing is chosen
 // that anyone uses, and the smallest selection is run)
-kvx_h2o_args h2o_args(PyObject* cache, bool full, int64_t k, int64_t input_pos) {
+kvx_h2o_args h2o_args(PyObject* cache, bool full, int64_t k, int64_t input_pos, Held& held) {
   kvx_h2o_args a{};
   a.B = (int32_t)attr_int(cache, names.batch_size);
   a.Hkv = (int32_t)attr_int(cache, names.n_query_groups);
@@ -548,16 +580,16 @@ kvx_h2o_args h2o_args(PyObject* cache, bool full, int64_t k, int64_t input_pos) 
   a.normalize = full && truth(attr(cache, names.normalize_scores).p);
   a.input_pos = (int32_t)input_pos;
   a.prefill_len = (int32_t)attr_int(cache, names.prefill_length);
-  const at::Tensor sc = attr_tensor(cache, names.scores), tp = attr_tensor(cache, names.token_pos);
+  const at::Tensor &sc = held(attr_tensor(cache, names.scores)), &tp = held(attr_tensor(cache, names.token_pos));
   a.scores = (float*)sc.data_ptr();
   a.sc_stride_b = sc.stride(0);
   a.sc_stride_h = sc.stride(1);
   a.token_pos = (const int32_t*)tp.data_ptr();
   a.tp_stride_b = tp.stride(0);
   a.tp_stride_h = tp.stride(1);
-  if (auto t = attr_opt_tensor(cache, names.v_norm)) a.v_norm = (const float*)t->data_ptr();
+  if (auto t = attr_opt_tensor(cache, names.v_norm)) a.v_norm = (const float*)held(*t).data_ptr();
   if (full)  // only the selection reads the errors
-    if (auto t = attr_opt_tensor(cache, names.q_errors)) a.q_errors = (const float*)t->data_ptr();
+    if (auto t = attr_opt_tensor(cache, names.q_errors)) a.q_errors = (const float*)held(*t).data_ptr();
   a.combination = real(attr(cache, names.combination_constant).p);
   return a;
 }
@@ -566,14 +598,13 @@ kvx_h2o_args h2o_args(PyObject* cache, bool full, int64_t k, int64_t input_pos) 
 // better form, which is what a workspace without room for sorted lists selects: spread over the device the choice is
 // over sooner but holds up the matrix products beside it (two layers of the long-context stack, 4096 slots: 5.60 ms
 // against 5.88).
-void run_update(kvx_h2o_args& a, const Launch& L, const at::Tensor& next, bool background) {
-  a.next_index = (int32_t*)next.data_ptr();
+int run_update(kvx_h2o_args& a, const Launch& L, bool background) {
   size_t bytes = lib.kvx_h2o_workspace_bytes(&a);
   if (background) bytes = std::min(bytes, (size_t)a.B * a.Hkv * (8 + 16) + 32);  // a bound and four statistics per row
   const at::Tensor ws = L.scratch(bytes);
   a.workspace = data(ws);
   a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
-  check(lib.kvx_h2o_update_select(&a, L.stream));
+  return lib.kvx_h2o_update_select(&a, L.stream);
 }
 
 // cache_update(cache, weights or None, query_length, k, full, background): scores += weights, then the next k slots into
@@ -582,14 +613,21 @@ PyObject* cache_update(PyObject* const* args, Py_ssize_t n) {
   require_args(n, 6, "cache_update");
   PyObject* cache = args[0];
   const bool full = truth(args[4]);
-  kvx_h2o_args a = h2o_args(cache, full, integer(args[3]), attr_int(cache, names._input_pos));
-  const at::Tensor sc = attr_tensor(cache, names.scores);
-  const Launch L(sc);
-  at::Tensor w;
-  if (const at::Tensor* t = opt_tensor(args[1], "attn_weights")) w = t->contiguous();
-  a.w = (const float*)data(w);
+  Held held;
+  kvx_h2o_args a = h2o_args(cache, full, integer(args[3]), attr_int(cache, names._input_pos), held);
+  const Launch L(held.tensors[0]);
+  const at::Tensor* given = opt_tensor(args[1], "attn_weights");
   a.q_len = (int32_t)integer(args[2]);
-  run_update(a, L, full ? attr_tensor(cache, names._next_flat) : L.empty({(int64_t)a.B * a.Hkv}, at::kInt), truth(args[5]));
+  const bool background = truth(args[5]);
+  at::Tensor next, w;
+  if (full) next = attr_tensor(cache, names._next_flat);
+  check(unlocked([&] {
+    if (given) w = given->contiguous();
+    if (!full) next = L.empty({(int64_t)a.B * a.Hkv}, at::kInt);
+    a.w = (const float*)data(w);
+    a.next_index = (int32_t*)next.data_ptr();
+    return run_update(a, L, background);
+  }));
   Py_RETURN_NONE;
 }
 
@@ -633,16 +671,19 @@ PyObject* cache_decode_step(PyObject* const* args, Py_ssize_t n) {
   a.v_zp = c.v_zp;
   a.qs_stride_b = c.qs_stride_b;
   a.qs_stride_h = c.qs_stride_h;
-  kvx_h2o_args h = h2o_args(cache, true, 1, input_pos + 1);
+  Held held;
+  kvx_h2o_args h = h2o_args(cache, true, 1, input_pos + 1, held);
   h.q_len = 1;
-  const at::Tensor out = L.empty({a.B, 1, (int64_t)a.Hq * a.D}, q.scalar_type());
-  const at::Tensor next = attr_tensor(cache, names._next_flat);
-  set_o(a, out, (int64_t)a.Hq * a.D, a.D, a.D);
-  h.next_index = (int32_t*)next.data_ptr();
-  const at::Tensor ws = L.scratch(lib.kvx_h2o_decode_step_workspace_bytes(&a, &h));
-  a.workspace = data(ws);
-  a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
-  check(lib.kvx_h2o_decode_step(&c, &a, &h, L.stream));
+  h.next_index = (int32_t*)held(attr_tensor(cache, names._next_flat)).data_ptr();
+  at::Tensor out;
+  check(unlocked([&] {
+    out = L.empty({a.B, 1, (int64_t)a.Hq * a.D}, q.scalar_type());
+    set_o(a, out, (int64_t)a.Hq * a.D, a.D, a.D);
+    const at::Tensor ws = L.scratch(lib.kvx_h2o_decode_step_workspace_bytes(&a, &h));
+    a.workspace = data(ws);
+    a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
+    return lib.kvx_h2o_decode_step(&c, &a, &h, L.stream);
+  }));
   return wrap(out);
 }
 
@@ -654,7 +695,7 @@ at::Tensor block_view(const at::Tensor& x, bool over_heads) {
   bool ok = x.stride(3) == 1 && (reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0;
   for (int i = 0; i < 3; ++i) ok = ok && x.stride(i) % 8 == 0;
   if (!over_heads && x.size(0) > 1) ok = ok && x.stride(0) == x.size(1) * x.stride(1);
-  return ok ? x : x.contiguous();
+  return ok ? x : unlocked([&] { return x.contiguous(); });
 }
 
 // quantize_blocks(x, start, codes, scales, zero_points, over_heads, bits) and dequantize_blocks: x (B, Hkv, num, D) of
@@ -693,7 +734,7 @@ PyObject* blocks_call(PyObject* const* args, Py_ssize_t n, bool quantize) {
   a.scale = (float*)scale.data_ptr() + start;
   a.zp = (int32_t*)zp.data_ptr() + start;
   a.state_stride_outer = scale.stride(0);
-  check((quantize ? lib.kvx_quantize_blocks : lib.kvx_dequantize_blocks)(&a, L.stream));
+  check(unlocked([&] { return (quantize ? lib.kvx_quantize_blocks : lib.kvx_dequantize_blocks)(&a, L.stream); }));
   Py_RETURN_NONE;
 }
 PyObject* quantize_blocks(PyObject* const* args, Py_ssize_t n) { return blocks_call(args, n, true); }
@@ -704,9 +745,11 @@ PyObject* dequantize_rows(PyObject* const* args, Py_ssize_t n) {
   require_args(n, 5, "dequantize_rows");
   const at::Tensor &codes = tensor(args[0], "codes"), &scale = tensor(args[1], "scales"), &zp = tensor(args[2], "zero_points"), &out = tensor(args[4], "out");
   const Launch L(codes);
-  const int64_t d = out.size(-1);
-  check(lib.kvx_dequantize_rows_typed((const uint8_t*)codes.data_ptr(), (const float*)scale.data_ptr(), (const int32_t*)zp.data_ptr(), out.numel() / d,
-                                      (int32_t)d, (int32_t)integer(args[3]), elem_dtype(out.scalar_type()), out.data_ptr(), d, L.stream));
+  const int64_t d = out.size(-1), bits = integer(args[3]);
+  check(unlocked([&] {
+    return lib.kvx_dequantize_rows_typed((const uint8_t*)codes.data_ptr(), (const float*)scale.data_ptr(), (const int32_t*)zp.data_ptr(), out.numel() / d,
+                                         (int32_t)d, (int32_t)bits, elem_dtype(out.scalar_type()), out.data_ptr(), d, L.stream);
+  }));
   Py_RETURN_NONE;
 }
 
@@ -728,11 +771,16 @@ PyObject* rmsnorm(PyObject* const* args, Py_ssize_t n) {
   const int64_t dim = x.dim() ? x.size(-1) : 0;
   if (weight.dim() != 1 || weight.size(0) != dim) raise(PyExc_ValueError, "weight.shape = %s, must be (%lld,)", shape_str(weight).c_str(), (long long)dim);
   const Launch L(x);
-  const at::Tensor x2 = rows2d(x, dim);
-  const at::Tensor out = args[3] == Py_None ? L.empty(x.sizes(), x.scalar_type()) : tensor(args[3], "out");
-  const at::Tensor o2 = out.view({-1, dim});
-  check(lib.kvx_rmsnorm_rows(x2.data_ptr(), x2.stride(0), o2.data_ptr(), o2.stride(0), (const float*)weight.data_ptr(), x2.size(0), (int32_t)dim,
-                             (float)real(args[2]), L.stream));
+  const float eps = (float)real(args[2]);
+  at::Tensor x2, out;
+  if (args[3] != Py_None) out = tensor(args[3], "out");
+  check(unlocked([&] {
+    x2 = rows2d(x, dim);
+    if (!out.defined()) out = L.empty(x.sizes(), x.scalar_type());
+    const at::Tensor o2 = out.view({-1, dim});
+    return lib.kvx_rmsnorm_rows(x2.data_ptr(), x2.stride(0), o2.data_ptr(), o2.stride(0), (const float*)weight.data_ptr(), x2.size(0), (int32_t)dim, eps,
+                                L.stream);
+  }));
   return wrap(out);
 }
 
@@ -747,10 +795,14 @@ PyObject* add_rmsnorm(PyObject* const* args, Py_ssize_t n) {
   if (x.sizes() != delta.sizes() || weight.dim() != 1 || weight.size(0) != dim || !x.is_contiguous())
     raise(PyExc_ValueError, "x %s (contiguous), delta %s, weight %s do not fit", shape_str(x).c_str(), shape_str(delta).c_str(), shape_str(weight).c_str());
   const Launch L(x);
-  const at::Tensor d2 = rows2d(delta, dim);
-  const at::Tensor out = L.empty(x.sizes(), x.scalar_type());
-  check(lib.kvx_add_rmsnorm_rows(x.data_ptr(), dim, d2.data_ptr(), d2.stride(0), x.data_ptr(), dim, out.data_ptr(), dim, (const float*)weight.data_ptr(),
-                                 x.numel() / dim, (int32_t)dim, (float)real(args[3]), L.stream));
+  const float eps = (float)real(args[3]);
+  at::Tensor d2, out;
+  check(unlocked([&] {
+    d2 = rows2d(delta, dim);
+    out = L.empty(x.sizes(), x.scalar_type());
+    return lib.kvx_add_rmsnorm_rows(x.data_ptr(), dim, d2.data_ptr(), d2.stride(0), x.data_ptr(), dim, out.data_ptr(), dim, (const float*)weight.data_ptr(),
+                                    x.numel() / dim, (int32_t)dim, eps, L.stream);
+  }));
   return wrap(out);
 }
 
@@ -763,11 +815,14 @@ PyObject* swiglu(PyObject* const* args, Py_ssize_t n) {
     raise(PyExc_ValueError, "swiglu takes bfloat16 rows of even width, a multiple of 16");
   const int64_t dim = g.size(-1) / 2;
   const Launch L(g);
-  const at::Tensor g2 = rows2d(g, 2 * dim);
   std::vector<int64_t> sizes = g.sizes().vec();
   sizes.back() = dim;
-  const at::Tensor out = L.empty(sizes, g.scalar_type());
-  check(lib.kvx_swiglu_rows(g2.data_ptr(), g2.stride(0), out.data_ptr(), dim, g2.size(0), (int32_t)dim, L.stream));
+  at::Tensor g2, out;
+  check(unlocked([&] {
+    g2 = rows2d(g, 2 * dim);
+    out = L.empty(sizes, g.scalar_type());
+    return lib.kvx_swiglu_rows(g2.data_ptr(), g2.stride(0), out.data_ptr(), dim, g2.size(0), (int32_t)dim, L.stream);
+  }));
   return wrap(out);
 }
 
@@ -784,10 +839,14 @@ PyObject* qk_norm_rope(PyObject* const* args, Py_ssize_t n) {
   if (cos.sizes() != sin.sizes() || cos.dim() != 2 || cos.size(1) != d / 2 || cos.scalar_type() != at::kFloat)
     raise(PyExc_ValueError, "cos / sin must be float32 (positions, head_size / 2) tables");
   const at::Tensor *qw = opt_tensor(args[4], "q_weight"), *kw = opt_tensor(args[5], "k_weight");
+  const float eps = (float)real(args[6]);
+  const int64_t input_pos = integer(args[9]);
   const Launch L(qkv);
-  check(lib.kvx_qk_norm_rope(qkv.data_ptr(), qkv.stride(0), qkv.stride(1), (int32_t)qkv.size(0), (int32_t)qkv.size(1), (int32_t)hq, (int32_t)hkv, (int32_t)d,
-                             qw ? (const float*)qw->data_ptr() : nullptr, kw ? (const float*)kw->data_ptr() : nullptr, (float)real(args[6]),
-                             (const float*)cos.data_ptr(), (const float*)sin.data_ptr(), (int32_t)cos.size(0), (int32_t)integer(args[9]), L.stream));
+  check(unlocked([&] {
+    return lib.kvx_qk_norm_rope(qkv.data_ptr(), qkv.stride(0), qkv.stride(1), (int32_t)qkv.size(0), (int32_t)qkv.size(1), (int32_t)hq, (int32_t)hkv,
+                                (int32_t)d, qw ? (const float*)qw->data_ptr() : nullptr, kw ? (const float*)kw->data_ptr() : nullptr, eps,
+                                (const float*)cos.data_ptr(), (const float*)sin.data_ptr(), (int32_t)cos.size(0), (int32_t)input_pos, L.stream);
+  }));
   Py_RETURN_NONE;
 }
 
