@@ -181,14 +181,17 @@ std::string dtype_name(at::ScalarType t) {
   return t == at::kBFloat16 ? "torch.bfloat16" : t == at::kHalf ? "torch.float16" : t == at::kByte ? "torch.uint8" : t == at::kFloat ? "torch.float32" : s;
 }
 
+// A QuantState, any object with its attributes, or a bare tuple in its order; keys_only: the state of V is not looked at.
 struct Quant {
   at::Tensor ks, kz, vs, vz;
-  Quant(PyObject* o) {
-    if (!PyTuple_Check(o) || PyTuple_GET_SIZE(o) != 4) raise(PyExc_ValueError, "quant must be a QuantState");
-    ks = tensor(PyTuple_GET_ITEM(o, 0), "k_scale");
-    kz = tensor(PyTuple_GET_ITEM(o, 1), "k_zp");
-    vs = tensor(PyTuple_GET_ITEM(o, 2), "v_scale");
-    vz = tensor(PyTuple_GET_ITEM(o, 3), "v_zp");
+  explicit Quant(PyObject* o, bool keys_only = false) {
+    const bool bare = PyTuple_CheckExact(o);
+    if (bare && PyTuple_GET_SIZE(o) != 4) raise(PyExc_ValueError, "quant must be a QuantState");
+    auto field = [&](int i, PyObject* name) { return bare ? tensor(PyTuple_GET_ITEM(o, i), PyUnicode_AsUTF8(name)) : attr_tensor(o, name); };
+    ks = field(0, names.k_scale);
+    kz = field(1, names.k_zp);
+    vs = keys_only ? ks : field(2, names.v_scale);
+    vz = keys_only ? kz : field(3, names.v_zp);
   }
 };
 
@@ -377,11 +380,7 @@ PyObject* score_sum(PyObject* const* args, Py_ssize_t n) {
   check_bhtd("query", q);
   check_bhtd("key", k);
   std::optional<Quant> qs;
-  if (args[6] != Py_None) {
-    qs.emplace(args[6]);
-    qs->vs = qs->ks;
-    qs->vz = qs->kz;
-  }
+  if (args[6] != Py_None) qs.emplace(args[6], true);
   check_dtypes(q, k, nullptr, qs.has_value());
   const int64_t B = q.size(0), Hq = q.size(1), q_len = q.size(2);
   if (lse.dim() != 3 || lse.size(0) != B || lse.size(1) != q_len || lse.size(2) != Hq || lse.scalar_type() != at::kFloat || !lse.is_contiguous())

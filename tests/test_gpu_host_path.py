@@ -1,9 +1,11 @@
-"""The native host path (csrc/host.cpp): other Python threads run while a call allocates and launches."""
+"""The native host path (csrc/host.cpp): other Python threads run while a call allocates and launches, and the
+arguments it takes."""
 import ctypes
 import os
 import subprocess
 import threading
 import time
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -157,3 +159,49 @@ def test_two_threads_on_two_streams(gpu):
     assert not errors
     for one, other in zip(want, got):
         assert all(torch.equal(x, y) for x, y in zip(one, other))
+
+
+def _store(gpu, B, Hkv, T, D, bits=8, dtype=torch.bfloat16, seed=0):
+    gen = torch.Generator(device=gpu).manual_seed(seed)
+    codes, state, rows = [], [], []
+    for _ in range(2):
+        qz = RowQuantizer((B, Hkv, T, D), dtype, bits, allocate_buffers=True, device=gpu)
+        qz.quantize(0, T, torch.randn(B, Hkv, T, D, generator=gen, device=gpu).to(dtype))
+        codes.append(qz.quant_buffer.view(B, Hkv, T, -1))
+        state += [qz.quant_scales.view(B, Hkv, T), qz.quant_zero_points.view(B, Hkv, T)]
+        rows.append(qz.dequantize(0, T))
+    return codes, ops.QuantState(*state), rows
+
+
+def test_score_sums_need_the_state_of_the_keys_only(gpu):
+    B, Hq, Hkv, q_len, T, D = 2, 8, 2, 40, 300, 64
+    (kc, _), state, (kd, _) = _store(gpu, B, Hkv, T, D)
+    q = torch.randn(B, Hq, q_len, D, device=gpu).to(torch.bfloat16)
+    _, _, lse = ops.prefill_core(q, kd, kd, 0.125, T - q_len, return_lse=True)
+    want = ops.score_sum_core(q, kc, lse, 0.125, T - q_len, quant=state)
+    for given in (state._replace(v_scale=None, v_zp=None), SimpleNamespace(k_scale=state.k_scale, k_zp=state.k_zp)):
+        assert torch.equal(ops.score_sum_core(q, kc, lse, 0.125, T - q_len, quant=given), want)
+
+
+def test_state_objects_of_other_types(gpu):
+    """Any object with the four arrays is a quantiser state, and so is a bare tuple of them."""
+    B, Hq, Hkv, T, D = 1, 4, 2, 200, 64
+    (kc, vc), state, _ = _store(gpu, B, Hkv, T, D)
+
+    class State:
+        def __init__(self, s):
+            self.k_scale, self.k_zp, self.v_scale, self.v_zp = s
+
+        def __iter__(self):
+            return iter((self.k_scale, self.k_zp, self.v_scale, self.v_zp))
+
+    q = torch.randn(B, Hq, 16, D, device=gpu).to(torch.bfloat16)
+    out, _, _ = ops.prefill_core(q, kc, vc, 0.125, T - 16, quant=state)
+    assert torch.equal(ops.prefill_core(q, kc, vc, 0.125, T - 16, quant=State(state))[0], out)
+    one, _, _ = ops.decode_core(q[:, :, :1], kc, vc, 0.125, quant=state)
+    assert torch.equal(ops.decode_core(q[:, :, :1], kc, vc, 0.125, quant=State(state))[0], one)
+    assert torch.equal(ops.prefill_core(q, kc, vc, 0.125, T - 16, quant=tuple(state))[0], out)
+    with pytest.raises(ValueError, match="QuantState"):
+        ops.prefill_core(q, kc, vc, 0.125, T - 16, quant=tuple(state)[:3])
+    with pytest.raises(TypeError, match="v_zp"):
+        ops.prefill_core(q, kc, vc, 0.125, T - 16, quant=state._replace(v_zp=None))
