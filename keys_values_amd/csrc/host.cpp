@@ -133,6 +133,8 @@ struct Ref {  // an owned reference
   Ref(Ref&& o) : p(o.p) { o.p = nullptr; }
   ~Ref() { Py_XDECREF(p); }
 };
+// int(o): positions and counts may be floats and the like
+int64_t converted(PyObject* o) { return PyLong_Check(o) ? integer(o) : integer(Ref(PyNumber_Long(o)).p); }
 Ref attr(PyObject* o, PyObject* name) { return Ref(PyObject_GetAttr(o, name)); }
 int64_t attr_int(PyObject* o, PyObject* name) { return integer(attr(o, name).p); }
 at::Tensor attr_tensor(PyObject* o, PyObject* name) { return tensor(attr(o, name).p, PyUnicode_AsUTF8(name)); }
@@ -364,7 +366,7 @@ PyObject* prefill(PyObject* const* args, Py_ssize_t n) {
   check_heads(q.size(1), k.size(1));
   check_head_size(q.size(3));
   const Launch L(q);
-  kvx_sdpa_args a = sdpa_args(q, k, &v, real(args[3]), integer(args[4]), qs ? &*qs : nullptr, integer(args[10]));
+  kvx_sdpa_args a = sdpa_args(q, k, &v, real(args[3]), converted(args[4]), qs ? &*qs : nullptr, converted(args[10]));
   at::Tensor keep;
   set_positions(a, opt_tensor(args[5], "token_positions"), keep);
   const bool want_lse = truth(args[7]);
@@ -388,7 +390,7 @@ PyObject* score_sum(PyObject* const* args, Py_ssize_t n) {
           shape_str(lse).c_str(), dtype_name(lse.scalar_type()).c_str());
   check_head_size(q.size(3));
   const Launch L(q);
-  kvx_sdpa_args a = sdpa_args(q, k, nullptr, real(args[3]), integer(args[4]), qs ? &*qs : nullptr, 0);
+  kvx_sdpa_args a = sdpa_args(q, k, nullptr, real(args[3]), converted(args[4]), qs ? &*qs : nullptr, 0);
   at::Tensor keep;
   set_positions(a, opt_tensor(args[5], "token_positions"), keep);
   a.lse = (float*)lse.data_ptr();
@@ -421,7 +423,7 @@ PyObject* decode(PyObject* const* args, Py_ssize_t n) {
   check_head_size(q.size(3));
   const int64_t T = k.size(2);
   const Launch L(q);
-  kvx_sdpa_args a = sdpa_args(q, k, &v, real(args[3]), T > 0 ? T - 1 : 0, qs ? &*qs : nullptr, integer(args[7]));
+  kvx_sdpa_args a = sdpa_args(q, k, &v, real(args[3]), T > 0 ? T - 1 : 0, qs ? &*qs : nullptr, converted(args[7]));
   if (const at::Tensor* s = opt_tensor(args[8], "scratch_splits")) {
     if (s->scalar_type() != at::kInt || s->numel() != 1 || s->device() != q.device())
       raise(PyExc_ValueError, "scratch_splits must be a one-element int32 tensor on the query's device");
@@ -839,7 +841,7 @@ PyObject* qk_norm_rope(PyObject* const* args, Py_ssize_t n) {
     raise(PyExc_ValueError, "cos / sin must be float32 (positions, head_size / 2) tables");
   const at::Tensor *qw = opt_tensor(args[4], "q_weight"), *kw = opt_tensor(args[5], "k_weight");
   const float eps = (float)real(args[6]);
-  const int64_t input_pos = integer(args[9]);
+  const int64_t input_pos = converted(args[9]);
   const Launch L(qkv);
   check(unlocked([&] {
     return lib.kvx_qk_norm_rope(qkv.data_ptr(), qkv.stride(0), qkv.stride(1), (int32_t)qkv.size(0), (int32_t)qkv.size(1), (int32_t)hq, (int32_t)hkv,

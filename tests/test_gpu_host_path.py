@@ -205,3 +205,20 @@ def test_state_objects_of_other_types(gpu):
         ops.prefill_core(q, kc, vc, 0.125, T - 16, quant=tuple(state)[:3])
     with pytest.raises(TypeError, match="v_zp"):
         ops.prefill_core(q, kc, vc, 0.125, T - 16, quant=state._replace(v_zp=None))
+
+
+def test_positions_and_counts_of_other_types(gpu):
+    """They are converted as int() does."""
+    q, k = (torch.randn(1, h, n, 64, device=gpu).to(torch.bfloat16) for h, n in ((4, 16), (2, 200)))
+    out, w, lse = ops.prefill_core(q, k, k, 0.125, 184, return_weights=True, return_lse=True, num_splits=2)
+    for pos, splits in ((184.0, 2.0), (torch.tensor(184), torch.tensor(2.0)), ("184", "2")):
+        got = ops.prefill_core(q, k, k, 0.125, pos, return_weights=True, return_lse=True, num_splits=splits)
+        assert all(torch.equal(x, y) for x, y in zip(got, (out, w, lse)))
+        assert torch.equal(ops.score_sum_core(q, k, lse, 0.125, pos), ops.score_sum_core(q, k, lse, 0.125, 184))
+        one = ops.decode_core(q[:, :, :1], k, k, 0.125, num_splits=splits)[0]
+        assert torch.equal(one, ops.decode_core(q[:, :, :1], k, k, 0.125, num_splits=2)[0])
+    x, weight, table = torch.randn(1, 4, 8 * 64, device=gpu).to(torch.bfloat16), torch.ones(64, device=gpu), torch.rand(64, 32, device=gpu)
+    assert torch.equal(lops.qk_norm_rope_(x.clone(), 4, 2, 64, weight, weight, 1e-6, table, table, 3.0),
+                       lops.qk_norm_rope_(x.clone(), 4, 2, 64, weight, weight, 1e-6, table, table, 3))
+    with pytest.raises(TypeError):
+        ops.prefill_core(q, k, k, 0.125, None)
