@@ -111,13 +111,19 @@ def prefill_core(
     output_transposed: bool = True,
     quant: Optional[QuantState] = None,
     num_splits: int = 0,
+    fused_dequant: bool = False,
 ) -> Tuple[torch.Tensor, Optional[torch.Tensor], Optional[torch.Tensor]]:
     """Chunked-prefill attention on strided (B, H, len, D) views.
 
     Returns ``(out, weights, lse)``: ``out`` is (B, q, Hq, D) if ``output_transposed`` (the layout
     of the reference extension) else (B, Hq, q, D); ``weights`` fp32 (B, Hkv, T) summed over queries
-    and averaged over the group; ``lse`` fp32 (B, q, Hq) in base 2."""
-    return _lib.host().prefill(query, key, value, scale, input_pos, token_positions, return_weights, return_lse, output_transposed, quant, num_splits, False)
+    and averaged over the group; ``lse`` fp32 (B, q, Hq) in base 2.
+
+    ``fused_dequant``: over a quantised store a long chunk (from 1025 query rows, tokens x heads per KV head, on; 129 at
+    head size 256) takes scratch for a copy of the store in 16-bit rows, ``4 * B * Hkv * T * D`` bytes for the time of the
+    call, where the device has that much left. ``True``: never; the kernels dequantise for themselves."""
+    return _lib.host().prefill(query, key, value, scale, input_pos, token_positions, return_weights, return_lse, output_transposed, quant, num_splits,
+                               fused_dequant)
 
 
 def score_sum_core(query, key, lse, scale, input_pos, token_positions=None, quant: Optional[QuantState] = None):

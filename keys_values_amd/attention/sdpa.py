@@ -59,10 +59,14 @@ def sdpa_check_args(query, key, value, packed4: bool = False):
 
 class HipSDPA:
     """Same call surface as ``FlashInferSDPA``; ``available`` replaces its constructor-time probe
-    (keys_values/attention/flashinfer_wrapper.py:331-365)."""
+    (keys_values/attention/flashinfer_wrapper.py:331-365). ``fused_dequant=True``: calls over a quantised store take no
+    scratch for a 16-bit copy of it (see ``ops.prefill_core``); long chunks are slower then."""
 
-    def __init__(self):
+    fused_dequant = False
+
+    def __init__(self, fused_dequant: bool = False):
         self.available = ops.is_available()
+        self.fused_dequant = bool(fused_dequant)
 
     def scaled_dot_product_attention(
         self,
@@ -117,7 +121,7 @@ class HipSDPA:
         else:
             attn_outputs, attn_weights, _ = ops.prefill_core(
                 query, key, value, scale_factor, input_pos, token_positions, return_attn_weights,
-                return_lse=False, output_transposed=output_transposed, quant=quant,
+                return_lse=False, output_transposed=output_transposed, quant=quant, fused_dequant=self.fused_dequant,
             )
         if head_size_diff is not None:
             attn_outputs = attn_outputs[:, :, :, :head_size]
@@ -129,11 +133,12 @@ class HipMultiHeadSelfAttention:
     configurations the HIP kernels serve (no sliding window, no logit soft-capping): the cache passes the
     queries and a ``KeysAndValues`` holder and gets ``(attn_outputs (B, q_len, n_head * hs), attn_weights)``.
     ``input_pos`` 0 / None is the causal first chunk (no weights, keys_values/kvcache/base.py:567-581). A holder
-    of a quantised store (``key_codes`` / ``value_codes`` / ``quant``) is read in place by the kernels."""
+    of a quantised store (``key_codes`` / ``value_codes`` / ``quant``) is read in place by the kernels, or, long chunks
+    without ``fused_dequant``, copied to 16-bit rows for the call (see ``ops.prefill_core``)."""
 
-    def __init__(self, scale_factor: Optional[float] = None):
+    def __init__(self, scale_factor: Optional[float] = None, fused_dequant: bool = False):
         self.scale_factor = scale_factor
-        self._sdpa = get_hip_sdpa()
+        self._sdpa = HipSDPA(fused_dequant=True) if fused_dequant else get_hip_sdpa()
 
     def __call__(self, query: torch.Tensor, k_and_v, block_idx: int = 0, input_pos: Optional[int] = None,
                  return_attn_weights: bool = False, token_positions: Optional[torch.Tensor] = None):
@@ -156,7 +161,8 @@ class HipMultiHeadSelfAttention:
                 query, key, value, diff = _pad_head_size(query, key, value)
             else:
                 diff = None
-            out, _, _ = ops.prefill_core(query, key, value, scale, 0, None, return_weights=False, output_transposed=True, quant=quant)
+            out, _, _ = ops.prefill_core(query, key, value, scale, 0, None, return_weights=False, output_transposed=True, quant=quant,
+                                         fused_dequant=self._sdpa.fused_dequant)
             if diff is not None:
                 out = out[..., :head_size]
             return out.reshape(batch_size, q_len, -1), None

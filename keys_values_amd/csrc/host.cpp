@@ -17,7 +17,9 @@
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <dlfcn.h>
 
 #include <algorithm>
@@ -318,6 +320,26 @@ struct AttnOut {
   at::Tensor out, w, lse;
 };
 
+// Whether the allocator can hand out `bytes`. Asked when it cannot, it first gives every cached block back and waits for
+// the device, and would do so on every call of a program that fills the memory. What it holds but cannot give back are blocks
+// in use and the rest of blocks it has split.
+bool has_room(const Launch& L, size_t bytes) {
+  namespace allocator = c10::hip::HIPCachingAllocator;
+  constexpr size_t kAll = 0, kGranule = (size_t)2 << 20;  // CachingAllocator's StatType::AGGREGATE; large blocks are multiples of 2 MiB
+  try {
+    const auto s = allocator::getDeviceStats(L.dev);
+    const size_t reserved = s.reserved_bytes[kAll].current, kept = s.active_bytes[kAll].current + s.inactive_split_bytes[kAll].current;
+    if (kept + bytes + kGranule <= reserved) return true;
+    if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) return true;  // no queries while recording
+    size_t free = 0, total = 0;
+    if (hipMemGetInfo(&free, &total) != hipSuccess) return true;
+    const size_t most = std::min(free + reserved, (size_t)(allocator::getMemoryFraction(L.dev) * (double)total));
+    return kept + bytes + kGranule <= most;
+  } catch (const c10::Error&) {
+    return true;  // an allocator that keeps no such account
+  }
+}
+
 // prefill attention on checked operands; `copy`: a quantised store may be dequantised into the scratch where that is faster
 AttnOut run_prefill(kvx_sdpa_args& a, const Launch& L, at::ScalarType type, bool weights, bool want_lse, bool transposed, bool copy) {
   AttnOut r;
@@ -333,13 +355,15 @@ AttnOut run_prefill(kvx_sdpa_args& a, const Launch& L, at::ScalarType type, bool
     if (weights) r.w = L.empty({a.B, a.Hkv, a.kv_len}, at::kFloat);
     a.lse = (float*)data(r.lse);
     a.w = (float*)data(r.w);
+    const size_t least = lib.kvx_sdpa_prefill_workspace_bytes(&a), most = copy ? lib.kvx_sdpa_prefill_copying_workspace_bytes(&a) : least;
+    if (most > least) copy = has_room(L, most);  // not more where no copy pays, or where it spares as many partial results
     at::Tensor ws;
     try {
-      ws = L.scratch((copy ? lib.kvx_sdpa_prefill_copying_workspace_bytes : lib.kvx_sdpa_prefill_workspace_bytes)(&a));
+      ws = L.scratch(copy ? most : least);
     } catch (const c10::OutOfMemoryError&) {
       if (!copy) throw;
-      copy = false;  // no room for a copy of a quantised store: the form that needs none
-      ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
+      copy = false;  // no room for a copy of a quantised store after all: the form that needs none
+      ws = L.scratch(least);
     }
     a.workspace = data(ws);
     a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;

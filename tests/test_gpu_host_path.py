@@ -1,5 +1,5 @@
-"""The native host path (csrc/host.cpp): other Python threads run while a call allocates and launches, and the
-arguments it takes."""
+"""The native host path (csrc/host.cpp): other Python threads run while a call allocates and launches, the arguments it
+takes, and what a call over a quantised store allocates."""
 import ctypes
 import os
 import subprocess
@@ -10,8 +10,11 @@ from types import SimpleNamespace
 import pytest
 import torch
 
+from helpers import rel_err
 from keys_values_amd import _lib
 from keys_values_amd.attention import ops
+from keys_values_amd.attention.sdpa import HipMultiHeadSelfAttention, HipSDPA
+from keys_values_amd.kvcache.buffers import QuantizedKeysAndValues
 from keys_values_amd.kvcache.h2o import H2OKVCache, KVCacheParams
 from keys_values_amd.kvcache.quantize import RowQuantizer
 from keys_values_amd.longctx import ops as lops
@@ -222,3 +225,90 @@ def test_positions_and_counts_of_other_types(gpu):
                        lops.qk_norm_rope_(x.clone(), 4, 2, 64, weight, weight, 1e-6, table, table, 3))
     with pytest.raises(TypeError):
         ops.prefill_core(q, k, k, 0.125, None)
+
+
+# A long chunk over 8 x 16384 8-bit rows of 128: the copy of the store in 16-bit rows is 64 MiB
+_LONG = dict(B=1, Hkv=8, T=16384, D=128, Hq=32, q_len=512)
+_COPY = 2 * 8 * 16384 * 128 * 2
+
+
+def _long_call(gpu):
+    c = _LONG
+    codes, state, rows = _store(gpu, c["B"], c["Hkv"], c["T"], c["D"])
+    q = torch.randn(c["B"], c["Hq"], c["q_len"], c["D"], device=gpu).to(torch.bfloat16)
+    return q, codes, state, rows, (c["D"] ** -0.5, c["T"] - c["q_len"], None)
+
+
+def _extra_bytes(gpu, run):
+    """Largest amount of memory in use during run() beyond what was in use before."""
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats(gpu)
+    before = torch.cuda.memory_allocated(gpu)
+    out = run()
+    torch.cuda.synchronize()
+    return torch.cuda.max_memory_allocated(gpu) - before, out
+
+
+def test_the_caller_decides_on_the_copy_of_a_quantised_store(gpu):
+    q, codes, state, rows, args = _long_call(gpu)
+    want, w_want, _ = ops.prefill_core(q, *rows, *args, return_weights=True)
+    scale, pos, _ = args
+    mine = QuantizedKeysAndValues(*codes, state, _LONG["D"], 8, torch.bfloat16)
+    every = torch.arange(_LONG["T"], device=gpu).expand(1, 8, -1)
+    calls = {
+        "prefill_core": lambda **kw: ops.prefill_core(q, *codes, *args, return_weights=True, num_splits=1, quant=state, **kw)[:2],
+        "HipSDPA": lambda **kw: HipSDPA(**kw).scaled_dot_product_attention(q, *codes, scale, pos, None, True, output_transposed=True, quant=state),
+        "HipMultiHeadSelfAttention": lambda **kw: HipMultiHeadSelfAttention(**kw)(q, mine, 0, pos, True, every),
+    }
+    for name, call in calls.items():
+        copied, (out, w) = _extra_bytes(gpu, call)
+        fused, (out_f, w_f) = _extra_bytes(gpu, lambda: call(fused_dequant=True))
+        print(name, copied, fused, flush=True)
+        assert copied >= _COPY, name
+        assert fused <= copied - _COPY // 2, name
+        for o, x in ((out, w), (out_f, w_f)):
+            assert rel_err(o.float().view(want.shape), want.float()) < 1e-2
+            torch.testing.assert_close(x, w_want, rtol=1e-4, atol=1e-7)
+
+
+def test_no_room_for_the_copy(gpu):
+    """Where the memory for the copy is not there the call runs without one, and does not make the allocator empty its
+    cache to find out."""
+    q, codes, state, rows, args = _long_call(gpu)
+    want, _, _ = ops.prefill_core(q, *rows, *args)
+    del rows
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(gpu).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_allocated(gpu) + _COPY // 2) / total, gpu)
+        torch.cuda.reset_peak_memory_stats(gpu)
+        retries = torch.cuda.memory_stats(gpu)["num_alloc_retries"]
+        outs = [ops.prefill_core(q, *codes, *args, quant=state, num_splits=1)[0] for _ in range(3)]
+        torch.cuda.synchronize()
+        stats = torch.cuda.memory_stats(gpu)
+        assert stats["num_alloc_retries"] == retries and stats["num_ooms"] == 0
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, gpu)
+    for out in outs:
+        assert rel_err(out.float(), want.float()) < 1e-2
+    assert _extra_bytes(gpu, lambda: ops.prefill_core(q, *codes, *args, quant=state, num_splits=1))[0] >= _COPY  # room again: the copy
+
+
+def test_a_long_chunk_over_a_quantised_store_in_a_graph(gpu):
+    """Recorded with its copy, replayed between other work: the eager call's results each time."""
+    q, codes, state, _, args = _long_call(gpu)
+    q0, q1 = q.clone(), torch.randn_like(q)
+    run = lambda: ops.prefill_core(q, *codes, *args, return_weights=True, quant=state)[:2]  # noqa: E731
+    run()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()  # the recorded call's memory comes from the device
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out, w = run()
+    for query in (q0, q1, q0, q1):
+        q.copy_(query)
+        want, w_want = run()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(w, w_want)
