@@ -60,8 +60,13 @@ EAGER_SELECT = 4096
 # Query rows (tokens x heads per KV head) of a chunk from which dequantising the store once per chunk
 # is faster than dequantising it inside the attention kernels (every 256 rows walk the whole store):
 # the copy costs two passes over the store, the kernels gain in proportion to the rows.
-DEFAULT_DEQUANTIZE_CHUNK_ROWS = 2048
-DEFAULT_DEQUANTIZE_CHUNK_ROWS_256 = 129  # head size 256
+class _DefaultRows(int):
+    """A threshold nobody chose: below it the attention call may still decide for a copy of its own. The same number given
+    by a caller is a plain int, and kept to."""
+
+
+DEFAULT_DEQUANTIZE_CHUNK_ROWS = _DefaultRows(2048)
+DEFAULT_DEQUANTIZE_CHUNK_ROWS_256 = _DefaultRows(129)  # head size 256
 
 _dequant_buffers = {}
 _dequant_owner = {}  # per buffer: the cache whose rows it holds as that cache's working buffer (blocks over heads), else None
@@ -128,9 +133,9 @@ class H2OKVCache:
         self.blocks_over_heads = bool(blocks_over_heads) and quantized
         # dequantize_chunk_rows: a chunk with at least this many query rows (tokens x heads per KV head) is
         # attended to over a bf16 copy of the quantised store made once for the chunk; None = never. Left at its default it
-        # is lower at head size 256, where the dequantising kernel has no registers to spare.
-        self._default_chunk_rows = dequantize_chunk_rows == DEFAULT_DEQUANTIZE_CHUNK_ROWS
-        if dequantize_chunk_rows == DEFAULT_DEQUANTIZE_CHUNK_ROWS and params.head_size == 256:
+        # is lower at head size 256, where the dequantising kernel has no registers to spare, and shorter chunks (from 1025
+        # rows on) may be given a copy for the time of the call.
+        if isinstance(dequantize_chunk_rows, _DefaultRows) and params.head_size == 256:
             dequantize_chunk_rows = DEFAULT_DEQUANTIZE_CHUNK_ROWS_256
         self.dequantize_chunk_rows = dequantize_chunk_rows
         # overlap_select: launch the score update + eviction choice of a chunk step (and, for a long chunk over
@@ -546,7 +551,8 @@ class H2OKVCache:
             else:
                 # at the default threshold the call itself decides whether a copy pays below it; a threshold (or None) that
                 # the caller chose is kept to
-                out, w, _ = host.prefill(query, kc, vc, self.scale_factor, input_pos, tp, True, False, True, quant, 0, not self._default_chunk_rows)
+                fused = not isinstance(self.dequantize_chunk_rows, _DefaultRows)
+                out, w, _ = host.prefill(query, kc, vc, self.scale_factor, input_pos, tp, True, False, True, quant, 0, fused)
         self._update(w, num)
         return out.view(b, num, hq * d)
 

@@ -15,7 +15,7 @@ from keys_values_amd import _lib
 from keys_values_amd.attention import ops
 from keys_values_amd.attention.sdpa import HipMultiHeadSelfAttention, HipSDPA
 from keys_values_amd.kvcache.buffers import QuantizedKeysAndValues
-from keys_values_amd.kvcache.h2o import H2OKVCache, KVCacheParams
+from keys_values_amd.kvcache.h2o import H2OKVCache, KVCacheParams, create_kv_cache
 from keys_values_amd.kvcache.quantize import RowQuantizer
 from keys_values_amd.longctx import ops as lops
 
@@ -312,3 +312,29 @@ def test_a_long_chunk_over_a_quantised_store_in_a_graph(gpu):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want) and torch.equal(w, w_want)
+
+
+def test_a_chosen_threshold_is_kept_to(gpu):
+    """dequantize_chunk_rows given by the caller, or set later, holds, also where it is the default's number: chunks below it
+    never take a copy. Left at its default the call decides."""
+    Hkv, L, D, Hq, chunk = 8, 8192, 128, 32, 400  # 1600 query rows
+    extra = {}
+    for name, kw in (("default", {}), ("chosen", {"dequantize_chunk_rows": 2048}), ("never", {"dequantize_chunk_rows": None})):
+        for make in (lambda c: c, lambda c: c.clone()):
+            cache = make(create_kv_cache("h2o-torch-quantized8", KVCacheParams(1, Hkv, L, D, Hq), max_chunk_size=chunk, device=gpu, **kw))
+            first = [torch.randn(1, h, L, D, device=gpu).to(torch.bfloat16) for h in (Hq, Hkv, Hkv)]
+            cache.forward(*first)
+            step = [t[:, :, :chunk].contiguous() for t in first]
+            cache.forward(*step)
+            extra[name], _ = _extra_bytes(gpu, lambda: cache.forward(*step))
+        if name == "default":
+            cache.dequantize_chunk_rows = None
+            extra["set later"], _ = _extra_bytes(gpu, lambda: cache.forward(*step))
+    print(extra, flush=True)
+    copy = 2 * Hkv * L * D * 2
+    assert extra["default"] >= copy
+    assert extra["chosen"] == extra["never"] == extra["set later"] <= extra["default"] - copy // 2
+    p256 = KVCacheParams(1, 2, 256, 256, 4)
+    assert H2OKVCache(p256, quantized=True, device=gpu).dequantize_chunk_rows == 129
+    assert H2OKVCache(p256, quantized=True, device=gpu, dequantize_chunk_rows=2048).dequantize_chunk_rows == 2048
+    assert H2OKVCache(p256, quantized=True, device=gpu, dequantize_chunk_rows=None).dequantize_chunk_rows is None
