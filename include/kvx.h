@@ -164,11 +164,15 @@ size_t kvx_sdpa_prefill_copying_workspace_bytes(const kvx_sdpa_args* args);
  * (keys_values/attention/flashinfer_wrapper.py:471-481, keys_values/attention/flashinfer_ops.py:250-275).
  * Stands in for sdpa_decode of the reference extension (keys_values/csrc/bindings.cpp:86-489) and
  * optimized_batched_decode_kernel (keys_values/csrc/kernels/sdpa_decode.cu:616-898). One workgroup
- * per (batch, KV head, split) serves all G query heads, so K and V are read once. With args->w set, a
- * split keeps its logits on the chip, waits (boundedly) until the other splits of its (batch, KV head) row
- * have published their partial maxima and sums, and writes its part of W itself; the workspace holds
- * the split partials, the rows' arrival counters and room for the fp32 logits (B, Hq, kv_len) of the
- * splits that are too long for that or whose wait ran out. args->lse optional. */
+ * per (batch, KV head, split) serves all G query heads, so K and V are read once. A split that has published its
+ * partial outputs, maxima and sums waits (boundedly, see kvx_decode_tuning) until the other splits of its (batch,
+ * KV head) row have done so, with or without args->w, and then writes its share of the row's outputs and, with args->w
+ * set, its part of W from the logits it keeps on the chip. What splits whose wait ran out have left undone the row's last
+ * split does, so the results are the same; a call on a device that another stream fills with long kernels can hold its
+ * compute units for that long (about 30 ms at the defaults). Without args->w there is no wait where the splits of a row
+ * do not fit the device side by side. The workspace holds the split partials, the rows' arrival counters and, with
+ * args->w, room for the fp32 logits (B, Hq, kv_len) of the splits that are too long for the chip or whose wait ran out.
+ * args->lse optional. */
 int kvx_sdpa_decode(const kvx_sdpa_args* args, void* stream);
 size_t kvx_sdpa_decode_workspace_bytes(const kvx_sdpa_args* args);
 
@@ -185,10 +189,11 @@ struct kvx_h2o_args;
 int kvx_sdpa_decode_h2o(const kvx_sdpa_args* args, const struct kvx_h2o_args* h, void* stream);
 size_t kvx_sdpa_decode_h2o_workspace_bytes(const kvx_sdpa_args* args);
 
-/* Process-wide switches of the decode kernels' weights route, for tests and measurement; no counterpart in the
+/* Process-wide switches of the decode kernels, for tests and measurement; no counterpart in the
  * reference. resident: 0 sends every split's logits through the workspace and the tail kernel, 1 keeps them on the
- * chip where they fit. spin_limit: polls a split spends waiting for the other splits of its row before it gives up
- * and takes the workspace route (0 = never wait; clamped to 2^20). poll_sleep: pause between two polls in units of
+ * chip where they fit (calls with weights only). spin_limit: polls a split spends waiting for the other splits of its row
+ * before it leaves its share to the row's last one and its logits, if weights are wanted, to the workspace (0 = never
+ * wait; clamped to 2^20; every call whose splits finish the row themselves, with weights or without). poll_sleep: pause between two polls in units of
  * 512 cycles (clamped to 64). A negative value restores that switch to its default: the environment variables
  * KVX_DECODE_RESIDENT / KVX_DECODE_SPIN_LIMIT / KVX_DECODE_POLL_SLEEP as read once at the first decode call
  * (else 1, 32768, 4). A workspace size query and the call it is for must see the same setting of `resident`. */

@@ -608,3 +608,27 @@ def test_decode_output_at_large_logits(gpu, decode_route, D, G, store, T):
         out, _, lse = ops.decode_core(q, kd, vd, D ** -0.5, return_weights=weights, return_lse=True, quant=quant)
         assert lse.min() > 2.0 ** 17
         assert rel_err(out, want) < 1e-3, (weights, rel_err(out, want))
+
+
+def test_decode_without_weights_beside_other_work(gpu, decode_route):
+    """Without weights the splits of a row wait for each other too, before each writes its share of the outputs; where the
+    wait runs out the last one makes up for it. The same bits whoever does."""
+    B, Hq, Hkv, T, D = 2, 8, 2, 30000, 128
+    q, k, v, _ = make_qkv(4243, B, Hq, Hkv, 1, T, D)
+    qg, kg, vg = q.to(gpu), k.to(gpu), v.to(gpu)
+    scale = 1.0 / math.sqrt(D)
+    out0, _, lse0 = ops.decode_core(qg, kg, vg, scale, return_lse=True)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream(gpu)
+    busy = torch.randn(4096, 4096, device=gpu, dtype=torch.bfloat16)
+    side.wait_stream(torch.cuda.current_stream(gpu))
+    for _ in range(3):
+        with torch.cuda.stream(side):
+            for _ in range(20):
+                busy = (busy @ busy).clamp_(-1, 1)
+        out1, _, lse1 = ops.decode_core(qg, kg, vg, scale, return_lse=True)
+        torch.cuda.synchronize()
+        assert torch.equal(out0, out1) and torch.equal(lse0, lse1)
+    o_ref, _ = O.sdpa_in_blocks(q, k, v, scale, T - 1, None)
+    check_o(out0.unsqueeze(2), o_ref)
+    torch.testing.assert_close(lse0.cpu(), O.lse2(q, k, scale, T - 1, None), rtol=1e-4, atol=1e-3)
