@@ -632,3 +632,63 @@ def test_decode_without_weights_beside_other_work(gpu, decode_route):
     o_ref, _ = O.sdpa_in_blocks(q, k, v, scale, T - 1, None)
     check_o(out0.unsqueeze(2), o_ref)
     torch.testing.assert_close(lse0.cpu(), O.lse2(q, k, scale, T - 1, None), rtol=1e-4, atol=1e-3)
+
+
+@pytest.mark.parametrize("store", ["bf16", "u8", "u4"])
+@pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D,splits", [
+    (1, 24, 8, 11, 32769, 128, 0),    # 33 rows: two blocks over 8 x 32769 keys, their combination in the same launch
+    (2, 28, 4, 36, 32800, 128, 3),    # 252 rows, more than the launch combines: a launch of its own
+    (1, 16, 8, 128, 32768, 128, 2),   # 256 rows, the most
+    (1, 8, 8, 257, 32768, 128, 2),    # one more: the tiled kernel
+    (2, 10, 2, 26, 65536, 256, 2),    # 130 rows of 256: the tiled kernel
+    (2, 8, 2, 32, 65540, 256, 5),     # 128 rows of 256, the most
+    (1, 16, 4, 10, 65600, 256, 0),    # 40 rows of 256
+])
+def test_score_sums_with_streamed_keys_of_long_rows(gpu, store, B, Hq, Hkv, q_len, T, D, splits):
+    """Several blocks of rows over 256 K keys and more. The oracle takes one KV head of each batch element (its heads do not
+    meet); the others are checked by the sum of their weights."""
+    _check_some_heads(gpu, store, torch.bfloat16, B, Hq, Hkv, q_len, T, D, splits)
+
+
+@pytest.mark.parametrize("store", ["plain", "u8", "u4"])
+@pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D,splits", [
+    (2, 6, 2, 43, 190, 128, 3),       # few rows over few keys
+    (1, 12, 1, 85, 700, 256, 2),
+    (2, 8, 8, 4, 1100, 64, 2),        # streamed keys
+    (2, 24, 8, 10, 1090, 256, 5),
+    (1, 16, 8, 20, 32768, 128, 0),
+    (1, 7, 1, 298, 4500, 64, 0),      # tiles of whole queries
+    (2, 6, 2, 460, 900, 128, 0),
+])
+def test_score_sums_over_float16_stores(gpu, store, B, Hq, Hkv, q_len, T, D, splits):
+    """The three score-sum kernels on float16 rows and on codes that dequantise to them."""
+    _check_some_heads(gpu, store, torch.float16, B, Hq, Hkv, q_len, T, D, splits)
+
+
+def _check_some_heads(gpu, store, dtype, B, Hq, Hkv, q_len, T, D, splits):
+    G = Hq // Hkv
+    gen = torch.Generator(device=gpu).manual_seed(T + q_len)
+    q, k, v = (torch.randn(B, h, n, D, generator=gen, device=gpu).to(dtype) for h, n in ((Hq, q_len), (Hkv, T), (Hkv, T)))
+    quant, kd, vd = None, k, v
+    if store in ("u8", "u4"):
+        codes, state, rows = [], [], []
+        for x in (k, v):
+            qz = RowQuantizer((B, Hkv, T, D), dtype, 8 if store == "u8" else 4, allocate_buffers=True, device=gpu)
+            qz.quantize(0, T, x)
+            codes.append(qz.quant_buffer.view(B, Hkv, T, -1))
+            state += [qz.quant_scales.view(B, Hkv, T), qz.quant_zero_points.view(B, Hkv, T)]
+            rows.append(qz.dequantize(0, T))
+        (kd, vd), (k, v), quant = codes, rows, ops.QuantState(*state)
+    scale, pos = D ** -0.5, T - q_len
+    # every position in a slot of another KV head's order: the newest ones are spread over the row
+    tp = torch.rand(B, Hkv, T, generator=gen, device=gpu).argsort(-1).to(torch.int32)
+    out, w, lse = ops.prefill_core(q, kd, vd, scale, pos, tp, return_weights=True, return_lse=True, output_transposed=False, quant=quant, num_splits=splits)
+    torch.testing.assert_close(w.sum(-1).cpu(), torch.full((B, Hkv), float(q_len)), rtol=5e-5, atol=3e-4)
+    for b in range(B):
+        h = (Hkv - 1 + b) % Hkv
+        one, heads = slice(b, b + 1), slice(G * h, G * h + G)
+        qc, kc, vc, tc = q[one, heads].cpu(), k[one, h : h + 1].cpu(), v[one, h : h + 1].cpu(), tp[one, h : h + 1].cpu()
+        o_ref, w_ref = O.sdpa_in_blocks(qc, kc, vc, scale, pos, tc.to(torch.int64))
+        assert rel_err(out[one, heads].float().cpu(), o_ref.float()) < O_RTOL
+        torch.testing.assert_close(w[one, h : h + 1].cpu(), w_ref, rtol=W_RTOL, atol=1e-6)
+        torch.testing.assert_close(lse[one, :, heads].cpu(), O.lse2(qc, kc, scale, pos, tc), rtol=1e-4, atol=1e-3)

@@ -295,6 +295,27 @@ def test_no_room_for_the_copy(gpu):
     assert _extra_bytes(gpu, lambda: ops.prefill_core(q, *codes, *args, quant=state, num_splits=1))[0] >= _COPY  # room again: the copy
 
 
+def test_an_allocation_for_the_copy_that_fails_all_the_same(gpu):
+    """Memory that the allocator's account shows as free and that it cannot use (here: a graph's own) is found out by asking."""
+    q, codes, state, rows, args = _long_call(gpu)
+    want, _, _ = ops.prefill_core(q, *rows, *args)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        torch.empty(2 * _COPY, dtype=torch.uint8, device=gpu)[:1].add_(1)
+    try:
+        limit = torch.cuda.memory_reserved(gpu) + _COPY // 4
+        torch.cuda.set_per_process_memory_fraction(limit / torch.cuda.get_device_properties(gpu).total_memory, gpu)
+        failed = torch.cuda.memory_stats(gpu)["num_ooms"]
+        out, _, _ = ops.prefill_core(q, *codes, *args, quant=state, num_splits=1)
+        torch.cuda.synchronize()
+        assert torch.cuda.memory_stats(gpu)["num_ooms"] == failed + 1
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, gpu)
+    assert rel_err(out.float(), want.float()) < 1e-2
+
+
 def test_a_long_chunk_over_a_quantised_store_in_a_graph(gpu):
     """Recorded with its copy, replayed between other work: the eager call's results each time."""
     q, codes, state, _, args = _long_call(gpu)
