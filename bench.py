@@ -56,7 +56,7 @@ PEAK_HBM_GBS = 8000.0      # MI355X HBM3E
 TRAFFIC_SOURCE = "committed counter run (profiles/hbm_traffic_fetch_write_size.txt), not measured in this run"
 TRAFFIC_BYTES = {
     "prefill": int((70196.3 * 2.000 + 33283.4) * 1024),    # sdpa_prefill_kernel<128, KVX_KV_BF16>
-    "decode": int((2115128.0 * 2.000 + 37312.0) * 1024),   # decode_split_kernel<128, 4, KVX_KV_BF16>
+    "decode": int((2119320.5 * 2.000 + 37441.1) * 1024),   # decode_split_kernel<128, 4, KVX_KV_BF16>
     "quantize": int((65573.9 * 2.000 + 69632.0) * 1024),   # quantize_rows_kernel<128>
 }
 
@@ -164,15 +164,18 @@ def bench_prefill(args, torch, dev):
     a.o = o_view.data_ptr()
     a.o_stride_b, a.o_stride_h, a.o_stride_t = o_view.stride(0), o_view.stride(1), o_view.stride(2)
     a.lse, a.w = lse.data_ptr(), w.data_ptr()
-    nbytes = lib.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a))
-    ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=dev)
+    # over a quantised store as the Python operators call it: dequantised once per call into the workspace
+    attend, room = (lib.kvx_sdpa_prefill_copying, lib.kvx_sdpa_prefill_copying_workspace_bytes) if u8 else (lib.kvx_sdpa_prefill, lib.kvx_sdpa_prefill_workspace_bytes)
+    ws = torch.empty(max(room(ctypes.byref(a)), lib.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a)), 256), dtype=torch.uint8, device=dev)
     a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+    att = _lib.SdpaArgs.from_buffer_copy(a)  # attention alone, so that events can time the two passes
+    att.w = None
     st = _lib.stream_ptr(dev)
 
     def step(ev=None):
         if ev is not None:
             ev[0].record()
-        _lib.check(lib.kvx_sdpa_prefill(ctypes.byref(a), st))
+        _lib.check(attend(ctypes.byref(att), st))
         if ev is not None:
             ev[1].record()
         _lib.check(lib.kvx_score_sum(ctypes.byref(a), st))
@@ -202,11 +205,10 @@ def bench_prefill(args, torch, dev):
     rows = w.sum(-1).cpu()
     assert torch.allclose(rows, torch.full_like(rows, float(q_len)), rtol=1e-4, atol=5e-2), rows
 
-    # A quantised store, long chunk: what the cache object does instead of dequantising inside the attention
-    # kernels (where every workgroup of 256 rows dequantises the whole store again) is one dequantisation
-    # of the store into a bf16 copy for the attention kernel (the score-sum kernel dequantises each key once
-    # per wavefront anyway and stays on the codes). Timed here on the same inputs.
-    dq_ms = None
+    # A quantised store, long chunk, the other two ways: the cache object's (a bf16 copy in a buffer that its layers share,
+    # for the attention kernel; the score-sum kernel dequantises each key once per wavefront and stays on the codes in every
+    # form) and without a copy (every workgroup of 256 rows dequantises the whole store again). Timed on the same inputs.
+    dq_ms = fused_ms = None
     if u8:
         from keys_values_amd.kvcache.h2o import _dequant_scratch
 
@@ -220,17 +222,25 @@ def bench_prefill(args, torch, dev):
             _, _, lse_c = ops.prefill_core(q, kd, vd, scale, input_pos, None, return_lse=True)
             return ops.score_sum_core(q, k, lse_c, scale, input_pos, None, quant=quant)  # the score-sum pass keeps the codes
 
-        for _ in range(3):
-            w_copy = step_copy()
-        torch.cuda.synchronize()
-        torch.testing.assert_close(w_copy, w, rtol=1e-3, atol=1e-6)
-        d0, d1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        d0.record()
-        for _ in range(10):
-            step_copy()
-        d1.record()
-        torch.cuda.synchronize()
-        dq_ms = d0.elapsed_time(d1) / 10
+        def step_fused():
+            _lib.check(lib.kvx_sdpa_prefill_weights(ctypes.byref(a), st))
+            return w
+
+        w_first = w.clone()
+        ms = []
+        for other in (step_copy, step_fused):
+            for _ in range(3):
+                w_other = other()
+            torch.cuda.synchronize()
+            torch.testing.assert_close(w_other, w_first, rtol=1e-3, atol=1e-6)
+            d0, d1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            d0.record()
+            for _ in range(10):
+                other()
+            d1.record()
+            torch.cuda.synchronize()
+            ms.append(d0.elapsed_time(d1) / 10)
+        dq_ms, fused_ms = ms
 
     # The same chunk through the cache object (keys_values/kvcache/base.py:554-595): write the 1024 new
     # rows into the slots chosen by the step before, attend, score-sum, scores += W, choose the next
@@ -295,7 +305,7 @@ def bench_prefill(args, torch, dev):
         "dtype": "bf16",
         "data": "synthetic" if args.operands == "random" else "synthetic, ALL-ZERO operands (clock probe, not the benchmark)",
         "config": {
-            "workload": (f"BASELINE.json configs[2]: attention + score-sum over the {args.kv} cache (dequantised in the kernels), B1 Hq32 Hkv8 D128 T65536 q1024, seed 2"
+            "workload": (f"BASELINE.json configs[2]: attention + score-sum over the {args.kv} cache (dequantised once per call for the attention kernel, on load in the score-sum kernel), B1 Hq32 Hkv8 D128 T65536 q1024, seed 2"
                          if u8 else
                          "BASELINE.json configs[1]: chunked prefill attention + score-sum, B1 Hq32 Hkv8 D128 T32768 q1024, RoPE theta 1e6, seed 1"),
             "flops_algorithmic": flops_alg,
@@ -306,12 +316,13 @@ def bench_prefill(args, torch, dev):
             "ms_score_sum_kernel": round(ms_score, 4),
             "score_sum_tflops": round(2.0 * B * Hq * q_len * T * D / (ms_score * 1e-3) / 1e12, 2),
             "ms_step_over_dequantised_copy": None if dq_ms is None else round(dq_ms, 4),
+            "ms_step_dequantised_in_kernels": None if fused_ms is None else round(fused_ms, 4),
             "h2o_cache_chunk_ms": None if h2o_ms is None else round(h2o_ms, 4),
             "h2o_cache_chunk_tokens_per_s": None if h2o_ms is None else round(q_len / (h2o_ms * 1e-3), 1),
         },
         "roofline": {
             "bound": "mfma",
-            "kernel": "sdpa_prefill_kernel<128,%s> (+ split merge)" % {"bf16": "KVX_KV_BF16", "uint8": "KVX_KV_U8", "uint4": "KVX_KV_U4"}[args.kv],
+            "kernel": ("dequantize_kv_kernel<128,%s> + " % {"uint8": "KVX_KV_U8", "uint4": "KVX_KV_U4"}[args.kv] if u8 else "") + "sdpa_prefill_kernel<128,KVX_KV_BF16> (+ split merge)",
             "achieved": round(attn_tflops, 2),
             "peak": PEAK_BF16_TFLOPS,
             "unit": "TFLOP/s",
@@ -424,8 +435,8 @@ def bench_decode(args, torch, dev):
     # K + V once (bf16 rows, or codes + 8 bytes of row state), scores read-modify-write
     bytes_alg = 2 * B * Hkv * L * ((D // 2 if u4 else D) + 8 if u8 else 2 * D) + 2 * B * Hkv * L * 4
     gbs = bytes_alg / (ms_step * 1e-3) / 1e9
-    # the dominant launch alone: the fused attention + score update + argmin call (split attention,
-    # tail kernel), events on the launch stream around each call
+    # the dominant launch alone: the fused attention + score update + argmin call (the counters' reset and the split
+    # kernel, whose splits finish the row), events on the launch stream around each call
     launch, _ = cache._decode_h2o_prepare(qs[0], cache.k, cache.v, cache._quant_state(L))
     launch()
     torch.cuda.synchronize()
@@ -458,7 +469,7 @@ def bench_decode(args, torch, dev):
         "config": {"workload": "BASELINE.json configs[3]: decode + H2O eviction, B8 Hq32 Hkv8 D128 T131072, seed 3" + (f", {args.kv} cache" if u8 else ""),
                    "bytes_algorithmic_per_step": bytes_alg, "ms_per_step_gpu_events": round(ms_gpu, 4),
                    "decode_tokens_per_s": round(B / (ms_step * 1e-3), 1)},
-        "roofline": {"bound": "hbm", "kernel": "kvx_sdpa_decode_h2o: decode_split_kernel<128,4,%s> + tail (merge, scratch-route weights, slot publishing)" % {"bf16": "KVX_KV_BF16", "uint8": "KVX_KV_U8", "uint4": "KVX_KV_U4"}[args.kv],
+        "roofline": {"bound": "hbm", "kernel": "kvx_sdpa_decode_h2o: %s" % {"bf16": "decode_split_kernel<128,4,KVX_KV_BF16>", "uint8": "decode_mfma_kernel<128,4,KVX_KV_U8>", "uint4": "decode_mfma_kernel<128,4,KVX_KV_U4>"}[args.kv],
                      "achieved": round(bytes_alg / (ms_call * 1e-3) / 1e9, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": round(bytes_alg / (ms_call * 1e-3) / 1e9 / PEAK_HBM_GBS, 4), "ms_per_launch": round(ms_call, 4),
                      "traffic": None if u8 else TRAFFIC_BYTES["decode"], "traffic_source": None if u8 else TRAFFIC_SOURCE},
