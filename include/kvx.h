@@ -98,7 +98,7 @@ typedef struct kvx_sdpa_args {
   void* workspace;     /* scratch, kvx_sdpa_*_workspace_bytes(); may be NULL when that returns 0 */
   size_t workspace_bytes;
 
-  /* kvx_sdpa_decode / kvx_sdpa_decode_h2o with score-sums only, optional (NULL: not wanted): one device uint32 that the
+  /* the single-token calls with score-sums only, optional (NULL: not wanted): one device uint32 that the
    * call sets to the number of (batch, KV head, split) workgroups whose logits went through the fp32 scratch in HBM
    * instead of staying on the chip -- all of them when the splits are too long for the LDS or that form is switched
    * off, else those whose bounded wait for their row ran out (normally 0; such a call is about 15 % slower). */

@@ -14,9 +14,10 @@ The K/V store is either bf16 (``h2o-default``) or codes with per-row scale / zer
 (``h2o-torch-quantized8``) or 4 bits, two codes per byte (``h2o-torch-quantized4``;
 keys_values/kvcache/factory.py:50-66). In the second case the codes stay resident and are never
 written back: single tokens and short chunks are attended to by kernels that dequantise on load; for a
-long chunk (``dequantize_chunk_rows`` query rows or more) the store is dequantised once into a bf16
-buffer shared by all caches of a device and stream, because every workgroup of the attention kernels
-would otherwise dequantise the whole store again. The reference dequantises the whole cache into a
+long chunk (``dequantize_chunk_rows`` query rows or more, tokens x heads per KV head) the store is dequantised once into a
+16-bit buffer shared by all caches of a device and stream, because every workgroup of the attention kernels
+would otherwise dequantise the whole store again. With that threshold left at its default, chunks from 1025 rows on may
+take a copy for the time of the call as well; ``None`` switches both off. The reference dequantises the whole cache into a
 bf16 working buffer per layer and re-quantises it afterwards
 (keys_values/kvcache/quant_buffers.py:473-503,732-804).
 
