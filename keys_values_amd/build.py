@@ -15,7 +15,8 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libkvx.so")
 HOST = os.path.join(HERE, "_host.so")
-SOURCES = ["kvx_api.hip", "sdpa_prefill.hip", "score_sum.hip", "sdpa_decode.hip", "quantize.hip", "h2o.hip", "norm_rope.hip"]
+SOURCES = ["sdpa_decode_128.hip", "sdpa_decode_64.hip", "sdpa_decode_256.hip", "score_sum.hip", "sdpa_prefill.hip", "quantize.hip", "h2o.hip", "kvx_api.hip",
+           "sdpa_decode.hip", "norm_rope.hip"]  # the longest first
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [

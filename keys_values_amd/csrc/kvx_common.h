@@ -65,12 +65,14 @@ int launch_dequantize_rows(const uint8_t* codes, const float* scale, const int32
 int launch_dequantize_kv(const kvx_sdpa_args& a, void* out, hipStream_t st);
 int launch_quantize_blocks(const kvx_block_quant_args& a, hipStream_t st);
 int launch_dequantize_blocks(const kvx_block_quant_args& a, hipStream_t st);
-// Counters that a single-token step needs at zero when its split kernel starts: kDecodeCounters 32-bit words at the head
-// of a line of kDecodeCounterStride words per (batch, KV head) row, and the caller's count of scratch splits (or NULL).
+// What a single-token step needs at zero when its split kernel starts: kDecodeCounters 32-bit words at the head of a line of
+// kDecodeCounterStride words per (batch, KV head) row, the caller's count of scratch splits (or NULL), and the splits' pairs.
 constexpr int kDecodeCounterStride = 64, kDecodeCounters = 3;
 struct DecodeCounters {
   uint32_t* rows;
   uint32_t* scratch_splits;
+  unsigned long long* pair;
+  int64_t pairs;
 };
 // `clear`: counters the launch also sets to zero (a step of its own would cost as much as the write), or NULL
 int launch_cache_write(const kvx_cache_write_args& a, const DecodeCounters* clear, hipStream_t st);
@@ -95,6 +97,13 @@ int launch_qk_norm_rope(void* qkv, int64_t sb, int64_t stt, int B, int num, int 
 
 // Number of compute units of the current device (cached).
 int num_cus();
+
+// by `lanes` lanes, at least as many as rows
+__device__ __forceinline__ void clear_counters(const DecodeCounters& c, int64_t lane, int64_t lanes, int64_t rows) {
+  if (c.rows && lane < rows)
+    for (int i = 0; i < kDecodeCounters; ++i) c.rows[lane * kDecodeCounterStride + i] = 0u;
+  for (int64_t i = lane; i < c.pairs; i += lanes) c.pair[i] = 0ull;
+}
 
 // ---- device helpers ------------------------------------------------------------------------
 

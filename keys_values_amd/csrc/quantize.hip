@@ -569,8 +569,7 @@ __global__ __launch_bounds__(NTHREADS) void cache_write_kernel(const kvx_cache_w
   constexpr int LPR = D / 8;
   const int64_t gid = (int64_t)blockIdx.x * NTHREADS + threadIdx.x;
   if (clear.rows) {  // one line per (batch, KV head) row: there are at least as many lanes (LPR of them a job)
-    if (gid < (int64_t)a.B * a.Hkv)
-      for (int c = 0; c < kDecodeCounters; ++c) clear.rows[gid * kDecodeCounterStride + c] = 0u;
+    clear_counters(clear, gid, (int64_t)gridDim.x * NTHREADS, (int64_t)a.B * a.Hkv);
     if (gid == 0 && clear.scratch_splits) *clear.scratch_splits = 0u;
   }
   const int col = (int)(gid % LPR);
@@ -802,7 +801,7 @@ int launch_cache_write_d(const kvx_cache_write_args& a, const DecodeCounters& cl
 }
 
 int launch_cache_write(const kvx_cache_write_args& a, const DecodeCounters* clear, hipStream_t st) {
-  const DecodeCounters none{nullptr, nullptr}, &c = clear ? *clear : none;
+  const DecodeCounters none{}, &c = clear ? *clear : none;
   const int64_t total = (int64_t)a.B * a.Hkv * a.num * (a.D / 8);
   if (total == 0) return KVX_OK;
   const unsigned grid = (unsigned)((total + NTHREADS - 1) / NTHREADS);
