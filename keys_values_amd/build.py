@@ -15,7 +15,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libkvx.so")
 HOST = os.path.join(HERE, "_host.so")
-SOURCES = ["sdpa_decode_128.hip", "sdpa_decode_64.hip", "sdpa_decode_256.hip", "score_sum.hip", "sdpa_prefill.hip", "quantize.hip", "h2o.hip", "kvx_api.hip",
+SOURCES = ["sdpa_decode_128.hip", "sdpa_decode_64.hip", "sdpa_decode_256.hip", "score_sum.hip", "sdpa_prefill.hip", "sdpa_rows.hip", "quantize.hip", "h2o.hip", "kvx_api.hip",
            "sdpa_decode.hip", "norm_rope.hip"]  # the longest first
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -188,6 +188,12 @@ __device__ __forceinline__ float sum_halves(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// max with the 16-lane row beside (v_permlane16_swap), in every lane
+__device__ __forceinline__ float max_row_pairs(float v) {
+  const u32pair_t r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 // The affine 8-bit row quantiser, one element. `inv` = 1.0f / scale, `zf` = (float) zero point.
 // rint before the add, so the multiply can never fuse with it.
 // `qmax` = 255 (8-bit) or 15 (4-bit codes).

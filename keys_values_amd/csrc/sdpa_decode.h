@@ -32,7 +32,7 @@
 #pragma once
 #include <type_traits>
 
-#include "kvx_common.h"
+#include "key_blocks.h"
 
 namespace kvx {
 namespace decode {
@@ -114,10 +114,6 @@ __device__ __forceinline__ float swap_rows_add(float a, float b) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 __device__ __forceinline__ float sum_row_pairs(float v) { return swap_rows_add(v, v); }
-__device__ __forceinline__ float max_row_pairs(float v) {
-  const u32pair_t r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
 // lower half: sum of a over the two halves, upper half: sum of b
 __device__ __forceinline__ float swap_halves_add(float a, float b) {
   const u32pair_t r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
@@ -913,39 +909,18 @@ __global__ __launch_bounds__(NTHREADS) void decode_split_kernel(const DecodePara
 //
 // For quantised stores and for more than four query heads per KV head the kernel above is bound by its vector
 // arithmetic (G dot products per loaded pair of values on top of the dequantisation), not by HBM. Here the G heads are
-// padded to the 16 columns of v_mfma_f32_16x16x32: S^T = K Q^T per 16 keys (the lane that holds key m of the tile
-// loads 8 consecutive d of that row per matrix instruction: the row as it lies in memory is the A operand), then
-// O^T += V^T P^T per 32 keys. The accumulator layout of S^T (lane = (head, keys 4 kg .. 4 kg + 3)) becomes the B
-// operand of the second product without any exchange once the 32 keys of a block are taken in the order (tile 0:
-// 4 kg .. 4 kg + 3, tile 1: 4 kg .. 4 kg + 3) per lane group kg; V^T is gathered to match: a lane loads, from each of
-// its 8 keys, the D / 16 values of its d rows and regroups them (one byte permute per pair of bf16 values; for codes
-// the regrouping is part of the dequantisation). What is left for the vector ALU is the dequantisation (3.5
+// padded to the 16 columns of v_mfma_f32_16x16x32 and the rows are operands as they come from memory (key_blocks.h).
+// What is left for the vector ALU is the dequantisation (3.5
 // instructions per element, as the reference rounds) or half an instruction per V element, and the softmax of 16
 // head columns per key. The running maximum is one per head (the four lane groups of a head column agree on it), it
 // moves lazily as above. Everything after the key loop is shared with the kernel above.
-template <bool F16>
-__device__ __forceinline__ f32x4_t mfma_16x16x32(u32x4_t a, u32x4_t b, f32x4_t c) {
-  if constexpr (F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-  else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-}
-
-// elem( (float)((int)code - zp) * scale ) for two codes with their own row state (two keys)
-template <bool F16>
-__device__ __forceinline__ uint32_t dequant_pair2(uint32_t c0, int32_t zp0, float sc0, uint32_t c1, int32_t zp1, float sc1) {
-  return pack_pair<F16>((float)((int32_t)c0 - zp0) * sc0, (float)((int32_t)c1 - zp1) * sc1);
-}
-
 template <int D, int G, int KV, bool VARIANT>
 __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel(const DecodeParams p, const kvx_h2o_args hh) {
   constexpr bool F16 = kv_elem_f16(KV);
   constexpr bool U8 = !kv_is_plain(KV);  // codes + row state (8-bit or 4-bit store)
-  constexpr bool U4 = kv_is_u4(KV);
-  constexpr int KJ = D / 32;   // matrix instructions of the first product per 16-key tile
-  constexpr int DPL = D / 16;  // d rows per lane = matrix instructions of the second product per 32-key block
-  constexpr int CH = 32;       // keys per wavefront and step
-  constexpr int NL4 = D >= 128 ? D / 128 : 1;                              // 4-bit rows: 16-byte loads per key of K
-  constexpr int KR = U4 ? NL4 : (U8 ? D / 64 : KJ);                        // 16-byte loads per key of K
-  constexpr int VW = U4 ? (DPL + 7) / 8 : (U8 ? (DPL + 3) / 4 : DPL / 2);  // dwords per key of V
+  using Blocks = KeyBlocks<D, KV, true>;
+  using Rows = typename Blocks::Rows;
+  constexpr int KJ = Blocks::KJ, DPL = Blocks::DPL, CH = Blocks::CH;
   constexpr int LGK = logit_floats(G, D, U8) / G;
   __shared__ __align__(16) float lgbuf[LGK * G];  // [key][head]
   __shared__ __align__(16) float red[WAVES][G][D];
@@ -960,36 +935,15 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
   const int k_begin = split * p.keys_per_split;
   const int k_end = min(k_begin + p.keys_per_split, p.kv_len);
 
-  // first d of the 8 this lane group supplies to matrix instruction e of the first product
-  auto kslice = [&](int e) -> int {
-    if constexpr (!U8) return 8 * (kg + 4 * e);
-    else if constexpr (U4 && D == 64) return 8 * kg + 32 * e;
-    else if constexpr (U4) return 16 * kg + 8 * (e & 1) + 64 * ((e >> 1) % NL4) + (D / 2) * (e / (2 * NL4));
-    else return 16 * kg + 8 * (e & 1) + 64 * (e >> 1);
-  };
-  // d of row `mrow` of matrix instruction t of the second product
-  auto dmap = [&](int t, int mrow) -> int {
-    if constexpr (U4) return t < DPL / 2 ? (DPL / 2) * mrow + t : D / 2 + (DPL / 2) * mrow + (t - DPL / 2);
-    else return DPL * mrow + t;
-  };
-
   u32x4_t qb[KJ];  // B operands of the first product: head m (zero beyond the group), d slice of lane group kg
 #pragma unroll
   for (int e = 0; e < KJ; ++e) {
     qb[e] = u32x4_t{0u, 0u, 0u, 0u};
-    if (m < p.Gr) qb[e] = *(const u32x4_t*)(p.q + b * p.q_sb + (int64_t)(kvh * p.Gr + m) * p.q_sh + kslice(e));
+    if (m < p.Gr) qb[e] = *(const u32x4_t*)(p.q + b * p.q_sb + (int64_t)(kvh * p.Gr + m) * p.q_sh + Blocks::kslice(e, kg));
   }
-  constexpr int ES = U8 ? 1 : 2;
-  const uint8_t* kbase = (const uint8_t*)p.k + (b * p.k_sb + kvh * p.k_sh) * ES;
-  const uint8_t* vbase = (const uint8_t*)p.v + (b * p.v_sb + kvh * p.v_sh) * ES;
-  const uint32_t k_rowb = (uint32_t)p.k_st * ES, v_rowb = (uint32_t)p.v_st * ES;
-  const uint32_t k_lane = (U4 && D == 64) ? 8 * kg : 16 * kg;              // + 64 r for the r-th load of the row
-  const uint32_t v_lane = (uint32_t)m * (U4 ? DPL / 2 : (U8 ? DPL : 2 * DPL));
-  const int64_t qs_off = b * p.qs_sb + kvh * p.qs_sh;
-  const char* ksb = (const char*)(p.k_scale + qs_off);
-  const char* kzb = (const char*)(p.k_zp + qs_off);
-  const char* vsb = (const char*)(p.v_scale + qs_off);
-  const char* vzb = (const char*)(p.v_zp + qs_off);
+  Blocks blocks;
+  blocks.init(p.k, p.v, p.k_scale, p.k_zp, p.v_scale, p.v_zp, b * p.k_sb + kvh * p.k_sh, b * p.v_sb + kvh * p.v_sh, b * p.qs_sb + kvh * p.qs_sh, p.k_st, p.v_st,
+              p.qs_vec, m, kg, k_end);
   float* lgrow = p.logits ? p.logits + ((int64_t)b * p.Hkv + kvh) * p.Tpad * G : nullptr;
   int lg_base = k_begin;
 
@@ -998,147 +952,13 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
   for (int t = 0; t < DPL; ++t) acc[t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
   float m_run = kNegBig, l_run = 0.0f;
 
-  struct Rows {
-    u32x4_t k[2][KR];
-    float ks[2];
-    int32_t kz[2];
-    uint32_t v[8][VW];
-    float vs[8];
-    int32_t vz[8];
-  };
-  // Byte offsets of this lane's rows in the block at `chunk0`: K rows chunk0 + m and chunk0 + 16 + m, V rows
-  // chunk0 + 4 kg (+ 0..3, + 16..19). A full block addresses them from two per-lane offsets that advance with the
-  // block and multiples of the row stride; a block that reaches past the end clamps every key to the last valid row
-  // (its logits become -inf below).
-  const uint32_t k16 = 16u * k_rowb, v16 = 16u * v_rowb;
-  auto load_k = [&](Rows& r, int gi, uint32_t off, int key) {
-    const uint8_t* row = kbase + off;
-#pragma unroll
-    for (int x = 0; x < KR; ++x) {
-      if constexpr (U4 && D == 64) {
-        const u32x2_t c = __builtin_nontemporal_load((const u32x2_t*)row);
-        r.k[gi][x] = u32x4_t{c[0], c[1], 0u, 0u};
-      } else {
-        r.k[gi][x] = __builtin_nontemporal_load((const u32x4_t*)(row + 64 * x));
-      }
-    }
-    if constexpr (U8) {  // uniform base + 32-bit offset
-      r.ks[gi] = *(const float*)(ksb + (uint32_t)key * 4u);
-      r.kz[gi] = *(const int32_t*)(kzb + (uint32_t)key * 4u);
-    }
-  };
-  auto load_v = [&](Rows& r, int j, uint32_t off) {
-    const uint8_t* row = vbase + off;
-    constexpr int BYTES = U4 ? DPL / 2 : (U8 ? DPL : 2 * DPL);  // this lane's share of the row
-    if constexpr (BYTES == 16) {
-      const u32x4_t x = __builtin_nontemporal_load((const u32x4_t*)row);
-      r.v[j][0] = x[0]; r.v[j][1] = x[1]; r.v[j][2] = x[2]; r.v[j][3] = x[3];
-    } else if constexpr (BYTES == 8) {
-      const u32x2_t x = __builtin_nontemporal_load((const u32x2_t*)row);
-      r.v[j][0] = x[0]; r.v[j][1] = x[1];
-    } else if constexpr (BYTES == 4) {
-      r.v[j][0] = __builtin_nontemporal_load((const uint32_t*)row);
-    } else {
-      static_assert(BYTES == 2, "4-bit rows of 64 values");
-      r.v[j][0] = (uint32_t)__builtin_nontemporal_load((const uint16_t*)row);
-    }
-  };
-  auto issue = [&](Rows& r, int chunk0) {
-    if (chunk0 + CH <= k_end) {
-      const uint32_t ko = (uint32_t)(chunk0 + m) * k_rowb + k_lane;
-      load_k(r, 0, ko, chunk0 + m);
-      load_k(r, 1, ko + k16, chunk0 + 16 + m);
-      const int q0 = chunk0 + 4 * kg;
-      if constexpr (U8) {
-        if (p.qs_vec) {  // the four keys of a tile this lane group owns are neighbours: one 16-byte load each
-#pragma unroll
-          for (int gi = 0; gi < 2; ++gi) {
-            const f32x4_t sc = *(const f32x4_t*)(vsb + (uint32_t)(q0 + 16 * gi) * 4u);
-            const int4 zp = *(const int4*)(vzb + (uint32_t)(q0 + 16 * gi) * 4u);
-            r.vs[4 * gi] = sc[0]; r.vs[4 * gi + 1] = sc[1]; r.vs[4 * gi + 2] = sc[2]; r.vs[4 * gi + 3] = sc[3];
-            r.vz[4 * gi] = zp.x; r.vz[4 * gi + 1] = zp.y; r.vz[4 * gi + 2] = zp.z; r.vz[4 * gi + 3] = zp.w;
-          }
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            r.vs[j] = *(const float*)(vsb + (uint32_t)(q0 + 16 * (j >> 2) + (j & 3)) * 4u);
-            r.vz[j] = *(const int32_t*)(vzb + (uint32_t)(q0 + 16 * (j >> 2) + (j & 3)) * 4u);
-          }
-        }
-      }
-      const uint32_t vo = (uint32_t)q0 * v_rowb + v_lane;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) load_v(r, j, vo + (uint32_t)(j & 3) * v_rowb + (j >> 2) * v16);
-    } else {
-#pragma unroll
-      for (int gi = 0; gi < 2; ++gi) {
-        const int key = min(chunk0 + 16 * gi + m, k_end - 1);
-        load_k(r, gi, (uint32_t)key * k_rowb + k_lane, key);
-      }
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int key = min(chunk0 + 16 * (j >> 2) + 4 * kg + (j & 3), k_end - 1);
-        if constexpr (U8) {
-          r.vs[j] = *(const float*)(vsb + (uint32_t)key * 4u);
-          r.vz[j] = *(const int32_t*)(vzb + (uint32_t)key * 4u);
-        }
-        load_v(r, j, (uint32_t)key * v_rowb + v_lane);
-      }
-    }
-  };
-  // A operand e of the first product for tile gi
-  auto k_operand = [&](const Rows& r, int gi, int e) -> u32x4_t {
-    if constexpr (!U8) {
-      return r.k[gi][e];
-    } else if constexpr (!U4) {
-      const u32x4_t w = r.k[gi][e >> 1];
-      return (e & 1) ? dequant_words<F16>(w[2], w[3], r.kz[gi], r.ks[gi]) : dequant_words<F16>(w[0], w[1], r.kz[gi], r.ks[gi]);
-    } else {
-      const u32x4_t w = r.k[gi][D >= 128 ? (e >> 1) % NL4 : 0];
-      u32x2_t bytes;
-      int shift;
-      if constexpr (D >= 128) {
-        bytes = (e & 1) ? u32x2_t{w[2], w[3]} : u32x2_t{w[0], w[1]};
-        shift = (e / (2 * NL4)) ? 0 : 4;
-      } else {
-        bytes = u32x2_t{w[0], w[1]};
-        shift = e ? 0 : 4;
-      }
-      const u32x2_t c = u4_codes(bytes, shift);
-      return dequant_words<F16>(c[0], c[1], r.kz[gi], r.ks[gi]);
-    }
-  };
-  // A operand t of the second product: value t of each of this lane's 8 keys, in key order
-  auto v_operand = [&](const Rows& r, int t) -> u32x4_t {
-    u32x4_t a;
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int j0 = 2 * jj, j1 = 2 * jj + 1;
-      if constexpr (!U8) {
-        a[jj] = __builtin_amdgcn_perm(r.v[j1][t >> 1], r.v[j0][t >> 1], (t & 1) ? 0x07060302u : 0x05040100u);
-      } else {
-        uint32_t c0, c1;
-        if constexpr (!U4) {
-          c0 = (r.v[j0][t >> 2] >> (8 * (t & 3))) & 0xffu;
-          c1 = (r.v[j1][t >> 2] >> (8 * (t & 3))) & 0xffu;
-        } else {
-          const int tb = t < DPL / 2 ? t : t - DPL / 2;  // byte of this lane's share; first half of the row: high nibble
-          const int sh = 8 * (tb & 3) + (t < DPL / 2 ? 4 : 0);
-          c0 = (r.v[j0][tb >> 2] >> sh) & 0xfu;
-          c1 = (r.v[j1][tb >> 2] >> sh) & 0xfu;
-        }
-        a[jj] = dequant_pair2<F16>(c0, r.vz[j0], r.vs[j0], c1, r.vz[j1], r.vs[j1]);
-      }
-    }
-    return a;
-  };
   auto consume = [&](Rows& r, int chunk0) {
     f32x4_t s[2];
 #pragma unroll
     for (int gi = 0; gi < 2; ++gi) {
       s[gi] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int e = 0; e < KJ; ++e) s[gi] = mfma_16x16x32<F16>(k_operand(r, gi, e), qb[e], s[gi]);
+      for (int e = 0; e < KJ; ++e) s[gi] = mfma_16x16x32<F16>(Blocks::k_operand(r, gi, e), qb[e], s[gi]);
     }
     // this lane: head m, keys chunk0 + 16 gi + 4 kg + i (log2 units)
     float sv[8];
@@ -1181,7 +1001,7 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
     }
     const u32x4_t pb = {pack_pair<F16>(pv[0], pv[1]), pack_pair<F16>(pv[2], pv[3]), pack_pair<F16>(pv[4], pv[5]), pack_pair<F16>(pv[6], pv[7])};
 #pragma unroll
-    for (int t = 0; t < DPL; ++t) acc[t] = mfma_16x16x32<F16>(v_operand(r, t), pb, acc[t]);
+    for (int t = 0; t < DPL; ++t) acc[t] = mfma_16x16x32<F16>(Blocks::v_operand(r, t), pb, acc[t]);
   };
 
   // Two steps in flight per wavefront: the loads of step i + 1 are issued before step i is consumed.
@@ -1191,14 +1011,14 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
   constexpr int FLUSH_STEPS = LGK / (CH * WAVES);
   static_assert(LGK % (CH * WAVES) == 0 && FLUSH_STEPS >= 2 && FLUSH_STEPS % 2 == 0, "the loop below advances two steps at a time");
   Rows ra, rb;
-  issue(ra, chunk);
+  blocks.issue(ra, chunk);
   const RowAt at = row_at<D>(p, hh, b, kvh);
   for (int i = 0; i + 1 < nsteps; i += 2) {
-    issue(rb, chunk + stride);
+    blocks.issue(rb, chunk + stride);
     __builtin_amdgcn_sched_barrier(0);
     consume(ra, chunk);
     __builtin_amdgcn_sched_barrier(0);  // the loads below reuse the registers consumed above
-    issue(ra, chunk + 2 * stride);
+    blocks.issue(ra, chunk + 2 * stride);
     __builtin_amdgcn_sched_barrier(0);
     consume(rb, chunk + stride);
     __builtin_amdgcn_sched_barrier(0);
@@ -1228,7 +1048,7 @@ __global__ __launch_bounds__(NTHREADS, D <= 128 ? 2 : 1) void decode_mfma_kernel
 #pragma unroll
     for (int t = 0; t < DPL; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) red[wave][m][dmap(t, 4 * kg + i)] = acc[t][i];
+      for (int i = 0; i < 4; ++i) red[wave][m][Blocks::dmap(t, 4 * kg + i)] = acc[t][i];
     if (kg == 0) {
       rml[wave][m][0] = m_run;
       rml[wave][m][1] = l;

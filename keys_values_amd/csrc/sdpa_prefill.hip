@@ -25,7 +25,7 @@
 #include <type_traits>
 #include <utility>
 
-#include "prefill_merge.h"
+#include "prefill_params.h"
 
 namespace kvx {
 namespace {
@@ -37,27 +37,6 @@ constexpr float kSlackLog2 = 8.0f;  // see the running-maximum update in the ker
 // two sizes run alike and the smaller one leaves more workgroups for short chunks. At head size 256 the
 // output accumulators (128 registers) leave no room for two wavefronts per SIMD: four for every store.
 constexpr int nwaves(int kv, int D) { return (kv_is_plain(kv) || D > 128) ? 4 : 8; }  // kv: enum kvx_kv_dtype
-constexpr int BN = 64;   // keys per tile
-
-struct PrefillParams {
-  const uint16_t* q;
-  const void* k;
-  const void* v;
-  const float* k_scale;
-  const int32_t* k_zp;
-  const float* v_scale;
-  const int32_t* v_zp;
-  const int32_t* tp;
-  uint16_t* o;
-  float* lse;
-  float* part_o;   // [split][group][R][D] fp32, unnormalised
-  float* part_ml;  // [split][group][R][2]  (max in log2 units, sum)
-  int32_t B, Hq, Hkv, G, q_len, kv_len, R, input_pos;
-  int32_t num_splits, tiles_per_split, num_tiles, m_blocks;
-  float c;  // sm_scale * log2(e)
-  int64_t q_sb, q_sh, q_st, k_sb, k_sh, k_st, v_sb, v_sh, v_st, o_sb, o_sh, o_st;
-  int64_t qs_sb, qs_sh, tp_sb, tp_sh;
-};
 
 // K and V tiles in LDS: [key][16-byte chunk], rows unpadded (D * 2 bytes), chunk c of row r stored at
 // position c ^ key(r). Unpadded rows are what the global -> LDS DMA writes (a wavefront fills 1024
@@ -619,7 +598,6 @@ __global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(const MergePara
 // the rule avoids: 2 x 4 heads, 333 queries x 7, 5001 keys: 4 splits (608 workgroups, three to a unit) 83 us, 3 splits
 // (456, two) 63 us, 5 splits (760, three) 73 us; 4 x 4 heads, 541 x 7 over 5238: 2 splits 177, none 152.
 int pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
-  if (a.num_splits > 0) return min(a.num_splits, num_tiles);
   const int64_t base = (int64_t)a.B * a.Hkv * m_blocks, cus = num_cus();
   const bool plain = kv_is_plain(a.kv_dtype);
   int64_t tile_ns = a.D == 64 ? 700 : a.D == 128 ? 1130 : 2050;
@@ -663,9 +641,11 @@ void fill_params(PrefillParams& p, const kvx_sdpa_args& a) {
   p.R = a.q_len * p.G;
   p.input_pos = a.input_pos;
   p.num_tiles = (a.kv_len + BN - 1) / BN;
-  const int bm = 32 * nwaves(a.kv_dtype, a.D);
+  const RowsPlan rows = rows_plan(a);
+  p.columns = rows.columns;
+  const int bm = p.columns ? p.columns : 32 * nwaves(a.kv_dtype, a.D);
   p.m_blocks = (p.R + bm - 1) / bm;
-  p.num_splits = pick_splits(a, p.m_blocks, p.num_tiles);
+  p.num_splits = a.num_splits > 0 ? min(a.num_splits, p.num_tiles) : p.columns ? rows.splits : pick_splits(a, p.m_blocks, p.num_tiles);
   p.tiles_per_split = (p.num_tiles + p.num_splits - 1) / p.num_splits;
   p.num_splits = (p.num_tiles + p.tiles_per_split - 1) / p.tiles_per_split;
   p.c = a.sm_scale * kLog2e;
@@ -675,6 +655,8 @@ void fill_params(PrefillParams& p, const kvx_sdpa_args& a) {
   p.o_sb = a.o_stride_b; p.o_sh = a.o_stride_h; p.o_st = a.o_stride_t;
   p.qs_sb = a.qs_stride_b; p.qs_sh = a.qs_stride_h;
   p.tp_sb = a.tp_stride_b; p.tp_sh = a.tp_stride_h;
+  p.qs_vec = (((uintptr_t)a.k_scale | (uintptr_t)a.k_zp | (uintptr_t)a.v_scale | (uintptr_t)a.v_zp) & 15) == 0 && a.qs_stride_b % 4 == 0 && a.qs_stride_h % 4 == 0;
+  p.tp_vec = ((uintptr_t)a.token_positions & 15) == 0 && a.tp_stride_b % 4 == 0 && a.tp_stride_h % 4 == 0;
   p.part_o = nullptr;
   p.part_ml = nullptr;
 }
@@ -688,9 +670,14 @@ size_t partial_bytes(const PrefillParams& p, int D) {
 // `rest`: where the partials are left for another launch to combine, their description (num_splits 1: nothing to combine)
 template <int D, int KV>
 int launch_t(PrefillParams& p, hipStream_t st, MergeParams* rest) {
-  dim3 grid(p.B * p.Hkv, p.m_blocks, p.num_splits);
-  hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
-  KVX_HIP(hipGetLastError());
+  if (p.columns) {
+    const int rc = launch_sdpa_rows(p, D, KV, st);
+    if (rc != KVX_OK) return rc;
+  } else {
+    dim3 grid(p.B * p.Hkv, p.m_blocks, p.num_splits);
+    hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
+    KVX_HIP(hipGetLastError());
+  }
   const MergeParams m = {p.part_o, p.part_ml, p.o, p.lse, p.B, p.Hq, p.Hkv, p.G, p.q_len, p.R, p.num_splits, p.o_sb, p.o_sh, p.o_st};
   if (rest) {
     *rest = m;

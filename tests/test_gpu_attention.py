@@ -177,6 +177,53 @@ def test_score_sums_with_streamed_keys(gpu, store, B, Hq, Hkv, q_len, T, D, spli
     test_score_sums_of_few_rows_over_few_keys(gpu, store, B, Hq, Hkv, q_len, T, D, splits)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("store", ["plain", "u8", "u4"])
+@pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D,splits", [
+    (1, 1, 1, 2, 2, 128, 0),         # two rows and keys
+    (2, 4, 2, 8, 31, 64, 0),         # a full tile of 16 rows, a key short of a block
+    (1, 17, 1, 2, 129, 128, 0),      # 34 rows, one key beyond a round of the four wavefronts
+    (1, 3, 1, 11, 385, 256, 2),      # 33 rows; codes: 256 columns of V over two tiles of rows
+    (1, 6, 2, 43, 1535, 64, 0),      # 129 rows of 3 heads, the last block short
+    (3, 8, 8, 5, 4097, 128, 0),      # 5 rows, many splits, the last one of a single key
+    (1, 8, 2, 4, 700, 128, 11),      # a split a tile
+    (2, 16, 2, 16, 640, 256, 0),     # 128 rows of 256, the most over codes
+    (1, 32, 8, 75, 1000, 128, 0),    # 300 rows in splits
+    (1, 8, 2, 384, 640, 128, 0),     # 1536 rows, as many as keys of them are new: most blocks are masked
+    (2, 16, 4, 260, 640, 128, 0),    # 1040 rows, above the line in every store: the tiled kernel
+])
+def test_attention_of_few_rows(gpu, dtype, store, B, Hq, Hkv, q_len, T, D, splits):
+    # dense, offset and scattered positions; rows, positions and row state on 4-element bounds and off them
+    # tolerances of the path
+    q, k, v, gen = make_qkv(510 + T, B, Hq, Hkv, q_len, T, D, dtype=dtype)
+    state = None
+    if store != "plain":
+        bits = 8 if store == "u8" else 4
+        (kc, ks, kz), (vc, vs, vz) = (O.quantize_rows(x.reshape(-1, D), bits) for x in (k, v))
+        k, v = (O.dequantize_rows(*t, dtype).view(B, Hkv, T, D) for t in ((kc, ks, kz), (vc, vs, vz)))
+        if bits == 4:
+            kc, vc = O.compress4(kc), O.compress4(vc)
+        kd, vd = kc.view(B, Hkv, T, -1), vc.view(B, Hkv, T, -1)
+        state = [t.view(B, Hkv, T) for t in (ks, kz, vs, vz)]
+    else:
+        kd, vd = k, v
+    scale = 1.0 / math.sqrt(D)
+
+    def shifted(x, by):
+        """``x`` on the device in a buffer whose rows are 3 longer and begin ``by`` in"""
+        buf = torch.zeros(B, Hkv, T + 3, *x.shape[3:], dtype=x.dtype, device=gpu)
+        buf[:, :, by : by + T] = x.to(gpu)
+        return buf[:, :, by : by + T]
+
+    for pos, tp, by in ((T - q_len, None, 0), (2 * T, scattered_positions(gen, B, Hkv, T, 2 * T, q_len), 0), (T, scattered_positions(gen, B, Hkv, T, T, q_len), 1)):
+        move = (lambda x: x.to(gpu)) if by == 0 else (lambda x: shifted(x, by))
+        o_ref, _ = O.sdpa_in_blocks(q, k, v, scale, pos, None if tp is None else tp.to(torch.int64))
+        out, _, lse = ops.prefill_core(q.to(gpu), move(kd), move(vd), scale, pos, None if tp is None else move(tp), return_lse=True, output_transposed=False,
+                                       quant=None if state is None else ops.QuantState(*(move(t) for t in state)), num_splits=splits)
+        check_o(out, o_ref)
+        torch.testing.assert_close(lse.cpu(), O.lse2(q, k, scale, pos, tp), rtol=1e-4, atol=1e-3)
+
+
 @pytest.mark.parametrize("scattered", [False, True])
 @pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D", [
     (1, 7, 1, 297, 600, 128),    # 2079 rows: 33 tiles of 63, all full
