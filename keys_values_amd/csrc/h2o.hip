@@ -8,7 +8,7 @@
 //   k == 1 (single-token decode): a streaming pass over all rows with many workgroups; each folds
 //          its slice into one 64-bit key (ordered value bits << 32 | slot) and publishes it with
 //          an integer atomicMin, which is order independent and therefore deterministic.
-//   k  > 1 (chunked prefill): a row is spread over workgroups of 1024 slots. The first launch adds the weights
+//   k  > 1 (chunked prefill): a row is spread over workgroups of 256 or 1024 slots. The first launch adds the weights
 //          and sorts every workgroup's 64-bit (value, slot) keys; the second gives every key that can be among
 //          the first k its rank in the row by binary searches in the other lists and writes it there.
 //          Without the workspace for the lists (one workgroup per row): the first pass adds the weights and
@@ -90,7 +90,7 @@ __device__ __forceinline__ float select_value(float score, const kvx_h2o_args& a
 constexpr int SEL_THREADS = 1024;
 
 // Deterministic workgroup reductions (wavefront butterfly, then the 16 partials in a fixed order).
-template <typename Op>
+template <int THREADS = SEL_THREADS, typename Op>
 __device__ __forceinline__ float block_reduce(float v, float* red, Op op) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v = op(v, __shfl_xor(v, off, 64));
@@ -98,7 +98,7 @@ __device__ __forceinline__ float block_reduce(float v, float* red, Op op) {
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
   float r = red[0];
-  for (int i = 1; i < SEL_THREADS / 64; ++i) r = op(r, red[i]);
+  for (int i = 1; i < THREADS / 64; ++i) r = op(r, red[i]);
   return r;
 }
 
@@ -315,38 +315,78 @@ __global__ __launch_bounds__(SEL_THREADS) void select_one_kernel(const kvx_h2o_a
 // ---- k > 1, a row over several workgroups -----------------------------------------------------
 //
 // A row has few keys for a device (8 rows of 16384 slots) and many for one workgroup: with one workgroup per row the
-// choice of 1024 slots took 40 us, bound by one compute unit's LDS and instruction issue. Lists of 1024 keys are sorted
-// side by side instead, and ranks need no hand-over between workgroups but the launch boundary.
-// List c of a row takes the 64-slot blocks c, c + C, c + 2C, ... (C lists): old and new tokens lie in runs of slots, and
-// this way every list is a sample of the whole row, so that the bound below is tight whatever the order of the slots.
+// choice of 1024 slots took 40 us, bound by one compute unit's LDS and instruction issue. Lists of 256 or 1024 keys are
+// sorted side by side instead, and ranks need no hand-over between workgroups but the launch boundary.
+// List c of a row takes the 16-slot blocks c, c + C, c + 2C, ... (C lists): old and new tokens lie in runs of slots, and
+// this way every list is a sample of the whole row, so that the bound below is tight whatever the order of the slots. Blocks of
+// 64 slots were too long for that: 1024 new slots in a run met 16 lists of 64 (ranks of 1024 among 16 x 1024 slots 11.2 -> 6.4 us).
 
-constexpr int LIST = 1024;  // keys per list, one per thread of the sorting workgroup
+constexpr int LIST = 1024;  // slots a workgroup of the passes before the sort, one per thread
 constexpr int RANK_THREADS = 512;
 constexpr int RANK_STAGED = 6144;  // keys of the lists' heads that the ranking workgroup holds in LDS
 
-// What the launches hand on, per (row, list).
+// What the launches hand on, per (row, part) or (row, list).
 struct SelectLists {
-  unsigned long long* keys;  // LIST sorted keys
-  float* part_z;             // v_norm: sum of v_norm * w
+  unsigned long long* keys;  // sorted keys
+  float* part_z;             // v_norm: sum of v_norm * w (nullptr: the statistics' workgroups add the row up themselves)
   float* stats;              // q_errors: extremes of the compared value and of the errors (4 floats)
-  int C;
+  int C;                     // parts of LIST slots: norm and statistics
+  int lists;                 // sorted lists
 };
-__device__ __forceinline__ int list_slot(int c, int C, int t) { return ((t >> 6) * C + c) * 64 + (t & 63); }
+__device__ __forceinline__ int part_slot(int c, int C, int t) { return ((t >> 6) * C + c) * 64 + (t & 63); }
+__device__ __forceinline__ int list_slot(int c, int lists, int t) { return ((t >> 4) * lists + c) * 16 + (t & 15); }
 
 __global__ __launch_bounds__(LIST) void list_norm_kernel(const kvx_h2o_args a, const SelectLists sl) {
   __shared__ float red[LIST / 64];
   const int c = blockIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
-  const int slot = list_slot(c, sl.C, threadIdx.x);
+  const int slot = part_slot(c, sl.C, threadIdx.x);
   float x = 0.0f;
   if (slot < a.kv_len) x = a.v_norm[b * a.sc_stride_b + hh * a.sc_stride_h + slot] * a.w[(int64_t)row * a.kv_len + slot];
   x = block_reduce(x, red, [](float u, float v) { return u + v; });
   if (threadIdx.x == 0) sl.part_z[row * sl.C + c] = x;
 }
 
-// The score of this thread's slot after the update (stored), and the slot. Every product and sum rounded on its own.
-__device__ __forceinline__ float updated_score(const kvx_h2o_args& a, const SelectLists& sl, float* red, int row, int b, int hh, int slot) {
+__device__ __forceinline__ float wave_total(float x);
+
+// Sum of v_norm * w over a row: of the parts' sums, or from the products by every workgroup of LIST threads for itself, the same bits
+// (64 products, the 16 wavefronts of a part, the parts). Rows of at most Z_SLOTS slots are added up anew by each of their workgroups
+// (24000 products a workgroup of 16 rows of 6000: norm and statistics 9.7 us as two launches, 7.9 as one); a launch of its own reads a long
+// row once. Ahead of the sort the launch stays for all rows: workgroups of 256 threads took 9 us more for the sum.
+constexpr int Z_SLOTS = 8192, Z_PARTS = Z_SLOTS / LIST;
+template <int THREADS>
+__device__ __forceinline__ float parts_norm(const SelectLists& sl, float* red, int row) {
+  const float z = (int)threadIdx.x < sl.C ? sl.part_z[row * sl.C + threadIdx.x] : 0.0f;
+  return block_reduce<THREADS>(z, red, [](float u, float v) { return u + v; });
+}
+__device__ __forceinline__ float row_norm(const kvx_h2o_args& a, int C, int row, int b, int hh) {
+  constexpr int WAVES = LIST / 64;
+  __shared__ float red[WAVES * Z_PARTS];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const float *vn = a.v_norm + b * a.sc_stride_b + hh * a.sc_stride_h, *w = a.w + (int64_t)row * a.kv_len;
+  float x[Z_PARTS];
+#pragma unroll
+  for (int c = 0; c < Z_PARTS; ++c) {
+    const int slot = part_slot(c, C, threadIdx.x);
+    x[c] = c < C && slot < a.kv_len ? vn[slot] * w[slot] : 0.0f;
+  }
+#pragma unroll
+  for (int c = 0; c < Z_PARTS; ++c) {
+    const float t = wave_total(x[c]);
+    if (lane == 0) red[wave * Z_PARTS + c] = t;
+  }
+  __syncthreads();
+  float z = 0.0f;
+  if (lane < C) {
+    z = red[lane];
+    for (int i = 1; i < WAVES; ++i) z += red[i * Z_PARTS + lane];
+  }
+  return wave_total(z);
+}
+
+// The score of this thread's slot after the update (stored), and the slot; `z`: the row's sum of v_norm * w. Every product and sum
+// rounded on its own.
+__device__ __forceinline__ float updated_score(const kvx_h2o_args& a, float z, int row, int b, int hh, int slot) {
   const int64_t off = b * a.sc_stride_b + hh * a.sc_stride_h;
-  float z = 1.0f;
   const bool in = slot < a.kv_len;
   const float s = in ? a.scores[off + slot] : 0.0f;
   if (!a.w) return s;
@@ -354,9 +394,6 @@ __device__ __forceinline__ float updated_score(const kvx_h2o_args& a, const Sele
   float inst = w;
   if (a.v_norm) {
     const float vn = in ? a.v_norm[off + slot] : 0.0f;
-    z = 0.0f;
-    for (int i = threadIdx.x; i < sl.C; i += LIST) z += sl.part_z[row * sl.C + i];
-    z = block_reduce(z, red, [](float u, float v) { return u + v; });
     inst = __fmul_rn(__fmul_rn(vn, w) / z, (float)a.q_len);
   }
   const float v = __fadd_rn(s, inst);
@@ -368,10 +405,11 @@ __device__ __forceinline__ float updated_score(const kvx_h2o_args& a, const Sele
 __global__ __launch_bounds__(LIST) void list_stats_kernel(const kvx_h2o_args a, const SelectLists sl) {
   __shared__ float red[LIST / 64];
   const int c = blockIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
-  const int slot = list_slot(c, sl.C, threadIdx.x);
+  const int slot = part_slot(c, sl.C, threadIdx.x);
   const bool in = slot < a.limit;
   const float qe = in ? a.q_errors[b * a.sc_stride_b + hh * a.sc_stride_h + slot] : 0.0f;
-  const float v = updated_score(a, sl, red, row, b, hh, slot);
+  const float z = !a.w || !a.v_norm ? 1.0f : sl.part_z ? parts_norm<LIST>(sl, red, row) : row_norm(a, sl.C, row, b, hh);
+  const float v = updated_score(a, z, row, b, hh, slot);
   const int32_t* tpr = a.token_pos ? a.token_pos + b * a.tp_stride_b + hh * a.tp_stride_h : nullptr;
   const float cv = in ? residency_value(v, a, tpr, slot) : 0.0f;
   auto mn = [](float x, float y) { return fminf(x, y); };
@@ -398,6 +436,17 @@ __device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
   }
 }
 
+// Sum over the wavefront in the order of block_reduce's exchanges.
+__device__ __forceinline__ float wave_total(float x) {
+  auto add = [](float v, uint32_t y) { return v + __uint_as_float(y); };
+  x = add(x, lane_xor<32>(__float_as_uint(x)));
+  x = add(x, lane_xor<16>(__float_as_uint(x)));
+  x = add(x, lane_xor<8>(__float_as_uint(x)));
+  x = add(x, lane_xor<4>(__float_as_uint(x)));
+  x = add(x, lane_xor<2>(__float_as_uint(x)));
+  return add(x, lane_xor<1>(__float_as_uint(x)));
+}
+
 template <int S>
 __device__ __forceinline__ unsigned long long sort_step(unsigned long long x, int size) {
   const unsigned long long y = ((unsigned long long)lane_xor<S>((uint32_t)(x >> 32)) << 32) | lane_xor<S>((uint32_t)x);
@@ -405,13 +454,14 @@ __device__ __forceinline__ unsigned long long sort_step(unsigned long long x, in
   return (y < x) == keep_min ? y : x;
 }
 
-// Bitonic sort of LIST keys, one a thread: steps between lanes of a wavefront on the vector ALU, the ten others through
-// LDS (two buffers in turn: one barrier each).
-__device__ __forceinline__ unsigned long long sort_list(unsigned long long x, unsigned long long (&buf)[2][LIST]) {
+// Bitonic sort of L keys, one a thread: steps between lanes of a wavefront on the vector ALU, the others through LDS (two
+// buffers in turn: one barrier each).
+template <int L>
+__device__ __forceinline__ unsigned long long sort_list(unsigned long long x, unsigned long long (&buf)[2][L]) {
   const int t = threadIdx.x;
   int which = 0;
 #pragma unroll 1
-  for (int size = 2; size <= LIST; size <<= 1) {
+  for (int size = 2; size <= L; size <<= 1) {
 #pragma unroll 1
     for (int stride = size >> 1; stride >= 64; stride >>= 1) {
       buf[which][t] = x;
@@ -431,11 +481,12 @@ __device__ __forceinline__ unsigned long long sort_list(unsigned long long x, un
   return x;
 }
 
-__global__ __launch_bounds__(LIST) void list_sort_kernel(const kvx_h2o_args a, const SelectLists sl) {
-  __shared__ float red[LIST / 64];
-  __shared__ unsigned long long buf[2][LIST];
+template <int L>
+__global__ __launch_bounds__(L) void list_sort_kernel(const kvx_h2o_args a, const SelectLists sl) {
+  __shared__ float red[L / 64];
+  __shared__ unsigned long long buf[2][L];
   const int tid = threadIdx.x, c = blockIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
-  const int slot = list_slot(c, sl.C, tid);
+  const int slot = list_slot(c, sl.lists, tid);
   const bool in = slot < a.limit;
   const int32_t* tpr = a.token_pos ? a.token_pos + b * a.tp_stride_b + hh * a.tp_stride_h : nullptr;
   unsigned long long x = ~0ull;
@@ -444,7 +495,7 @@ __global__ __launch_bounds__(LIST) void list_sort_kernel(const kvx_h2o_args a, c
     const float v = in ? a.scores[off + slot] : 0.0f, qe = in ? a.q_errors[off + slot] : 0.0f;
     float v4[4] = {INFINITY, -INFINITY, INFINITY, -INFINITY};
     const float* st = sl.stats + (int64_t)b * a.Hkv * sl.C * 4;
-    for (int i = tid; i < a.Hkv * sl.C; i += LIST) {
+    for (int i = tid; i < a.Hkv * sl.C; i += L) {
       const f32x4_t s4 = *(const f32x4_t*)(st + i * 4);
       v4[0] = fminf(v4[0], s4[0]);
       v4[1] = fmaxf(v4[1], s4[1]);
@@ -454,40 +505,42 @@ __global__ __launch_bounds__(LIST) void list_sort_kernel(const kvx_h2o_args a, c
     auto mn = [](float u, float w) { return fminf(u, w); };
     auto mx = [](float u, float w) { return fmaxf(u, w); };
     Modify m;
-    m.smin = block_reduce(v4[0], red, mn);
-    m.sden = block_reduce(v4[1], red, mx) - m.smin;
-    m.qmin = block_reduce(v4[2], red, mn);
-    m.qden = block_reduce(v4[3], red, mx) - m.qmin;
+    m.smin = block_reduce<L>(v4[0], red, mn);
+    m.sden = block_reduce<L>(v4[1], red, mx) - m.smin;
+    m.qmin = block_reduce<L>(v4[2], red, mn);
+    m.qden = block_reduce<L>(v4[3], red, mx) - m.qmin;
     m.c = (float)a.combination;
     m.c2 = (float)((a.combination - 1.0) / 2.0);
     m.c3 = (float)(1.0 - a.combination);
     if (in) x = ((unsigned long long)ordered_bits(combined_value(residency_value(v, a, tpr, slot), qe, m)) << 32) | (unsigned)slot;
   } else {
-    const float v = updated_score(a, sl, red, row, b, hh, slot);
+    const float z = a.w && a.v_norm ? parts_norm<L>(sl, red, row) : 1.0f;
+    const float v = updated_score(a, z, row, b, hh, slot);
     if (in) x = ((unsigned long long)ordered_bits(residency_value(v, a, tpr, slot)) << 32) | (unsigned)slot;
   }
-  x = sort_list(x, buf);
-  if (sl.C == 1) {  // the row is one list
+  x = sort_list<L>(x, buf);
+  if (sl.lists == 1) {  // the row is one list
     if (tid < a.k) a.next_index[(int64_t)row * a.k + tid] = (int32_t)(x & 0xffffffffull);
   } else {
-    sl.keys[((int64_t)row * sl.C + c) * LIST + tid] = x;
+    sl.keys[((int64_t)row * sl.lists + c) * L + tid] = x;
   }
 }
 
 // Ranks of the keys of list c. `per` = ceil(k / C) keys of every list are at or below U, the largest of the lists'
 // per-th keys, so the first k keys of the row are all at or below U: about per of each list when the lists are alike.
 // Only those are ranked: a key's rank is its place in its list plus its places in the others, found by binary search in
-// the lists' heads (`staged` keys each, in LDS; in memory beyond them).
+// the lists' heads (2^staged keys each, in LDS; in memory beyond them).
+template <int L>
 __global__ __launch_bounds__(RANK_THREADS) void list_rank_kernel(const unsigned long long* __restrict__ lists, int C, int k, int per, int staged, int32_t* __restrict__ next) {
   __shared__ unsigned long long head[RANK_STAGED];
-  __shared__ uint32_t rank[LIST];
+  __shared__ uint32_t rank[L];
   __shared__ unsigned long long wmax[RANK_THREADS / 64];
-  const int tid = threadIdx.x, c = blockIdx.x, row = blockIdx.y;
-  const unsigned long long* base = lists + (int64_t)row * C * LIST;
-  for (int i = tid; i < C * staged; i += RANK_THREADS) head[i] = base[(i / staged) * LIST + i % staged];
+  const int tid = threadIdx.x, c = blockIdx.x, row = blockIdx.y, S = 1 << staged;
+  const unsigned long long* base = lists + (int64_t)row * C * L;
+  for (int i = tid; i < C << staged; i += RANK_THREADS) head[i] = base[(i >> staged) * L + (i & (S - 1))];
   unsigned long long u = 0ull;
   for (int i = tid; i < C; i += RANK_THREADS) {
-    const unsigned long long x = base[i * LIST + per - 1];
+    const unsigned long long x = base[i * L + per - 1];
     u = x > u ? x : u;
   }
 #pragma unroll
@@ -496,36 +549,36 @@ __global__ __launch_bounds__(RANK_THREADS) void list_rank_kernel(const unsigned 
     u = o > u ? o : u;
   }
   if ((tid & 63) == 0) wmax[tid >> 6] = u;
-  for (int i = tid; i < LIST; i += RANK_THREADS) rank[i] = 0u;
+  for (int i = tid; i < L; i += RANK_THREADS) rank[i] = 0u;
   __syncthreads();
   for (int i = 0; i < RANK_THREADS / 64; ++i) u = wmax[i] > u ? wmax[i] : u;
   u = u == ~0ull ? u - 1 : u;  // places without a slot are never ranked
-  auto at = [&](int list, int i) { return i < staged ? head[list * staged + i] : base[list * LIST + i]; };
-  // keys of `list` below x (or up to and including it)
-  auto below = [&](int list, unsigned long long x, bool inclusive) {
-    int lo = 0, n = LIST;
-    if (staged < LIST && (inclusive ? head[list * staged + staged - 1] > x : head[list * staged + staged - 1] >= x)) n = staged;
-    while (n > 0) {
-      const int half = n >> 1;
-      const unsigned long long y = at(list, lo + half);
-      if (inclusive ? y <= x : y < x) {
-        lo += half + 1;
-        n -= half + 1;
-      } else {
-        n = half;
+  // keys of `list` below x
+  auto below = [&](int list, unsigned long long x) {
+    const unsigned long long* h = head + (list << staged);
+    int lo = 0;
+    for (int half = S >> 1; half > 0; half >>= 1) lo += h[lo + half - 1] < x ? half : 0;
+    lo += h[lo] < x ? 1 : 0;
+    if (lo == S && S < L) {
+      for (int n = L - S; n > 0;) {
+        const int half = n >> 1;
+        const bool up = base[list * L + lo + half] < x;
+        lo += up ? half + 1 : 0;
+        n = up ? n - half - 1 : half;
       }
     }
     return lo;
   };
-  const int n = below(c, u, true);
+  auto at = [&](int e) { return e < S ? head[(c << staged) + e] : base[c * L + e]; };
+  const int n = below(c, u + 1);
   for (int i = tid; i < n * C; i += RANK_THREADS) {
     const int list = i / n, e = i - list * n;
-    const int r = list == c ? e : below(list, at(c, e), false);
+    const int r = list == c ? e : below(list, at(e));
     if (r) atomicAdd(&rank[e], (uint32_t)r);
   }
   __syncthreads();
   for (int e = tid; e < n; e += RANK_THREADS)
-    if (rank[e] < (uint32_t)k) next[(int64_t)row * k + rank[e]] = (int32_t)(at(c, e) & 0xffffffffull);
+    if (rank[e] < (uint32_t)k) next[(int64_t)row * k + rank[e]] = (int32_t)(at(e) & 0xffffffffull);
 }
 
 // ---- k > 1, one workgroup per row --------------------------------------------------------------
@@ -771,10 +824,14 @@ static size_t best_bytes(const kvx_h2o_args& a) {
 // what the one-workgroup-per-row form cannot do without
 static size_t min_workspace(const kvx_h2o_args& a) { return best_bytes(a) + (a.q_errors ? (size_t)a.B * a.Hkv * 4 * sizeof(float) : 0); }
 
-// Sorted lists of 1024 keys for k > 1: taken while their number and size stay reasonable (256 lists a row, 1 GiB), else
-// (and where the caller's workspace does not hold them) one workgroup per row.
+// Sorted lists for k > 1: taken while their number and size stay reasonable (256 lists of 1024 keys a row, 1 GiB), else
+// (and where the caller's workspace does not hold them) one workgroup per row. Lists of 256 keys sort in 36 steps, 3 of them through LDS,
+// where 1024 keys take 55 and 10 (6000 slots with errors 9.7 -> 6.4 us, plain 7.7 -> 5.0), but every candidate is looked up in four times as
+// many lists, which costs k times their number: sort and ranks of 128 of 30208 slots (118 lists) 14.8 us (1024 keys: 17.7), of 700 of
+// 12000 (47 lists) 16.5 (15.2), of 1024 of 16384 (64 lists) 22 (14.5), of 1000 of 32000 (125 lists) 25 (13.7).
 struct ListPlan {
-  int C;  // lists per row, 0: not this way
+  int C;         // parts of LIST slots per row, 0: not this way
+  int L, lists;  // keys of a sorted list, lists per row
   size_t off_z, off_stats, total;
 };
 static ListPlan list_plan(const kvx_h2o_args& a) {
@@ -783,8 +840,10 @@ static ListPlan list_plan(const kvx_h2o_args& a) {
   const int64_t C = ((int64_t)a.kv_len + LIST - 1) / LIST, rows = (int64_t)a.B * a.Hkv;
   if (C > 256 || rows * C * LIST * 8 > (1ll << 30)) return p;
   p.C = (int)C;
+  p.L = a.kv_len <= 32768 && (int64_t)a.k * ((a.kv_len + 255) / 256) <= 16384 ? 256 : LIST;
+  p.lists = (a.kv_len + p.L - 1) / p.L;
   const size_t n = (size_t)(rows * C);
-  p.off_z = C > 1 ? n * LIST * 8 : 0;
+  p.off_z = p.lists > 1 ? (size_t)rows * p.lists * p.L * 8 : 0;
   p.off_stats = p.off_z + (n * 4 + 15) / 16 * 16;
   p.total = p.off_stats + n * 16;
   return p;
@@ -795,24 +854,31 @@ size_t h2o_workspace(const kvx_h2o_args& a) {
   return least > lists ? least : lists;
 }
 
+template <int L>
+static void launch_sorted(const kvx_h2o_args& a, const SelectLists& sl, hipStream_t st) {
+  const dim3 grid(sl.lists, a.B * a.Hkv);
+  hipLaunchKernelGGL(list_sort_kernel<L>, grid, dim3(L), 0, st, a, sl);
+  if (sl.lists == 1) return;
+  const int per = (a.k + sl.lists - 1) / sl.lists;
+  int staged = 4;
+  while ((1 << staged) < 2 * per && (1 << staged) < L) ++staged;
+  while (sl.lists << staged > RANK_STAGED) --staged;
+  hipLaunchKernelGGL(list_rank_kernel<L>, grid, dim3(RANK_THREADS), 0, st, (const unsigned long long*)sl.keys, sl.lists, a.k, per, staged, a.next_index);
+}
+
 static int launch_lists(const kvx_h2o_args& a, const ListPlan& p, hipStream_t st) {
   SelectLists sl;
   char* ws = (char*)a.workspace;
   sl.keys = (unsigned long long*)ws;
-  sl.part_z = (float*)(ws + p.off_z);
+  sl.part_z = a.kv_len > Z_SLOTS || !a.q_errors ? (float*)(ws + p.off_z) : nullptr;
   sl.stats = (float*)(ws + p.off_stats);
   sl.C = p.C;
+  sl.lists = p.lists;
   const dim3 grid(p.C, a.B * a.Hkv);
-  if (a.w && a.v_norm) hipLaunchKernelGGL(list_norm_kernel, grid, dim3(LIST), 0, st, a, sl);
+  if (a.w && a.v_norm && sl.part_z) hipLaunchKernelGGL(list_norm_kernel, grid, dim3(LIST), 0, st, a, sl);
   if (a.q_errors) hipLaunchKernelGGL(list_stats_kernel, grid, dim3(LIST), 0, st, a, sl);
-  hipLaunchKernelGGL(list_sort_kernel, grid, dim3(LIST), 0, st, a, sl);
-  if (p.C > 1) {
-    const int per = (a.k + p.C - 1) / p.C;
-    int staged = 16;
-    while (staged < 2 * per && staged < LIST) staged <<= 1;
-    while (staged * p.C > RANK_STAGED) staged >>= 1;
-    hipLaunchKernelGGL(list_rank_kernel, grid, dim3(RANK_THREADS), 0, st, (const unsigned long long*)sl.keys, p.C, a.k, per, staged, a.next_index);
-  }
+  if (p.L == 256) launch_sorted<256>(a, sl, st);
+  else launch_sorted<LIST>(a, sl, st);
   KVX_HIP(hipGetLastError());
   return KVX_OK;
 }

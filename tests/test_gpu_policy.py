@@ -432,3 +432,19 @@ def test_selection_over_lists_matches_one_workgroup_per_row(kvx, gpu, B, Hkv, L,
     else:
         torch.testing.assert_close(s0, s1, rtol=1e-5, atol=0)
         _sets_equal_away_from_ties(n0, n1, s1[..., :limit], k)
+
+
+@pytest.mark.parametrize("B,Hkv,L,gp,k", [
+    (2, 2, 256, 0, 256),       # one list of 256 keys, all of it chosen
+    (1, 3, 257, 1, 31),        # a second list of one slot, behind the limit
+    (1, 2, 4000, 15, 1024),    # lists of 256 at the line, 16 of them
+    (1, 2, 4000, 15, 1025),    # beyond it: lists of 1024
+    (2, 2, 8192, 5, 200),      # the longest row whose norm the statistics add up
+    (1, 2, 8193, 0, 100),      # a longer one
+    (1, 1, 32768, 0, 64),      # 128 lists of 256
+    (1, 1, 32769, 0, 64),      # 33 lists of 1024
+])
+def test_selection_over_short_and_long_lists(kvx, gpu, B, Hkv, L, gp, k):
+    for policy in ("h2o", "vlen", "q_errors"):
+        test_selection_over_lists_matches_one_workgroup_per_row(kvx, gpu, B, Hkv, L, gp, k, policy)
+    test_update_select_variants_direct(kvx, gpu, B, Hkv, L, L - gp, k, True, True, True)
