@@ -12,6 +12,7 @@ struct MergeParams {
   float* lse;  // (B, q_len, Hq) or NULL
   int32_t B, Hq, Hkv, G, q_len, R, num_splits;
   int64_t o_sb, o_sh, o_st;
+  int32_t input_pos, split_keys;  // slots in position order: keys of a split; a row has no partial in splits behind its position. 0: all splits
 };
 
 // Combine the per-split partials of a row: D / 4 threads a row, each four values, times SC split classes that take
@@ -32,11 +33,11 @@ __device__ __forceinline__ void merge_job(const MergeParams& p, const int64_t bl
   static_assert(ROWS >= 1, "a row's threads fit a workgroup");
   __shared__ f32x4_t red_o[SC > 1 ? 256 : 1];
   __shared__ float red_l[SC > 1 ? 256 : 1];
-  const int S = p.num_splits;
   const int64_t total_rows = (int64_t)p.B * p.Hkv * p.R;
   const int64_t grow = block * ROWS + threadIdx.x / (TPR * SC);
   const bool live = grow < total_rows;
   const int64_t growc = live ? grow : total_rows - 1;
+  const int S = p.split_keys ? min(p.num_splits, (p.input_pos + (int)(growc % p.R) / p.G) / p.split_keys + 1) : p.num_splits;
   const int dq = threadIdx.x % TPR, j = (threadIdx.x / TPR) % SC;
   const f32x2_t* ml = (const f32x2_t*)p.part_ml + growc;  // (maximum, sum) of split s at s * total_rows
   const float* po = p.part_o + growc * D + dq * 4;

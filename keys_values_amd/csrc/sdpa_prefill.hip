@@ -254,7 +254,32 @@ struct Loader {
   }
 };
 
-template <int D, int KV>
+// Jobs of a causal first chunk in splits, in the order of their length. A split covers the keys of `period` blocks of rows, so that the
+// rows of period i see the splits before i whole and their own in part: first all the whole ones, then the others from the longest on.
+__device__ __forceinline__ void causal_job(const PrefillParams& p, int job, int& mblk, int& split) {
+  const int P = p.period, n = p.num_splits, last = p.m_blocks - (n - 1) * P;  // blocks of the last period, 1 to P
+  for (int i = n - 1; i > 0; --i) {
+    const int blocks = i == n - 1 ? last : P;
+    if (job < blocks * i) {
+      mblk = i * P + job / i;
+      split = job % i;
+      return;
+    }
+    job -= blocks * i;
+  }
+  const int longer = (P - last) * (n - 1);  // places in a period that the last one does not have
+  if (job < longer) {
+    split = job % (n - 1);
+    mblk = split * P + P - 1 - job / (n - 1);
+  } else {
+    job -= longer;
+    split = job % n;
+    mblk = split * P + last - 1 - job / n;
+  }
+}
+
+// PERIODS: jobs of a causal first chunk in splits (causal_job; decided at run time it cost every call 0.2 us)
+template <int D, int KV, bool PERIODS>
 __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ? 2 : 1) void sdpa_prefill_kernel(const PrefillParams p) {
   constexpr bool F16 = kv_elem_f16(KV);  // element type of q, k, v, o
   constexpr int BM = 32 * nwaves(KV, D);  // rows per workgroup
@@ -271,8 +296,8 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
   const int group = blockIdx.x;  // b * Hkv + kvh: fastest-varying so that a KV head stays on one XCD
   // slots in position order (a causal first chunk): the later rows see more tiles; they start first, so that the short
   // ones fill up the end (a first chunk of 8192 tokens, 32 heads of 128: 597 -> 543 us)
-  const int mblk = p.tp ? blockIdx.y : gridDim.y - 1 - blockIdx.y;
-  const int split = blockIdx.z;
+  int mblk = p.tp ? blockIdx.y : gridDim.y - 1 - blockIdx.y, split = blockIdx.z;
+  if constexpr (PERIODS) causal_job(p, blockIdx.y, mblk, split);
   const int b = group / p.Hkv;
   const int kvh = group % p.Hkv;
 
@@ -321,15 +346,9 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
     // see are masked out completely (the upper triangle of a causal first chunk) and are skipped
     const int qpos_max = p.input_pos + min(mblk * BM + BM - 1, p.R - 1) / p.G;
     tile_end = min(tile_end, qpos_max / BN + 1);
-    if (tile_end <= tile_begin) {  // whole split invisible: an empty partial (only with num_splits > 1)
+    if (tile_end <= tile_begin) {  // whole split invisible (only with num_splits > 1): its output is not read
       if (row_ok) {
         const int64_t prow = ((int64_t)split * p.B * p.Hkv + group) * p.R + row;
-        float* po = p.part_o + prow * D;
-        const f32x4_t z = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int a = 0; a < 4; ++a) *(f32x4_t*)(po + dt * 32 + 8 * a + 4 * h) = z;
         if (h == 0) {
           p.part_ml[prow * 2] = -INFINITY;
           p.part_ml[prow * 2 + 1] = 0.0f;
@@ -621,6 +640,40 @@ int pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
   return best;
 }
 
+// Splits of a causal first chunk (rows see the keys up to their own), by estimated time: tiles of a split, at whose bounds a block of rows
+// begins. Splits of all rows alike left units idle: the jobs differ in length, and those that see nothing still wrote and merged empty partials
+// (8 heads of 128 over 2, 4096 tokens: 4 splits 74 us, 3 57, 2 68). Here jobs without keys are not launched, a row merges the splits that it sees,
+// and the jobs run in the order of their length (causal_job), so the walk takes the sum of the tiles that are seen and the jobs' begin and
+// end, and a quarter of a split at the end; never less than one split, and more where two of them share a unit from the start. Calls of
+// 8 heads over 2 of 4096 tokens 67.7 -> 60.9 us, of 2048 39.1 -> 33.1; 4 over 1, 8000 tokens 106 -> 91; 16 of 64 over 4, 3000 51.1 -> 48.2; 8 of
+// 256 over 2, 3000 113 -> 83. Where the rows alone fill the device one split stays the best (32 over 8, 4096 tokens 148; two: 190).
+int causal_split_tiles(const kvx_sdpa_args& a, int bm, int m_blocks) {
+  const int G = a.Hq / a.Hkv, tiles = (a.q_len + BN - 1) / BN;
+  const int64_t groups = (int64_t)a.B * a.Hkv, cus = num_cus(), rows = groups * G * a.q_len;
+  const int64_t tile_ns = a.D == 64 ? 700 : a.D == 128 ? 1130 : 2050, job_ns = 3000;
+  const bool pairs = a.D <= 128;
+  const int share = pairs ? 80 : 100;  // percent: two workgroups of a unit gain 20 %
+  const int64_t seen = groups * m_blocks * (tiles + 1) / 2;
+  int unit = 1;
+  while (unit * BN * G % bm) unit *= 2;
+  int best = tiles;
+  int64_t best_ns = INT64_MAX;
+  for (int s = 1; s <= min(16, tiles); ++s) {
+    const int tps = s == 1 ? tiles : ((tiles + s - 1) / s + unit - 1) / unit * unit;
+    if (s > 1 && (tps >= tiles || (int64_t)m_blocks * (s + 1) / 2 + m_blocks > 65535)) break;  // (jobs are a grid's second dimension)
+    const int64_t jobs = groups * m_blocks * (s + 1) / 2, one = tps * tile_ns + job_ns;
+    const int64_t sum = (seen * tile_ns + jobs * job_ns) * share / 100 / cus;
+    const int64_t alone = pairs && jobs > cus && jobs <= 2 * cus ? one * 115 / 100 : one;  // all at once, two to most units
+    const int64_t walk = jobs <= cus ? one : max(alone, sum + (s == 1 ? 0 : one / 4));
+    const int64_t merge = s == 1 ? 0 : 2000 + rows * (s + 1) / 2 * (a.D * 4 + 8) / 4000;
+    if (walk + merge < best_ns) {
+      best_ns = walk + merge;
+      best = tps;
+    }
+  }
+  return best;
+}
+
 void fill_params(PrefillParams& p, const kvx_sdpa_args& a) {
   p.q = (const uint16_t*)a.q;
   p.k = a.k;
@@ -648,6 +701,13 @@ void fill_params(PrefillParams& p, const kvx_sdpa_args& a) {
   p.num_splits = a.num_splits > 0 ? min(a.num_splits, p.num_tiles) : p.columns ? rows.splits : pick_splits(a, p.m_blocks, p.num_tiles);
   p.tiles_per_split = (p.num_tiles + p.num_splits - 1) / p.num_splits;
   p.num_splits = (p.num_tiles + p.tiles_per_split - 1) / p.tiles_per_split;
+  p.period = 0;
+  if (!a.token_positions && a.input_pos == 0 && a.q_len <= a.kv_len && kv_is_plain(a.kv_dtype) && a.num_splits <= 0 && !p.columns) {
+    p.num_tiles = (a.q_len + BN - 1) / BN;  // nobody sees the keys behind
+    p.tiles_per_split = causal_split_tiles(a, bm, p.m_blocks);
+    p.num_splits = (p.num_tiles + p.tiles_per_split - 1) / p.tiles_per_split;
+    if (p.num_splits > 1) p.period = p.tiles_per_split * BN * p.G / bm;
+  }
   p.c = a.sm_scale * kLog2e;
   p.q_sb = a.q_stride_b; p.q_sh = a.q_stride_h; p.q_st = a.q_stride_t;
   p.k_sb = a.k_stride_b; p.k_sh = a.k_stride_h; p.k_st = a.k_stride_t;
@@ -675,10 +735,26 @@ int launch_t(PrefillParams& p, hipStream_t st, MergeParams* rest) {
     if (rc != KVX_OK) return rc;
   } else {
     dim3 grid(p.B * p.Hkv, p.m_blocks, p.num_splits);
-    hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
+    if (p.period) {
+      const int n = p.num_splits, last = p.m_blocks - (n - 1) * p.period;
+      grid.y = (unsigned)(p.m_blocks + p.period * ((n - 1) * (n - 2) / 2) + last * (n - 1));
+      grid.z = 1;
+      if (rest) {  // whoever combines the partials reads the (empty) ones of all splits
+        grid.y = (unsigned)p.m_blocks;
+        grid.z = (unsigned)n;
+        p.period = 0;
+      }
+    }
+    bool periods = false;
+    if constexpr (kv_is_plain(KV)) {
+      periods = p.period != 0;
+      if (periods) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, true>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
+    }
+    if (!periods) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, false>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
     KVX_HIP(hipGetLastError());
   }
-  const MergeParams m = {p.part_o, p.part_ml, p.o, p.lse, p.B, p.Hq, p.Hkv, p.G, p.q_len, p.R, p.num_splits, p.o_sb, p.o_sh, p.o_st};
+  const MergeParams m = {p.part_o, p.part_ml, p.o, p.lse, p.B, p.Hq, p.Hkv, p.G, p.q_len, p.R, p.num_splits, p.o_sb, p.o_sh, p.o_st,
+                         p.input_pos, p.tp ? 0 : p.tiles_per_split * BN};
   if (rest) {
     *rest = m;
     return KVX_OK;

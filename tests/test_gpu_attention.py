@@ -741,3 +741,27 @@ def _check_some_heads(gpu, store, dtype, B, Hq, Hkv, q_len, T, D, splits):
         assert rel_err(out[one, heads].float().cpu(), o_ref.float()) < O_RTOL
         torch.testing.assert_close(w[one, h : h + 1].cpu(), w_ref, rtol=W_RTOL, atol=1e-6)
         torch.testing.assert_close(lse[one, :, heads].cpu(), O.lse2(qc, kc, scale, pos, tc), rtol=1e-4, atol=1e-3)
+
+
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,q_len,behind,D", [
+    (torch.bfloat16, 1, 8, 2, 2048, 0, 128),   # whole periods of blocks
+    (torch.float16, 1, 7, 1, 2311, 0, 128),    # 7 heads: splits of an even number of tiles; the last period short, its last block ragged
+    (torch.bfloat16, 1, 2, 1, 4000, 77, 128),  # keys that nobody sees behind the chunk
+    (torch.bfloat16, 1, 12, 2, 1921, 0, 64),   # one token beyond 30 tiles
+    (torch.float16, 1, 4, 2, 1500, 1, 256),
+    (torch.bfloat16, 1, 1, 1, 9000, 0, 64),    # one head, many splits
+])
+def test_causal_first_chunk_in_splits(gpu, dtype, B, Hq, Hkv, q_len, behind, D):
+    # tolerances of the path; and against the same call in one split and in three of all rows alike
+    T, scale = q_len + behind, D ** -0.5
+    q, k, v, _ = make_qkv(17 + T, B, Hq, Hkv, q_len, T, D, dtype=dtype)
+    qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+    out, _, lse = ops.prefill_core(qd, kd, vd, scale, 0, return_lse=True, output_transposed=False)
+    for splits in (1, 3):
+        o2, _, l2 = ops.prefill_core(qd, kd, vd, scale, 0, return_lse=True, output_transposed=False, num_splits=splits)
+        check_o(out, o2.cpu())
+        torch.testing.assert_close(lse, l2, rtol=1e-4, atol=1e-3)
+    heads = slice(0, Hq // Hkv)  # one KV head against the oracle
+    qc, kc, vc = q[:1, heads], k[:1, :1], v[:1, :1]
+    check_o(out[:1, heads], O.sdpa_in_blocks(qc, kc, vc, scale, 0, None)[0])
+    torch.testing.assert_close(lse[:1, :, heads].cpu(), O.lse2(qc, kc, scale, 0, None), rtol=1e-4, atol=1e-3)
