@@ -68,7 +68,7 @@ struct DecodeParams {
   int32_t qs_vec;            // quantiser state arrays are 16-byte aligned with strides that keep them so (vector loads of 4 keys)
   int32_t resident;          // the logits of a split stay in LDS
   int32_t one_launch;        // the splits themselves combine their outputs (always, but for logits through the scratch by plan)
-  int32_t spin_limit;        // polls of row_count before a workgroup gives up and sends its logits out
+  int32_t spin_limit;        // polls of the other splits' pairs before a workgroup gives up and sends its logits out
   int32_t poll_sleep;        // pause between two polls, in units of 512 cycles
   int32_t B, Hq, Hkv, kv_len, Tpad, num_splits, keys_per_split;
   int32_t Gr;  // query heads per KV head; the kernels' G is Gr rounded up to a power of two (heads Gr .. G - 1 are
