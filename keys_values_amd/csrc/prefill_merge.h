@@ -19,6 +19,8 @@ struct MergeParams {
 // splits j, j + SC, ... and are added through LDS. Bound by HBM (every partial is read once) where there are many rows;
 // with few rows (32 queries over 32768 keys: 1024 rows of 32 splits) a thread's walk over the splits was the time, a memory
 // latency per split and 15 us of a 46 us call: four loads in flight and SC classes make it about two latencies.
+// The first four partials are asked for together with their maxima, and up to four splits the maxima are read once: 32768 rows of 2 splits of
+// 128 values 11.3 -> 9.4 us (4.6 TB/s), 24000 of 2 to 3 of 256 14.0 -> 11.4, 960 of 16 of 64 7.2 -> 5.9.
 // ROWS: rows of one workgroup of 256 threads.
 constexpr int merge_rows(int D, int SC) { return 256 / (D / 4 * SC); }  // D: 64, 128 or 256
 // split classes while a walk is longer than four splits and the rows alone leave the device short of threads
@@ -41,23 +43,37 @@ __device__ __forceinline__ void merge_job(const MergeParams& p, const int64_t bl
   const int dq = threadIdx.x % TPR, j = (threadIdx.x / TPR) % SC;
   const f32x2_t* ml = (const f32x2_t*)p.part_ml + growc;  // (maximum, sum) of split s at s * total_rows
   const float* po = p.part_o + growc * D + dq * 4;
-  float M = -INFINITY;
-  for (int s0 = 0; s0 < S; s0 += 4) {
+  // the partials of splits s0, s0 + SC, ... (four at most), all asked for at once; nothing where there is no such split
+  f32x2_t m[4];
+  f32x4_t x[4];
+  auto load = [&](int s0) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) M = fmaxf(M, ml[(int64_t)min(s0 + u, S - 1) * total_rows][0]);
+    for (int u = 0; u < 4; ++u) {
+      m[u] = f32x2_t{-INFINITY, 0.0f};
+      x[u] = f32x4_t{0, 0, 0, 0};
+      if (s0 + u * SC < S) {
+        const int64_t at = (int64_t)(s0 + u * SC) * total_rows;
+        m[u] = ml[at];
+        x[u] = *(const f32x4_t*)(po + at * D);
+      }
+    }
+  };
+  load(j);
+  float M;
+  if (SC == 1 && S <= 4) {
+    M = fmaxf(fmaxf(m[0][0], m[1][0]), fmaxf(m[2][0], m[3][0]));
+  } else {
+    M = -INFINITY;
+    for (int s0 = 0; s0 < S; s0 += 4) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) M = fmaxf(M, ml[(int64_t)min(s0 + u, S - 1) * total_rows][0]);
+    }
   }
   const float Mu = (M == -INFINITY) ? 0.0f : M;
   float L = 0.0f;
   f32x4_t acc = {0, 0, 0, 0};
   for (int s0 = j; s0 < S; s0 += 4 * SC) {
-    f32x2_t m[4];
-    f32x4_t x[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int64_t at = (int64_t)min(s0 + u * SC, S - 1) * total_rows;
-      m[u] = ml[at];
-      x[u] = *(const f32x4_t*)(po + at * D);
-    }
+    if (s0 != j) load(s0);
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       if (s0 + u * SC < S) {
