@@ -164,8 +164,11 @@ constexpr int logit_floats(int G, int D, bool codes) {
   if (D == 256 && codes) return G == 8 ? 30720 : 32768;
   return G * D <= 512 ? 16384 : (G * D <= 1024 ? (G == 16 ? 12288 : 14336) : 8192);
 }
-// Splits of a row: their weights (finish_split) share the LDS of the wavefronts' outputs.
-constexpr int max_splits(int D) { return min(512, WAVES * D); }
+constexpr int kMaxSplits = 512;  // of a row
+// The weights of a row's splits (finish_split) take the LDS of the wavefronts' outputs, which has room for WAVES * D of them a head:
+// for all at head sizes from 128 on, for 256 at 64. Those of more splits take the place of the logits, once these are used; a
+// buffer of their own would leave a compute unit one workgroup of 16 heads instead of two.
+constexpr bool weights_beside_logits(int D, int S) { return WAVES * D >= kMaxSplits || S <= WAVES * D; }
 constexpr int kCountStride = 64;  // a row's counters have 256 bytes to themselves: the polls of different rows go to different channels
 constexpr int kArrived = 0, kFinished = 1, kSelected = 2;
 static_assert(kCountStride == kDecodeCounterStride, "the slot write clears these counters");
@@ -229,6 +232,7 @@ template <int G>
 struct FinishShared {
   float lse[G];
   float inv[G];  // 1 / sum of the head relative to its maximum
+  float top[G];  // its maximum, where the splits' weights come later
   float z;  // scores weighted by the V norms: the row's sum of |V row| W
   float vn[G];
   float red[WAVES][4];
@@ -276,13 +280,17 @@ __device__ __forceinline__ P at_byte(P base, uint32_t bytes) {
   return (P)((global_ptr<char>)base + bytes);
 }
 
+// Maximum of a head in a split, by its place in [head][split], once the pairs have been found.
+__device__ __forceinline__ float split_maximum(const RowAt& at, const int i) { return __uint_as_float((uint32_t)coherent_load(at_byte(at.ml, (uint32_t)i * 8u))); }
+
 // The row's maxima, sums and log-sum-exps (and z) from its splits' partials, in LDS for the whole workgroup, and every split's
-// weight 2^(maximum - row's maximum) in wt ([head][split]). wait: the splits may still be on their way. The pairs themselves say
-// so: they are zero before the launch and never afterwards, so a poll that finds them all has them already (a count of the
+// weight 2^(maximum - row's maximum) in wt ([head][split]; unless early, late_weights forms these). wait: the splits may still be
+// on their way. The pairs themselves say so: they are zero before the launch and never afterwards, so a poll that finds them all has them already (a count of the
 // splits that have arrived costs a wait for the pairs' store, the atomic add behind it and, once the count is full, another
 // read: 1 us of a 16 us step). Bounded; returns whether all were found.
 template <int G, bool VARIANT>
-__device__ __forceinline__ bool row_state(const DecodeParams& p, const RowAt& at, const bool wait, const bool vnorm, const int row, FinishShared<G>& sh, float* wt) {
+__device__ __forceinline__ bool row_state(const DecodeParams& p, const RowAt& at, const bool wait, const bool vnorm, const int row, FinishShared<G>& sh, float* wt,
+                                          const bool early) {
   constexpr int HPW = (G + WAVES - 1) / WAVES;  // heads of a wavefront: wave, wave + WAVES, ...; lane s takes splits s, s + 64, ...
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), S = p.num_splits;
   RowSum rs[HPW];
@@ -314,7 +322,7 @@ __device__ __forceinline__ bool row_state(const DecodeParams& p, const RowAt& at
     for (int h = 0; h < HPW; ++h) {
       const int g = wave + WAVES * h;
       rs[h].add(pair[h]);
-      if (g < G && sp < S) wt[g * S + sp] = __uint_as_float((uint32_t)pair[h]);
+      if (early && g < G && sp < S) wt[g * S + sp] = __uint_as_float((uint32_t)pair[h]);
     }
   }
 #pragma unroll
@@ -324,11 +332,18 @@ __device__ __forceinline__ bool row_state(const DecodeParams& p, const RowAt& at
     rs[h].join_lanes();
     const float lse = g < p.Gr ? rs[h].lse() : INFINITY;  // dummy heads: exp2(x - inf) = 0
     float z = 0.0f;
-    for (int sp = lane; sp < S; sp += 64) {  // the lane's own entries
-      const float m = wt[g * S + sp];
+    if (__builtin_expect(early, 1)) {
+      for (int sp = lane; sp < S; sp += 64) {  // the lane's own entries
+        const float m = wt[g * S + sp];
+        if constexpr (VARIANT)
+          if (vnorm && g < p.Gr && ok) z += coherent_load(p.part_vn + ((int64_t)row * p.Gr + g) * S + sp) * fast_exp2(m - lse);
+        wt[g * S + sp] = fast_exp2(m - rs[h].top);
+      }
+    } else {
       if constexpr (VARIANT)
-        if (vnorm && g < p.Gr && ok) z += coherent_load(p.part_vn + ((int64_t)row * p.Gr + g) * S + sp) * fast_exp2(m - lse);
-      wt[g * S + sp] = fast_exp2(m - rs[h].top);
+        if (vnorm && g < p.Gr && ok)
+          for (int sp = lane; sp < S; sp += 64) z += coherent_load(p.part_vn + ((int64_t)row * p.Gr + g) * S + sp) * fast_exp2(split_maximum(at, g * S + sp) - lse);
+      if (lane == 0) sh.top[g] = rs[h].top;
     }
     if (VARIANT && vnorm) z = wave_sum(z);
     if (lane == 0) {
@@ -350,6 +365,14 @@ __device__ __forceinline__ bool row_state(const DecodeParams& p, const RowAt& at
     __syncthreads();
   }
   return ok;
+}
+
+// The splits' weights behind row_state, for the whole workgroup.
+template <int G>
+__device__ __forceinline__ void late_weights(const DecodeParams& p, const RowAt& at, const FinishShared<G>& sh, float* wt) {
+  for (int g = 0; g < p.Gr; ++g)
+    for (int sp = threadIdx.x; sp < p.num_splits; sp += NTHREADS) wt[g * p.num_splits + sp] = fast_exp2(split_maximum(at, g * p.num_splits + sp) - sh.top[g]);
+  __syncthreads();
 }
 
 // The row's outputs for the value pairs [e0, e1) of its E = Gr D / 2: O = (sum over the splits of part_o weight) / sum. J
@@ -509,16 +532,18 @@ __device__ __forceinline__ void publish_choice(const DecodeParams& p, const kvx_
 // for by one lane, one key weighed a pass and reductions through LDS -> as here: 8 rows of 4096 keys 16.2 -> 12.7 us, 32 rows
 // of 16384 8-bit keys 44.0 -> 40.9.
 template <int D, int G, bool F16, bool VARIANT>
-__device__ __forceinline__ void finish_split(const DecodeParams& p, const kvx_h2o_args& hh, const RowAt& at, const float* lgbuf, float (&red)[WAVES][G][D],
+__device__ __forceinline__ void finish_split(const DecodeParams& p, const kvx_h2o_args& hh, const RowAt& at, float* lgbuf, float (&red)[WAVES][G][D],
                                              const float (&rml)[WAVES][G][2], float* lgrow, const int k_begin, const int k_end) {
   __shared__ FinishShared<G> sh;
+  static_assert(WAVES * D >= kMaxSplits || G * kMaxSplits <= logit_floats(G, D, true), "late weights take the logits' place");
   const int tid = threadIdx.x;
   const int split = blockIdx.x, kvh = blockIdx.y, b = blockIdx.z;
   const int row = b * p.Hkv + kvh, S = p.num_splits, E = p.Gr * (D / 2);
   const bool vnorm = VARIANT && hh.v_norm;
   const float* vn = vnorm ? hh.v_norm + b * hh.sc_stride_b + kvh * hh.sc_stride_h : nullptr;
   const float* qe = VARIANT && hh.q_errors ? hh.q_errors + b * hh.sc_stride_b + kvh * hh.sc_stride_h : nullptr;
-  float* wt = &red[0][0][0];  // [head][split], at most max_splits(D) of them
+  const bool early = weights_beside_logits(D, S);
+  float* wt = early ? &red[0][0][0] : lgbuf;  // [head][split]
   auto publish_sums = [&] {   // read by other workgroups while this kernel runs, as are the outputs
     if (tid < p.Gr) {
       float M = rml[0][tid][0], l = 0.0f;
@@ -584,7 +609,7 @@ __device__ __forceinline__ void finish_split(const DecodeParams& p, const kvx_h2
   __syncthreads();
   if (tid == 0 && S > 1) __hip_atomic_fetch_add(at.cnt + kArrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   bool ready = p.spin_limit > 0;
-  if (S > 1 || ready) ready = row_state<G, VARIANT>(p, at, S > 1, vnorm, row, sh, wt);
+  if (S > 1 || ready) ready = row_state<G, VARIANT>(p, at, S > 1, vnorm, row, sh, wt, early);
   uint32_t left = 0, finished = 0;  // left to the row's last split: 1 the weights, 2 the outputs
   auto count_in = [&] {
     if (tid == 0) {
@@ -626,6 +651,7 @@ __device__ __forceinline__ void finish_split(const DecodeParams& p, const kvx_h2
       sh.outputs = arrived >= (uint32_t)S;
     }
     __syncthreads();
+    if (__builtin_expect(!early, 0)) late_weights<G>(p, at, sh, wt);  // behind the barrier: the logits are used
     if (p.scores) publish_choice<G, VARIANT>(p, hh, at, sh, row, split);
     const int e0 = p.share * split;
     if (!sh.outputs) left = 2;
@@ -649,7 +675,10 @@ __device__ __forceinline__ void finish_split(const DecodeParams& p, const kvx_h2
 
   // ---- the row's last split: what the splits that gave up left, the log-sum-exps, the chosen slot -------------------
   if (finished >= kPending) {
-    if (!ready) row_state<G, VARIANT>(p, at, false, vnorm, row, sh, wt);
+    if (!ready) {
+      row_state<G, VARIANT>(p, at, false, vnorm, row, sh, wt, early);
+      if (!early) late_weights<G>(p, at, sh, wt);
+    }
     for (int sp = 0; sp < S; ++sp) {
       const uint32_t todo = coherent_load(at.pending + sp);  // the same for every thread
       if (todo & 2) merge_pairs<D, F16, G>(p, at, sh, wt, p.share * sp, min(p.share * (sp + 1), E), [] {});

@@ -87,11 +87,15 @@ Plan make_plan(const kvx_sdpa_args& a, bool fused_h2o) {
     n = min(n, min((int64_t)(a.kv_len + 127) / 128, (int64_t)(a.kv_len < 16384 ? 64 : 128)));
     if (allow_resident && a.kv_len > n * lgk) {
       const int64_t least = (a.kv_len + lgk - 1) / lgk;
-      n = max(least, in_rounds((least * rows + cus - 1) / cus));
+      // More than 256 splits a row (head size 64: 8 heads from 524289 keys on, 16 from 196609) only where the device holds all of
+      // the call's at once. Through the scratch -> on the chip, us: one row of 16 heads over 197000 keys 37 -> 34, 393216
+      // 50 -> 42, of 8 heads over 600000 61 -> 47; two rows of 16 heads over 197000 keys 41 -> 61, over 393216 68 -> 81, four
+      // rows over 262144 8-bit keys 66 -> 115.
+      if (least <= WAVES * a.D || least * rows <= 2 * cus) n = max(least, in_rounds((least * rows + cus - 1) / cus));
     }
-    splits = (int)min(n, (int64_t)max_splits(a.D));
+    splits = (int)min(n, (int64_t)kMaxSplits);
   }
-  splits = max(1, min(splits, max_splits(a.D)));
+  splits = max(1, min(splits, kMaxSplits));
   int kps = (a.kv_len + splits - 1) / splits;
   kps = ((kps + 63) / 64) * 64;  // keeps the chunks of a split aligned to the logits rows
   pl.keys_per_split = kps;

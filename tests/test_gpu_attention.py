@@ -364,6 +364,56 @@ def test_decode_reports_the_splits_that_took_the_scratch_route(kvx, gpu):
     assert int(n.item()) == 0  # no logits, nothing through the scratch
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,T,store,splits,on_chip", [
+    (1, 16, 1, 196608, "plain", 0, True),   # 256 splits of 768 keys or fewer: their weights fit beside the logits
+    (1, 16, 1, 196609, "plain", 0, True),   # more: they take the logits' place
+    (1, 12, 1, 262144, "plain", 0, True),   # 12 heads padded to 16
+    (1, 24, 2, 262144, "plain", 0, False),  # two rows of them: not all side by side, through the scratch
+    (1, 16, 1, 393216, "u8", 0, True),      # 512 full splits, the most that stays on the chip
+    (1, 8, 1, 32769, "u4", 512, True),      # asked for: 257 splits, the last one of a single key
+    (2, 4, 1, 32768, "plain", 512, True),   # 512 splits of 64 keys, the kernel without matrix instructions
+    (1, 2, 2, 33000, "plain", 400, True),
+])
+def test_decode_at_head_size_64_in_more_than_256_splits(gpu, decode_route, B, Hq, Hkv, T, store, splits, on_chip):
+    """A row of up to 512 splits can be one launch with the logits on the chip. Tolerances of the path."""
+    D, scale = 64, 0.125
+    q, k, v, _ = make_qkv(T + Hq, B, Hq, Hkv, 1, T, D)
+    quant, kd, vd = None, k.to(gpu), v.to(gpu)
+    if store != "plain":
+        bits, codes, state, rows = 8 if store == "u8" else 4, [], [], []
+        for x in (kd, vd):
+            qz = RowQuantizer((B, Hkv, T, D), torch.bfloat16, bits, allocate_buffers=True, device=gpu)
+            qz.quantize(0, T, x)
+            codes.append(qz.quant_buffer.view(B, Hkv, T, -1))
+            state += [qz.quant_scales.view(B, Hkv, T), qz.quant_zero_points.view(B, Hkv, T)]
+            rows.append(qz.dequantize(0, T).cpu())
+        (kd, vd), (k, v), quant = codes, rows, ops.QuantState(*state)
+    o_ref, w_ref = O.sdpa_in_blocks(q, k, v, scale, T - 1, None)
+    n = torch.full((1,), -5, dtype=torch.int32, device=gpu)
+    out, w, lse = ops.decode_core(q.to(gpu), kd, vd, scale, return_weights=True, return_lse=True, quant=quant, num_splits=splits, scratch_splits=n)
+    if decode_route == "resident":
+        assert (int(n.item()) == 0) == on_chip
+    check_o(out.unsqueeze(2), o_ref)
+    torch.testing.assert_close(lse.cpu(), O.lse2(q, k, scale, T - 1, None), rtol=1e-4, atol=1e-3)
+    check_w(w, w_ref, 1)
+    out2, _, lse2 = ops.decode_core(q.to(gpu), kd, vd, scale, return_lse=True, quant=quant, num_splits=splits or 300)
+    check_o(out2.unsqueeze(2), o_ref)
+    torch.testing.assert_close(lse2, lse, rtol=1e-4, atol=1e-3)
+
+
+def test_decode_workspace_counts_the_splits_asked_for(kvx, gpu):
+    """Up to 512 splits a row at every head size: 512 partial outputs of fp32 values, and no more for a larger number."""
+    for D in (64, 128, 256):
+        q, k, v, _ = make_qkv(D, 1, 1, 1, 1, 32768, D)
+        a = _lib.SdpaArgs()
+        need = []
+        for splits in (511, 512, 600):
+            ops._fill_common(a, q, k, v, 1.0, 32767, None, None, splits)
+            need.append(kvx.kvx_sdpa_decode_workspace_bytes(ctypes.byref(a)))
+        # splits are whole multiples of 64 keys: 511 are 256 of 128
+        assert need[1] == need[2] and need[1] - need[0] >= 256 * D * 4, need
+
+
 def test_full_size_prefill_properties(gpu):
     """Configuration 2 at its real shape (B1, 32/8 heads, D128, 32768 slots, 1024 queries, RoPE):
     one KV head against the oracle, row sums, and layout independence (scattered slots give the

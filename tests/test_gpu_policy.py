@@ -385,6 +385,34 @@ def test_fused_single_token_step_matches_the_separate_calls(gpu, decode_route, n
         assert torch.equal(fused._next_index, apart._next_index), f"step {i}"
 
 
+@pytest.mark.parametrize("name", ["h2o-default", "h2o-vlen-default", "qh2o-vlen-torch-quantized8"])
+def test_fused_single_token_step_over_more_than_256_splits(gpu, decode_route, name):
+    """The same over rows of 196700 slots of 16 heads of 64: more splits than the wavefronts' outputs hold weights of. The
+    sums over the row differ by their order, a few 2^-24 sqrt(L)."""
+    B, Hq, Hkv, D, L, chunk = 1, 16, 1, 64, 196700, 16
+    gen = torch.Generator(device=gpu).manual_seed(5)
+    q, k, v = (torch.randn(B, h, L + chunk + 2, D, generator=gen, device=gpu).to(torch.bfloat16) for h in (Hq, Hkv, Hkv))
+    v.mul_(torch.rand(B, Hkv, L + chunk + 2, 1, generator=gen, device=gpu).to(torch.bfloat16) + 0.5)
+    fused, apart = (create_kv_cache(name, KVCacheParams(B, Hkv, L, D, Hq), max_chunk_size=chunk, device=gpu) for _ in range(2))
+    for c in (fused, apart):
+        c.forward(q[:, :, :L], k[:, :, :L], v[:, :, :L])
+        c.forward(q[:, :, L : L + chunk], k[:, :, L : L + chunk], v[:, :, L : L + chunk])
+    rtol = 2.0 ** -22 * L ** 0.5
+    for i in range(L + chunk, L + chunk + 2):
+        new = tuple(t[:, :, i : i + 1] for t in (q, k, v))
+        apart.set_next_positions(fused._next_index[:, :, :1])
+        out = fused.forward(*new)
+        apart._write(apart._next_index_for(1), new[1], new[2], apart.input_pos)
+        apart._input_pos += 1
+        o_ref, w, _ = ops.decode_core(new[0], apart.k, apart.v, apart.scale_factor, return_weights=True, quant=apart._quant_state(L))
+        apart._update(w, 1, select=1)
+        for x, y in ((fused.k, apart.k), (fused.v, apart.v), (fused.token_pos, apart.token_pos)):
+            assert torch.equal(x, y)
+        torch.testing.assert_close(out.view(B, Hq, D).float(), o_ref.float(), rtol=2e-2, atol=1e-3)
+        torch.testing.assert_close(fused.scores, apart.scores, rtol=rtol, atol=1e-9)
+        assert torch.equal(fused._next_index[:, :, :1], apart._next_index[:, :, :1]), f"step {i}"
+
+
 @pytest.mark.parametrize("policy", ["h2o", "normalize", "vlen", "q_errors"])
 @pytest.mark.parametrize("B,Hkv,L,gp,k", [
     (1, 2, 100, 0, 7),         # one list, partly filled
