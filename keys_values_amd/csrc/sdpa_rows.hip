@@ -11,6 +11,8 @@
 // Whole calls, before -> after: 20 rows over 32 x 36928 keys of 128, 8-bit codes 214 -> 132 us, 4-bit 213 -> 110; 8 over 8 x 8192,
 // 8-bit 21.4 -> 17.3, plain 20.3 -> 16.1; 60 of 64 over 8 x 9000, 8-bit 22.4 -> 19.1; 64 of 256 over 4 x 10590, 8-bit 53 -> 41; 200 over
 // 8 x 2000, 8-bit 36 -> 25, plain 32 -> 22; 512 over 8 x 600, 8-bit 30 -> 24, plain 25 -> 21; 512 of 64 over 8 x 1024, plain 17.0 -> 15.1.
+#include <float.h>
+
 #include "key_blocks.h"
 #include "prefill_params.h"
 
@@ -18,7 +20,7 @@ namespace kvx {
 namespace {
 
 constexpr int WAVES = 4;
-constexpr float kNegBig = -1.0e30f;  // running maximum before the first visible key (finite: no inf - inf)
+constexpr float kNegBig = -FLT_MAX;  // running maximum before the first visible key: finite (no inf - inf), and below the logits of any key
 
 // Two workgroups per compute unit where the accumulators (NC D / 4 registers) leave room for two blocks in flight, else one: with 32
 // rows of 128 a bound of two spills the blocks of plain and 8-bit keys, 4-bit ones fit.

@@ -224,6 +224,19 @@ def test_attention_of_few_rows(gpu, dtype, store, B, Hq, Hkv, q_len, T, D, split
         torch.testing.assert_close(lse.cpu(), O.lse2(q, k, scale, pos, tp), rtol=1e-4, atol=1e-3)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D,splits", [(1, 4, 2, 9, 200, 64, 0), (2, 4, 1, 20, 333, 128, 3)])
+def test_attention_of_few_rows_whose_logits_lie_far_below_zero(gpu, B, Hq, Hkv, q_len, T, D, splits):
+    """Finite logits are weighed however low they are: all keys alike, q.k = -2^112 or so (a power of two, so that its scaling is
+    exact), the outputs are means of V. A mean of fewer than 2^9 rows in 16 bits: 2^-8 of the largest value."""
+    gen = torch.Generator().manual_seed(T)
+    v = torch.randn(B, Hkv, T, D, generator=gen).to(torch.bfloat16)
+    q, k = torch.full((B, Hq, q_len, D), 2.0 ** 53, dtype=torch.bfloat16), torch.full((B, Hkv, T, D), -(2.0 ** 53), dtype=torch.bfloat16)
+    out, _, lse = ops.prefill_core(q.to(gpu), k.to(gpu), v.to(gpu), 0.125, T - q_len, return_lse=True, output_transposed=False, num_splits=splits)
+    ref = torch.stack([v[:, :, : T - q_len + i + 1].double().mean(2) for i in range(q_len)], 2).repeat_interleave(Hq // Hkv, 1)
+    torch.testing.assert_close(out.double().cpu(), ref, rtol=2.0 ** -8, atol=2.0 ** -8)
+    torch.testing.assert_close(lse.double().cpu(), torch.full((B, q_len, Hq), -(2.0 ** 106) * D * 0.125 * math.log2(math.e), dtype=torch.float64), rtol=1e-6, atol=0)
+
+
 @pytest.mark.parametrize("scattered", [False, True])
 @pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D", [
     (1, 7, 1, 297, 600, 128),    # 2079 rows: 33 tiles of 63, all full
