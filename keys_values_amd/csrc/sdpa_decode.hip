@@ -91,7 +91,12 @@ Plan make_plan(const kvx_sdpa_args& a, bool fused_h2o) {
       // the call's at once. Through the scratch -> on the chip, us: one row of 16 heads over 197000 keys 37 -> 34, 393216
       // 50 -> 42, of 8 heads over 600000 61 -> 47; two rows of 16 heads over 197000 keys 41 -> 61, over 393216 68 -> 81, four
       // rows over 262144 8-bit keys 66 -> 115.
-      if (least <= WAVES * a.D || least * rows <= 2 * cus) n = max(least, in_rounds((least * rows + cus - 1) / cus));
+      // Rows whose logits fit the chip in no 512 splits go through the scratch anyway: one workgroup per compute unit, also for a
+      // single row, whose 128 splits would use half the device. 128 -> 256 splits, us: one row of 16 heads of 64 over 600000 keys
+      // 70 -> 66, over 1.5 M 155 -> 126, of 128 over 300000 62 -> 59, over 600000 108 -> 93, 8 of 128 over 950000 151 -> 118; 512
+      // splits: 83, 139, 76, 112, 136.
+      const bool fits = least <= kMaxSplits && (least <= WAVES * a.D || least * rows <= 2 * cus);
+      n = fits ? max(least, in_rounds((least * rows + cus - 1) / cus)) : max(n, in_rounds(1));
     }
     splits = (int)min(n, (int64_t)kMaxSplits);
   }

@@ -427,6 +427,20 @@ def test_decode_workspace_counts_the_splits_asked_for(kvx, gpu):
         assert need[1] == need[2] and need[1] - need[0] >= 256 * D * 4, need
 
 
+def test_decode_splits_of_long_rows_through_the_scratch(kvx, gpu):
+    """Logits that fit the chip in no 512 splits: as many splits as give every compute unit one workgroup, whatever the number of rows."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for Hq, Hkv, T, D in ((16, 1, 600000, 64), (16, 1, 270000, 128), (8, 1, 950000, 128), (32, 2, 600000, 64), (32, 2, 300000, 128)):
+        a = _lib.SdpaArgs()
+        need = []
+        for splits in (0, cus // Hkv):
+            a.B, a.Hq, a.Hkv, a.q_len, a.kv_len, a.D, a.input_pos, a.sm_scale, a.num_splits = 1, Hq, Hkv, 1, T, D, T - 1, 1.0, splits
+            a.q = a.k = a.v = a.w = 16  # for the size alone
+            a.q_stride_h = a.q_stride_t = a.k_stride_t = a.v_stride_t = D
+            need.append(kvx.kvx_sdpa_decode_workspace_bytes(ctypes.byref(a)))
+        assert need[0] == need[1] > 0, (Hq, Hkv, T, D)
+
+
 def test_full_size_prefill_properties(gpu):
     """Configuration 2 at its real shape (B1, 32/8 heads, D128, 32768 slots, 1024 queries, RoPE):
     one KV head against the oracle, row sums, and layout independence (scattered slots give the
