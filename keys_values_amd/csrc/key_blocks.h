@@ -89,10 +89,14 @@ struct KeyBlocks {
     qs_vec = vec;
   }
 
+  // The calls ask for slot, head and batch strides of whole 8 elements: rows of codes begin on 8 bytes, plain ones on 16. A wider load
+  // of codes says so (the same instruction: global loads of 16 bytes need no more than 4).
   template <typename T>
   __device__ __forceinline__ static T get(const void* p) {
-    if constexpr (NT) return __builtin_nontemporal_load((const T*)p);
-    else return *(const T*)p;
+    constexpr size_t ALIGN = U8 && sizeof(T) > 8 ? 8 : sizeof(T);
+    typedef T row_part __attribute__((aligned(ALIGN)));
+    if constexpr (NT) return __builtin_nontemporal_load((const row_part*)p);
+    else return *(const row_part*)p;
   }
   __device__ __forceinline__ void load_k(Rows& r, int gi, uint32_t off, int key) const {
     const uint8_t* row = kbase + off;

@@ -224,6 +224,34 @@ def test_attention_of_few_rows(gpu, dtype, store, B, Hq, Hkv, q_len, T, D, split
         torch.testing.assert_close(lse.cpu(), O.lse2(q, k, scale, pos, tp), rtol=1e-4, atol=1e-3)
 
 
+@pytest.mark.parametrize("q_len", [1, 9])
+@pytest.mark.parametrize("bits,D", [(8, 64), (8, 128), (8, 256), (4, 64), (4, 128), (4, 256)])
+def test_rows_of_codes_that_begin_on_8_bytes(gpu, bits, D, q_len):
+    # strides of whole 8 bytes are what the calls ask for: every other row of codes is not 16-byte aligned. The same bits as over
+    # adjacent rows.
+    B, Hq, Hkv, T = 1, 8, 2, 333
+    q, k, v, _ = make_qkv(60 + D, B, Hq, Hkv, q_len, T, D)
+    row = D * bits // 8
+    codes, wide, state = [], [], []
+    for x in (k, v):
+        c, s, z = O.quantize_rows(x.reshape(-1, D), bits)
+        c = (O.compress4(c) if bits == 4 else c).view(B, Hkv, T, row).to(gpu)
+        buf = torch.full((B, Hkv, T, row + 8), 255, dtype=torch.uint8, device=gpu)
+        buf[..., :row] = c
+        codes.append(c)
+        wide.append(buf[..., :row])
+        state += [s.view(B, Hkv, T).to(gpu), z.view(B, Hkv, T).to(gpu)]
+    quant = ops.QuantState(*state)
+    assert wide[0].stride(2) == row + 8
+    got = []
+    for kd, vd in (codes, wide):
+        if q_len == 1:
+            got.append(ops.decode_core(q.to(gpu), kd, vd, 0.1, return_weights=True, quant=quant))
+        else:
+            got.append(ops.prefill_core(q.to(gpu), kd, vd, 0.1, T - q_len, return_weights=True, quant=quant))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D,splits", [(1, 4, 2, 9, 200, 64, 0), (2, 4, 1, 20, 333, 128, 3)])
 def test_attention_of_few_rows_whose_logits_lie_far_below_zero(gpu, B, Hq, Hkv, q_len, T, D, splits):
     """Finite logits are weighed however low they are: all keys alike, q.k = -2^112 or so (a power of two, so that its scaling is
