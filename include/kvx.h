@@ -159,6 +159,11 @@ int kvx_sdpa_prefill_weights(const kvx_sdpa_args* args, void* stream);
 int kvx_sdpa_prefill_copying(const kvx_sdpa_args* args, void* stream);
 size_t kvx_sdpa_prefill_copying_workspace_bytes(const kvx_sdpa_args* args);
 
+/* Query rows (queries x heads of a KV head) that a workgroup of the attention kernel takes in kvx_sdpa_prefill, or with `copying` in
+ * kvx_sdpa_prefill_copying with all the workspace it asks for: 16 or 32 in the kernel for few rows or few keys, 128 or 256 in
+ * the tiled one. For tests and measurement, on the host alone; 0 for arguments that the calls refuse. No counterpart in the reference. */
+int kvx_sdpa_prefill_block_rows(const kvx_sdpa_args* args, int copying);
+
 /* Single-token decode (q_len == 1): O over the whole cache and, if args->w is set, the score-sums
  * W = (1/G) sum_g softmax_g. No mask: the new token is the newest
  * (keys_values/attention/flashinfer_wrapper.py:471-481, keys_values/attention/flashinfer_ops.py:250-275).

@@ -102,6 +102,7 @@ SYMBOLS = {
     "kvx_sdpa_prefill_workspace_bytes": (c_size_t, [POINTER(SdpaArgs)]),
     "kvx_sdpa_prefill_copying": (ctypes.c_int, [POINTER(SdpaArgs), c_void_p]),
     "kvx_sdpa_prefill_copying_workspace_bytes": (c_size_t, [POINTER(SdpaArgs)]),
+    "kvx_sdpa_prefill_block_rows": (ctypes.c_int, [POINTER(SdpaArgs), ctypes.c_int]),
     "kvx_score_sum": (ctypes.c_int, [POINTER(SdpaArgs), c_void_p]),
     "kvx_sdpa_prefill_weights": (ctypes.c_int, [POINTER(SdpaArgs), c_void_p]),
     "kvx_sdpa_decode": (ctypes.c_int, [POINTER(SdpaArgs), c_void_p]),

@@ -128,6 +128,11 @@ size_t kvx_sdpa_prefill_copying_workspace_bytes(const kvx_sdpa_args* a) {
   return sdpa_prefill_workspace(*a, true);
 }
 
+int kvx_sdpa_prefill_block_rows(const kvx_sdpa_args* a, int copying) {
+  if (check_sdpa_common(a, "kvx_sdpa_prefill_block_rows", false) != KVX_OK) return 0;
+  return sdpa_prefill_block_rows(*a, copying != 0);
+}
+
 static int prefill_checked(const kvx_sdpa_args* a, const char* who, bool weights, bool may_copy, hipStream_t st) {
   int rc = check_sdpa_common(a, who, true);
   if (rc != KVX_OK) return rc;

@@ -52,6 +52,7 @@ int launch_sdpa_prefill(const kvx_sdpa_args& a, bool may_copy, hipStream_t st, M
 // whether launch_score_sum takes the kernel that can combine the attention's partials in the same launch
 bool score_sum_combines(const kvx_sdpa_args& a);
 size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy);
+int sdpa_prefill_block_rows(const kvx_sdpa_args& a, bool may_copy);
 int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* rest = nullptr);
 size_t score_sum_workspace(const kvx_sdpa_args& a);
 int launch_sdpa_decode(const kvx_sdpa_args& a, const kvx_h2o_args* fused_h2o, hipStream_t st);

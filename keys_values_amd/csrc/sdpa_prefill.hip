@@ -739,7 +739,7 @@ int launch_t(PrefillParams& p, hipStream_t st, MergeParams* rest) {
       const int n = p.num_splits, last = p.m_blocks - (n - 1) * p.period;
       grid.y = (unsigned)(p.m_blocks + p.period * ((n - 1) * (n - 2) / 2) + last * (n - 1));
       grid.z = 1;
-      if (rest) {  // whoever combines the partials reads the (empty) ones of all splits
+      if (rest) {  // the score-sum jobs read the maxima and sums of all splits of a row (its outputs are combined from those it sees)
         grid.y = (unsigned)p.m_blocks;
         grid.z = (unsigned)n;
         p.period = 0;
@@ -808,6 +808,13 @@ static kvx_sdpa_args on_copy(const kvx_sdpa_args& a, void* rows) {
   c.k_stride_h = c.v_stride_h = (int64_t)a.kv_len * a.D;
   c.k_stride_b = c.v_stride_b = (int64_t)a.Hkv * a.kv_len * a.D;
   return c;
+}
+
+int sdpa_prefill_block_rows(const kvx_sdpa_args& a, bool may_copy) {
+  const kvx_sdpa_args c = may_copy && wants_copy(a) ? on_copy(a, nullptr) : prefill_block(a);
+  PrefillParams p;
+  fill_params(p, c);
+  return p.columns ? p.columns : 32 * nwaves(c.kv_dtype, c.D);
 }
 
 size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy) {

@@ -192,6 +192,7 @@ def test_random_arguments_are_answered_not_trusted(kvx):
         assert kvx.kvx_sdpa_decode_h2o(ctypes.byref(a), ctypes.byref(h), None) in codes
         for fn in (kvx.kvx_sdpa_prefill_workspace_bytes, kvx.kvx_sdpa_prefill_copying_workspace_bytes, kvx.kvx_sdpa_decode_workspace_bytes, kvx.kvx_sdpa_decode_h2o_workspace_bytes):
             assert fn(ctypes.byref(a)) >= 0
+        assert kvx.kvx_sdpa_prefill_block_rows(ctypes.byref(a), it & 4) in (0, 16, 32, 128, 256)
         assert kvx.kvx_h2o_update_select(ctypes.byref(h), None) in codes
         assert kvx.kvx_h2o_workspace_bytes(ctypes.byref(h)) >= 0
         assert kvx.kvx_cache_write(ctypes.byref(fill(_lib.CacheWriteArgs())), None) in codes

@@ -190,9 +190,25 @@ def test_score_sums_with_streamed_keys(gpu, store, B, Hq, Hkv, q_len, T, D, spli
     (2, 16, 2, 16, 640, 256, 0),     # 128 rows of 256, the most over codes
     (1, 32, 8, 75, 1000, 128, 0),    # 300 rows in splits
     (1, 8, 2, 384, 640, 128, 0),     # 1536 rows, as many as keys of them are new: most blocks are masked
-    (2, 16, 4, 260, 640, 128, 0),    # 1040 rows, above the line in every store: the tiled kernel
+    (2, 16, 4, 260, 640, 128, 0),    # 1040 rows: over plain rows above the line to the tiled kernel, over codes below it
+    (2, 16, 4, 260, 900, 128, 0),    # above it in every store
 ])
-def test_attention_of_few_rows(gpu, dtype, store, B, Hq, Hkv, q_len, T, D, splits):
+def test_attention_of_few_rows(kvx, gpu, dtype, store, B, Hq, Hkv, q_len, T, D, splits):
+    # plain rows of 256 values always take the tiled kernel
+    few = T != 900 and not (store == "plain" and (D == 256 or T == 640 and q_len == 260))
+    check_attention(kvx, gpu, dtype, store, B, Hq, Hkv, q_len, T, D, splits, few, False)
+
+
+def block_rows(kvx, q, k, v, input_pos, tp=None, quant=None, copying=False):
+    """query rows of a workgroup of the attention kernel: up to 32 in the one for few rows"""
+    a = _lib.SdpaArgs()
+    ops._fill_common(a, q, k, v, 1.0, input_pos, tp, quant, 0)
+    rows = kvx.kvx_sdpa_prefill_block_rows(ctypes.byref(a), copying)
+    assert rows in (16, 32, 128, 256)
+    return rows
+
+
+def check_attention(kvx, gpu, dtype, store, B, Hq, Hkv, q_len, T, D, splits, few_rows, fused_dequant):
     # dense, offset and scattered positions; rows, positions and row state on 4-element bounds and off them
     # tolerances of the path
     q, k, v, gen = make_qkv(510 + T, B, Hq, Hkv, q_len, T, D, dtype=dtype)
@@ -218,10 +234,62 @@ def test_attention_of_few_rows(gpu, dtype, store, B, Hq, Hkv, q_len, T, D, split
     for pos, tp, by in ((T - q_len, None, 0), (2 * T, scattered_positions(gen, B, Hkv, T, 2 * T, q_len), 0), (T, scattered_positions(gen, B, Hkv, T, T, q_len), 1)):
         move = (lambda x: x.to(gpu)) if by == 0 else (lambda x: shifted(x, by))
         o_ref, _ = O.sdpa_in_blocks(q, k, v, scale, pos, None if tp is None else tp.to(torch.int64))
-        out, _, lse = ops.prefill_core(q.to(gpu), move(kd), move(vd), scale, pos, None if tp is None else move(tp), return_lse=True, output_transposed=False,
-                                       quant=None if state is None else ops.QuantState(*(move(t) for t in state)), num_splits=splits)
+        qg, kg, vg, tpg, quant = q.to(gpu), move(kd), move(vd), None if tp is None else move(tp), None if state is None else ops.QuantState(*(move(t) for t in state))
+        assert (block_rows(kvx, qg, kg, vg, pos, tpg, quant, not fused_dequant) <= 32) == few_rows
+        out, _, lse = ops.prefill_core(qg, kg, vg, scale, pos, tpg, return_lse=True, output_transposed=False, quant=quant, num_splits=splits, fused_dequant=fused_dequant)
         check_o(out, o_ref)
         torch.testing.assert_close(lse.cpu(), O.lse2(q, k, scale, pos, tp), rtol=1e-4, atol=1e-3)
+
+
+@pytest.mark.parametrize("store", ["plain", "u8", "u4"])
+@pytest.mark.parametrize("dtype,B,Hq,Hkv,q_len,T,D,splits", [
+    (torch.bfloat16, 8, 48, 16, 27, 961, 64, 0),    # 81 rows of 3 heads; the last tile a single key
+    (torch.float16, 8, 48, 16, 27, 1023, 128, 0),   # one key short of whole tiles
+    (torch.bfloat16, 12, 128, 16, 60, 60, 64, 0),   # less than a tile of keys, all of them new
+    (torch.float16, 12, 128, 16, 50, 63, 128, 2),   # more splits than tiles
+    (torch.bfloat16, 4, 56, 8, 33, 1300, 128, 3),   # 231 rows of 7 heads, 21 tiles
+    (torch.float16, 4, 36, 4, 60, 1345, 64, 2),     # 540 rows of 9 heads, 22 tiles, the last one a single key
+    (torch.bfloat16, 8, 32, 32, 65, 511, 128, 3),   # 65 rows; the last split one tile shorter
+    (torch.float16, 1, 6, 2, 45, 700, 256, 0),      # 135 rows of 256, over codes the fewest
+])
+def test_attention_of_many_rows(kvx, gpu, store, dtype, B, Hq, Hkv, q_len, T, D, splits):
+    """The tiled kernel, over codes the form that dequantises for itself, above every line to the kernel for few rows."""
+    check_attention(kvx, gpu, dtype, store, B, Hq, Hkv, q_len, T, D, splits, False, True)
+
+
+@pytest.mark.parametrize("scattered", [False, True])
+@pytest.mark.parametrize("store,B,Hkv,T,D,most", [
+    # the most queries of 2 heads per KV head that take the kernel for few rows
+    ("plain", 2, 8, 1000, 128, 160), ("plain", 2, 8, 1000, 64, 256), ("plain", 100, 20, 40, 128, 8),
+    ("u8", 2, 8, 1000, 64, 320), ("u4", 2, 8, 1000, 64, 224), ("u8", 2, 8, 1000, 128, 192), ("u4", 2, 8, 1000, 128, 192),
+    ("u8", 4, 8, 8000, 128, 32), ("u4", 4, 8, 8000, 64, 32), ("u8", 2, 8, 1000, 256, 64), ("u4", 2, 8, 1000, 256, 64),
+])
+def test_both_sides_of_the_lines_between_the_attention_kernels(kvx, gpu, store, B, Hkv, T, D, most, scattered):
+    """Just below a line, and the same queries in a call with one more just above it. On each side the outputs are rounded to 8 bits and the
+    probabilities before, by up to 2^-9 either way: 2^-9 / sqrt(3) each in the mean square, four of them 2.3e-3 in the norm."""
+    gen = torch.Generator().manual_seed(T + D)
+    q = torch.randn(B, 2 * Hkv, most + 1, D, generator=gen).to(torch.bfloat16).to(gpu)
+    rows = [torch.randn(B, Hkv, T, D, generator=gen).to(torch.bfloat16).to(gpu) for _ in range(2)]
+    quant = None
+    if store != "plain":
+        bits, state = 8 if store == "u8" else 4, []
+        for i, x in enumerate(rows):
+            qz = RowQuantizer((B, Hkv, T, D), torch.bfloat16, bits, allocate_buffers=True, device=gpu)
+            qz.quantize(0, T, x)
+            rows[i] = qz.quant_buffer.view(B, Hkv, T, -1)
+            state += [qz.quant_scales.view(B, Hkv, T), qz.quant_zero_points.view(B, Hkv, T)]
+        quant = ops.QuantState(*state)
+    pos, tp = T - most - 1, None
+    if scattered:
+        pos, tp = 2 * T, scattered_positions(gen, B, Hkv, T, 2 * T, most + 1).to(gpu)
+    got = []
+    for n in (most, most + 1):
+        qn = q[:, :, :n]
+        assert (block_rows(kvx, qn, *rows, pos, tp, quant) <= 32) == (n == most)
+        got.append(ops.prefill_core(qn, *rows, D ** -0.5, pos, tp, return_lse=True, output_transposed=False, quant=quant, fused_dequant=True))
+    (below, _, lse), (above, _, lse_above) = got
+    assert rel_err(below.float(), above[:, :, :most].float()) < 4 * 2.3e-3
+    torch.testing.assert_close(lse, lse_above[:, :most], rtol=1e-5, atol=1e-4)
 
 
 @pytest.mark.parametrize("q_len", [1, 9])
@@ -870,3 +938,36 @@ def test_causal_first_chunk_in_splits(gpu, dtype, B, Hq, Hkv, q_len, behind, D):
     qc, kc, vc = q[:1, heads], k[:1, :1], v[:1, :1]
     check_o(out[:1, heads], O.sdpa_in_blocks(qc, kc, vc, scale, 0, None)[0])
     torch.testing.assert_close(lse[:1, :, heads].cpu(), O.lse2(qc, kc, scale, 0, None), rtol=1e-4, atol=1e-3)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D", [
+    (1, 4, 1, 256, 256, 256),
+    (1, 16, 16, 1024, 1024, 128),
+    (1, 16, 16, 1000, 1024, 64),   # keys that nobody sees behind the chunk
+    (1, 16, 8, 511, 1024, 128),    # 1022 rows
+])
+def test_causal_first_chunk_in_splits_with_weights(kvx, gpu, B, Hq, Hkv, q_len, T, D):
+    """Splits that the score-sum launch combines, in a workspace of NaN: what the attention kernel leaves unwritten is not used.
+    Tolerances of the path."""
+    q, k, v, _ = make_qkv(27 + T, B, Hq, Hkv, q_len, T, D)
+    scale = D ** -0.5
+    qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+    assert block_rows(kvx, qd, kd, vd, 0) >= 128
+    o_ref, w_ref = O.sdpa_in_blocks(q, k, v, scale, 0, None)
+    l_ref = O.lse2(q, k, scale, 0, None)
+    a = _lib.SdpaArgs()
+    ops._fill_common(a, qd, kd, vd, scale, 0, None, None, 0)
+    n = kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a))
+    rows = B * Hq * q_len * (D + 2) * 4
+    assert n >= 2 * rows and n % rows == 0  # splits, and no sums of the score-sum pass: it combines them
+    for call in (kvx.kvx_sdpa_prefill_weights, kvx.kvx_sdpa_prefill):
+        ws = torch.full((n // 4,), math.nan, device=gpu)
+        out, lse = torch.full_like(qd, math.nan), torch.full((B, q_len, Hq), math.nan, device=gpu)
+        w = torch.full((B, Hkv, T), math.nan, device=gpu)
+        a.o, a.lse, a.w, a.workspace, a.workspace_bytes = out.data_ptr(), lse.data_ptr(), w.data_ptr(), ws.data_ptr(), n
+        a.o_stride_b, a.o_stride_h, a.o_stride_t = out.stride(0), out.stride(1), out.stride(2)
+        _lib.check(call(ctypes.byref(a), _lib.stream_ptr(gpu)))
+        check_o(out, o_ref)
+        torch.testing.assert_close(lse.cpu(), l_ref, rtol=1e-4, atol=1e-3)
+        if call is kvx.kvx_sdpa_prefill_weights:
+            check_w(w, w_ref, q_len)
