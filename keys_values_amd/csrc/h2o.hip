@@ -529,7 +529,9 @@ __global__ __launch_bounds__(L) void list_sort_kernel(const kvx_h2o_args a, cons
 // Ranks of the keys of list c. `per` = ceil(k / C) keys of every list are at or below U, the largest of the lists'
 // per-th keys, so the first k keys of the row are all at or below U: about per of each list when the lists are alike.
 // Only those are ranked: a key's rank is its place in its list plus its places in the others, found by binary search in
-// the lists' heads (2^staged keys each, in LDS; in memory beyond them).
+// the lists' heads (2^staged keys each, in LDS; in memory beyond them, a latency a step). The list with the most keys at or below U has
+// about 2 per + 14 of them over many lists and rows, and one search beyond the heads is what the launch waits for: with heads of 2 per keys (16 at least),
+// sort and ranks of 256 of 8192 slots, 12 rows, 14.9 us, now 10.8; 16 of 4096 slots, 64 rows, 13.6, now 11.7.
 template <int L>
 __global__ __launch_bounds__(RANK_THREADS) void list_rank_kernel(const unsigned long long* __restrict__ lists, int C, int k, int per, int staged, int32_t* __restrict__ next) {
   __shared__ unsigned long long head[RANK_STAGED];
@@ -861,7 +863,7 @@ static void launch_sorted(const kvx_h2o_args& a, const SelectLists& sl, hipStrea
   if (sl.lists == 1) return;
   const int per = (a.k + sl.lists - 1) / sl.lists;
   int staged = 4;
-  while ((1 << staged) < 2 * per && (1 << staged) < L) ++staged;
+  while ((1 << staged) < 2 * per + 14 && (1 << staged) < L) ++staged;
   while (sl.lists << staged > RANK_STAGED) --staged;
   hipLaunchKernelGGL(list_rank_kernel<L>, grid, dim3(RANK_THREADS), 0, st, (const unsigned long long*)sl.keys, sl.lists, a.k, per, staged, a.next_index);
 }

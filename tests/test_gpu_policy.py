@@ -476,3 +476,22 @@ def test_selection_over_short_and_long_lists(kvx, gpu, B, Hkv, L, gp, k):
     for policy in ("h2o", "vlen", "q_errors"):
         test_selection_over_lists_matches_one_workgroup_per_row(kvx, gpu, B, Hkv, L, gp, k, policy)
     test_update_select_variants_direct(kvx, gpu, B, Hkv, L, L - gp, k, True, True, True)
+
+
+@pytest.mark.parametrize("k", [16, 17, 288, 289, 800, 801])  # 1, 2, 9, 10, 25, 26 keys a list of 32: heads of 16, 32, 32, 64, 64, 128
+@pytest.mark.parametrize("lists,full", [(32, 0), (32, 5), (8, 3)])
+def test_selection_ranks_beyond_the_heads(kvx, gpu, lists, full, k):
+    """All the slots to choose in one sorted list (its 16-slot blocks of a row of 8192 slots: 32 lists of 256 keys, or 8 of 1024), so that
+    far more of its keys are ranked than the heads in LDS hold. Values are distinct: the slots are those of a sort."""
+    gen = torch.Generator().manual_seed(lists + k)
+    L = 8192
+    scores = torch.randperm(2 * L, generator=gen)[: 2 * L].view(1, 2, L).float()
+    scores[..., (torch.arange(L) // 16) % lists != full] += 4.0 * L
+    sd, nxt = scores.to(gpu), torch.full((1, 2, k), -1, dtype=torch.int32, device=gpu)
+    a = _lib.H2OArgs()
+    a.B, a.Hkv, a.kv_len, a.limit, a.k, a.q_len = 1, 2, L, L, k, 5
+    a.scores, a.sc_stride_b, a.sc_stride_h, a.next_index = sd.data_ptr(), sd.stride(0), sd.stride(1), nxt.data_ptr()
+    ws = torch.empty(kvx.kvx_h2o_workspace_bytes(ctypes.byref(a)), dtype=torch.uint8, device=gpu)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+    _lib.check(kvx.kvx_h2o_update_select(ctypes.byref(a), _lib.stream_ptr(gpu)))
+    assert torch.equal(nxt.cpu().long(), scores.argsort(dim=-1)[..., :k])
