@@ -828,9 +828,13 @@ static size_t min_workspace(const kvx_h2o_args& a) { return best_bytes(a) + (a.q
 
 // Sorted lists for k > 1: taken while their number and size stay reasonable (256 lists of 1024 keys a row, 1 GiB), else
 // (and where the caller's workspace does not hold them) one workgroup per row. Lists of 256 keys sort in 36 steps, 3 of them through LDS,
-// where 1024 keys take 55 and 10 (6000 slots with errors 9.7 -> 6.4 us, plain 7.7 -> 5.0), but every candidate is looked up in four times as
-// many lists, which costs k times their number: sort and ranks of 128 of 30208 slots (118 lists) 14.8 us (1024 keys: 17.7), of 700 of
-// 12000 (47 lists) 16.5 (15.2), of 1024 of 16384 (64 lists) 22 (14.5), of 1000 of 32000 (125 lists) 25 (13.7).
+// where 1024 keys take 55 and 10, but every candidate is looked up in four times as many lists, by four times as many workgroups that
+// each read the heads of all. They pay while the device holds the workgroups side by side, three to a unit, and the look-ups, k times the
+// lists of all rows, are few for it. Whole choices, lists of 256 / of 1024, us: 16 of 8192 slots (32 lists), 24 rows 10.0 / 11.6, 32 rows 12.4 / 11.8;
+// 256 of 4096 (16 lists), 32 rows 10.3 / 12.3, 64 rows 14.3 / 12.5; 1000 of 4096, 24 rows 13.9 / 15.2, 48 rows 16.9 / 16.0; 1000 of 16384 (64 lists), 8 rows 14.3 / 15.9,
+// with new tokens in a run of slots 22 / 14.5.
+// Rows of up to 1024 slots are one list whatever k is: its sort ends the choice and hands nothing on (64 of 1000 slots, 32 rows: 9.9 us as
+// four lists, 7.2 as one; in the 128 KiB of the static entry point, too little for four lists of 32 rows, 14.1 and 7.2).
 struct ListPlan {
   int C;         // parts of LIST slots per row, 0: not this way
   int L, lists;  // keys of a sorted list, lists per row
@@ -842,7 +846,9 @@ static ListPlan list_plan(const kvx_h2o_args& a) {
   const int64_t C = ((int64_t)a.kv_len + LIST - 1) / LIST, rows = (int64_t)a.B * a.Hkv;
   if (C > 256 || rows * C * LIST * 8 > (1ll << 30)) return p;
   p.C = (int)C;
-  p.L = a.kv_len <= 32768 && (int64_t)a.k * ((a.kv_len + 255) / 256) <= 16384 ? 256 : LIST;
+  const int64_t n256 = (a.kv_len + 255) / 256, cus = num_cus();
+  const bool few = C > 1 && a.kv_len <= 32768 && rows * n256 <= 3 * cus && a.k * n256 <= 32768 && rows * a.k * n256 <= 2048 * cus;
+  p.L = n256 == 1 || few ? 256 : LIST;
   p.lists = (a.kv_len + p.L - 1) / p.L;
   const size_t n = (size_t)(rows * C);
   p.off_z = p.lists > 1 ? (size_t)rows * p.lists * p.L * 8 : 0;

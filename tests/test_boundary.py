@@ -280,3 +280,24 @@ def test_c_oracle_builds():
     from oracle import c_oracle
 
     assert os.path.exists(c_oracle.build())
+
+
+@pytest.mark.parametrize("rows,kv_len,k,keys", [
+    (32, 256, 200, 0),           # one list: its sort is the choice, no keys are handed on
+    (32, 257, 8, 0),
+    (32, 1024, 1000, 0),
+    (32, 1025, 8, 5 * 256),      # sorted lists of 256 keys
+    (24, 7936, 16, 31 * 256),    # three workgroups to each of 256 units
+    (25, 7936, 16, 8 * 1024),    # more of them: lists of 1024
+    (8, 7936, 1057, 31 * 256),
+    (8, 7936, 1058, 8 * 1024),   # too many look-ups for a row
+    (32, 3840, 1092, 15 * 256),
+    (32, 3840, 1093, 4 * 1024),  # for all rows
+])
+def test_workspace_of_a_choice_is_its_lists(kvx, rows, kv_len, k, keys):
+    """Which lists a row is sorted in, by the workspace that a choice asks for (on 256 compute units, what is assumed without a device):
+    the keys, 20 bytes of statistics for 1024 slots, rounded up to 16."""
+    a = _lib.H2OArgs()
+    a.B, a.Hkv, a.kv_len, a.limit, a.k = 1, rows, kv_len, kv_len, k
+    parts = rows * ((kv_len + 1023) // 1024)
+    assert kvx.kvx_h2o_workspace_bytes(ctypes.byref(a)) == rows * keys * 8 + (parts * 4 + 15) // 16 * 16 + parts * 16

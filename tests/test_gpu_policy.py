@@ -464,9 +464,16 @@ def test_selection_over_lists_matches_one_workgroup_per_row(kvx, gpu, B, Hkv, L,
 
 @pytest.mark.parametrize("B,Hkv,L,gp,k", [
     (2, 2, 256, 0, 256),       # one list of 256 keys, all of it chosen
-    (1, 3, 257, 1, 31),        # a second list of one slot, behind the limit
-    (1, 2, 4000, 15, 1024),    # lists of 256 at the line, 16 of them
-    (1, 2, 4000, 15, 1025),    # beyond it: lists of 1024
+    (1, 3, 257, 1, 31),        # one list of 1024 keys, as for every row of up to 1024 slots
+    (1, 3, 1025, 1, 31),       # a fifth list of one slot, behind the limit
+    (1, 2, 4000, 15, 1024),    # 16 lists of 256, half of the look-ups that they are taken for
+    (1, 2, 4000, 15, 1025),
+    (1, 1, 8192, 9, 1024),     # 32 lists of 256 at the line of a row's look-ups
+    (1, 1, 8192, 9, 1025),     # beyond it: lists of 1024
+    (16, 3, 4096, 0, 40),      # 48 rows of 16 lists of 256, three workgroups to each of 256 units
+    (7, 7, 4096, 0, 40),       # beyond: lists of 1024
+    (8, 4, 4096, 3, 1024),     # the line of all rows' look-ups
+    (8, 4, 4096, 3, 1025),
     (2, 2, 8192, 5, 200),      # the longest row whose norm the statistics add up
     (1, 2, 8193, 0, 100),      # a longer one
     (1, 1, 32768, 0, 64),      # 128 lists of 256
