@@ -262,27 +262,38 @@ namespace {
 
 // Splits of the keys for workgroups of `columns` rows. Every workgroup walks its share at the same pace, so the walk ends with the
 // most loaded compute unit: its rounds of 128 keys, and a second workgroup beside the first costs nine tenths of one more (it hides
-// latency only, the pipes are shared). The splits' merge is a launch, a chain over its splits and a read of their partials. The rates are
-// fits to calls of 2 to 1000 rows over 600 to 37000 keys: over codes a round takes 1.3 us at 16 rows of 128 (64: 0.9), half as much
-// again at 32. As many splits as fit two to a unit gave 29.5 us at 200 rows over 8 x 2000 4-bit keys, where this takes half as many: 22.9.
+// latency only, the pipes are shared). A workgroup's begin and end (first loads; the exchange in LDS) take a microsecond at 16 rows of 128, two at
+// 32. The splits' merge is a launch, a chain over its splits (32 are one pass) and a read of their partials. The rates are
+// fits to calls of 2 to 1200 rows over 64 to 12000 keys: over codes a round takes 1.3 us at 16 rows of 128 (64: 0.9), half as much
+// again at 32; the splits chosen take 1.0 % longer than the best of each call in the mean, without the workgroups' begin and end and
+// with twice as much for a split 2.0 %. As many splits as fit two to a unit gave 29.5 us at 200 rows over 8 x 2000 4-bit keys, where this takes half as many: 22.9.
 RowsPlan plan_of(const kvx_sdpa_args& a, int columns) {
-  const bool plain = kv_is_plain(a.kv_dtype), pairs = per_cu(a.D, columns / 16, kv_is_u4(a.kv_dtype)) == 2;
+  const bool plain = kv_is_plain(a.kv_dtype);
+  const int per_unit = per_cu(a.D, columns / 16, kv_is_u4(a.kv_dtype));
   const int64_t rows = (int64_t)a.q_len * (a.Hq / a.Hkv), cus = num_cus();
   const int64_t wgs = (int64_t)a.B * a.Hkv * ((rows + columns - 1) / columns), steps = (a.kv_len + 127) / 128;  // 32 keys a wavefront
   int64_t step_ns = a.D == 64 ? 900 : a.D == 128 ? 1300 : 2600;
   if (plain) step_ns = step_ns * 77 / 100;
   if (columns == 32) step_ns = step_ns * (a.D == 64 ? 135 : 150) / 100;
-  RowsPlan best = {columns, 1, INT64_MAX};
+  const int64_t ends_ns = (columns == 16 ? 1000 : 2000) * a.D / 128;
+  RowsPlan best = {0, 0, INT64_MAX};
+  int64_t best_per = 0;
   for (int64_t n = 1; n <= min(steps, (int64_t)64); ++n) {
     const int64_t per = (steps + n - 1) / n;
     if ((steps + per - 1) / per != n) continue;
     const int64_t c = (wgs * n + cus - 1) / cus;
-    const int64_t walk = per * step_ns * (pairs ? 180 * (c / 2) + 100 * (c % 2) : 100 * c) / 100;
-    const int64_t merge = n == 1 ? 0 : 2000 + 120 * n + n * a.B * a.Hq * a.q_len * (a.D * 4 + 8) / 4000;
-    if (walk + merge < best.ns) best = {columns, (int)n, walk + merge};
+    const int64_t walk = (per * step_ns + ends_ns) * (per_unit == 2 ? 180 * (c / 2) + 100 * (c % 2) : 100 * c) / 100;
+    const int64_t merge = n == 1 ? 0 : 2000 + 60 * n + (n > 32 ? 1000 : 0) + n * a.B * a.Hq * a.q_len * (a.D * 4 + 8) / 4000;
+    if (walk + merge < best.ns) {
+      best = {columns, (int)n, walk + merge};
+      best_per = per;
+    }
   }
-  const int64_t per = (steps + best.splits - 1) / best.splits;  // splits of whole steps, in tiles
-  best.splits = (int)(((a.kv_len + BN - 1) / BN + 2 * per - 1) / (2 * per));
+  // many short workgroups, fewer over a tile of keys: the tiled kernel (rows_plan)
+  const int64_t all = wgs * best.splits;
+  if (all > per_unit * cus && best_per <= (plain ? 3 : a.D == 256 ? 4 : 2)) return {0, 0, INT64_MAX};
+  if (a.kv_len <= BN && a.D <= 128 && all * (columns / 16) > cus) return {0, 0, INT64_MAX};
+  best.splits = (int)(((a.kv_len + BN - 1) / BN + 2 * best_per - 1) / (2 * best_per));  // splits of whole steps, in tiles
   return best;
 }
 
@@ -298,6 +309,12 @@ RowsPlan plan_of(const kvx_sdpa_args& a, int columns) {
 // most 64 rows over codes always (64 over 8 x 30000 65 -> 62, 64 of 64 over 8 x 60000 65 -> 51). Rows of 256: the accumulators of plain
 // keys' pipeline do not fit, over codes the tiled kernel is so slow that up to 128 rows win (128 over 4 x 15000 64 -> 50); above, a long call
 // goes over a copy of the store in 16-bit rows.
+// Many short workgroups stay there too (plan_of): one begins and ends with more than a step's work, so
+// where the device takes the workgroups in turns and each has up to three steps of 128 keys (over codes two, of 256 four) the tiled
+// kernel's few win: 133 rows over 256 x 64 plain keys of 128 9.4 there, 25.5 here; 279 over 64 x 254 12.2, 22.7; 198 over 64 x 219 12.1, 15.8;
+// 312 over 64 x 121 8-bit keys 13.8, 19.2; 66 of 256 over 128 x 512 8-bit keys 47.8, 53.8; but with four steps both take the same, and over codes three win by
+// 1.1 to 2.2 here. Over at most a tile of keys more workgroups than units are too many, half of that at 32 rows: 35 over
+// 128 x 64 5.2, 6.2.
 RowsPlan rows_plan(const kvx_sdpa_args& a) {
   const RowsPlan none = {0, 0, 0};
   const bool plain = kv_is_plain(a.kv_dtype);

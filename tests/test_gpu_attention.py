@@ -260,9 +260,11 @@ def test_attention_of_many_rows(kvx, gpu, store, dtype, B, Hq, Hkv, q_len, T, D,
 @pytest.mark.parametrize("scattered", [False, True])
 @pytest.mark.parametrize("store,B,Hkv,T,D,most", [
     # the most queries of 2 heads per KV head that take the kernel for few rows
-    ("plain", 2, 8, 1000, 128, 160), ("plain", 2, 8, 1000, 64, 256), ("plain", 100, 20, 40, 128, 8),
+    ("plain", 2, 8, 1000, 128, 160), ("plain", 2, 8, 1000, 64, 256), ("plain", 16, 16, 40, 128, 8),
     ("u8", 2, 8, 1000, 64, 320), ("u4", 2, 8, 1000, 64, 224), ("u8", 2, 8, 1000, 128, 192), ("u4", 2, 8, 1000, 128, 192),
     ("u8", 4, 8, 8000, 128, 32), ("u4", 4, 8, 8000, 64, 32), ("u8", 2, 8, 1000, 256, 64), ("u4", 2, 8, 1000, 256, 64),
+    # and few keys: as many workgroups as the units hold; over a tile of keys, one for each unit
+    ("plain", 4, 16, 250, 128, 64), ("plain", 4, 16, 250, 64, 128), ("u8", 8, 8, 250, 128, 64), ("u4", 8, 8, 250, 128, 128), ("plain", 8, 16, 64, 128, 16),
 ])
 def test_both_sides_of_the_lines_between_the_attention_kernels(kvx, gpu, store, B, Hkv, T, D, most, scattered):
     """Just below a line, and the same queries in a call with one more just above it. On each side the outputs are rounded to 8 bits and the
