@@ -34,7 +34,8 @@ struct RowsPlan {
   int columns, splits;
   int64_t ns;
 };
-RowsPlan rows_plan(const kvx_sdpa_args& a);
+// `combined`: the score-sum launch that follows combines the splits
+RowsPlan rows_plan(const kvx_sdpa_args& a, bool combined);
 int launch_sdpa_rows(const PrefillParams& p, int D, int kv, hipStream_t st);
 
 }  // namespace kvx

@@ -674,7 +674,7 @@ int causal_split_tiles(const kvx_sdpa_args& a, int bm, int m_blocks) {
   return best;
 }
 
-void fill_params(PrefillParams& p, const kvx_sdpa_args& a) {
+void fill_params(PrefillParams& p, const kvx_sdpa_args& a, bool combined = false) {
   p.q = (const uint16_t*)a.q;
   p.k = a.k;
   p.v = a.v;
@@ -694,7 +694,7 @@ void fill_params(PrefillParams& p, const kvx_sdpa_args& a) {
   p.R = a.q_len * p.G;
   p.input_pos = a.input_pos;
   p.num_tiles = (a.kv_len + BN - 1) / BN;
-  const RowsPlan rows = rows_plan(a);
+  const RowsPlan rows = rows_plan(a, combined);
   p.columns = rows.columns;
   const int bm = p.columns ? p.columns : 32 * nwaves(a.kv_dtype, a.D);
   p.m_blocks = (p.R + bm - 1) / bm;
@@ -820,9 +820,13 @@ int sdpa_prefill_block_rows(const kvx_sdpa_args& a, bool may_copy) {
 size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy) {
   PrefillParams p;
   const bool copy = may_copy && wants_copy(a);
-  fill_params(p, copy ? on_copy(a, nullptr) : prefill_block(a));
+  size_t partials = 0;
+  for (const bool combined : {false, true}) {
+    fill_params(p, copy ? on_copy(a, nullptr) : prefill_block(a), combined);
+    partials = max(partials, partial_bytes(p, a.D));
+  }
   // the score-sum pass that may follow on the same stream reuses the workspace for its partial sums
-  const size_t own = partial_bytes(p, a.D) + (copy ? copy_bytes(a) : 0), after = score_sum_workspace(a);
+  const size_t own = partials + (copy ? copy_bytes(a) : 0), after = score_sum_workspace(a);
   return own > after ? own : after;
 }
 
@@ -832,7 +836,7 @@ int launch_sdpa_prefill(const kvx_sdpa_args& a_in, bool may_copy, hipStream_t st
   if (may_copy && wants_copy(a)) {
     // a workspace too small for the copy (sized for another call, or by a caller that has no room): the fused form
     const kvx_sdpa_args c = on_copy(a, a.workspace);
-    fill_params(p, c);
+    fill_params(p, c, rest != nullptr);
     if (a.workspace && a.workspace_bytes >= copy_bytes(a) + partial_bytes(p, a.D)) {
       const int rc = launch_dequantize_kv(a, a.workspace, st);
       if (rc != KVX_OK) return rc;
@@ -841,7 +845,8 @@ int launch_sdpa_prefill(const kvx_sdpa_args& a_in, bool may_copy, hipStream_t st
       a.workspace_bytes = a_in.workspace_bytes - copy_bytes(a_in);
     }
   }
-  fill_params(p, a);
+  fill_params(p, a, rest != nullptr);
+  if (rest && (!a.workspace || a.workspace_bytes < partial_bytes(p, a.D))) fill_params(p, a);  // no room: the (fewer) splits of a call without weights
   const size_t need = partial_bytes(p, a.D);
   if (need) {
     KVX_REQUIRE(a.workspace && a.workspace_bytes >= need, KVX_ERR_WORKSPACE,

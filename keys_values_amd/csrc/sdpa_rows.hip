@@ -263,11 +263,13 @@ namespace {
 // Splits of the keys for workgroups of `columns` rows. Every workgroup walks its share at the same pace, so the walk ends with the
 // most loaded compute unit: its rounds of 128 keys, and a second workgroup beside the first costs nine tenths of one more (it hides
 // latency only, the pipes are shared). A workgroup's begin and end (first loads; the exchange in LDS) take a microsecond at 16 rows of 128, two at
-// 32. The splits' merge is a launch, a chain over its splits (32 are one pass) and a read of their partials. The rates are
+// 32. The splits' merge is a launch, a chain over its splits (32 are one pass) and a read of their partials; combined in a score-sum launch that
+// is there anyway they cost next to nothing, and one step a split is often the best (attention with weights of 8 rows over 4 x 3060 8-bit keys 14.6 us
+// in 12 splits, 12.6 in 24; 32 over 4 x 384 plain keys 13.1 in one, 11.7 in 3). The rates are
 // fits to calls of 2 to 1200 rows over 64 to 12000 keys: over codes a round takes 1.3 us at 16 rows of 128 (64: 0.9), half as much
 // again at 32; the splits chosen take 1.0 % longer than the best of each call in the mean, without the workgroups' begin and end and
 // with twice as much for a split 2.0 %. As many splits as fit two to a unit gave 29.5 us at 200 rows over 8 x 2000 4-bit keys, where this takes half as many: 22.9.
-RowsPlan plan_of(const kvx_sdpa_args& a, int columns) {
+RowsPlan plan_of(const kvx_sdpa_args& a, int columns, bool combined) {
   const bool plain = kv_is_plain(a.kv_dtype);
   const int per_unit = per_cu(a.D, columns / 16, kv_is_u4(a.kv_dtype));
   const int64_t rows = (int64_t)a.q_len * (a.Hq / a.Hkv), cus = num_cus();
@@ -283,7 +285,7 @@ RowsPlan plan_of(const kvx_sdpa_args& a, int columns) {
     if ((steps + per - 1) / per != n) continue;
     const int64_t c = (wgs * n + cus - 1) / cus;
     const int64_t walk = (per * step_ns + ends_ns) * (per_unit == 2 ? 180 * (c / 2) + 100 * (c % 2) : 100 * c) / 100;
-    const int64_t merge = n == 1 ? 0 : 2000 + 60 * n + (n > 32 ? 1000 : 0) + n * a.B * a.Hq * a.q_len * (a.D * 4 + 8) / 4000;
+    const int64_t merge = n == 1 ? 0 : (combined ? 300 + 30 * n : 2000 + 60 * n + (n > 32 ? 1000 : 0)) + n * a.B * a.Hq * a.q_len * (a.D * 4 + 8) / 4000;
     if (walk + merge < best.ns) {
       best = {columns, (int)n, walk + merge};
       best_per = per;
@@ -315,7 +317,7 @@ RowsPlan plan_of(const kvx_sdpa_args& a, int columns) {
 // 312 over 64 x 121 8-bit keys 13.8, 19.2; 66 of 256 over 128 x 512 8-bit keys 47.8, 53.8; but with four steps both take the same, and over codes three win by
 // 1.1 to 2.2 here. Over at most a tile of keys more workgroups than units are too many, half of that at 32 rows: 35 over
 // 128 x 64 5.2, 6.2.
-RowsPlan rows_plan(const kvx_sdpa_args& a) {
+RowsPlan rows_plan(const kvx_sdpa_args& a, bool combined) {
   const RowsPlan none = {0, 0, 0};
   const bool plain = kv_is_plain(a.kv_dtype);
   const int64_t rows = (int64_t)a.q_len * (a.Hq / a.Hkv), keys = (int64_t)a.B * a.Hkv * a.kv_len, es = plain ? 2 : 1;
@@ -326,9 +328,9 @@ RowsPlan rows_plan(const kvx_sdpa_args& a) {
   } else {
     if ((a.D == 256 && rows > 128) || (rows > 64 && work > (a.D == 64 ? (kv_is_u4(a.kv_dtype) ? 7 : 10) : a.D == 128 ? 6 : 8) * num_cus())) return none;
   }
-  const RowsPlan one = plan_of(a, 16);
+  const RowsPlan one = plan_of(a, 16, combined);
   if (rows <= 16) return one;
-  const RowsPlan two = plan_of(a, 32);
+  const RowsPlan two = plan_of(a, 32, combined);
   return one.ns < two.ns ? one : two;
 }
 

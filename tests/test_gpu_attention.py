@@ -973,3 +973,39 @@ def test_causal_first_chunk_in_splits_with_weights(kvx, gpu, B, Hq, Hkv, q_len, 
         torch.testing.assert_close(lse.cpu(), l_ref, rtol=1e-4, atol=1e-3)
         if call is kvx.kvx_sdpa_prefill_weights:
             check_w(w, w_ref, q_len)
+
+
+@pytest.mark.parametrize("room", [False, True])
+@pytest.mark.parametrize("store,Hq,Hkv,q_len,T,D", [
+    ("plain", 32, 2, 2, 384, 128),   # with room one split a step of keys, without it one split
+    ("plain", 16, 8, 72, 571, 64),
+    ("u8", 64, 8, 2, 235, 128),
+])
+def test_weights_of_few_rows_with_and_without_a_workspace(kvx, gpu, store, Hq, Hkv, q_len, T, D, room):
+    """Splits are nearly free where the score-sum launch combines them, and a call takes more of them if the workspace has room. Tolerances
+    of the path."""
+    q, k, v, _ = make_qkv(31 + T, 1, Hq, Hkv, q_len, T, D)
+    kd, vd, quant = k.to(gpu), v.to(gpu), None
+    if store == "u8":
+        (kc, ks, kz), (vc, vs, vz) = (O.quantize_rows(x.reshape(-1, D), 8) for x in (k, v))
+        k, v = (O.dequantize_rows(*t, torch.bfloat16).view(1, Hkv, T, D) for t in ((kc, ks, kz), (vc, vs, vz)))
+        kd, vd = kc.view(1, Hkv, T, D).to(gpu), vc.view(1, Hkv, T, D).to(gpu)
+        quant = ops.QuantState(*(t.view(1, Hkv, T).to(gpu) for t in (ks, kz, vs, vz)))
+    scale, pos, qd = D ** -0.5, T - q_len, q.to(gpu)
+    o_ref, w_ref = O.sdpa_in_blocks(q, k, v, scale, pos, None)
+    a = _lib.SdpaArgs()
+    ops._fill_common(a, qd, kd, vd, scale, pos, None, quant, 0)
+    n = kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a))
+    assert n > 0 and block_rows(kvx, qd, kd, vd, pos, None, quant) <= 32
+    ws = torch.full((n // 4,), math.nan, device=gpu)
+    out, lse = torch.full_like(qd, math.nan), torch.full((1, q_len, Hq), math.nan, device=gpu)
+    w = torch.full((1, Hkv, T), math.nan, device=gpu)
+    a.o, a.lse, a.w = out.data_ptr(), lse.data_ptr(), w.data_ptr()
+    a.o_stride_b, a.o_stride_h, a.o_stride_t = out.stride(0), out.stride(1), out.stride(2)
+    if room:
+        a.workspace, a.workspace_bytes = ws.data_ptr(), n
+    _lib.check(kvx.kvx_sdpa_prefill_weights(ctypes.byref(a), _lib.stream_ptr(gpu)))
+    check_o(out, o_ref)
+    check_w(w, w_ref, q_len)
+    torch.testing.assert_close(lse.cpu(), O.lse2(q, k, scale, pos, None), rtol=1e-4, atol=1e-3)
+    assert torch.isnan(ws).all().item() != room  # the splits' results lie there
