@@ -22,6 +22,7 @@
 #include <stddef.h>
 #include <string.h>
 
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -823,7 +824,7 @@ size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy) {
   size_t partials = 0;
   for (const bool combined : {false, true}) {
     fill_params(p, copy ? on_copy(a, nullptr) : prefill_block(a), combined);
-    partials = max(partials, partial_bytes(p, a.D));
+    partials = std::max(partials, partial_bytes(p, a.D));  // (max on the host is one of ints)
   }
   // the score-sum pass that may follow on the same stream reuses the workspace for its partial sums
   const size_t own = partials + (copy ? copy_bytes(a) : 0), after = score_sum_workspace(a);

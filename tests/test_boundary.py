@@ -301,3 +301,21 @@ def test_workspace_of_a_choice_is_its_lists(kvx, rows, kv_len, k, keys):
     a.B, a.Hkv, a.kv_len, a.limit, a.k = 1, rows, kv_len, kv_len, k
     parts = rows * ((kv_len + 1023) // 1024)
     assert kvx.kvx_h2o_workspace_bytes(ctypes.byref(a)) == rows * keys * 8 + (parts * 4 + 15) // 16 * 16 + parts * 16
+
+
+def _prefill_block(B, heads, kv_heads, q_len, kv_len, D, splits):
+    a = _lib.SdpaArgs()
+    a.B, a.Hq, a.Hkv, a.q_len, a.kv_len, a.D, a.num_splits = B, heads, kv_heads, q_len, kv_len, D, splits
+    a.kv_dtype, a.sm_scale = _lib.elem_kv_dtype(torch.bfloat16), 1.0
+    a.q = a.k = a.v = a.o = 4096
+    a.q_stride_b, a.q_stride_h, a.q_stride_t = heads * q_len * D, q_len * D, D
+    a.k_stride_b, a.k_stride_h, a.k_stride_t = kv_heads * kv_len * D, kv_len * D, D
+    a.v_stride_b, a.v_stride_h, a.v_stride_t = kv_heads * kv_len * D, kv_len * D, D
+    return a
+
+
+@pytest.mark.parametrize("B,heads,kv_heads,q_len,splits", [(1, 4, 2, 100, 2), (4, 64, 16, 1446, 6), (8, 64, 16, 4096, 3)])
+def test_workspace_of_splits_of_any_size(kvx, B, heads, kv_heads, q_len, splits):
+    # the second and third beyond 2^31 and 2^32 bytes
+    a = _prefill_block(B, heads, kv_heads, q_len, 8192, 256, splits)
+    assert kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a)) == splits * B * heads * q_len * (256 + 2) * 4
