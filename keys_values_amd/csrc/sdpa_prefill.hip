@@ -665,7 +665,7 @@ int causal_split_tiles(const kvx_sdpa_args& a, int bm, int m_blocks) {
     const int64_t jobs = groups * m_blocks * (s + 1) / 2, one = tps * tile_ns + job_ns;
     const int64_t sum = (seen * tile_ns + jobs * job_ns) * share / 100 / cus;
     const int64_t alone = pairs && jobs > cus && jobs <= 2 * cus ? one * 115 / 100 : one;  // all at once, two to most units
-    const int64_t walk = jobs <= cus ? one : max(alone, sum + (s == 1 ? 0 : one / 4));
+    const int64_t walk = jobs <= cus ? one : std::max(alone, sum + (s == 1 ? 0 : one / 4));  // (max on the host is one of ints)
     const int64_t merge = s == 1 ? 0 : 2000 + rows * (s + 1) / 2 * (a.D * 4 + 8) / 4000;
     if (walk + merge < best_ns) {
       best_ns = walk + merge;

@@ -319,3 +319,10 @@ def test_workspace_of_splits_of_any_size(kvx, B, heads, kv_heads, q_len, splits)
     # the second and third beyond 2^31 and 2^32 bytes
     a = _prefill_block(B, heads, kv_heads, q_len, 8192, 256, splits)
     assert kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a)) == splits * B * heads * q_len * (256 + 2) * 4
+
+
+@pytest.mark.parametrize("q_len", [400000, 600000, 700000, 1000000])
+def test_long_first_chunks_are_not_split(kvx, q_len):
+    # 32 heads fill the device: one split and no workspace, also where the estimates pass 2^31 ns
+    a = _prefill_block(1, 32, 8, q_len, q_len, 128, 0)
+    assert kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a)) == 0
