@@ -177,7 +177,8 @@ int kvx_sdpa_prefill_block_rows(const kvx_sdpa_args* args, int copying);
  * compute units for that long (about 30 ms at the defaults). Without args->w there is no wait where the splits of a row
  * do not fit the device side by side. The workspace holds the split partials, the rows' arrival counters and, with
  * args->w, room for the fp32 logits (B, Hq, kv_len) of the splits that are too long for the chip or whose wait ran out.
- * args->lse optional. */
+ * Counters and the splits' maxima and sums, which are waited for, are cleared by the call itself, in the launch ahead of the splits': the
+ * workspace may hold anything before. args->lse optional. */
 int kvx_sdpa_decode(const kvx_sdpa_args* args, void* stream);
 size_t kvx_sdpa_decode_workspace_bytes(const kvx_sdpa_args* args);
 

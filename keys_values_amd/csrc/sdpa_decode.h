@@ -56,7 +56,7 @@ struct DecodeParams {
   float* part_ml;  // (B, Hq, S, 2): maximum and sum of a split; one-launch form: zero until the split has published them
   // one-launch form (everything but logits that go through the scratch by plan):
   uint32_t* row_count;            // a line per (b, kvh) row: [kArrived] splits whose outputs (part_o) are there,
-                                  // [kFinished] splits that have chosen among their keys and read the row's outputs
+                                  // [kFinished] splits whose choice and split_pending are there (their reads of part_o may be on the way)
   unsigned long long* part_best;  // (B, Hkv, S): (value, slot) minimum of the split's keys (fused H2O form)
   float* part_vn;                 // (B, Hq, S): sum of |V row| 2^(logit - maximum) (scores weighted by the V norms)
   float* part_stats;              // (B, Hkv, S, 4): extremes of the compared value and of the quantisation errors

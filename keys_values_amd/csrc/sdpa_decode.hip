@@ -201,7 +201,7 @@ int decode_params(DecodeParams& p, const kvx_sdpa_args& a, const kvx_h2o_args* h
   return KVX_OK;
 }
 
-// The counters' reset (unless `counters_clear`: the slot write before did it, or there is a single split), then the kernels.
+// The reset of counters and of the splits' maxima and sums (unless `counters_clear`: the slot write before did it, or there is a single split), then the kernels.
 int launch_split(const DecodeParams& p, int D, int G, int kv, const kvx_h2o_args* hh, bool counters_clear, hipStream_t st) {
   const int rows = p.B * p.Hkv;
   const bool counts = p.one_launch ? p.num_splits > 1 && !counters_clear : hh != nullptr;

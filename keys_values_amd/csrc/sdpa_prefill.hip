@@ -642,12 +642,14 @@ int pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
 }
 
 // Splits of a causal first chunk (rows see the keys up to their own), by estimated time: tiles of a split, at whose bounds a block of rows
-// begins. Splits of all rows alike left units idle: the jobs differ in length, and those that see nothing still wrote and merged empty partials
-// (8 heads of 128 over 2, 4096 tokens: 4 splits 74 us, 3 57, 2 68). Here jobs without keys are not launched, a row merges the splits that it sees,
+// begins. Splits of all rows alike leave units idle: the jobs differ in length, those that see nothing still write and merge empty partials, and
+// the best number of splits varies from size to size (8 heads of 128 over 2, 4096 tokens: 4 splits 68.5 us, 3 53.1, 2 60.7, one 79.4; 2048 tokens: 4
+// 29.2, 3 31.1, 2 33.9, one 42.4). Here jobs without keys are not launched, a row merges the splits that it sees,
 // and the jobs run in the order of their length (causal_job), so the walk takes the sum of the tiles that are seen and the jobs' begin and
 // end, and a quarter of a split at the end; never less than one split, and more where two of them share a unit from the start. Calls of
-// 8 heads over 2 of 4096 tokens 67.7 -> 60.9 us, of 2048 39.1 -> 33.1; 4 over 1, 8000 tokens 106 -> 91; 16 of 64 over 4, 3000 51.1 -> 48.2; 8 of
-// 256 over 2, 3000 113 -> 83. Where the rows alone fill the device one split stays the best (32 over 8, 4096 tokens 148; two: 190).
+// 8 heads over 2 of 4096 tokens 66.3 -> 56.7 us, of 2048 34.3 -> 27.5; 4 over 1, 8000 tokens 99.6 -> 82.2; 16 of 64 over 4, 3000 45.5 -> 40.6; 8 of
+// 256 over 2, 3000 106.6 -> 74.4 (two splits of all rows alike are as good there, and at 4096 tokens three are better). Where the rows alone
+// fill the device one split stays the best (32 over 8, 4096 tokens 133; two: 168).
 int causal_split_tiles(const kvx_sdpa_args& a, int bm, int m_blocks) {
   const int G = a.Hq / a.Hkv, tiles = (a.q_len + BN - 1) / BN;
   const int64_t groups = (int64_t)a.B * a.Hkv, cus = num_cus(), rows = groups * G * a.q_len;

@@ -8,9 +8,10 @@
 // barriers in the loop; a block's operands are dequantised once and serve all the columns. The wavefronts' partial results meet in LDS
 // at the end. Bound by the read of K and V, and where that is short by latency: loads, a few blocks, the exchange, the merge.
 //
-// Whole calls, before -> after: 20 rows over 32 x 36928 keys of 128, 8-bit codes 214 -> 132 us, 4-bit 213 -> 110; 8 over 8 x 8192,
-// 8-bit 21.4 -> 17.3, plain 20.3 -> 16.1; 60 of 64 over 8 x 9000, 8-bit 22.4 -> 19.1; 64 of 256 over 4 x 10590, 8-bit 53 -> 41; 200 over
-// 8 x 2000, 8-bit 36 -> 25, plain 32 -> 22; 512 over 8 x 600, 8-bit 30 -> 24, plain 25 -> 21; 512 of 64 over 8 x 1024, plain 17.0 -> 15.1.
+// Attention without weights, calls in a row, in the tiled kernel -> here: 20 rows over 32 x 36928 keys of 128, 8-bit codes 176 -> 87 us, 4-bit
+// 176 -> 67; 8 over 8 x 8192, 8-bit 19.2 -> 11.8, plain 17.0 -> 10.4; 60 of 64 over 8 x 9000, 8-bit 19.5 -> 14.0; 64 of 256 over 4 x 10590, 8-bit
+// 40.6 -> 28.3; 200 over 8 x 2000, 8-bit 25.3 -> 18.5, plain 21.4 -> 14.8; 512 over 8 x 600, 8-bit 22.1 -> 11.4, plain 17.5 -> 9.1; 512 of 64 over
+// 8 x 1024, plain 14.5 -> 8.8.
 #include <float.h>
 
 #include "key_blocks.h"
@@ -268,7 +269,8 @@ namespace {
 // in 12 splits, 12.6 in 24; 32 over 4 x 384 plain keys 13.1 in one, 11.7 in 3). The rates are
 // fits to calls of 2 to 1200 rows over 64 to 12000 keys: over codes a round takes 1.3 us at 16 rows of 128 (64: 0.9), half as much
 // again at 32; the splits chosen take 1.0 % longer than the best of each call in the mean, without the workgroups' begin and end and
-// with twice as much for a split 2.0 %. As many splits as fit two to a unit gave 29.5 us at 200 rows over 8 x 2000 4-bit keys, where this takes half as many: 22.9.
+// with twice as much for a split 2.0 %. 200 rows over 8 x 2000 4-bit keys take 16.9 us in 4
+// splits, 23.1 in 2, 20.6 in 5, 19.4 in 8 and 26.6 in 16; 17 as chosen.
 RowsPlan plan_of(const kvx_sdpa_args& a, int columns, bool combined) {
   const bool plain = kv_is_plain(a.kv_dtype);
   const int per_unit = per_cu(a.D, columns / 16, kv_is_u4(a.kv_dtype));
