@@ -641,16 +641,23 @@ int pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
   return best;
 }
 
-// Splits of a causal first chunk (rows see the keys up to their own), by estimated time: tiles of a split, at whose bounds a block of rows
-// begins. Splits of all rows alike leave units idle: the jobs differ in length, those that see nothing still write and merge empty partials, and
+// Splits of a causal first chunk (rows see the keys up to their own), by estimated time: tiles of a split, and whether a block of rows begins
+// at the bounds of splits, for causal_job. Splits of all rows alike leave units idle: the jobs differ in length, those that see nothing still write and merge empty partials, and
 // the best number of splits varies from size to size (8 heads of 128 over 2, 4096 tokens: 4 splits 68.5 us, 3 53.1, 2 60.7, one 79.4; 2048 tokens: 4
 // 29.2, 3 31.1, 2 33.9, one 42.4). Here jobs without keys are not launched, a row merges the splits that it sees,
 // and the jobs run in the order of their length (causal_job), so the walk takes the sum of the tiles that are seen and the jobs' begin and
 // end, and a quarter of a split at the end; never less than one split, and more where two of them share a unit from the start. Calls of
 // 8 heads over 2 of 4096 tokens 66.3 -> 56.7 us, of 2048 34.3 -> 27.5; 4 over 1, 8000 tokens 99.6 -> 82.2; 16 of 64 over 4, 3000 45.5 -> 40.6; 8 of
 // 256 over 2, 3000 106.6 -> 74.4 (two splits of all rows alike are as good there, and at 4096 tokens three are better). Where the rows alone
-// fill the device one split stays the best (32 over 8, 4096 tokens 133; two: 168).
-int causal_split_tiles(const kvx_sdpa_args& a, int bm, int m_blocks) {
+// fill the device one split stays the best (32 over 8, 4096 tokens 133; two: 168). While a unit gets one job at most, splits of all rows alike can be
+// shorter (a tile where bounds of blocks are two apart: one head of 256, 380 tokens 18.6 us in splits of two tiles, 15.5 in splits of one). A merge of
+// their own counts as 4 us and 0.1 a split; as 2 us, the price in the score-sum launch (`combined`), splits were taken that one split beats: 24 heads of 256 over 8, 353 tokens 32.1 in three, 28.3 in one.
+// Of 260 calls of 100 to 8000 tokens the splits chosen take 1.1 % longer than the best in the mean.
+struct CausalSplits {
+  int tiles;
+  bool jobs;
+};
+CausalSplits causal_splits(const kvx_sdpa_args& a, int bm, int m_blocks, bool combined) {
   const int G = a.Hq / a.Hkv, tiles = (a.q_len + BN - 1) / BN;
   const int64_t groups = (int64_t)a.B * a.Hkv, cus = num_cus(), rows = groups * G * a.q_len;
   const int64_t tile_ns = a.D == 64 ? 700 : a.D == 128 ? 1130 : 2050, job_ns = 3000;
@@ -659,8 +666,18 @@ int causal_split_tiles(const kvx_sdpa_args& a, int bm, int m_blocks) {
   const int64_t seen = groups * m_blocks * (tiles + 1) / 2;
   int unit = 1;
   while (unit * BN * G % bm) unit *= 2;
-  int best = tiles;
+  auto merge_ns = [&](int s) { return combined ? 2000 : 4000 + 100 * s; };
+  CausalSplits best = {tiles, false};
   int64_t best_ns = INT64_MAX;
+  auto consider = [&](int tps, bool jobs, int64_t walk, int64_t merge) {
+    if (walk + merge >= best_ns) return;
+    best_ns = walk + merge;
+    best = {tps, jobs};
+  };
+  for (int s = 2; s <= min(16, tiles) && groups * m_blocks * s <= cus; ++s) {
+    const int tps = (tiles + s - 1) / s;
+    if ((tiles + tps - 1) / tps == s) consider(tps, false, tps * tile_ns + job_ns, merge_ns(s) + s * rows * (a.D * 4 + 8) / 4000);
+  }
   for (int s = 1; s <= min(16, tiles); ++s) {
     const int tps = s == 1 ? tiles : ((tiles + s - 1) / s + unit - 1) / unit * unit;
     if (s > 1 && (tps >= tiles || (int64_t)m_blocks * (s + 1) / 2 + m_blocks > 65535)) break;  // (jobs are a grid's second dimension)
@@ -668,11 +685,8 @@ int causal_split_tiles(const kvx_sdpa_args& a, int bm, int m_blocks) {
     const int64_t sum = (seen * tile_ns + jobs * job_ns) * share / 100 / cus;
     const int64_t alone = pairs && jobs > cus && jobs <= 2 * cus ? one * 115 / 100 : one;  // all at once, two to most units
     const int64_t walk = jobs <= cus ? one : std::max(alone, sum + (s == 1 ? 0 : one / 4));  // (max on the host is one of ints)
-    const int64_t merge = s == 1 ? 0 : 2000 + rows * (s + 1) / 2 * (a.D * 4 + 8) / 4000;
-    if (walk + merge < best_ns) {
-      best_ns = walk + merge;
-      best = tps;
-    }
+    const int64_t merge = s == 1 ? 0 : merge_ns(s) + rows * (s + 1) / 2 * (a.D * 4 + 8) / 4000;
+    consider(tps, s > 1, walk, merge);
   }
   return best;
 }
@@ -707,9 +721,10 @@ void fill_params(PrefillParams& p, const kvx_sdpa_args& a, bool combined = false
   p.period = 0;
   if (!a.token_positions && a.input_pos == 0 && a.q_len <= a.kv_len && kv_is_plain(a.kv_dtype) && a.num_splits <= 0 && !p.columns) {
     p.num_tiles = (a.q_len + BN - 1) / BN;  // nobody sees the keys behind
-    p.tiles_per_split = causal_split_tiles(a, bm, p.m_blocks);
+    const CausalSplits cs = causal_splits(a, bm, p.m_blocks, combined);
+    p.tiles_per_split = cs.tiles;
     p.num_splits = (p.num_tiles + p.tiles_per_split - 1) / p.tiles_per_split;
-    if (p.num_splits > 1) p.period = p.tiles_per_split * BN * p.G / bm;
+    if (cs.jobs) p.period = p.tiles_per_split * BN * p.G / bm;
   }
   p.c = a.sm_scale * kLog2e;
   p.q_sb = a.q_stride_b; p.q_sh = a.q_stride_h; p.q_st = a.q_stride_t;

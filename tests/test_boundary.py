@@ -326,3 +326,13 @@ def test_long_first_chunks_are_not_split(kvx, q_len):
     # 32 heads fill the device: one split and no workspace, also where the estimates pass 2^31 ns
     a = _prefill_block(1, 32, 8, q_len, q_len, 128, 0)
     assert kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a)) == 0
+
+
+@pytest.mark.parametrize("heads,kv_heads,q_len,splits", [
+    (1, 1, 380, 6),    # a unit has one job at most: a tile a split, whatever the bounds of row blocks
+    (6, 2, 209, 4),
+])
+def test_splits_of_short_first_chunks(kvx, heads, kv_heads, q_len, splits):
+    """By the workspace that the partial results ask for (on 256 compute units, what is assumed without a device)."""
+    a = _prefill_block(1, heads, kv_heads, q_len, q_len, 256, 0)
+    assert kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a)) == splits * heads * q_len * (256 + 2) * 4

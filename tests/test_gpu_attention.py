@@ -975,6 +975,31 @@ def test_causal_first_chunk_in_splits_with_weights(kvx, gpu, B, Hq, Hkv, q_len, 
             check_w(w, w_ref, q_len)
 
 
+@pytest.mark.parametrize("Hq,Hkv,q_len,splits", [
+    (1, 1, 380, 6),    # splits of a tile, for all rows alike
+    (24, 8, 353, 1),   # a merge that costs more than splits save
+    (24, 8, 196, 1),
+])
+def test_splits_of_short_first_chunks_without_weights(kvx, gpu, Hq, Hkv, q_len, splits):
+    # what is written of a workspace of NaN tells the splits: a maximum and a sum for every row in each. Tolerances of the path.
+    D, scale = 256, 0.0625
+    q, k, v, _ = make_qkv(q_len, 1, Hq, Hkv, q_len, q_len, D)
+    qd, kd, vd = q.to(gpu), k.to(gpu), v.to(gpu)
+    a = _lib.SdpaArgs()
+    ops._fill_common(a, qd, kd, vd, scale, 0, None, None, 0)
+    n = kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a))
+    ws, out = torch.full((n // 4,), math.nan, device=gpu), torch.full_like(qd, math.nan)
+    a.o, a.workspace, a.workspace_bytes = out.data_ptr(), ws.data_ptr(), n
+    a.o_stride_b, a.o_stride_h, a.o_stride_t = out.stride(0), out.stride(1), out.stride(2)
+    _lib.check(kvx.kvx_sdpa_prefill(ctypes.byref(a), _lib.stream_ptr(gpu)))
+    check_o(out, O.sdpa_in_blocks(q, k, v, scale, 0, None)[0])
+    rows = Hq * q_len
+    if splits == 1:
+        assert torch.isnan(ws).all()
+    else:
+        assert ws.numel() == splits * rows * (D + 2) and not torch.isnan(ws[splits * rows * D:]).any()
+
+
 @pytest.mark.parametrize("room", [False, True])
 @pytest.mark.parametrize("store,Hq,Hkv,q_len,T,D", [
     ("plain", 32, 2, 2, 384, 128),   # with room one split a step of keys, without it one split
