@@ -147,7 +147,9 @@ int kvx_score_sum(const kvx_sdpa_args* args, void* stream);
 /* kvx_sdpa_prefill followed by kvx_score_sum on the same stream: the whole
  * FlashInferSDPA._flashinfer_sdpa_fused_prefill step
  * (keys_values/attention/flashinfer_wrapper.py:476-494). args->lse must be given (it carries the
- * log-sum-exp between the two kernels); workspace as for kvx_sdpa_prefill. */
+ * log-sum-exp between the two kernels); workspace as for kvx_sdpa_prefill. Calls of few rows or keys are one launch where the
+ * workspace has the bytes that kvx_sdpa_prefill_workspace_bytes gives with args->w set; its workgroups wait for each other, boundedly
+ * (kvx_decode_tuning). */
 int kvx_sdpa_prefill_weights(const kvx_sdpa_args* args, void* stream);
 
 /* kvx_sdpa_prefill (args->w NULL) or kvx_sdpa_prefill_weights, for callers with memory to spare. Every workgroup of the
@@ -199,7 +201,8 @@ size_t kvx_sdpa_decode_h2o_workspace_bytes(const kvx_sdpa_args* args);
  * reference. resident: 0 sends every split's logits through the workspace and the tail kernel, 1 keeps them on the
  * chip where they fit (calls with weights only). spin_limit: polls a split spends waiting for the other splits of its row
  * before it leaves its share to the row's last one and its logits, if weights are wanted, to the workspace (0 = never
- * wait; clamped to 2^20; every call whose splits finish the row themselves, with weights or without). poll_sleep: pause between two polls in units of
+ * wait; clamped to 2^20; every call whose splits finish the row themselves, with weights or without, and chunks with weights that are one
+ * launch). poll_sleep: pause between two polls in units of
  * 512 cycles (clamped to 64). A negative value restores that switch to its default: the environment variables
  * KVX_DECODE_RESIDENT / KVX_DECODE_SPIN_LIMIT / KVX_DECODE_POLL_SLEEP as read once at the first decode call
  * (else 1, 32768, 4). A workspace size query and the call it is for must see the same setting of `resident`. */

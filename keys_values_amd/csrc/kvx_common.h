@@ -53,10 +53,15 @@ int launch_sdpa_prefill(const kvx_sdpa_args& a, bool may_copy, hipStream_t st, M
 bool score_sum_combines(const kvx_sdpa_args& a);
 size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy);
 int sdpa_prefill_block_rows(const kvx_sdpa_args& a, bool may_copy);
+bool wants_copy(const kvx_sdpa_args& a);  // whether a call over a quantised store that may copy goes over dequantised rows
+// attention with weights in one launch, where a workgroup holds the logits of its rows (sdpa_rows.hip); `done`: whether the call took it
+size_t rows_weights_workspace(const kvx_sdpa_args& a);
+int launch_rows_weights(const kvx_sdpa_args& a, hipStream_t st, bool& done);
 int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* rest = nullptr);
 size_t score_sum_workspace(const kvx_sdpa_args& a);
 int launch_sdpa_decode(const kvx_sdpa_args& a, const kvx_h2o_args* fused_h2o, hipStream_t st);
 size_t sdpa_decode_workspace(const kvx_sdpa_args& a, bool fused_h2o);
+void decode_wait(int& spin_limit, int& poll_sleep);  // how long a split waits for others
 void set_decode_tuning(int resident, int spin_limit, int poll_sleep);
 int launch_quantize_rows(const void* x, int64_t x_row_stride, int64_t rows, int D, int bits, bool f16, uint8_t* codes, float* scale,
                          int32_t* zp, hipStream_t st);

@@ -37,5 +37,6 @@ struct RowsPlan {
 // `combined`: the score-sum launch that follows combines the splits
 RowsPlan rows_plan(const kvx_sdpa_args& a, bool combined);
 int launch_sdpa_rows(const PrefillParams& p, int D, int kv, hipStream_t st);
+void common_params(PrefillParams& p, const kvx_sdpa_args& a);
 
 }  // namespace kvx

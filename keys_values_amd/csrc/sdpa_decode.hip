@@ -150,6 +150,11 @@ void set_decode_tuning(int resident, int spin_limit, int poll_sleep) {
   t.poll_sleep = poll_sleep < 0 ? t.env_sleep : clampi(poll_sleep, 0, kSleepMax);
 }
 
+void decode_wait(int& spin_limit, int& poll_sleep) {
+  spin_limit = tuning().spin_limit.load();
+  poll_sleep = tuning().poll_sleep.load();
+}
+
 namespace {
 int decode_params(DecodeParams& p, const kvx_sdpa_args& a, const kvx_h2o_args* hh, const Plan& pl) {
   KVX_REQUIRE(a.workspace && a.workspace_bytes >= pl.total, KVX_ERR_WORKSPACE,

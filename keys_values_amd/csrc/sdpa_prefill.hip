@@ -692,25 +692,7 @@ CausalSplits causal_splits(const kvx_sdpa_args& a, int bm, int m_blocks, bool co
 }
 
 void fill_params(PrefillParams& p, const kvx_sdpa_args& a, bool combined = false) {
-  p.q = (const uint16_t*)a.q;
-  p.k = a.k;
-  p.v = a.v;
-  p.k_scale = a.k_scale;
-  p.k_zp = a.k_zp;
-  p.v_scale = a.v_scale;
-  p.v_zp = a.v_zp;
-  p.tp = a.token_positions;
-  p.o = (uint16_t*)a.o;
-  p.lse = a.lse;
-  p.B = a.B;
-  p.Hq = a.Hq;
-  p.Hkv = a.Hkv;
-  p.G = a.Hq / a.Hkv;
-  p.q_len = a.q_len;
-  p.kv_len = a.kv_len;
-  p.R = a.q_len * p.G;
-  p.input_pos = a.input_pos;
-  p.num_tiles = (a.kv_len + BN - 1) / BN;
+  common_params(p, a);
   const RowsPlan rows = rows_plan(a, combined);
   p.columns = rows.columns;
   const int bm = p.columns ? p.columns : 32 * nwaves(a.kv_dtype, a.D);
@@ -718,7 +700,6 @@ void fill_params(PrefillParams& p, const kvx_sdpa_args& a, bool combined = false
   p.num_splits = a.num_splits > 0 ? min(a.num_splits, p.num_tiles) : p.columns ? rows.splits : pick_splits(a, p.m_blocks, p.num_tiles);
   p.tiles_per_split = (p.num_tiles + p.num_splits - 1) / p.num_splits;
   p.num_splits = (p.num_tiles + p.tiles_per_split - 1) / p.tiles_per_split;
-  p.period = 0;
   if (!a.token_positions && a.input_pos == 0 && a.q_len <= a.kv_len && kv_is_plain(a.kv_dtype) && a.num_splits <= 0 && !p.columns) {
     p.num_tiles = (a.q_len + BN - 1) / BN;  // nobody sees the keys behind
     const CausalSplits cs = causal_splits(a, bm, p.m_blocks, combined);
@@ -726,17 +707,6 @@ void fill_params(PrefillParams& p, const kvx_sdpa_args& a, bool combined = false
     p.num_splits = (p.num_tiles + p.tiles_per_split - 1) / p.tiles_per_split;
     if (cs.jobs) p.period = p.tiles_per_split * BN * p.G / bm;
   }
-  p.c = a.sm_scale * kLog2e;
-  p.q_sb = a.q_stride_b; p.q_sh = a.q_stride_h; p.q_st = a.q_stride_t;
-  p.k_sb = a.k_stride_b; p.k_sh = a.k_stride_h; p.k_st = a.k_stride_t;
-  p.v_sb = a.v_stride_b; p.v_sh = a.v_stride_h; p.v_st = a.v_stride_t;
-  p.o_sb = a.o_stride_b; p.o_sh = a.o_stride_h; p.o_st = a.o_stride_t;
-  p.qs_sb = a.qs_stride_b; p.qs_sh = a.qs_stride_h;
-  p.tp_sb = a.tp_stride_b; p.tp_sh = a.tp_stride_h;
-  p.qs_vec = (((uintptr_t)a.k_scale | (uintptr_t)a.k_zp | (uintptr_t)a.v_scale | (uintptr_t)a.v_zp) & 15) == 0 && a.qs_stride_b % 4 == 0 && a.qs_stride_h % 4 == 0;
-  p.tp_vec = ((uintptr_t)a.token_positions & 15) == 0 && a.tp_stride_b % 4 == 0 && a.tp_stride_h % 4 == 0;
-  p.part_o = nullptr;
-  p.part_ml = nullptr;
 }
 
 size_t partial_bytes(const PrefillParams& p, int D) {
@@ -792,6 +762,45 @@ int launch_t(PrefillParams& p, hipStream_t st, MergeParams* rest) {
 
 }  // namespace
 
+// Operands and sizes of a call, one split over all its keys.
+void common_params(PrefillParams& p, const kvx_sdpa_args& a) {
+  p.q = (const uint16_t*)a.q;
+  p.k = a.k;
+  p.v = a.v;
+  p.k_scale = a.k_scale;
+  p.k_zp = a.k_zp;
+  p.v_scale = a.v_scale;
+  p.v_zp = a.v_zp;
+  p.tp = a.token_positions;
+  p.o = (uint16_t*)a.o;
+  p.lse = a.lse;
+  p.B = a.B;
+  p.Hq = a.Hq;
+  p.Hkv = a.Hkv;
+  p.G = a.Hq / a.Hkv;
+  p.q_len = a.q_len;
+  p.kv_len = a.kv_len;
+  p.R = a.q_len * p.G;
+  p.input_pos = a.input_pos;
+  p.num_tiles = (a.kv_len + BN - 1) / BN;
+  p.num_splits = 1;
+  p.tiles_per_split = p.num_tiles;
+  p.m_blocks = 0;
+  p.period = 0;
+  p.columns = 0;
+  p.c = a.sm_scale * kLog2e;
+  p.q_sb = a.q_stride_b; p.q_sh = a.q_stride_h; p.q_st = a.q_stride_t;
+  p.k_sb = a.k_stride_b; p.k_sh = a.k_stride_h; p.k_st = a.k_stride_t;
+  p.v_sb = a.v_stride_b; p.v_sh = a.v_stride_h; p.v_st = a.v_stride_t;
+  p.o_sb = a.o_stride_b; p.o_sh = a.o_stride_h; p.o_st = a.o_stride_t;
+  p.qs_sb = a.qs_stride_b; p.qs_sh = a.qs_stride_h;
+  p.tp_sb = a.tp_stride_b; p.tp_sh = a.tp_stride_h;
+  p.qs_vec = (((uintptr_t)a.k_scale | (uintptr_t)a.k_zp | (uintptr_t)a.v_scale | (uintptr_t)a.v_zp) & 15) == 0 && a.qs_stride_b % 4 == 0 && a.qs_stride_h % 4 == 0;
+  p.tp_vec = ((uintptr_t)a.token_positions & 15) == 0 && a.tp_stride_b % 4 == 0 && a.tp_stride_h % 4 == 0;
+  p.part_o = nullptr;
+  p.part_ml = nullptr;
+}
+
 // Whether a call over a quantised store first dequantises the store into the workspace and then attends over plain rows.
 // Every workgroup of the attention kernel walks the whole store (of its split) and the dequantising one pays its vector work
 // each time, once per 256 rows; the copy pays it once, for one write and one more read of the 16-bit rows. Measured on
@@ -802,7 +811,7 @@ int launch_t(PrefillParams& p, hipStream_t st, MergeParams* rest) {
 // values the copy's launch is what counts (8 x 1500 of 128, 600 queries 28.2 -> 28.9). At head size 256 the
 // dequantising kernel runs 128 rows a workgroup out of its registers (4 x 4 heads, 541 x 7 queries over 5238: 890 us against
 // 26 + 340), and the copy pays from the second workgroup on.
-static bool wants_copy(const kvx_sdpa_args& a) {
+bool wants_copy(const kvx_sdpa_args& a) {
   if (kv_is_plain(a.kv_dtype) || (int64_t)a.B * a.Hkv > 65535) return false;  // pairs are a grid dimension of 16 bits
   const int64_t rows = (int64_t)a.q_len * (a.Hq / a.Hkv);
   if (a.D == 256) return rows > 128;
@@ -844,8 +853,8 @@ size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy) {
     partials = std::max(partials, partial_bytes(p, a.D));  // (max on the host is one of ints)
   }
   // the score-sum pass that may follow on the same stream reuses the workspace for its partial sums
-  const size_t own = partials + (copy ? copy_bytes(a) : 0), after = score_sum_workspace(a);
-  return own > after ? own : after;
+  const size_t own = partials + (copy ? copy_bytes(a) : 0);
+  return std::max({own, score_sum_workspace(a), a.w ? rows_weights_workspace(a) : 0});  // (max on the host is one of ints)
 }
 
 int launch_sdpa_prefill(const kvx_sdpa_args& a_in, bool may_copy, hipStream_t st, MergeParams* rest) {
