@@ -7,12 +7,13 @@ namespace kvx {
 
 struct MergeParams {
   const float* part_o;   // [split][group][R][D] fp32, unnormalised
-  const float* part_ml;  // [split][group][R][2]  (max in log2 units, sum)
+  const float* part_ml;  // [split][team][group][R][2]  (max in log2 units, sum)
   uint16_t* o;
   float* lse;  // (B, q_len, Hq) or NULL
   int32_t B, Hq, Hkv, G, q_len, R, num_splits;
   int64_t o_sb, o_sh, o_st;
   int32_t input_pos, split_keys;  // slots in position order: keys of a split; a row has no partial in splits behind its position. 0: all splits
+  int32_t teams;  // 1, or 2 where a split's partial is of two teams (relative to the larger of their maxima): the sums are added as if of two splits
 };
 
 // Combine the per-split partials of a row: D / 4 threads a row, each four values, times SC split classes that take
@@ -41,19 +42,20 @@ __device__ __forceinline__ void merge_job(const MergeParams& p, const int64_t bl
   const int64_t growc = live ? grow : total_rows - 1;
   const int S = p.split_keys ? min(p.num_splits, (p.input_pos + (int)(growc % p.R) / p.G) / p.split_keys + 1) : p.num_splits;
   const int dq = threadIdx.x % TPR, j = (threadIdx.x / TPR) % SC;
-  const f32x2_t* ml = (const f32x2_t*)p.part_ml + growc;  // (maximum, sum) of split s at s * total_rows
+  const f32x2_t* ml = (const f32x2_t*)p.part_ml + growc;  // (maximum, sum) of split s at s * teams * total_rows, of its second team behind it
   const float* po = p.part_o + growc * D + dq * 4;
   // the partials of splits s0, s0 + SC, ... (four at most), all asked for at once; nothing where there is no such split
-  f32x2_t m[4];
+  f32x2_t m[4], m2[4];
   f32x4_t x[4];
   auto load = [&](int s0) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      m[u] = f32x2_t{-INFINITY, 0.0f};
+      m[u] = m2[u] = f32x2_t{-INFINITY, 0.0f};
       x[u] = f32x4_t{0, 0, 0, 0};
       if (s0 + u * SC < S) {
         const int64_t at = (int64_t)(s0 + u * SC) * total_rows;
-        m[u] = ml[at];
+        m[u] = ml[at * p.teams];
+        if (p.teams > 1) m2[u] = ml[at * 2 + total_rows];
         x[u] = *(const f32x4_t*)(po + at * D);
       }
     }
@@ -61,12 +63,15 @@ __device__ __forceinline__ void merge_job(const MergeParams& p, const int64_t bl
   load(j);
   float M;
   if (SC == 1 && S <= 4) {
-    M = fmaxf(fmaxf(m[0][0], m[1][0]), fmaxf(m[2][0], m[3][0]));
+    M = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) M = fmaxf(M, fmaxf(m[u][0], m2[u][0]));
   } else {
     M = -INFINITY;
-    for (int s0 = 0; s0 < S; s0 += 4) {
+    const int n = S * p.teams;
+    for (int s0 = 0; s0 < n; s0 += 4) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) M = fmaxf(M, ml[(int64_t)min(s0 + u, S - 1) * total_rows][0]);
+      for (int u = 0; u < 4; ++u) M = fmaxf(M, ml[(int64_t)min(s0 + u, n - 1) * total_rows][0]);
     }
   }
   const float Mu = (M == -INFINITY) ? 0.0f : M;
@@ -77,9 +82,10 @@ __device__ __forceinline__ void merge_job(const MergeParams& p, const int64_t bl
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       if (s0 + u * SC < S) {
-        const float w = fast_exp2(m[u][0] - Mu);
+        const float w = fast_exp2(m[u][0] - Mu), w2 = fast_exp2(m2[u][0] - Mu);
         L += m[u][1] * w;
-        acc += x[u] * w;
+        L += m2[u][1] * w2;
+        acc += x[u] * fmaxf(w, w2);
       }
   }
   if constexpr (SC > 1) {

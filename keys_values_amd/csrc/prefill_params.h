@@ -18,10 +18,11 @@ struct PrefillParams {
   uint16_t* o;
   float* lse;
   float* part_o;   // [split][group][R][D] fp32, unnormalised
-  float* part_ml;  // [split][group][R][2]  (max in log2 units, sum)
+  float* part_ml;  // [split][team][group][R][2]  (max in log2 units, sum)
   int32_t B, Hq, Hkv, G, q_len, kv_len, R, input_pos;
   int32_t num_splits, tiles_per_split, num_tiles, m_blocks;
   int32_t period;  // a causal first chunk in splits: blocks of rows that a split's keys cover, 0: all splits of all rows
+  int32_t pair;    // two teams of a workgroup walk the halves of a split
   float c;  // sm_scale * log2(e)
   int64_t q_sb, q_sh, q_st, k_sb, k_sh, k_st, v_sb, v_sh, v_st, o_sb, o_sh, o_st;
   int64_t qs_sb, qs_sh, tp_sb, tp_sh;

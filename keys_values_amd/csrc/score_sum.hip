@@ -426,17 +426,17 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
 }
 
 // The base-2 log-sum-exps and positions of the rows of nblk blocks of 32, in LDS, by a workgroup of 256; rows past the end
-// weigh nothing. With KV splits (m.num_splits) from their (maximum, sum) pairs, else from p.lse. A pass over 16 splits is a memory
+// weigh nothing. With KV splits (m.num_splits > 1) from their (maximum, sum) pairs, else from p.lse. A pass over 16 splits is a memory
 // latency of 1 to 2 us; few rows share a row's splits out over up to eight neighbouring lanes.
 __device__ __forceinline__ void row_weights(const ScoreParams& p, const MergeParams& m, int b, int kvh, int nblk, float* lse_sh, int32_t* qpos_sh) {
   const float inv_G = 1.0f / (float)p.G;
-  const int S = m.num_splits, group = b * p.Hkv + kvh;
+  const int S = m.num_splits * m.teams, group = b * p.Hkv + kvh;
   const int64_t total_rows = (int64_t)p.B * p.Hkv * p.R;
   const int lt = nblk <= 1 ? 3 : nblk <= 2 ? 2 : nblk <= 4 ? 1 : 0, T = 1 << lt, part = threadIdx.x & (T - 1);
   for (int r = threadIdx.x >> lt; r < nblk * 32; r += 256 >> lt) {  // the lanes of a row leave the loop together
     const int rc = min(r, p.R - 1), qi = (int)(((float)rc + 0.5f) * inv_G);
     float lse;
-    if (S <= 1) {
+    if (m.num_splits <= 1) {
       lse = p.lse[((int64_t)b * p.q_len + qi) * p.Hq + kvh * p.G + (rc - qi * p.G)];
     } else {
       const f32x2_t* ml = (const f32x2_t*)m.part_ml + (int64_t)group * p.R + rc;

@@ -38,6 +38,7 @@ constexpr float kSlackLog2 = 8.0f;  // see the running-maximum update in the ker
 // two sizes run alike and the smaller one leaves more workgroups for short chunks. At head size 256 the
 // output accumulators (128 registers) leave no room for two wavefronts per SIMD: four for every store.
 constexpr int nwaves(int kv, int D) { return (kv_is_plain(kv) || D > 128) ? 4 : 8; }  // kv: enum kvx_kv_dtype
+constexpr bool pairs(int kv, int D) { return kv_is_plain(kv) && D <= 128; }  // two workgroups of a compute unit side by side
 
 // K and V tiles in LDS: [key][16-byte chunk], rows unpadded (D * 2 bytes), chunk c of row r stored at
 // position c ^ key(r). Unpadded rows are what the global -> LDS DMA writes (a wavefront fills 1024
@@ -280,15 +281,25 @@ __device__ __forceinline__ void causal_job(const PrefillParams& p, int job, int&
 }
 
 // PERIODS: jobs of a causal first chunk in splits (causal_job; decided at run time it cost every call 0.2 us)
-template <int D, int KV, bool PERIODS>
-__global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ? 2 : 1) void sdpa_prefill_kernel(const PrefillParams p) {
+// PAIR: two teams of four wavefronts walk the two halves of the split for the same rows, as two workgroups of a compute unit would, and combine
+// them in LDS: two splits' partials neither go through memory nor take a launch (pick_splits). The teams have barriers of their own: with the
+// workgroup's barrier each waits for the other at every tile (4096 rows of 128, 8 x 32768 keys 515 us; two workgroups 483 and the merge). A
+// wavefront arrives at its team's barrier, a word in LDS, with the last quarter of the second product still to issue and looks for the others
+// behind it: 483 -> 477, 8 x 16384 scattered keys 272 -> 266 (two workgroups and the merge 277).
+template <int D, int KV, bool PERIODS, bool PAIR>
+__global__ __launch_bounds__(64 * nwaves(KV, D) * (PAIR ? 2 : 1), (kv_is_plain(KV) && D <= 128) ? 2 : 1) void sdpa_prefill_kernel(const PrefillParams p) {
+  static_assert(!PAIR || (pairs(KV, D) && !PERIODS), "two teams fit a compute unit");
   constexpr bool F16 = kv_elem_f16(KV);  // element type of q, k, v, o
   constexpr int BM = 32 * nwaves(KV, D);  // rows per workgroup
   constexpr int CPR = D / 8;
   constexpr int KS = D / 16;  // k-steps of the first product
   constexpr int DT = D / 32;  // d tiles of the second product
-  __shared__ Smem<D> sm;
-  const int tid = threadIdx.x;
+  constexpr int TEAM = 64 * nwaves(KV, D);
+  __shared__ Smem<D> sms[PAIR ? 2 : 1];
+  const int team = PAIR ? __builtin_amdgcn_readfirstlane(threadIdx.x / TEAM) : 0;
+  Smem<D>& sm = sms[team];
+  __shared__ uint32_t arrivals[PAIR ? 2 : 1][4];
+  const int tid = PAIR ? threadIdx.x % TEAM : threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int n = lane & 31;  // row (query) owned by this lane within the wavefront's 32 rows
@@ -340,7 +351,7 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
     va[dt] = (uint32_t)((vrow * CPR + (c ^ swz_v<CPR>(vrow))) * 16 + (vcol & 7) * 2);
   }
 
-  const int tile_begin = split * p.tiles_per_split;
+  int tile_begin = split * p.tiles_per_split;
   int tile_end = min(tile_begin + p.tiles_per_split, p.num_tiles);
   if (!p.tp) {
     // slots hold positions 0, 1, 2, ...: tiles past the last position any row of this workgroup may
@@ -349,7 +360,7 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
     tile_end = min(tile_end, qpos_max / BN + 1);
     if (tile_end <= tile_begin) {  // whole split invisible (only with num_splits > 1): its output is not read
       if (row_ok) {
-        const int64_t prow = ((int64_t)split * p.B * p.Hkv + group) * p.R + row;
+        const int64_t prow = ((int64_t)(PAIR ? 2 * split + team : split) * p.B * p.Hkv + group) * p.R + row;
         if (h == 0) {
           p.part_ml[prow * 2] = -INFINITY;
           p.part_ml[prow * 2 + 1] = 0.0f;
@@ -358,6 +369,13 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
       return;
     }
   }
+  // The teams' halves are those of a whole split, as if each were a split of its own; the second team may be left without a tile
+  if constexpr (PAIR) {
+    const int half = tile_begin + (p.tiles_per_split + 1) / 2;
+    if (team == 0) tile_end = min(tile_end, half);
+    else tile_begin = min(half, tile_end);
+  }
+  const int mine = tile_end - tile_begin;
 
   f32x16_t o[DT];
 #pragma unroll
@@ -423,6 +441,16 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
       o[dt] = mfma_32x32x16<F16>(u32x4_t{lo[0], lo[1], hi[0], hi[1]}, pf, o[dt]);
     }
   };
+  auto v_operand = [&](int buf, int i) {
+    const int mt = i / (2 * DT), j = (i / DT) % 2, dt = i % DT;
+    const lds_ptr_t v = (lds_ptr_t)((const char*)&sm.v[buf][0][0] + va[dt]) + (32 * mt + 16 * j) * CPR * 16;
+    const u32x2_t lo = lds_read_tr16(v), hi = lds_read_tr16(v + 8 * CPR * 16);
+    return u32x4_t{lo[0], lo[1], hi[0], hi[1]};
+  };
+  auto pv_one = [&](const uint32_t (&pb)[2][8], int i, u32x4_t v) {
+    const int mt = i / (2 * DT), j = (i / DT) % 2, dt = i % DT;
+    o[dt] = mfma_32x32x16<F16>(v, u32x4_t{pb[mt][4 * j], pb[mt][4 * j + 1], pb[mt][4 * j + 2], pb[mt][4 * j + 3]}, o[dt]);
+  };
   auto pv = [&](const uint32_t (&pb)[2][8], int buf) {
     pv_part(pb, buf, std::integral_constant<int, 0>{}, std::integral_constant<int, 4 * DT>{});
   };
@@ -438,12 +466,37 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
   Loader<D, KV> ld;
   ld.init(p, sm, b, kvh, tid);
   uint32_t pbs[2][2][8];  // packed P of the tile in buffer 0 / 1: written by one step, multiplied by the next
+  // The team's barrier: how often each of its wavefronts has arrived. All eight wavefronts of a workgroup are resident, and each arrives once a
+  // tile whatever the other team does, so a wait ends.
+  uint32_t due = 0;
+  if constexpr (PAIR) {
+    if (threadIdx.x < 8) arrivals[threadIdx.x >> 2][threadIdx.x & 3] = 0;
+    __syncthreads();
+  }
+  auto arrive = [&] {
+    if constexpr (PAIR) {
+      ++due;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      __hip_atomic_store(&arrivals[team][wave], due, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+  };
+  auto sync = [&] {
+    if constexpr (PAIR) {
+      while (__any(__hip_atomic_load(&arrivals[team][lane & 3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < due)) {
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    } else {
+      __syncthreads();
+    }
+  };
   // every split owns at least one tile (the host sizes the splits that way)
-  ld.template issue_one<true>(sm, tile_begin, 0, tid);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the first K tile and the Q fragments have arrived
-  ld.template land<true>(sm, tile_begin, 0, tid);
-  __syncthreads();
-  // one pipeline step; the first one has no previous tile to multiply
+  if (!PAIR || mine > 0) {
+    ld.template issue_one<true>(sm, tile_begin, 0, tid);
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the first K tile and the Q fragments have arrived
+    ld.template land<true>(sm, tile_begin, 0, tid);
+    arrive();
+    sync();
+  }
   // one pipeline step on the tile in buffer CUR (compile time: LDS offsets become immediates and P
   // alternates between two register sets instead of being copied)
   auto step = [&](auto first_tag, auto cur_tag, auto steady_tag, int t) {
@@ -461,6 +514,18 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
       ld.template issue_one<false>(sm, t, cur, tid);
       if (has1) ld.template issue_one<true>(sm, t + 1, cur ^ 1, tid);
     }
+    // publish the tiles that were in flight
+    auto publish = [&] {
+      __builtin_amdgcn_s_setprio(3);
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's DMA / loads have landed
+      if constexpr (STEADY) {
+        ld.land_steady(sm, t + 1, cur ^ 1, tid);
+      } else {
+        ld.template land<false>(sm, t, cur, tid);
+        if (has1) ld.template land<true>(sm, t + 1, cur ^ 1, tid);
+      }
+      arrive();
+    };
     f32x16_t s[2];
     // Issue priority rises through the tile (0 for the first product, 1 for the dependent chain mask ->
     // maximum -> rescaling decision, 2 for the exponentials beside the second product, 3 for the way to the
@@ -492,30 +557,33 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
     }
     // ---- O += V(t-1) P(t-1) on the matrix cores, P(t) = exp2(c S(t) - c m) on the vector ALU ----
     __builtin_amdgcn_s_setprio(2);
-    if constexpr (!FIRST) pv_part(pb_prev, cur ^ 1, std::integral_constant<int, NPRE>{}, std::integral_constant<int, 4 * DT - NPRE>{});
+    // PAIR: the last quarter of it comes behind the arrival at the team's barrier
+    constexpr int NREST = 4 * DT - NPRE, NLAST = PAIR && !FIRST ? NREST / 4 : 0;
+    if constexpr (!FIRST) pv_part(pb_prev, cur ^ 1, std::integral_constant<int, NPRE>{}, std::integral_constant<int, NREST - NLAST>{});
     const float mc = (m == -INFINITY) ? 0.0f : m * p.c;
     float rs0 = 0.0f, rs1 = 0.0f;
+    auto weigh = [&](int mt, int i0, int i1) {
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-      for (int i = 0; i < 16; i += 2) {
+      for (int i = i0; i < i1; i += 2) {
         const float p0 = fast_exp2(fmaf(s[mt][i], p.c, -mc));
         const float p1 = fast_exp2(fmaf(s[mt][i + 1], p.c, -mc));
         rs0 += p0;
         rs1 += p1;
         pb[mt][i >> 1] = pack_pair<F16>(p0, p1);
       }
-    l += rs0 + rs1;
+    };
+    weigh(0, 0, 16);
+    weigh(1, 0, NLAST ? 8 : 16);
+    if constexpr (NLAST == 0) l += rs0 + rs1;
     if constexpr (!FIRST) {
       // interleave in the instruction stream: each matrix instruction of the second product is
       // followed by the two LDS reads of the next one and by its share of the softmax arithmetic,
       // so the vector ALU works in the shadow of the matrix core instead of after it
       __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // operands of the first two go out ahead
-      constexpr int NREST = 4 * DT - NPRE;
       constexpr int NV = (80 + NREST - 1) / NREST;  // VALU per matrix instruction: 80 per tile (fma, add, cvt)
       constexpr int NX = (32 + NREST - 1) / NREST;  // transcendental: 32 exp2 per tile
 #pragma unroll
-      for (int i = 0; i < NREST; ++i) {
+      for (int i = 0; i < NREST - NLAST; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // 1 MFMA
         __builtin_amdgcn_sched_group_barrier(0x002, (NV + 1) / 2, 0);  // half of its vector work,
         __builtin_amdgcn_sched_group_barrier(0x400, (NX + 1) / 2, 0);
@@ -528,8 +596,28 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-        for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(pb[mt][i]));
+        for (int i = 0; i < (NLAST && mt == 1 ? 4 : 8); ++i) asm volatile("" : "+v"(pb[mt][i]));
       asm volatile("" : "+v"(l));
+      if constexpr (NLAST > 0) {
+        u32x4_t vl[NLAST];
+#pragma unroll
+        for (int i = 0; i < NLAST; ++i) vl[i] = v_operand(cur ^ 1, 4 * DT - NLAST + i);
+        publish();
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < NLAST; ++i) pv_one(pb_prev, 4 * DT - NLAST + i, vl[i]);
+        weigh(1, 8, 16);
+        l += rs0 + rs1;
+#pragma unroll
+        for (int i = 0; i < NLAST; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, (20 + NLAST - 1) / NLAST, 0);
+          __builtin_amdgcn_sched_group_barrier(0x400, (8 + NLAST - 1) / NLAST, 0);
+        }
+#pragma unroll
+        for (int i = 4; i < 8; ++i) asm volatile("" : "+v"(pb[1][i]));
+        asm volatile("" : "+v"(l));
+      }
       if (resc) {  // O (now including tile t-1) moves to the new reference maximum
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
@@ -537,42 +625,88 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
           for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
       }
     }
-    // ---- publish the tiles that were in flight -------------------------------------------------
-    __builtin_amdgcn_s_setprio(3);
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's DMA / loads have landed
-    if constexpr (STEADY) {
-      ld.land_steady(sm, t + 1, cur ^ 1, tid);
-    } else {
-      ld.template land<false>(sm, t, cur, tid);
-      if (has1) ld.template land<true>(sm, t + 1, cur ^ 1, tid);
-    }
-    __syncthreads();
+    if constexpr (NLAST == 0) publish();
+    sync();
   };
   constexpr std::integral_constant<int, 0> B0{};
   constexpr std::integral_constant<int, 1> B1{};
   constexpr std::true_type YES{};
   constexpr std::false_type NO{};
-  step(YES, B0, NO, tile_begin);
-  int t = tile_begin + 1;
-  // tiles whose successor is a full tile of this walk take the step without bounds checks
-  const int steady_end = min(tile_end - 1, p.kv_len / BN - 1);  // t < steady_end: tiles t, t + 1 full, t + 1 < tile_end
-  for (; t + 1 < steady_end; t += 2) {
-    step(NO, B1, YES, t);
-    step(NO, B0, YES, t + 1);
-  }
-  for (; t + 1 < tile_end; t += 2) {
-    step(NO, B1, NO, t);
-    step(NO, B0, NO, t + 1);
-  }
-  if (t < tile_end) {
-    step(NO, B1, NO, t);
-    pv(pbs[1], 1);
-  } else {
-    pv(pbs[0], 0);
+  if (!PAIR || mine > 0) {
+    step(YES, B0, NO, tile_begin);
+    int t = tile_begin + 1;
+    // tiles whose successor is a full tile of this walk take the step without bounds checks
+    const int steady_end = min(tile_end - 1, p.kv_len / BN - 1);  // t < steady_end: tiles t, t + 1 full, t + 1 < tile_end
+    for (; t + 1 < steady_end; t += 2) {
+      step(NO, B1, YES, t);
+      step(NO, B0, YES, t + 1);
+    }
+    for (; t + 1 < tile_end; t += 2) {
+      step(NO, B1, NO, t);
+      step(NO, B0, NO, t + 1);
+    }
+    if (t < tile_end) {
+      step(NO, B1, NO, t);
+      pv(pbs[1], 1);
+    } else {
+      pv(pbs[0], 0);
+    }
   }
 
   // ---- epilogue -----------------------------------------------------------------------------
   const float lt = sum_halves(l);
+  if constexpr (PAIR) {
+    // Each team completes half of the columns. The tiles' place holds what the other one needs: [register quad][thread], and behind it the
+    // rows' maxima and sums. Products and sums are those of the combining launch, and where more splits follow the row's sum is left to it: maxima and
+    // sums of both teams, as of two splits, so that the log-sum-exp does not depend on who walks a split.
+    constexpr int HALF = DT / 2;
+    const float mr = m * p.c;
+    __syncthreads();  // the tiles have been multiplied
+    f32x4_t* mail = (f32x4_t*)&sms[team];
+    f32x2_t* stat = (f32x2_t*)(mail + 4 * HALF * TEAM);
+    const f32x4_t* from = (const f32x4_t*)&sms[team ^ 1];
+    const f32x2_t* from_stat = (const f32x2_t*)(from + 4 * HALF * TEAM);
+    auto send = [&](auto first_tag) {
+      constexpr int FIRST = decltype(first_tag)::value;
+#pragma unroll
+      for (int i = 0; i < 4 * HALF; ++i) {
+        const f32x16_t& x = o[FIRST + i / 4];
+        mail[i * TEAM + tid] = f32x4_t{x[4 * (i % 4)], x[4 * (i % 4) + 1], x[4 * (i % 4) + 2], x[4 * (i % 4) + 3]};
+      }
+    };
+    if (team == 0) send(std::integral_constant<int, HALF>{});
+    else send(std::integral_constant<int, 0>{});
+    if (h == 0) stat[32 * wave + n] = f32x2_t{mr, lt};
+    __syncthreads();
+    const f32x2_t other = from_stat[32 * wave + n];
+    const float M = fmaxf(mr, other[0]), Mu = M == -INFINITY ? 0.0f : M;
+    const float w_own = fast_exp2(mr - Mu), w_other = fast_exp2(other[0] - Mu);
+    const float L = lt * w_own + other[1] * w_other;
+    const int64_t prow = ((int64_t)split * p.B * p.Hkv + group) * p.R + row;
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    uint16_t* op = p.o + b * p.o_sb + (int64_t)(kvh * p.G + g) * p.o_sh + (int64_t)qi * p.o_st;
+    auto finish = [&](auto first_tag) {
+      constexpr int FIRST = decltype(first_tag)::value;
+#pragma unroll
+      for (int i = 0; i < 4 * HALF; ++i) {
+        const f32x4_t x = from[i * TEAM + tid];
+        const int dt = FIRST + i / 4, a = i % 4;
+        f32x4_t y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = o[dt][4 * a + e] * w_own + x[e] * w_other;
+        if (!row_ok) continue;
+        if (p.num_splits == 1) *(u32x2_t*)(op + dt * 32 + 8 * a + 4 * h) = u32x2_t{pack_pair<F16>(y[0] * inv, y[1] * inv), pack_pair<F16>(y[2] * inv, y[3] * inv)};
+        else *(f32x4_t*)(p.part_o + prow * D + dt * 32 + 8 * a + 4 * h) = y;
+      }
+    };
+    if (team == 0) finish(std::integral_constant<int, 0>{});
+    else finish(std::integral_constant<int, HALF>{});
+    if (h == 0 && row_ok) {
+      if (p.num_splits > 1) *(f32x2_t*)(p.part_ml + (((int64_t)(2 * split + team) * p.B * p.Hkv + group) * p.R + row) * 2) = f32x2_t{mr, lt};
+      else if (p.lse && team == 0) p.lse[((int64_t)b * p.q_len + qi) * p.Hq + kvh * p.G + g] = Mu + fast_log2(L);
+    }
+    return;
+  }
   if (p.num_splits == 1) {
     const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
     if (row_ok) {
@@ -610,32 +744,46 @@ __global__ __launch_bounds__(64 * nwaves(KV, D), (kv_is_plain(KV) && D <= 128) ?
 template <int D, bool F16, int SC>
 __global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(const MergeParams p) { merge_job<D, F16, SC>(p, blockIdx.x); }
 
-// The number of KV splits with the least estimated time: c workgroups share a compute unit, one after the other or side by
-// side, and each walks its split's tiles; more splits balance the device better and shorten the walk, but every partial
-// is written, read again and combined by one more launch. The constants are measured (ns): a tile of 64 keys for a workgroup
-// that has its compute unit to itself is 700 / 1130 / 2050 at head size 64 / 128 / 256, two side by side gain 20 %; the
-// combining launch takes 2 us and reads its partials at 4 TB/s. A full count of rounds with a nearly empty last one is what
-// the rule avoids: 2 x 4 heads, 333 queries x 7, 5001 keys: 4 splits (608 workgroups, three to a unit) 83 us, 3 splits
+// The number of KV splits with the least estimated time, and whether a split is walked by a pair of teams (PAIR): c workgroups share a compute
+// unit, one after the other or side by side, and each walks its split's tiles; more splits balance the device better and shorten the walk, but
+// every partial is written, read again and combined by one more launch. Constants in ns: a tile of 64 keys for a workgroup that has its compute unit
+// to itself 600 / 1130 / 2050 at head size 64 / 128 / 256, for two side by side 1.45 of that, for an odd one after them 0.75; a pair takes two tiles in
+// 1.45 as well and needs no partials where the split is the only one. Workgroups over codes or of head size 256 run one after the other.
+// Over 195 calls of 40 to 1100 rows of 1 to 7 heads, 8 to 600 blocks of rows, 500 to 40000 keys, the plan chosen takes 0.8 % longer than the best of up to 30
+// in the mean; the best plan without pairs 11 %. us, best without pairs -> with: 80 blocks x 13 tiles 24.8 -> 20.0, 120 x 13 27.9 -> 20.4,
+// 32 x 94 30.7 -> 27.1, 60 x 396 of 64 values 77.3 -> 72.8; 256 x 64 90.8 -> 78, x 256 277 -> 266, x 512 483 -> 477. A full count of rounds with a nearly
+// empty last one is what the rule avoids: 2 x 4 heads, 333 queries x 7, 5001 keys: 4 splits (608 workgroups, three to a unit) 83 us, 3 splits
 // (456, two) 63 us, 5 splits (760, three) 73 us; 4 x 4 heads, 541 x 7 over 5238: 2 splits 177, none 152.
-int pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
+struct Splits {
+  int n;
+  bool pair;
+};
+Splits pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
   const int64_t base = (int64_t)a.B * a.Hkv * m_blocks, cus = num_cus();
   const bool plain = kv_is_plain(a.kv_dtype);
-  int64_t tile_ns = a.D == 64 ? 700 : a.D == 128 ? 1130 : 2050;
-  if (!plain) tile_ns = a.D == 256 ? 5500 : 2 * tile_ns + 300;  // 256 rows a workgroup, codes to dequantise (at 256: 128 rows)
-  const bool pairs = plain && a.D <= 128;
+  int64_t tile_ns = a.D == 64 ? 600 : a.D == 128 ? 1130 : 2050;
+  if (!plain) tile_ns = a.D == 256 ? 5500 : a.D == 64 ? 1700 : 2560;  // 256 rows a workgroup, codes to dequantise (at 256: 128 rows)
+  const bool two = pairs(a.kv_dtype, a.D);
   const int64_t rows = (int64_t)a.B * a.Hq * a.q_len;
-  int best = 1;
+  Splits best = {1, false};
   int64_t best_ns = INT64_MAX;
   for (int s = 1; s <= min(64, num_tiles); ++s) {
     const int tps = (num_tiles + s - 1) / s;
     if ((num_tiles + tps - 1) / tps != s) continue;
     const int64_t c = (base * s + cus - 1) / cus;
     // an odd workgroup after the pairs gains nothing and waits for one of them to end
-    const int64_t walk = tps * tile_ns * (!pairs || c == 1 ? 100 * c : 160 * (c / 2) + 135 * (c % 2)) / 100;
-    const int64_t merge = s == 1 ? 0 : 2000 + s * rows * (a.D * 4 + 8) / 4000;
-    if (walk + merge < best_ns) {
+    const int64_t partials = s * rows * (a.D * 4 + 8);
+    const int64_t merge = s == 1 ? 0 : two ? 2500 + 25 * s + partials / 2200 : 2000 + partials / 4000;
+    auto consider = [&](int64_t walk, bool pair) {
+      if (walk + merge >= best_ns) return;
       best_ns = walk + merge;
-      best = s;
+      best = {s, pair};
+    };
+    if (!two) {
+      consider(tps * tile_ns * c, false);
+    } else {
+      consider(tps * tile_ns * (c == 1 ? 100 : 145 * (c / 2) + 75 * (c % 2)) / 100 + 200 * ((c + 1) / 2), false);
+      if (tps > 1) consider((tps + 1) / 2 * tile_ns * c * 145 / 100 + 600 * c, true);
     }
   }
   return best;
@@ -697,7 +845,15 @@ void fill_params(PrefillParams& p, const kvx_sdpa_args& a, bool combined = false
   p.columns = rows.columns;
   const int bm = p.columns ? p.columns : 32 * nwaves(a.kv_dtype, a.D);
   p.m_blocks = (p.R + bm - 1) / bm;
-  p.num_splits = a.num_splits > 0 ? min(a.num_splits, p.num_tiles) : p.columns ? rows.splits : pick_splits(a, p.m_blocks, p.num_tiles);
+  if (a.num_splits > 0) {
+    p.num_splits = min(a.num_splits, p.num_tiles);
+  } else if (p.columns) {
+    p.num_splits = rows.splits;
+  } else {
+    const Splits s = pick_splits(a, p.m_blocks, p.num_tiles);
+    p.num_splits = s.n;
+    p.pair = s.pair;
+  }
   p.tiles_per_split = (p.num_tiles + p.num_splits - 1) / p.num_splits;
   p.num_splits = (p.num_tiles + p.tiles_per_split - 1) / p.tiles_per_split;
   if (!a.token_positions && a.input_pos == 0 && a.q_len <= a.kv_len && kv_is_plain(a.kv_dtype) && a.num_splits <= 0 && !p.columns) {
@@ -705,6 +861,7 @@ void fill_params(PrefillParams& p, const kvx_sdpa_args& a, bool combined = false
     const CausalSplits cs = causal_splits(a, bm, p.m_blocks, combined);
     p.tiles_per_split = cs.tiles;
     p.num_splits = (p.num_tiles + p.tiles_per_split - 1) / p.tiles_per_split;
+    p.pair = 0;
     if (cs.jobs) p.period = p.tiles_per_split * BN * p.G / bm;
   }
 }
@@ -712,7 +869,7 @@ void fill_params(PrefillParams& p, const kvx_sdpa_args& a, bool combined = false
 size_t partial_bytes(const PrefillParams& p, int D) {
   if (p.num_splits <= 1) return 0;
   const size_t rows = (size_t)p.num_splits * p.B * p.Hkv * p.R;
-  return rows * (size_t)D * 4 + rows * 2 * 4;
+  return rows * (size_t)D * 4 + rows * 2 * 4 * (p.pair ? 2 : 1);
 }
 
 // `rest`: where the partials are left for another launch to combine, their description (num_splits 1: nothing to combine)
@@ -733,16 +890,22 @@ int launch_t(PrefillParams& p, hipStream_t st, MergeParams* rest) {
         p.period = 0;
       }
     }
-    bool periods = false;
+    bool general = true;
     if constexpr (kv_is_plain(KV)) {
-      periods = p.period != 0;
-      if (periods) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, true>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
+      general = p.period == 0;
+      if (!general) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, true, false>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
     }
-    if (!periods) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, false>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
+    if constexpr (pairs(KV, D)) {
+      if (p.pair) {
+        general = false;
+        hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, false, true>), grid, dim3(2 * 64 * nwaves(KV, D)), 0, st, p);
+      }
+    }
+    if (general) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, false, false>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
     KVX_HIP(hipGetLastError());
   }
   const MergeParams m = {p.part_o, p.part_ml, p.o, p.lse, p.B, p.Hq, p.Hkv, p.G, p.q_len, p.R, p.num_splits, p.o_sb, p.o_sh, p.o_st,
-                         p.input_pos, p.tp ? 0 : p.tiles_per_split * BN};
+                         p.input_pos, p.tp ? 0 : p.tiles_per_split * BN, p.pair ? 2 : 1};
   if (rest) {
     *rest = m;
     return KVX_OK;
@@ -787,6 +950,7 @@ void common_params(PrefillParams& p, const kvx_sdpa_args& a) {
   p.tiles_per_split = p.num_tiles;
   p.m_blocks = 0;
   p.period = 0;
+  p.pair = 0;
   p.columns = 0;
   p.c = a.sm_scale * kLog2e;
   p.q_sb = a.q_stride_b; p.q_sh = a.q_stride_h; p.q_st = a.q_stride_t;
