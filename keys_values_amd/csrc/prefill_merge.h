@@ -29,20 +29,18 @@ constexpr int merge_classes(int D) { return 256 / (D / 4) < 8 ? 256 / (D / 4) : 
 inline bool merge_wants_classes(const MergeParams& p, int D) {
   return p.num_splits > 4 && (int64_t)p.B * p.Hkv * p.R * (D / 4) < (int64_t)num_cus() * 256;
 }
-template <int D, bool F16, int SC>
-__device__ __forceinline__ void merge_job(const MergeParams& p, const int64_t block) {
+template <int D, bool F16, int SC, int TEAMS>
+__device__ __forceinline__ void merge_rows_job(const MergeParams& p, const int64_t block, f32x4_t* red_o, float* red_l) {
   constexpr int TPR = D / 4;                // threads per row and split class
   constexpr int ROWS = merge_rows(D, SC);    // rows per workgroup
   static_assert(ROWS >= 1, "a row's threads fit a workgroup");
-  __shared__ f32x4_t red_o[SC > 1 ? 256 : 1];
-  __shared__ float red_l[SC > 1 ? 256 : 1];
   const int64_t total_rows = (int64_t)p.B * p.Hkv * p.R;
   const int64_t grow = block * ROWS + threadIdx.x / (TPR * SC);
   const bool live = grow < total_rows;
   const int64_t growc = live ? grow : total_rows - 1;
   const int S = p.split_keys ? min(p.num_splits, (p.input_pos + (int)(growc % p.R) / p.G) / p.split_keys + 1) : p.num_splits;
   const int dq = threadIdx.x % TPR, j = (threadIdx.x / TPR) % SC;
-  const f32x2_t* ml = (const f32x2_t*)p.part_ml + growc;  // (maximum, sum) of split s at s * teams * total_rows, of its second team behind it
+  const f32x2_t* ml = (const f32x2_t*)p.part_ml + growc;  // (maximum, sum) of split s at s * TEAMS * total_rows, of its second team behind it
   const float* po = p.part_o + growc * D + dq * 4;
   // the partials of splits s0, s0 + SC, ... (four at most), all asked for at once; nothing where there is no such split
   f32x2_t m[4], m2[4];
@@ -54,8 +52,8 @@ __device__ __forceinline__ void merge_job(const MergeParams& p, const int64_t bl
       x[u] = f32x4_t{0, 0, 0, 0};
       if (s0 + u * SC < S) {
         const int64_t at = (int64_t)(s0 + u * SC) * total_rows;
-        m[u] = ml[at * p.teams];
-        if (p.teams > 1) m2[u] = ml[at * 2 + total_rows];
+        m[u] = ml[at * TEAMS];
+        if constexpr (TEAMS > 1) m2[u] = ml[at * TEAMS + total_rows];
         x[u] = *(const f32x4_t*)(po + at * D);
       }
     }
@@ -65,14 +63,13 @@ __device__ __forceinline__ void merge_job(const MergeParams& p, const int64_t bl
   if (SC == 1 && S <= 4) {
     M = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) M = fmaxf(M, fmaxf(m[u][0], m2[u][0]));
+    for (int u = 0; u < 4; ++u) M = fmaxf(M, TEAMS > 1 ? fmaxf(m[u][0], m2[u][0]) : m[u][0]);
   } else {
     M = -INFINITY;
-    const int n = S * p.teams;
-    for (int s0 = 0; s0 < n; s0 += 4) {
+    // a lane each; every thread reading them all was two thirds of the launch (1976 rows of 18 maxima 12 us)
+    for (int i = dq; i < S * TEAMS; i += TPR) M = fmaxf(M, ml[(int64_t)i * total_rows][0]);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) M = fmaxf(M, ml[(int64_t)min(s0 + u, n - 1) * total_rows][0]);
-    }
+    for (int off = TPR / 2; off >= 1; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
   }
   const float Mu = (M == -INFINITY) ? 0.0f : M;
   float L = 0.0f;
@@ -82,10 +79,14 @@ __device__ __forceinline__ void merge_job(const MergeParams& p, const int64_t bl
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       if (s0 + u * SC < S) {
-        const float w = fast_exp2(m[u][0] - Mu), w2 = fast_exp2(m2[u][0] - Mu);
+        float w = fast_exp2(m[u][0] - Mu);
         L += m[u][1] * w;
-        L += m2[u][1] * w2;
-        acc += x[u] * fmaxf(w, w2);
+        if constexpr (TEAMS > 1) {
+          const float w2 = fast_exp2(m2[u][0] - Mu);
+          L += m2[u][1] * w2;
+          w = fmaxf(w, w2);
+        }
+        acc += x[u] * w;
       }
   }
   if constexpr (SC > 1) {
@@ -111,6 +112,14 @@ __device__ __forceinline__ void merge_job(const MergeParams& p, const int64_t bl
   w2[1] = pack_pair<F16>(acc[2] * inv, acc[3] * inv);
   *(u32x2_t*)op = w2;
   if (p.lse && dq == 0) p.lse[((int64_t)b * p.q_len + qi) * p.Hq + kvh * p.G + g] = Mu + fast_log2(L);
+}
+
+template <int D, bool F16, int SC>
+__device__ __forceinline__ void merge_job(const MergeParams& p, const int64_t block) {
+  __shared__ f32x4_t red_o[SC > 1 ? 256 : 1];
+  __shared__ float red_l[SC > 1 ? 256 : 1];
+  if (p.teams > 1) merge_rows_job<D, F16, SC, 2>(p, block, red_o, red_l);
+  else merge_rows_job<D, F16, SC, 1>(p, block, red_o, red_l);
 }
 
 }  // namespace kvx

@@ -747,10 +747,11 @@ __global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(const MergePara
 // The number of KV splits with the least estimated time, and whether a split is walked by a pair of teams (PAIR): c workgroups share a compute
 // unit, one after the other or side by side, and each walks its split's tiles; more splits balance the device better and shorten the walk, but
 // every partial is written, read again and combined by one more launch. Constants in ns: a tile of 64 keys for a workgroup that has its compute unit
-// to itself 600 / 1130 / 2050 at head size 64 / 128 / 256, for two side by side 1.45 of that, for an odd one after them 0.75; a pair takes two tiles in
-// 1.45 as well and needs no partials where the split is the only one. Workgroups over codes or of head size 256 run one after the other.
-// Over 195 calls of 40 to 1100 rows of 1 to 7 heads, 8 to 600 blocks of rows, 500 to 40000 keys, the plan chosen takes 0.8 % longer than the best of up to 30
-// in the mean; the best plan without pairs 11 %. us, best without pairs -> with: 80 blocks x 13 tiles 24.8 -> 20.0, 120 x 13 27.9 -> 20.4,
+// to itself 840 / 1130 / 2050 at head size 64 / 128 / 256; at 128 two workgroups side by side take 1.48 of that, an odd one after them 1.06; at 64
+// two 1.46 and three, all that run side by side, 1.95, one and two after them 1.13 and 1.41; a pair takes 1.6 (of 64: 1.5) for two tiles and needs
+// no partials where the split is the only one. Workgroups over codes or of head size 256 run one after the other.
+// Over 450 calls of 40 to 1100 rows of 1 to 8 heads, 4 to 1100 blocks of rows, 500 to 40000 keys, the plan chosen takes 0.5 % longer than the best of up to 30
+// in the mean, the best plan without pairs 6 %. us, best without pairs -> with: 80 blocks x 13 tiles 24.8 -> 20.0, 120 x 13 27.9 -> 20.4,
 // 32 x 94 30.7 -> 27.1, 60 x 396 of 64 values 77.3 -> 72.8; 256 x 64 90.8 -> 78, x 256 277 -> 266, x 512 483 -> 477. A full count of rounds with a nearly
 // empty last one is what the rule avoids: 2 x 4 heads, 333 queries x 7, 5001 keys: 4 splits (608 workgroups, three to a unit) 83 us, 3 splits
 // (456, two) 63 us, 5 splits (760, three) 73 us; 4 x 4 heads, 541 x 7 over 5238: 2 splits 177, none 152.
@@ -761,7 +762,7 @@ struct Splits {
 Splits pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
   const int64_t base = (int64_t)a.B * a.Hkv * m_blocks, cus = num_cus();
   const bool plain = kv_is_plain(a.kv_dtype);
-  int64_t tile_ns = a.D == 64 ? 600 : a.D == 128 ? 1130 : 2050;
+  int64_t tile_ns = a.D == 64 ? 840 : a.D == 128 ? 1130 : 2050;
   if (!plain) tile_ns = a.D == 256 ? 5500 : a.D == 64 ? 1700 : 2560;  // 256 rows a workgroup, codes to dequantise (at 256: 128 rows)
   const bool two = pairs(a.kv_dtype, a.D);
   const int64_t rows = (int64_t)a.B * a.Hq * a.q_len;
@@ -773,7 +774,7 @@ Splits pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
     const int64_t c = (base * s + cus - 1) / cus;
     // an odd workgroup after the pairs gains nothing and waits for one of them to end
     const int64_t partials = s * rows * (a.D * 4 + 8);
-    const int64_t merge = s == 1 ? 0 : two ? 2500 + 25 * s + partials / 2200 : 2000 + partials / 4000;
+    const int64_t merge = s == 1 ? 0 : two ? 3400 + 30 * s + partials / 2000 : 2000 + partials / 4000;
     auto consider = [&](int64_t walk, bool pair) {
       if (walk + merge >= best_ns) return;
       best_ns = walk + merge;
@@ -782,8 +783,11 @@ Splits pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
     if (!two) {
       consider(tps * tile_ns * c, false);
     } else {
-      consider(tps * tile_ns * (c == 1 ? 100 : 145 * (c / 2) + 75 * (c % 2)) / 100 + 200 * ((c + 1) / 2), false);
-      if (tps > 1) consider((tps + 1) / 2 * tile_ns * c * 145 / 100 + 600 * c, true);
+      const int64_t side = a.D == 64 ? 3 : 2;  // side by side
+      static const int64_t first[3] = {0, 100, 146}, after64[3] = {0, 113, 141}, after128[2] = {0, 106};
+      const int64_t walk = c < side ? first[c] : a.D == 64 ? 195 * (c / 3) + after64[c % 3] : 148 * (c / 2) + after128[c % 2];
+      consider(tps * tile_ns * walk / 100 + 200 * ((c + side - 1) / side), false);
+      if (tps > 1) consider((tps + 1) / 2 * tile_ns * c * (a.D == 64 ? 150 : 160) / 100 + 600 * c, true);
     }
   }
   return best;
