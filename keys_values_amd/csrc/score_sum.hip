@@ -193,6 +193,7 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
   constexpr int BK = NW * W;  // keys per workgroup
   constexpr bool F16 = kv_elem_f16(KV);  // element type of q and k
   __shared__ Smem<D> sm;
+  __shared__ uint32_t arrivals[W];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
@@ -281,10 +282,10 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
 #pragma unroll
     for (int a = 0; a < 4; ++a) ls[a] = *(const f32x4_t*)&sm.lse[BUF][MT * 32 + 8 * a + 4 * h];
   };
-  // S block = 32 query rows x 64 keys, K in registers
-  auto mfma_block = [&](f32x16_t (&s)[2], const u32x4_t (&qq)[D / 16]) {
+  // S block = 32 query rows x 64 keys, K in registers; k-steps J0 .. J1 - 1
+  auto mfma_part = [&](f32x16_t (&s)[2], const u32x4_t (&qq)[D / 16], auto j0_tag, auto j1_tag) {
 #pragma unroll
-    for (int j = 0; j < D / 16; ++j) {
+    for (int j = decltype(j0_tag)::value; j < decltype(j1_tag)::value; ++j) {
 #pragma unroll
       for (int nt = 0; nt < 2; ++nt) {
         if (j == 0) {
@@ -296,11 +297,11 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
       }
     }
   };
-  // p = exp2(c S - lse) summed over the block's rows
-  auto valu_block = [&](auto mask_tag, const f32x16_t (&s)[2], const f32x4_t (&ls)[4], int ring, int mt) {
+  // p = exp2(c S - lse) summed over the block's rows, quarters A0 .. A1 - 1
+  auto valu_part = [&](auto mask_tag, const f32x16_t (&s)[2], const f32x4_t (&ls)[4], int ring, int mt, auto a0_tag, auto a1_tag) {
     constexpr bool MASK = decltype(mask_tag)::value;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
+    for (int a = decltype(a0_tag)::value; a < decltype(a1_tag)::value; ++a) {
       int4 qp = {0, 0, 0, 0};
       if constexpr (MASK) qp = *(const int4*)&sm.qpos[ring][mt * 32 + 8 * a + 4 * h];
 #pragma unroll
@@ -321,10 +322,10 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
   };
   // one matrix instruction, then its share of the other block's vector work (6 or 10 instructions per matrix
   // instruction, 2 of them transcendental)
-  auto interleave = [&](auto mask_tag) {
+  auto interleave = [&](auto mask_tag, auto quarters_tag) {
     constexpr bool MASK = decltype(mask_tag)::value;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
+    for (int a = 0; a < decltype(quarters_tag)::value; ++a) {
       if constexpr (MASK) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // the positions of rows 8 a .. 8 a + 7
 #pragma unroll
       for (int i = 0; i < (D / 16) / 2; ++i) {
@@ -343,6 +344,25 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
   };
   constexpr std::integral_constant<int, 0> I0{};
   constexpr std::integral_constant<int, 1> I1{};
+  constexpr std::integral_constant<int, 3> I3{};
+  constexpr std::integral_constant<int, 4> I4{};
+  constexpr std::integral_constant<int, D / 16> KS{};
+  constexpr std::integral_constant<int, D / 16 * 3 / 4> KS3{};
+  // The workgroup's barrier, once a tile, in two halves: a wavefront arrives, in a word of LDS, when its transfers have landed and what it needs of the
+  // tile is in registers, and looks for the others behind the last quarter of that block's work. As one barrier (us): 4096 rows over 8 x 32768 keys
+  // 289 -> 283 of 760, 600 over 16 x 6000 30.8 -> 29.2, of 64 over 8 x 16384 123 -> 116. All wavefronts of a workgroup are resident and arrive once a tile, so the wait ends.
+  uint32_t due = 0;
+  auto arrive = [&] {
+    ++due;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __hip_atomic_store(&arrivals[wave], due, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  auto wait_for_all = [&] {
+    while (__any(__hip_atomic_load(&arrivals[lane % W], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < due)) {
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  };
+  if (tid < W) arrivals[tid] = 0;
   ld.issue(sm, 0, 0);
   if (num_qt > 1) ld.issue(sm, 1, 1);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the K fragments and the first tiles have arrived
@@ -352,7 +372,7 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
   f32x16_t sa[2], sb[2];  // blocks 0 and 1 of the current tile
   u32x4_t qq[D / 16];
   load_q(qq, I0, I0);
-  mfma_block(sa, qq);
+  mfma_part(sa, qq, I0, KS);
 
   // Software pipeline: the matrix work of one block runs under the vector work of the block before.
   // Tile t + 2 is requested right behind the barrier of step t (the buffers of tile t are free from there on: its
@@ -364,21 +384,28 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
     constexpr std::integral_constant<int, BUF ^ 1> NEXT{};
     const int ring = t & 3;
     const bool more = STEADY || t + 1 < num_qt;
-    f32x4_t ls[4];
+    f32x4_t ls[4], ls1[4];
     load_q(qq, buf_tag, I1);
     load_lse(ls, buf_tag, I0);
     __builtin_amdgcn_sched_barrier(0);
-    mfma_block(sb, qq);
-    valu_block(mask_tag, sa, ls, ring, 0);
-    interleave(mask_tag);
+    mfma_part(sb, qq, I0, KS3);
+    valu_part(mask_tag, sa, ls, ring, 0, I0, I3);
+    interleave(mask_tag, I3);
     pin(sb);
     __builtin_amdgcn_sched_barrier(0);
-    load_lse(ls, buf_tag, I1);  // into registers before the barrier that hands the buffer to tile t + 2
+    load_lse(ls1, buf_tag, I1);  // into registers before the barrier that hands the buffer to tile t + 2
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's part of tile t + 1 has landed
     if (!STEADY || RT < BQ) {
       if (more) ld.land(sm, (tbase + t + 1) * RT, BUF ^ 1);
     }
-    __syncthreads();
+    arrive();
+    __builtin_amdgcn_sched_barrier(0);
+    mfma_part(sb, qq, KS3, KS);
+    valu_part(mask_tag, sa, ls, ring, 0, I3, I4);
+    interleave(mask_tag, I1);
+    pin(sb);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_for_all();
     if constexpr (STEADY) {
       ld.template issue_steady<BUF>(sm, (t + 2) & 3);
     } else {
@@ -387,13 +414,13 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
     if (more) {
       load_q(qq, NEXT, I0);
       __builtin_amdgcn_sched_barrier(0);
-      mfma_block(sa, qq);
-      valu_block(mask_tag, sb, ls, ring, 1);
-      interleave(mask_tag);
+      mfma_part(sa, qq, I0, KS);
+      valu_part(mask_tag, sb, ls1, ring, 1, I0, I4);
+      interleave(mask_tag, I4);
       pin(sa);
       __builtin_amdgcn_sched_barrier(0);
     } else {
-      valu_block(mask_tag, sb, ls, ring, 1);
+      valu_part(mask_tag, sb, ls1, ring, 1, I0, I4);
     }
   };
   constexpr std::true_type YES{};
