@@ -748,8 +748,8 @@ __global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(const MergePara
 // unit, one after the other or side by side, and each walks its split's tiles; more splits balance the device better and shorten the walk, but
 // every partial is written, read again and combined by one more launch. Constants in ns: a tile of 64 keys for a workgroup that has its compute unit
 // to itself 840 / 1130 / 2050 at head size 64 / 128 / 256; at 128 two workgroups side by side take 1.48 of that, an odd one after them 1.06; at 64
-// two 1.46 and three, all that run side by side, 1.95, one and two after them 1.13 and 1.41; a pair takes 1.6 (of 64: 1.5) for two tiles and needs
-// no partials where the split is the only one. Workgroups over codes or of head size 256 run one after the other.
+// two 1.46 and three, all that run side by side, 1.95, one and two after them 1.13 and 1.41; a pair takes 1.45, 1.6 with others after it, of 64 1.5,
+// for two tiles and needs no partials where the split is the only one. Workgroups over codes or of head size 256 run one after the other.
 // Over 450 calls of 40 to 1100 rows of 1 to 8 heads, 4 to 1100 blocks of rows, 500 to 40000 keys, the plan chosen takes 0.5 % longer than the best of up to 30
 // in the mean, the best plan without pairs 6 %. us, best without pairs -> with: 80 blocks x 13 tiles 24.8 -> 20.0, 120 x 13 27.9 -> 20.4,
 // 32 x 94 30.7 -> 27.1, 60 x 396 of 64 values 77.3 -> 72.8; 256 x 64 90.8 -> 78, x 256 277 -> 266, x 512 483 -> 477. A full count of rounds with a nearly
@@ -787,7 +787,7 @@ Splits pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
       static const int64_t first[3] = {0, 100, 146}, after64[3] = {0, 113, 141}, after128[2] = {0, 106};
       const int64_t walk = c < side ? first[c] : a.D == 64 ? 195 * (c / 3) + after64[c % 3] : 148 * (c / 2) + after128[c % 2];
       consider(tps * tile_ns * walk / 100 + 200 * ((c + side - 1) / side), false);
-      if (tps > 1) consider((tps + 1) / 2 * tile_ns * c * (a.D == 64 ? 150 : 160) / 100 + 600 * c, true);
+      if (tps > 1) consider((tps + 1) / 2 * tile_ns * c * (a.D == 64 ? 150 : c == 1 ? 145 : 160) / 100 + 600 * c, true);
     }
   }
   return best;
