@@ -130,34 +130,21 @@ __device__ __forceinline__ void quantize_rows_in_flight(const u32x4_t (&raw)[ROW
   }
 }
 
-// Quantise the 8 values of this lane's share of a row; every lane of the row returns the same
-// scale / zero point.
+// Quantise the 8 values of this lane's share of a K and a V row. Even lanes work out the scale and zero point of the K row, odd ones of
+// the V row, and each fetches 1 / scale and the zero point of the other from its neighbour; (scale, zp): the lane's own row's.
 template <int LPR, bool F16>
-__device__ __forceinline__ u32x2_t quantize8(u32x4_t raw, float& scale, int32_t& zp) {
-  float x[8];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    x[2 * e] = elem_lo<F16>(raw[e]);
-    x[2 * e + 1] = elem_hi<F16>(raw[e]);
-  }
-  float mn = x[0], mx = x[0];
-#pragma unroll
-  for (int e = 1; e < 8; ++e) {
-    mn = fminf(mn, x[e]);
-    mx = fmaxf(mx, x[e]);
-  }
-  mn = row_min<LPR>(mn);
-  mx = row_max<LPR>(mx);
-  if (row_any<LPR>(has_nan8(x))) mn = mx = __builtin_nanf("");  // aminmax propagates NaN, fminf / fmaxf drop it
-  quant_params(mn, mx, scale, zp);
-  const float inv = 1.0f / scale;
-  const float zf = (float)zp;
-  u32x2_t out;
-  out[0] = quant_code(x[0], inv, zf) | (quant_code(x[1], inv, zf) << 8) | (quant_code(x[2], inv, zf) << 16) |
-           (quant_code(x[3], inv, zf) << 24);
-  out[1] = quant_code(x[4], inv, zf) | (quant_code(x[5], inv, zf) << 8) | (quant_code(x[6], inv, zf) << 16) |
-           (quant_code(x[7], inv, zf) << 24);
-  return out;
+__device__ __forceinline__ void quantize8_kv(const u32x4_t& k, const u32x4_t& v, u32x2_t& kc, u32x2_t& vc, float& scale, int32_t& zp) {
+  float xk[8], xv[8], mnk, mxk, mnv, mxv;
+  row_extremes<LPR, F16>(k, xk, mnk, mxk);
+  row_extremes<LPR, F16>(v, xv, mnv, mxv);
+  const bool odd = __lane_id() & 1u;
+  quant_params(odd ? mnv : mnk, odd ? mxv : mxk, scale, zp);
+  const int inv = __builtin_bit_cast(int, 1.0f / scale), zf = __builtin_bit_cast(int, (float)zp);
+  auto of_k = [](int x) { return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0xA0, 0xf, 0xf, true)); };  // quad_perm [0,0,2,2]
+  auto of_v = [](int x) { return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0xF5, 0xf, 0xf, true)); };  // quad_perm [1,1,3,3]
+  const float ik = of_k(inv), zk = of_k(zf), iv = of_v(inv), zv = of_v(zf);
+  kc = u32x2_t{codes4_u8(xk[0], xk[1], xk[2], xk[3], ik, zk), codes4_u8(xk[4], xk[5], xk[6], xk[7], ik, zk)};
+  vc = u32x2_t{codes4_u8(xv[0], xv[1], xv[2], xv[3], iv, zv), codes4_u8(xv[4], xv[5], xv[6], xv[7], iv, zv)};
 }
 
 // Where the rows of a call lie: `n_outer` runs of `rows` rows each. A contiguous store is one run; a range of slots of a
@@ -562,7 +549,7 @@ __device__ __forceinline__ float row_quant_error(u32x4_t raw, u32x2_t codes, flo
 // the read and the write of that slot are issued by the same wavefront, in this order, and the
 // read's data is consumed before the write is issued.
 template <int D, int KV>
-__global__ __launch_bounds__(NTHREADS) void cache_write_kernel(const kvx_cache_write_args a, const DecodeCounters clear) {
+__global__ __launch_bounds__(NTHREADS) void cache_write_kernel(const kvx_cache_write_args a, const DecodeCounters clear, const uint32_t jobs) {
   constexpr bool U8 = !kv_is_plain(KV);  // a quantised store: codes + row state
   constexpr bool U4 = kv_is_u4(KV);       // two codes per byte: only the lanes of the first half of a row store
   constexpr bool F16 = kv_elem_f16(KV);   // the rows are float16
@@ -572,14 +559,12 @@ __global__ __launch_bounds__(NTHREADS) void cache_write_kernel(const kvx_cache_w
     clear_counters(clear, gid, (int64_t)gridDim.x * NTHREADS, (int64_t)a.B * a.Hkv);
     if (gid == 0 && clear.scratch_splits) *clear.scratch_splits = 0u;
   }
-  const int col = (int)(gid % LPR);
-  const int64_t rid = gid / LPR;
-  const int64_t total = (int64_t)a.B * a.Hkv * a.num;
-  const bool live = rid < total;
-  const int64_t ridc = live ? rid : 0;
-  const int j = (int)(ridc % a.num);
-  const int hh = (int)((ridc / a.num) % a.Hkv);
-  const int b = (int)(ridc / ((int64_t)a.num * a.Hkv));
+  const int col = threadIdx.x % LPR;
+  const uint32_t rid = blockIdx.x * (NTHREADS / LPR) + threadIdx.x / LPR;
+  const bool live = rid < jobs;
+  const uint32_t ridc = live ? rid : 0, pair = ridc / (uint32_t)a.num;
+  const int j = (int)(ridc - pair * a.num);
+  const int b = (int)(pair / (uint32_t)a.Hkv), hh = (int)(pair - b * a.Hkv);
   const int slot = a.index[b * a.index_stride_b + hh * a.index_stride_h + j];
   const bool moves = j < a.grace_num;
   const int ring = moves ? a.grace_slots[j] : -1;
@@ -605,8 +590,19 @@ __global__ __launch_bounds__(NTHREADS) void cache_write_kernel(const kvx_cache_w
   auto put = [&](const u32x4_t& krow, const u32x4_t& vrow, int target, bool doit, bool want_err) -> float {
     float s1, s2, err = 0.0f;
     int32_t z1, z2;
-    u32x2_t kc = U4 ? quantize4<LPR, F16>(krow, s1, z1) : quantize8<LPR, F16>(krow, s1, z1);
-    u32x2_t vc = U4 ? quantize4<LPR, F16>(vrow, s2, z2) : quantize8<LPR, F16>(vrow, s2, z2);
+    u32x2_t kc, vc;
+    if constexpr (U4) {
+      kc = quantize4<LPR, F16>(krow, s1, z1);
+      vc = quantize4<LPR, F16>(vrow, s2, z2);
+    } else {
+      float s;
+      int32_t z;
+      quantize8_kv<LPR, F16>(krow, vrow, kc, vc, s, z);
+      s1 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, s), 0xA0, 0xf, 0xf, true));
+      s2 = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, s), 0xF5, 0xf, 0xf, true));
+      z1 = __builtin_amdgcn_mov_dpp(z, 0xA0, 0xf, 0xf, true);
+      z2 = __builtin_amdgcn_mov_dpp(z, 0xF5, 0xf, 0xf, true);
+    }
     if (want_err) err = row_quant_error<LPR, F16>(krow, kc, s1, z1) + row_quant_error<LPR, F16>(vrow, vc, s2, z2);  // uniform branch
     if constexpr (U4) {  // byte j = code[j] << 4 | code[j + D/2]: the partner lane holds the low nibbles
       kc = u32x2_t{(kc[0] << 4) | (uint32_t)__shfl_xor(kc[0], LPR / 2, 64), (kc[1] << 4) | (uint32_t)__shfl_xor(kc[1], LPR / 2, 64)};
@@ -787,14 +783,14 @@ int launch_quantize_blocks(const kvx_block_quant_args& a, hipStream_t st) { retu
 int launch_dequantize_blocks(const kvx_block_quant_args& a, hipStream_t st) { return launch_blocks(a, false, st); }
 
 template <int D>
-int launch_cache_write_d(const kvx_cache_write_args& a, const DecodeCounters& clear, unsigned grid, hipStream_t st) {
+int launch_cache_write_d(const kvx_cache_write_args& a, const DecodeCounters& clear, unsigned grid, uint32_t jobs, hipStream_t st) {
   switch (a.kv_dtype) {
-    case KVX_KV_F16: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_F16>), dim3(grid), dim3(NTHREADS), 0, st, a, clear); break;
-    case KVX_KV_BF16: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_BF16>), dim3(grid), dim3(NTHREADS), 0, st, a, clear); break;
-    case KVX_KV_U4: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U4>), dim3(grid), dim3(NTHREADS), 0, st, a, clear); break;
-    case KVX_KV_U8: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U8>), dim3(grid), dim3(NTHREADS), 0, st, a, clear); break;
-    case KVX_KV_U4_F16: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U4_F16>), dim3(grid), dim3(NTHREADS), 0, st, a, clear); break;
-    default: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U8_F16>), dim3(grid), dim3(NTHREADS), 0, st, a, clear); break;
+    case KVX_KV_F16: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_F16>), dim3(grid), dim3(NTHREADS), 0, st, a, clear, jobs); break;
+    case KVX_KV_BF16: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_BF16>), dim3(grid), dim3(NTHREADS), 0, st, a, clear, jobs); break;
+    case KVX_KV_U4: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U4>), dim3(grid), dim3(NTHREADS), 0, st, a, clear, jobs); break;
+    case KVX_KV_U8: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U8>), dim3(grid), dim3(NTHREADS), 0, st, a, clear, jobs); break;
+    case KVX_KV_U4_F16: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U4_F16>), dim3(grid), dim3(NTHREADS), 0, st, a, clear, jobs); break;
+    default: hipLaunchKernelGGL((cache_write_kernel<D, KVX_KV_U8_F16>), dim3(grid), dim3(NTHREADS), 0, st, a, clear, jobs); break;
   }
   KVX_HIP(hipGetLastError());
   return KVX_OK;
@@ -805,9 +801,10 @@ int launch_cache_write(const kvx_cache_write_args& a, const DecodeCounters* clea
   const int64_t total = (int64_t)a.B * a.Hkv * a.num * (a.D / 8);
   if (total == 0) return KVX_OK;
   const unsigned grid = (unsigned)((total + NTHREADS - 1) / NTHREADS);
-  if (a.D == 256) return launch_cache_write_d<256>(a, c, grid, st);
-  if (a.D == 128) return launch_cache_write_d<128>(a, c, grid, st);
-  return launch_cache_write_d<64>(a, c, grid, st);
+  const uint32_t jobs = (uint32_t)((int64_t)a.B * a.Hkv * a.num);  // a grid's threads are counted in 32 bits
+  if (a.D == 256) return launch_cache_write_d<256>(a, c, grid, jobs, st);
+  if (a.D == 128) return launch_cache_write_d<128>(a, c, grid, jobs, st);
+  return launch_cache_write_d<64>(a, c, grid, jobs, st);
 }
 
 }  // namespace kvx
