@@ -12,6 +12,8 @@
 // The fused kernel keeps both casts, so it returns what the two separate steps return. It works in
 // place on the output of the QKV projection, (B, num, (Hq + 2 Hkv) * D): the value heads are left as
 // they are and no transposed copies are made (the attention and cache kernels take strides).
+#include <type_traits>
+
 #include "kvx_common.h"
 
 namespace kvx {
@@ -19,40 +21,76 @@ namespace {
 
 constexpr int NT = 256;
 
+// These kernels move two or four bytes a value, and what bounded them was the vector ALU: an IEEE division takes a dozen instructions and a 64-bit index
+// division about a hundred. Values of a row are divided by the row's norm, so one division serves them: with r = RN(1 / b), q = RN(a r) and
+// the remainder a - q b, exact in a fused multiply-add, q + (a - q b) r is RN(a / b) (Markstein, "Computation of elementary functions on the IBM
+// RISC System/6000 processor", 1990) while nothing over- or underflows: by norms of 2^-40 to 2^40 of values of a row no larger than its
+// norm times sqrt(dim). Other norms (zero rows with eps = 0, infinities, NaN) are divided by as they are.
+struct Divisor {
+  float b, r;
+  bool plain;
+  __device__ __forceinline__ explicit Divisor(float x) : b(x), r(1.0f / x), plain(x > 0x1p-40f && x < 0x1p40f) {}
+  __device__ __forceinline__ float under(float a) const {
+    const float q = a * r;
+    return fmaf(fmaf(-q, b, a), r, q);
+  }
+};
+// v of one lane, 8 values, divided by the norm, times the weights
+template <typename Store>
+__device__ __forceinline__ void normalised(const float (&x)[8], const Divisor& d, const f32x4_t& w0, const f32x4_t& w1, Store store) {
+  float y[8];
+  if (__all(d.plain)) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = d.under(x[e]) * (e < 4 ? w0[e] : w1[e - 4]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = (x[e] / d.b) * (e < 4 ? w0[e] : w1[e - 4]);
+  }
+  store(y);
+}
+__device__ __forceinline__ void unpack(const u32x4_t& v, float (&x)[8]) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    x[2 * e] = bf16_lo(v[e]);
+    x[2 * e + 1] = bf16_hi(v[e]);
+  }
+}
+__device__ __forceinline__ u32x4_t packed(const float (&y)[8]) {
+  return u32x4_t{pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3]), pack_bf16(y[4], y[5]), pack_bf16(y[6], y[7])};
+}
+
 __device__ __forceinline__ float wave_sum(float x) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off, 64);
   return x;
 }
 
-// Sum over the WPR wavefronts that share a row (WPR = 1: the wavefront's own sum; WPR = NT / 64: the
-// whole workgroup, through LDS, added in wavefront order).
-template <int WPR>
+// Sum over the wavefronts that share a row (WHOLE: all of the workgroup, through LDS, added in wavefront order; else one).
+constexpr int MAX_WAVES = 8;
+template <bool WHOLE>
 __device__ __forceinline__ float row_total(float ss) {
   ss = wave_sum(ss);
-  if constexpr (WPR > 1) {
-    static_assert(WPR == NT / 64, "a row is one wavefront or the whole workgroup");
-    __shared__ float part[WPR];
+  if constexpr (WHOLE) {
+    __shared__ float part[MAX_WAVES];
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
     __syncthreads();
     ss = part[0];
-#pragma unroll
-    for (int i = 1; i < WPR; ++i) ss += part[i];
+    for (int i = 1; i < (int)blockDim.x / 64; ++i) ss += part[i];
   }
   return ss;
 }
 
-// WPR wavefronts per row; a lane holds up to MAXC chunks of 8 elements (dim <= 64 * WPR * 8 * MAXC).
-// Few long rows (a 1024-token chunk of hidden states) take the whole workgroup per row: four times the
-// loads in flight per row, and enough workgroups to cover the chip.
-template <int MAXC, int WPR>
-__global__ __launch_bounds__(NT) void rmsnorm_rows_kernel(const uint16_t* __restrict__ x, int64_t x_rs, uint16_t* __restrict__ out,
+// A wavefront a row, or (WHOLE) the workgroup; a lane holds up to MAXC chunks of 8 elements (dim <= threads of the row * 8 * MAXC).
+// Few long rows (a 1024-token chunk of hidden states) take the whole workgroup per row, of as many wavefronts as the row has chunks for
+// (row_waves): 2560 values are 320 lanes, and four wavefronts were a second round for one of them.
+template <int MAXC, bool WHOLE>
+__global__ __launch_bounds__(64 * MAX_WAVES) void rmsnorm_rows_kernel(const uint16_t* __restrict__ x, int64_t x_rs, uint16_t* __restrict__ out,
                                                           int64_t o_rs, const float* __restrict__ weight, int64_t rows, int dim,
                                                           float eps, float factor) {
-  constexpr int TPR = 64 * WPR;  // threads per row
-  const int lane = threadIdx.x % TPR;
-  const int64_t row = (int64_t)blockIdx.x * (NT / TPR) + threadIdx.x / TPR;
-  if (row >= rows) return;  // uniform over the threads of a row (and over the workgroup when WPR > 1)
+  const int TPR = WHOLE ? blockDim.x : 64;  // threads per row
+  const int lane = WHOLE ? threadIdx.x : threadIdx.x & 63;
+  const int64_t row = WHOLE ? blockIdx.x : (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
+  if (row >= rows) return;  // uniform over the threads of a row (and over the workgroup where it shares one)
   const int nchunks = dim / 8;
   const uint16_t* xr = x + row * x_rs;
   u32x4_t v[MAXC];
@@ -69,8 +107,8 @@ __global__ __launch_bounds__(NT) void rmsnorm_rows_kernel(const uint16_t* __rest
       ss += b * b;
     }
   }
-  ss = row_total<WPR>(ss);
-  const float denom = sqrtf(ss) * factor + eps;
+  ss = row_total<WHOLE>(ss);
+  const Divisor denom(sqrtf(ss) * factor + eps);
   uint16_t* orow = out + row * o_rs;
 #pragma unroll
   for (int c = 0; c < MAXC; ++c) {
@@ -78,14 +116,9 @@ __global__ __launch_bounds__(NT) void rmsnorm_rows_kernel(const uint16_t* __rest
     if (ch >= nchunks) break;
     const f32x4_t w0 = *(const f32x4_t*)(weight + ch * 8);
     const f32x4_t w1 = *(const f32x4_t*)(weight + ch * 8 + 4);
-    u32x4_t o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float wa = e < 2 ? w0[2 * e] : w1[2 * e - 4];
-      const float wb = e < 2 ? w0[2 * e + 1] : w1[2 * e - 3];
-      o[e] = pack_bf16((bf16_lo(v[c][e]) / denom) * wa, (bf16_hi(v[c][e]) / denom) * wb);
-    }
-    *(u32x4_t*)(orow + ch * 8) = o;
+    float f[8];
+    unpack(v[c], f);
+    normalised(f, denom, w0, w1, [&](const float (&y)[8]) { *(u32x4_t*)(orow + ch * 8) = packed(y); });
   }
 }
 
@@ -93,14 +126,14 @@ __global__ __launch_bounds__(NT) void rmsnorm_rows_kernel(const uint16_t* __rest
 // the normalisation that follows it (keys_values/model.py:560-584: x = attention_output + x, then
 // norm_2(x); x = mlp_output + x, then the next block's norm_1). The sum is rounded to bf16 before it is
 // normalised, as the two separate steps do. In place is allowed (x_out == x).
-template <int MAXC, int WPR>
-__global__ __launch_bounds__(NT) void add_rmsnorm_rows_kernel(const uint16_t* x, int64_t x_rs, const uint16_t* __restrict__ delta,
+template <int MAXC, bool WHOLE>
+__global__ __launch_bounds__(64 * MAX_WAVES) void add_rmsnorm_rows_kernel(const uint16_t* x, int64_t x_rs, const uint16_t* __restrict__ delta,
                                                               int64_t d_rs, uint16_t* x_out, int64_t xo_rs,
                                                               uint16_t* __restrict__ out, int64_t o_rs, const float* __restrict__ weight,
                                                               int64_t rows, int dim, float eps, float factor) {
-  constexpr int TPR = 64 * WPR;
-  const int lane = threadIdx.x % TPR;
-  const int64_t row = (int64_t)blockIdx.x * (NT / TPR) + threadIdx.x / TPR;
+  const int TPR = WHOLE ? blockDim.x : 64;
+  const int lane = WHOLE ? threadIdx.x : threadIdx.x & 63;
+  const int64_t row = WHOLE ? blockIdx.x : (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
   if (row >= rows) return;
   const int nchunks = dim / 8;
   u32x4_t v[MAXC];
@@ -123,8 +156,8 @@ __global__ __launch_bounds__(NT) void add_rmsnorm_rows_kernel(const uint16_t* x,
       ss += b * b;
     }
   }
-  ss = row_total<WPR>(ss);
-  const float denom = sqrtf(ss) * factor + eps;
+  ss = row_total<WHOLE>(ss);
+  const Divisor denom(sqrtf(ss) * factor + eps);
   uint16_t* orow = out + row * o_rs;
 #pragma unroll
   for (int c = 0; c < MAXC; ++c) {
@@ -132,14 +165,9 @@ __global__ __launch_bounds__(NT) void add_rmsnorm_rows_kernel(const uint16_t* x,
     if (ch >= nchunks) break;
     const f32x4_t w0 = *(const f32x4_t*)(weight + ch * 8);
     const f32x4_t w1 = *(const f32x4_t*)(weight + ch * 8 + 4);
-    u32x4_t o;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float wa = e < 2 ? w0[2 * e] : w1[2 * e - 4];
-      const float wb = e < 2 ? w0[2 * e + 1] : w1[2 * e - 3];
-      o[e] = pack_bf16((bf16_lo(v[c][e]) / denom) * wa, (bf16_hi(v[c][e]) / denom) * wb);
-    }
-    *(u32x4_t*)(orow + ch * 8) = o;
+    float f[8];
+    unpack(v[c], f);
+    normalised(f, denom, w0, w1, [&](const float (&y)[8]) { *(u32x4_t*)(orow + ch * 8) = packed(y); });
   }
 }
 
@@ -147,92 +175,120 @@ __global__ __launch_bounds__(NT) void add_rmsnorm_rows_kernel(const uint16_t* x,
 // gated activation of LLaMAMLP (proj(silu(fc_1 x) * fc_2 x)) on the output of one GEMM over the stacked
 // fc_1 / fc_2 weights. silu is x / (1 + exp(-x)) in fp32, rounded to bf16 before the product, as the
 // two separate tensor operations round.
+// exp(-x) is 2^h (1 + l ln 2) with h + l = -x log2(e), h rounded; the quotient as in Divisor, of a reciprocal that is an ulp off. Values below -80, whose
+// exponential is near the type's end, and NaN take the divisions. With expf, a division each and 64-bit indexes the kernel was bound by the vector ALU:
+// 4096 / 1024 rows of 9728 values 42.2 -> 39.3 and 13.3 -> 12.1 us.
+__device__ __forceinline__ float silu(float x) {
+  constexpr float L2E = 1.4426950408889634f, L2E_LOW = (float)(1.4426950408889634 - (double)L2E), LN2 = 0.6931471805599453f;
+  const float h = x * -L2E, l = fmaf(x, -L2E, -h) + x * -L2E_LOW;
+  const float p = fast_exp2(h), d = 1.0f + fmaf(p, l * LN2, p);
+  const float r = __builtin_amdgcn_rcpf(d), q = x * r;
+  return fmaf(fmaf(-q, d, x), r, q);
+}
 __global__ __launch_bounds__(NT) void swiglu_rows_kernel(const uint16_t* __restrict__ gate_up, int64_t g_rs, uint16_t* __restrict__ out,
-                                                         int64_t o_rs, int64_t rows, int dim) {
-  const int cpr = dim / 8;
-  const int64_t gid = (int64_t)blockIdx.x * NT + threadIdx.x;
-  if (gid >= rows * cpr) return;
+                                                         int64_t o_rs, uint32_t rows, int dim) {
+  const uint32_t cpr = dim / 8, gid = blockIdx.x * NT + threadIdx.x;
   const int64_t r = gid / cpr;
-  const int c = (int)(gid % cpr);
+  const int c = gid % cpr;
+  if (r >= rows) return;
   const u32x4_t g = *(const u32x4_t*)(gate_up + r * g_rs + c * 8);
   const u32x4_t u = *(const u32x4_t*)(gate_up + r * g_rs + dim + c * 8);
+  float x[8];
+  unpack(g, x);
+  bool plain = true;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) plain = plain && x[e] > -80.0f && x[e] < 0x1p100f;
+  u32x4_t act;
+  if (__all(plain)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) act[e] = pack_bf16(silu(x[2 * e]), silu(x[2 * e + 1]));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) act[e] = pack_bf16(x[2 * e] / (1.0f + expf(-x[2 * e])), x[2 * e + 1] / (1.0f + expf(-x[2 * e + 1])));
+  }
   u32x4_t o;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const float g0 = bf16_lo(g[e]), g1 = bf16_hi(g[e]);
-    const uint32_t act = pack_bf16(g0 / (1.0f + expf(-g0)), g1 / (1.0f + expf(-g1)));
-    o[e] = pack_bf16(bf16_lo(act) * bf16_lo(u[e]), bf16_hi(act) * bf16_hi(u[e]));
-  }
+  for (int e = 0; e < 4; ++e) o[e] = pack_bf16(bf16_lo(act[e]) * bf16_lo(u[e]), bf16_hi(act[e]) * bf16_hi(u[e]));
   *(u32x4_t*)(out + r * o_rs + c * 8) = o;
 }
 
-// One lane per 8 elements of a head row; LPR = D / 8 lanes share a row. Rows are (b, t, head) with
-// head in [0, Hq + Hkv): the query heads, then the key heads, of token t.
-template <int D>
-__global__ __launch_bounds__(NT) void qk_norm_rope_kernel(uint16_t* __restrict__ qkv, int64_t sb, int64_t st, int B, int num, int Hq,
+// A workgroup per token: the rows are its query heads, then its key heads; LPR = D / 8 lanes a row hold four values of either half of it, so
+// a value and the one it is rotated with are in the same lane; the angles and weights of a lane are the same for all its rows. With a row's values in a
+// stretch a lane, partners through LDS and a row's place by 64-bit divisions: 27 -> 20.8 us for 40 heads of 4096 tokens, 10.4 -> 7.4 of 1024.
+template <int D, int U>  // U: rows of a lane in flight
+__global__ __launch_bounds__(64 * MAX_WAVES) void qk_norm_rope_kernel(uint16_t* __restrict__ qkv, int64_t sb, int64_t st, int num, int Hq,
                                                           int Hkv, const float* __restrict__ qw, const float* __restrict__ kw,
                                                           float eps, float factor, const float* __restrict__ cos_t,
                                                           const float* __restrict__ sin_t, int input_pos) {
   constexpr int LPR = D / 8;
   constexpr int HALF = D / 2;
-  const int col = threadIdx.x % LPR;
-  const int64_t rid = (int64_t)blockIdx.x * (NT / LPR) + threadIdx.x / LPR;
+  const int col = threadIdx.x % LPR, first = threadIdx.x / LPR, rows = blockDim.x / LPR;
   const int heads = Hq + Hkv;
-  const int64_t total = (int64_t)B * num * heads;
-  const bool live = rid < total;
-  const int64_t r = live ? rid : 0;  // dead lanes follow row 0 so that the shuffles below stay defined
-  const int head = (int)(r % heads);
-  const int t = (int)((r / heads) % num);
-  const int b = (int)(r / ((int64_t)heads * num));
-  uint16_t* p = qkv + b * sb + (int64_t)t * st + (int64_t)head * D + col * 8;
-  const u32x4_t raw = *(const u32x4_t*)p;
-  float y[8];
+  const int b = blockIdx.x / num, t = blockIdx.x - b * num;
+  uint16_t* p = qkv + b * sb + (int64_t)t * st + col * 4;
+  const f32x4_t cv = *(const f32x4_t*)(cos_t + (int64_t)(input_pos + t) * HALF + col * 4);
+  const f32x4_t sv = *(const f32x4_t*)(sin_t + (int64_t)(input_pos + t) * HALF + col * 4);
+  for (int begin = 0; begin < heads; begin += U * rows) {
+    u32x2_t lo[U], hi[U];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    y[2 * e] = bf16_lo(raw[e]);
-    y[2 * e + 1] = bf16_hi(raw[e]);
-  }
-  const float* w = head < Hq ? qw : kw;
-  if (w) {  // uniform: either both weights are given or none
-    float ss = 0.0f;
+    for (int i = 0; i < U; ++i) {
+      const int head = min(begin + i * rows + first, heads - 1);
+      lo[i] = *(const u32x2_t*)(p + head * D);
+      hi[i] = *(const u32x2_t*)(p + head * D + HALF);
+    }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) ss += y[e] * y[e];
+    for (int i = 0; i < U; ++i) {
+      const int head = begin + i * rows + first;
+      float y[8];
+      unpack(u32x4_t{lo[i][0], lo[i][1], hi[i][0], hi[i][1]}, y);
+      if (qw) {  // either both weights are given or none
+        float ss = 0.0f;
 #pragma unroll
-    for (int off = 1; off < LPR; off <<= 1) ss += __shfl_xor(ss, off, 64);
-    const float denom = sqrtf(ss) * factor + eps;
-    const f32x4_t w0 = *(const f32x4_t*)(w + col * 8);
-    const f32x4_t w1 = *(const f32x4_t*)(w + col * 8 + 4);
+        for (int e = 0; e < 8; ++e) ss += y[e] * y[e];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float wv = e < 4 ? w0[e] : w1[e - 4];
-      // the reference casts the normalised head back to bf16 before it is rotated
-      y[e] = bf16_bits_to_f32(pack_bf16((y[e] / denom) * wv, 0.0f) & 0xffffu);
+        for (int off = 1; off < LPR; off <<= 1) ss += __shfl_xor(ss, off, 64);
+        const float* w = (head < Hq ? qw : kw) + col * 4;
+        normalised(y, Divisor(sqrtf(ss) * factor + eps), *(const f32x4_t*)w, *(const f32x4_t*)(w + HALF), [&](const float (&z)[8]) {
+          // the reference casts the normalised head back to bf16 before it is rotated
+          unpack(packed(z), y);
+        });
+      }
+      // rotation: the first half gets -x2, the second +x1
+      float x[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        x[e] = y[e] * cv[e] + -y[e + 4] * sv[e];
+        x[e + 4] = y[e + 4] * cv[e] + y[e] * sv[e];
+      }
+      const u32x4_t o = packed(x);
+      if (head < heads) {
+        *(u32x2_t*)(p + head * D) = u32x2_t{o[0], o[1]};
+        *(u32x2_t*)(p + head * D + HALF) = u32x2_t{o[2], o[3]};
+      }
     }
   }
-  // rotation: element d pairs with d +- D/2, held by the lane LPR/2 away; first half gets -x2, second +x1
-  const bool first = col < LPR / 2;
-  const int j0 = (col * 8) % HALF;
-  const float* cr = cos_t + (int64_t)(input_pos + t) * HALF + j0;
-  const float* sr = sin_t + (int64_t)(input_pos + t) * HALF + j0;
-  const f32x4_t c0 = *(const f32x4_t*)cr, c1 = *(const f32x4_t*)(cr + 4);
-  const f32x4_t s0 = *(const f32x4_t*)sr, s1 = *(const f32x4_t*)(sr + 4);
-  u32x4_t o;
-  float res[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float other = __shfl_xor(y[e], LPR / 2, 64);
-    const float rot = first ? -other : other;
-    const float cv = e < 4 ? c0[e] : c1[e - 4];
-    const float sv = e < 4 ? s0[e] : s1[e - 4];
-    res[e] = y[e] * cv + rot * sv;
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) o[e] = pack_bf16(res[2 * e], res[2 * e + 1]);
-  if (live) *(u32x4_t*)p = o;
 }
 
-// Rows of at least 2048 values, too few of them to fill the chip with a wavefront each.
-bool workgroup_per_row(int64_t rows, int dim) { return dim >= 2048 && dim <= NT * 8 * 4 && rows <= 16384; }
+// Wavefronts of a workgroup that takes a row, where rows of at least 2048 values are too few to fill the chip with a wavefront each (0: a wavefront
+// a row). us, four wavefronts and a division a value -> now: sum and norm of 4096 rows of 2560 18.7 -> 17.0, of 1024 7.4 -> 6.8.
+int row_waves(int64_t rows, int dim) {
+  if (dim < 2048 || dim > 64 * MAX_WAVES * 8 * 4 || rows > 16384) return 0;
+  const int chunks = (dim + 511) / 512;  // of a wavefront
+  const int each = (chunks + MAX_WAVES - 1) / MAX_WAVES;
+  return (chunks + each - 1) / each;
+}
+
+// `launch(chunks a lane, whole workgroup a row, grid, threads)`
+template <typename Launch>
+void by_row_length(int64_t rows, int dim, Launch launch) {
+  const int waves = row_waves(rows, dim);
+  const unsigned grid = (unsigned)(waves ? rows : (rows + NT / 64 - 1) / (NT / 64));
+  const int chunks = (dim / 8 + 64 * max(waves, 1) - 1) / (64 * max(waves, 1));
+  if (waves && chunks == 1) launch(std::integral_constant<int, 1>{}, std::true_type{}, grid, 64 * waves);
+  else if (waves) launch(std::integral_constant<int, 4>{}, std::true_type{}, grid, 64 * waves);
+  else if (chunks <= 4) launch(std::integral_constant<int, 4>{}, std::false_type{}, grid, NT);
+  else launch(std::integral_constant<int, 16>{}, std::false_type{}, grid, NT);
+}
 
 }  // namespace
 
@@ -240,17 +296,10 @@ int launch_rmsnorm_rows(const void* x, int64_t x_rs, void* out, int64_t o_rs, co
                         hipStream_t st) {
   if (rows == 0) return KVX_OK;
   const float factor = 1.0f / sqrtf((float)dim);
-  const unsigned grid = (unsigned)((rows + NT / 64 - 1) / (NT / 64));
-  const int chunks_per_lane = (dim / 8 + 63) / 64;
-  if (workgroup_per_row(rows, dim))
-    hipLaunchKernelGGL((rmsnorm_rows_kernel<4, NT / 64>), dim3((unsigned)rows), dim3(NT), 0, st, (const uint16_t*)x, x_rs, (uint16_t*)out, o_rs,
-                       weight, rows, dim, eps, factor);
-  else if (chunks_per_lane <= 4)
-    hipLaunchKernelGGL((rmsnorm_rows_kernel<4, 1>), dim3(grid), dim3(NT), 0, st, (const uint16_t*)x, x_rs, (uint16_t*)out, o_rs, weight, rows,
-                       dim, eps, factor);
-  else
-    hipLaunchKernelGGL((rmsnorm_rows_kernel<16, 1>), dim3(grid), dim3(NT), 0, st, (const uint16_t*)x, x_rs, (uint16_t*)out, o_rs, weight, rows,
-                       dim, eps, factor);
+  by_row_length(rows, dim, [&](auto chunks, auto whole, unsigned grid, int threads) {
+    hipLaunchKernelGGL((rmsnorm_rows_kernel<decltype(chunks)::value, decltype(whole)::value>), dim3(grid), dim3(threads), 0, st, (const uint16_t*)x, x_rs,
+                       (uint16_t*)out, o_rs, weight, rows, dim, eps, factor);
+  });
   KVX_HIP(hipGetLastError());
   return KVX_OK;
 }
@@ -259,45 +308,45 @@ int launch_add_rmsnorm_rows(const void* x, int64_t x_rs, const void* delta, int6
                             int64_t o_rs, const float* weight, int64_t rows, int dim, float eps, hipStream_t st) {
   if (rows == 0) return KVX_OK;
   const float factor = 1.0f / sqrtf((float)dim);
-  const unsigned grid = (unsigned)((rows + NT / 64 - 1) / (NT / 64));
-  if (workgroup_per_row(rows, dim))
-    hipLaunchKernelGGL((add_rmsnorm_rows_kernel<4, NT / 64>), dim3((unsigned)rows), dim3(NT), 0, st, (const uint16_t*)x, x_rs,
+  by_row_length(rows, dim, [&](auto chunks, auto whole, unsigned grid, int threads) {
+    hipLaunchKernelGGL((add_rmsnorm_rows_kernel<decltype(chunks)::value, decltype(whole)::value>), dim3(grid), dim3(threads), 0, st, (const uint16_t*)x, x_rs,
                        (const uint16_t*)delta, d_rs, (uint16_t*)x_out, xo_rs, (uint16_t*)out, o_rs, weight, rows, dim, eps, factor);
-  else if ((dim / 8 + 63) / 64 <= 4)
-    hipLaunchKernelGGL((add_rmsnorm_rows_kernel<4, 1>), dim3(grid), dim3(NT), 0, st, (const uint16_t*)x, x_rs, (const uint16_t*)delta, d_rs,
-                       (uint16_t*)x_out, xo_rs, (uint16_t*)out, o_rs, weight, rows, dim, eps, factor);
-  else
-    hipLaunchKernelGGL((add_rmsnorm_rows_kernel<16, 1>), dim3(grid), dim3(NT), 0, st, (const uint16_t*)x, x_rs, (const uint16_t*)delta, d_rs,
-                       (uint16_t*)x_out, xo_rs, (uint16_t*)out, o_rs, weight, rows, dim, eps, factor);
+  });
   KVX_HIP(hipGetLastError());
   return KVX_OK;
 }
 
 int launch_swiglu_rows(const void* gate_up, int64_t g_rs, void* out, int64_t o_rs, int64_t rows, int dim, hipStream_t st) {
-  const int64_t total = rows * (dim / 8);
-  if (total == 0) return KVX_OK;
-  hipLaunchKernelGGL(swiglu_rows_kernel, dim3((unsigned)((total + NT - 1) / NT)), dim3(NT), 0, st, (const uint16_t*)gate_up, g_rs,
-                     (uint16_t*)out, o_rs, rows, dim);
-  KVX_HIP(hipGetLastError());
+  const int64_t at_once = (1u << 31) / (dim / 8);  // rows whose chunks have 32-bit indexes
+  for (int64_t done = 0; done < rows; done += at_once) {
+    const int64_t n = rows - done < at_once ? rows - done : at_once;
+    hipLaunchKernelGGL(swiglu_rows_kernel, dim3((unsigned)((n * (dim / 8) + NT - 1) / NT)), dim3(NT), 0, st, (const uint16_t*)gate_up + done * g_rs, g_rs,
+                       (uint16_t*)out + done * o_rs, o_rs, (uint32_t)n, dim);
+    KVX_HIP(hipGetLastError());
+  }
   return KVX_OK;
 }
 
 int launch_qk_norm_rope(void* qkv, int64_t sb, int64_t stt, int B, int num, int Hq, int Hkv, int D, const float* qw, const float* kw,
                         float eps, const float* cos_t, const float* sin_t, int input_pos, hipStream_t st) {
-  const int64_t total = (int64_t)B * num * (Hq + Hkv);
-  if (total == 0) return KVX_OK;
+  if (B == 0 || num == 0 || Hq + Hkv == 0) return KVX_OK;
   const float factor = 1.0f / sqrtf((float)D);
-  const int rpb = NT / (D / 8);
-  const unsigned grid = (unsigned)((total + rpb - 1) / rpb);
-  if (D == 256)
-    hipLaunchKernelGGL(qk_norm_rope_kernel<256>, dim3(grid), dim3(NT), 0, st, (uint16_t*)qkv, sb, stt, B, num, Hq, Hkv, qw, kw, eps, factor,
-                       cos_t, sin_t, input_pos);
-  else if (D == 128)
-    hipLaunchKernelGGL(qk_norm_rope_kernel<128>, dim3(grid), dim3(NT), 0, st, (uint16_t*)qkv, sb, stt, B, num, Hq, Hkv, qw, kw, eps, factor,
-                       cos_t, sin_t, input_pos);
-  else
-    hipLaunchKernelGGL(qk_norm_rope_kernel<64>, dim3(grid), dim3(NT), 0, st, (uint16_t*)qkv, sb, stt, B, num, Hq, Hkv, qw, kw, eps, factor,
-                       cos_t, sin_t, input_pos);
+  const int lanes = (Hq + Hkv) * (D / 8), rows = lanes <= NT ? 1 : 2;  // of a lane, and more where the workgroup is too small
+  const int threads = min(64 * MAX_WAVES, (lanes / rows + 63) / 64 * 64);
+  const int at_once = max(1, (1 << 22) / num);  // batch elements whose threads a grid can count
+  auto launch = [&](auto kernel) {
+    for (int done = 0; done < B; done += at_once)
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(min(at_once, B - done) * num)), dim3(threads), 0, st, (uint16_t*)qkv + done * sb, sb, stt, num, Hq, Hkv, qw, kw, eps,
+                         factor, cos_t, sin_t, input_pos);
+  };
+  auto launch_d = [&](auto d_tag) {
+    constexpr int HEAD = decltype(d_tag)::value;
+    if (rows == 1) launch(qk_norm_rope_kernel<HEAD, 1>);
+    else launch(qk_norm_rope_kernel<HEAD, 2>);
+  };
+  if (D == 256) launch_d(std::integral_constant<int, 256>{});
+  else if (D == 128) launch_d(std::integral_constant<int, 128>{});
+  else launch_d(std::integral_constant<int, 64>{});
   KVX_HIP(hipGetLastError());
   return KVX_OK;
 }

@@ -1,0 +1,67 @@
+"""Normalisation, activation and rotary rows (csrc/norm_rope.hip) where their arithmetic or their split of a row changes: every 16-bit gate,
+norms beyond the range of the shared reciprocal, row lengths and head counts on both sides of a workgroup's sizes."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from keys_values_amd.longctx import ops
+from oracle import longctx_oracle as LO
+
+pytestmark = pytest.mark.gpu
+
+
+def test_swiglu_of_every_gate(gpu):
+    # neighbours share a wavefront with the extremes, and once without them
+    gates = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    for g in (gates, gates[(gates.float() > -79) & (gates.float() < 1e30)]):
+        g = g[: g.numel() // 16 * 16].view(1, -1)
+        out = ops.swiglu(torch.cat((g, torch.ones_like(g)), 1).to(gpu)).cpu()
+        g64 = g.double()
+        exact = torch.where(g64 == -float("inf"), torch.nan, g64 / (1 + torch.exp(-g64)))  # -inf / inf
+        seen = exact.abs() > 2.7e-37  # exp(88.73) is infinite in 32 bits, as it is in torch: gates from there on, of -2.6e-37, give 0
+        assert torch.equal(out.isnan(), exact.isnan())
+        torch.testing.assert_close(out.double()[seen], exact[seen], rtol=2**-8 + 1e-6, atol=0)  # half a unit of 8 bits, and 32-bit arithmetic
+        assert (out.double()[~seen & ~exact.isnan()].abs() < 2.8e-37).all()
+        ref = F.silu(g)
+        assert ((out != ref) & ~ref.isnan()).float().mean().item() < 1e-3
+
+
+@pytest.mark.parametrize("dim", [8, 520, 2040, 2048, 2560, 4104, 8192])
+def test_norms_out_of_range(gpu, dim):
+    gen = torch.Generator().manual_seed(dim)
+    x = torch.randn(9, dim, generator=gen).to(torch.bfloat16)
+    x[1] = 0.0  # with eps = 0: 0 / 0
+    x[2] *= 1e30  # the sum of squares is infinite
+    x[3] *= 1e-15  # norm below the range
+    x[4] *= 1e14  # above
+    x[5, 0] = float("inf")
+    x[6, 0] = float("nan")
+    weight = torch.rand(dim, generator=gen) + 0.5
+    for eps in (0.0, 1e-6):
+        ref = LO.rmsnorm(x, weight, eps)
+        ref[2] = 0.0  # the row's norm overflows in 32 bits
+        assert torch.equal(ref[1].isnan(), torch.full((dim,), eps == 0.0))
+        out = ops.rmsnorm(x.to(gpu), weight.to(gpu), eps).cpu()
+        half = (x.float() / 2).to(torch.bfloat16)
+        added = ops.add_rmsnorm_(half.to(gpu), half.to(gpu), weight.to(gpu), eps).cpu()
+        for got in (out, added):
+            torch.testing.assert_close(got.float(), ref.float(), rtol=2**-7, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(1, 1, 64), (8, 2, 64), (28, 4, 64), (29, 4, 64), (12, 4, 128), (13, 4, 128), (32, 8, 128), (64, 8, 128), (32, 8, 256)])
+def test_rope_head_counts(gpu, Hq, Hkv, D):
+    gen = torch.Generator().manual_seed(Hq)
+    B, num, pos = 2, 5, 11
+    qkv = (torch.randn(B, num, (Hq + 2 * Hkv) * D, generator=gen) * 2).to(torch.bfloat16)
+    qkv[0, 0, :D] = 0.0
+    qw, kw = (torch.rand(D, generator=gen) + 0.5 for _ in range(2))
+    cos, sin = LO.rope_tables(64, D, 1e6)
+    for w in ((qw, kw), (None, None)):
+        refs = LO.qk_norm_rope(qkv, Hq, Hkv, D, *w, 1e-6, cos, sin, pos)
+        g = qkv.to(gpu)
+        ops.qk_norm_rope_(g, Hq, Hkv, D, *(None if t is None else t.to(gpu) for t in w), 1e-6, cos.to(gpu), sin.to(gpu), pos)
+        out = g.cpu().view(B, num, Hq + 2 * Hkv, D).transpose(1, 2)
+        for got, ref in zip(out.split((Hq, Hkv, Hkv), 1), refs):
+            # one rounding to 16 bits may go the other way before the rotation and one after it
+            torch.testing.assert_close(got.float(), ref.float(), rtol=2**-6, atol=2**-6)
+            assert (got != ref).float().mean().item() < 5e-3
