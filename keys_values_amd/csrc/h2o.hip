@@ -102,6 +102,50 @@ __device__ __forceinline__ float block_reduce(float v, float* red, Op op) {
   return r;
 }
 
+// The value of the lane whose index differs in bit log2(S), on the vector ALU.
+template <int S>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+  auto dpp = [](uint32_t x, auto ctrl) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, decltype(ctrl)::value, 0xf, 0xf, true); };
+  if constexpr (S == 1) return dpp(v, std::integral_constant<int, 0xB1>{});        // quad_perm [1,0,3,2]
+  else if constexpr (S == 2) return dpp(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+  else if constexpr (S == 4) return dpp(dpp(v, std::integral_constant<int, 0x141>{}), std::integral_constant<int, 0x1B>{});  // half mirror, quad mirror
+  else if constexpr (S == 8) return dpp(v, std::integral_constant<int, 0x128>{});  // row_ror:8
+  else if constexpr (S == 16) {
+    const u32pair_t r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return (threadIdx.x & 16) ? r[0] : r[1];
+  } else {
+    const u32pair_t r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return (threadIdx.x & 32) ? r[0] : r[1];
+  }
+}
+
+// Least, largest, least and largest of a workgroup's four values in one exchange: four reductions one after the other took a third of the launches that
+// need them (16 rows of 6000 slots, us: statistics 8.2 -> 7.3, sort 6.3 -> 5.5). Called once by a kernel.
+template <int THREADS>
+__device__ __forceinline__ f32x4_t block_extremes(f32x4_t v) {
+  __shared__ f32x4_t red[THREADS / 64];
+  auto fold = [](const f32x4_t& x, const f32x4_t& y) { return f32x4_t{fminf(x[0], y[0]), fmaxf(x[1], y[1]), fminf(x[2], y[2]), fmaxf(x[3], y[3])}; };
+  auto lanes = [&](auto s_tag) {
+    constexpr int S = decltype(s_tag)::value;
+    f32x4_t o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = __uint_as_float(lane_xor<S>(__float_as_uint(v[i])));
+    v = fold(v, o);
+  };
+  lanes(std::integral_constant<int, 32>{});
+  lanes(std::integral_constant<int, 16>{});
+  lanes(std::integral_constant<int, 8>{});
+  lanes(std::integral_constant<int, 4>{});
+  lanes(std::integral_constant<int, 2>{});
+  lanes(std::integral_constant<int, 1>{});
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  f32x4_t r = red[0];
+#pragma unroll
+  for (int i = 1; i < THREADS / 64; ++i) r = fold(r, red[i]);
+  return r;
+}
+
 // One workgroup per (batch, head) row: scores += instantaneous score, where the latter is w or,
 // with v_norm, (v_norm*w / sum(v_norm*w)) * q_len (keys_values/kvcache/h2o.py:297-314); and the row's
 // min / max of the compared value and of q_errors over the slots below limit, for the combination.
@@ -157,13 +201,8 @@ __global__ __launch_bounds__(SEL_THREADS) void accumulate_kernel(const kvx_h2o_a
     }
   }
   if (qe) {
-    auto mn = [](float x, float y) { return fminf(x, y); };
-    auto mx = [](float x, float y) { return fmaxf(x, y); };
-    smin = block_reduce(smin, red, mn);
-    smax = block_reduce(smax, red, mx);
-    qmin = block_reduce(qmin, red, mn);
-    qmax = block_reduce(qmax, red, mx);
-    if (tid == 0) *(f32x4_t*)(stats + (int64_t)row * 4) = f32x4_t{smin, smax, qmin, qmax};
+    const f32x4_t x = block_extremes<SEL_THREADS>(f32x4_t{smin, smax, qmin, qmax});
+    if (tid == 0) *(f32x4_t*)(stats + (int64_t)row * 4) = x;
   }
 }
 
@@ -246,7 +285,6 @@ constexpr int SEL_ONE = 8 * SEL_THREADS;
 
 __global__ __launch_bounds__(SEL_THREADS) void select_one_kernel(const kvx_h2o_args a, const float* stats, int per_row, uint32_t* counters,
                                                                  unsigned long long* part) {
-  __shared__ float red[SEL_THREADS / 64];
   __shared__ unsigned long long wbest[SEL_THREADS / 64];
   __shared__ uint32_t last;
   const int tid = threadIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
@@ -270,14 +308,13 @@ __global__ __launch_bounds__(SEL_THREADS) void select_one_kernel(const kvx_h2o_a
     s8[i] = sc[k];
     q8[i] = qe[k];
   }
-  auto mn = [](float x, float y) { return fminf(x, y); };
-  auto mx = [](float x, float y) { return fmaxf(x, y); };
+  const f32x4_t ex = block_extremes<SEL_THREADS>(f32x4_t{v4[0], v4[1], v4[2], v4[3]});
   Modify m;
   m.qe = qe;
-  m.smin = block_reduce(v4[0], red, mn);
-  m.sden = block_reduce(v4[1], red, mx) - m.smin;
-  m.qmin = block_reduce(v4[2], red, mn);
-  m.qden = block_reduce(v4[3], red, mx) - m.qmin;
+  m.smin = ex[0];
+  m.sden = ex[1] - m.smin;
+  m.qmin = ex[2];
+  m.qden = ex[3] - m.qmin;
   m.c = (float)a.combination;
   m.c2 = (float)((a.combination - 1.0) / 2.0);
   m.c3 = (float)(1.0 - a.combination);
@@ -412,28 +449,8 @@ __global__ __launch_bounds__(LIST) void list_stats_kernel(const kvx_h2o_args a, 
   const float v = updated_score(a, z, row, b, hh, slot);
   const int32_t* tpr = a.token_pos ? a.token_pos + b * a.tp_stride_b + hh * a.tp_stride_h : nullptr;
   const float cv = in ? residency_value(v, a, tpr, slot) : 0.0f;
-  auto mn = [](float x, float y) { return fminf(x, y); };
-  auto mx = [](float x, float y) { return fmaxf(x, y); };
-  const float smin = block_reduce(in ? cv : INFINITY, red, mn), smax = block_reduce(in ? cv : -INFINITY, red, mx);
-  const float qmin = block_reduce(in ? qe : INFINITY, red, mn), qmax = block_reduce(in ? qe : -INFINITY, red, mx);
-  if (threadIdx.x == 0) *(f32x4_t*)(sl.stats + ((int64_t)row * sl.C + c) * 4) = f32x4_t{smin, smax, qmin, qmax};
-}
-
-// The value of the lane whose index differs in bit log2(S), on the vector ALU.
-template <int S>
-__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
-  auto dpp = [](uint32_t x, auto ctrl) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, decltype(ctrl)::value, 0xf, 0xf, true); };
-  if constexpr (S == 1) return dpp(v, std::integral_constant<int, 0xB1>{});        // quad_perm [1,0,3,2]
-  else if constexpr (S == 2) return dpp(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
-  else if constexpr (S == 4) return dpp(dpp(v, std::integral_constant<int, 0x141>{}), std::integral_constant<int, 0x1B>{});  // half mirror, quad mirror
-  else if constexpr (S == 8) return dpp(v, std::integral_constant<int, 0x128>{});  // row_ror:8
-  else if constexpr (S == 16) {
-    const u32pair_t r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    return (threadIdx.x & 16) ? r[0] : r[1];
-  } else {
-    const u32pair_t r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    return (threadIdx.x & 32) ? r[0] : r[1];
-  }
+  const f32x4_t ex = block_extremes<LIST>(f32x4_t{in ? cv : INFINITY, in ? cv : -INFINITY, in ? qe : INFINITY, in ? qe : -INFINITY});
+  if (threadIdx.x == 0) *(f32x4_t*)(sl.stats + ((int64_t)row * sl.C + c) * 4) = ex;
 }
 
 // Sum over the wavefront in the order of block_reduce's exchanges.
@@ -502,13 +519,12 @@ __global__ __launch_bounds__(L) void list_sort_kernel(const kvx_h2o_args a, cons
       v4[2] = fminf(v4[2], s4[2]);
       v4[3] = fmaxf(v4[3], s4[3]);
     }
-    auto mn = [](float u, float w) { return fminf(u, w); };
-    auto mx = [](float u, float w) { return fmaxf(u, w); };
+    const f32x4_t ex = block_extremes<L>(f32x4_t{v4[0], v4[1], v4[2], v4[3]});
     Modify m;
-    m.smin = block_reduce<L>(v4[0], red, mn);
-    m.sden = block_reduce<L>(v4[1], red, mx) - m.smin;
-    m.qmin = block_reduce<L>(v4[2], red, mn);
-    m.qden = block_reduce<L>(v4[3], red, mx) - m.qmin;
+    m.smin = ex[0];
+    m.sden = ex[1] - m.smin;
+    m.qmin = ex[2];
+    m.qden = ex[3] - m.qmin;
     m.c = (float)a.combination;
     m.c2 = (float)((a.combination - 1.0) / 2.0);
     m.c3 = (float)(1.0 - a.combination);
