@@ -35,10 +35,12 @@ __device__ __forceinline__ uint32_t ordered_bits(float x) {
 
 // Value the selection compares: the score, or the score divided by the slot's residency
 // (keys_values/kvcache/h2o.py:183-196).
-__device__ __forceinline__ float residency_value(float score, const kvx_h2o_args& a, const int32_t* tp_row, int idx) {
+__device__ __forceinline__ float residency_of(float score, const kvx_h2o_args& a, int position) {  // (of a slot's token)
   if (!a.normalize) return score;
-  const int t = max(tp_row[idx], a.prefill_len - 1);
-  return score / (float)(a.input_pos - t);
+  return score / (float)(a.input_pos - max(position, a.prefill_len - 1));
+}
+__device__ __forceinline__ float residency_value(float score, const kvx_h2o_args& a, const int32_t* tp_row, int idx) {
+  return residency_of(score, a, a.normalize ? tp_row[idx] : 0);
 }
 
 // Q-Hitter combination (keys_values/kvcache/qh2o.py:178-210): both terms are min-max normalised over
@@ -420,21 +422,28 @@ __device__ __forceinline__ float row_norm(const kvx_h2o_args& a, int C, int row,
   return wave_total(z);
 }
 
-// The score of this thread's slot after the update (stored), and the slot; `z`: the row's sum of v_norm * w. Every product and sum
-// rounded on its own.
-__device__ __forceinline__ float updated_score(const kvx_h2o_args& a, float z, int row, int b, int hh, int slot) {
-  const int64_t off = b * a.sc_stride_b + hh * a.sc_stride_h;
+// What a thread needs of its slot, asked for at once and ahead of the sums over the row, behind whose barriers each would be a latency of its own.
+struct Slot {
+  float score, w, v_norm;
+  int position;
+};
+__device__ __forceinline__ Slot load_slot(const kvx_h2o_args& a, int row, int b, int hh, int slot) {
+  const int64_t off = b * a.sc_stride_b + hh * a.sc_stride_h + slot;
   const bool in = slot < a.kv_len;
-  const float s = in ? a.scores[off + slot] : 0.0f;
-  if (!a.w) return s;
-  const float w = in ? a.w[(int64_t)row * a.kv_len + slot] : 0.0f;
-  float inst = w;
-  if (a.v_norm) {
-    const float vn = in ? a.v_norm[off + slot] : 0.0f;
-    inst = __fmul_rn(__fmul_rn(vn, w) / z, (float)a.q_len);
-  }
-  const float v = __fadd_rn(s, inst);
-  if (in) a.scores[off + slot] = v;
+  Slot s;
+  s.score = in ? a.scores[off] : 0.0f;
+  s.w = in && a.w ? a.w[(int64_t)row * a.kv_len + slot] : 0.0f;
+  s.v_norm = in && a.w && a.v_norm ? a.v_norm[off] : 0.0f;
+  s.position = in && a.normalize ? a.token_pos[b * a.tp_stride_b + hh * a.tp_stride_h + slot] : 0;
+  return s;
+}
+// The slot's score after the update (stored); `z`: the row's sum of v_norm * w. Every product and sum rounded on its own.
+__device__ __forceinline__ float updated_score(const kvx_h2o_args& a, const Slot& s, float z, int b, int hh, int slot) {
+  if (!a.w) return s.score;
+  float inst = s.w;
+  if (a.v_norm) inst = __fmul_rn(__fmul_rn(s.v_norm, s.w) / z, (float)a.q_len);
+  const float v = __fadd_rn(s.score, inst);
+  if (slot < a.kv_len) a.scores[b * a.sc_stride_b + hh * a.sc_stride_h + slot] = v;
   return v;
 }
 
@@ -445,10 +454,10 @@ __global__ __launch_bounds__(LIST) void list_stats_kernel(const kvx_h2o_args a, 
   const int slot = part_slot(c, sl.C, threadIdx.x);
   const bool in = slot < a.limit;
   const float qe = in ? a.q_errors[b * a.sc_stride_b + hh * a.sc_stride_h + slot] : 0.0f;
+  const Slot s = load_slot(a, row, b, hh, slot);
   const float z = !a.w || !a.v_norm ? 1.0f : sl.part_z ? parts_norm<LIST>(sl, red, row) : row_norm(a, sl.C, row, b, hh);
-  const float v = updated_score(a, z, row, b, hh, slot);
-  const int32_t* tpr = a.token_pos ? a.token_pos + b * a.tp_stride_b + hh * a.tp_stride_h : nullptr;
-  const float cv = in ? residency_value(v, a, tpr, slot) : 0.0f;
+  const float v = updated_score(a, s, z, b, hh, slot);
+  const float cv = in ? residency_of(v, a, s.position) : 0.0f;
   const f32x4_t ex = block_extremes<LIST>(f32x4_t{in ? cv : INFINITY, in ? cv : -INFINITY, in ? qe : INFINITY, in ? qe : -INFINITY});
   if (threadIdx.x == 0) *(f32x4_t*)(sl.stats + ((int64_t)row * sl.C + c) * 4) = ex;
 }
@@ -505,11 +514,11 @@ __global__ __launch_bounds__(L) void list_sort_kernel(const kvx_h2o_args a, cons
   const int tid = threadIdx.x, c = blockIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
   const int slot = list_slot(c, sl.lists, tid);
   const bool in = slot < a.limit;
-  const int32_t* tpr = a.token_pos ? a.token_pos + b * a.tp_stride_b + hh * a.tp_stride_h : nullptr;
   unsigned long long x = ~0ull;
   if (a.q_errors) {
     const int64_t off = b * a.sc_stride_b + hh * a.sc_stride_h;
     const float v = in ? a.scores[off + slot] : 0.0f, qe = in ? a.q_errors[off + slot] : 0.0f;
+    const int position = in && a.normalize ? a.token_pos[b * a.tp_stride_b + hh * a.tp_stride_h + slot] : 0;
     float v4[4] = {INFINITY, -INFINITY, INFINITY, -INFINITY};
     const float* st = sl.stats + (int64_t)b * a.Hkv * sl.C * 4;
     for (int i = tid; i < a.Hkv * sl.C; i += L) {
@@ -528,11 +537,12 @@ __global__ __launch_bounds__(L) void list_sort_kernel(const kvx_h2o_args a, cons
     m.c = (float)a.combination;
     m.c2 = (float)((a.combination - 1.0) / 2.0);
     m.c3 = (float)(1.0 - a.combination);
-    if (in) x = ((unsigned long long)ordered_bits(combined_value(residency_value(v, a, tpr, slot), qe, m)) << 32) | (unsigned)slot;
+    if (in) x = ((unsigned long long)ordered_bits(combined_value(residency_of(v, a, position), qe, m)) << 32) | (unsigned)slot;
   } else {
+    const Slot s = load_slot(a, row, b, hh, slot);
     const float z = a.w && a.v_norm ? parts_norm<L>(sl, red, row) : 1.0f;
-    const float v = updated_score(a, z, row, b, hh, slot);
-    if (in) x = ((unsigned long long)ordered_bits(residency_value(v, a, tpr, slot)) << 32) | (unsigned)slot;
+    const float v = updated_score(a, s, z, b, hh, slot);
+    if (in) x = ((unsigned long long)ordered_bits(residency_of(v, a, s.position)) << 32) | (unsigned)slot;
   }
   x = sort_list<L>(x, buf);
   if (sl.lists == 1) {  // the row is one list
