@@ -8,7 +8,7 @@
 //   k == 1 (single-token decode): a streaming pass over all rows with many workgroups; each folds
 //          its slice into one 64-bit key (ordered value bits << 32 | slot) and publishes it with
 //          an integer atomicMin, which is order independent and therefore deterministic.
-//   k  > 1 (chunked prefill): a row is spread over workgroups of 256 or 1024 slots. The first launch adds the weights
+//   k  > 1 (chunked prefill): a row is spread over workgroups of 256, 512 or 1024 slots. The first launch adds the weights
 //          and sorts every workgroup's 64-bit (value, slot) keys; the second gives every key that can be among
 //          the first k its rank in the row by binary searches in the other lists and writes it there.
 //          Without the workspace for the lists (one workgroup per row): the first pass adds the weights and
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(SEL_THREADS) void select_one_kernel(const kvx_h2o_a
 // ---- k > 1, a row over several workgroups -----------------------------------------------------
 //
 // A row has few keys for a device (8 rows of 16384 slots) and many for one workgroup: with one workgroup per row the
-// choice of 1024 slots took 40 us, bound by one compute unit's LDS and instruction issue. Lists of 256 or 1024 keys are
+// choice of 1024 slots took 40 us, bound by one compute unit's LDS and instruction issue. Lists of 256, 512 or 1024 keys are
 // sorted side by side instead, and ranks need no hand-over between workgroups but the launch boundary.
 // List c of a row takes the 16-slot blocks c, c + C, c + 2C, ... (C lists): old and new tokens lie in runs of slots, and
 // this way every list is a sample of the whole row, so that the bound below is tight whatever the order of the slots. Blocks of
@@ -852,13 +852,14 @@ static size_t best_bytes(const kvx_h2o_args& a) {
 // what the one-workgroup-per-row form cannot do without
 static size_t min_workspace(const kvx_h2o_args& a) { return best_bytes(a) + (a.q_errors ? (size_t)a.B * a.Hkv * 4 * sizeof(float) : 0); }
 
-// Sorted lists for k > 1: taken while their number and size stay reasonable (256 lists of 1024 keys a row, 1 GiB), else
-// (and where the caller's workspace does not hold them) one workgroup per row. Lists of 256 keys sort in 36 steps, 3 of them through LDS,
-// where 1024 keys take 55 and 10, but every candidate is looked up in four times as many lists, by four times as many workgroups that
-// each read the heads of all. They pay while the device holds the workgroups side by side, three to a unit, and the look-ups, k times the
-// lists of all rows, are few for it. Whole choices, lists of 256 / of 1024, us: 16 of 8192 slots (32 lists), 24 rows 10.0 / 11.6, 32 rows 12.4 / 11.8;
-// 256 of 4096 (16 lists), 32 rows 10.3 / 12.3, 64 rows 14.3 / 12.5; 1000 of 4096, 24 rows 13.9 / 15.2, 48 rows 16.9 / 16.0; 1000 of 16384 (64 lists), 8 rows 14.3 / 15.9,
-// with new tokens in a run of slots 22 / 14.5.
+// Sorted lists for k > 1: taken while their number and size stay reasonable (256 parts of 1024 slots a row, 1 GiB), else
+// (and where the caller's workspace does not hold them) one workgroup per row. Lists of 256 keys sort in 36 steps, 3 of them through LDS, of 512 in 45
+// and 6, of 1024 in 55 and 10 by four times the wavefronts of a list of 256; but every candidate is looked up in all lists, by as many workgroups that
+// each read the heads of all, and the shorter the lists, the more a run of new tokens fills one of them.
+// Whole choices in us, tokens mixed / new ones in a run, lists of 256, 512, 1024: 64 of 3534 slots, 16 rows 8.6 / 9.9, 9.5 / 9.5, 11.7; 512 of 8192, 8 rows 10.3 / 10.1,
+// 11.0 / 10.9, 13.4; 200 of 6000, 16 rows 9.8 / 13.4, 9.9 / 9.9, 12.2; 1024 of 16384, 8 rows 14.4 / 13.4, 13.6 / 13.1, 16.0 / 15.6; 881 of 12598, 64 rows 43.7, 34.6, 42.3;
+// 114 of 36535, 64 rows 82 / 105, 60 / 62, 75 / 79; 23 of 38378, 4 rows 12.9 / 16.5, 11.8 / 13.5, 12.3; 1024 of 65536, 8 rows 50 / 63, 26.8 / 36.5, 24.0 / 23.6.
+// So 256 while the device holds the workgroups side by side, three to a unit, and the look-ups are few for it, 512 up to 72 of them, and 1024 beyond.
 // Rows of up to 1024 slots are one list whatever k is: its sort ends the choice and hands nothing on (64 of 1000 slots, 32 rows: 9.9 us as
 // four lists, 7.2 as one; in the 128 KiB of the static entry point, too little for four lists of 32 rows, 14.1 and 7.2).
 struct ListPlan {
@@ -874,7 +875,7 @@ static ListPlan list_plan(const kvx_h2o_args& a) {
   p.C = (int)C;
   const int64_t n256 = (a.kv_len + 255) / 256, cus = num_cus();
   const bool few = C > 1 && a.kv_len <= 32768 && rows * n256 <= 3 * cus && a.k * n256 <= 32768 && rows * a.k * n256 <= 2048 * cus;
-  p.L = n256 == 1 || few ? 256 : LIST;
+  p.L = n256 == 1 || few ? 256 : C > 1 && C <= 36 ? 512 : LIST;
   p.lists = (a.kv_len + p.L - 1) / p.L;
   const size_t n = (size_t)(rows * C);
   p.off_z = p.lists > 1 ? (size_t)rows * p.lists * p.L * 8 : 0;
@@ -912,6 +913,7 @@ static int launch_lists(const kvx_h2o_args& a, const ListPlan& p, hipStream_t st
   if (a.w && a.v_norm && sl.part_z) hipLaunchKernelGGL(list_norm_kernel, grid, dim3(LIST), 0, st, a, sl);
   if (a.q_errors) hipLaunchKernelGGL(list_stats_kernel, grid, dim3(LIST), 0, st, a, sl);
   if (p.L == 256) launch_sorted<256>(a, sl, st);
+  else if (p.L == 512) launch_sorted<512>(a, sl, st);
   else launch_sorted<LIST>(a, sl, st);
   KVX_HIP(hipGetLastError());
   return KVX_OK;

@@ -288,7 +288,7 @@ def test_c_oracle_builds():
     (32, 1024, 1000, 0),
     (32, 1025, 8, 5 * 256),      # sorted lists of 256 keys
     (24, 7936, 16, 31 * 256),    # three workgroups to each of 256 units
-    (25, 7936, 16, 8 * 1024),    # more of them: lists of 1024
+    (25, 7936, 16, 8 * 1024),    # more of them: lists of 512, the same room
     (8, 7936, 1057, 31 * 256),
     (8, 7936, 1058, 8 * 1024),   # too many look-ups for a row
     (32, 3840, 1092, 15 * 256),

@@ -469,20 +469,32 @@ def test_selection_over_lists_matches_one_workgroup_per_row(kvx, gpu, B, Hkv, L,
     (1, 2, 4000, 15, 1024),    # 16 lists of 256, half of the look-ups that they are taken for
     (1, 2, 4000, 15, 1025),
     (1, 1, 8192, 9, 1024),     # 32 lists of 256 at the line of a row's look-ups
-    (1, 1, 8192, 9, 1025),     # beyond it: lists of 1024
+    (1, 1, 8192, 9, 1025),     # beyond it: lists of 512
     (16, 3, 4096, 0, 40),      # 48 rows of 16 lists of 256, three workgroups to each of 256 units
-    (7, 7, 4096, 0, 40),       # beyond: lists of 1024
+    (7, 7, 4096, 0, 40),       # beyond: lists of 512
     (8, 4, 4096, 3, 1024),     # the line of all rows' look-ups
     (8, 4, 4096, 3, 1025),
     (2, 2, 8192, 5, 200),      # the longest row whose norm the statistics add up
     (1, 2, 8193, 0, 100),      # a longer one
     (1, 1, 32768, 0, 64),      # 128 lists of 256
-    (1, 1, 32769, 0, 64),      # 33 lists of 1024
+    (1, 1, 32769, 0, 64),      # 65 lists of 512
 ])
 def test_selection_over_short_and_long_lists(kvx, gpu, B, Hkv, L, gp, k):
     for policy in ("h2o", "vlen", "q_errors"):
         test_selection_over_lists_matches_one_workgroup_per_row(kvx, gpu, B, Hkv, L, gp, k, policy)
     test_update_select_variants_direct(kvx, gpu, B, Hkv, L, L - gp, k, True, True, True)
+
+
+@pytest.mark.parametrize("B,Hkv,L,gp,k", [
+    (6, 8, 4097, 0, 40),       # 9 lists of 512, the last one of a single slot
+    (3, 1, 1537, 0, 1500),     # rows of few lists, the last one of a single slot, nearly all of it chosen
+    (1, 1, 36864, 7, 513),     # 72 lists of 512
+    (1, 1, 36865, 7, 513),     # 37 lists of 1024
+    (9, 8, 12598, 0, 881),     # 25 lists of 512, more rows than compute units for them
+])
+def test_selection_on_both_sides_of_lists_of_512(kvx, gpu, B, Hkv, L, gp, k):
+    for policy in ("h2o", "vlen", "q_errors"):
+        test_selection_over_lists_matches_one_workgroup_per_row(kvx, gpu, B, Hkv, L, gp, k, policy)
 
 
 @pytest.mark.parametrize("k", [16, 17, 288, 289, 800, 801])  # 1, 2, 9, 10, 25, 26 keys a list of 32: heads of 16, 32, 32, 64, 64, 128
