@@ -336,6 +336,8 @@ typedef struct kvx_cache_write_args {
    * log_pos = input_pos - cache_length of the first new token. NULL: nothing is recorded. */
   uint32_t* replay_log;
   int32_t log_blocksize;
+  int32_t clear_behind; /* not 0, the first chunk of a sequence: scores, v_norm and q_errors of the slots num .. cache_len - 1, which hold nothing
+                         * yet, are set to zero in the same launch. No ring move; B * Hkv * cache_len below 2^31. */
   int64_t log_pos;
   int64_t log_stride_block, log_stride_b, log_stride_h;
 } kvx_cache_write_args;

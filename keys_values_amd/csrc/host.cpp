@@ -593,6 +593,17 @@ PyObject* cache_write(PyObject* const* args, Py_ssize_t n) {
   Py_RETURN_NONE;
 }
 
+// cache_write_first(cache, index, key, value): the first chunk of a sequence; the other slots' scores, norms and errors become zero
+PyObject* cache_write_first(PyObject* const* args, Py_ssize_t n) {
+  require_args(n, 4, "cache_write_first");
+  const at::Tensor &key = tensor(args[2], "key"), &value = tensor(args[3], "value");
+  const Launch L(key);
+  WriteCall w = write_args(args[0], opt_tensor(args[1], "index"), key, value, 0, Py_None, Py_None);
+  w.a.clear_behind = 1;
+  check(unlocked([&] { return lib.kvx_cache_write(&w.a, L.stream); }));
+  Py_RETURN_NONE;
+}
+
 // Arguments of the score update and the choice of k slots; `full`: the cache has no free slot (else nothing is chosen
 // that anyone uses, and the smallest selection is run)
 kvx_h2o_args h2o_args(PyObject* cache, bool full, int64_t k, int64_t input_pos, Held& held) {
@@ -916,7 +927,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define METHOD(name) {#name, (PyCFunction)(void (*)(void))entry<name>, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"bind", (PyCFunction)(void (*)(void))entry<bind, false>, METH_FASTCALL, nullptr},
-    METHOD(prefill), METHOD(score_sum), METHOD(decode), METHOD(check_qkv), METHOD(cache_write), METHOD(cache_update), METHOD(cache_decode_step),
+    METHOD(prefill), METHOD(score_sum), METHOD(decode), METHOD(check_qkv), METHOD(cache_write), METHOD(cache_write_first), METHOD(cache_update), METHOD(cache_decode_step),
     METHOD(quantize_blocks), METHOD(dequantize_blocks), METHOD(dequantize_rows), METHOD(rmsnorm), METHOD(add_rmsnorm),
     METHOD(swiglu), METHOD(qk_norm_rope), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", "Native host path of the kernels (see csrc/host.cpp).", -1, methods};

@@ -298,6 +298,11 @@ static int check_cache_write(const kvx_cache_write_args* a) {
   KVX_REQUIRE(!a->replay_log || (a->log_blocksize > 0 && a->log_pos >= 0), KVX_ERR_INVALID,
               "kvx_cache_write: replay log needs log_blocksize > 0 and log_pos >= 0");
   KVX_REQUIRE(!a->q_errors || !kv_is_plain(a->kv_dtype), KVX_ERR_INVALID, "kvx_cache_write: q_errors needs a quantised cache");
+  if (a->clear_behind) {
+    KVX_REQUIRE(a->grace_num == 0, KVX_ERR_INVALID, "kvx_cache_write: a first chunk has no ring to move");
+    KVX_REQUIRE((int64_t)a->B * a->Hkv * a->cache_len < (1ll << 31), KVX_ERR_UNSUPPORTED, "kvx_cache_write: clear_behind over %lld slots, must be below 2^31",
+                (long long)a->B * a->Hkv * a->cache_len);
+  }
   return KVX_OK;
 }
 

@@ -647,12 +647,14 @@ class H2OKVCache:
             raise ValueError(f"prefill length {num} exceeds cache_length {self.cache_length}")
         self.batch_size = b
         index = self._run_of_slots(0, num)
-        self.scores.zero_()
-        for extra in (self.v_norm, self.q_errors):
-            if extra is not None:
-                extra.zero_()
         self.current_length = num
-        self._write(index, key, value, 0)
+        if b == self.max_batch_size and not self.blocks_over_heads and self.scores.numel() < 2**31:
+            _lib.host().cache_write_first(self, index, key, value)  # the slots behind the chunk become zero in the same launch
+        else:  # rows that the chunk does not write, or errors that are written elsewhere
+            for t in (self.scores, self.v_norm, self.q_errors):
+                if t is not None:
+                    t.zero_()
+            self._write(index, key, value, 0)
         if self.blocks_over_heads:
             self._block_errors(index, None, key, value)
             self._write_back(index, None, (0, num))
