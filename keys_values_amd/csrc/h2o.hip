@@ -860,8 +860,8 @@ static size_t min_workspace(const kvx_h2o_args& a) { return best_bytes(a) + (a.q
 // 11.0 / 10.9, 13.4; 200 of 6000, 16 rows 9.8 / 13.4, 9.9 / 9.9, 12.2; 1024 of 16384, 8 rows 14.4 / 13.4, 13.6 / 13.1, 16.0 / 15.6; 881 of 12598, 64 rows 43.7, 34.6, 42.3;
 // 114 of 36535, 64 rows 82 / 105, 60 / 62, 75 / 79; 23 of 38378, 4 rows 12.9 / 16.5, 11.8 / 13.5, 12.3; 1024 of 65536, 8 rows 50 / 63, 26.8 / 36.5, 24.0 / 23.6.
 // So 256 while the device holds the workgroups side by side, three to a unit, and the look-ups are few for it, 512 up to 72 of them, and 1024 beyond.
-// Rows of up to 1024 slots are one list whatever k is: its sort ends the choice and hands nothing on (64 of 1000 slots, 32 rows: 9.9 us as
-// four lists, 7.2 as one; in the 128 KiB of the static entry point, too little for four lists of 32 rows, 14.1 and 7.2).
+// Rows of up to 1024 slots are one list whatever k is, the shortest that holds them: its sort ends the choice and hands nothing on (64 of 1000 slots, 32 rows: 9.9 us as
+// four lists, 7.2 as one; in the 128 KiB of the static entry point, too little for four lists of 32 rows, 14.1 and 7.2); of 257 to 512 slots in a list of 512, not of 1024: 6.8 -> 5.0.
 struct ListPlan {
   int C;         // parts of LIST slots per row, 0: not this way
   int L, lists;  // keys of a sorted list, lists per row
@@ -875,7 +875,7 @@ static ListPlan list_plan(const kvx_h2o_args& a) {
   p.C = (int)C;
   const int64_t n256 = (a.kv_len + 255) / 256, cus = num_cus();
   const bool few = C > 1 && a.kv_len <= 32768 && rows * n256 <= 3 * cus && a.k * n256 <= 32768 && rows * a.k * n256 <= 2048 * cus;
-  p.L = n256 == 1 || few ? 256 : C > 1 && C <= 36 ? 512 : LIST;
+  p.L = n256 == 1 || few ? 256 : n256 == 2 || (C > 1 && C <= 36) ? 512 : LIST;
   p.lists = (a.kv_len + p.L - 1) / p.L;
   const size_t n = (size_t)(rows * C);
   p.off_z = p.lists > 1 ? (size_t)rows * p.lists * p.L * 8 : 0;

@@ -464,7 +464,7 @@ def test_selection_over_lists_matches_one_workgroup_per_row(kvx, gpu, B, Hkv, L,
 
 @pytest.mark.parametrize("B,Hkv,L,gp,k", [
     (2, 2, 256, 0, 256),       # one list of 256 keys, all of it chosen
-    (1, 3, 257, 1, 31),        # one list of 1024 keys, as for every row of up to 1024 slots
+    (1, 3, 257, 1, 31),        # one list of 512 keys: rows of up to 1024 slots are one list
     (1, 3, 1025, 1, 31),       # a fifth list of one slot, behind the limit
     (1, 2, 4000, 15, 1024),    # 16 lists of 256, half of the look-ups that they are taken for
     (1, 2, 4000, 15, 1025),
@@ -486,6 +486,8 @@ def test_selection_over_short_and_long_lists(kvx, gpu, B, Hkv, L, gp, k):
 
 
 @pytest.mark.parametrize("B,Hkv,L,gp,k", [
+    (2, 3, 512, 0, 500),       # one list of 512, full
+    (2, 3, 513, 0, 500),       # one list of 1024
     (6, 8, 4097, 0, 40),       # 9 lists of 512, the last one of a single slot
     (3, 1, 1537, 0, 1500),     # rows of few lists, the last one of a single slot, nearly all of it chosen
     (1, 1, 36864, 7, 513),     # 72 lists of 512
