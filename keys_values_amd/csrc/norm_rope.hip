@@ -23,16 +23,17 @@ constexpr int NT = 256;
 
 // These kernels move two or four bytes a value, and what bounded them was the vector ALU: an IEEE division takes a dozen instructions and a 64-bit index
 // division about a hundred. Values of a row are divided by the row's norm, so one division serves them: with r = RN(1 / b), q = RN(a r) and
-// the remainder a - q b, exact in a fused multiply-add, q + (a - q b) r is RN(a / b) (Markstein, "Computation of elementary functions on the IBM
-// RISC System/6000 processor", 1990) while nothing over- or underflows: by norms of 2^-40 to 2^40 of values of a row no larger than its
-// norm times sqrt(dim). Other norms (zero rows with eps = 0, infinities, NaN) are divided by as they are.
+// the remainder q b - a, exact in a fused multiply-add, q - (q b - a) r is RN(a / b) (Markstein, "Computation of elementary functions on the IBM
+// RISC System/6000 processor", 1990) while nothing over- or underflows: by norms of 2^-40 to 2^40, of values from 2^-85 (the quotient is
+// above 2^-126, the remainder's last bit above 2^-149) to the norm times sqrt(dim). Of smaller ones the last bit of the quotient may differ. The remainder is formed as q b - a and not as a - q b, so that a zero keeps its sign. Other norms (zero rows with eps = 0,
+// infinities, NaN) are divided by as they are.
 struct Divisor {
   float b, r;
   bool plain;
   __device__ __forceinline__ explicit Divisor(float x) : b(x), r(1.0f / x), plain(x > 0x1p-40f && x < 0x1p40f) {}
   __device__ __forceinline__ float under(float a) const {
     const float q = a * r;
-    return fmaf(fmaf(-q, b, a), r, q);
+    return fmaf(fmaf(q, b, -a), -r, q);
   }
 };
 // v of one lane, 8 values, divided by the norm, times the weights
@@ -176,14 +177,15 @@ __global__ __launch_bounds__(64 * MAX_WAVES) void add_rmsnorm_rows_kernel(const 
 // fc_1 / fc_2 weights. silu is x / (1 + exp(-x)) in fp32, rounded to bf16 before the product, as the
 // two separate tensor operations round.
 // exp(-x) is 2^h (1 + l ln 2) with h + l = -x log2(e), h rounded; the quotient as in Divisor, of a reciprocal that is an ulp off. Values below -80, whose
-// exponential is near the type's end, and NaN take the divisions. With expf, a division each and 64-bit indexes the kernel was bound by the vector ALU:
+// exponential is near the type's end, and NaN take the divisions. Of all 16-bit gates the error is 0.069 of the last of 24 bits in the mean and 1.77 at most, that of
+// expf and a division 0.068 and 1.75, and the 16 bits that are kept are the same. With expf, a division each and 64-bit indexes the kernel was bound by the vector ALU:
 // 4096 / 1024 rows of 9728 values 42.2 -> 39.3 and 13.3 -> 12.1 us.
 __device__ __forceinline__ float silu(float x) {
   constexpr float L2E = 1.4426950408889634f, L2E_LOW = (float)(1.4426950408889634 - (double)L2E), LN2 = 0.6931471805599453f;
   const float h = x * -L2E, l = fmaf(x, -L2E, -h) + x * -L2E_LOW;
   const float p = fast_exp2(h), d = 1.0f + fmaf(p, l * LN2, p);
   const float r = __builtin_amdgcn_rcpf(d), q = x * r;
-  return fmaf(fmaf(-q, d, x), r, q);
+  return fmaf(fmaf(q, d, -x), -r, q);
 }
 __global__ __launch_bounds__(NT) void swiglu_rows_kernel(const uint16_t* __restrict__ gate_up, int64_t g_rs, uint16_t* __restrict__ out,
                                                          int64_t o_rs, uint32_t rows, int dim) {

@@ -36,6 +36,8 @@ def test_norms_out_of_range(gpu, dim):
     x[4] *= 1e14  # above
     x[5, 0] = float("inf")
     x[6, 0] = float("nan")
+    x[7, ::3] *= 2.0 ** -100  # tiny values among ordinary ones: remainders and quotients below the normal range
+    x[8, 1::2] = x[8, 1::2].sign() * x[8, 1::2].abs().clamp_min(1.0) * 2.0 ** -125  # (whose halves, below, are exact)
     weight = torch.rand(dim, generator=gen) + 0.5
     for eps in (0.0, 1e-6):
         ref = LO.rmsnorm(x, weight, eps)
@@ -45,7 +47,29 @@ def test_norms_out_of_range(gpu, dim):
         half = (x.float() / 2).to(torch.bfloat16)
         added = ops.add_rmsnorm_(half.to(gpu), half.to(gpu), weight.to(gpu), eps).cpu()
         for got in (out, added):
-            torch.testing.assert_close(got.float(), ref.float(), rtol=2**-7, atol=0, equal_nan=True)
+            torch.testing.assert_close(got.float(), ref.float(), rtol=2**-7, atol=2**-133, equal_nan=True)  # (2^-133: a unit of 16-bit denormals)
+
+
+def test_zeros_keep_their_sign(gpu):
+    gen = torch.Generator().manual_seed(3)
+    x = torch.randn(5, 2048, generator=gen).to(torch.bfloat16)
+    x[:, ::7], x[:, 3::7] = -0.0, 0.0
+    weight = torch.rand(2048, generator=gen) + 0.5
+    ref = LO.rmsnorm(x, weight, 1e-6)
+    half = (x.float() / 2).to(torch.bfloat16).to(gpu)
+    for got in (ops.rmsnorm(x.to(gpu), weight.to(gpu), 1e-6), ops.add_rmsnorm_(half.clone(), half, weight.to(gpu), 1e-6)):
+        assert torch.equal(got.cpu().signbit(), ref.signbit())
+    up = torch.randn(5, 2048, generator=gen).to(torch.bfloat16)
+    assert torch.equal(ops.swiglu(torch.cat((x, up), 1).to(gpu)).cpu().signbit(), (F.silu(x) * up).signbit())
+    # rotated by the angles of position 0, whose sines are zero: a head's value and minus its partner times zero
+    qkv = x.view(1, 5, 2048)[:, :1].clone()
+    cos, sin = LO.rope_tables(4, 128, 1e6)
+    w = torch.ones(128)
+    q, k, _ = LO.qk_norm_rope(qkv, 8, 4, 128, w, w, 1e-6, cos, sin, 0)
+    g = qkv.to(gpu)
+    ops.qk_norm_rope_(g, 8, 4, 128, w.to(gpu), w.to(gpu), 1e-6, cos.to(gpu), sin.to(gpu), 0)
+    got = g.cpu().view(1, 1, 16, 128).transpose(1, 2)
+    assert torch.equal(got[:, :12].signbit(), torch.cat((q, k), 1).signbit())
 
 
 @pytest.mark.parametrize("Hq,Hkv,D", [(1, 1, 64), (8, 2, 64), (28, 4, 64), (29, 4, 64), (12, 4, 128), (13, 4, 128), (32, 8, 128), (64, 8, 128), (32, 8, 256)])
