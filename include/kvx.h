@@ -336,12 +336,15 @@ typedef struct kvx_cache_write_args {
    * log_pos = input_pos - cache_length of the first new token. NULL: nothing is recorded. */
   uint32_t* replay_log;
   int32_t log_blocksize;
-  int32_t clear_behind; /* not 0, the first chunk of a sequence: scores, v_norm and q_errors of the slots num .. cache_len - 1, which hold nothing
-                         * yet, are set to zero in the same launch. No ring move; B * Hkv * cache_len below 2^31. */
   int64_t log_pos;
   int64_t log_stride_block, log_stride_b, log_stride_h;
 } kvx_cache_write_args;
 int kvx_cache_write(const kvx_cache_write_args* args, void* stream);
+
+/* kvx_cache_write of the first chunk of a sequence: scores, v_norm and q_errors (where given) of the slots num .. cache_len - 1, which hold
+ * nothing yet, are set to zero in the same launch. input_pos must be 0, without a ring move and a replay log; B * Hkv * cache_len below 2^31, and
+ * fewer than 2^24 workgroups of 256 threads: D / 8 of them a new row, and one for four of the other slots. */
+int kvx_cache_write_first(const kvx_cache_write_args* args, void* stream);
 
 /* H2O score update and eviction choice, AttnWeightsKVCache._update with H2OKVCache._compute_scores
  * (keys_values/kvcache/attn_weights.py:721-783, keys_values/kvcache/h2o.py:146-199):

@@ -60,7 +60,7 @@ class CacheWriteArgs(ctypes.Structure):
         ("scores", c_void_p), ("sc_stride_b", c_int64), ("sc_stride_h", c_int64),
         ("grace_num", c_int32), ("grace_period", c_int32), ("grace_slots", c_void_p),
         ("v_norm", c_void_p), ("q_errors", c_void_p),
-        ("replay_log", c_void_p), ("log_blocksize", c_int32), ("clear_behind", c_int32), ("log_pos", c_int64),
+        ("replay_log", c_void_p), ("log_blocksize", c_int32), ("log_pos", c_int64),
         ("log_stride_block", c_int64), ("log_stride_b", c_int64), ("log_stride_h", c_int64),
     ]
 
@@ -119,6 +119,7 @@ SYMBOLS = {
     "kvx_quantize_blocks": (ctypes.c_int, [POINTER(BlockQuantArgs), c_void_p]),
     "kvx_dequantize_blocks": (ctypes.c_int, [POINTER(BlockQuantArgs), c_void_p]),
     "kvx_cache_write": (ctypes.c_int, [POINTER(CacheWriteArgs), c_void_p]),
+    "kvx_cache_write_first": (ctypes.c_int, [POINTER(CacheWriteArgs), c_void_p]),
     "kvx_h2o_update_select": (ctypes.c_int, [POINTER(H2OArgs), c_void_p]),
     "kvx_h2o_decode_step": (ctypes.c_int, [POINTER(CacheWriteArgs), POINTER(SdpaArgs), POINTER(H2OArgs), c_void_p]),
     "kvx_h2o_decode_step_workspace_bytes": (c_size_t, [POINTER(SdpaArgs), POINTER(H2OArgs)]),

@@ -37,7 +37,7 @@ namespace {
   X(kvx_last_error) X(kvx_sdpa_prefill) X(kvx_sdpa_prefill_workspace_bytes) X(kvx_score_sum) X(kvx_sdpa_prefill_weights)     \
   X(kvx_sdpa_prefill_copying) X(kvx_sdpa_prefill_copying_workspace_bytes)                                                    \
   X(kvx_sdpa_decode) X(kvx_sdpa_decode_workspace_bytes) X(kvx_h2o_decode_step) X(kvx_h2o_decode_step_workspace_bytes)        \
-  X(kvx_quantize_blocks) X(kvx_dequantize_blocks) X(kvx_dequantize_rows_typed) X(kvx_cache_write) \
+  X(kvx_quantize_blocks) X(kvx_dequantize_blocks) X(kvx_dequantize_rows_typed) X(kvx_cache_write) X(kvx_cache_write_first) \
   X(kvx_h2o_update_select) X(kvx_h2o_workspace_bytes) X(kvx_rmsnorm_rows) X(kvx_add_rmsnorm_rows) X(kvx_swiglu_rows)         \
   X(kvx_qk_norm_rope)
 
@@ -598,9 +598,8 @@ PyObject* cache_write_first(PyObject* const* args, Py_ssize_t n) {
   require_args(n, 4, "cache_write_first");
   const at::Tensor &key = tensor(args[2], "key"), &value = tensor(args[3], "value");
   const Launch L(key);
-  WriteCall w = write_args(args[0], opt_tensor(args[1], "index"), key, value, 0, Py_None, Py_None);
-  w.a.clear_behind = 1;
-  check(unlocked([&] { return lib.kvx_cache_write(&w.a, L.stream); }));
+  const WriteCall w = write_args(args[0], opt_tensor(args[1], "index"), key, value, 0, Py_None, Py_None);
+  check(unlocked([&] { return lib.kvx_cache_write_first(&w.a, L.stream); }));
   Py_RETURN_NONE;
 }
 

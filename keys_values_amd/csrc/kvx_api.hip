@@ -298,17 +298,22 @@ static int check_cache_write(const kvx_cache_write_args* a) {
   KVX_REQUIRE(!a->replay_log || (a->log_blocksize > 0 && a->log_pos >= 0), KVX_ERR_INVALID,
               "kvx_cache_write: replay log needs log_blocksize > 0 and log_pos >= 0");
   KVX_REQUIRE(!a->q_errors || !kv_is_plain(a->kv_dtype), KVX_ERR_INVALID, "kvx_cache_write: q_errors needs a quantised cache");
-  if (a->clear_behind) {
-    KVX_REQUIRE(a->grace_num == 0, KVX_ERR_INVALID, "kvx_cache_write: a first chunk has no ring to move");
-    KVX_REQUIRE((int64_t)a->B * a->Hkv * a->cache_len < (1ll << 31), KVX_ERR_UNSUPPORTED, "kvx_cache_write: clear_behind over %lld slots, must be below 2^31",
-                (long long)a->B * a->Hkv * a->cache_len);
-  }
   return KVX_OK;
 }
 
 int kvx_cache_write(const kvx_cache_write_args* a, void* stream) {
   const int rc = check_cache_write(a);
   return rc != KVX_OK ? rc : launch_cache_write(*a, nullptr, (hipStream_t)stream);
+}
+
+int kvx_cache_write_first(const kvx_cache_write_args* a, void* stream) {
+  const int rc = check_cache_write(a);
+  if (rc != KVX_OK) return rc;
+  KVX_REQUIRE(a->input_pos == 0 && a->grace_num == 0 && !a->replay_log, KVX_ERR_INVALID, "kvx_cache_write_first: a first chunk begins at position 0, without a ring and a log");
+  const int64_t slots = (int64_t)a->B * a->Hkv * a->cache_len, workgroups = cache_write_workgroups(*a, true);  // 32-bit indexes of slots, and of threads
+  KVX_REQUIRE(slots < (1ll << 31) && workgroups < (1ll << 24), KVX_ERR_UNSUPPORTED,
+              "kvx_cache_write_first: %lld slots in %lld workgroups, must be below 2^31 and 2^24", (long long)slots, (long long)workgroups);
+  return launch_cache_write(*a, nullptr, (hipStream_t)stream, true);
 }
 
 size_t kvx_h2o_workspace_bytes(const kvx_h2o_args* a) { return a ? h2o_workspace(*a) : 0; }

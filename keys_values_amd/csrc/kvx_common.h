@@ -81,7 +81,9 @@ struct DecodeCounters {
   int64_t pairs;
 };
 // `clear`: counters the launch also sets to zero (a step of its own would cost as much as the write), or NULL
-int launch_cache_write(const kvx_cache_write_args& a, const DecodeCounters* clear, hipStream_t st);
+// `first`: the first chunk of a sequence, which sets the state of the slots behind it to zero
+int launch_cache_write(const kvx_cache_write_args& a, const DecodeCounters* clear, hipStream_t st, bool first = false);
+int64_t cache_write_workgroups(const kvx_cache_write_args& a, bool first);
 int launch_decode_step(const kvx_cache_write_args& w, const kvx_sdpa_args& a, const kvx_h2o_args& h, hipStream_t st);
 size_t decode_step_workspace(const kvx_sdpa_args& a, const kvx_h2o_args& h);
 // the k == 1 choice of the Q-Hitter combination from `per_row` statistics records a row (4 floats each: extremes of the

@@ -814,14 +814,20 @@ int launch_cache_write_d(const kvx_cache_write_args& a, const DecodeCounters& cl
   return KVX_OK;
 }
 
-int launch_cache_write(const kvx_cache_write_args& a, const DecodeCounters* clear, hipStream_t st) {
+// Workgroups for the rows, and behind them for the `rest` slots of each (batch, KV head) row that a first chunk leaves empty
+static uint32_t rest_of(const kvx_cache_write_args& a, bool first) { return first ? (uint32_t)(a.cache_len - a.num) : 0; }
+int64_t cache_write_workgroups(const kvx_cache_write_args& a, bool first) {
+  const int64_t pairs = (int64_t)a.B * a.Hkv;
+  return (pairs * a.num * (a.D / 8) + NTHREADS - 1) / NTHREADS + (pairs * rest_of(a, first) + CLEARED * NTHREADS - 1) / (CLEARED * NTHREADS);
+}
+
+int launch_cache_write(const kvx_cache_write_args& a, const DecodeCounters* clear, hipStream_t st, bool first) {
   const DecodeCounters none{}, &c = clear ? *clear : none;
-  const int64_t total = (int64_t)a.B * a.Hkv * a.num * (a.D / 8);
-  if (total == 0) return KVX_OK;
+  if ((int64_t)a.B * a.Hkv * a.num * (a.D / 8) == 0) return KVX_OK;
   // A launch each for scores, norms and errors was 2 to 5 us, the most of a short first chunk (us, calls in a row: 90 tokens of 24 heads, 512 slots 19.1 -> 15.0; 384,
   // 2803 slots, norms and errors 29.0 -> 18.3; 8192 of 16384 slots 515.5 -> 511.9).
-  const uint32_t rest = a.clear_behind ? (uint32_t)(a.cache_len - a.num) : 0;
-  const unsigned grid = (unsigned)((total + NTHREADS - 1) / NTHREADS + ((int64_t)a.B * a.Hkv * rest + CLEARED * NTHREADS - 1) / (CLEARED * NTHREADS));
+  const uint32_t rest = rest_of(a, first);
+  const unsigned grid = (unsigned)cache_write_workgroups(a, first);
   const uint32_t jobs = (uint32_t)((int64_t)a.B * a.Hkv * a.num);  // a grid's threads are counted in 32 bits
   if (a.D == 256) return launch_cache_write_d<256>(a, c, grid, jobs, rest, st);
   if (a.D == 128) return launch_cache_write_d<128>(a, c, grid, jobs, rest, st);

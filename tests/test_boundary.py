@@ -282,6 +282,27 @@ def test_c_oracle_builds():
     assert os.path.exists(c_oracle.build())
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the pointers are made up: where nothing can be launched")
+def test_first_chunk_write_refuses(kvx):
+    def call(**fields):
+        a = _lib.CacheWriteArgs()
+        a.B, a.Hkv, a.num, a.D, a.cache_len = 1, 8, 4, 64, 4096
+        a.index = a.key = a.value = a.k_cache = a.v_cache = a.token_pos = 4096
+        a.key_stride_t = a.value_stride_t = a.kc_stride_t = a.vc_stride_t = 64
+        for name, value in fields.items():
+            setattr(a, name, value)
+        return kvx.kvx_cache_write_first(ctypes.byref(a), None)
+
+    assert call() == _lib.KVX_ERR_HIP  # a call like any other: no device
+    assert call(input_pos=4) == _lib.KVX_ERR_INVALID  # not the first chunk
+    assert call(replay_log=4096, log_blocksize=64) == _lib.KVX_ERR_INVALID
+    assert call(grace_num=1, grace_period=1, grace_slots=4096, input_pos=1) == _lib.KVX_ERR_INVALID
+    assert call(Hkv=65536, cache_len=32767) == _lib.KVX_ERR_HIP
+    assert call(Hkv=65536, cache_len=32768) == _lib.KVX_ERR_UNSUPPORTED  # 2^31 slots
+    assert call(Hkv=65536, cache_len=65536) == _lib.KVX_ERR_UNSUPPORTED
+    assert call(Hkv=65536, cache_len=32767, num=2047, D=256) == _lib.KVX_ERR_UNSUPPORTED  # 2^24 workgroups
+
+
 @pytest.mark.parametrize("rows,kv_len,k,keys", [
     (32, 256, 200, 0),           # one list: its sort is the choice, no keys are handed on
     (32, 257, 8, 0),

@@ -38,12 +38,33 @@ def test_slots_behind_the_first_chunk(kvx, gpu, name, B, Hkv, T, D, lengths, spa
             assert torch.isfinite(cache.q_errors).all() and (cache.q_errors[:B, :, :num] > 0).all()
 
 
-def test_refusals(kvx):
-    a = _lib.CacheWriteArgs()
-    a.B, a.Hkv, a.num, a.D, a.cache_len = 1, 65536, 1, 64, 65536
-    a.index = a.key = a.value = a.k_cache = a.v_cache = 4096
-    a.key_stride_t = a.value_stride_t = a.kc_stride_t = a.vc_stride_t = 64
-    a.clear_behind = 1
-    assert kvx.kvx_cache_write(ctypes.byref(a), None) != 0  # 2^32 slots
-    a.Hkv, a.token_pos, a.grace_num, a.grace_period, a.grace_slots, a.input_pos = 1, 4096, 1, 1, 4096, 1
-    assert kvx.kvx_cache_write(ctypes.byref(a), None) != 0
+def test_padding_means_nothing(kvx, gpu):
+    # a caller that sets every field and leaves the bytes between them as they are
+    B, Hkv, T, D, num = 1, 2, 64, 64, 3
+    gen = torch.Generator().manual_seed(1)
+    key, value = (randn(gen, B, Hkv, num, D).to(gpu) for _ in range(2))
+    k, v = (torch.zeros(B, Hkv, T, D, dtype=key.dtype, device=gpu) for _ in range(2))
+    scores = torch.full((B, Hkv, T), 5.0, device=gpu)
+    token_pos = torch.arange(T, dtype=torch.int32, device=gpu).expand(B, Hkv, T).contiguous()
+    index = torch.tensor([7, 9, 11], dtype=torch.int32, device=gpu)
+    ring = torch.tensor([60], dtype=torch.int32, device=gpu)
+    for grace in (0, 1):
+        a = _lib.CacheWriteArgs()
+        ctypes.memset(ctypes.byref(a), 0xFF, ctypes.sizeof(a))
+        for name, _ in a._fields_:
+            setattr(a, name, 0)
+        a.B, a.Hkv, a.num, a.D, a.cache_len, a.input_pos, a.kv_dtype = B, Hkv, num, D, T, T, _lib.KVX_KV_BF16
+        a.index, a.key, a.value, a.k_cache, a.v_cache = (t.data_ptr() for t in (index, key, value, k, v))
+        a.key_stride_b, a.key_stride_h, a.key_stride_t = key.stride()[:3]
+        a.value_stride_b, a.value_stride_h, a.value_stride_t = value.stride()[:3]
+        a.kc_stride_b, a.kc_stride_h, a.kc_stride_t = k.stride()[:3]
+        a.vc_stride_b, a.vc_stride_h, a.vc_stride_t = v.stride()[:3]
+        a.token_pos, a.tp_stride_b, a.tp_stride_h = token_pos.data_ptr(), *token_pos.stride()[:2]
+        a.scores, a.sc_stride_b, a.sc_stride_h = scores.data_ptr(), *scores.stride()[:2]
+        a.grace_num, a.grace_period, a.grace_slots = grace, grace, ring.data_ptr()
+        _lib.check(kvx.kvx_cache_write(ctypes.byref(a), _lib.stream_ptr(gpu)))
+    want = torch.full((B, Hkv, T), 5.0)
+    want[:, :, [7, 9, 11, 60]] = 0.0  # the ring's slot holds a new token, its former one moved to slot 7 with a score of 5 or 0
+    got = scores.cpu()
+    got[:, :, 7] = 0.0
+    assert torch.equal(got, want)
