@@ -139,6 +139,7 @@ static int prefill_checked(const kvx_sdpa_args* a, const char* who, bool weights
   KVX_REQUIRE(a->q_len <= a->kv_len, KVX_ERR_INVALID, "%s: q_len=%d exceeds kv_len=%d", who, a->q_len, a->kv_len);
   KVX_REQUIRE(!weights || (a->lse && a->w), KVX_ERR_INVALID, "%s: lse and w must be given", who);
   KVX_REQUIRE(aligned16(a->workspace), KVX_ERR_WORKSPACE, "%s: workspace must be 16-byte aligned", who);
+  if (weights && (rc = check_score_sum(*a)) != KVX_OK) return rc;
   if (weights && !(may_copy && wants_copy(*a))) {
     bool done;
     rc = launch_rows_weights(*a, st, done);

@@ -58,6 +58,7 @@ bool wants_copy(const kvx_sdpa_args& a);  // whether a call over a quantised sto
 size_t rows_weights_workspace(const kvx_sdpa_args& a);
 int launch_rows_weights(const kvx_sdpa_args& a, hipStream_t st, bool& done);
 int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* rest = nullptr);
+int check_score_sum(const kvx_sdpa_args& a);  // what the score-sums refuse, whichever launch forms them
 size_t score_sum_workspace(const kvx_sdpa_args& a);
 int launch_sdpa_decode(const kvx_sdpa_args& a, const kvx_h2o_args* fused_h2o, hipStream_t st);
 size_t sdpa_decode_workspace(const kvx_sdpa_args& a, bool fused_h2o);

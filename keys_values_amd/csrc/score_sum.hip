@@ -896,17 +896,21 @@ size_t score_sum_workspace(const kvx_sdpa_args& a) {
   return pl.splits > 1 ? (size_t)pl.splits * a.B * a.Hkv * a.kv_len * sizeof(float) : 0;
 }
 
+// The query rows are fetched at a uniform base plus a 32-bit byte offset per lane.
+int check_score_sum(const kvx_sdpa_args& a) {
+  const int64_t G = a.Hq / a.Hkv;
+  KVX_REQUIRE(a.q_stride_h >= 0 && a.q_stride_t >= 0 && ((G - 1) * a.q_stride_h + (int64_t)(a.q_len - 1) * a.q_stride_t + a.D) * 2 < (1ll << 32),
+              KVX_ERR_UNSUPPORTED, "kvx_score_sum: the query rows of one (batch, KV head) pair must span less than 4 GiB (strides %lld / %lld)",
+              (long long)a.q_stride_h, (long long)a.q_stride_t);
+  return KVX_OK;
+}
+
 int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* rest) {
   // the query rows are split only if the caller's workspace holds the partial sums
   ScorePlan pl = score_plan(a);
   if (pl.splits > 1 && !(a.workspace && a.workspace_bytes >= score_sum_workspace(a) && ((uintptr_t)a.workspace & 15) == 0)) pl = {1, 0, pl.waves};
-  // the query rows are fetched at a uniform base plus a 32-bit byte offset per lane
-  {
-    const int64_t G = a.Hq / a.Hkv;
-    KVX_REQUIRE(a.q_stride_h >= 0 && a.q_stride_t >= 0 && ((G - 1) * a.q_stride_h + (int64_t)(a.q_len - 1) * a.q_stride_t + a.D) * 2 < (1ll << 32),
-                KVX_ERR_UNSUPPORTED, "kvx_score_sum: the query rows of one (batch, KV head) pair must span less than 4 GiB (strides %lld / %lld)",
-                (long long)a.q_stride_h, (long long)a.q_stride_t);
-  }
+  const int rc = check_score_sum(a);
+  if (rc != KVX_OK) return rc;
   ScoreParams p;
   p.part = pl.splits > 1 ? (float*)a.workspace : nullptr;
   p.tiles_per_z = pl.tiles_per_z;

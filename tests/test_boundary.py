@@ -335,6 +335,20 @@ def _prefill_block(B, heads, kv_heads, q_len, kv_len, D, splits):
     return a
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the pointers are made up: where nothing can be launched")
+@pytest.mark.parametrize("q_len,kv_len", [(4, 100), (300, 9000)])  # one launch, two
+def test_weights_refuse_query_rows_of_4_gib(kvx, q_len, kv_len):
+    for call in (kvx.kvx_sdpa_prefill_weights, kvx.kvx_sdpa_prefill_copying):
+        a = _prefill_block(1, 8, 2, q_len, kv_len, 64, 0)
+        a.lse = a.w = a.workspace = 4096
+        a.workspace_bytes = kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a))
+        assert call(ctypes.byref(a), None) == _lib.KVX_ERR_HIP  # no device
+        for name, stride in (("q_stride_h", 2**30), ("q_stride_t", 2**30), ("q_stride_h", -64)):
+            b = _lib.SdpaArgs.from_buffer_copy(a)
+            setattr(b, name, stride)
+            assert call(ctypes.byref(b), None) == _lib.KVX_ERR_UNSUPPORTED
+
+
 @pytest.mark.parametrize("B,heads,kv_heads,q_len,splits", [(1, 4, 2, 100, 2), (4, 64, 16, 1446, 6), (8, 64, 16, 4096, 3)])
 def test_workspace_of_splits_of_any_size(kvx, B, heads, kv_heads, q_len, splits):
     # the second and third beyond 2^31 and 2^32 bytes
