@@ -163,8 +163,25 @@ size_t kvx_sdpa_prefill_copying_workspace_bytes(const kvx_sdpa_args* args);
 
 /* Query rows (queries x heads of a KV head) that a workgroup of the attention kernel takes in kvx_sdpa_prefill, or with `copying` in
  * kvx_sdpa_prefill_copying with all the workspace it asks for: 16 or 32 in the kernel for few rows or few keys, 128 or 256 in
- * the tiled one. For tests and measurement, on the host alone; 0 for arguments that the calls refuse. No counterpart in the reference. */
+ * the tiled one. args->w is ignored (kvx_sdpa_prefill_plan). For tests and measurement, on the host alone; 0 for arguments that the calls refuse. No counterpart
+ * in the reference. */
 int kvx_sdpa_prefill_block_rows(const kvx_sdpa_args* args, int copying);
+
+/* How kvx_sdpa_prefill (args->w NULL) or kvx_sdpa_prefill_weights, with `copying` kvx_sdpa_prefill_copying, takes a call that has all the
+ * workspace it asks for. For tests and measurement, on the host alone. No counterpart in the reference. */
+enum kvx_score_sum_kind { KVX_SCORE_SUM_NONE = 0, KVX_SCORE_SUM_TILED = 1, KVX_SCORE_SUM_SHORT = 2, KVX_SCORE_SUM_STREAMED = 3 };
+typedef struct kvx_prefill_plan {
+  int32_t one_launch;    /* not 0: weights are formed in the attention launch, whose workgroups wait for each other */
+  int32_t block_rows;    /* query rows of a workgroup */
+  int32_t row_blocks;    /* of a KV head */
+  int32_t splits;        /* of the keys */
+  int32_t split_keys;    /* of a split, the last one may have fewer */
+  int32_t teams;         /* 2: the halves of a split are walked by a team of wavefronts each */
+  int32_t copied;        /* not 0: over a dequantised copy of the store */
+  int32_t score_sum;     /* enum kvx_score_sum_kind: the launch that forms the weights */
+  int32_t combined;      /* not 0: the splits' partials are combined in it */
+} kvx_prefill_plan;
+int kvx_sdpa_prefill_plan(const kvx_sdpa_args* args, int copying, kvx_prefill_plan* plan);
 
 /* Single-token decode (q_len == 1): O over the whole cache and, if args->w is set, the score-sums
  * W = (1/G) sum_g softmax_g. No mask: the new token is the newest

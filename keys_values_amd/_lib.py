@@ -8,6 +8,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libkvx.so")
 
+KVX_SCORE_SUM_NONE, KVX_SCORE_SUM_TILED, KVX_SCORE_SUM_SHORT, KVX_SCORE_SUM_STREAMED = 0, 1, 2, 3
 KVX_OK, KVX_ERR_INVALID, KVX_ERR_UNSUPPORTED, KVX_ERR_HIP, KVX_ERR_WORKSPACE = 0, 1, 2, 3, 4
 KVX_KV_BF16, KVX_KV_U8, KVX_KV_U4, KVX_KV_F16, KVX_KV_U8_F16, KVX_KV_U4_F16 = 0, 1, 2, 3, 4, 5
 
@@ -65,6 +66,12 @@ class CacheWriteArgs(ctypes.Structure):
     ]
 
 
+class PrefillPlan(ctypes.Structure):
+    """struct kvx_prefill_plan"""
+
+    _fields_ = [(name, c_int32) for name in ("one_launch", "block_rows", "row_blocks", "splits", "split_keys", "teams", "copied", "score_sum", "combined")]
+
+
 class H2OArgs(ctypes.Structure):
     """struct kvx_h2o_args"""
 
@@ -102,6 +109,7 @@ SYMBOLS = {
     "kvx_sdpa_prefill_workspace_bytes": (c_size_t, [POINTER(SdpaArgs)]),
     "kvx_sdpa_prefill_copying": (ctypes.c_int, [POINTER(SdpaArgs), c_void_p]),
     "kvx_sdpa_prefill_copying_workspace_bytes": (c_size_t, [POINTER(SdpaArgs)]),
+    "kvx_sdpa_prefill_plan": (ctypes.c_int, [POINTER(SdpaArgs), ctypes.c_int, POINTER(PrefillPlan)]),
     "kvx_sdpa_prefill_block_rows": (ctypes.c_int, [POINTER(SdpaArgs), ctypes.c_int]),
     "kvx_score_sum": (ctypes.c_int, [POINTER(SdpaArgs), c_void_p]),
     "kvx_sdpa_prefill_weights": (ctypes.c_int, [POINTER(SdpaArgs), c_void_p]),

@@ -133,6 +133,13 @@ int kvx_sdpa_prefill_block_rows(const kvx_sdpa_args* a, int copying) {
   return sdpa_prefill_block_rows(*a, copying != 0);
 }
 
+int kvx_sdpa_prefill_plan(const kvx_sdpa_args* a, int copying, kvx_prefill_plan* plan) {
+  KVX_REQUIRE(plan, KVX_ERR_INVALID, "kvx_sdpa_prefill_plan: plan is NULL");
+  const int rc = check_sdpa_common(a, "kvx_sdpa_prefill_plan", false);
+  if (rc == KVX_OK) *plan = sdpa_prefill_plan(*a, copying != 0);
+  return rc;
+}
+
 static int prefill_checked(const kvx_sdpa_args* a, const char* who, bool weights, bool may_copy, hipStream_t st) {
   int rc = check_sdpa_common(a, who, true);
   if (rc != KVX_OK) return rc;

@@ -53,9 +53,12 @@ int launch_sdpa_prefill(const kvx_sdpa_args& a, bool may_copy, hipStream_t st, M
 bool score_sum_combines(const kvx_sdpa_args& a);
 size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy);
 int sdpa_prefill_block_rows(const kvx_sdpa_args& a, bool may_copy);
+kvx_prefill_plan sdpa_prefill_plan(const kvx_sdpa_args& a, bool may_copy);
+int score_sum_kind(const kvx_sdpa_args& a);  // enum kvx_score_sum_kind
 bool wants_copy(const kvx_sdpa_args& a);  // whether a call over a quantised store that may copy goes over dequantised rows
 // attention with weights in one launch, where a workgroup holds the logits of its rows (sdpa_rows.hip); `done`: whether the call took it
 size_t rows_weights_workspace(const kvx_sdpa_args& a);
+bool rows_weights_plan(const kvx_sdpa_args& a, kvx_prefill_plan& plan);
 int launch_rows_weights(const kvx_sdpa_args& a, hipStream_t st, bool& done);
 int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* rest = nullptr);
 int check_score_sum(const kvx_sdpa_args& a);  // what the score-sums refuse, whichever launch forms them

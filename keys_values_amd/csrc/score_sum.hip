@@ -807,8 +807,6 @@ ScorePlan score_plan(const kvx_sdpa_args& a) {
   return best;
 }
 
-enum { TILED, SHORT, STREAMED };
-
 // Few rows over few keys take the short kernel: 64 keys a workgroup then still leave one compute unit a workgroup, and the
 // wavefronts that walk the query rows side by side would idle otherwise. Attention with weights, us, long -> short kernel:
 // 2 KV heads x 1024 keys of 64, 128 / 512 / 1024 / 2000 rows 16.0 -> 12.3, 23.7 -> 17.3, 26.5 -> 24.2, 30.9 -> 37.9; 8 x 1024 of 128,
@@ -838,7 +836,7 @@ bool is_streamed(const kvx_sdpa_args& a) {
 template <int D, int KV>
 int launch_t(const ScoreParams& p, int splits, int waves, const MergeParams* rest, int kind, hipStream_t st) {
   const int groups = p.B * p.Hkv;
-  if (kind == SHORT) {
+  if (kind == KVX_SCORE_SUM_SHORT) {
     const int64_t score_jobs = (int64_t)groups * ((p.kv_len + NW - 1) / NW);
     const MergeParams m = rest ? *rest : MergeParams{};
     auto launch = [&](auto sc_tag) {
@@ -851,7 +849,7 @@ int launch_t(const ScoreParams& p, int splits, int waves, const MergeParams* res
     KVX_HIP(hipGetLastError());
     return KVX_OK;
   }
-  if (kind == STREAMED) {
+  if (kind == KVX_SCORE_SUM_STREAMED) {
     const MergeParams m = rest ? *rest : MergeParams{};
     const int nkb = (p.kv_len + NW - 1) / NW, most = (nkb + 3) / 4;
     const int per_group = max(1, min(most, (D <= 128 ? 2 : 1) * num_cus() / groups));
@@ -888,6 +886,7 @@ int launch_t(const ScoreParams& p, int splits, int waves, const MergeParams* res
 
 }  // namespace
 
+int score_sum_kind(const kvx_sdpa_args& a) { return is_short(a) ? KVX_SCORE_SUM_SHORT : is_streamed(a) ? KVX_SCORE_SUM_STREAMED : KVX_SCORE_SUM_TILED; }
 bool score_sum_combines(const kvx_sdpa_args& a) { return is_short(a) || (is_streamed(a) && merge_fits(a)); }
 
 size_t score_sum_workspace(const kvx_sdpa_args& a) {
@@ -930,7 +929,7 @@ int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* 
   p.k_sb = a.k_stride_b; p.k_sh = a.k_stride_h; p.k_st = a.k_stride_t;
   p.qs_sb = a.qs_stride_b; p.qs_sh = a.qs_stride_h;
   p.tp_sb = a.tp_stride_b; p.tp_sh = a.tp_stride_h;
-  const int kind = is_short(a) ? SHORT : is_streamed(a) ? STREAMED : TILED;
+  const int kind = score_sum_kind(a);
 #define KVX_SCORE_SUM_CASE(KV) \
   case KV: \
     return a.D == 256 ? launch_t<256, KV>(p, pl.splits, pl.waves, rest, kind, st) : a.D == 128 ? launch_t<128, KV>(p, pl.splits, pl.waves, rest, kind, st) \

@@ -1012,6 +1012,23 @@ int sdpa_prefill_block_rows(const kvx_sdpa_args& a, bool may_copy) {
   return p.columns ? p.columns : 32 * nwaves(c.kv_dtype, c.D);
 }
 
+kvx_prefill_plan sdpa_prefill_plan(const kvx_sdpa_args& a, bool may_copy) {
+  kvx_prefill_plan plan{};
+  plan.copied = may_copy && wants_copy(a);
+  if (a.w && !plan.copied && rows_weights_plan(a, plan)) return plan;
+  const kvx_sdpa_args c = plan.copied ? on_copy(a, nullptr) : prefill_block(a);
+  plan.combined = a.w && score_sum_combines(a);
+  PrefillParams p;
+  fill_params(p, c, plan.combined);
+  plan.block_rows = p.columns ? p.columns : 32 * nwaves(c.kv_dtype, c.D);
+  plan.row_blocks = p.m_blocks;
+  plan.splits = p.num_splits;
+  plan.split_keys = p.tiles_per_split * BN;
+  plan.teams = p.pair ? 2 : 1;
+  plan.score_sum = a.w ? score_sum_kind(a) : KVX_SCORE_SUM_NONE;
+  return plan;
+}
+
 size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy) {
   PrefillParams p;
   const bool copy = may_copy && wants_copy(a);

@@ -802,6 +802,18 @@ size_t rows_weights_workspace(const kvx_sdpa_args& a) {
   return pl.columns ? weights_layout(a, pl).total : 0;
 }
 
+bool rows_weights_plan(const kvx_sdpa_args& a, kvx_prefill_plan& plan) {
+  const WeightsPlan pl = weights_plan(a);
+  if (!pl.columns) return false;
+  plan.one_launch = 1;
+  plan.block_rows = pl.columns;
+  plan.row_blocks = (a.q_len * (a.Hq / a.Hkv) + pl.columns - 1) / pl.columns;
+  plan.splits = pl.splits;
+  plan.split_keys = pl.split_keys;
+  plan.teams = 1;
+  return true;
+}
+
 int launch_rows_weights(const kvx_sdpa_args& a, hipStream_t st, bool& done) {
   done = false;
   const WeightsPlan pl = weights_plan(a);

@@ -1,5 +1,9 @@
 """Shared input builders for the tests (seeded, CPU generators as the benchmark inputs are)."""
+import ctypes
+
 import torch
+
+from keys_values_amd import _lib
 
 
 def randn(gen, *shape, dtype=torch.bfloat16):
@@ -26,6 +30,13 @@ def scattered_positions(gen, B, Hkv, T, input_pos, q_len):
             allp = torch.cat((old, torch.arange(input_pos, input_pos + q_len, dtype=torch.int32)))
             tp[b, h] = allp[torch.randperm(T, generator=gen)]
     return tp
+
+
+def prefill_plan(args, copying=0):
+    """How the library takes a call (``kvx_sdpa_prefill_plan``)."""
+    plan = _lib.PrefillPlan()
+    _lib.check(_lib.load().kvx_sdpa_prefill_plan(ctypes.byref(args), copying, ctypes.byref(plan)))
+    return plan
 
 
 def rel_err(a, b):

@@ -35,7 +35,8 @@ def test_library_exports_every_declared_symbol(kvx):
 
 def test_struct_layouts_match_c(tmp_path):
     src = ['#include <stdio.h>', '#include <stddef.h>', f'#include "{HEADER}"', "int main(void){"]
-    structs = {"kvx_sdpa_args": _lib.SdpaArgs, "kvx_cache_write_args": _lib.CacheWriteArgs, "kvx_h2o_args": _lib.H2OArgs}
+    structs = {"kvx_sdpa_args": _lib.SdpaArgs, "kvx_cache_write_args": _lib.CacheWriteArgs, "kvx_h2o_args": _lib.H2OArgs,
+               "kvx_prefill_plan": _lib.PrefillPlan}
     for cname, cls in structs.items():
         src.append(f'printf("{cname} %zu\\n", sizeof({cname}));')
         for fname, _ in cls._fields_:
@@ -193,6 +194,7 @@ def test_random_arguments_are_answered_not_trusted(kvx):
         for fn in (kvx.kvx_sdpa_prefill_workspace_bytes, kvx.kvx_sdpa_prefill_copying_workspace_bytes, kvx.kvx_sdpa_decode_workspace_bytes, kvx.kvx_sdpa_decode_h2o_workspace_bytes):
             assert fn(ctypes.byref(a)) >= 0
         assert kvx.kvx_sdpa_prefill_block_rows(ctypes.byref(a), it & 4) in (0, 16, 32, 128, 256)
+        assert kvx.kvx_sdpa_prefill_plan(ctypes.byref(a), it & 4, ctypes.byref(_lib.PrefillPlan())) in codes
         assert kvx.kvx_h2o_update_select(ctypes.byref(h), None) in codes
         assert kvx.kvx_h2o_workspace_bytes(ctypes.byref(h)) >= 0
         assert kvx.kvx_cache_write(ctypes.byref(fill(_lib.CacheWriteArgs())), None) in codes

@@ -860,7 +860,8 @@ def test_decode_without_weights_beside_other_work(gpu, decode_route):
 
 @pytest.mark.parametrize("store", ["bf16", "u8", "u4"])
 @pytest.mark.parametrize("B,Hq,Hkv,q_len,T,D,splits", [
-    (1, 24, 8, 11, 32769, 128, 0),    # 33 rows: two blocks over 8 x 32769 keys, their combination in the same launch
+    (1, 24, 8, 11, 32769, 128, 0),    # 33 rows: two blocks over 8 x 32769 keys, their combination in a launch of its own
+    (1, 24, 8, 10, 32769, 128, 0),    # 30 rows, their combination in the same launch
     (2, 28, 4, 36, 32800, 128, 3),    # 252 rows, more than the launch combines: a launch of its own
     (1, 16, 8, 128, 32768, 128, 2),   # 256 rows, the most
     (1, 8, 8, 257, 32768, 128, 2),    # one more: the tiled kernel

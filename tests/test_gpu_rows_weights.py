@@ -1,11 +1,11 @@
 """Attention with weights of few rows or keys in one launch (csrc/sdpa_rows.hip) against the CPU oracle, with its waits as they are and
-with waits that run out; recorded in a graph; on two streams at once."""
+with waits that run out; recorded in a graph; on two streams at once. Every case asserts that the library takes it that way (on 256 compute units)."""
 import ctypes
 
 import pytest
 import torch
 
-from helpers import make_qkv, rel_err, scattered_positions
+from helpers import make_qkv, prefill_plan, rel_err, scattered_positions
 from keys_values_amd import _lib
 from keys_values_amd.attention import ops
 from oracle import kvx_oracle as O
@@ -32,18 +32,21 @@ def stored(k, v, store, dtype):
     return seen, codes, [t.view(B, H, T) for r in rows for t in r[1:]]
 
 
-@pytest.mark.parametrize("dtype,store,B,Hq,Hkv,q_len,T,D,where", [
-    (torch.bfloat16, "plain", 1, 8, 2, 128, 1024, 64, "end"),     # blocks of rows and splits of keys
-    (torch.float16, "plain", 2, 6, 2, 11, 999, 128, "scattered"),  # 33 rows: a block of one; an odd number of keys
-    (torch.bfloat16, "plain", 1, 4, 1, 3, 64, 64, "end"),         # one block, one split: no workspace
-    (torch.bfloat16, "plain", 1, 16, 8, 130, 130, 128, "first"),  # as many queries as keys
-    (torch.float16, "u8", 1, 8, 2, 200, 257, 64, "end"),          # a last split of one key
-    (torch.bfloat16, "u4", 2, 8, 4, 40, 1500, 128, "scattered"),
-    (torch.bfloat16, "u8", 1, 7, 1, 5, 700, 256, "scattered"),
-    (torch.bfloat16, "plain", 1, 4, 2, 100, 700, 128, "first"),   # splits of which some rows see no key
-    (torch.bfloat16, "u8", 1, 2, 1, 8, 8000, 128, "end"),         # 63 splits
+# plan: rows of a workgroup, blocks of rows of a KV head, splits of the keys
+@pytest.mark.parametrize("dtype,store,B,Hq,Hkv,q_len,T,D,where,plan", [
+    (torch.bfloat16, "plain", 1, 8, 2, 128, 1024, 64, "end", (32, 16, 8)),      # blocks of rows and splits of keys
+    (torch.float16, "plain", 2, 6, 2, 11, 999, 128, "scattered", (16, 3, 16)),  # 33 rows: a block of one; an odd number of keys
+    (torch.bfloat16, "plain", 1, 4, 1, 3, 64, 64, "end", (16, 1, 1)),           # one block, one split: no workspace
+    (torch.bfloat16, "plain", 1, 16, 8, 130, 130, 128, "first", (16, 17, 1)),   # as many queries as keys
+    (torch.float16, "u8", 1, 8, 2, 200, 257, 64, "end", (16, 50, 1)),           # many blocks, a last tile of one key
+    (torch.float16, "u8", 1, 8, 2, 3, 257, 64, "end", (16, 1, 5)),              # a last split of one key
+    (torch.bfloat16, "u8", 1, 16, 2, 10, 321, 128, "scattered", (16, 5, 6)),    # and several blocks
+    (torch.bfloat16, "u4", 2, 8, 4, 40, 1500, 128, "scattered", (16, 5, 6)),
+    (torch.bfloat16, "u8", 1, 7, 1, 5, 700, 256, "scattered", (16, 3, 11)),
+    (torch.bfloat16, "plain", 1, 4, 2, 100, 700, 128, "first", (16, 13, 6)),    # splits of which some rows see no key
+    (torch.bfloat16, "u8", 1, 2, 1, 8, 8000, 128, "end", (16, 1, 63)),
 ])
-def test_weights_in_one_launch(kvx, gpu, waits, dtype, store, B, Hq, Hkv, q_len, T, D, where):
+def test_weights_in_one_launch(kvx, gpu, waits, dtype, store, B, Hq, Hkv, q_len, T, D, where, plan):
     q, k, v, gen = make_qkv(900 + T + q_len, B, Hq, Hkv, q_len, T, D, dtype=dtype)
     (ks, vs), (kd, vd), state = stored(k, v, store, dtype)
     pos, tp = {"end": T - q_len, "first": 0, "scattered": 2 * T}[where], None
@@ -58,6 +61,8 @@ def test_weights_in_one_launch(kvx, gpu, waits, dtype, store, B, Hq, Hkv, q_len,
     out, lse = torch.full_like(qd, float("nan")), torch.full((B, q_len, Hq), float("nan"), device=gpu)
     w = torch.full((B, Hkv, T), float("nan"), device=gpu)
     a.o, a.lse, a.w = out.data_ptr(), lse.data_ptr(), w.data_ptr()
+    taken = prefill_plan(a)
+    assert taken.one_launch and (taken.block_rows, taken.row_blocks, taken.splits) == plan
     n = kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a))
     ws = torch.full((n,), 255, dtype=torch.uint8, device=gpu)
     a.o_stride_b, a.o_stride_h, a.o_stride_t = out.stride(0), out.stride(1), out.stride(2)
