@@ -37,8 +37,8 @@ constexpr int per_cu(int D, int NC, bool u4) { return NC * D <= 128 || (NC * D =
 // Attention with weights in one launch (the template argument W): what a call needs beside PrefillParams.
 struct RowsWeights {
   float* w;
-  u32x4_t* sums;                    // [group][row block][pair of keys]: sums over the rows of a block, and the token; NULL with one block
-  u32x4_t* pairs;                   // [group][row block][row][split]: a split's maximum and sum, and the token
+  u32x4_t* sums;                    // [group][row block][pair of keys]: sums over the rows of a block, and the token (store_marked); NULL with one block
+  u32x4_t* pairs;                   // [group][row block][row][split]: a split's maximum and sum, and the token (store_marked)
   unsigned long long* missed_rows;  // flags [group][row block][split]: a split whose wait for the others ran out
   unsigned long long* missed_sums;  // flags [group][split][row block]: a block whose wait for the others' sums ran out
   float* logits;                    // [group][row block][split][split_keys columns]: of splits whose wait ran out
@@ -53,18 +53,19 @@ template <typename P>
 __device__ __forceinline__ auto coherent_load(P q) { return __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 template <typename P, typename T>
 __device__ __forceinline__ void coherent_store(P q, T v) { __hip_atomic_store(q, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-// Two words beside a call's token in 16 bytes: one store and one load of a lane, which the memory that the dies share performs whole.
+// Two words and a call's token in 16 bytes, one store and one load of a lane: a word and half of the token in each aligned 8 bytes, which the memory
+// that the dies share performs whole, so that a word is never taken for another call's.
 constexpr int kCoherent = 16;  // sc1
 typedef __amdgpu_buffer_rsrc_t rsrc_t;
 __device__ __forceinline__ rsrc_t words_at(const void* base) { return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0xffffffff, 0x00027000); }
 __device__ __forceinline__ void store_marked(rsrc_t at, uint32_t i, float x, float y, unsigned long long token) {
-  __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{__float_as_uint(x), __float_as_uint(y), (uint32_t)token, (uint32_t)(token >> 32)}, at, i * 16u, 0, kCoherent);
+  __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{__float_as_uint(x), (uint32_t)token, __float_as_uint(y), (uint32_t)(token >> 32)}, at, i * 16u, 0, kCoherent);
 }
 __device__ __forceinline__ u32x4_t load_marked(rsrc_t at, uint32_t i) {
   asm volatile("" ::: "memory");  // others write what is read: every time anew
   return __builtin_amdgcn_raw_buffer_load_b128(at, i * 16u, 0, kCoherent);
 }
-__device__ __forceinline__ bool is_marked(u32x4_t v, unsigned long long token) { return v[2] == (uint32_t)token && v[3] == (uint32_t)(token >> 32); }
+__device__ __forceinline__ bool is_marked(u32x4_t v, unsigned long long token) { return v[1] == (uint32_t)token && v[3] == (uint32_t)(token >> 32); }
 __device__ __forceinline__ unsigned long long join_words(uint32_t lo, uint32_t hi) { return ((unsigned long long)hi << 32) | lo; }
 
 template <int CTRL>
@@ -167,11 +168,11 @@ __device__ __forceinline__ void finish_weights(const PrefillParams& p, const Row
 #pragma unroll
       for (int u = 0; u < PER; ++u) {
         const int s = j + J * u;
-        u32x4_t v = {0xff800000u, 0u, (uint32_t)x.token, (uint32_t)(x.token >> 32)};
+        u32x4_t v = {0xff800000u, (uint32_t)x.token, 0u, (uint32_t)(x.token >> 32)};
         if (s < S) v = load_marked(pairs, (uint32_t)(r * S + s));
         all = all && is_marked(v, x.token);
         ms[u] = __uint_as_float(v[0]);
-        ls[u] = __uint_as_float(v[1]);
+        ls[u] = __uint_as_float(v[2]);
       }
       ok = __all(all);
       if (ok) break;
@@ -278,7 +279,7 @@ __device__ __forceinline__ void finish_weights(const PrefillParams& p, const Row
         __builtin_amdgcn_s_sleep(4);
       }
       ok = ok && is_marked(v, x.token);
-      all[i] = f32x2_t{__uint_as_float(v[0]), __uint_as_float(v[1])};
+      all[i] = f32x2_t{__uint_as_float(v[0]), __uint_as_float(v[2])};
     }
     if (!agree(__all(ok))) return false;
     for (int i = tid; i < 2 * count; i += NT) {

@@ -79,6 +79,39 @@ def test_weights_in_one_launch(kvx, gpu, waits, dtype, store, B, Hq, Hkv, q_len,
             t.fill_(float("nan"))
 
 
+def test_what_is_handed_on_carries_its_token_in_every_8_bytes(kvx, gpu):
+    # the heads of the workspace: maxima and sums of rows and splits, then weights of pairs of keys of every block of rows; of two words each half as
+    # wide as what is performed whole, each beside half of the call's token
+    B, Hq, Hkv, q_len, T, D = 1, 12, 2, 17, 999, 128  # 102 rows of a KV head: 7 blocks of 16
+    q, k, v, _ = make_qkv(4, B, Hq, Hkv, q_len, T, D)
+    qd, kd, vd = (t.to(gpu) for t in (q, k, v))
+    a = _lib.SdpaArgs()
+    ops._fill_common(a, qd, kd, vd, 0.09, T - q_len, None, None, 0)
+    out, lse, w = torch.empty_like(qd), torch.empty(B, q_len, Hq, device=gpu), torch.empty(B, Hkv, T, device=gpu)
+    a.o, a.lse, a.w = out.data_ptr(), lse.data_ptr(), w.data_ptr()
+    a.o_stride_b, a.o_stride_h, a.o_stride_t = out.stride(0), out.stride(1), out.stride(2)
+    plan = prefill_plan(a)
+    assert plan.one_launch and plan.block_rows == 16 and plan.row_blocks == 7 and plan.splits > 1
+    n = kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a))
+    ws = torch.full((n,), 255, dtype=torch.uint8, device=gpu)
+    a.workspace, a.workspace_bytes = ws.data_ptr(), n
+    tokens = []
+    for _ in range(2):
+        _lib.check(kvx.kvx_sdpa_prefill_weights(ctypes.byref(a), _lib.stream_ptr(gpu)))
+        words = ws[: n // 16 * 16].view(torch.int32).view(-1, 4).cpu()
+        blocks = B * Hkv * plan.row_blocks
+        pairs, sums = words[: blocks * 16 * plan.splits], words[blocks * 16 * plan.splits :][: blocks * ((T + 1) // 2)]
+        for part in (pairs, sums):
+            assert (part[:, 1::2] == pairs[0, 1::2]).all()
+        tokens.append(tuple(pairs[0, 1::2].tolist()))
+        m, s = pairs[:, ::2].contiguous().view(torch.float32).view(Hkv, -1, plan.splits, 2)[:, : q_len * Hq // Hkv].unbind(-1)
+        rows = torch.logsumexp(m.double() * 0.6931471805599453 + s.double().log(), -1) / 0.6931471805599453
+        torch.testing.assert_close(rows.view(Hkv, q_len, Hq // Hkv).transpose(0, 1).reshape(1, q_len, Hq).float(), lse.cpu(), rtol=1e-5, atol=1e-4)
+        of_keys = sums[:, ::2].contiguous().view(torch.float32).view(Hkv, plan.row_blocks, -1).sum(1)[:, :T] / (Hq // Hkv)
+        torch.testing.assert_close(of_keys, w[0].cpu(), rtol=1e-5, atol=1e-7)
+    assert tokens[0] != tokens[1]
+
+
 def test_repeats_itself_and_the_call_without_weights(gpu):
     # 16-bit outputs of other splits: 2^-9 / sqrt(3) in the mean square, probabilities and outputs on either side
     q, k, v, _ = (t.to(gpu) if isinstance(t, torch.Tensor) else t for t in make_qkv(5, 1, 16, 4, 60, 1200, 128))
