@@ -37,7 +37,7 @@ namespace {
   X(kvx_last_error) X(kvx_sdpa_prefill) X(kvx_sdpa_prefill_workspace_bytes) X(kvx_score_sum) X(kvx_sdpa_prefill_weights)     \
   X(kvx_sdpa_prefill_copying) X(kvx_sdpa_prefill_copying_workspace_bytes)                                                    \
   X(kvx_sdpa_decode) X(kvx_sdpa_decode_workspace_bytes) X(kvx_h2o_decode_step) X(kvx_h2o_decode_step_workspace_bytes)        \
-  X(kvx_quantize_blocks) X(kvx_dequantize_blocks) X(kvx_dequantize_rows_typed) X(kvx_cache_write) X(kvx_cache_write_first) \
+  X(kvx_quantize_blocks) X(kvx_dequantize_blocks) X(kvx_dequantize_rows_typed) X(kvx_cache_write) \
   X(kvx_h2o_update_select) X(kvx_h2o_workspace_bytes) X(kvx_rmsnorm_rows) X(kvx_add_rmsnorm_rows) X(kvx_swiglu_rows)         \
   X(kvx_qk_norm_rope)
 
@@ -45,6 +45,7 @@ struct Lib {
 #define X(name) decltype(&::name) name = nullptr;
   KVX_HOST_SYMBOLS(X)
 #undef X
+  decltype(&::kvx_cache_write_first) kvx_cache_write_first = nullptr;  // libraries from before it bind too
   bool bound = false;
 } lib;
 
@@ -596,6 +597,7 @@ PyObject* cache_write(PyObject* const* args, Py_ssize_t n) {
 // cache_write_first(cache, index, key, value): the first chunk of a sequence; the other slots' scores, norms and errors become zero
 PyObject* cache_write_first(PyObject* const* args, Py_ssize_t n) {
   require_args(n, 4, "cache_write_first");
+  if (!lib.kvx_cache_write_first) raise(PyExc_ImportError, "the bound library does not export kvx_cache_write_first");
   const at::Tensor &key = tensor(args[2], "key"), &value = tensor(args[3], "value");
   const Launch L(key);
   const WriteCall w = write_args(args[0], opt_tensor(args[1], "index"), key, value, 0, Py_None, Py_None);
@@ -900,6 +902,7 @@ PyObject* bind(PyObject* const* args, Py_ssize_t n) {
   if (!l.name) raise(PyExc_ImportError, "%s does not export %s", path, #name);
   KVX_HOST_SYMBOLS(X)
 #undef X
+  l.kvx_cache_write_first = (decltype(l.kvx_cache_write_first))dlsym(h, "kvx_cache_write_first");
   l.bound = true;
   lib = l;
   Py_XSETREF(kvx_error, Py_NewRef(args[1]));

@@ -284,6 +284,20 @@ def test_c_oracle_builds():
     assert os.path.exists(c_oracle.build())
 
 
+def test_libraries_without_the_first_chunk_write_bind(kvx, tmp_path):
+    src, so = tmp_path / "stub.c", tmp_path / "libstub.so"
+    names = [n for n in _declared_symbols() if n != "kvx_cache_write_first"]
+    src.write_text("".join(f"int {n}(void) {{ return 1; }}\n" for n in names))
+    subprocess.check_call(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)])
+    host = _lib.host()
+    try:
+        host.bind(str(so), _lib.KvxError, torch.OutOfMemoryError)
+        with pytest.raises(ImportError):
+            host.cache_write_first(None, None, None, None)
+    finally:
+        host.bind(_lib.LIB_PATH, _lib.KvxError, torch.OutOfMemoryError)
+
+
 @pytest.mark.skipif(torch.cuda.is_available(), reason="the pointers are made up: where nothing can be launched")
 def test_first_chunk_write_refuses(kvx):
     def call(**fields):
