@@ -65,6 +65,17 @@ class CacheWriteArgs(ctypes.Structure):
         ("log_stride_block", c_int64), ("log_stride_b", c_int64), ("log_stride_h", c_int64),
     ]
 
+    # The slots behind a first chunk are cleared by kvx_cache_write_first; a block that asks kvx_cache_write for it, as a field of this name once did,
+    # is refused (an unknown kv_dtype) and not written as if it had not asked.
+    @property
+    def clear_behind(self):
+        return int(self.kv_dtype == -1)
+
+    @clear_behind.setter
+    def clear_behind(self, value):
+        if value:
+            self.kv_dtype = -1
+
 
 class PrefillPlan(ctypes.Structure):
     """struct kvx_prefill_plan"""

@@ -352,6 +352,19 @@ def _prefill_block(B, heads, kv_heads, q_len, kv_len, D, splits):
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="the pointers are made up: where nothing can be launched")
+def test_slot_write_that_asks_for_a_first_chunk_is_refused(kvx):
+    a = _lib.CacheWriteArgs()
+    a.B, a.Hkv, a.num, a.D, a.cache_len = 1, 8, 4, 64, 4096
+    a.index = a.key = a.value = a.k_cache = a.v_cache = a.token_pos = 4096
+    a.key_stride_t = a.value_stride_t = a.kc_stride_t = a.vc_stride_t = 64
+    assert kvx.kvx_cache_write(ctypes.byref(a), None) == _lib.KVX_ERR_HIP  # no device
+    a.clear_behind = 0
+    assert kvx.kvx_cache_write(ctypes.byref(a), None) == _lib.KVX_ERR_HIP
+    a.clear_behind = 1
+    assert kvx.kvx_cache_write(ctypes.byref(a), None) == _lib.KVX_ERR_UNSUPPORTED
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the pointers are made up: where nothing can be launched")
 @pytest.mark.parametrize("q_len,kv_len", [(4, 100), (300, 9000)])  # one launch, two
 def test_weights_refuse_query_rows_of_4_gib(kvx, q_len, kv_len):
     for call in (kvx.kvx_sdpa_prefill_weights, kvx.kvx_sdpa_prefill_copying):

@@ -38,6 +38,17 @@ def test_slots_behind_the_first_chunk(kvx, gpu, name, B, Hkv, T, D, lengths, spa
             assert torch.isfinite(cache.q_errors).all() and (cache.q_errors[:B, :, :num] > 0).all()
 
 
+def test_refusals(kvx):
+    a = _lib.CacheWriteArgs()
+    a.B, a.Hkv, a.num, a.D, a.cache_len = 1, 65536, 1, 64, 65536
+    a.index = a.key = a.value = a.k_cache = a.v_cache = 4096
+    a.key_stride_t = a.value_stride_t = a.kc_stride_t = a.vc_stride_t = 64
+    a.clear_behind = 1
+    assert kvx.kvx_cache_write(ctypes.byref(a), None) != 0  # 2^32 slots
+    a.Hkv, a.token_pos, a.grace_num, a.grace_period, a.grace_slots, a.input_pos = 1, 4096, 1, 1, 4096, 1
+    assert kvx.kvx_cache_write(ctypes.byref(a), None) != 0
+
+
 def test_padding_means_nothing(kvx, gpu):
     # a caller that sets every field and leaves the bytes between them as they are
     B, Hkv, T, D, num = 1, 2, 64, 64, 3
