@@ -648,7 +648,9 @@ class H2OKVCache:
         self.batch_size = b
         index = self._run_of_slots(0, num)
         self.current_length = num
-        if b == self.max_batch_size and not self.blocks_over_heads and self.scores.numel() < 2**26:  # (more slots: more threads than a launch counts)
+        if b == self.max_batch_size and not self.blocks_over_heads and num == self.cache_length:  # every slot is written
+            self._write(index, key, value, 0)
+        elif b == self.max_batch_size and not self.blocks_over_heads and self.scores.numel() < 2**26:  # (more slots: more threads than a launch counts)
             _lib.host().cache_write_first(self, index, key, value)  # the slots behind the chunk become zero in the same launch
         else:  # rows that the chunk does not write, or errors that are written elsewhere
             for t in (self.scores, self.v_norm, self.q_errors):
