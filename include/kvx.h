@@ -180,6 +180,7 @@ typedef struct kvx_prefill_plan {
   int32_t copied;        /* not 0: over a dequantised copy of the store */
   int32_t score_sum;     /* enum kvx_score_sum_kind: the launch that forms the weights */
   int32_t combined;      /* not 0: the splits' partials are combined in it */
+  int32_t polls;         /* one launch: looks of a workgroup that waits for others, 2 us each at most by default, before it leaves its share to them */
 } kvx_prefill_plan;
 int kvx_sdpa_prefill_plan(const kvx_sdpa_args* args, int copying, kvx_prefill_plan* plan);
 
@@ -219,7 +220,7 @@ size_t kvx_sdpa_decode_h2o_workspace_bytes(const kvx_sdpa_args* args);
  * chip where they fit (calls with weights only). spin_limit: polls a split spends waiting for the other splits of its row
  * before it leaves its share to the row's last one and its logits, if weights are wanted, to the workspace (0 = never
  * wait; clamped to 2^20; every call whose splits finish the row themselves, with weights or without, and chunks with weights that are one
- * launch). poll_sleep: pause between two polls in units of
+ * launch, which by themselves wait about ten times the time of the call and not longer). poll_sleep: pause between two polls in units of
  * 512 cycles (clamped to 64). A negative value restores that switch to its default: the environment variables
  * KVX_DECODE_RESIDENT / KVX_DECODE_SPIN_LIMIT / KVX_DECODE_POLL_SLEEP as read once at the first decode call
  * (else 1, 32768, 4). A workspace size query and the call it is for must see the same setting of `resident`. */

@@ -80,7 +80,7 @@ class CacheWriteArgs(ctypes.Structure):
 class PrefillPlan(ctypes.Structure):
     """struct kvx_prefill_plan"""
 
-    _fields_ = [(name, c_int32) for name in ("one_launch", "block_rows", "row_blocks", "splits", "split_keys", "teams", "copied", "score_sum", "combined")]
+    _fields_ = [(name, c_int32) for name in ("one_launch", "block_rows", "row_blocks", "splits", "split_keys", "teams", "copied", "score_sum", "combined", "polls")]
 
 
 class H2OArgs(ctypes.Structure):

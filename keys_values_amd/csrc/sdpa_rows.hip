@@ -83,8 +83,8 @@ constexpr int kMaxSplits = 64;  // of a block of rows whose splits wait for each
 // (weights_plan). Nothing has to be cleared before the launch: what is waited for carries the call's token of 64 bits, a number that no other call has
 // (what the workspace held before equals it in one of 2^64 cases). A call that is being captured will be repeated with its token: a launch that clears goes before it.
 //
-// Both waits are bounded. One that runs out, as when other work holds the places of the workgroups that are waited for, says so in a flag, set by an exchange, and
-// looks once more; what is still missing is then done by those that come later: each looks at the flags of the others once its own results
+// Both waits are bounded, by a few times what the whole call takes (weights_plan). One that runs out, as when other work, a second such call among it, holds
+// the places of the workgroups that are waited for, says so in a flag, set by an exchange, and looks once more; what is still missing is then done by those that come later: each looks at the flags of the others once its own results
 // have reached the memory that the dies share, so of two at least one finds what the other left. Several may do the same work: they write the same bits.
 template <int D, int NC, bool F16>
 __device__ __forceinline__ void finish_weights(const PrefillParams& p, const RowsWeights& x, float* lg, float* red, const float* rml, const int group, const int mblk, const int split,
@@ -276,7 +276,8 @@ __device__ __forceinline__ void finish_weights(const PrefillParams& p, const Row
       for (;;) {
         v = load_marked(from, (uint32_t)(blk * kv_pairs + (i - blk * count)));
         if (is_marked(v, x.token) || ++spin >= limit) break;
-        __builtin_amdgcn_s_sleep(4);
+        const int pause = min(2 * x.poll_sleep, 1 + (spin >> 1));
+        for (int z = 0; z < pause; ++z) __builtin_amdgcn_s_sleep(4);
       }
       ok = ok && is_marked(v, x.token);
       all[i] = f32x2_t{__uint_as_float(v[0]), __uint_as_float(v[2])};
@@ -740,11 +741,15 @@ namespace {
 // 22.1 -> 19.6; 256 of 256 over 2 x 1500 8-bit keys 33.9 -> 19.7. Splits of more than 11 steps (of 256: 8) are bound by the walk, and
 // two launches share it out better: 322 rows over 2 x 12513 keys of 64 29.5 -> 35.7, 60 over 8 x 15028 30.4 -> 33.6, 210 of 256 over 16 x 1414
 // 8-bit keys 50.7 -> 52.9.
+//
+// A wait is given up behind as many polls as take about ten times the estimate and 60 us more, the fetch of instructions by a first call among them; a poll
+// is 1.5 to 2 us. What is given up is done by others from the workspace, for some us; held on to, the places of waiting workgroups are missing to those that they wait
+// for, as between two calls on two streams that fill the device each.
 struct WeightsPlan {
-  int columns, splits, split_keys;
+  int columns, splits, split_keys, polls;
 };
 WeightsPlan weights_plan(const kvx_sdpa_args& a) {
-  WeightsPlan best = {0, 0, 0};
+  WeightsPlan best = {0, 0, 0, 0};
   const bool plain = kv_is_plain(a.kv_dtype);
   const int64_t es = plain ? 2 : 1, cus = num_cus(), groups = (int64_t)a.B * a.Hkv, rows = (int64_t)a.q_len * (a.Hq / a.Hkv);
   if (a.num_splits > 1 || (plain && a.D == 256) || (a.D != 64 && a.D != 128 && a.D != 256)) return best;
@@ -763,7 +768,7 @@ WeightsPlan weights_plan(const kvx_sdpa_args& a) {
       const int64_t ns = (c == 1 ? 100 : 180) * walk / 100 + (n > 1 ? 2500 + 30 * n : 0);
       if (ns < best_ns) {
         best_ns = ns;
-        best = {columns, (int)n, (int)per * BN};
+        best = {columns, (int)n, (int)per * BN, (int)(40 + ns / 150)};
       }
     }
   }
@@ -811,6 +816,7 @@ bool rows_weights_plan(const kvx_sdpa_args& a, kvx_prefill_plan& plan) {
   plan.row_blocks = (a.q_len * (a.Hq / a.Hkv) + pl.columns - 1) / pl.columns;
   plan.splits = pl.splits;
   plan.split_keys = pl.split_keys;
+  plan.polls = pl.polls;
   plan.teams = 1;
   return true;
 }
@@ -840,6 +846,7 @@ int launch_rows_weights(const kvx_sdpa_args& a, hipStream_t st, bool& done) {
   x.token = call_token();
   x.split_keys = pl.split_keys;
   decode_wait(x.spin_limit, x.poll_sleep);
+  x.spin_limit = min(x.spin_limit, pl.polls);
   done = true;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (l.cleared && (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)) {

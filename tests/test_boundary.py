@@ -10,6 +10,7 @@ import tempfile
 import pytest
 import torch
 
+from helpers import prefill_plan
 from keys_values_amd import _lib
 from keys_values_amd.attention import ops
 from keys_values_amd.attention.sdpa import HipSDPA
@@ -376,6 +377,15 @@ def test_weights_refuse_query_rows_of_4_gib(kvx, q_len, kv_len):
             b = _lib.SdpaArgs.from_buffer_copy(a)
             setattr(b, name, stride)
             assert call(ctypes.byref(b), None) == _lib.KVX_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("B,heads,kv_heads,q_len,kv_len,D", [(1, 4, 1, 3, 64, 64), (1, 8, 2, 128, 1024, 64), (1, 16, 4, 128, 1500, 64), (1, 2, 1, 8, 8000, 128)])
+def test_a_chunk_waits_for_a_few_times_its_own_time(kvx, B, heads, kv_heads, q_len, kv_len, D):
+    # a poll is 1.5 to 2 us, these calls take 10 to 20; the single-token step waits for 2^15 polls
+    a = _prefill_block(B, heads, kv_heads, q_len, kv_len, D, 0)
+    a.lse = a.w = 4096
+    plan = prefill_plan(a)
+    assert plan.one_launch and 40 <= plan.polls <= 200
 
 
 @pytest.mark.parametrize("B,heads,kv_heads,q_len,splits", [(1, 4, 2, 100, 2), (4, 64, 16, 1446, 6), (8, 64, 16, 4096, 3)])

@@ -162,3 +162,27 @@ def test_two_streams_at_once(gpu):
         torch.cuda.synchronize()
         for x, y in zip(want, got):
             assert torch.equal(x[0], y[0]) and torch.equal(x[1], y[1])
+
+
+@pytest.mark.parametrize("Hq,Hkv,q_len,T,D", [(16, 4, 128, 1500, 64), (32, 8, 256, 512, 64)])  # splits and blocks of rows; blocks of rows alone
+def test_two_streams_that_fill_the_device_each(kvx, gpu, Hq, Hkv, q_len, T, D):
+    # more workgroups than units hold of both calls: those that wait take places of those that are waited for
+    tensors = [[t.to(gpu) for t in make_qkv(90 + i, 1, Hq, Hkv, q_len, T, D)[:3]] for i in range(2)]
+    a = _lib.SdpaArgs()
+    ops._fill_common(a, *tensors[0], 0.125, T - q_len, None, None, 0)
+    a.o, a.lse, a.w = (tensors[0][0].data_ptr(),) * 3  # (nothing is launched with them)
+    a.o_stride_b, a.o_stride_h, a.o_stride_t = tensors[0][0].stride()[:3]
+    plan = prefill_plan(a)
+    lds = plan.block_rows * (4 * 4 * (D + 4) + 4 * plan.split_keys)  # of a workgroup, without the smaller parts
+    assert plan.one_launch and plan.row_blocks > 1 and lds > 80 * 1024 and plan.row_blocks * Hkv * plan.splits > 128
+    want = [ops.prefill_core(*t, 0.125, T - q_len, None, return_weights=True) for t in tensors]
+    streams = [torch.cuda.Stream(gpu) for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(10):
+        got = []
+        for s, t in zip(streams, tensors):
+            with torch.cuda.stream(s):
+                got.append(ops.prefill_core(*t, 0.125, T - q_len, None, return_weights=True))
+        torch.cuda.synchronize()
+        for x, y in zip(want, got):
+            assert torch.equal(x[0], y[0]) and torch.equal(x[1], y[1])
