@@ -39,5 +39,6 @@ struct RowsPlan {
 RowsPlan rows_plan(const kvx_sdpa_args& a, bool combined);
 int launch_sdpa_rows(const PrefillParams& p, int D, int kv, hipStream_t st);
 void common_params(PrefillParams& p, const kvx_sdpa_args& a);
+int64_t prefill_ns(const kvx_sdpa_args& a);  // estimate of a call's attention launch where a score-sum launch follows
 
 }  // namespace kvx

@@ -758,6 +758,7 @@ __global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(const MergePara
 struct Splits {
   int n;
   bool pair;
+  int64_t ns;
 };
 Splits pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
   const int64_t base = (int64_t)a.B * a.Hkv * m_blocks, cus = num_cus();
@@ -766,8 +767,7 @@ Splits pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
   if (!plain) tile_ns = a.D == 256 ? 5500 : a.D == 64 ? 1700 : 2560;  // 256 rows a workgroup, codes to dequantise (at 256: 128 rows)
   const bool two = pairs(a.kv_dtype, a.D);
   const int64_t rows = (int64_t)a.B * a.Hq * a.q_len;
-  Splits best = {1, false};
-  int64_t best_ns = INT64_MAX;
+  Splits best = {1, false, INT64_MAX};
   for (int s = 1; s <= min(64, num_tiles); ++s) {
     const int tps = (num_tiles + s - 1) / s;
     if ((num_tiles + tps - 1) / tps != s) continue;
@@ -776,9 +776,7 @@ Splits pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
     const int64_t partials = s * rows * (a.D * 4 + 8);
     const int64_t merge = s == 1 ? 0 : two ? 3400 + 30 * s + partials / 2000 : 2000 + partials / 4000;
     auto consider = [&](int64_t walk, bool pair) {
-      if (walk + merge >= best_ns) return;
-      best_ns = walk + merge;
-      best = {s, pair};
+      if (walk + merge < best.ns) best = {s, pair, walk + merge};
     };
     if (!two) {
       consider(tps * tile_ns * c, false);
@@ -1003,6 +1001,12 @@ static kvx_sdpa_args on_copy(const kvx_sdpa_args& a, void* rows) {
   c.k_stride_h = c.v_stride_h = (int64_t)a.kv_len * a.D;
   c.k_stride_b = c.v_stride_b = (int64_t)a.Hkv * a.kv_len * a.D;
   return c;
+}
+
+int64_t prefill_ns(const kvx_sdpa_args& a) {
+  const RowsPlan rows = rows_plan(a, score_sum_combines(a));
+  const int bm = 32 * nwaves(a.kv_dtype, a.D);
+  return rows.columns ? rows.ns : pick_splits(a, (int)(((int64_t)a.q_len * (a.Hq / a.Hkv) + bm - 1) / bm), (a.kv_len + BN - 1) / BN).ns;
 }
 
 int sdpa_prefill_block_rows(const kvx_sdpa_args& a, bool may_copy) {

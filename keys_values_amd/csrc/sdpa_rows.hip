@@ -731,7 +731,8 @@ int launch_sdpa_rows(const PrefillParams& p, int D, int kv, hipStream_t st) { re
 
 namespace {
 
-// Attention with weights in one launch: rows of a workgroup and keys of a split with the least estimated time, 0 where a call takes two.
+// Attention with weights in one launch: rows of a workgroup and keys of a split with the least estimated time, 0 where a call takes two
+// (two_launches_win among them).
 //
 // All workgroups have to fit the device at once, because they wait for each other: for the splits of their rows, and for the sums of the other
 // blocks of rows. The waits take 2.5 us and 30 ns a split, a step half as long again as without weights, one of 64 keys six tenths of that; 172 of 220
@@ -748,6 +749,31 @@ namespace {
 struct WeightsPlan {
   int columns, splits, split_keys, polls;
 };
+
+// Whether two launches are estimated to take less than the one: for calls of several blocks of rows and several splits, where both waits are paid. (One split or
+// rows of 256 values never lost in 378 calls, one block of rows 4 % at most; they are not priced.) Both prices are fits to GPU times of 1513 such calls of 17 to 2000 rows over 64 to 40000
+// keys, 4 % off in the mean square. Always one launch took 2.3 % longer than the better of both in the mean (at most 23 %), two launches 7.1 % (53 %), as
+// chosen 0.6 % (17 %). one / two launches, us: 105 rows over 16 x 756 15.7 / 14.8, 184 of 64 over 4 x 3428 8-bit keys 16.0 / 14.6, 20 of 64 over 2 x 15221
+// 13.4 / 10.9, 120 over 8 x 1326 4-bit 19.3 / 16.1; 508 of 64 over 2 x 2336 14.1 / 17.1.
+bool two_launches_win(const kvx_sdpa_args& a, const WeightsPlan& pl, int64_t one_ns) {
+  const int64_t groups = (int64_t)a.B * a.Hkv, rows = (int64_t)a.q_len * (a.Hq / a.Hkv), blocks = (rows + 31) / 32, row_blocks = (rows + pl.columns - 1) / pl.columns;
+  const int64_t c = (groups * row_blocks * pl.splits + num_cus() - 1) / num_cus();
+  const bool narrow = a.D == 64;
+  const int64_t one = one_ns * 115 / 100 + 5700 + (narrow ? 20 : 45) * row_blocks - 900 * (c - 1) - (narrow ? pl.split_keys * 3 / 2 : 0);
+  int64_t second;  // and what both launches have besides their walks
+  switch (score_sum_kind(a)) {
+    case KVX_SCORE_SUM_SHORT: second = (narrow ? 6300 : 7000) + (narrow ? 1200 : 1300) * ((blocks + 3) / 4); break;
+    case KVX_SCORE_SUM_STREAMED: {
+      const int64_t rounds = (groups * ((a.kv_len + 63) / 64) + 2047) / 2048;
+      second = narrow ? 6000 + 600 * rounds + 900 * blocks : 3200 + 1600 * rounds + 3200 * blocks;
+      break;
+    }
+    default: second = 8200 + (narrow ? 230 : 400) * ((groups * ((a.kv_len + 255) / 256) + 255) / 256) * ((rows + 63) / 64);
+  }
+  if (!kv_is_plain(a.kv_dtype) && !narrow) second += 400;
+  return one > second && one > second + prefill_ns(a) * (narrow ? 119 : 131) / 100;
+}
+
 WeightsPlan weights_plan(const kvx_sdpa_args& a) {
   WeightsPlan best = {0, 0, 0, 0};
   const bool plain = kv_is_plain(a.kv_dtype);
@@ -772,6 +798,7 @@ WeightsPlan weights_plan(const kvx_sdpa_args& a) {
       }
     }
   }
+  if (best.splits > 1 && rows > best.columns && a.D <= 128 && two_launches_win(a, best, best_ns)) return {0, 0, 0, 0};
   return best;
 }
 

@@ -388,6 +388,25 @@ def test_a_chunk_waits_for_a_few_times_its_own_time(kvx, B, heads, kv_heads, q_l
     assert plan.one_launch and 40 <= plan.polls <= 200
 
 
+@pytest.mark.parametrize("B,heads,kv_heads,q_len,kv_len,D,kv_dtype,one_launch", [
+    (2, 56, 8, 15, 756, 128, _lib.KVX_KV_BF16, 0),    # 105 rows: several splits and blocks of rows
+    (1, 16, 4, 46, 3428, 64, _lib.KVX_KV_U8, 0),      # 184
+    (1, 28, 2, 2, 15221, 64, _lib.KVX_KV_F16, 0),     # 28 rows, streamed
+    (1, 24, 8, 12, 14390, 128, _lib.KVX_KV_BF16, 0),  # 36 rows, tiled
+    (1, 8, 2, 128, 1024, 64, _lib.KVX_KV_BF16, 1),
+    (1, 28, 4, 30, 400, 128, _lib.KVX_KV_U4, 1),
+    (1, 4, 2, 8, 4000, 64, _lib.KVX_KV_BF16, 1),      # one block of rows
+    (1, 32, 8, 20, 200, 64, _lib.KVX_KV_BF16, 1),     # one split
+])
+def test_weights_in_one_launch_or_two(kvx, B, heads, kv_heads, q_len, kv_len, D, kv_dtype, one_launch):
+    # the launches that measured faster (on 256 compute units)
+    a = _prefill_block(B, heads, kv_heads, q_len, kv_len, D, 0)
+    a.lse = a.w = 4096
+    a.kv_dtype = kv_dtype
+    a.k_scale = a.k_zp = a.v_scale = a.v_zp = 4096
+    assert bool(prefill_plan(a).one_launch) == bool(one_launch)
+
+
 @pytest.mark.parametrize("B,heads,kv_heads,q_len,splits", [(1, 4, 2, 100, 2), (4, 64, 16, 1446, 6), (8, 64, 16, 4096, 3)])
 def test_workspace_of_splits_of_any_size(kvx, B, heads, kv_heads, q_len, splits):
     # the second and third beyond 2^31 and 2^32 bytes
