@@ -122,8 +122,10 @@ __device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
 }
 
 // Least, largest, least and largest of a workgroup's four values in one exchange: four reductions one after the other took a third of the launches that
-// need them (16 rows of 6000 slots, us: statistics 8.2 -> 7.3, sort 6.3 -> 5.5). Called once by a kernel.
-template <int THREADS>
+// need them (16 rows of 6000 slots, us: statistics 8.2 -> 7.3, sort 6.3 -> 5.5). Called once by a kernel. AT_ONCE: wavefronts whose
+// values are read together; all 16 of 1024 threads are 60 registers, with which the sort of 1024 keys left a unit room for one workgroup, not two
+// (20 choices of 1 to 32 rows of 37000 to 115000 slots: 39.2 us in the mean, 48.1 that way).
+template <int THREADS, int AT_ONCE = THREADS / 64>
 __device__ __forceinline__ f32x4_t block_extremes(f32x4_t v) {
   __shared__ f32x4_t red[THREADS / 64];
   auto fold = [](const f32x4_t& x, const f32x4_t& y) { return f32x4_t{fminf(x[0], y[0]), fmaxf(x[1], y[1]), fminf(x[2], y[2]), fmaxf(x[3], y[3])}; };
@@ -143,7 +145,7 @@ __device__ __forceinline__ f32x4_t block_extremes(f32x4_t v) {
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
   f32x4_t r = red[0];
-#pragma unroll
+#pragma unroll AT_ONCE
   for (int i = 1; i < THREADS / 64; ++i) r = fold(r, red[i]);
   return r;
 }
@@ -508,7 +510,7 @@ __device__ __forceinline__ unsigned long long sort_list(unsigned long long x, un
 }
 
 template <int L>
-__global__ __launch_bounds__(L) void list_sort_kernel(const kvx_h2o_args a, const SelectLists sl) {
+__global__ __launch_bounds__(L, 8) void list_sort_kernel(const kvx_h2o_args a, const SelectLists sl) {
   __shared__ float red[L / 64];
   __shared__ unsigned long long buf[2][L];
   const int tid = threadIdx.x, c = blockIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
@@ -528,7 +530,7 @@ __global__ __launch_bounds__(L) void list_sort_kernel(const kvx_h2o_args a, cons
       v4[2] = fminf(v4[2], s4[2]);
       v4[3] = fmaxf(v4[3], s4[3]);
     }
-    const f32x4_t ex = block_extremes<L>(f32x4_t{v4[0], v4[1], v4[2], v4[3]});
+    const f32x4_t ex = block_extremes<L, (L > 512 ? 8 : L / 64)>(f32x4_t{v4[0], v4[1], v4[2], v4[3]});
     Modify m;
     m.smin = ex[0];
     m.sden = ex[1] - m.smin;
