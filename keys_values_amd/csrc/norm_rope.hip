@@ -66,31 +66,35 @@ __device__ __forceinline__ float wave_sum(float x) {
   return x;
 }
 
-// Sum over the wavefronts that share a row (WHOLE: all of the workgroup, through LDS, added in wavefront order; else one).
-constexpr int MAX_WAVES = 8;
-template <bool WHOLE>
+// Sum over the WPR wavefronts that share a row (more than one: through LDS, added in wavefront order).
+template <int WPR>
 __device__ __forceinline__ float row_total(float ss) {
   ss = wave_sum(ss);
-  if constexpr (WHOLE) {
-    __shared__ float part[MAX_WAVES];
+  if constexpr (WPR > 1) {
+    __shared__ float part[WPR];
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
     __syncthreads();
     ss = part[0];
-    for (int i = 1; i < (int)blockDim.x / 64; ++i) ss += part[i];
+#pragma unroll
+    for (int i = 1; i < WPR; ++i) ss += part[i];
   }
   return ss;
 }
 
-// A wavefront a row, or (WHOLE) the workgroup; a lane holds up to MAXC chunks of 8 elements (dim <= threads of the row * 8 * MAXC).
-// Few long rows (a 1024-token chunk of hidden states) take the whole workgroup per row, of as many wavefronts as the row has chunks for
-// (row_waves): 2560 values are 320 lanes, and four wavefronts were a second round for one of them.
-template <int MAXC, bool WHOLE>
-__global__ __launch_bounds__(64 * MAX_WAVES) void rmsnorm_rows_kernel(const uint16_t* __restrict__ x, int64_t x_rs, uint16_t* __restrict__ out,
+// Threads of a workgroup: one row of several wavefronts, or rows of one each. The kernels of the latter are compiled for 512, which schedules the sum's loads 2 %
+// better in the mean and the plain norm's 2 % worse.
+constexpr int norm_threads(int WPR) { return WPR > 1 ? 64 * WPR : NT; }
+constexpr int norm_bound(int WPR) { return WPR > 1 ? 64 * WPR : 512; }
+
+// WPR wavefronts a row; a lane holds up to MAXC chunks of 8 elements (dim <= 64 * WPR * 8 * MAXC).
+// Few long rows (a 1024-token chunk of hidden states) take a workgroup per row (by_row_length).
+template <int MAXC, int WPR>
+__global__ __launch_bounds__(norm_bound(WPR)) void rmsnorm_rows_kernel(const uint16_t* __restrict__ x, int64_t x_rs, uint16_t* __restrict__ out,
                                                           int64_t o_rs, const float* __restrict__ weight, int64_t rows, int dim,
                                                           float eps, float factor) {
-  const int TPR = WHOLE ? blockDim.x : 64;  // threads per row
-  const int lane = WHOLE ? threadIdx.x : threadIdx.x & 63;
-  const int64_t row = WHOLE ? blockIdx.x : (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
+  constexpr int TPR = 64 * WPR;  // threads per row
+  const int lane = threadIdx.x % TPR;
+  const int64_t row = (int64_t)blockIdx.x * (norm_threads(WPR) / TPR) + threadIdx.x / TPR;
   if (row >= rows) return;  // uniform over the threads of a row (and over the workgroup where it shares one)
   const int nchunks = dim / 8;
   const uint16_t* xr = x + row * x_rs;
@@ -108,7 +112,7 @@ __global__ __launch_bounds__(64 * MAX_WAVES) void rmsnorm_rows_kernel(const uint
       ss += b * b;
     }
   }
-  ss = row_total<WHOLE>(ss);
+  ss = row_total<WPR>(ss);
   const Divisor denom(sqrtf(ss) * factor + eps);
   uint16_t* orow = out + row * o_rs;
 #pragma unroll
@@ -127,14 +131,14 @@ __global__ __launch_bounds__(64 * MAX_WAVES) void rmsnorm_rows_kernel(const uint
 // the normalisation that follows it (keys_values/model.py:560-584: x = attention_output + x, then
 // norm_2(x); x = mlp_output + x, then the next block's norm_1). The sum is rounded to bf16 before it is
 // normalised, as the two separate steps do. In place is allowed (x_out == x).
-template <int MAXC, bool WHOLE>
-__global__ __launch_bounds__(64 * MAX_WAVES) void add_rmsnorm_rows_kernel(const uint16_t* x, int64_t x_rs, const uint16_t* __restrict__ delta,
+template <int MAXC, int WPR>
+__global__ __launch_bounds__(norm_bound(WPR)) void add_rmsnorm_rows_kernel(const uint16_t* x, int64_t x_rs, const uint16_t* __restrict__ delta,
                                                               int64_t d_rs, uint16_t* x_out, int64_t xo_rs,
                                                               uint16_t* __restrict__ out, int64_t o_rs, const float* __restrict__ weight,
                                                               int64_t rows, int dim, float eps, float factor) {
-  const int TPR = WHOLE ? blockDim.x : 64;
-  const int lane = WHOLE ? threadIdx.x : threadIdx.x & 63;
-  const int64_t row = WHOLE ? blockIdx.x : (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
+  constexpr int TPR = 64 * WPR;
+  const int lane = threadIdx.x % TPR;
+  const int64_t row = (int64_t)blockIdx.x * (norm_threads(WPR) / TPR) + threadIdx.x / TPR;
   if (row >= rows) return;
   const int nchunks = dim / 8;
   u32x4_t v[MAXC];
@@ -157,7 +161,7 @@ __global__ __launch_bounds__(64 * MAX_WAVES) void add_rmsnorm_rows_kernel(const 
       ss += b * b;
     }
   }
-  ss = row_total<WHOLE>(ss);
+  ss = row_total<WPR>(ss);
   const Divisor denom(sqrtf(ss) * factor + eps);
   uint16_t* orow = out + row * o_rs;
 #pragma unroll
@@ -217,6 +221,7 @@ __global__ __launch_bounds__(NT) void swiglu_rows_kernel(const uint16_t* __restr
 // A workgroup per token: the rows are its query heads, then its key heads; LPR = D / 8 lanes a row hold four values of either half of it, so
 // a value and the one it is rotated with are in the same lane; the angles and weights of a lane are the same for all its rows. With a row's values in a
 // stretch a lane, partners through LDS and a row's place by 64-bit divisions: 27 -> 20.8 us for 40 heads of 4096 tokens, 10.4 -> 7.4 of 1024.
+constexpr int MAX_WAVES = 8;
 template <int D, int U>  // U: rows of a lane in flight
 __global__ __launch_bounds__(64 * MAX_WAVES) void qk_norm_rope_kernel(uint16_t* __restrict__ qkv, int64_t sb, int64_t st, int num, int Hq,
                                                           int Hkv, const float* __restrict__ qw, const float* __restrict__ kw,
@@ -271,25 +276,30 @@ __global__ __launch_bounds__(64 * MAX_WAVES) void qk_norm_rope_kernel(uint16_t* 
   }
 }
 
-// Wavefronts of a workgroup that takes a row, where rows of at least 2048 values are too few to fill the chip with a wavefront each (0: a wavefront
-// a row). us, four wavefronts and a division a value -> now: sum and norm of 4096 rows of 2560 18.7 -> 17.0, of 1024 7.4 -> 6.8.
-int row_waves(int64_t rows, int dim) {
-  if (dim < 2048 || dim > 64 * MAX_WAVES * 8 * 4 || rows > 16384) return 0;
-  const int chunks = (dim + 511) / 512;  // of a wavefront
-  const int each = (chunks + MAX_WAVES - 1) / MAX_WAVES;
-  return (chunks + each - 1) / each;
-}
-
-// `launch(chunks a lane, whole workgroup a row, grid, threads)`
+// Rows of at least 2048 values take a workgroup each where they are too few to fill the chip with a wavefront each: four wavefronts, and five to eight above
+// 4096 values, so that a lane holds two chunks at most. A wavefront for each chunk of a lane, counted at run time, held fewer rows in flight on a unit, and the count came from
+// memory. us, norm of 1024 rows of 2560 4.6 that way, 3.6 now (with a division a value and four wavefronts 4.1), of 4096 x 4096 15.8, 12.3 (13.7), of 16384 x 2560 31.5, 25.3 (27.7);
+// sum and norm of 1024 x 2560 5.4, 5.0 (5.7), 1024 x 4096 7.7, 5.9 (6.7), 1024 x 8192 10.2, 9.6 (11.6). Beyond the last-level cache eight wavefronts win from about 3600 values on: sums of
+// 16384 x 4096 95.7 with four, 91.3, of 12000 x 3840 60.6, 58.9, but of 10000 x 4096 46.9, 47.7 and of 16384 x 3072 65.5, 67.2. Above 4096 sums take no wavefront that half a row
+// leaves idle (8000 x 7168: seven 71, eight 74.4), norms alone eight (16384 x 7168: 88, 84). Rows of
+// 2048 take the kernel of two chunks as well, at the same bits: 1024 rows 3.3, with the second chunk left out 3.9. `tensors`: read and written.
+// `launch(chunks a lane, wavefronts a row, grid)`
 template <typename Launch>
-void by_row_length(int64_t rows, int dim, Launch launch) {
-  const int waves = row_waves(rows, dim);
-  const unsigned grid = (unsigned)(waves ? rows : (rows + NT / 64 - 1) / (NT / 64));
-  const int chunks = (dim / 8 + 64 * max(waves, 1) - 1) / (64 * max(waves, 1));
-  if (waves && chunks == 1) launch(std::integral_constant<int, 1>{}, std::true_type{}, grid, 64 * waves);
-  else if (waves) launch(std::integral_constant<int, 4>{}, std::true_type{}, grid, 64 * waves);
-  else if (chunks <= 4) launch(std::integral_constant<int, 4>{}, std::false_type{}, grid, NT);
-  else launch(std::integral_constant<int, 16>{}, std::false_type{}, grid, NT);
+void by_row_length(int64_t rows, int dim, int tensors, Launch launch) {
+  constexpr std::integral_constant<int, 1> I1{};
+  constexpr std::integral_constant<int, 2> I2{};
+  constexpr std::integral_constant<int, 4> I4{};
+  if (dim >= 2048 && rows <= 16384) {
+    if (dim <= 3584 || (dim <= 4096 && rows * dim * 2 * tensors <= (336ll << 20))) launch(I2, I4, (unsigned)rows);
+    else if (dim <= 4096 || dim > 7168 || tensors == 2) launch(I2, std::integral_constant<int, 8>{}, (unsigned)rows);
+    else if (dim <= 5120) launch(I2, std::integral_constant<int, 5>{}, (unsigned)rows);
+    else if (dim <= 6144) launch(I2, std::integral_constant<int, 6>{}, (unsigned)rows);
+    else launch(I2, std::integral_constant<int, 7>{}, (unsigned)rows);
+  } else if (dim <= 64 * 8 * 4) {
+    launch(I4, I1, (unsigned)((rows + NT / 64 - 1) / (NT / 64)));
+  } else {
+    launch(std::integral_constant<int, 16>{}, I1, (unsigned)((rows + NT / 64 - 1) / (NT / 64)));
+  }
 }
 
 }  // namespace
@@ -298,8 +308,9 @@ int launch_rmsnorm_rows(const void* x, int64_t x_rs, void* out, int64_t o_rs, co
                         hipStream_t st) {
   if (rows == 0) return KVX_OK;
   const float factor = 1.0f / sqrtf((float)dim);
-  by_row_length(rows, dim, [&](auto chunks, auto whole, unsigned grid, int threads) {
-    hipLaunchKernelGGL((rmsnorm_rows_kernel<decltype(chunks)::value, decltype(whole)::value>), dim3(grid), dim3(threads), 0, st, (const uint16_t*)x, x_rs,
+  by_row_length(rows, dim, 2, [&](auto chunks, auto waves, unsigned grid) {
+    constexpr int MAXC = decltype(chunks)::value, WPR = decltype(waves)::value;
+    hipLaunchKernelGGL((rmsnorm_rows_kernel<MAXC, WPR>), dim3(grid), dim3(norm_threads(WPR)), 0, st, (const uint16_t*)x, x_rs,
                        (uint16_t*)out, o_rs, weight, rows, dim, eps, factor);
   });
   KVX_HIP(hipGetLastError());
@@ -310,8 +321,9 @@ int launch_add_rmsnorm_rows(const void* x, int64_t x_rs, const void* delta, int6
                             int64_t o_rs, const float* weight, int64_t rows, int dim, float eps, hipStream_t st) {
   if (rows == 0) return KVX_OK;
   const float factor = 1.0f / sqrtf((float)dim);
-  by_row_length(rows, dim, [&](auto chunks, auto whole, unsigned grid, int threads) {
-    hipLaunchKernelGGL((add_rmsnorm_rows_kernel<decltype(chunks)::value, decltype(whole)::value>), dim3(grid), dim3(threads), 0, st, (const uint16_t*)x, x_rs,
+  by_row_length(rows, dim, 4, [&](auto chunks, auto waves, unsigned grid) {
+    constexpr int MAXC = decltype(chunks)::value, WPR = decltype(waves)::value;
+    hipLaunchKernelGGL((add_rmsnorm_rows_kernel<MAXC, WPR>), dim3(grid), dim3(norm_threads(WPR)), 0, st, (const uint16_t*)x, x_rs,
                        (const uint16_t*)delta, d_rs, (uint16_t*)x_out, xo_rs, (uint16_t*)out, o_rs, weight, rows, dim, eps, factor);
   });
   KVX_HIP(hipGetLastError());

@@ -50,6 +50,20 @@ def test_norms_out_of_range(gpu, dim):
             torch.testing.assert_close(got.float(), ref.float(), rtol=2**-7, atol=2**-133, equal_nan=True)  # (2^-133: a unit of 16-bit denormals)
 
 
+# the longest row of 4, 5, 6, 7 and 8 wavefronts, and one chunk more; sums beyond the last-level cache, and rows of a wavefront each
+@pytest.mark.parametrize("rows,dim", [(3, 2048), (2, 3584), (3, 3592), (2, 4096), (3, 4104), (2, 5120), (3, 5128), (2, 6144), (3, 6152), (2, 7168), (3, 7176), (2, 8192),
+                                      (16384, 3592), (16385, 2056)])
+def test_norms_at_the_ends_of_a_split(gpu, rows, dim):
+    gen = torch.Generator().manual_seed(rows + dim)
+    half = (torch.randn(rows, dim, generator=gen) * 2).to(torch.bfloat16)
+    x, weight = half * 2, torch.rand(dim, generator=gen) + 0.5
+    ref = LO.rmsnorm(x, weight, 1e-6)
+    added = half.to(gpu)
+    for got in (ops.rmsnorm(x.to(gpu), weight.to(gpu), 1e-6), ops.add_rmsnorm_(added, half.to(gpu), weight.to(gpu), 1e-6)):
+        torch.testing.assert_close(got.cpu().float(), ref.float(), rtol=2**-7, atol=0)  # a unit of the 8 bits kept
+    assert torch.equal(added.cpu(), x)
+
+
 def test_zeros_keep_their_sign(gpu):
     gen = torch.Generator().manual_seed(3)
     x = torch.randn(5, 2048, generator=gen).to(torch.bfloat16)
