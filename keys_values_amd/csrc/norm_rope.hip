@@ -218,24 +218,24 @@ __global__ __launch_bounds__(NT) void swiglu_rows_kernel(const uint16_t* __restr
   *(u32x4_t*)(out + r * o_rs + c * 8) = o;
 }
 
-// A workgroup per token: the rows are its query heads, then its key heads; LPR = D / 8 lanes a row hold four values of either half of it, so
-// a value and the one it is rotated with are in the same lane; the angles and weights of a lane are the same for all its rows. With a row's values in a
-// stretch a lane, partners through LDS and a row's place by 64-bit divisions: 27 -> 20.8 us for 40 heads of 4096 tokens, 10.4 -> 7.4 of 1024.
-constexpr int MAX_WAVES = 8;
+// A workgroup, or several (grid y), per token: the rows are its query heads, then its key heads; LPR = D / 8 lanes a row hold four values of either half of it, so
+// a value and the one it is rotated with are in the same lane; the angles and weights of a lane are the same for all its rows. `rows` of a workgroup at a time (each of U), every
+// `stride` heads. With a row's values in a stretch a lane, partners through LDS and a row's place by 64-bit divisions: 22.4 -> 16.8 us for 40 heads of 128 of 4096 tokens,
+// 8.0 -> 5.8 of 1024.
 template <int D, int U>  // U: rows of a lane in flight
-__global__ __launch_bounds__(64 * MAX_WAVES) void qk_norm_rope_kernel(uint16_t* __restrict__ qkv, int64_t sb, int64_t st, int num, int Hq,
+__global__ __launch_bounds__(512) void qk_norm_rope_kernel(uint16_t* __restrict__ qkv, int64_t sb, int64_t st, int num, int Hq,
                                                           int Hkv, const float* __restrict__ qw, const float* __restrict__ kw,
                                                           float eps, float factor, const float* __restrict__ cos_t,
-                                                          const float* __restrict__ sin_t, int input_pos) {
+                                                          const float* __restrict__ sin_t, int input_pos, int rows, int stride) {
   constexpr int LPR = D / 8;
   constexpr int HALF = D / 2;
-  const int col = threadIdx.x % LPR, first = threadIdx.x / LPR, rows = blockDim.x / LPR;
+  const int col = threadIdx.x % LPR, first = threadIdx.x / LPR;
   const int heads = Hq + Hkv;
   const int b = blockIdx.x / num, t = blockIdx.x - b * num;
   uint16_t* p = qkv + b * sb + (int64_t)t * st + col * 4;
   const f32x4_t cv = *(const f32x4_t*)(cos_t + (int64_t)(input_pos + t) * HALF + col * 4);
   const f32x4_t sv = *(const f32x4_t*)(sin_t + (int64_t)(input_pos + t) * HALF + col * 4);
-  for (int begin = 0; begin < heads; begin += U * rows) {
+  for (int begin = blockIdx.y * U * rows; begin < heads; begin += stride) {
     u32x2_t lo[U], hi[U];
 #pragma unroll
     for (int i = 0; i < U; ++i) {
@@ -345,13 +345,20 @@ int launch_qk_norm_rope(void* qkv, int64_t sb, int64_t stt, int B, int num, int 
                         float eps, const float* cos_t, const float* sin_t, int input_pos, hipStream_t st) {
   if (B == 0 || num == 0 || Hq + Hkv == 0) return KVX_OK;
   const float factor = 1.0f / sqrtf((float)D);
-  const int lanes = (Hq + Hkv) * (D / 8), rows = lanes <= NT ? 1 : 2;  // of a lane, and more where the workgroup is too small
-  const int threads = min(64 * MAX_WAVES, (lanes / rows + 63) / 64 * 64);
+  const int lanes = (Hq + Hkv) * (D / 8), lpr = D / 8;
   const int at_once = max(1, (1 << 22) / num);  // batch elements whose threads a grid can count
+  const int64_t tokens = (int64_t)min(at_once, B) * num;
+  // A token's rows over several workgroups where few tokens leave units idle or its rows are many; over one, two rows a lane, where up to 640 lanes of many
+  // tokens would read the angles again. us, one / several: 16 tokens of 72 heads of 256 5.8 / 2.6, of 40 of 128 3.2 / 2.5, 1024 of 72 of 128 10.7 / 8.6; 4096 of 40 of
+  // 64 9.8 / 11.2, of 10 of 256 10.0 / 11.4, 1024 of 40 of 128 5.8 / 6.1. (A workgroup a token for all: 16 of 72 of 256 6.1, as lanes of rows in a
+  // stretch 3.2.)
+  const int parts = lanes > 2 * NT + 128 || tokens <= 2 * num_cus() ? min((lanes + NT - 1) / NT, 65535) : 1;
+  const int rows = parts > 1 || lanes <= NT ? 1 : 2;  // of a lane
+  const int threads = parts > 1 ? NT : (lanes / rows + 63) / 64 * 64;
   auto launch = [&](auto kernel) {
     for (int done = 0; done < B; done += at_once)
-      hipLaunchKernelGGL(kernel, dim3((unsigned)(min(at_once, B - done) * num)), dim3(threads), 0, st, (uint16_t*)qkv + done * sb, sb, stt, num, Hq, Hkv, qw, kw, eps,
-                         factor, cos_t, sin_t, input_pos);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(min(at_once, B - done) * num), parts), dim3(threads), 0, st, (uint16_t*)qkv + done * sb, sb, stt, num, Hq, Hkv, qw, kw, eps,
+                         factor, cos_t, sin_t, input_pos, threads / lpr, parts * rows * (threads / lpr));
   };
   auto launch_d = [&](auto d_tag) {
     constexpr int HEAD = decltype(d_tag)::value;

@@ -103,3 +103,19 @@ def test_rope_head_counts(gpu, Hq, Hkv, D):
             # one rounding to 16 bits may go the other way before the rotation and one after it
             torch.testing.assert_close(got.float(), ref.float(), rtol=2**-6, atol=2**-6)
             assert (got != ref).float().mean().item() < 5e-3
+
+
+# tokens for two workgroups a unit and more: one workgroup of two rows a lane up to 640 lanes of rows, several of one row a lane above
+@pytest.mark.parametrize("num,Hq,Hkv,D", [(512, 32, 8, 64), (513, 32, 8, 64), (700, 35, 5, 128), (600, 36, 5, 128), (513, 33, 4, 64), (520, 28, 4, 256), (530, 9, 2, 256)])
+def test_rope_of_many_tokens(gpu, num, Hq, Hkv, D):
+    gen = torch.Generator().manual_seed(num + Hq)
+    qkv = torch.randn(1, num, (Hq + 2 * Hkv) * D, generator=gen).to(torch.bfloat16)
+    qw, kw = (torch.rand(D, generator=gen) + 0.5 for _ in range(2))
+    cos, sin = LO.rope_tables(num, D, 1e6)
+    refs = LO.qk_norm_rope(qkv, Hq, Hkv, D, qw, kw, 1e-6, cos, sin, 0)
+    g = qkv.to(gpu)
+    ops.qk_norm_rope_(g, Hq, Hkv, D, qw.to(gpu), kw.to(gpu), 1e-6, cos.to(gpu), sin.to(gpu), 0)
+    out = g.cpu().view(1, num, Hq + 2 * Hkv, D).transpose(1, 2)
+    for got, ref in zip(out.split((Hq, Hkv, Hkv), 1), refs):
+        torch.testing.assert_close(got.float(), ref.float(), rtol=2**-6, atol=2**-6)  # (as above)
+        assert (got != ref).float().mean().item() < 5e-3
