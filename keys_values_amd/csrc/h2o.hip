@@ -858,10 +858,13 @@ static size_t min_workspace(const kvx_h2o_args& a) { return best_bytes(a) + (a.q
 // (and where the caller's workspace does not hold them) one workgroup per row. Lists of 256 keys sort in 36 steps, 3 of them through LDS, of 512 in 45
 // and 6, of 1024 in 55 and 10 by four times the wavefronts of a list of 256; but every candidate is looked up in all lists, by as many workgroups that
 // each read the heads of all, and the shorter the lists, the more a run of new tokens fills one of them.
-// Whole choices in us, tokens mixed / new ones in a run, lists of 256, 512, 1024: 64 of 3534 slots, 16 rows 8.6 / 9.9, 9.5 / 9.5, 11.7; 512 of 8192, 8 rows 10.3 / 10.1,
-// 11.0 / 10.9, 13.4; 200 of 6000, 16 rows 9.8 / 13.4, 9.9 / 9.9, 12.2; 1024 of 16384, 8 rows 14.4 / 13.4, 13.6 / 13.1, 16.0 / 15.6; 881 of 12598, 64 rows 43.7, 34.6, 42.3;
-// 114 of 36535, 64 rows 82 / 105, 60 / 62, 75 / 79; 23 of 38378, 4 rows 12.9 / 16.5, 11.8 / 13.5, 12.3; 1024 of 65536, 8 rows 50 / 63, 26.8 / 36.5, 24.0 / 23.6.
-// So 256 while the device holds the workgroups side by side, three to a unit, and the look-ups are few for it, 512 up to 72 of them, and 1024 beyond.
+// So 256 while the device holds the workgroups side by side, three to a unit, and the look-ups are few for it; 512 up to 72 of them while the device holds their
+// workgroups, three to a unit, and where neither those nor those of 1024 keys (half as many, two to a unit) fit at once and a row's look-ups are few; 1024 else. (The
+// line was at 72 lists for any number of rows, priced against a sort of 1024 keys that had a unit to itself.)
+// Whole choices in us, lists of 256, 512, 1024:
+// 8 rows of 2336 slots 10.6, 9.1, 11.0; 32 x 3227 17.0, 15.1, 17.1; 16 x 30667 23.5, 20.0, 17.2; 32 x 27297 43.9, 33.9, 30.1; 64 x 14079 39.6, 30.7, 27.8;
+// 64 x 34634 97.0, 66.9, 53.0; 4 x 38257 11.1, 10.2, 11.5; 8 x 45366 with errors 27.3, 20.7, 22.9; 402 of 49003, 4 rows: 512 14.8, 1024 13.7; of 512 and 1024, 526 of 27297, 32 rows 33.9, 30.1, 2 of 20422 33.9, 36.9,
+// 558 of 26300, 16 rows 22.9, 18.5, 26 of 21229, 64 rows 34.3, 36.0.
 // Rows of up to 1024 slots are one list whatever k is, the shortest that holds them: its sort ends the choice and hands nothing on (64 of 1000 slots, 32 rows: 9.9 us as
 // four lists, 7.2 as one; in the 128 KiB of the static entry point, too little for four lists of 32 rows, 14.1 and 7.2); of 257 to 512 slots in a list of 512, not of 1024: 6.8 -> 5.0.
 struct ListPlan {
@@ -877,7 +880,9 @@ static ListPlan list_plan(const kvx_h2o_args& a) {
   p.C = (int)C;
   const int64_t n256 = (a.kv_len + 255) / 256, cus = num_cus();
   const bool few = C > 1 && a.kv_len <= 32768 && rows * n256 <= 3 * cus && a.k * n256 <= 32768 && rows * a.k * n256 <= 2048 * cus;
-  p.L = n256 == 1 || few ? 256 : n256 == 2 || (C > 1 && C <= 36) ? 512 : LIST;
+  const int64_t n512 = (a.kv_len + 511) / 512;
+  const bool medium = C > 1 && n512 <= 72 && (rows * n512 <= 3 * cus || (rows * n512 > 4 * cus && a.k * n512 <= 3072));
+  p.L = n256 == 1 || few ? 256 : n256 == 2 || medium ? 512 : LIST;
   p.lists = (a.kv_len + p.L - 1) / p.L;
   const size_t n = (size_t)(rows * C);
   p.off_z = p.lists > 1 ? (size_t)rows * p.lists * p.L * 8 : 0;

@@ -331,6 +331,13 @@ def test_first_chunk_write_refuses(kvx):
     (8, 7936, 1058, 8 * 1024),   # too many look-ups for a row
     (32, 3840, 1092, 15 * 256),
     (32, 3840, 1093, 4 * 1024),  # for all rows
+    (16, 24000, 500, 47 * 512),  # lists of 512: three workgroups to each of 256 units
+    (17, 24000, 500, 24 * 1024),
+    (21, 24000, 65, 24 * 1024),  # 987 workgroups: those of 1024 keys fit at once
+    (22, 24000, 65, 47 * 512),   # neither do: 3055 look-ups a row
+    (22, 24000, 66, 24 * 1024),
+    (8, 36300, 20, 71 * 512),    # up to 72 of them
+    (4, 36865, 20, 37 * 1024),
 ])
 def test_workspace_of_a_choice_is_its_lists(kvx, rows, kv_len, k, keys):
     """Which lists a row is sorted in, by the workspace that a choice asks for (on 256 compute units, what is assumed without a device):
