@@ -119,3 +119,51 @@ def test_rope_of_many_tokens(gpu, num, Hq, Hkv, D):
     for got, ref in zip(out.split((Hq, Hkv, Hkv), 1), refs):
         torch.testing.assert_close(got.float(), ref.float(), rtol=2**-6, atol=2**-6)  # (as above)
         assert (got != ref).float().mean().item() < 5e-3
+
+
+def in_turn(x):
+    """Sum over the last axis, one after the other, in the type of x."""
+    total = torch.zeros_like(x[..., 0])
+    for i in range(x.shape[-1]):
+        total = total + x[..., i]
+    return total
+
+
+def rounded_root(x):
+    return x.double().sqrt().float()  # (the root of 32-bit tensors on the CPU may be a unit off)
+
+
+@pytest.mark.parametrize("dim", [2048, 2560, 3592, 4096])
+def test_norms_add_their_squares_in_this_order(gpu, dim):
+    # 256 lanes: a lane's chunks of eight values one after the other, the lanes of a wavefront in pairs that lie 32, 16, ... 1 apart, four wavefronts in turn
+    gen = torch.Generator().manual_seed(dim)
+    x = torch.randn(400, dim, generator=gen).to(torch.bfloat16)
+    weight = torch.rand(dim, generator=gen) + 0.5
+    squares = F.pad(x.float(), (0, 4096 - dim)) ** 2
+    lanes = in_turn(squares.view(-1, 2, 4, 64, 8).permute(0, 2, 3, 1, 4).reshape(-1, 4, 64, 16))
+    while lanes.shape[-1] > 1:
+        half = lanes.shape[-1] // 2
+        lanes = lanes[..., :half] + lanes[..., half:]
+    norm = rounded_root(in_turn(lanes[..., 0])) * (1.0 / rounded_root(torch.tensor(float(dim)))) + 1e-6
+    ref = (x.float() / norm[:, None] * weight).to(torch.bfloat16)
+    assert torch.equal(ops.rmsnorm(x.to(gpu), weight.to(gpu), 1e-6).cpu(), ref)
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_heads_add_their_squares_in_this_order(gpu, D):
+    # runs of eight values one after the other, then the runs in pairs of neighbours
+    gen = torch.Generator().manual_seed(D)
+    num, Hq, Hkv = 300, 8, 4
+    qkv = torch.randn(1, num, (Hq + 2 * Hkv) * D, generator=gen).to(torch.bfloat16)
+    w = torch.rand(D, generator=gen) + 0.5
+    cos, sin = LO.rope_tables(num, D, 1e6)
+    x = qkv.float().view(num, Hq + 2 * Hkv, D)[:, : Hq + Hkv]
+    runs = in_turn((x * x).view(num, Hq + Hkv, D // 8, 8))
+    while runs.shape[-1] > 1:
+        runs = runs[..., 0::2] + runs[..., 1::2]
+    y = (x / (rounded_root(runs) * (1.0 / rounded_root(torch.tensor(float(D)))) + 1e-6) * w).to(torch.bfloat16).float()
+    lo, hi, c, s = y[..., : D // 2], y[..., D // 2 :], cos[:num, None, : D // 2], sin[:num, None, : D // 2]
+    ref = torch.cat((lo * c + -hi * s, hi * c + lo * s), -1).to(torch.bfloat16)
+    g = qkv.to(gpu)
+    ops.qk_norm_rope_(g, Hq, Hkv, D, w.to(gpu), w.to(gpu), 1e-6, cos.to(gpu), sin.to(gpu), 0)
+    assert torch.equal(g.cpu().view(num, Hq + 2 * Hkv, D)[:, : Hq + Hkv], ref)
