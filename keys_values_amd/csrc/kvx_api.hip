@@ -153,10 +153,9 @@ static int prefill_checked(const kvx_sdpa_args* a, const char* who, bool weights
     if (rc != KVX_OK || done) return rc;
   }
   MergeParams rest{};
-  const bool combines = weights && score_sum_combines(*a);
-  rc = launch_sdpa_prefill(*a, may_copy, st, combines ? &rest : nullptr);
+  rc = launch_sdpa_prefill(*a, may_copy, st, weights ? &rest : nullptr);
   if (rc != KVX_OK || !weights) return rc;
-  return launch_score_sum(*a, st, combines ? &rest : nullptr);
+  return launch_score_sum(*a, st, &rest);
 }
 
 int kvx_sdpa_prefill(const kvx_sdpa_args* a, void* stream) { return prefill_checked(a, "kvx_sdpa_prefill", false, false, (hipStream_t)stream); }

@@ -49,8 +49,11 @@ struct MergeParams;  // prefill_merge.h
 // may_copy: a quantised store may be dequantised into the workspace first; no field behind workspace_bytes is read.
 // `rest` not NULL: the KV splits' partials are left in the workspace, described in *rest, for launch_score_sum to combine
 int launch_sdpa_prefill(const kvx_sdpa_args& a, bool may_copy, hipStream_t st, MergeParams* rest = nullptr);
-// whether launch_score_sum takes the kernel that can combine the attention's partials in the same launch
+// whether launch_score_sum takes a kernel whose launch combines the attention's partials whatever the splits
 bool score_sum_combines(const kvx_sdpa_args& a);
+// whether the launches of the tiled kernel combine these partials (splits, teams and rows of m), in less time than a launch of their own would take. `room`: the
+// workspace has what sdpa_prefill_workspace asks for; else it is looked at
+bool score_sum_merges(const kvx_sdpa_args& a, const MergeParams& m, bool room);
 size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy);
 int sdpa_prefill_block_rows(const kvx_sdpa_args& a, bool may_copy);
 kvx_prefill_plan sdpa_prefill_plan(const kvx_sdpa_args& a, bool may_copy);

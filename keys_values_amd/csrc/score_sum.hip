@@ -48,11 +48,16 @@ struct ScoreParams {
 template <int CPR>
 __device__ __forceinline__ int swz(int r) { return CPR >= 16 ? (r & 15) : ((r >> 1) & 7); }
 
-template <int D>
+// Where the log-sum-exps come from the pairs of the attention's KV splits (MERGE): the most tiles a workgroup may walk, their log-sum-exps all in LDS.
+// (Tables of 8192 rows leave no room for workgroups of other streams' kernels on a unit: two layers of a stack with its score-sums on
+// a second stream 5.26 -> 5.48 ms. A table filled again every 32 tiles keeps its arguments alive in the loop: 40.9 -> 45 us of scattered slots' masked tiles.)
+constexpr int LT = 32;
+
+template <int D, bool MERGE>
 struct alignas(16) Smem {
   static constexpr int CPR = D / 8;  // 16-byte chunks per row
   u32x4_t q[2][BQ][CPR];
-  float lse[2][BQ];     // a tile's log-sum-exps are in registers before the barrier that frees its Q buffer
+  float lse[MERGE ? LT : 2][BQ];  // MERGE: of all tiles (fill_lse), +inf where a tile has no row; else a tile's are in registers before the barrier that frees its Q buffer
   int32_t qpos[4][BQ];  // read through the whole step (only by tiles that need the mask): a ring of four
 };
 
@@ -68,14 +73,14 @@ constexpr int tile_rows(int G) { return G <= BQ && BQ / G * G >= BQ - BQ / 8 ? B
 // w, w + W, ... of the CPR that make a tile (RPW = 64 / CPR rows each); lane l of instruction i fills LDS position
 // l % CPR of row i RPW + l / CPR, so it fetches the chunk that belongs there under the swizzle. Addresses are a
 // uniform base plus a 32-bit byte offset per lane (the host checks the range). Wavefront 0 also fetches the rows'
-// log-sum-exps (4 bytes per lane) and writes their positions.
+// log-sum-exps (4 bytes per lane; MERGE: fill_lse) and writes their positions.
 //   issue_steady: the tile is one of whole queries and full. Every row keeps its head and moves by BQ / G
 //     queries from tile to tile: the base advances by scalar adds and the lane offsets stay.
 //   issue: any tile. The offsets are formed per lane from the row's (query, head); rows past the end re-read the
 //     last valid row.
 //   land() overwrites the log-sum-exps of the rows a tile leaves empty and of those past the end with +inf: their weight
 //     is exactly zero.
-template <int D, int W>
+template <int D, int W, bool MERGE>
 struct QLoader {
   static constexpr int CPR = D / 8;
   static constexpr int RPW = 64 / CPR;
@@ -94,11 +99,11 @@ struct QLoader {
   float inv_g;         // 1 / G: (int)((r + 0.5f) * inv_g) == r / G for the small r of a tile
   int G, R, RT, Hq, input_pos, dq, dg, wave, lane;
   int q0, g0;          // (query, head) of the first row of the next tile to fetch
-  uint32_t lds_qw, lds_lse, lds_qpos;
+  uint32_t lds_qw, lds_lse;
   int next_row0;       // first row of the next tile to fetch
 
   // steady_first: index (counted from row_start) of the first tile issue_steady will be asked for
-  __device__ __forceinline__ void init(const ScoreParams& p, Smem<D>& sm, int b, int kvh, int tid, int row_start, int steady_first) {
+  __device__ __forceinline__ void init(const ScoreParams& p, Smem<D, MERGE>& sm, int b, int kvh, int tid, int row_start, int steady_first) {
     wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     lane = tid & 63;
     G = p.G; R = p.R; RT = p.rows_per_tile; Hq = p.Hq; input_pos = p.input_pos;
@@ -116,8 +121,6 @@ struct QLoader {
     ltile = lbase + (uint64_t)(qs * Hq) * 4u;
     qpv = input_pos + qs + lane / G;
     lds_qw = __builtin_amdgcn_readfirstlane(lds_addr_of(&sm.q[0][0][0]) + (uint32_t)(wave * 1024));
-    lds_lse = __builtin_amdgcn_readfirstlane(lds_addr_of(&sm.lse[0][0]));
-    lds_qpos = lds_addr_of(&sm.qpos[0][0]) + (uint32_t)(lane * 4);
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       rin[i] = (wave + W * i) * RPW + lane / CPR;
@@ -125,6 +128,7 @@ struct QLoader {
       const int rt = min(rin[i], RT - 1);  // the rows a tile leaves empty re-read its last one
       voff0[i] = (uint32_t)(rt % G) * q_shb + (uint32_t)(rt / G) * q_stb + cb[i];
     }
+    lds_lse = __builtin_amdgcn_readfirstlane(lds_addr_of(&sm.lse[0][0]));
     const int lt = min(lane, RT - 1);
     loff0 = (uint32_t)((lt / G) * Hq + lt % G) * 4u;
     next_row0 = row_start;
@@ -136,10 +140,10 @@ struct QLoader {
     if constexpr (I + 1 < NI) dma_q_steady<BUF, I + 1>();
   }
   template <int BUF>
-  __device__ __forceinline__ void issue_steady(Smem<D>& sm, int ring) {
+  __device__ __forceinline__ void issue_steady(Smem<D, MERGE>& sm, int ring) {
     dma_q_steady<BUF>();
     if (wave == 0) {
-      dma4_at<(uint32_t)(BUF * BQ * 4)>(ltile, loff0, lds_lse);
+      if constexpr (!MERGE) dma4_at<(uint32_t)(BUF * BQ * 4)>(ltile, loff0, lds_lse);
       sm.qpos[ring][lane] = qpv;
       qpv += dq;
     }
@@ -149,8 +153,8 @@ struct QLoader {
     next_row0 += RT;
   }
 
-  // start the transfers of the next tile into Q / lse buffer `buf` and position buffer `ring`
-  __device__ __forceinline__ void issue(Smem<D>& sm, int buf, int ring) {
+  // start the transfers of the next tile into Q buffer `buf` and position buffer `ring`
+  __device__ __forceinline__ void issue(Smem<D, MERGE>& sm, int buf, int ring) {
     const int row0 = next_row0;
     const int rl = R - 1;
 #pragma unroll
@@ -163,7 +167,7 @@ struct QLoader {
       const bool ok = row0 + lane < R;
       const int r = min(g0 + lane + q0 * G, rl) - q0 * G;
       const int dqi = (int)(((float)r + 0.5f) * inv_g);
-      dma4(lbase, (uint32_t)((q0 + dqi) * Hq + (r - dqi * G)) * 4u, lds_lse + (uint32_t)(buf * BQ * 4));
+      if constexpr (!MERGE) dma4(lbase, (uint32_t)((q0 + dqi) * Hq + (r - dqi * G)) * 4u, lds_lse + (uint32_t)(buf * BQ * 4));
       sm.qpos[ring][lane] = ok ? input_pos + q0 + dqi : INT_MAX;
     }
     q0 += dq;
@@ -176,23 +180,101 @@ struct QLoader {
   }
 
   // after s_waitcnt vmcnt(0), before the barrier that publishes the tile whose first row is row0
-  __device__ __forceinline__ void land(Smem<D>& sm, int row0, int buf) const {
-    if (wave == 0 && (lane >= RT || row0 + lane >= R)) sm.lse[buf][lane] = INFINITY;  // exp2(... - inf) = 0
+  __device__ __forceinline__ void land(Smem<D, MERGE>& sm, int row0, int buf) const {
+    if (!MERGE && wave == 0 && (lane >= RT || row0 + lane >= R)) sm.lse[buf][lane] = INFINITY;  // exp2(... - inf) = 0
   }
 };
 
+// The base-2 log-sum-exp of a row from the S (maximum, sum) pairs of its KV splits at ml[s * total_rows], shared out over T neighbouring lanes
+// (a power of two; `part`: which of them this one is). Up to 16 T pairs are one memory latency.
+__device__ __forceinline__ float combined_lse(const f32x2_t* ml, int64_t total_rows, int S, int part, int T) {
+  float M = -INFINITY, L = 0.0f;
+  for (int s0 = part; s0 < S; s0 += 16 * T) {
+    f32x2_t x[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) x[u] = ml[(int64_t)min(s0 + u * T, S - 1) * total_rows];
+    float Mn = M;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) Mn = fmaxf(Mn, x[u][0]);
+    const float Mu = Mn == -INFINITY ? 0.0f : Mn;
+    L *= fast_exp2(M - Mu);
+    M = Mn;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) L += s0 + u * T < S ? x[u][1] * fast_exp2(x[u][0] - Mu) : 0.0f;
+  }
+  float Mr = M;
+  for (int off = 1; off < T; off <<= 1) Mr = fmaxf(Mr, __shfl_xor(Mr, off, 64));
+  const float Mu = Mr == -INFINITY ? 0.0f : Mr;
+  L *= fast_exp2(M - Mu);
+  for (int off = 1; off < T; off <<= 1) L += __shfl_xor(L, off, 64);
+  return Mu + fast_log2(L);
+}
+
+// The log-sum-exps of the rows of `tiles` tiles from row0 on, by a workgroup of THREADS, from the pairs of the attention's KV splits. A combination
+// ahead of this launch is 5 to 9 us and its gap; every workgroup working its rows' pairs out again is a latency beside that of its
+// keys: 16 pairs a thread are in flight.
+template <int THREADS>
+__device__ __forceinline__ void fill_lse(const ScoreParams& p, const MergeParams& m, int b, int kvh, int tid, int row0, int tiles, float* lse_sh) {
+  const int S = m.num_splits * m.teams, RT = p.rows_per_tile, n = tiles * BQ;
+  const int64_t total_rows = (int64_t)p.B * p.Hkv * p.R;
+  const f32x2_t* ml = (const f32x2_t*)m.part_ml + (int64_t)(b * p.Hkv + kvh) * p.R;
+  auto row_of = [&](int i) { return row0 + i / BQ * RT + i % BQ; };
+  auto has_row = [&](int i) { return i % BQ < RT && row_of(i) < p.R; };
+  auto rows = [&](auto pairs_tag) {  // up to PAIRS pairs a row, N rows at a time
+    constexpr int PAIRS = decltype(pairs_tag)::value, N = 16 / PAIRS;
+    for (int i0 = tid; i0 < n; i0 += N * THREADS) {
+      f32x2_t x[N][PAIRS];
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int k = 0; k < PAIRS; ++k) x[u][k] = ml[(int64_t)min(k, S - 1) * total_rows + min(row_of(i0 + u * THREADS), p.R - 1)];
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+        const int i = i0 + u * THREADS;
+        float M = x[u][0][0], L = 0.0f;
+#pragma unroll
+        for (int k = 1; k < PAIRS; ++k) M = fmaxf(M, x[u][k][0]);
+        const float Mu = M == -INFINITY ? 0.0f : M;
+#pragma unroll
+        for (int k = 0; k < PAIRS; ++k) L += k < S ? x[u][k][1] * fast_exp2(x[u][k][0] - Mu) : 0.0f;
+        if (i < n) lse_sh[i] = has_row(i) ? Mu + fast_log2(L) : INFINITY;
+      }
+    }
+  };
+  if (S <= 4) {
+    rows(std::integral_constant<int, 4>{});
+  } else if (S <= 8) {
+    rows(std::integral_constant<int, 8>{});
+  } else {
+    const int lt = S <= 16 ? 0 : S <= 32 ? 1 : S <= 64 ? 2 : 3, T = 1 << lt, part = tid & (T - 1);
+    for (int i = tid >> lt; i < n; i += THREADS >> lt) {  // the lanes of a row leave the loop together
+      const float lse = combined_lse(ml + min(row_of(i), p.R - 1), total_rows, S, part, T);
+      if (part == 0) lse_sh[i] = has_row(i) ? lse : INFINITY;
+    }
+  }
+}
+
 // QSPLIT: the query rows are split over blockIdx.z (short caches that would otherwise leave compute units
 // idle); every split writes its sums to p.part and a second kernel adds them in a fixed order.
+// MERGE: the attention's KV splits are still to be combined. That second kernel does it, or, without splits of the query rows, workgroups behind those of
+// the key_blocks blocks of keys (merge_beside).
 //
 // The kernel is bound by the number of instructions a wavefront issues per tile (two wavefronts per SIMD issue
 // about one instruction per ten cycles each, whatever its kind), so the tile loop comes in three forms: tiles that
 // need the position mask and tiles that do not, each unrolled by two with every LDS address an immediate and the
 // transfers of the tile after next sent without bounds checks ("steady"), and a general form for the last tiles.
-template <int D, int KV, int W, bool QSPLIT>
-__global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(const ScoreParams p) {
+template <int D, int KV, int W, bool QSPLIT, bool MERGE>
+__global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(const ScoreParams p, const MergeParams m, const int key_blocks) {
   constexpr int BK = NW * W;  // keys per workgroup
   constexpr bool F16 = kv_elem_f16(KV);  // element type of q and k
-  __shared__ Smem<D> sm;
+  if constexpr (MERGE && !QSPLIT) {
+    if ((int)blockIdx.y >= key_blocks) {
+      const int64_t job = ((int64_t)((int)blockIdx.y - key_blocks) * gridDim.x + blockIdx.x) * (W / 4);
+      merge_job<D, F16, 1>(m, job + threadIdx.x / 256, threadIdx.x % 256);
+      return;
+    }
+  }
+  __shared__ Smem<D, MERGE> sm;
   __shared__ uint32_t arrivals[W];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -259,7 +341,7 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
     t_masked = (int)max((int64_t)0, min(tiles, (int64_t)num_qt));
     t_masked = min((t_masked + 1) & ~1, t_steady);
   }
-  QLoader<D, W> ld;
+  QLoader<D, W, MERGE> ld;
   ld.init(p, sm, b, kvh, tid, tbase * RT, 2);
   // LDS byte offsets of this lane's Q fragments (A operand): row mt 32 + n, chunk 2 j + h at position chunk ^ swz(row)
   constexpr int CPR = D / 8;
@@ -277,10 +359,11 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
     for (int j = 0; j < D / 16; ++j) qq[j] = *(const u32x4_t*)(qb + qa[j]);
   };
   // accumulator rows of a lane are 8 a + 4 h + (0..3)
-  auto load_lse = [&](f32x4_t (&ls)[4], auto buf_tag, auto mt_tag) {
+  auto load_lse = [&](f32x4_t (&ls)[4], int t, auto buf_tag, auto mt_tag) {
     constexpr int BUF = decltype(buf_tag)::value, MT = decltype(mt_tag)::value;
+    const float* l = &sm.lse[MERGE ? t : BUF][4 * h];
 #pragma unroll
-    for (int a = 0; a < 4; ++a) ls[a] = *(const f32x4_t*)&sm.lse[BUF][MT * 32 + 8 * a + 4 * h];
+    for (int a = 0; a < 4; ++a) ls[a] = *(const f32x4_t*)(l + MT * 32 + 8 * a);
   };
   // S block = 32 query rows x 64 keys, K in registers; k-steps J0 .. J1 - 1
   auto mfma_part = [&](f32x16_t (&s)[2], const u32x4_t (&qq)[D / 16], auto j0_tag, auto j1_tag) {
@@ -365,14 +448,8 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
   if (tid < W) arrivals[tid] = 0;
   ld.issue(sm, 0, 0);
   if (num_qt > 1) ld.issue(sm, 1, 1);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the K fragments and the first tiles have arrived
-  ld.land(sm, tbase * RT, 0);
-  if (num_qt > 1) ld.land(sm, (tbase + 1) * RT, 1);
-  __syncthreads();
   f32x16_t sa[2], sb[2];  // blocks 0 and 1 of the current tile
   u32x4_t qq[D / 16];
-  load_q(qq, I0, I0);
-  mfma_part(sa, qq, I0, KS);
 
   // Software pipeline: the matrix work of one block runs under the vector work of the block before.
   // Tile t + 2 is requested right behind the barrier of step t (the buffers of tile t are free from there on: its
@@ -386,16 +463,16 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
     const bool more = STEADY || t + 1 < num_qt;
     f32x4_t ls[4], ls1[4];
     load_q(qq, buf_tag, I1);
-    load_lse(ls, buf_tag, I0);
+    load_lse(ls, t, buf_tag, I0);
     __builtin_amdgcn_sched_barrier(0);
     mfma_part(sb, qq, I0, KS3);
     valu_part(mask_tag, sa, ls, ring, 0, I0, I3);
     interleave(mask_tag, I3);
     pin(sb);
     __builtin_amdgcn_sched_barrier(0);
-    load_lse(ls1, buf_tag, I1);  // into registers before the barrier that hands the buffer to tile t + 2
+    load_lse(ls1, t, buf_tag, I1);  // into registers before the barrier that hands the buffer to tile t + 2
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wavefront's part of tile t + 1 has landed
-    if (!STEADY || RT < BQ) {
+    if (!MERGE && (!STEADY || RT < BQ)) {
       if (more) ld.land(sm, (tbase + t + 1) * RT, BUF ^ 1);
     }
     arrive();
@@ -425,6 +502,13 @@ __global__ __launch_bounds__(64 * W, D <= 128 ? 2 : 1) void score_sum_kernel(con
   };
   constexpr std::true_type YES{};
   constexpr std::false_type NO{};
+  if constexpr (MERGE) fill_lse<64 * W>(p, m, b, kvh, tid, tbase * RT, num_qt, &sm.lse[0][0]);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the K fragments and the first tiles have arrived
+  ld.land(sm, tbase * RT, 0);
+  if (num_qt > 1) ld.land(sm, (tbase + 1) * RT, 1);
+  __syncthreads();
+  load_q(qq, I0, I0);
+  mfma_part(sa, qq, I0, KS);
   int t = 0;
   for (; t < t_masked; t += 2) {
     step(YES, YES, I0, t);
@@ -466,27 +550,7 @@ __device__ __forceinline__ void row_weights(const ScoreParams& p, const MergePar
     if (m.num_splits <= 1) {
       lse = p.lse[((int64_t)b * p.q_len + qi) * p.Hq + kvh * p.G + (rc - qi * p.G)];
     } else {
-      const f32x2_t* ml = (const f32x2_t*)m.part_ml + (int64_t)group * p.R + rc;
-      float M = -INFINITY, L = 0.0f;
-      for (int s0 = part; s0 < S; s0 += 16 * T) {
-        f32x2_t x[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) x[u] = ml[(int64_t)min(s0 + u * T, S - 1) * total_rows];
-        float Mn = M;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) Mn = fmaxf(Mn, x[u][0]);
-        const float Mu = Mn == -INFINITY ? 0.0f : Mn;
-        L *= fast_exp2(M - Mu);
-        M = Mn;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) L += s0 + u * T < S ? x[u][1] * fast_exp2(x[u][0] - Mu) : 0.0f;
-      }
-      float Mr = M;
-      for (int off = 1; off < T; off <<= 1) Mr = fmaxf(Mr, __shfl_xor(Mr, off, 64));
-      const float Mu = Mr == -INFINITY ? 0.0f : Mr;
-      L *= fast_exp2(M - Mu);
-      for (int off = 1; off < T; off <<= 1) L += __shfl_xor(L, off, 64);
-      lse = Mu + fast_log2(L);
+      lse = combined_lse((const f32x2_t*)m.part_ml + (int64_t)group * p.R + rc, total_rows, S, part, T);
     }
     if (part == 0) {
       lse_sh[r] = r < p.R ? lse : INFINITY;
@@ -511,7 +575,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void score_sum_short_kernel(
   constexpr bool F16 = kv_elem_f16(KV);
   constexpr int KS = D / 16;
   if ((int)blockIdx.x >= score_jobs) {
-    merge_job<D, F16, SC>(m, (int)blockIdx.x - score_jobs);
+    merge_job<D, F16, SC>(m, (int)blockIdx.x - score_jobs, threadIdx.x);
     return;
   }
   __shared__ __align__(16) float lse_sh[SHORT_ROWS];
@@ -637,7 +701,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void score_sum_stream_kernel
   constexpr bool F16 = kv_elem_f16(KV), PLAIN = kv_is_plain(KV), U4 = kv_is_u4(KV);
   constexpr int KS = D / 16, CPR = D / 8, ROWS = stream_rows(D);
   if ((int)blockIdx.x < merge_jobs) {
-    merge_job<D, F16, SC>(m, (int)blockIdx.x);
+    merge_job<D, F16, SC>(m, (int)blockIdx.x, threadIdx.x);
     return;
   }
   __shared__ u32x4_t q_sh[ROWS][CPR];  // chunk c of row r at c ^ swz(r)
@@ -764,9 +828,15 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void score_sum_stream_kernel
   }
 }
 
-// W = (1/G) * (part[0] + part[1] + ...), in that order.
-__global__ void score_sum_reduce_kernel(const float* part, float* w, int64_t n, int splits, float inv_g) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// What a split of the query rows leaves behind, in one launch: the first merge_jobs workgroups combine the attention's KV splits, the others add the
+// splits' sums, W = (1/G) * (part[0] + part[1] + ...), in that order.
+template <int D, bool F16>
+__global__ __launch_bounds__(256) void score_sum_finish_kernel(const MergeParams m, const int merge_jobs, const float* part, float* w, int64_t n, int splits, float inv_g) {
+  if ((int)blockIdx.x < merge_jobs) {
+    merge_job<D, F16, 1>(m, blockIdx.x, threadIdx.x);
+    return;
+  }
+  const int64_t i = (int64_t)((int)blockIdx.x - merge_jobs) * 256 + threadIdx.x;
   if (i >= n) return;
   float acc = part[i];
   for (int z = 1; z < splits; ++z) acc += part[(int64_t)z * n + i];
@@ -840,8 +910,8 @@ int launch_t(const ScoreParams& p, int splits, int waves, const MergeParams* res
     const int64_t score_jobs = (int64_t)groups * ((p.kv_len + NW - 1) / NW);
     const MergeParams m = rest ? *rest : MergeParams{};
     auto launch = [&](auto sc_tag) {
-      constexpr int SC = decltype(sc_tag)::value, ROWS = merge_rows(D, SC);
-      const int64_t merge_jobs = m.num_splits > 1 ? ((int64_t)groups * p.R + ROWS - 1) / ROWS : 0;
+      constexpr int SC = decltype(sc_tag)::value;
+      const int64_t merge_jobs = m.num_splits > 1 ? merge_blocks(m, D, SC) : 0;
       hipLaunchKernelGGL((score_sum_short_kernel<D, KV, SC>), dim3((unsigned)(score_jobs + merge_jobs)), dim3(256), 0, st, p, m, (int)score_jobs);
     };
     if (merge_wants_classes(m, D)) launch(std::integral_constant<int, merge_classes(D)>{});
@@ -854,8 +924,8 @@ int launch_t(const ScoreParams& p, int splits, int waves, const MergeParams* res
     const int nkb = (p.kv_len + NW - 1) / NW, most = (nkb + 3) / 4;
     const int per_group = max(1, min(most, (D <= 128 ? 2 : 1) * num_cus() / groups));
     auto launch = [&](auto sc_tag) {
-      constexpr int SC = decltype(sc_tag)::value, ROWS = merge_rows(D, SC);
-      const int64_t merge_jobs = m.num_splits > 1 ? ((int64_t)groups * p.R + ROWS - 1) / ROWS : 0;
+      constexpr int SC = decltype(sc_tag)::value;
+      const int64_t merge_jobs = m.num_splits > 1 ? merge_blocks(m, D, SC) : 0;
       hipLaunchKernelGGL((score_sum_stream_kernel<D, KV, SC>), dim3((unsigned)(merge_jobs + (int64_t)groups * per_group)), dim3(256), 0, st, p, m, (int)merge_jobs,
                          per_group);
     };
@@ -864,30 +934,71 @@ int launch_t(const ScoreParams& p, int splits, int waves, const MergeParams* res
     KVX_HIP(hipGetLastError());
     return KVX_OK;
   }
+  const MergeParams m = rest ? *rest : MergeParams{};
+  const int64_t jobs = m.num_splits > 1 ? merge_blocks(m, D, 1) : 0;
+  auto tiled = [&](auto waves_tag, auto split_tag, auto merge_tag) {
+    constexpr int W = decltype(waves_tag)::value;
+    constexpr bool QSPLIT = decltype(split_tag)::value, MERGE = decltype(merge_tag)::value;
+    const int key_blocks = (p.kv_len + W * NW - 1) / (W * NW), per_y = groups * (W / 4);
+    const dim3 grid(groups, key_blocks + (unsigned)(QSPLIT ? 0 : (jobs + per_y - 1) / per_y), splits);
+    hipLaunchKernelGGL((score_sum_kernel<D, KV, W, QSPLIT, MERGE>), grid, dim3(64 * W), 0, st, p, m, key_blocks);
+  };
+  auto tiled_any = [&](auto waves_tag, auto split_tag) {
+    if (jobs) tiled(waves_tag, split_tag, std::true_type{});
+    else tiled(waves_tag, split_tag, std::false_type{});
+  };
   if (splits > 1) {
-    hipLaunchKernelGGL((score_sum_kernel<D, KV, 4, true>), dim3(groups, (p.kv_len + 4 * NW - 1) / (4 * NW), splits), dim3(256), 0, st, p);
+    tiled_any(std::integral_constant<int, 4>{}, std::true_type{});
     KVX_HIP(hipGetLastError());
     const int64_t n = (int64_t)groups * p.kv_len;
-    hipLaunchKernelGGL(score_sum_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p.part, p.w, n, splits, p.inv_g);
-    KVX_HIP(hipGetLastError());
-    return KVX_OK;
-  }
-  if constexpr (D <= 128) {
-    if (waves == 8) {
-      hipLaunchKernelGGL((score_sum_kernel<D, KV, 8, false>), dim3(groups, (p.kv_len + 8 * NW - 1) / (8 * NW)), dim3(512), 0, st, p);
-      KVX_HIP(hipGetLastError());
-      return KVX_OK;
+    hipLaunchKernelGGL((score_sum_finish_kernel<D, kv_elem_f16(KV)>), dim3((unsigned)(jobs + (n + 255) / 256)), dim3(256), 0, st, m, (int)jobs, p.part, p.w, n, splits, p.inv_g);
+  } else {
+    bool wide = false;
+    if constexpr (D <= 128) wide = waves == 8;
+    if constexpr (D <= 128) {
+      if (wide) tiled_any(std::integral_constant<int, 8>{}, std::false_type{});
     }
+    if (!wide) tiled_any(std::integral_constant<int, 4>{}, std::false_type{});
   }
-  hipLaunchKernelGGL((score_sum_kernel<D, KV, 4, false>), dim3(groups, (p.kv_len + 4 * NW - 1) / (4 * NW)), dim3(256), 0, st, p);
   KVX_HIP(hipGetLastError());
   return KVX_OK;
+}
+
+// Where the score-sums' partial sums go: the workspace, but not over partials of the attention that are still to be combined. NULL: no room.
+float* score_scratch(const kvx_sdpa_args& a, const MergeParams* rest) {
+  const size_t need = score_sum_workspace(a);
+  if (!a.workspace || ((uintptr_t)a.workspace & 15)) return nullptr;
+  size_t at = 0;
+  if (rest && rest->num_splits > 1) {
+    const char* ml_end = (const char*)(rest->part_ml + (size_t)2 * rest->num_splits * rest->teams * rest->B * rest->Hkv * rest->R);
+    if ((size_t)((const char*)rest->part_o - (const char*)a.workspace) < need) at = ((size_t)(ml_end - (const char*)a.workspace) + 15) & ~(size_t)15;
+  }
+  return a.workspace_bytes >= at + need ? (float*)((char*)a.workspace + at) : nullptr;
+}
+
+// Whether workgroups beside the score jobs combine the attention's partials: the jobs' last round leaves `spare` places, for the time of a walk, and a
+// workgroup takes 2.5 us there. Where they do not fit they end behind the score jobs, a few to a unit, and a launch of their own ahead is shorter. Attention with
+// weights, us, launch ahead -> beside: 600 rows over 16 x 6000 keys 74 -> 71, 404 over 8 x 9444 50.3 -> 46.2, 564 of 64 over 8 x 6138 36.6 -> 33.6, 140 over
+// 16 x 2443 29.9 -> 24.0. Combined in the launch that adds the sums of a split of the query rows: 460 over 8 x 4238 50.1 -> 43.7, 1716 of 64 over
+// 8 x 1800 41.9 -> 35.3, 434 of 64 over 32 x 1216 35.7 -> 28.3, 2331 scattered over 8 x 5001 107.0 -> 105.6.
+bool merge_beside(const kvx_sdpa_args& a, const ScorePlan& pl, const MergeParams& m) {
+  const int64_t groups = (int64_t)a.B * a.Hkv, places = (int64_t)num_cus() * (pl.waves == 4 && a.D <= 128 ? 2 : 1);
+  const int64_t wgs = groups * ((a.kv_len + pl.waves * NW - 1) / (pl.waves * NW)), spare = (places - wgs % places) % places;
+  const int64_t jobs = merge_blocks(m, a.D, 1) / (pl.waves / 4);
+  const int64_t walk = ((int64_t)pl.tiles_per_z * (pl.waves == 8 ? 2500 : 1500) + 3000) * a.D / 128;
+  return jobs * 2500 <= spare * walk;
 }
 
 }  // namespace
 
 int score_sum_kind(const kvx_sdpa_args& a) { return is_short(a) ? KVX_SCORE_SUM_SHORT : is_streamed(a) ? KVX_SCORE_SUM_STREAMED : KVX_SCORE_SUM_TILED; }
 bool score_sum_combines(const kvx_sdpa_args& a) { return is_short(a) || (is_streamed(a) && merge_fits(a)); }
+
+bool score_sum_merges(const kvx_sdpa_args& a, const MergeParams& m, bool room) {
+  if (score_sum_kind(a) != KVX_SCORE_SUM_TILED || m.num_splits <= 1 || m.num_splits * m.teams > 32 || merge_wants_classes(m, a.D)) return false;
+  const ScorePlan pl = score_plan(a);
+  return pl.tiles_per_z <= LT && (pl.splits > 1 ? room || score_scratch(a, &m) != nullptr : merge_beside(a, pl, m));
+}
 
 size_t score_sum_workspace(const kvx_sdpa_args& a) {
   if (is_short(a) || is_streamed(a)) return 0;
@@ -907,11 +1018,12 @@ int check_score_sum(const kvx_sdpa_args& a) {
 int launch_score_sum(const kvx_sdpa_args& a, hipStream_t st, const MergeParams* rest) {
   // the query rows are split only if the caller's workspace holds the partial sums
   ScorePlan pl = score_plan(a);
-  if (pl.splits > 1 && !(a.workspace && a.workspace_bytes >= score_sum_workspace(a) && ((uintptr_t)a.workspace & 15) == 0)) pl = {1, 0, pl.waves};
+  float* scratch = pl.splits > 1 ? score_scratch(a, rest) : nullptr;
+  if (pl.splits > 1 && !scratch) pl = {1, 0, pl.waves};
   const int rc = check_score_sum(a);
   if (rc != KVX_OK) return rc;
   ScoreParams p;
-  p.part = pl.splits > 1 ? (float*)a.workspace : nullptr;
+  p.part = scratch;
   p.tiles_per_z = pl.tiles_per_z;
   p.rows_per_tile = tile_rows(a.Hq / a.Hkv);
   p.q = (const uint16_t*)a.q;

@@ -742,7 +742,7 @@ __global__ __launch_bounds__(64 * nwaves(KV, D) * (PAIR ? 2 : 1), (kv_is_plain(K
 }
 
 template <int D, bool F16, int SC>
-__global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(const MergeParams p) { merge_job<D, F16, SC>(p, blockIdx.x); }
+__global__ __launch_bounds__(256) void sdpa_prefill_merge_kernel(const MergeParams p) { merge_job<D, F16, SC>(p, blockIdx.x, threadIdx.x); }
 
 // The number of KV splits with the least estimated time, and whether a split is walked by a pair of teams (PAIR): c workgroups share a compute
 // unit, one after the other or side by side, and each walks its split's tiles; more splits balance the device better and shorten the walk, but
@@ -874,9 +874,14 @@ size_t partial_bytes(const PrefillParams& p, int D) {
   return rows * (size_t)D * 4 + rows * 2 * 4 * (p.pair ? 2 : 1);
 }
 
-// `rest`: where the partials are left for another launch to combine, their description (num_splits 1: nothing to combine)
+MergeParams merge_params(const PrefillParams& p) {
+  return {p.part_o, p.part_ml, p.o, p.lse, p.B, p.Hq, p.Hkv, p.G, p.q_len, p.R, p.num_splits, p.o_sb, p.o_sh, p.o_st,
+          p.input_pos, p.tp ? 0 : p.tiles_per_split * BN, p.pair ? 2 : 1};
+}
+
+// `rest`: where the score-sum launch of `a` follows, what is left for it to combine (num_splits 1: nothing). `combined`: its kernel takes any splits
 template <int D, int KV>
-int launch_t(PrefillParams& p, hipStream_t st, MergeParams* rest) {
+int launch_t(PrefillParams& p, const kvx_sdpa_args& a, hipStream_t st, MergeParams* rest, bool combined) {
   if (p.columns) {
     const int rc = launch_sdpa_rows(p, D, KV, st);
     if (rc != KVX_OK) return rc;
@@ -886,7 +891,7 @@ int launch_t(PrefillParams& p, hipStream_t st, MergeParams* rest) {
       const int n = p.num_splits, last = p.m_blocks - (n - 1) * p.period;
       grid.y = (unsigned)(p.m_blocks + p.period * ((n - 1) * (n - 2) / 2) + last * (n - 1));
       grid.z = 1;
-      if (rest) {  // the score-sum jobs read the maxima and sums of all splits of a row (its outputs are combined from those it sees)
+      if (combined) {  // the score-sum jobs read the maxima and sums of all splits of a row (its outputs are combined from those it sees)
         grid.y = (unsigned)p.m_blocks;
         grid.z = (unsigned)n;
         p.period = 0;
@@ -906,17 +911,16 @@ int launch_t(PrefillParams& p, hipStream_t st, MergeParams* rest) {
     if (general) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, false, false>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
     KVX_HIP(hipGetLastError());
   }
-  const MergeParams m = {p.part_o, p.part_ml, p.o, p.lse, p.B, p.Hq, p.Hkv, p.G, p.q_len, p.R, p.num_splits, p.o_sb, p.o_sh, p.o_st,
-                         p.input_pos, p.tp ? 0 : p.tiles_per_split * BN, p.pair ? 2 : 1};
+  const MergeParams m = merge_params(p);
   if (rest) {
     *rest = m;
-    return KVX_OK;
+    if (combined || (!p.period && score_sum_merges(a, m, false))) return KVX_OK;
+    rest->num_splits = 1;
   }
   if (p.num_splits > 1) {
-    const int64_t total_rows = (int64_t)p.B * p.Hkv * p.R;
     auto merge = [&](auto sc_tag) {
-      constexpr int SC = decltype(sc_tag)::value, ROWS = merge_rows(D, SC);
-      hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kv_elem_f16(KV), SC>), dim3((unsigned)((total_rows + ROWS - 1) / ROWS)), dim3(256), 0, st, m);
+      constexpr int SC = decltype(sc_tag)::value;
+      hipLaunchKernelGGL((sdpa_prefill_merge_kernel<D, kv_elem_f16(KV), SC>), dim3((unsigned)merge_blocks(m, D, SC)), dim3(256), 0, st, m);
     };
     if (merge_wants_classes(m, D)) merge(std::integral_constant<int, merge_classes(D)>{});
     else merge(std::integral_constant<int, 1>{});
@@ -1030,6 +1034,7 @@ kvx_prefill_plan sdpa_prefill_plan(const kvx_sdpa_args& a, bool may_copy) {
   plan.split_keys = p.tiles_per_split * BN;
   plan.teams = p.pair ? 2 : 1;
   plan.score_sum = a.w ? score_sum_kind(a) : KVX_SCORE_SUM_NONE;
+  if (a.w && !p.period && score_sum_merges(a, merge_params(p), true)) plan.combined = 1;
   return plan;
 }
 
@@ -1041,18 +1046,20 @@ size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy) {
     fill_params(p, copy ? on_copy(a, nullptr) : prefill_block(a), combined);
     partials = std::max(partials, partial_bytes(p, a.D));  // (max on the host is one of ints)
   }
-  // the score-sum pass that may follow on the same stream reuses the workspace for its partial sums
-  const size_t own = partials + (copy ? copy_bytes(a) : 0);
-  return std::max({own, score_sum_workspace(a), a.w ? rows_weights_workspace(a) : 0});  // (max on the host is one of ints)
+  // the score-sum pass that may follow on the same stream takes the place of the copy, or behind partials that it combines itself
+  const size_t sums = score_sum_workspace(a);
+  const size_t own = copy ? copy_bytes(a) + partials : partials && a.w ? (partials + 15) / 16 * 16 + sums : partials;
+  return std::max({own, sums, a.w ? rows_weights_workspace(a) : 0});  // (max on the host is one of ints)
 }
 
 int launch_sdpa_prefill(const kvx_sdpa_args& a_in, bool may_copy, hipStream_t st, MergeParams* rest) {
   PrefillParams p;
   kvx_sdpa_args a = prefill_block(a_in);
+  const bool combined = rest && score_sum_combines(a_in);
   if (may_copy && wants_copy(a)) {
     // a workspace too small for the copy (sized for another call, or by a caller that has no room): the fused form
     const kvx_sdpa_args c = on_copy(a, a.workspace);
-    fill_params(p, c, rest != nullptr);
+    fill_params(p, c, combined);
     if (a.workspace && a.workspace_bytes >= copy_bytes(a) + partial_bytes(p, a.D)) {
       const int rc = launch_dequantize_kv(a, a.workspace, st);
       if (rc != KVX_OK) return rc;
@@ -1061,8 +1068,8 @@ int launch_sdpa_prefill(const kvx_sdpa_args& a_in, bool may_copy, hipStream_t st
       a.workspace_bytes = a_in.workspace_bytes - copy_bytes(a_in);
     }
   }
-  fill_params(p, a, rest != nullptr);
-  if (rest && (!a.workspace || a.workspace_bytes < partial_bytes(p, a.D))) fill_params(p, a);  // no room: the (fewer) splits of a call without weights
+  fill_params(p, a, combined);
+  if (combined && (!a.workspace || a.workspace_bytes < partial_bytes(p, a.D))) fill_params(p, a);  // no room: the (fewer) splits of a call without weights
   const size_t need = partial_bytes(p, a.D);
   if (need) {
     KVX_REQUIRE(a.workspace && a.workspace_bytes >= need, KVX_ERR_WORKSPACE,
@@ -1072,7 +1079,7 @@ int launch_sdpa_prefill(const kvx_sdpa_args& a_in, bool may_copy, hipStream_t st
     p.part_ml = p.part_o + rows * (size_t)a.D;
   }
 #define KVX_PREFILL_CASE(KV) \
-  case KV: return a.D == 256 ? launch_t<256, KV>(p, st, rest) : a.D == 128 ? launch_t<128, KV>(p, st, rest) : launch_t<64, KV>(p, st, rest);
+  case KV: return a.D == 256 ? launch_t<256, KV>(p, a_in, st, rest, combined) : a.D == 128 ? launch_t<128, KV>(p, a_in, st, rest, combined) : launch_t<64, KV>(p, a_in, st, rest, combined);
   if (a.D == 256 || a.D == 128 || a.D == 64) {
     switch (a.kv_dtype) {
       KVX_PREFILL_CASE(KVX_KV_BF16)
