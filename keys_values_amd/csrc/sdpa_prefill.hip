@@ -632,7 +632,22 @@ __global__ __launch_bounds__(64 * nwaves(KV, D) * (PAIR ? 2 : 1), (kv_is_plain(K
   constexpr std::integral_constant<int, 1> B1{};
   constexpr std::true_type YES{};
   constexpr std::false_type NO{};
-  if (!PAIR || mine > 0) {
+  // A wavefront behind the last row has its share of the tiles to bring and nothing to multiply: those that have rows get the issue slots. us: 128 rows over
+  // 8 x 32768 8-bit keys (four of eight wavefronts) 49.3 -> 38.6, 4-bit 51.5 -> 39.6, of 64 values 32.5 -> 26.9, 35.5 -> 26.3; 136 / 260 / 520 plain rows 40.7 -> 36.3,
+  // 56.1 -> 51.7, 86.1 -> 81.7. (Of 256 values the kernel spills as it is, and with this beside it takes 1.4 times as long.)
+  const bool idle = D <= 128 && __builtin_amdgcn_readfirstlane(row0w) >= p.R;
+  if (D <= 128 && idle) {
+    for (int t = tile_begin, cur = 0; t < tile_end; ++t, cur ^= 1) {
+      const bool has1 = t + 1 < tile_end;
+      ld.template issue_one<false>(sm, t, cur, tid);
+      if (has1) ld.template issue_one<true>(sm, t + 1, cur ^ 1, tid);
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+      ld.template land<false>(sm, t, cur, tid);
+      if (has1) ld.template land<true>(sm, t + 1, cur ^ 1, tid);
+      arrive();
+      sync();
+    }
+  } else if (!PAIR || mine > 0) {
     step(YES, B0, NO, tile_begin);
     int t = tile_begin + 1;
     // tiles whose successor is a full tile of this walk take the step without bounds checks
@@ -765,6 +780,7 @@ Splits pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
   const bool plain = kv_is_plain(a.kv_dtype);
   int64_t tile_ns = a.D == 64 ? 840 : a.D == 128 ? 1130 : 2050;
   if (!plain) tile_ns = a.D == 256 ? 5500 : a.D == 64 ? 1700 : 2560;  // 256 rows a workgroup, codes to dequantise (at 256: 128 rows)
+  if (!plain && a.D <= 128 && a.q_len * (a.Hq / a.Hkv) <= 128) tile_ns = a.D == 64 ? 1150 : 1850;  // half of the wavefronts have rows
   const bool two = pairs(a.kv_dtype, a.D);
   const int64_t rows = (int64_t)a.B * a.Hq * a.q_len;
   Splits best = {1, false, INT64_MAX};
@@ -1008,7 +1024,7 @@ static kvx_sdpa_args on_copy(const kvx_sdpa_args& a, void* rows) {
 }
 
 int64_t prefill_ns(const kvx_sdpa_args& a) {
-  const RowsPlan rows = rows_plan(a, score_sum_combines(a));
+  const RowsPlan rows = rows_plan(a, score_sum_combines(a), true);  // one launch against two was measured with these estimates
   const int bm = 32 * nwaves(a.kv_dtype, a.D);
   return rows.columns ? rows.ns : pick_splits(a, (int)(((int64_t)a.q_len * (a.Hq / a.Hkv) + bm - 1) / bm), (a.kv_len + BN - 1) / BN).ns;
 }
