@@ -364,6 +364,11 @@ int kvx_cache_write(const kvx_cache_write_args* args, void* stream);
  * fewer than 2^24 workgroups of 256 threads: D / 8 of them a new row, and one for four of the other slots. */
 int kvx_cache_write_first(const kvx_cache_write_args* args, void* stream);
 
+/* kvx_cache_write_first and kvx_sdpa_prefill: the slot write of a first chunk and the attention over its rows, in one launch where the attention's workgroups
+ * can write the rows as well (head sizes 64 and 128, a causal chunk: input_pos 0, no token positions, q_len == kv_len == num, rows of the store's element type), else
+ * one after the other. Nothing of what either reads may overlap what the other writes. */
+int kvx_sdpa_prefill_first(const kvx_sdpa_args* args, const kvx_cache_write_args* write, void* stream);
+
 /* H2O score update and eviction choice, AttnWeightsKVCache._update with H2OKVCache._compute_scores
  * (keys_values/kvcache/attn_weights.py:721-783, keys_values/kvcache/h2o.py:146-199):
  *   scores[b,h,:kv_len] += w[b,h,:kv_len]           (skipped when w is NULL)

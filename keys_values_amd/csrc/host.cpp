@@ -46,6 +46,7 @@ struct Lib {
   KVX_HOST_SYMBOLS(X)
 #undef X
   decltype(&::kvx_cache_write_first) kvx_cache_write_first = nullptr;  // libraries from before it bind too
+  decltype(&::kvx_sdpa_prefill_first) kvx_sdpa_prefill_first = nullptr;  // likewise: the two calls it stands for
   bool bound = false;
 } lib;
 
@@ -605,6 +606,37 @@ PyObject* cache_write_first(PyObject* const* args, Py_ssize_t n) {
   Py_RETURN_NONE;
 }
 
+// prefill_first(cache, index, query, key, value, scale) -> out (B, num, Hq, D): the first chunk of a sequence into its slots, as cache_write_first, and its causal attention
+PyObject* prefill_first(PyObject* const* args, Py_ssize_t n) {
+  require_args(n, 6, "prefill_first");
+  const at::Tensor &q = tensor(args[2], "query"), &key = tensor(args[3], "key"), &value = tensor(args[4], "value");
+  const Launch L(q);
+  const WriteCall w = write_args(args[0], opt_tensor(args[1], "index"), key, value, 0, Py_None, Py_None);
+  const bool fills = w.a.num == w.a.cache_len;  // no slots behind the chunk: an ordinary write
+  if (!fills && !lib.kvx_cache_write_first) raise(PyExc_ImportError, "the bound library does not export kvx_cache_write_first");
+  for (const at::Tensor* t : {&q, &w.key, &w.value}) require_gpu(*t);
+  check_bhtd("query", q);
+  check_bhtd("key", w.key);
+  check_bhtd("value", w.value);
+  check_dtypes(q, w.key, &w.value, false);
+  check_kv(q, w.key, w.value, false);
+  check_heads(q.size(1), key.size(1));
+  check_head_size(q.size(3));
+  kvx_sdpa_args a = sdpa_args(q, w.key, &w.value, real(args[5]), 0, nullptr, 0);
+  at::Tensor out;
+  check(unlocked([&] {
+    out = L.empty({a.B, a.q_len, a.Hq, a.D}, q.scalar_type());
+    set_o(a, out, out.stride(0), out.stride(2), out.stride(1));
+    const at::Tensor ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
+    a.workspace = data(ws);
+    a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
+    if (lib.kvx_sdpa_prefill_first) return lib.kvx_sdpa_prefill_first(&a, &w.a, L.stream);
+    const int rc = (fills ? lib.kvx_cache_write : lib.kvx_cache_write_first)(&w.a, L.stream);
+    return rc ? rc : lib.kvx_sdpa_prefill(&a, L.stream);
+  }));
+  return wrap(out);
+}
+
 // Arguments of the score update and the choice of k slots; `full`: the cache has no free slot (else nothing is chosen
 // that anyone uses, and the smallest selection is run)
 kvx_h2o_args h2o_args(PyObject* cache, bool full, int64_t k, int64_t input_pos, Held& held) {
@@ -903,6 +935,7 @@ PyObject* bind(PyObject* const* args, Py_ssize_t n) {
   KVX_HOST_SYMBOLS(X)
 #undef X
   l.kvx_cache_write_first = (decltype(l.kvx_cache_write_first))dlsym(h, "kvx_cache_write_first");
+  l.kvx_sdpa_prefill_first = (decltype(l.kvx_sdpa_prefill_first))dlsym(h, "kvx_sdpa_prefill_first");
   l.bound = true;
   lib = l;
   Py_XSETREF(kvx_error, Py_NewRef(args[1]));
@@ -929,7 +962,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t n) {
 #define METHOD(name) {#name, (PyCFunction)(void (*)(void))entry<name>, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
     {"bind", (PyCFunction)(void (*)(void))entry<bind, false>, METH_FASTCALL, nullptr},
-    METHOD(prefill), METHOD(score_sum), METHOD(decode), METHOD(check_qkv), METHOD(cache_write), METHOD(cache_write_first), METHOD(cache_update), METHOD(cache_decode_step),
+    METHOD(prefill), METHOD(score_sum), METHOD(decode), METHOD(check_qkv), METHOD(cache_write), METHOD(cache_write_first), METHOD(prefill_first), METHOD(cache_update), METHOD(cache_decode_step),
     METHOD(quantize_blocks), METHOD(dequantize_blocks), METHOD(dequantize_rows), METHOD(rmsnorm), METHOD(add_rmsnorm),
     METHOD(swiglu), METHOD(qk_norm_rope), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host", "Native host path of the kernels (see csrc/host.cpp).", -1, methods};

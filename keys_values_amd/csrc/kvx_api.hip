@@ -313,14 +313,29 @@ int kvx_cache_write(const kvx_cache_write_args* a, void* stream) {
   return rc != KVX_OK ? rc : launch_cache_write(*a, nullptr, (hipStream_t)stream);
 }
 
-int kvx_cache_write_first(const kvx_cache_write_args* a, void* stream) {
+static int check_cache_write_first(const kvx_cache_write_args* a, const char* who) {
   const int rc = check_cache_write(a);
   if (rc != KVX_OK) return rc;
-  KVX_REQUIRE(a->input_pos == 0 && a->grace_num == 0 && !a->replay_log, KVX_ERR_INVALID, "kvx_cache_write_first: a first chunk begins at position 0, without a ring and a log");
+  KVX_REQUIRE(a->input_pos == 0 && a->grace_num == 0 && !a->replay_log, KVX_ERR_INVALID, "%s: a first chunk begins at position 0, without a ring and a log", who);
   const int64_t slots = (int64_t)a->B * a->Hkv * a->cache_len, workgroups = cache_write_workgroups(*a, true);  // 32-bit indexes of slots, and of threads
-  KVX_REQUIRE(slots < (1ll << 31) && workgroups < (1ll << 24), KVX_ERR_UNSUPPORTED,
-              "kvx_cache_write_first: %lld slots in %lld workgroups, must be below 2^31 and 2^24", (long long)slots, (long long)workgroups);
-  return launch_cache_write(*a, nullptr, (hipStream_t)stream, true);
+  KVX_REQUIRE(slots < (1ll << 31) && workgroups < (1ll << 24), KVX_ERR_UNSUPPORTED, "%s: %lld slots in %lld workgroups, must be below 2^31 and 2^24", who, (long long)slots,
+              (long long)workgroups);
+  return KVX_OK;
+}
+
+int kvx_cache_write_first(const kvx_cache_write_args* a, void* stream) {
+  const int rc = check_cache_write_first(a, "kvx_cache_write_first");
+  return rc != KVX_OK ? rc : launch_cache_write(*a, nullptr, (hipStream_t)stream, true);
+}
+
+int kvx_sdpa_prefill_first(const kvx_sdpa_args* a, const kvx_cache_write_args* w, void* stream) {
+  const char* who = "kvx_sdpa_prefill_first";
+  int rc = check_sdpa_common(a, who, true);
+  if (rc != KVX_OK) return rc;
+  KVX_REQUIRE(a->q_len <= a->kv_len, KVX_ERR_INVALID, "%s: q_len=%d exceeds kv_len=%d", who, a->q_len, a->kv_len);
+  KVX_REQUIRE(aligned16(a->workspace), KVX_ERR_WORKSPACE, "%s: workspace must be 16-byte aligned", who);
+  rc = check_cache_write_first(w, who);
+  return rc != KVX_OK ? rc : launch_sdpa_prefill(*a, false, (hipStream_t)stream, nullptr, w);
 }
 
 size_t kvx_h2o_workspace_bytes(const kvx_h2o_args* a) { return a ? h2o_workspace(*a) : 0; }

@@ -48,7 +48,8 @@ int hip_error(hipError_t e, const char* what);
 struct MergeParams;  // prefill_merge.h
 // may_copy: a quantised store may be dequantised into the workspace first; no field behind workspace_bytes is read.
 // `rest` not NULL: the KV splits' partials are left in the workspace, described in *rest, for launch_score_sum to combine
-int launch_sdpa_prefill(const kvx_sdpa_args& a, bool may_copy, hipStream_t st, MergeParams* rest = nullptr);
+// `first`: the slot write of the first chunk that the call attends over (checked), ahead of it or in the same launch
+int launch_sdpa_prefill(const kvx_sdpa_args& a, bool may_copy, hipStream_t st, MergeParams* rest = nullptr, const kvx_cache_write_args* first = nullptr);
 // whether launch_score_sum takes a kernel whose launch combines the attention's partials whatever the splits
 bool score_sum_combines(const kvx_sdpa_args& a);
 // whether the launches of the tiled kernel combine these partials (splits, teams and rows of m), in less time than a launch of their own would take. `room`: the

@@ -27,6 +27,7 @@
 #include <utility>
 
 #include "prefill_params.h"
+#include "row_write.h"
 
 namespace kvx {
 namespace {
@@ -286,8 +287,20 @@ __device__ __forceinline__ void causal_job(const PrefillParams& p, int job, int&
 // workgroup's barrier each waits for the other at every tile (4096 rows of 128, 8 x 32768 keys 515 us; two workgroups 483 and the merge). A
 // wavefront arrives at its team's barrier, a word in LDS, with the last quarter of the second product still to issue and looks for the others
 // behind it: 483 -> 477, 8 x 16384 scattered keys 272 -> 266 (two workgroups and the merge 277).
-template <int D, int KV, bool PERIODS, bool PAIR>
-__global__ __launch_bounds__(64 * nwaves(KV, D) * (PAIR ? 2 : 1), (kv_is_plain(KV) && D <= 128) ? 2 : 1) void sdpa_prefill_kernel(const PrefillParams p) {
+// WRITE: a first chunk whose rows the launch also writes to their slots. Each workgroup (of a row's splits the first) does so ahead of its own work for the
+// tokens whose first rows it has, and clears its share of the slots behind the chunk's. The write's loads and quantisation run under
+// the products of the unit's other workgroup. As a launch of its own the write of 8192 x 8 rows took 14.5 us before an attention of 503. (Behind its own
+// work the same code made the compiler order the exponentials worse: 512 -> 544 us.)
+struct NoWrite {};
+struct FirstWrite {
+  kvx_cache_write_args a;
+  uint32_t rest;  // slots behind the chunk's, of a row
+};
+
+template <int D, int KV, bool PERIODS, bool PAIR, bool WRITE = false>
+__global__ __launch_bounds__(64 * nwaves(KV, D) * (PAIR ? 2 : 1), (kv_is_plain(KV) && D <= 128) ? 2 : 1) void sdpa_prefill_kernel(const PrefillParams p,
+                                                                                                                                                               const std::conditional_t<WRITE, FirstWrite, NoWrite> wr) {
+  static_assert(!WRITE || (kv_is_plain(KV) && !PAIR && nwaves(KV, D) * 64 == NTHREADS), "a first chunk's own rows");
   static_assert(!PAIR || (pairs(KV, D) && !PERIODS), "two teams fit a compute unit");
   constexpr bool F16 = kv_elem_f16(KV);  // element type of q, k, v, o
   constexpr int BM = 32 * nwaves(KV, D);  // rows per workgroup
@@ -321,6 +334,28 @@ __global__ __launch_bounds__(64 * nwaves(KV, D) * (PAIR ? 2 : 1), (kv_is_plain(K
   const int g = rowc % p.G;
   const int qpos = p.input_pos + qi;
   const int qpos_min_w = p.input_pos + min(row0w, p.R - 1) / p.G;
+
+  if constexpr (WRITE) {
+    if (split == 0) {
+      const kvx_cache_write_args& a = wr.a;
+      const int t0 = (mblk * BM + p.G - 1) / p.G, t1 = min((mblk * BM + BM + p.G - 1) / p.G, p.q_len);
+      switch (a.kv_dtype) {
+        case KVX_KV_BF16:
+        case KVX_KV_F16: write_tokens<D, KV>(a, b, kvh, t0, t1); break;
+        case KVX_KV_U8:
+        case KVX_KV_U8_F16: write_tokens<D, F16 ? KVX_KV_U8_F16 : KVX_KV_U8>(a, b, kvh, t0, t1); break;
+        default: write_tokens<D, F16 ? KVX_KV_U4_F16 : KVX_KV_U4>(a, b, kvh, t0, t1);
+      }
+      const uint32_t total = (uint32_t)(a.B * a.Hkv) * wr.rest, step = (uint32_t)(p.B * p.Hkv * p.m_blocks) * NTHREADS;  // (below 2^31 both: checked by the host)
+      for (uint32_t at = (uint32_t)(mblk * p.B * p.Hkv + group) * NTHREADS + threadIdx.x; at < total; at += step) {
+        const uint32_t row = at / wr.rest;
+        const int64_t to = row / a.Hkv * a.sc_stride_b + row % a.Hkv * a.sc_stride_h + a.num + (at - row * wr.rest);
+        if (a.scores) a.scores[to] = 0.0f;
+        if (a.v_norm) a.v_norm[to] = 0.0f;
+        if (a.q_errors) a.q_errors[to] = 0.0f;
+      }
+    }
+  }
 
   // Q fragments (B operand): lane holds row n, d = 16 j + 8 h .. +8
   u32x4_t qf[KS];
@@ -897,7 +932,7 @@ MergeParams merge_params(const PrefillParams& p) {
 
 // `rest`: where the score-sum launch of `a` follows, what is left for it to combine (num_splits 1: nothing). `combined`: its kernel takes any splits
 template <int D, int KV>
-int launch_t(PrefillParams& p, const kvx_sdpa_args& a, hipStream_t st, MergeParams* rest, bool combined) {
+int launch_t(PrefillParams& p, const kvx_sdpa_args& a, hipStream_t st, MergeParams* rest, bool combined, const FirstWrite* write) {
   if (p.columns) {
     const int rc = launch_sdpa_rows(p, D, KV, st);
     if (rc != KVX_OK) return rc;
@@ -915,16 +950,20 @@ int launch_t(PrefillParams& p, const kvx_sdpa_args& a, hipStream_t st, MergePara
     }
     bool general = true;
     if constexpr (kv_is_plain(KV)) {
-      general = p.period == 0;
-      if (!general) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, true, false>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
+      general = p.period == 0 && !write;
+      if constexpr (D <= 128) {
+        if (write && p.period) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, true, false, true>), grid, dim3(64 * nwaves(KV, D)), 0, st, p, *write);
+        if (write && !p.period) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, false, false, true>), grid, dim3(64 * nwaves(KV, D)), 0, st, p, *write);
+      }
+      if (p.period && !write) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, true, false>), grid, dim3(64 * nwaves(KV, D)), 0, st, p, NoWrite{});
     }
     if constexpr (pairs(KV, D)) {
       if (p.pair) {
         general = false;
-        hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, false, true>), grid, dim3(2 * 64 * nwaves(KV, D)), 0, st, p);
+        hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, false, true>), grid, dim3(2 * 64 * nwaves(KV, D)), 0, st, p, NoWrite{});
       }
     }
-    if (general) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, false, false>), grid, dim3(64 * nwaves(KV, D)), 0, st, p);
+    if (general) hipLaunchKernelGGL((sdpa_prefill_kernel<D, KV, false, false>), grid, dim3(64 * nwaves(KV, D)), 0, st, p, NoWrite{});
     KVX_HIP(hipGetLastError());
   }
   const MergeParams m = merge_params(p);
@@ -1068,7 +1107,18 @@ size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy) {
   return std::max({own, sums, a.w ? rows_weights_workspace(a) : 0});  // (max on the host is one of ints)
 }
 
-int launch_sdpa_prefill(const kvx_sdpa_args& a_in, bool may_copy, hipStream_t st, MergeParams* rest) {
+// Whether the attention launch of a first chunk writes the chunk's rows too: the tiled kernel, for one team, over the rows that are written, where its workgroups
+// have few tokens each (64 of two heads, 128 of one, begin so late that the longest ends later) and are few: a write on its own runs at the memory's
+// rate where it is long. us, two launches -> one: 253 tokens of 2 x 32 heads over 4 19.2 -> 14.7, 343 of 32 over 4 19.2 -> 16.6, 1163 of 32 over 8 35.7 -> 33.5,
+// 2109 of 28 over 4 57.1 -> 55.5, 566 of 64 values, 2 x 16 heads over 8 16.7 -> 14.6; but 1967 of 16 over 8 45.4 -> 46.8, 4214 of 32 over 8 166.1 -> 166.6, 8192
+// 517 -> 518.
+static bool writes_first(const kvx_sdpa_args& a, const PrefillParams& p, const kvx_cache_write_args& w) {
+  return a.D <= 128 && kv_is_plain(a.kv_dtype) && !p.columns && !p.pair && !a.token_positions && a.input_pos == 0 && a.q_len == a.kv_len && w.B == a.B && w.Hkv == a.Hkv &&
+         w.num == a.q_len && w.D == a.D && kv_elem_f16(w.kv_dtype) == kv_elem_f16(a.kv_dtype) && (int64_t)p.B * p.Hkv * p.m_blocks <= 4 * num_cus() &&
+         (p.G > 2 || a.q_len <= 1024);
+}
+
+int launch_sdpa_prefill(const kvx_sdpa_args& a_in, bool may_copy, hipStream_t st, MergeParams* rest, const kvx_cache_write_args* first) {
   PrefillParams p;
   kvx_sdpa_args a = prefill_block(a_in);
   const bool combined = rest && score_sum_combines(a_in);
@@ -1094,8 +1144,19 @@ int launch_sdpa_prefill(const kvx_sdpa_args& a_in, bool may_copy, hipStream_t st
     p.part_o = (float*)a.workspace;
     p.part_ml = p.part_o + rows * (size_t)a.D;
   }
+  FirstWrite fused;
+  const FirstWrite* write = nullptr;
+  if (first) {
+    if (writes_first(a, p, *first)) {
+      fused = {*first, (uint32_t)(first->cache_len - first->num)};
+      write = &fused;
+    } else {
+      const int rc = launch_cache_write(*first, nullptr, st, first->cache_len > first->num);
+      if (rc != KVX_OK) return rc;
+    }
+  }
 #define KVX_PREFILL_CASE(KV) \
-  case KV: return a.D == 256 ? launch_t<256, KV>(p, a_in, st, rest, combined) : a.D == 128 ? launch_t<128, KV>(p, a_in, st, rest, combined) : launch_t<64, KV>(p, a_in, st, rest, combined);
+  case KV: return a.D == 256 ? launch_t<256, KV>(p, a_in, st, rest, combined, write) : a.D == 128 ? launch_t<128, KV>(p, a_in, st, rest, combined, write) : launch_t<64, KV>(p, a_in, st, rest, combined, write);
   if (a.D == 256 || a.D == 128 || a.D == 64) {
     switch (a.kv_dtype) {
       KVX_PREFILL_CASE(KVX_KV_BF16)

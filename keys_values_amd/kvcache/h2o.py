@@ -648,14 +648,15 @@ class H2OKVCache:
         self.batch_size = b
         index = self._run_of_slots(0, num)
         self.current_length = num
-        if b == self.max_batch_size and not self.blocks_over_heads and num == self.cache_length:  # every slot is written
-            self._write(index, key, value, 0)
-        elif b == self.max_batch_size and not self.blocks_over_heads and self.scores.numel() < 2**26:  # (more slots: more threads than a launch counts)
-            _lib.host().cache_write_first(self, index, key, value)  # the slots behind the chunk become zero in the same launch
+        out = None
+        if b == self.max_batch_size and not self.blocks_over_heads and self.scores.numel() < 2**26:  # (more slots: more threads than a launch counts)
+            # rows, zeros in the slots behind the chunk, and attention
+            out = _lib.host().prefill_first(self, index, query, key, value, self.scale_factor)
         else:  # rows that the chunk does not write, or errors that are written elsewhere
-            for t in (self.scores, self.v_norm, self.q_errors):
-                if t is not None:
-                    t.zero_()
+            if b < self.max_batch_size or self.blocks_over_heads or num < self.cache_length:
+                for t in (self.scores, self.v_norm, self.q_errors):
+                    if t is not None:
+                        t.zero_()
             self._write(index, key, value, 0)
         if self.blocks_over_heads:
             self._block_errors(index, None, key, value)
@@ -666,8 +667,9 @@ class H2OKVCache:
         self._use_initial_rule = num == self.cache_length
         self._have_next = False
         self._input_pos = num
-        out, _, _ = ops.prefill_core(query, key.to(self.dtype), value.to(self.dtype), self.scale_factor, 0, None,
-                                     return_weights=False, output_transposed=True)
+        if out is None:
+            out, _, _ = ops.prefill_core(query, key.to(self.dtype), value.to(self.dtype), self.scale_factor, 0, None,
+                                         return_weights=False, output_transposed=True)
         return out.view(b, num, hq * d)
 
     def _ring_and_log(self, num: int, input_pos: int):

@@ -1,0 +1,48 @@
+"""The first chunk's rows written by the attention launch (csrc/sdpa_prefill.hip) against the slot write and the attention as two launches: the same bits."""
+import ctypes
+
+import pytest
+import torch
+
+from helpers import randn
+from keys_values_amd import _lib
+from keys_values_amd.kvcache.h2o import KVCacheParams, create_kv_cache
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("name,dtype,B,Hq,Hkv,T,num,D", [
+    ("h2o-default", torch.bfloat16, 1, 32, 8, 300, 253, 128),             # the last block has 20 of 32 tokens
+    ("h2o-vlen-torch-quantized8", torch.float16, 2, 28, 4, 517, 517, 128),  # tokens whose heads lie in two blocks; no slot behind the chunk
+    ("qh2o-vlen-torch-quantized4", torch.bfloat16, 1, 8, 8, 2000, 137, 128),  # 128 tokens a workgroup; many slots to clear
+    ("qh2o-torch-quantized8", torch.bfloat16, 1, 24, 8, 700, 650, 64),    # in splits that end at bounds of blocks
+    ("h2o-torch-quantized4", torch.float16, 2, 32, 4, 1300, 1001, 64),
+    ("h2o-vlen-default", torch.float16, 1, 6, 2, 900, 641, 128),
+    ("qh2o-vlen-torch-quantized8", torch.bfloat16, 1, 16, 8, 1100, 1030, 128),  # two launches
+    ("qh2o-vlen-torch-quantized8", torch.bfloat16, 1, 8, 2, 400, 300, 256),     # likewise
+])
+def test_first_chunk_in_one_launch(kvx, gpu, name, dtype, B, Hq, Hkv, T, num, D):
+    gen = torch.Generator().manual_seed(num)
+    q, k, v = (randn(gen, B, h, num, D, dtype=dtype).to(gpu) for h in (Hq, Hkv, Hkv))
+    k, v = k.transpose(1, 2).contiguous().transpose(1, 2), v  # a token's heads side by side, and rows side by side
+    got = []
+    for one in (True, False):
+        cache = create_kv_cache(name, KVCacheParams(B, Hkv, T, D, Hq, dtype))
+        tensors = [getattr(cache, n, None) for n in ("k", "v", "k_scale", "k_zp", "v_scale", "v_zp", "token_pos", "scores", "v_norm", "q_errors")]
+        tensors = [t for t in tensors if t is not None]
+        for t in tensors:
+            t.fill_(7)
+        if one:
+            out = cache.forward(q, k, v)
+        else:  # what the one launch stands for
+            cache.batch_size = B
+            index = cache._run_of_slots(0, num)
+            _lib.host().cache_write_first(cache, index, k, v) if num < T else cache._write(index, k, v, 0)
+            out = _lib.host().prefill(q, k, v, cache.scale_factor, 0, None, False, False, True, None, 0, False)[0].view(B, num, Hq * D)
+        got.append([out] + tensors)
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+
+
+def test_refusals(kvx):
+    a, w = _lib.SdpaArgs(), _lib.CacheWriteArgs()
+    assert kvx.kvx_sdpa_prefill_first(ctypes.byref(a), ctypes.byref(w), None) != 0  # nothing set
