@@ -379,7 +379,7 @@ __device__ __forceinline__ int list_slot(int c, int lists, int t) { return ((t >
 
 __global__ __launch_bounds__(LIST) void list_norm_kernel(const kvx_h2o_args a, const SelectLists sl) {
   __shared__ float red[LIST / 64];
-  const int c = blockIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
+  const int c = blockIdx.y, row = blockIdx.x, b = row / a.Hkv, hh = row % a.Hkv;
   const int slot = part_slot(c, sl.C, threadIdx.x);
   float x = 0.0f;
   if (slot < a.kv_len) x = a.v_norm[b * a.sc_stride_b + hh * a.sc_stride_h + slot] * a.w[(int64_t)row * a.kv_len + slot];
@@ -452,7 +452,7 @@ __device__ __forceinline__ float updated_score(const kvx_h2o_args& a, const Slot
 // q_errors: the update and the lists' extremes, before anything can be compared
 __global__ __launch_bounds__(LIST) void list_stats_kernel(const kvx_h2o_args a, const SelectLists sl) {
   __shared__ float red[LIST / 64];
-  const int c = blockIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
+  const int c = blockIdx.y, row = blockIdx.x, b = row / a.Hkv, hh = row % a.Hkv;
   const int slot = part_slot(c, sl.C, threadIdx.x);
   const bool in = slot < a.limit;
   const float qe = in ? a.q_errors[b * a.sc_stride_b + hh * a.sc_stride_h + slot] : 0.0f;
@@ -513,7 +513,7 @@ template <int L>
 __global__ __launch_bounds__(L, 8) void list_sort_kernel(const kvx_h2o_args a, const SelectLists sl) {
   __shared__ float red[L / 64];
   __shared__ unsigned long long buf[2][L];
-  const int tid = threadIdx.x, c = blockIdx.x, row = blockIdx.y, b = row / a.Hkv, hh = row % a.Hkv;
+  const int tid = threadIdx.x, c = blockIdx.y, row = blockIdx.x, b = row / a.Hkv, hh = row % a.Hkv;
   const int slot = list_slot(c, sl.lists, tid);
   const bool in = slot < a.limit;
   unsigned long long x = ~0ull;
@@ -565,7 +565,7 @@ __global__ __launch_bounds__(RANK_THREADS) void list_rank_kernel(const unsigned 
   __shared__ unsigned long long head[RANK_STAGED];
   __shared__ uint32_t rank[L];
   __shared__ unsigned long long wmax[RANK_THREADS / 64];
-  const int tid = threadIdx.x, c = blockIdx.x, row = blockIdx.y, S = 1 << staged;
+  const int tid = threadIdx.x, c = blockIdx.y, row = blockIdx.x, S = 1 << staged;
   const unsigned long long* base = lists + (int64_t)row * C * L;
   for (int i = tid; i < C << staged; i += RANK_THREADS) head[i] = base[(i >> staged) * L + (i & (S - 1))];
   unsigned long long u = 0ull;
@@ -898,7 +898,7 @@ size_t h2o_workspace(const kvx_h2o_args& a) {
 
 template <int L>
 static void launch_sorted(const kvx_h2o_args& a, const SelectLists& sl, hipStream_t st) {
-  const dim3 grid(sl.lists, a.B * a.Hkv);
+  const dim3 grid(a.B * a.Hkv, sl.lists);
   hipLaunchKernelGGL(list_sort_kernel<L>, grid, dim3(L), 0, st, a, sl);
   if (sl.lists == 1) return;
   const int per = (a.k + sl.lists - 1) / sl.lists;
@@ -916,7 +916,8 @@ static int launch_lists(const kvx_h2o_args& a, const ListPlan& p, hipStream_t st
   sl.stats = (float*)(ws + p.off_stats);
   sl.C = p.C;
   sl.lists = p.lists;
-  const dim3 grid(p.C, a.B * a.Hkv);
+  // rows fastest: a row's workgroups, of every launch, are on the die (of eight, which take workgroups in turn) whose L2 the one before has written
+  const dim3 grid(a.B * a.Hkv, p.C);
   if (a.w && a.v_norm && sl.part_z) hipLaunchKernelGGL(list_norm_kernel, grid, dim3(LIST), 0, st, a, sl);
   if (a.q_errors) hipLaunchKernelGGL(list_stats_kernel, grid, dim3(LIST), 0, st, a, sl);
   if (p.L == 256) launch_sorted<256>(a, sl, st);

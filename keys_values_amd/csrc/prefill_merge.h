@@ -30,12 +30,16 @@ inline bool merge_wants_classes(const MergeParams& p, int D) {
   return p.num_splits > 4 && (int64_t)p.B * p.Hkv * p.R * (D / 4) < (int64_t)num_cus() * 256;
 }
 // Where a (batch, KV head) pair has many blocks of rows, they go round the pairs: pair g's on the die (of eight, which take workgroups in turn) whose
-// L2 cache the attention kernel's workgroups of g have written (294 rows over 16 x 1996 keys of 128, no weights: 21.7 -> 19.0 us a call).
-__host__ __device__ inline bool merge_by_pair(const MergeParams& p, int rows) { return p.R >= 8 * rows; }
+// L2 cache the attention kernel's workgroups of g have written. Rows in order -> round the pairs, calls without weights, us: 294 rows over 16 x 1996 keys of 128
+// 21.7 -> 19.0, 214 of 256 over 8 x 1127 25.4 -> 20.6, 1716 of 64 over 8 x 1800 19.5 -> 17.6. Partials that do not fit the dies' 8 x 4 MB come from memory, in
+// order the faster: 1597 tokens of 16 heads of 256 over 8 58.7, round the pairs 59.7.
+__host__ __device__ inline bool merge_by_pair(const MergeParams& p, int D, int rows) {
+  return p.R >= 8 * rows && (int64_t)p.num_splits * p.B * p.Hkv * p.R * D <= (8 << 20);
+}
 inline int64_t merge_blocks(const MergeParams& p, int D, int SC) {
   const int rows = merge_rows(D, SC);
   const int64_t pairs = (int64_t)p.B * p.Hkv;
-  return merge_by_pair(p, rows) ? pairs * ((p.R + rows - 1) / rows) : (pairs * p.R + rows - 1) / rows;
+  return merge_by_pair(p, D, rows) ? pairs * ((p.R + rows - 1) / rows) : (pairs * p.R + rows - 1) / rows;
 }
 template <int D, bool F16, int SC, int TEAMS>
 __device__ __forceinline__ void merge_rows_job(const MergeParams& p, const int64_t block, const int tid, f32x4_t* red_o, float* red_l) {
@@ -45,7 +49,7 @@ __device__ __forceinline__ void merge_rows_job(const MergeParams& p, const int64
   const int64_t total_rows = (int64_t)p.B * p.Hkv * p.R;
   int64_t grow = block * ROWS + tid / (TPR * SC);
   bool live = grow < total_rows;
-  if (merge_by_pair(p, ROWS)) {
+  if (merge_by_pair(p, D, ROWS)) {
     const uint32_t pairs = (uint32_t)(p.B * p.Hkv), at = (uint32_t)block / pairs;
     const int row = (int)at * ROWS + tid / (TPR * SC);
     live = row < p.R;

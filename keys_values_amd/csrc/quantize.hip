@@ -175,15 +175,16 @@ __global__ __launch_bounds__(NTHREADS) void dequantize_kv_kernel(const kvx_sdpa_
   constexpr int LPR = U4 ? D / 16 : D / 8;  // lanes per row: 8 bytes of codes each
   constexpr int RPB = NTHREADS / LPR;
   const bool is_v = blockIdx.z != 0;
-  const int b = blockIdx.y / a.Hkv, h = blockIdx.y % a.Hkv;
+  const uint32_t pairs = a.B * a.Hkv, at = blockIdx.x / pairs, pair = blockIdx.x - at * pairs;  // pairs fastest: on the die whose workgroups will read its rows
+  const int b = (int)pair / a.Hkv, h = (int)pair % a.Hkv;
   const int64_t sb = is_v ? a.v_stride_b : a.k_stride_b, sh = is_v ? a.v_stride_h : a.k_stride_h, stt = is_v ? a.v_stride_t : a.k_stride_t;
   const uint8_t* __restrict__ codes = (const uint8_t*)(is_v ? a.v : a.k) + b * sb + h * sh;
   const int64_t so = b * a.qs_stride_b + h * a.qs_stride_h;
   const float* __restrict__ scale = (is_v ? a.v_scale : a.k_scale) + so;
   const int32_t* __restrict__ zp = (is_v ? a.v_zp : a.k_zp) + so;
-  uint16_t* __restrict__ o = out + ((int64_t)blockIdx.z * a.B * a.Hkv + blockIdx.y) * a.kv_len * D;
+  uint16_t* __restrict__ o = out + ((int64_t)blockIdx.z * pairs + pair) * a.kv_len * D;
   const int col = threadIdx.x % LPR;
-  const int row0 = blockIdx.x * (RPB * ROWS_PER_THREAD) + threadIdx.x / LPR;
+  const int row0 = (int)at * (RPB * ROWS_PER_THREAD) + threadIdx.x / LPR;
   u32x2_t c[ROWS_PER_THREAD];
   float s[ROWS_PER_THREAD];
   int32_t z[ROWS_PER_THREAD];
@@ -498,7 +499,9 @@ int launch_dequantize_rows(const uint8_t* codes, const float* scale, const int32
 template <int D>
 int launch_dequantize_kv_d(const kvx_sdpa_args& a, void* out, hipStream_t st) {
   const int lpr = kv_is_u4(a.kv_dtype) ? D / 16 : D / 8, rpb = NTHREADS / lpr * ROWS_PER_THREAD;
-  const dim3 grid((a.kv_len + rpb - 1) / rpb, a.B * a.Hkv, 2);
+  const int64_t blocks = (int64_t)((a.kv_len + rpb - 1) / rpb) * a.B * a.Hkv;
+  KVX_REQUIRE(blocks < (1ll << 31), KVX_ERR_UNSUPPORTED, "dequantised copy: %lld blocks of rows", (long long)blocks);
+  const dim3 grid((unsigned)blocks, 1, 2);
   switch (a.kv_dtype) {
     case KVX_KV_U8: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U8>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out); break;
     case KVX_KV_U4: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U4>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out); break;

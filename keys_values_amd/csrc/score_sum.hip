@@ -831,13 +831,15 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void score_sum_stream_kernel
 // What a split of the query rows leaves behind, in one launch: the first merge_jobs workgroups combine the attention's KV splits, the others add the
 // splits' sums, W = (1/G) * (part[0] + part[1] + ...), in that order.
 template <int D, bool F16>
-__global__ __launch_bounds__(256) void score_sum_finish_kernel(const MergeParams m, const int merge_jobs, const float* part, float* w, int64_t n, int splits, float inv_g) {
+__global__ __launch_bounds__(256) void score_sum_finish_kernel(const MergeParams m, const int merge_jobs, const float* part, float* w, int pairs, int kv_len, int splits, float inv_g) {
   if ((int)blockIdx.x < merge_jobs) {
     merge_job<D, F16, 1>(m, blockIdx.x, threadIdx.x);
     return;
   }
-  const int64_t i = (int64_t)((int)blockIdx.x - merge_jobs) * 256 + threadIdx.x;
-  if (i >= n) return;
+  // pairs fastest: on the die whose L2 has the pair's sums
+  const uint32_t job = blockIdx.x - merge_jobs, at = job / (uint32_t)pairs, key = at * 256 + threadIdx.x;
+  if (key >= (uint32_t)kv_len) return;
+  const int64_t n = (int64_t)pairs * kv_len, i = (int64_t)(job - at * pairs) * kv_len + key;
   float acc = part[i];
   for (int z = 1; z < splits; ++z) acc += part[(int64_t)z * n + i];
   w[i] = acc * inv_g;
@@ -950,8 +952,9 @@ int launch_t(const ScoreParams& p, int splits, int waves, const MergeParams* res
   if (splits > 1) {
     tiled_any(std::integral_constant<int, 4>{}, std::true_type{});
     KVX_HIP(hipGetLastError());
-    const int64_t n = (int64_t)groups * p.kv_len;
-    hipLaunchKernelGGL((score_sum_finish_kernel<D, kv_elem_f16(KV)>), dim3((unsigned)(jobs + (n + 255) / 256)), dim3(256), 0, st, m, (int)jobs, p.part, p.w, n, splits, p.inv_g);
+    const int64_t sums = (int64_t)groups * ((p.kv_len + 255) / 256);
+    hipLaunchKernelGGL((score_sum_finish_kernel<D, kv_elem_f16(KV)>), dim3((unsigned)(jobs + sums)), dim3(256), 0, st, m, (int)jobs, p.part, p.w, groups, p.kv_len, splits,
+                       p.inv_g);
   } else {
     bool wide = false;
     if constexpr (D <= 128) wide = waves == 8;
