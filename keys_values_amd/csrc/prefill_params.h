@@ -35,8 +35,8 @@ struct RowsPlan {
   int columns, splits;
   int64_t ns;
 };
-// `combined`: the score-sum launch that follows combines the splits. `before_halves`: also where the tiled kernel with half of its wavefronts takes the call
-RowsPlan rows_plan(const kvx_sdpa_args& a, bool combined, bool before_halves = false);
+// `combined`: the score-sum launch that follows combines the splits
+RowsPlan rows_plan(const kvx_sdpa_args& a, bool combined);
 int launch_sdpa_rows(const PrefillParams& p, int D, int kv, hipStream_t st);
 void common_params(PrefillParams& p, const kvx_sdpa_args& a);
 int64_t prefill_ns(const kvx_sdpa_args& a);  // estimate of a call's attention launch where a score-sum launch follows

@@ -815,7 +815,6 @@ Splits pick_splits(const kvx_sdpa_args& a, int m_blocks, int num_tiles) {
   const bool plain = kv_is_plain(a.kv_dtype);
   int64_t tile_ns = a.D == 64 ? 840 : a.D == 128 ? 1130 : 2050;
   if (!plain) tile_ns = a.D == 256 ? 5500 : a.D == 64 ? 1700 : 2560;  // 256 rows a workgroup, codes to dequantise (at 256: 128 rows)
-  if (!plain && a.D <= 128 && a.q_len * (a.Hq / a.Hkv) <= 128) tile_ns = a.D == 64 ? 1150 : 1850;  // half of the wavefronts have rows
   const bool two = pairs(a.kv_dtype, a.D);
   const int64_t rows = (int64_t)a.B * a.Hq * a.q_len;
   Splits best = {1, false, INT64_MAX};
@@ -1063,7 +1062,7 @@ static kvx_sdpa_args on_copy(const kvx_sdpa_args& a, void* rows) {
 }
 
 int64_t prefill_ns(const kvx_sdpa_args& a) {
-  const RowsPlan rows = rows_plan(a, score_sum_combines(a), true);  // one launch against two was measured with these estimates
+  const RowsPlan rows = rows_plan(a, score_sum_combines(a));
   const int bm = 32 * nwaves(a.kv_dtype, a.D);
   return rows.columns ? rows.ns : pick_splits(a, (int)(((int64_t)a.q_len * (a.Hq / a.Hkv) + bm - 1) / bm), (a.kv_len + BN - 1) / BN).ns;
 }

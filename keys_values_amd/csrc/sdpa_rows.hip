@@ -700,21 +700,17 @@ RowsPlan plan_of(const kvx_sdpa_args& a, int columns, bool combined) {
 //   plain, 64      8 a unit  512 rows 22.4 -> 22.3, 1000 rows 27.6 -> 27.0
 //   codes, 128     6 a unit  300 rows 39.2 -> 37.8 (4-bit: 35.2), 512 rows (4) 41.1 -> 36.5;  7: 600 rows .88, 12: 96 rows .95
 //   codes, 64      8-bit 10 a unit, 4-bit 7: 1000 rows (8) 33.8 -> 30.3, 300 rows (8) 31.1 -> 29.1;  4-bit 512 rows (7.5) .98
-// At most 16 plain rows win while the keys stay in the last-level cache, 128 Ki of them (8 x 8192 20.3 -> 16.1, 32 x 36928 .98).
-// Over codes the tiled kernel takes up to 128 rows with half of its wavefronts bringing tiles only, and wins over more than 1024 keys, from 33 rows of 128
-// values on (with 32 KV heads or more both win some of the calls of 33 to 64 rows: the line is at 65) or 65 of 64. here -> tiled: 128, 8-bit: 48 rows over 8 x 2000 12.2 -> 11.5, 64 over 8 x 30000 38.1 -> 33.1, 64 over 16 x 5500 21.8 -> 19.0, 112 over 32 x 1500
-// 20.8 -> 16.7; 4-bit: 48 over 8 x 9000 19.5 -> 16.4, 40 over 32 x 12000 58.0 -> 47.4, but 60 over 32 x 2500 18.6 -> 19.5; 64: 80 over 8 x 12000 18.4 -> 14.9, 120 over 8 x 5000 13.6 -> 12.6, but
-// 64 over 32 x 36000 66 -> 82. Up to 1024 keys the splits' own launch costs more: 112 over 8 x 256 8.8 -> 11.1, 128 of 64 over 32 x 1000 10.5 -> 11.8; of 64 the more so the more
-// heads there are: 120 over 64 x 1100 13.8 -> 16.2, 68 over 32 x 1100 12.2 -> 12.8, 80 over 64 x 2000 the same.
-// Rows of 256: the accumulators of plain keys' pipeline do not fit, over codes the tiled kernel is so slow that up to 128 rows win (128 over
-// 4 x 15000 64 -> 50); above, a long call goes over a copy of the store in 16-bit rows.
+// At most 16 plain rows win while the keys stay in the last-level cache, 128 Ki of them (8 x 8192 20.3 -> 16.1, 32 x 36928 .98); at
+// most 64 rows over codes always (64 over 8 x 30000 65 -> 62, 64 of 64 over 8 x 60000 65 -> 51). Rows of 256: the accumulators of plain
+// keys' pipeline do not fit, over codes the tiled kernel is so slow that up to 128 rows win (128 over 4 x 15000 64 -> 50); above, a long call
+// goes over a copy of the store in 16-bit rows.
 // Many short workgroups stay there too (plan_of): one begins and ends with more than a step's work, so
 // where the device takes the workgroups in turns and each has up to three steps of 128 keys (over codes two, of 256 four) the tiled
 // kernel's few win: 133 rows over 256 x 64 plain keys of 128 9.4 there, 25.5 here; 279 over 64 x 254 12.2, 22.7; 198 over 64 x 219 12.1, 15.8;
 // 312 over 64 x 121 8-bit keys 13.8, 19.2; 66 of 256 over 128 x 512 8-bit keys 47.8, 53.8; but with four steps both take the same, and over codes three win by
 // 1.1 to 2.2 here. Over at most a tile of keys more workgroups than units are too many, half of that at 32 rows: 35 over
 // 128 x 64 5.2, 6.2.
-RowsPlan rows_plan(const kvx_sdpa_args& a, bool combined, bool before_halves) {
+RowsPlan rows_plan(const kvx_sdpa_args& a, bool combined) {
   const RowsPlan none = {0, 0, 0};
   const bool plain = kv_is_plain(a.kv_dtype);
   const int64_t rows = (int64_t)a.q_len * (a.Hq / a.Hkv), keys = (int64_t)a.B * a.Hkv * a.kv_len, es = plain ? 2 : 1;
@@ -723,11 +719,7 @@ RowsPlan rows_plan(const kvx_sdpa_args& a, bool combined, bool before_halves) {
   if (plain) {
     if (a.D == 256 || !((rows <= 16 && keys <= 128 * 1024) || work <= (a.D == 64 ? 8 : 5) * num_cus())) return none;
   } else {
-    const int64_t most = a.D == 64 ? (kv_is_u4(a.kv_dtype) ? 7 : 10) : a.D == 128 ? 6 : 8;
-    const int64_t groups = (int64_t)a.B * a.Hkv;
-    const bool half = !before_halves && a.kv_len > 1024 && rows <= 128 &&
-                      (a.D == 128 ? rows > (groups < 32 ? 32 : 64) : a.D == 64 && rows > 64 && a.kv_len > 48 * groups);
-    if (half || (a.D == 256 && rows > 128) || (rows > 64 && work > most * num_cus())) return none;
+    if ((a.D == 256 && rows > 128) || (rows > 64 && work > (a.D == 64 ? (kv_is_u4(a.kv_dtype) ? 7 : 10) : a.D == 128 ? 6 : 8) * num_cus())) return none;
   }
   const RowsPlan one = plan_of(a, 16, combined);
   if (rows <= 16) return one;

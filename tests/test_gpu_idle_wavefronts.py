@@ -16,11 +16,11 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype,bits,B,Hq,Hkv,q_len,T,D,where,block,teams", [
-    (torch.bfloat16, 8, 1, 32, 8, 32, 2049, 128, "scattered", 256, 1),  # 128 rows: four of eight wavefronts; a last tile of one key
-    (torch.float16, 4, 1, 28, 4, 15, 1100, 128, "end", 256, 1),         # 105 rows
-    (torch.bfloat16, 8, 2, 8, 8, 33, 1090, 128, "start", 256, 1),       # one row in the second wavefront; splits that no row sees
-    (torch.float16, 8, 1, 16, 4, 31, 3000, 64, "end", 256, 1),
-    (torch.bfloat16, 4, 1, 32, 4, 16, 1153, 64, "scattered", 256, 1),
+    (torch.bfloat16, 8, 1, 32, 8, 32, 12801, 128, "scattered", 256, 1),  # 128 rows: four of eight wavefronts; a last tile of one key
+    (torch.float16, 4, 1, 28, 4, 15, 15000, 128, "end", 256, 1),         # 105 rows
+    (torch.bfloat16, 8, 2, 8, 8, 67, 9090, 128, "start", 256, 1),        # three rows in the third wavefront; splits that no row sees
+    (torch.float16, 8, 1, 16, 4, 31, 40000, 64, "end", 256, 1),
+    (torch.bfloat16, 4, 1, 32, 4, 16, 33153, 64, "scattered", 256, 1),
     (torch.bfloat16, 8, 16, 32, 8, 72, 600, 128, "end", 256, 1),        # a whole block of rows ahead of one wavefront's
     (torch.bfloat16, 16, 1, 32, 8, 33, 5000, 128, "scattered", 128, 2), # plain rows, two teams: a block of four rows
     (torch.float16, 16, 1, 8, 2, 1001, 1001, 128, "first", 128, 1),     # a first chunk in splits that end at bounds of blocks
