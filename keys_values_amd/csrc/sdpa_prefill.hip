@@ -1109,11 +1109,11 @@ size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy) {
 // Whether the attention launch of a first chunk writes the chunk's rows too: the tiled kernel, for one team, over the rows that are written, where its workgroups
 // have few tokens each (64 of two heads, 128 of one, begin so late that the longest ends later) and are few: a write on its own runs at the memory's
 // rate where it is long. us, two launches -> one: 253 tokens of 2 x 32 heads over 4 19.2 -> 14.7, 343 of 32 over 4 19.2 -> 16.6, 1163 of 32 over 8 35.7 -> 33.5,
-// 2109 of 28 over 4 57.1 -> 55.5, 566 of 64 values, 2 x 16 heads over 8 16.7 -> 14.6; but 1967 of 16 over 8 45.4 -> 46.8, 4214 of 32 over 8 166.1 -> 166.6, 8192
-// 517 -> 518.
+// 2109 of 28 over 4 57.1 -> 55.5, 566 of 64 values, 2 x 16 heads over 8 16.7 -> 14.6; 1408 of 2 x 32 over 8 53.8 -> 53.1; but 1967 of 16 over 8 45.4 -> 46.8,
+// 4096 of 32 over 8 145.7 -> 146.3, 4214 166.1 -> 166.6, 8192 517 -> 518.
 static bool writes_first(const kvx_sdpa_args& a, const PrefillParams& p, const kvx_cache_write_args& w) {
   return a.D <= 128 && kv_is_plain(a.kv_dtype) && !p.columns && !p.pair && !a.token_positions && a.input_pos == 0 && a.q_len == a.kv_len && w.B == a.B && w.Hkv == a.Hkv &&
-         w.num == a.q_len && w.D == a.D && kv_elem_f16(w.kv_dtype) == kv_elem_f16(a.kv_dtype) && (int64_t)p.B * p.Hkv * p.m_blocks <= 4 * num_cus() &&
+         w.num == a.q_len && w.D == a.D && kv_elem_f16(w.kv_dtype) == kv_elem_f16(a.kv_dtype) && (int64_t)p.B * p.Hkv * p.m_blocks <= 3 * num_cus() &&
          (p.G > 2 || a.q_len <= 1024);
 }
 
