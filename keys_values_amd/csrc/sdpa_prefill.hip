@@ -298,8 +298,8 @@ struct FirstWrite {
 };
 
 template <int D, int KV, bool PERIODS, bool PAIR, bool WRITE = false>
-__global__ __launch_bounds__(64 * nwaves(KV, D) * (PAIR ? 2 : 1), (kv_is_plain(KV) && D <= 128) ? 2 : 1) void sdpa_prefill_kernel(const PrefillParams p,
-                                                                                                                                                               const std::conditional_t<WRITE, FirstWrite, NoWrite> wr) {
+__global__ __launch_bounds__(64 * nwaves(KV, D) * (PAIR ? 2 : 1), (kv_is_plain(KV) && D <= 128) ? 2 : 1) void sdpa_prefill_kernel(
+    const PrefillParams p, const std::conditional_t<WRITE, FirstWrite, NoWrite> wr) {
   static_assert(!WRITE || (kv_is_plain(KV) && !PAIR && nwaves(KV, D) * 64 == NTHREADS), "a first chunk's own rows");
   static_assert(!PAIR || (pairs(KV, D) && !PERIODS), "two teams fit a compute unit");
   constexpr bool F16 = kv_elem_f16(KV);  // element type of q, k, v, o
