@@ -167,24 +167,24 @@ __global__ __launch_bounds__(NTHREADS) void dequantize_rows4_kernel(const RowRun
   }
 }
 
-// K (blockIdx.z = 0) and V (1) of an attention call's quantised store, one (batch, KV head) pair per blockIdx.y, to dense
-// rows. A lane owns 8 values of ROWS_PER_THREAD rows, as above; the codes' rows lie wherever the strides say.
+// K (blockIdx.z = 0) and V (1) of an attention call's quantised store to dense rows: a (batch, KV head) pair per blockIdx.y and blocks of its rows along
+// blockIdx.x, or the other way round (by_pair). A lane owns 8 values of ROWS_PER_THREAD rows, as above; the codes' rows lie wherever the strides say.
 template <int D, int KV>
-__global__ __launch_bounds__(NTHREADS) void dequantize_kv_kernel(const kvx_sdpa_args a, uint16_t* __restrict__ out) {
+__global__ __launch_bounds__(NTHREADS) void dequantize_kv_kernel(const kvx_sdpa_args a, uint16_t* __restrict__ out, const bool by_pair) {
   constexpr bool U4 = kv_is_u4(KV), F16 = kv_elem_f16(KV);
   constexpr int LPR = U4 ? D / 16 : D / 8;  // lanes per row: 8 bytes of codes each
   constexpr int RPB = NTHREADS / LPR;
   const bool is_v = blockIdx.z != 0;
-  const uint32_t pairs = a.B * a.Hkv, at = blockIdx.x / pairs, pair = blockIdx.x - at * pairs;  // pairs fastest: on the die whose workgroups will read its rows
-  const int b = (int)pair / a.Hkv, h = (int)pair % a.Hkv;
+  const int pair = by_pair ? blockIdx.x : blockIdx.y, at = by_pair ? blockIdx.y : blockIdx.x;
+  const int b = pair / a.Hkv, h = pair % a.Hkv;
   const int64_t sb = is_v ? a.v_stride_b : a.k_stride_b, sh = is_v ? a.v_stride_h : a.k_stride_h, stt = is_v ? a.v_stride_t : a.k_stride_t;
   const uint8_t* __restrict__ codes = (const uint8_t*)(is_v ? a.v : a.k) + b * sb + h * sh;
   const int64_t so = b * a.qs_stride_b + h * a.qs_stride_h;
   const float* __restrict__ scale = (is_v ? a.v_scale : a.k_scale) + so;
   const int32_t* __restrict__ zp = (is_v ? a.v_zp : a.k_zp) + so;
-  uint16_t* __restrict__ o = out + ((int64_t)blockIdx.z * pairs + pair) * a.kv_len * D;
+  uint16_t* __restrict__ o = out + ((int64_t)blockIdx.z * a.B * a.Hkv + pair) * a.kv_len * D;
   const int col = threadIdx.x % LPR;
-  const int row0 = (int)at * (RPB * ROWS_PER_THREAD) + threadIdx.x / LPR;
+  const int row0 = at * (RPB * ROWS_PER_THREAD) + threadIdx.x / LPR;
   u32x2_t c[ROWS_PER_THREAD];
   float s[ROWS_PER_THREAD];
   int32_t z[ROWS_PER_THREAD];
@@ -496,17 +496,22 @@ int launch_dequantize_rows(const uint8_t* codes, const float* scale, const int32
   return launch_rows(RowRuns{(uint16_t*)out, out_row_stride, 0, (uint8_t*)codes, 0, (float*)scale, (int32_t*)zp, 0, rows, 1}, D, bits, f16, false, st);
 }
 
+// While the 16-bit rows of K and V, 32 MB at 8 M values each, fit the L2 caches of the eight dies, pairs are the fastest index: the rows are written on the die whose
+// attention workgroups read them. Beyond, no reader finds them there, and in the rows' order the writes run the faster. Rows' order against pairs' (us;
+// attention of 512 queries of four heads behind it): calls over 16 x 1500 rows of 128 70.9, 68.3; 16 x 2000 of 64 92.0, 88.6; 8 x 5000 and 8 x 7000 alike; copies
+// of 8 x 16384 15.8, 16.2; 8 x 32768 31.9, 33.7; 8 x 65536 60.2, 63.6, of 4-bit codes 52.6, 55.4.
+constexpr int64_t COPY_BY_PAIR = 8ll << 20;
 template <int D>
 int launch_dequantize_kv_d(const kvx_sdpa_args& a, void* out, hipStream_t st) {
   const int lpr = kv_is_u4(a.kv_dtype) ? D / 16 : D / 8, rpb = NTHREADS / lpr * ROWS_PER_THREAD;
-  const int64_t blocks = (int64_t)((a.kv_len + rpb - 1) / rpb) * a.B * a.Hkv;
-  KVX_REQUIRE(blocks < (1ll << 31), KVX_ERR_UNSUPPORTED, "dequantised copy: %lld blocks of rows", (long long)blocks);
-  const dim3 grid((unsigned)blocks, 1, 2);
+  const unsigned pairs = (unsigned)(a.B * a.Hkv), blocks = (unsigned)(a.kv_len / rpb + (a.kv_len % rpb != 0));
+  const bool by_pair = (int64_t)pairs * a.kv_len * D <= COPY_BY_PAIR;
+  const dim3 grid(by_pair ? pairs : blocks, by_pair ? blocks : pairs, 2);
   switch (a.kv_dtype) {
-    case KVX_KV_U8: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U8>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out); break;
-    case KVX_KV_U4: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U4>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out); break;
-    case KVX_KV_U8_F16: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U8_F16>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out); break;
-    default: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U4_F16>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out); break;
+    case KVX_KV_U8: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U8>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out, by_pair); break;
+    case KVX_KV_U4: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U4>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out, by_pair); break;
+    case KVX_KV_U8_F16: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U8_F16>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out, by_pair); break;
+    default: hipLaunchKernelGGL((dequantize_kv_kernel<D, KVX_KV_U4_F16>), grid, dim3(NTHREADS), 0, st, a, (uint16_t*)out, by_pair); break;
   }
   KVX_HIP(hipGetLastError());
   return KVX_OK;
