@@ -505,6 +505,7 @@ template <int D>
 int launch_dequantize_kv_d(const kvx_sdpa_args& a, void* out, hipStream_t st) {
   const int lpr = kv_is_u4(a.kv_dtype) ? D / 16 : D / 8, rpb = NTHREADS / lpr * ROWS_PER_THREAD;
   const unsigned pairs = (unsigned)(a.B * a.Hkv), blocks = (unsigned)(a.kv_len / rpb + (a.kv_len % rpb != 0));
+  KVX_REQUIRE(blocks < (1u << 24), KVX_ERR_UNSUPPORTED, "dequantised copy: %u blocks of rows, must be below 2^24", blocks);  // a dimension's threads are counted in 32 bits
   const bool by_pair = (int64_t)pairs * a.kv_len * D <= COPY_BY_PAIR;
   const dim3 grid(by_pair ? pairs : blocks, by_pair ? blocks : pairs, 2);
   switch (a.kv_dtype) {

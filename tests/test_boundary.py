@@ -386,6 +386,15 @@ def test_weights_refuse_query_rows_of_4_gib(kvx, q_len, kv_len):
             assert call(ctypes.byref(b), None) == _lib.KVX_ERR_UNSUPPORTED
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the pointers are made up: where nothing can be launched")
+def test_copy_of_a_store_is_refused_beyond_the_blocks_of_a_launch(kvx):
+    for kv_len, status in ((2**30 - 64, _lib.KVX_ERR_HIP), (2**30, _lib.KVX_ERR_UNSUPPORTED)):  # 2^24 - 1 workgroups of 64 rows (no device), 2^24
+        a = _prefill_block(1, 16, 1, 128, kv_len, 128, 0)
+        a.kv_dtype, a.k_scale, a.k_zp, a.v_scale, a.v_zp = _lib.KVX_KV_U8, 4096, 4096, 4096, 4096
+        a.workspace, a.workspace_bytes = 4096, 2**50
+        assert kvx.kvx_sdpa_prefill_copying(ctypes.byref(a), None) == status
+
+
 @pytest.mark.parametrize("B,heads,kv_heads,q_len,kv_len,D", [(1, 4, 1, 3, 64, 64), (1, 8, 2, 128, 1024, 64), (1, 16, 4, 128, 1500, 64), (1, 2, 1, 8, 8000, 128)])
 def test_a_chunk_waits_for_a_few_times_its_own_time(kvx, B, heads, kv_heads, q_len, kv_len, D):
     # a poll is 1.5 to 2 us, these calls take 10 to 20; the single-token step waits for 2^15 polls
