@@ -520,17 +520,21 @@ void set_cache_tensors(kvx_cache_write_args& a, PyObject* cache, Held& held) {
     if (auto t = attr_opt_tensor(cache, names.q_errors)) a.q_errors = (float*)held(*t).data_ptr();
 }
 
-at::Tensor rows_of(const at::Tensor& t, at::ScalarType type) {
+// `t` as rows of `type`; `strided`: set where the head dimension is not contiguous in that type and a copy makes it so
+at::Tensor rows_of(const at::Tensor& t, at::ScalarType type, bool& strided) {
   if (t.scalar_type() == type && t.stride(3) == 1) return t;
   return unlocked([&] {
     at::Tensor r = t.to(type);
-    return r.stride(3) == 1 ? r : r.contiguous();
+    if (r.stride(3) == 1) return r;
+    strided = true;
+    return r.contiguous();
   });
 }
 
 struct WriteCall {
   kvx_cache_write_args a{};
   at::Tensor key, value;  // as handed to the kernel
+  bool strided = false;   // copies of rows that lie strided
   Held held;
 };
 // key / value (B, Hkv, num, D) into the slots `index` (int32, strides for batch and head; NULL: the slots chosen last)
@@ -540,8 +544,8 @@ WriteCall write_args(PyObject* cache, const at::Tensor* index, const at::Tensor&
   set_cache_tensors(a, cache, w.held);
   const at::ScalarType type =
       (a.kv_dtype == KVX_KV_F16 || a.kv_dtype == KVX_KV_U8_F16 || a.kv_dtype == KVX_KV_U4_F16) ? at::kHalf : at::kBFloat16;
-  w.key = rows_of(key, type);
-  w.value = rows_of(value, type);
+  w.key = rows_of(key, type, w.strided);
+  w.value = rows_of(value, type, w.strided);
   a.B = (int32_t)key.size(0);
   a.Hkv = (int32_t)key.size(1);
   a.num = (int32_t)key.size(2);
@@ -616,8 +620,7 @@ PyObject* prefill_first(PyObject* const* args, Py_ssize_t n) {
   if (!fills && !lib.kvx_cache_write_first) raise(PyExc_ImportError, "the bound library does not export kvx_cache_write_first");
   for (const at::Tensor* t : {&q, &w.key, &w.value}) require_gpu(*t);
   check_bhtd("query", q);
-  check_bhtd("key", w.key);
-  check_bhtd("value", w.value);
+  if (w.strided) raise(PyExc_ValueError, "key, value: the head dimension must be contiguous");  // as for any attention over the caller's rows
   check_dtypes(q, w.key, &w.value, false);
   check_kv(q, w.key, w.value, false);
   check_heads(q.size(1), key.size(1));

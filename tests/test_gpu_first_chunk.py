@@ -38,6 +38,19 @@ def test_slots_behind_the_first_chunk(kvx, gpu, name, B, Hkv, T, D, lengths, spa
             assert torch.isfinite(cache.q_errors).all() and (cache.q_errors[:B, :, :num] > 0).all()
 
 
+@pytest.mark.parametrize("which", [0, 1])
+@pytest.mark.parametrize("name,dtype,spare", [("h2o-default", torch.bfloat16, 0), ("h2o-torch-quantized8", torch.float32, 0), ("h2o-default", torch.bfloat16, 1)])
+def test_rows_with_a_strided_head_dimension_are_refused(kvx, gpu, name, dtype, spare, which):
+    gen = torch.Generator().manual_seed(5)
+    q, k, v = (randn(gen, 1, h, 40, 64).to(gpu) for h in (4, 2, 2))
+    kv = [k.to(dtype), v.to(dtype)]
+    kv[which] = kv[which].transpose(2, 3).contiguous().transpose(2, 3)
+    cache = create_kv_cache(name, KVCacheParams(1 + spare, 2, 300, 64, 4))
+    with pytest.raises(ValueError, match="head dimension must be contiguous"):
+        cache.forward(q, *kv)
+    assert cache.forward(q, k, v).shape == (1, 40, 256)
+
+
 def test_refusals(kvx):
     a = _lib.CacheWriteArgs()
     a.B, a.Hkv, a.num, a.D, a.cache_len = 1, 65536, 1, 64, 65536
