@@ -422,9 +422,9 @@ PyObject* score_sum(PyObject* const* args, Py_ssize_t n) {
   a.lse = (float*)lse.data_ptr();
   at::Tensor w;
   check(unlocked([&] {
+    const at::Tensor ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));  // asked without w: no partials of an attention lie ahead of the sums
     w = L.empty({a.B, a.Hkv, a.kv_len}, at::kFloat);
     a.w = (float*)w.data_ptr();
-    const at::Tensor ws = L.scratch(lib.kvx_sdpa_prefill_workspace_bytes(&a));
     a.workspace = data(ws);
     a.workspace_bytes = ws.defined() ? (size_t)ws.numel() : 0;
     return lib.kvx_score_sum(&a, L.stream);

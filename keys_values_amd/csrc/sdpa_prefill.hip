@@ -1096,13 +1096,15 @@ size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy) {
   PrefillParams p;
   const bool copy = may_copy && wants_copy(a);
   size_t partials = 0;
+  bool merged = false;  // by the launches of the tiled score-sums
   for (const bool combined : {false, true}) {
     fill_params(p, copy ? on_copy(a, nullptr) : prefill_block(a), combined);
     partials = std::max(partials, partial_bytes(p, a.D));  // (max on the host is one of ints)
+    if (!combined) merged = a.w && !p.period && score_sum_merges(a, merge_params(p), true);
   }
-  // the score-sum pass that may follow on the same stream takes the place of the copy, or behind partials that it combines itself
+  // the score-sum pass that may follow on the same stream takes the place of the copy or of the partials, and where it combines those a place behind them
   const size_t sums = score_sum_workspace(a);
-  const size_t own = copy ? copy_bytes(a) + partials : partials && a.w ? (partials + 15) / 16 * 16 + sums : partials;
+  const size_t own = copy ? copy_bytes(a) + partials : merged ? (partials + 15) / 16 * 16 + sums : partials;
   return std::max({own, sums, a.w ? rows_weights_workspace(a) : 0});  // (max on the host is one of ints)
 }
 

@@ -395,6 +395,23 @@ def test_copy_of_a_store_is_refused_beyond_the_blocks_of_a_launch(kvx):
         assert kvx.kvx_sdpa_prefill_copying(ctypes.byref(a), None) == status
 
 
+@pytest.mark.parametrize("B,heads,kv_heads,q_len,kv_len,D,input_pos,combined", [
+    (1, 32, 8, 101, 3013, 128, 2912, 1),   # the sums lie behind the partials that the same launches combine
+    (1, 8, 2, 152, 11212, 64, 11060, 0),   # 44 pairs a row: combined in a launch of their own, the sums take their place
+    (1, 8, 2, 596, 14030, 64, 0, 0),       # a causal first chunk in splits
+    (1, 16, 8, 809, 36679, 64, 0, 0),      # one split
+])
+def test_workspace_of_weights_holds_partials_and_sums_where_both_are_read(kvx, B, heads, kv_heads, q_len, kv_len, D, input_pos, combined):
+    a = _prefill_block(B, heads, kv_heads, q_len, kv_len, D, 0)
+    a.input_pos = input_pos
+    without = kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a))  # the larger of partials and sums
+    a.lse = a.w = 4096
+    plan = prefill_plan(a)
+    assert (plan.one_launch, plan.score_sum, plan.combined) == (0, _lib.KVX_SCORE_SUM_TILED, combined)
+    need = kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a))
+    assert need > without if combined else need == without
+
+
 @pytest.mark.parametrize("B,heads,kv_heads,q_len,kv_len,D", [(1, 4, 1, 3, 64, 64), (1, 8, 2, 128, 1024, 64), (1, 16, 4, 128, 1500, 64), (1, 2, 1, 8, 8000, 128)])
 def test_a_chunk_waits_for_a_few_times_its_own_time(kvx, B, heads, kv_heads, q_len, kv_len, D):
     # a poll is 1.5 to 2 us, these calls take 10 to 20; the single-token step waits for 2^15 polls
