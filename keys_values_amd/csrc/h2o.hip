@@ -874,7 +874,7 @@ struct ListPlan {
 };
 static ListPlan list_plan(const kvx_h2o_args& a) {
   ListPlan p{};
-  if (a.k <= 1 || a.B <= 0 || a.Hkv <= 0 || a.kv_len <= 0 || (int64_t)a.B * a.Hkv > 65535) return p;
+  if (a.k <= 1 || a.B <= 0 || a.Hkv <= 0 || a.kv_len <= 0 || (int64_t)a.B * a.Hkv > 65535) return p;  // (more rows: a workgroup each fills the device)
   const int64_t C = ((int64_t)a.kv_len + LIST - 1) / LIST, rows = (int64_t)a.B * a.Hkv;
   if (C > 256 || rows * C * LIST * 8 > (1ll << 30)) return p;
   p.C = (int)C;

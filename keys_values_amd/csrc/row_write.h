@@ -141,7 +141,7 @@ __device__ __forceinline__ void quantize8_kv(const u32x4_t& k, const u32x4_t& v,
   vc = u32x2_t{codes4_u8(xv[0], xv[1], xv[2], xv[3], iv, zv), codes4_u8(xv[4], xv[5], xv[6], xv[7], iv, zv)};
 }
 
-// Codes of the lane's 8 values as bytes (0..15), same layout as quantize8.
+// Codes of the lane's 8 values as bytes (0..15), in the layout of quantize8_kv.
 template <int LPR, bool F16>
 __device__ __forceinline__ u32x2_t quantize4(u32x4_t raw, float& scale, int32_t& zp) {
   float x[8];
