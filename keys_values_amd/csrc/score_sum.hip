@@ -212,7 +212,8 @@ __device__ __forceinline__ float combined_lse(const f32x2_t* ml, int64_t total_r
 
 // The log-sum-exps of the rows of `tiles` tiles from row0 on, by a workgroup of THREADS, from the pairs of the attention's KV splits. A combination
 // ahead of this launch is 5 to 9 us and its gap; every workgroup working its rows' pairs out again is a latency beside that of its
-// keys: 16 pairs a thread are in flight.
+// keys: 16 pairs a thread are in flight. Up to 16 pairs are added in the order of the combination (merge_rows_job), and the weights have the bits that
+// its log-sum-exps give; of 17 to 32, the most (score_sum_merges), two lanes add every other one each, and the last bit may differ.
 template <int THREADS>
 __device__ __forceinline__ void fill_lse(const ScoreParams& p, const MergeParams& m, int b, int kvh, int tid, int row0, int tiles, float* lse_sh) {
   const int S = m.num_splits * m.teams, RT = p.rows_per_tile, n = tiles * BQ;
@@ -246,7 +247,7 @@ __device__ __forceinline__ void fill_lse(const ScoreParams& p, const MergeParams
   } else if (S <= 8) {
     rows(std::integral_constant<int, 8>{});
   } else {
-    const int lt = S <= 16 ? 0 : S <= 32 ? 1 : S <= 64 ? 2 : 3, T = 1 << lt, part = tid & (T - 1);
+    const int lt = S <= 16 ? 0 : 1, T = 1 << lt, part = tid & (T - 1);
     for (int i = tid >> lt; i < n; i += THREADS >> lt) {  // the lanes of a row leave the loop together
       const float lse = combined_lse(ml + min(row_of(i), p.R - 1), total_rows, S, part, T);
       if (part == 0) lse_sh[i] = has_row(i) ? lse : INFINITY;
