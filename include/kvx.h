@@ -368,6 +368,8 @@ int kvx_cache_write_first(const kvx_cache_write_args* args, void* stream);
  * can write the rows as well (head sizes 64 and 128, a causal chunk: input_pos 0, no token positions, q_len == kv_len == num, rows of the store's element type), else
  * one after the other. Nothing of what either reads may overlap what the other writes. */
 int kvx_sdpa_prefill_first(const kvx_sdpa_args* args, const kvx_cache_write_args* write, void* stream);
+/* How kvx_sdpa_prefill_first takes the call: 1: the attention's workgroups write the rows, 0: a launch ahead of it does (or the call is refused). */
+int kvx_sdpa_prefill_first_in_one_launch(const kvx_sdpa_args* args, const kvx_cache_write_args* write);
 
 /* H2O score update and eviction choice, AttnWeightsKVCache._update with H2OKVCache._compute_scores
  * (keys_values/kvcache/attn_weights.py:721-783, keys_values/kvcache/h2o.py:146-199):

@@ -140,6 +140,7 @@ SYMBOLS = {
     "kvx_cache_write": (ctypes.c_int, [POINTER(CacheWriteArgs), c_void_p]),
     "kvx_cache_write_first": (ctypes.c_int, [POINTER(CacheWriteArgs), c_void_p]),
     "kvx_sdpa_prefill_first": (ctypes.c_int, [POINTER(SdpaArgs), POINTER(CacheWriteArgs), c_void_p]),
+    "kvx_sdpa_prefill_first_in_one_launch": (ctypes.c_int, [POINTER(SdpaArgs), POINTER(CacheWriteArgs)]),
     "kvx_h2o_update_select": (ctypes.c_int, [POINTER(H2OArgs), c_void_p]),
     "kvx_h2o_decode_step": (ctypes.c_int, [POINTER(CacheWriteArgs), POINTER(SdpaArgs), POINTER(H2OArgs), c_void_p]),
     "kvx_h2o_decode_step_workspace_bytes": (c_size_t, [POINTER(SdpaArgs), POINTER(H2OArgs)]),

@@ -328,14 +328,21 @@ int kvx_cache_write_first(const kvx_cache_write_args* a, void* stream) {
   return rc != KVX_OK ? rc : launch_cache_write(*a, nullptr, (hipStream_t)stream, true);
 }
 
-int kvx_sdpa_prefill_first(const kvx_sdpa_args* a, const kvx_cache_write_args* w, void* stream) {
-  const char* who = "kvx_sdpa_prefill_first";
-  int rc = check_sdpa_common(a, who, true);
+static int check_prefill_first(const kvx_sdpa_args* a, const kvx_cache_write_args* w, const char* who) {
+  const int rc = check_sdpa_common(a, who, true);
   if (rc != KVX_OK) return rc;
   KVX_REQUIRE(a->q_len <= a->kv_len, KVX_ERR_INVALID, "%s: q_len=%d exceeds kv_len=%d", who, a->q_len, a->kv_len);
   KVX_REQUIRE(aligned16(a->workspace), KVX_ERR_WORKSPACE, "%s: workspace must be 16-byte aligned", who);
-  rc = check_cache_write_first(w, who);
+  return check_cache_write_first(w, who);
+}
+
+int kvx_sdpa_prefill_first(const kvx_sdpa_args* a, const kvx_cache_write_args* w, void* stream) {
+  const int rc = check_prefill_first(a, w, "kvx_sdpa_prefill_first");
   return rc != KVX_OK ? rc : launch_sdpa_prefill(*a, false, (hipStream_t)stream, nullptr, w);
+}
+
+int kvx_sdpa_prefill_first_in_one_launch(const kvx_sdpa_args* a, const kvx_cache_write_args* w) {
+  return check_prefill_first(a, w, "kvx_sdpa_prefill_first_in_one_launch") == KVX_OK && sdpa_prefill_writes_first(*a, *w);
 }
 
 size_t kvx_h2o_workspace_bytes(const kvx_h2o_args* a) { return a ? h2o_workspace(*a) : 0; }

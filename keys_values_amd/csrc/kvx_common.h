@@ -55,6 +55,7 @@ bool score_sum_combines(const kvx_sdpa_args& a);
 // whether the launches of the tiled kernel combine these partials (splits, teams and rows of m), in less time than a launch of their own would take. `room`: the
 // workspace has what sdpa_prefill_workspace asks for; else it is looked at
 bool score_sum_merges(const kvx_sdpa_args& a, const MergeParams& m, bool room);
+bool sdpa_prefill_writes_first(const kvx_sdpa_args& a, const kvx_cache_write_args& w);  // whether launch_sdpa_prefill does so in the same launch
 size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy);
 int sdpa_prefill_block_rows(const kvx_sdpa_args& a, bool may_copy);
 kvx_prefill_plan sdpa_prefill_plan(const kvx_sdpa_args& a, bool may_copy);

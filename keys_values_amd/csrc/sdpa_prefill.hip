@@ -1119,6 +1119,12 @@ static bool writes_first(const kvx_sdpa_args& a, const PrefillParams& p, const k
          (p.G > 2 || a.q_len <= 1024);
 }
 
+bool sdpa_prefill_writes_first(const kvx_sdpa_args& a, const kvx_cache_write_args& w) {
+  PrefillParams p;
+  fill_params(p, prefill_block(a));
+  return writes_first(a, p, w);
+}
+
 int launch_sdpa_prefill(const kvx_sdpa_args& a_in, bool may_copy, hipStream_t st, MergeParams* rest, const kvx_cache_write_args* first) {
   PrefillParams p;
   kvx_sdpa_args a = prefill_block(a_in);

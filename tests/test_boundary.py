@@ -400,6 +400,7 @@ def test_copy_of_a_store_is_refused_beyond_the_blocks_of_a_launch(kvx):
     (1, 8, 2, 152, 11212, 64, 11060, 0),   # 44 pairs a row: combined in a launch of their own, the sums take their place
     (1, 8, 2, 596, 14030, 64, 0, 0),       # a causal first chunk in splits
     (1, 16, 8, 809, 36679, 64, 0, 0),      # one split
+    (1, 28, 4, 703, 6646, 256, 5943, 0),   # 40 tiles of rows
 ])
 def test_workspace_of_weights_holds_partials_and_sums_where_both_are_read(kvx, B, heads, kv_heads, q_len, kv_len, D, input_pos, combined):
     a = _prefill_block(B, heads, kv_heads, q_len, kv_len, D, 0)
@@ -410,6 +411,51 @@ def test_workspace_of_weights_holds_partials_and_sums_where_both_are_read(kvx, B
     assert (plan.one_launch, plan.score_sum, plan.combined) == (0, _lib.KVX_SCORE_SUM_TILED, combined)
     need = kvx.kvx_sdpa_prefill_workspace_bytes(ctypes.byref(a))
     assert need > without if combined else need == without
+
+
+def _first_chunk_blocks(heads, kv_heads, tokens, **fields):
+    """Argument blocks of a first chunk: fields of the slot write, or of the attention with a leading ``a_``."""
+    a, w = _prefill_block(1, heads, kv_heads, tokens, tokens, 128, 0), _lib.CacheWriteArgs()
+    a.workspace, a.workspace_bytes = 4096, 2**40
+    w.B, w.Hkv, w.num, w.D, w.cache_len, w.kv_dtype = 1, kv_heads, tokens, 128, 4096, _lib.KVX_KV_U8
+    w.index = w.key = w.value = w.k_cache = w.v_cache = w.token_pos = w.k_scale = w.k_zp = w.v_scale = w.v_zp = 4096
+    w.key_stride_t = w.value_stride_t = w.kc_stride_t = w.vc_stride_t = 128
+    for name, value in fields.items():
+        setattr(*((a, name[2:]) if name.startswith("a_") else (w, name)), value)
+    return ctypes.byref(a), ctypes.byref(w)
+
+
+def test_first_chunks_in_one_launch(kvx):
+    """Which first chunks are one launch (on 256 compute units, what is assumed without a device)."""
+    def one(heads=16, kv_heads=8, tokens=1000, **fields):
+        return kvx.kvx_sdpa_prefill_first_in_one_launch(*_first_chunk_blocks(heads, kv_heads, tokens, **fields))
+
+    assert one() == 1
+    for fields in ({"num": 999}, {"kv_dtype": _lib.KVX_KV_U8_F16}, {"D": 64}, {"B": 2}, {"a_input_pos": 1}, {"a_token_positions": 4096}, {"a_kv_len": 1001},
+                   {"a_kv_dtype": _lib.KVX_KV_F16}):
+        assert one(**fields) == 0  # other rows than those attended over, or not a first chunk
+    assert one(tokens=1024) == 1 and one(tokens=1025) == 0  # two heads a KV head
+    assert one(heads=32, tokens=3072) == 1 and one(heads=32, tokens=3073) == 0  # three blocks of rows a unit
+    assert one(input_pos=1) == 0  # refused
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the pointers are made up: where nothing can be launched")
+@pytest.mark.parametrize("heads,kv_heads,tokens,one", [(16, 8, 1000, 1), (8, 8, 137, 0)])
+def test_first_chunk_with_its_attention_refuses(kvx, heads, kv_heads, tokens, one):
+    def call(**fields):
+        return kvx.kvx_sdpa_prefill_first(*_first_chunk_blocks(heads, kv_heads, tokens, **fields), None)
+
+    assert kvx.kvx_sdpa_prefill_first_in_one_launch(*_first_chunk_blocks(heads, kv_heads, tokens)) == one
+    assert call() == _lib.KVX_ERR_HIP  # a call like any other: no device
+    assert call(num=tokens - 1) == call(a_input_pos=5) == call(a_token_positions=4096) == call(kv_dtype=_lib.KVX_KV_U8_F16) == _lib.KVX_ERR_HIP  # two launches
+    assert call(input_pos=4) == _lib.KVX_ERR_INVALID  # not the first chunk
+    assert call(replay_log=4096, log_blocksize=64) == _lib.KVX_ERR_INVALID
+    assert call(grace_num=1, grace_period=1, grace_slots=4096, input_pos=1) == _lib.KVX_ERR_INVALID
+    assert call(key=0) == call(key=4100) == call(cache_len=tokens - 1) == call(k_scale=0) == _lib.KVX_ERR_INVALID
+    assert call(Hkv=65536, cache_len=32768) == _lib.KVX_ERR_UNSUPPORTED  # 2^31 slots
+    assert call(Hkv=65536, cache_len=32767, num=4096) == _lib.KVX_ERR_UNSUPPORTED  # 2^24 workgroups
+    assert call(a_kv_len=tokens - 1) == call(a_q=0) == _lib.KVX_ERR_INVALID
+    assert call(a_workspace=4100) == _lib.KVX_ERR_WORKSPACE
 
 
 @pytest.mark.parametrize("B,heads,kv_heads,q_len,kv_len,D", [(1, 4, 1, 3, 64, 64), (1, 8, 2, 128, 1024, 64), (1, 16, 4, 128, 1500, 64), (1, 2, 1, 8, 8000, 128)])

@@ -130,6 +130,35 @@ def test_other_threads_run_during_a_call(gpu, stub):
         assert stub.value == before + launches
 
 
+def test_first_chunks_with_libraries_from_before_the_one_call(gpu, tmp_path):
+    """The two calls that it stands for, in their order: the write of a chunk that fills the cache is an ordinary one."""
+    names = {"kvx_cache_write": 1, "kvx_cache_write_first": 2, "kvx_sdpa_prefill": 3}
+    host = _lib.host()
+    try:
+        for without in ((), ("kvx_cache_write_first",)):
+            src, so = tmp_path / f"stub{len(without)}.c", tmp_path / f"libstub{len(without)}.so"
+            calls = "".join(f"int {n}(const void* a) {{ order[n++] = {i}; return 0; }}\n" for n, i in names.items() if n not in without)
+            others = "".join(f"size_t {n}(void) {{ return 0; }}\n" for n in _lib.SYMBOLS if n not in names and n not in ("kvx_sdpa_prefill_first",))
+            src.write_text("#include <stddef.h>\nint order[16], n;\n" + calls + others)
+            subprocess.check_call(["gcc", "-shared", "-fPIC", str(src), "-o", str(so)])
+            host.bind(str(so), _lib.KvxError, torch.OutOfMemoryError)
+            lib = ctypes.CDLL(str(so))
+            n, order = ctypes.c_int.in_dll(lib, "n"), (ctypes.c_int * 16).in_dll(lib, "order")
+            for num, want in ((64, [1, 3]), (40, [2, 3])):
+                cache = H2OKVCache(KVCacheParams(1, 2, 64, 64, 4), device=gpu)
+                q, k = (torch.zeros(1, h, num, 64, dtype=torch.bfloat16, device=gpu) for h in (4, 2))
+                n.value = 0
+                if num < 64 and without:
+                    with pytest.raises(ImportError):
+                        cache.forward(q, k, k)
+                    assert n.value == 0
+                else:
+                    assert cache.forward(q, k, k).shape == (1, num, 256)
+                    assert order[:n.value] == want
+    finally:
+        host.bind(_lib.LIB_PATH, _lib.KvxError, torch.OutOfMemoryError)
+
+
 def test_two_threads_on_two_streams(gpu):
     """Caches stepped by two threads at once, each on its stream: the bits of the same steps one after the other."""
 
