@@ -1109,13 +1109,19 @@ size_t sdpa_prefill_workspace(const kvx_sdpa_args& a, bool may_copy) {
 }
 
 // Whether the attention launch of a first chunk writes the chunk's rows too: the tiled kernel, for one team, over the rows that are written, where its workgroups
-// have few tokens each (64 of two heads, 128 of one, begin so late that the longest ends later) and are few: a write on its own runs at the memory's
-// rate where it is long. us, two launches -> one: 253 tokens of 2 x 32 heads over 4 19.2 -> 14.7, 343 of 32 over 4 19.2 -> 16.6, 1163 of 32 over 8 35.7 -> 33.5,
-// 2109 of 28 over 4 57.1 -> 55.5, 566 of 64 values, 2 x 16 heads over 8 16.7 -> 14.6; 1408 of 2 x 32 over 8 53.8 -> 53.1; but 1967 of 16 over 8 45.4 -> 46.8,
-// 4096 of 32 over 8 145.7 -> 146.3, 4214 166.1 -> 166.6, 8192 517 -> 518.
+// are few: a write on its own runs at the memory's rate where it is long. us, two launches -> one: 253 tokens of 2 x 32 heads over 4 19.2 -> 14.7, 343 of 32 over 4
+// 19.2 -> 16.6, 1163 of 32 over 8 35.7 -> 33.5, 2109 of 28 over 4 57.1 -> 55.5, 566 of 64 values, 2 x 16 heads over 8 16.7 -> 14.6; 1408 of 2 x 32 over 8 53.8 -> 53.1; but 1967
+// of 16 over 8 45.4 -> 46.8, 4096 of 32 over 8 145.7 -> 146.3, 4214 166.1 -> 166.6, 8192 517 -> 518.
+// And where a workgroup's share of the write, the rows of 128 / G tokens, is short, or there are workgroups enough that others' products run beside it: of up to three heads a KV
+// head it is spread over the device by a launch of its own where blocks of rows a unit are fewer than its values / 12288, rows that are not quantised counting a third. Codes: 969 tokens of
+// 8 heads over 8 (0.25 blocks a unit, 1.33 is the line) 21.8 -> 29.3, 304 of 4 x 8 over 8 17.7 -> 24.0, 516 of 16 over 8 (0.28, 0.67) 18.6 -> 20.5, 233 of 2 x 24 over 8 (0.38, 0.44) 15.7 -> 17.1, but
+// 968 of 2 x 16 over 8 (1.0) 32.7 -> 32.4, 954 31.1 -> 29.8, 836 of 2 x 32 over 16 (1.75) 36.5 -> 33.5; plain 947 of 8 over 8 (0.25, 0.44) 20.4 -> 21.1, 419 of 4 x 8 over 8 (0.5) 18.3 -> 18.0.
+// Over 303 such calls of 0.12 to 1.6 blocks a unit, 1 to 8 heads a KV head, the choice takes 0.04 % longer than the better of both in the mean,
+// always one launch 1.9 %, always two 6 %.
 static bool writes_first(const kvx_sdpa_args& a, const PrefillParams& p, const kvx_cache_write_args& w) {
+  const int64_t blocks = (int64_t)p.B * p.Hkv * p.m_blocks, values = 128 * a.D / p.G / (kv_is_plain(w.kv_dtype) ? 3 : 1);
   return a.D <= 128 && kv_is_plain(a.kv_dtype) && !p.columns && !p.pair && !a.token_positions && a.input_pos == 0 && a.q_len == a.kv_len && w.B == a.B && w.Hkv == a.Hkv &&
-         w.num == a.q_len && w.D == a.D && kv_elem_f16(w.kv_dtype) == kv_elem_f16(a.kv_dtype) && (int64_t)p.B * p.Hkv * p.m_blocks <= 3 * num_cus() &&
+         w.num == a.q_len && w.D == a.D && kv_elem_f16(w.kv_dtype) == kv_elem_f16(a.kv_dtype) && blocks <= 3 * num_cus() && (p.G > 3 || blocks * 12288 >= num_cus() * values) &&
          (p.G > 2 || a.q_len <= 1024);
 }
 

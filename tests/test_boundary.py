@@ -427,20 +427,23 @@ def _first_chunk_blocks(heads, kv_heads, tokens, **fields):
 
 def test_first_chunks_in_one_launch(kvx):
     """Which first chunks are one launch (on 256 compute units, what is assumed without a device)."""
-    def one(heads=16, kv_heads=8, tokens=1000, **fields):
+    def one(heads=32, kv_heads=8, tokens=1000, **fields):
         return kvx.kvx_sdpa_prefill_first_in_one_launch(*_first_chunk_blocks(heads, kv_heads, tokens, **fields))
 
     assert one() == 1
     for fields in ({"num": 999}, {"kv_dtype": _lib.KVX_KV_U8_F16}, {"D": 64}, {"B": 2}, {"a_input_pos": 1}, {"a_token_positions": 4096}, {"a_kv_len": 1001},
                    {"a_kv_dtype": _lib.KVX_KV_F16}):
         assert one(**fields) == 0  # other rows than those attended over, or not a first chunk
-    assert one(tokens=1024) == 1 and one(tokens=1025) == 0  # two heads a KV head
-    assert one(heads=32, tokens=3072) == 1 and one(heads=32, tokens=3073) == 0  # three blocks of rows a unit
+    assert one(tokens=3072) == 1 and one(tokens=3073) == 0  # three blocks of rows a unit
+    assert one(kv_heads=16, tokens=1024) == 1 and one(kv_heads=16, tokens=1025) == 0  # two heads a KV head
+    assert one(kv_heads=16, tokens=641) == 1 and one(kv_heads=16, tokens=640) == 0  # 176 and 160 blocks of rows, 64 tokens of 128 codes to write each
+    plain = {"kv_dtype": _lib.KVX_KV_BF16, "heads": 16, "kv_heads": 16}  # 128 and 112, 128 tokens each
+    assert one(tokens=897, **plain) == 1 and one(tokens=896, **plain) == 0 and one(16, 16, 897) == 0
     assert one(input_pos=1) == 0  # refused
 
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="the pointers are made up: where nothing can be launched")
-@pytest.mark.parametrize("heads,kv_heads,tokens,one", [(16, 8, 1000, 1), (8, 8, 137, 0)])
+@pytest.mark.parametrize("heads,kv_heads,tokens,one", [(32, 8, 1000, 1), (8, 8, 137, 0)])
 def test_first_chunk_with_its_attention_refuses(kvx, heads, kv_heads, tokens, one):
     def call(**fields):
         return kvx.kvx_sdpa_prefill_first(*_first_chunk_blocks(heads, kv_heads, tokens, **fields), None)

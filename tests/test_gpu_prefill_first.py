@@ -29,16 +29,19 @@ def route(kvx, cache, q, k, v):
     ("h2o-vlen-default", torch.float16, 1, 8, 2, 2000, 1001, 128, 1, 4),        # in splits that end at bounds of blocks: the first ones write
     ("h2o-default", torch.bfloat16, 1, 8, 2, 3000, 2111, 64, 1, 4),
     ("h2o-vlen-torch-quantized8", torch.float16, 2, 28, 4, 517, 517, 128, 1, 1),  # tokens whose heads lie in two blocks; no slot behind the chunk
-    ("qh2o-vlen-torch-quantized8", torch.bfloat16, 1, 16, 8, 1100, 1000, 128, 1, 3),
-    ("qh2o-vlen-torch-quantized4", torch.bfloat16, 1, 8, 8, 4200, 900, 128, 1, 4),  # 128 tokens a workgroup; many slots to clear
+    ("qh2o-vlen-torch-quantized8", torch.bfloat16, 2, 16, 8, 1100, 1000, 128, 1, 1),
+    ("qh2o-vlen-torch-quantized8", torch.bfloat16, 1, 8, 2, 2500, 2001, 128, 1, 4),
+    ("h2o-vlen-default", torch.bfloat16, 2, 8, 8, 4200, 900, 128, 1, 4),        # 128 tokens a workgroup; many slots to clear
+    ("qh2o-vlen-torch-quantized4", torch.bfloat16, 4, 8, 8, 1500, 1001, 64, 1, 1),
     ("h2o-torch-quantized4", torch.float16, 1, 16, 2, 1500, 1100, 128, 1, 3),
     ("qh2o-torch-quantized8", torch.bfloat16, 1, 24, 8, 700, 650, 64, 1, 1),
     ("h2o-torch-quantized4", torch.float16, 2, 32, 4, 1300, 1001, 64, 1, 1),
     ("qh2o-vlen-torch-quantized4", torch.float16, 1, 16, 4, 1500, 1201, 64, 1, 3),
-    # two launches: the kernel for few rows, one of two heads with more than 1024 tokens, heads of 256
+    # two launches: the kernel for few rows, workgroups with many rows to write and no others beside them, two heads with more than 1024 tokens, heads of 256
     ("h2o-default", torch.bfloat16, 1, 32, 8, 300, 253, 128, 0, 1),
     ("qh2o-vlen-torch-quantized4", torch.bfloat16, 1, 8, 8, 2000, 137, 128, 0, 1),
     ("h2o-vlen-default", torch.float16, 1, 6, 2, 900, 641, 128, 0, 1),
+    ("qh2o-vlen-torch-quantized4", torch.bfloat16, 1, 8, 8, 1200, 900, 128, 0, 4),
     ("qh2o-vlen-torch-quantized8", torch.bfloat16, 1, 16, 8, 1100, 1030, 128, 0, 4),
     ("qh2o-vlen-torch-quantized8", torch.bfloat16, 1, 8, 2, 400, 300, 256, 0, 5),
 ])
