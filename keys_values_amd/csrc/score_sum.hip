@@ -993,6 +993,17 @@ bool merge_beside(const kvx_sdpa_args& a, const ScorePlan& pl, const MergeParams
   return jobs * 2500 <= spare * walk;
 }
 
+// Whether the score jobs' workgroups have few enough pairs to read between them, of all splits of their rows each (fill_lse): at 56 KB per us and unit (fitted over 420
+// calls, 0.7 us beside it) they spend on it what a launch of its own takes, 3 us, from about 24 K pairs a unit on. Attention with weights, us, combined here -> in a
+// launch of its own: up to 2500 pairs a unit 6 % longer in the mean, 10 to 12 K 2, 15 to 20 K alike; 1092 rows of 64 over 4 x 52480 keys (46 K) 147.0 -> 141.3,
+// 896 of 128 over 4 x 46790 (88 K) 157.1 -> 145.5, 1336 of 64 over 4 x 45027 (118 K) 170.0 -> 152.6, 270 of 256 over 8 x 46297 (58 K) 336.8 -> 321.5. Over the 420 the
+// choice takes 0.12 % longer than the better of both in the mean; always here 0.7 %, never 3.5 %.
+bool pairs_are_few(const kvx_sdpa_args& a, const ScorePlan& pl, const MergeParams& m) {
+  const int S = m.num_splits * m.teams, asked = S <= 4 ? 4 : S <= 8 ? 8 : S <= 16 ? 16 : 32;
+  const int64_t wgs = (int64_t)a.B * a.Hkv * ((a.kv_len + pl.waves * NW - 1) / (pl.waves * NW)) * pl.splits;
+  return wgs * pl.tiles_per_z * BQ * asked <= (int64_t)num_cus() * (24 << 10);
+}
+
 }  // namespace
 
 int score_sum_kind(const kvx_sdpa_args& a) { return is_short(a) ? KVX_SCORE_SUM_SHORT : is_streamed(a) ? KVX_SCORE_SUM_STREAMED : KVX_SCORE_SUM_TILED; }
@@ -1001,7 +1012,7 @@ bool score_sum_combines(const kvx_sdpa_args& a) { return is_short(a) || (is_stre
 bool score_sum_merges(const kvx_sdpa_args& a, const MergeParams& m, bool room) {
   if (score_sum_kind(a) != KVX_SCORE_SUM_TILED || m.num_splits <= 1 || m.num_splits * m.teams > 32 || merge_wants_classes(m, a.D)) return false;
   const ScorePlan pl = score_plan(a);
-  return pl.tiles_per_z <= LT && (pl.splits > 1 ? room || score_scratch(a, &m) != nullptr : merge_beside(a, pl, m));
+  return pl.tiles_per_z <= LT && pairs_are_few(a, pl, m) && (pl.splits > 1 ? room || score_scratch(a, &m) != nullptr : merge_beside(a, pl, m));
 }
 
 size_t score_sum_workspace(const kvx_sdpa_args& a) {

@@ -413,6 +413,23 @@ def test_workspace_of_weights_holds_partials_and_sums_where_both_are_read(kvx, B
     assert need > without if combined else need == without
 
 
+@pytest.mark.parametrize("heads,kv_heads,q_len,D,kv_len,pairs", [
+    (16, 4, 488, 128, 50688, 8),   # eight wavefronts
+    (28, 4, 110, 128, 30208, 18),  # likewise, over 16 pairs a row
+    (28, 4, 340, 128, 19968, 6),   # a split of the query rows
+    (28, 4, 73, 256, 43520, 16),
+    (8, 2, 262, 128, 23040, 28),
+    (32, 8, 422, 64, 28672, 6),
+])
+def test_weights_over_long_stores_leave_the_splits_to_a_launch_of_their_own(kvx, heads, kv_heads, q_len, D, kv_len, pairs):
+    """The line lies where all workgroups of the score-sums together would read 24 K (maximum, sum) pairs a compute unit."""
+    for more in (0, 1):  # one more block of keys
+        a = _prefill_block(1, heads, kv_heads, q_len, kv_len + more, D, 0)
+        a.input_pos, a.lse, a.w = kv_len + more - q_len, 4096, 4096
+        plan = prefill_plan(a)
+        assert (plan.score_sum, plan.splits * plan.teams, plan.combined) == (_lib.KVX_SCORE_SUM_TILED, pairs, 1 - more)
+
+
 def _first_chunk_blocks(heads, kv_heads, tokens, **fields):
     """Argument blocks of a first chunk: fields of the slot write, or of the attention with a leading ``a_``."""
     a, w = _prefill_block(1, heads, kv_heads, tokens, tokens, 128, 0), _lib.CacheWriteArgs()

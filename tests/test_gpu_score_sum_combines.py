@@ -131,3 +131,18 @@ def test_same_bits_as_launches_of_their_own(kvx, gpu, dtype, bits, copying, B, H
             torch.testing.assert_close(got[2], want[2], rtol=4e-6, atol=0)
     check_out(out, lse, ref)
     torch.testing.assert_close(w.cpu(), ref[1], rtol=1e-3, atol=1e-6)
+
+
+@pytest.mark.parametrize("kv_len,combined", [(19968, 1), (19969, 0)])
+def test_on_both_sides_of_the_line_of_long_stores(kvx, gpu, kv_len, combined):
+    q, k, v, _ = make_qkv(41, 1, 28, 4, 340, kv_len, 128)
+    q, k, v = q.to(gpu), k.to(gpu), v.to(gpu)
+    scale, pos = 128 ** -0.5, kv_len - 340
+    a = _lib.SdpaArgs()
+    ops._fill_common(a, q, k, v, scale, pos, None, None, 0)
+    a.o = a.lse = a.w = q.data_ptr()  # nothing is launched: any aligned address
+    assert prefill_plan(a).combined == combined
+    out, w, lse = ops.prefill_core(q, k, v, scale, pos, return_weights=True, return_lse=True)
+    out1, _, lse1 = ops.prefill_core(q, k, v, scale, pos, return_lse=True)
+    assert torch.equal(out, out1) and torch.equal(lse, lse1)
+    assert torch.equal(w, ops.score_sum_core(q, k, lse, scale, pos))
